@@ -1,0 +1,146 @@
+'''The convolution / matrix-product kernels on the bf16 matrix cores (csrc/kernels/conv_split.h): every operand is taken apart
+into three bf16 numbers. Integer-valued data make every product and sum exact, so those results have to be equal; on
+random data the error against 64-bit sums is bounded by what three parts and fp32 accumulation can lose.'''
+import numpy as np
+import pytest
+
+import vkjax_amd
+from vkjax_amd import kernels as K
+from vkjax_amd import minijax as mj
+from vkjax_amd.jaxpr_interpreter import JaxprInterpreter
+
+from .common import check_against_oracle
+
+lax, nn, jnp = mj.lax, mj.nn, mj.numpy
+DN = ('NHWC', 'HWIO', 'NHWC')
+rng = np.random.RandomState(23)
+
+
+def ints(shape, low=-4, high=5):
+    return rng.randint(low, high, size=shape).astype(np.float32)
+
+
+def conv(stride=(1, 1), padding='SAME', dilation=(1, 1)):
+    return lambda x, k: lax.conv_general_dilated(x, k, stride, padding, rhs_dilation=dilation, dimension_numbers=DN)
+
+
+def split_kernels(fn):
+    return [l.kernel for l in list(fn._jaxpr_interpreters.values())[0].launches if l.kernel.startswith('conv_gemm')]
+
+
+#rows, columns and contractions around the tile edges (128 rows, 64 or 128 columns, k tiles of 32), one and an odd number
+#of k tiles, a contraction that ends inside a k tile, kernel taps outside the image, strides, dilation, negative padding's rows
+SHAPES = [
+    ('1x1, one k tile',                 [1, 11, 12, 32],  [1, 1, 32, 64],   conv()),
+    ('1x1, 127 rows, 3 k tiles',        [1, 127, 1, 96],  [1, 1, 96, 63],   conv()),
+    ('1x1, 129 rows, 65 columns',       [1, 129, 1, 64],  [1, 1, 64, 65],   conv()),
+    ('1x1, k ends in a tile, 2 rows',   [1, 2, 1, 132],   [1, 1, 132, 130], conv()),
+    ('1x1, 4 features',                 [1, 40, 7, 4],    [1, 1, 4, 33],    conv()),
+    ('1x1 stride 2',                    [3, 15, 14, 64],  [1, 1, 64, 40],   conv((2, 2))),
+    ('3x3 SAME',                        [2, 9, 11, 64],   [3, 3, 64, 70],   conv()),
+    ('3x3 VALID, odd number of k tiles', [2, 13, 12, 32], [3, 3, 32, 128],  conv(padding='VALID')),
+    ('3x3 stride 2, 96 features',       [2, 15, 15, 96],  [3, 3, 96, 129],  conv((2, 2))),
+    ('3x3 dilated',                     [1, 17, 13, 32],  [3, 3, 32, 20],   conv(dilation=(2, 3))),
+    ('5x5 SAME',                        [1, 10, 9, 32],   [5, 5, 32, 17],   conv()),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('tile', list(K.CONV_SPLIT_TILES))
+@pytest.mark.parametrize('desc,xs,ks,f', SHAPES, ids=[s[0] for s in SHAPES])
+def test_tile_edges_and_slices(tile, desc, xs, ks, f):
+    x, k = ints(xs), ints(ks, -3, 4)
+    ktiles = 2 * -(-int(np.prod(ks[:3])) // 64)
+    for slices in (1, 2, 3, 7):
+        if slices > 1 and ktiles < 2 * slices:
+            continue
+        print(f'case: {desc}, tile {tile}, {slices} slices', flush=True)
+        with K.overrides(conv_split=tile, conv_split_slices=slices):
+            _, _, fn = check_against_oracle(f, [x, k], exact=True)
+        assert split_kernels(fn) == [f'conv_gemm_split_{tile}'], split_kernels(fn)
+        #a second and third evaluation find the counters of the slices at zero again
+        first = fn(x, k)
+        assert np.array_equal(first, fn(x, k))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('slices', (1, 3))
+def test_epilogues_and_second_results(slices):
+    '''Batch norm, residual and ReLU in the launch, a centred result stored beside it, and an epilogue the kernels do not apply
+    (it stays a launch of its own).'''
+    x, k, r = ints([2, 14, 13, 64]), ints([3, 3, 64, 72], -3, 4), ints([2, 14, 13, 72], -50, 50)
+    mean, scale, beta = ints([72]), ints([72], 1, 4), ints([72], -9, 9)
+    def bn_residual(x, k, mean, scale, beta, r):
+        return nn.relu((conv()(x, k) - mean) * scale + beta + r)
+    def centred_too(x, k, mean, scale, beta, r):
+        c = conv()(x, k) - mean
+        return nn.relu(c * scale + beta), c
+    def other_order(x, k, mean, scale, beta, r):
+        return (conv()(x, k) * scale - mean) * beta
+    for f in (bn_residual, centred_too, other_order):
+        with K.overrides(conv_split=True, conv_split_slices=slices):
+            _, _, fn = check_against_oracle(f, [x, k, mean, scale, beta, r], exact=True)
+        assert len(split_kernels(fn)) == 1 and split_kernels(fn)[0].startswith('conv_gemm_split_')
+
+
+@pytest.mark.gpu
+def test_gradients_pack_transposed_and_reversed_kernels():
+    '''Input gradients of strided and unit-stride convolutions: the kernel operand is packed straight from the forward
+    kernel (swapped features, reversed taps, every other tap), results go to every other position of the array.'''
+    for stride, xs, ks in (((1, 1), [2, 10, 9, 32], [3, 3, 32, 64]), ((2, 2), [2, 12, 11, 32], [3, 3, 32, 64]), ((2, 2), [1, 9, 9, 64], [1, 1, 64, 32])):
+        g = lambda x, k: mj.grad(lambda v, w: (lax.conv_general_dilated(v, w, stride, 'SAME', dimension_numbers=DN) ** 2).sum())(x, k)
+        print(f'case: gradient, stride {stride}, {xs} {ks}', flush=True)
+        with K.overrides(conv_split=True):
+            _, _, fn = check_against_oracle(g, [ints(xs, -2, 3), ints(ks, -2, 3)], exact=True)
+        assert sum(name.startswith('conv_gemm_split') for name in split_kernels(fn)) >= 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('k', (32, 1000, 4608))
+def test_error_against_64_bit_sums(k):
+    '''|error| <= (2^-24 for the parts left out + (6 k / 16 + 16) 2^-24 for the roundings of the accumulator) sum |x||w|, and not
+    above that of the fp32 kernels in the 2-norm (0.4 to 0.9 times measured on data of one scale).'''
+    x, w = rng.standard_normal((300, k)).astype(np.float32), rng.standard_normal((k, 96)).astype(np.float32)
+    x[:, 0] *= 1e4                                       #parts of very different size in one sum
+    exact  = x.astype(np.float64) @ w.astype(np.float64)
+    limit  = (6 * k / 16 + 17) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64))
+    errors = {}
+    for choice in (True, False):
+        with K.overrides(conv_split=choice):
+            fn = vkjax_amd.wrap(lambda x, w: jnp.dot(x, w), frontend='minijax')
+            errors[choice] = np.abs(fn(x, w).astype(np.float64) - exact)
+        assert split_kernels(fn)[0].startswith('conv_gemm_split') == choice
+    assert (errors[True] <= limit).all()
+    assert np.linalg.norm(errors[True]) <= 1.05 * np.linalg.norm(errors[False])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('slices', (1, 2))
+def test_infinite_and_huge_operands(slices):
+    '''Operands that are infinite, NaN or beyond the largest bf16, in the rows and in the kernel, give what fp32 products give.'''
+    x, w = ints([140, 160]), ints([160, 70], -3, 4)
+    x[3, 5], x[70, 100], x[139, 159], x[20, 7] = np.inf, -np.inf, np.nan, 3.4e38
+    w[9, 2], w[159, 69], w[40, 33], w[41, 33] = np.inf, 3.4e38, -3.4e38, 1.0
+    x[:, 159] = np.where(np.isfinite(x[:, 159]), np.sign(x[:, 159]), x[:, 159])
+    x[:, 40] = np.sign(x[:, 40])
+    results = []
+    for choice in (True, False):
+        with K.overrides(conv_split=choice, conv_split_slices=slices if choice else None):
+            results.append(vkjax_amd.wrap(lambda x, w: jnp.dot(x, w), frontend='minijax')(x, w))
+    assert np.array_equal(results[0], results[1], equal_nan=True)
+    assert np.isnan(results[0]).any() and np.isinf(results[0]).any() and np.isfinite(results[0]).any()
+
+
+def test_plans_and_packed_layout():
+    '''Plan only: which products take these kernels, the argument block's tail, and the size of the packed operand.'''
+    def plan(m, k, n):
+        closed = mj.make_jaxpr(lambda x, w: jnp.dot(x, w))(np.zeros((m, k), np.float32), np.zeros((k, n), np.float32))
+        return JaxprInterpreter(closed, plan_only=True)
+    interp = plan(12544, 2304, 256)
+    assert [l.kernel for l in interp.launches][0] == 'conv_split_pack' and interp.launches[1].kernel.startswith('conv_gemm_split_')
+    pack, product = interp.launches
+    assert pack.buffers[0][0] is product.buffers[2][0] and pack.buffers[0][0].size * 4 == 8 * 36 * 12288 and pack.grid[0] == 8 * 72 * 2 // 4
+    whole, _, slices, each, extra = np.frombuffer(product.params, np.int32)[-5 - 9:-9]
+    assert each * slices + extra == 36 and product.grid[0] >= whole
+    for m, k, n in ((2048, 4608, 512), (12544, 64, 256), (4096, 256, 32)):          #too few rows, too short a contraction, too little work
+        assert all('split' not in l.kernel for l in plan(m, k, n).launches), (m, k, n)

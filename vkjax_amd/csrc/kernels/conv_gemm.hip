@@ -31,6 +31,7 @@
 // rows and columns outside the matrices are caught by the range check of the buffer descriptor
 // (an out-of-range load returns zeros, an out-of-range store is dropped); row decoding uses
 // multiply-high division by constants prepared on the host.
+#include <type_traits>
 #include "common.h"
 
 #define CONV_MAX_EPI 6
@@ -109,6 +110,30 @@ struct ConvDerived {
     uint32_t op[CONV_MAX_DERIVED];          // add / sub / mul / div / max / min / neg / rsqrt / sqrt, float
     uint32_t left[CONV_MAX_DERIVED];        // the operand is the left argument
 };
+
+// the derived operand from its arrays' values: same arithmetic, operation by operation, as the element-wise kernel
+__device__ __forceinline__ float conv_derived_value(const float (&in)[CONV_MAX_DERIVED + 1], const ConvDerived& Dk) {
+    float v = in[0];
+#pragma unroll
+    for (int k = 0; k < CONV_MAX_DERIVED; ++k) {
+        if (k < (int)Dk.nsteps) {
+            const float a = Dk.left[k] ? in[k + 1] : v, b = Dk.left[k] ? v : in[k + 1];
+            switch (Dk.op[k]) {
+                case CEW_ADD_F:   v = a + b; break;
+                case CEW_SUB_F:   v = a - b; break;
+                case CEW_MUL_F:   v = a * b; break;
+                case CEW_DIV_F:   v = a / b; break;
+                case CEW_MAX_F:   v = (a > b || a != a) ? a : b; break;
+                case CEW_MIN_F:   v = (a < b || a != a) ? a : b; break;
+                case CEW_NEG_F:   v = -v; break;
+                case CEW_RSQRT_F: v = 1.0f / sqrtf(v); break;
+                case CEW_SQRT_F:  v = sqrtf(v); break;
+                default: break;
+            }
+        }
+    }
+    return v;
+}
 
 // LEAN: the variant for the common case, with the rarely needed paths compiled out (they cost
 // registers, and with them resident waves, even when not taken): both operands on the 16-byte
@@ -495,26 +520,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
     if constexpr (EPI_BEHIND_TILES) request_epilogue_operands();
     if (tid < BN) {
         if (Dk.nsteps) {
-            // the derived operand: same arithmetic, operation by operation, as the element-wise kernel
-            float v = d_in[0];
-#pragma unroll
-            for (int k = 0; k < CONV_MAX_DERIVED; ++k) {
-                if (k < (int)Dk.nsteps) {
-                    const float a = Dk.left[k] ? d_in[k + 1] : v, b = Dk.left[k] ? v : d_in[k + 1];
-                    switch (Dk.op[k]) {
-                        case CEW_ADD_F:   v = a + b; break;
-                        case CEW_SUB_F:   v = a - b; break;
-                        case CEW_MUL_F:   v = a * b; break;
-                        case CEW_DIV_F:   v = a / b; break;
-                        case CEW_MAX_F:   v = (a > b || a != a) ? a : b; break;
-                        case CEW_MIN_F:   v = (a < b || a != a) ? a : b; break;
-                        case CEW_NEG_F:   v = -v; break;
-                        case CEW_RSQRT_F: v = 1.0f / sqrtf(v); break;
-                        case CEW_SQRT_F:  v = sqrtf(v); break;
-                        default: break;
-                    }
-                }
-            }
+            const float v = conv_derived_value(d_in, Dk);
 #pragma unroll
             for (int e = 0; e < CONV_MAX_EPI; ++e)
                 if (e == (int)Dk.step) e_reg[e] = v;
@@ -819,6 +825,8 @@ CONV_KERNEL(conv_gemm_32x32x64_ks4, 1, 1, 1, 1, 64, true, true, true, 4)
 CONV_MIX_KERNEL(conv_gemm_64x64x32_mix, 32)
 CONV_MIX_KERNEL(conv_gemm_64x64x64_mix, 64)
 
+#include "conv_split.h"
+
 // ---------------------------------------------------------------------------------------------
 // Convolutions of dense images with very few features (an RGB stem: 7 x 7 x 3, stride 2). The general kernel
 // above assembles the A tile element by element for them: 1650 vector instructions per 64 x 64 tile against
@@ -896,25 +904,7 @@ __device__ __forceinline__ void conv_stem_body(float* __restrict__ out, const fl
                 const bool vec = (Dk.vector_mask >> k) & 1u;
                 in[k] = buffer_load_x1(make_rsrc(Dp.p[k], Dp.p[k] == nullptr ? 0u : vec ? (uint32_t)P.N * 4u : 4u), vec ? (uint32_t)tid * 4u : 0u);
             }
-            float v = in[0];
-#pragma unroll
-            for (int k = 0; k < CONV_MAX_DERIVED; ++k) {
-                if (k < (int)Dk.nsteps) {
-                    const float a = Dk.left[k] ? in[k + 1] : v, b = Dk.left[k] ? v : in[k + 1];
-                    switch (Dk.op[k]) {
-                        case CEW_ADD_F:   v = a + b; break;
-                        case CEW_SUB_F:   v = a - b; break;
-                        case CEW_MUL_F:   v = a * b; break;
-                        case CEW_DIV_F:   v = a / b; break;
-                        case CEW_MAX_F:   v = (a > b || a != a) ? a : b; break;
-                        case CEW_MIN_F:   v = (a < b || a != a) ? a : b; break;
-                        case CEW_NEG_F:   v = -v; break;
-                        case CEW_RSQRT_F: v = 1.0f / sqrtf(v); break;
-                        case CEW_SQRT_F:  v = sqrtf(v); break;
-                        default: break;
-                    }
-                }
-            }
+            const float v = conv_derived_value(in, Dk);
 #pragma unroll
             for (int e = 0; e < CONV_MAX_EPI; ++e)
                 if (e == (int)Dk.step) e_reg[e] = v;

@@ -1,0 +1,552 @@
+// fp32 implicit GEMM on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16). Included by conv_gemm.hip, whose parameter block,
+// epilogue and addressing these kernels share.
+//
+// An fp32 number is the sum of three bf16 numbers: hi = its nearest bf16, mid = the nearest bf16 of what is left, lo = the
+// rest, which has at most 8 significant bits by then (24 = 8 + 8 + 8). A product of two such numbers is taken as the six
+// products hi.hi, hi.mid, mid.hi, hi.lo, mid.mid, lo.hi, each exact in fp32 and added in fp32 accumulators; the three that are
+// left out are below 2^-24 of the product together, the rounding of an fp32 accumulation. The matrix cores run bf16 sixteen
+// times as fast as fp32, so six products instead of one are still 2.6 times as fast at peak.
+//   - exact for numbers from 2^-109 up (below, lo loses what a bf16 cannot hold: an absolute error under 2^-134);
+//   - operands that are infinite, NaN or beyond the largest bf16 (3.39e38) leave sums that are not finite, because a part that is
+//     infinite meets parts that are zero: a wave whose results are not all finite computes its tile again with
+//     v_mfma_f32_32x32x2_f32 and fp32 operands, so that such results are what they always were.
+// Measured against 64-bit sums (4096 x K x 128, normal data): an error of 0.88, 0.63 and 0.39 times that of
+// v_mfma_f32_32x32x2_f32 at K = 64, 576 and 2304 (which rounds after every second product, this after every sixteenth).
+#pragma once
+
+typedef __bf16   bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16   bf16x2 __attribute__((ext_vector_type(2)));
+typedef float    f32x2  __attribute__((ext_vector_type(2)));
+
+// the two numbers' nearest bf16, the first in the low half
+__device__ __forceinline__ uint32_t to_bf16x2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
+// Consecutive workgroup ids go to the 8 XCDs in turn: renumbers [0, n) so that every XCD works through a contiguous range.
+__device__ __forceinline__ int xcd_range(int id, int n) {
+    const int per = n / 8;
+    return per > 0 && id < per * 8 ? (id & 7) * per + (id >> 3) : id;
+}
+// stores and loads that are seen by every workgroup of the GPU, whichever L2 it stands behind (agent scope)
+__device__ __forceinline__ void buffer_store_x4_agent(f32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, soff, 16);
+}
+__device__ __forceinline__ f32x4 buffer_load_x4_agent(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 16));
+}
+
+// ---- the kernel operand, taken apart and laid out for the matrix cores ----------------------------------------------
+// A program's weights serve every row of a product: a launch of this kernel takes them apart once, instead of every tile of
+// rows doing it again, and lays them out in the order in which the lanes of a wave want them, so that the product's waves
+// load them straight into registers (16 bytes per lane, 1 KB per wave and load), past the LDS:
+//     [block of 32 columns][k16 step][part hi, mid, lo][lane] x 8 bf16
+// Lane l of a k16 step holds column l % 32 and octet o = 2 (step % 2) + l / 32 of its k tile of 32: k = 4o .. 4o+3 and
+// 16+4o .. 16+4o+3 (the order in which four lanes that share a row of the other operand load 64 contiguous bytes each time).
+// The kernel operand may lie in any order (strides, negative ones too), which makes the transposed and reversed kernels of a
+// backward pass no work of their own.
+struct ConvPackParams {
+    int32_t N, K, Cin, KW;               // k = (ky * KW + kx) * Cin + c
+    int32_t ws_r, ws_s, ws_c, ws_n;      // element strides of ky, kx, c, n
+};
+struct ConvPackEntry {
+    uint32_t first_block, pad;
+    u32x4*       out;
+    const float* w;
+    ConvPackParams P;
+};
+static_assert(sizeof(ConvPackEntry) == 56, "the host lays the table out with 56-byte entries");
+
+__device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const float* __restrict__ w, const ConvPackParams& P, int block) {
+    const int id = block * 256 + (int)threadIdx.x, lane = id & 63, step = id >> 6, ksteps = (P.K + 63) / 64 * 4;
+    const int nb = step / ksteps, s = step - nb * ksteps, o = 2 * (s & 1) + (lane >> 5), n = nb * 32 + (lane & 31);
+    if (nb * 32 >= P.N) return;
+    float x[8];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k0 = (s >> 1) * 32 + h * 16 + 4 * o, rs = k0 / P.Cin;
+        int c = k0 - rs * P.Cin, ky = rs / P.KW, kx = rs - ky * P.KW;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float v = (k0 + q < P.K && n < P.N) ? w[(int64_t)ky * P.ws_r + (int64_t)kx * P.ws_s + (int64_t)c * P.ws_c + (int64_t)n * P.ws_n] : 0.f;
+            x[4 * h + q] = s & 4 ? -v : v;                  // every other pair of k tiles: see the product's sums
+            if (++c == P.Cin) { c = 0; if (++kx == P.KW) { kx = 0; ++ky; } }
+        }
+    }
+    u32x4 part[3];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        float a = x[2 * q], b = x[2 * q + 1];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            uint32_t v = to_bf16x2(a, b);
+            if (t == 0) {
+                // a finite number beyond the largest bf16 keeps its leading bits instead of becoming infinite; behind an
+                // infinity or a NaN nothing is left: the three parts of any number add up to it
+                const bool fa = __builtin_isfinite(a), fb = __builtin_isfinite(b);
+                if (fa && (v & 0x7FFFu) == 0x7F80u) v = (v & 0xFFFF0000u) | (f2u(a) >> 16);
+                if (fb && (v & 0x7FFF0000u) == 0x7F800000u) v = (v & 0xFFFFu) | (f2u(b) & 0xFFFF0000u);
+                a = fa ? a - u2f(v << 16) : 0.f;
+                b = fb ? b - u2f(v & 0xFFFF0000u) : 0.f;
+            } else {
+                a = a - u2f(v << 16);
+                b = b - u2f(v & 0xFFFF0000u);
+            }
+            part[t][q] = v;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 3; ++t) out[(size_t)step * 192 + t * 64 + lane] = part[t];
+}
+extern "C" __global__ __launch_bounds__(256) void conv_split_pack(u32x4* __restrict__ out, const float* __restrict__ w, ConvPackParams P) {
+    conv_pack_body(out, w, P, blockIdx.x);
+}
+// The weights of several layers in one launch: workgroup b belongs to the last entry of the table whose first_block is <= b.
+extern "C" __global__ __launch_bounds__(256) void conv_split_pack_layers(const ConvPackEntry* __restrict__ table, uint32_t entries) {
+    uint32_t lo = 0, hi = entries;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (table[mid].first_block <= blockIdx.x) lo = mid; else hi = mid;
+    }
+    const ConvPackEntry& e = table[__builtin_amdgcn_readfirstlane(lo)];
+    conv_pack_body(e.out, e.w, e.P, (int)(blockIdx.x - e.first_block));
+}
+
+// ---- the product ------------------------------------------------------------------------------------------------------
+// Block = WGM x WGN waves, each with TM x TN tiles of 32 x 32; k tile 32, i.e. two k16 steps, taken in pairs. A tile of the
+// rows' operand is loaded as fp32 (two items per thread, each a row's octet in two 16-byte vectors), taken apart in registers and
+// put into one of two LDS buffers, [part][octet][row] x 8 bf16 (rows permuted by the octet: neither the writes nor the reads
+// of eight lanes in a row meet in a bank); the packed kernel operand goes straight into registers. Between the MFMAs of a k16
+// step: the next step's A parts are read from LDS as soon as this step has used a part for its last column, one item of the
+// next k tile (the next but one behind the barrier) is taken apart, written to LDS and requested for the k tile after it, and
+// the columns' parts are requested for the next k tile. Everything a wave waits for has been requested some 40 MFMAs of
+// 32 cycles before. One barrier per k tile, in its second step. The order of instructions is written down (FENCE): left
+// alone, the compiler gathers loads and splitting in front of or behind the MFMAs (a 128 x 128 x 4608 tile alone on a CU:
+// 273 us with one stage after the other, 193 without a branch in the loop, 147 with the order written down).
+//
+// What bounds it: power. On 8192 x 2048 x 8192 the matrix cores are busy 73 to 79 % of the time at 1.64 to 1.71 GHz, 207 to 221
+// TFLOP/s of fp32 products (133 through v_mfma_f32_32x32x2_f32, which cannot exceed 157); a loop of these MFMAs and nothing
+// else runs at 1.8 to 1.9 GHz. So what moves less data is faster: 128 x 64 tiles reach 0.88 of the 128 x 128 tiles' rate. The
+// layers of a network are shorter: start, stores and the last round of blocks count (12544 x 2304 x 256: 163 TFLOP/s).
+//
+// Sharing out: the first P.split_tiles_m tiles of the grid are computed by one block each, the contraction of every tile behind
+// them by P.m_blocks blocks (slices of P.m_each or one more pairs of k tiles). A slice's sums go to `partial`, and whichever block arrives
+// last at the tile's counter adds all slices in their order and applies the epilogue: no block waits for another. The
+// counters are left at zero for the next launch.
+
+template <int WGM, int WGN, int TM, int TN>
+__device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float* __restrict__ Es, int* __restrict__ Rs,
+                                                float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
+                                                float* __restrict__ partial, uint32_t* __restrict__ arrivals, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
+                                                const ConvParams& P, const ConvDerived& Dk) {
+    constexpr int BM = 32 * WGM * TM, BN = 32 * WGN * TN, NT = 64 * WGM * WGN, BK = 32;
+    u32x4* const As = pool;                         // [2 buffers][3 parts][4 octets][BM rows]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WGN, wn = wave % WGN, l32 = lane & 31, half = lane >> 5;
+    const bool c_contig = P.flags & 1u, flat_rows = P.flags & 2u, masked = P.flags & 4u;
+    const int nepi = (P.flags >> 8) & 15u, epi_first_full = (int)((P.flags >> 16) & 15u) - 1;
+    auto step_desc = [&](int e) -> uint32_t { return ((e < 3 ? P.epi_desc[0] : P.epi_desc[1]) >> (10 * (e < 3 ? e : e - 3))) & 1023u; };
+
+    const int ktiles = (P.K + 2 * BK - 1) / (2 * BK) * 2, slices = P.m_blocks, whole = P.split_tiles_m;
+    int work = (int)blockIdx.x, tile, slice = 0, kbeg = 0, kend = ktiles;
+    if (work < whole) {
+        tile = xcd_range(work, whole);
+    } else {
+        const int rest = P.tiles_m * P.tiles_n - whole;
+        work  = xcd_range(work - whole, rest * slices);
+        slice = work / rest;
+        tile  = whole + work - slice * rest;
+        kbeg  = 2 * (slice * P.m_each + min(slice, P.m_extra));
+        kend  = kbeg + 2 * (P.m_each + (slice < P.m_extra ? 1 : 0));
+    }
+    const bool sliced = (int)blockIdx.x >= whole;
+    const int tile_m = tile / P.tiles_n, tile_n = tile - tile_m * P.tiles_n;
+    const int m0 = tile_m * BM, n0 = tile_n * BN, HoWo = P.Ho * P.Wo;
+
+    const uint32_t x_bias = (uint32_t)(P.PH * P.xs_h + P.PW * P.xs_w) * 4u;
+    const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(reinterpret_cast<const char*>(x) - x_bias, P.x_bytes + x_bias),
+                                 w_rsrc = make_rsrc(w, P.w_bytes), o_rsrc = make_rsrc(out, P.out_bytes);
+
+    // ---- load assignment: A item = (row, octet of k); octet o holds k = 4o..4o+3 and 16+4o..16+4o+3 of the k tile
+    constexpr int A_NI = BM * 4 / NT, A_RSTEP = NT / 4;
+    const int a_o = tid & 3, a_r0 = tid >> 2;
+    uint32_t a_voff[A_NI], a_inv[A_NI];
+#pragma unroll
+    for (int p = 0; p < A_NI; ++p) {
+        const int m = m0 + a_r0 + p * A_RSTEP;
+        a_inv[p] = 0u;
+        if (flat_rows) {
+            a_voff[p] = m < P.M ? (uint32_t)(m * P.xs_h + a_o * 4) * 4u : CONV_OOB;
+            continue;
+        }
+        const int b = magic_div(m, P.howo_magic, P.howo_shift);
+        const int r2 = m - b * HoWo;
+        const int ho = magic_div(r2, P.wo_magic, P.wo_shift);
+        const int wo = r2 - ho * P.Wo;
+        a_voff[p] = m < P.M ? (uint32_t)(b * P.xs_b + ho * P.SH * P.xs_h + wo * P.SW * P.xs_w + a_o * 4) * 4u : CONV_OOB;
+        if (masked) {
+            const int hi0 = ho * P.SH - P.PH, wi0 = wo * P.SW - P.PW;
+            uint32_t wbad = 0u;
+            for (int s = 0; s < P.KW; ++s) wbad |= ((uint32_t)(wi0 + s * P.DW) >= (uint32_t)P.W ? 1u : 0u) << s;
+            const uint32_t wall = (2u << (P.KW - 1)) - 1u;
+            for (int r = 0; r < P.KH; ++r)
+                a_inv[p] |= ((uint32_t)(hi0 + r * P.DH) >= (uint32_t)P.H ? wall : wbad) << (r * P.KW);
+        }
+    }
+    // the packed columns of this wave (blocks of columns beyond the last one lie outside the descriptor and read as zeros)
+    uint32_t b_soff[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) b_soff[j] = (uint32_t)(n0 / 32 + wn * TN + j) * (uint32_t)ktiles * 6144u;
+    const uint32_t b_lane = (uint32_t)lane * 16u;
+    int t_r = 0, t_s = 0, t_c = kbeg * BK;          // kernel tap and first feature of the next k tile to load
+    if (kbeg > 0 && P.KH * P.KW > 1) {
+        const int rs = t_c / P.Cin;
+        t_c -= rs * P.Cin; t_r = rs / P.KW; t_s = rs - t_r * P.KW;
+    }
+    const uint32_t rowb = (uint32_t)P.N * 4u;
+    static_assert(A_NI == 2 && TM == 2, "two items per thread, two rows of tiles per wave: the schedule below");
+    f32x4 raw[2][2];
+    // requests item p of k tile kt (beyond the contraction: zeros)
+    auto load_item = [&](f32x4 (&to)[2], int kt, int p) {
+        const uint32_t soff = (uint32_t)(t_r * P.DH * P.xs_h + t_s * P.DW * P.xs_w + t_c) * 4u, sh = 31u - (uint32_t)(t_r * P.KW + t_s);
+        const uint32_t bad0 = kt * BK + a_o * 4 >= P.K ? CONV_OOB : 0u, bad1 = kt * BK + 16 + a_o * 4 >= P.K ? CONV_OOB : 0u;
+        const uint32_t v = a_voff[p] | ((a_inv[p] << sh) & CONV_OOB);
+        to[0] = buffer_load_x4(x_rsrc, v | bad0, soff);
+        to[1] = buffer_load_x4(x_rsrc, v | bad1, soff + 64u);
+    };
+    auto advance = [&]() {
+        t_c += BK;
+        const bool wrap_c = t_c >= P.Cin; t_c = wrap_c ? 0 : t_c; t_s += wrap_c ? 1 : 0;
+        const bool wrap_s = t_s == P.KW; t_s = wrap_s ? 0 : t_s; t_r += wrap_s ? 1 : 0;
+    };
+    float acc[TM][TN][16];
+    f32x16 sum[TM * TN] = {};                        // the products of a pair of k tiles
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    u32x4 bf[2][TN][3], af[TM][3];
+    auto load_b = [&](int kt, int ks, int t, int j) {
+        bf[ks][j][t] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, b_lane, b_soff[j] + (uint32_t)(2 * kt + ks) * 3072u + t * 1024u, 0);
+    };
+    int a_slot[TM];                                  // k16 step 0; the other one: two octets on
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a_slot[i] = half * BM + (((wm * TM + i) * 32 + l32) ^ (half * 2));
+    auto read_a = [&](const u32x4* from, int ks, int t, int i) { af[i][t] = from[(t * 4 + 2 * ks) * BM + (a_slot[i] ^ (ks * 4))]; };
+#define FENCE() __builtin_amdgcn_sched_barrier(0)
+    // An item's next part, and what is left of it: the eight numbers' nearest bf16, to LDS at `to`
+    const int p_slot = a_o * BM + (a_r0 ^ (a_o * 2));
+    auto split_word = [&](f32x4 (&x)[2], int t, int q) {
+        f32x4& v = x[q >> 1];
+        const int e = 2 * (q & 1);
+        const uint32_t w2 = to_bf16x2(v[e], v[e + 1]);
+        if (t < 2) { v[e] = v[e] - u2f(w2 << 16); v[e + 1] = v[e + 1] - u2f(w2 & 0xFFFF0000u); }
+        return w2;
+    };
+    u32x4 part;
+    auto park = [&](u32x4* to, int p, int t) { to[t * 4 * BM + (p_slot ^ (p * A_RSTEP))] = part; };
+
+    // The matrix cores cut off what lies below the last bit of a sum, towards minus infinity. So the products of a pair of k
+    // tiles are summed from zero (TM x TN chains of four times six products each) and added to the accumulators by fp32
+    // operations, rounded to nearest, while the next chain runs; and the packed operand has its sign changed in every
+    // other pair, whose sums are subtracted, so that what is cut off goes up as often as down. (All products into one
+    // accumulator: an error 1.7 to 2.7 times that of fp32 products at K = 576, of mean -3e-8 of the results' rms; chains of
+    // one sign: that mean, the same in every layer, left ResNet-50's logits 1.3e-6 from 64-bit ones where fp32 products are
+    // 4.1e-7 off and these 3.5e-7.)
+    // The order of the parts frees A's first: (A part, B part).
+    constexpr int PA[6] = {0, 0, 0, 1, 1, 2}, PB[6] = {2, 1, 0, 1, 0, 0};
+    constexpr int CH = TM * TN, NS = 6 * CH;
+    float sign = kbeg & 2 ? -1.f : 1.f;
+    auto k16_step = [&](auto step_, int kt) {
+        constexpr int step = decltype(step_)::value, ks = step & 1, item = 1 - ks;   // step of the pair of k tiles, the second of its k tile
+        u32x4 *const mine = As + (step >> 1) * 12 * BM, *const other = As + ((step >> 1) ^ 1) * 12 * BM;
+        constexpr int BARRIER = 6 * TN - 4;                                     // second step only: in front of the first part of the next tile
+        constexpr int SPLIT = ks == 0 ? 0 : BARRIER, EACH = (NS - SPLIT) / 6;   // an item's three parts, in halves, then its reload
+        u32x4* const to = ks == 0 ? other : mine;                               // k tile kt + 1, or kt + 2
+        FENCE();
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+            const int c = n / 6, t = n % 6, i = c / TN, j = c % TN;
+            if (ks == 1 && n == BARRIER) { __syncthreads(); FENCE(); }
+            sum[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i][PA[t]]), __builtin_bit_cast(bf16x8, bf[ks][j][PB[t]]),
+                                                             step == 0 && t == 0 ? f32x16{} : sum[c], 0, 0, 0);
+            // the chain before has seen its last product
+            if (step == (c > 0 ? 3 : 0) && t >= 2) {
+                const int pc = (c + CH - 1) % CH;
+#pragma unroll
+                for (int v = 4 * t - 8; v < 4 * t - 4; ++v) acc[pc / TN][pc % TN][v] = __builtin_fmaf(sum[pc][v], sign, acc[pc / TN][pc % TN][v]);
+            }
+            // parts of A that have met their last column are replaced by the next step's
+            if (j == TN - 1 && (t == 2 || t == 4 || t == 5)) read_a(ks == 1 ? other : mine, 1 - ks, t == 2 ? 0 : t == 4 ? 1 : 2, i);
+            // an item of a later k tile
+            if (n >= SPLIT && (n - SPLIT) % EACH == EACH - 1 && (n - SPLIT) / EACH < 6) {
+                const int h = (n - SPLIT) / EACH, pt = h / 2;
+                part[2 * (h & 1)] = split_word(raw[item], pt, 2 * (h & 1));
+                part[2 * (h & 1) + 1] = split_word(raw[item], pt, 2 * (h & 1) + 1);
+                if (h & 1) park(to, item, pt);
+                if (h == 5) load_item(raw[item], kt + (ks == 0 ? 2 : 3), item);
+            }
+            // the columns' parts of the next k tile
+#pragma unroll
+            for (int q = 0; q < TN; ++q)
+                if (q < TN - 1 ? n == (CH - TN + q + 1) * 6 + 1 : n == NS - 1) { load_b(kt + 1, ks, 2, q); load_b(kt + 1, ks, 1, q); load_b(kt + 1, ks, 0, q); }
+            FENCE();
+        }
+        if constexpr (ks == 0) advance();
+        if constexpr (step == 0) { if (kt > kbeg) sign = -sign; }
+    };
+
+    // The loads of the first k tiles, the last of them in the order in which the loop below issues those of later ones.
+    f32x4 first[3][2];
+    load_item(first[0], kbeg, 0);
+    load_item(first[1], kbeg, 1);
+    advance();
+    load_item(first[2], kbeg + 1, 0);
+    FENCE();
+    load_item(raw[1], kbeg + 1, 1);
+    advance();
+    FENCE();
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int q = 0; q < TN; ++q) {
+            if (ks == 1 && q == TN - 1) { load_item(raw[0], kbeg + 2, 0); FENCE(); }
+#pragma unroll
+            for (int t = 2; t >= 0; --t) { load_b(kbeg, ks, t, q); FENCE(); }
+        }
+    // ---- epilogue operands
+    if (tid < BN) {
+        float e_reg[CONV_MAX_EPI], d_in[CONV_MAX_DERIVED + 1];
+#pragma unroll
+        for (int e = 0; e < CONV_MAX_EPI; ++e) {
+            const uint32_t kind = step_desc(e) >> 8;
+            const uint32_t present = epi.p[e] != nullptr ? 1u : 0u;
+            e_reg[e] = buffer_load_x1(make_rsrc(epi.p[e], kind == 1 ? 4u * present : kind == 2 ? (uint32_t)P.N * 4u * present : 0u),
+                                      kind == 2 ? (uint32_t)(n0 + tid) * 4u : 0u);
+        }
+        if (Dk.nsteps) {
+#pragma unroll
+            for (int k = 0; k <= CONV_MAX_DERIVED; ++k) {
+                const bool vec = (Dk.vector_mask >> k) & 1u;
+                d_in[k] = buffer_load_x1(make_rsrc(Dp.p[k], Dp.p[k] == nullptr ? 0u : vec ? (uint32_t)P.N * 4u : 4u),
+                                         vec ? (uint32_t)(n0 + tid) * 4u : 0u);
+            }
+            const float v = conv_derived_value(d_in, Dk);
+#pragma unroll
+            for (int e = 0; e < CONV_MAX_EPI; ++e)
+                if (e == (int)Dk.step) e_reg[e] = v;
+        }
+#pragma unroll
+        for (int e = 0; e < CONV_MAX_EPI; ++e)
+            if (e < nepi) Es[e * BN + tid] = e_reg[e];
+    }
+
+    {
+#pragma unroll
+        for (int f = 0; f < 3; ++f) {
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) part[q] = split_word(first[f], t, q);
+                park(As + f / 2 * 12 * BM, f & 1, t);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int t = 0; t < 3; ++t) read_a(As, 0, t, i);
+        for (int kt = kbeg; kt < kend; kt += 2) {
+            k16_step(std::integral_constant<int, 0>{}, kt);
+            k16_step(std::integral_constant<int, 1>{}, kt);
+            k16_step(std::integral_constant<int, 2>{}, kt + 1);
+            k16_step(std::integral_constant<int, 3>{}, kt + 1);
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[TM - 1][TN - 1][v] = __builtin_fmaf(sum[CH - 1][v], sign, acc[TM - 1][TN - 1][v]);
+        __syncthreads();
+    }
+
+    if (sliced) {
+        // store this slice's sums; the block that arrives last adds all of them, in the order of the slices
+        const int mine = tile - whole;
+        const uint32_t tile_bytes = BM * BN * 4;
+        const __amdgpu_buffer_rsrc_t p_rsrc = make_rsrc(reinterpret_cast<char*>(partial) + (size_t)mine * slices * tile_bytes, (uint32_t)slices * tile_bytes);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; v += 4)
+                    buffer_store_x4_agent(f32x4{acc[i][j][v], acc[i][j][v + 1], acc[i][j][v + 2], acc[i][j][v + 3]}, p_rsrc,
+                                          (uint32_t)tid * 16u, (uint32_t)slice * tile_bytes + (uint32_t)((i * TN + j) * 4 + v / 4) * (NT * 16u));
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the stores above have reached memory
+        __syncthreads();
+        if (tid == 0) {
+            const uint32_t n = __hip_atomic_fetch_add(arrivals + mine, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (n + 1u == (uint32_t)slices) __hip_atomic_store(arrivals + mine, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            Rs[0] = (int)n;
+        }
+        __syncthreads();
+        if (Rs[0] + 1 != slices) return;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+#pragma nounroll
+        for (int s = 0; s < slices; ++s)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; v += 4) {
+                        const f32x4 q = buffer_load_x4_agent(p_rsrc, (uint32_t)tid * 16u, (uint32_t)s * tile_bytes + (uint32_t)((i * TN + j) * 4 + v / 4) * (NT * 16u));
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) acc[i][j][v + u] += q[u];
+                    }
+    }
+
+    // An operand that is infinite, not a number, or beyond the largest bf16 leaves a sum that is not finite (infinity
+    // times the zero parts of the other operand): such sub-tiles are computed again with fp32 products.
+    // An operand that is infinite, not a number, or beyond the largest bf16 leaves a sum that is not finite (infinity
+    // times the zero parts of the other operand): such sub-tiles are computed again with fp32 products.
+    {
+        float t = 0.f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) t = __builtin_fmaf(acc[i][j][v], 0.f, t);
+        if (__builtin_amdgcn_ballot_w64(t != t)) {
+            auto packed_value = [&](int k, int n) {
+                const int kk = k & 31, o = (kk & 15) >> 2, e = (kk & 3) + (kk >> 4) * 4;
+                const uint32_t at = n < P.N && k < P.K ? (uint32_t)(n >> 5) * (uint32_t)ktiles * 6144u + (uint32_t)(2 * (k >> 5) + (o >> 1)) * 3072u
+                                                         + (uint32_t)((o & 1) * 32 + (n & 31)) * 16u + (uint32_t)e * 2u : CONV_OOB;
+                float v[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) v[q] = u2f((uint32_t)__builtin_amdgcn_raw_buffer_load_b16(w_rsrc, at, (uint32_t)q * 1024u, 0) << 16);
+                const float value = (v[2] + v[1]) + v[0];
+                return k & 64 ? -value : value;
+            };
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const int m = m0 + (wm * TM + i) * 32 + l32;
+                const int b = flat_rows ? 0 : magic_div(m, P.howo_magic, P.howo_shift), r2 = m - b * HoWo;
+                const int ho = flat_rows ? m : magic_div(r2, P.wo_magic, P.wo_shift), wo = flat_rows ? 0 : r2 - ho * P.Wo;
+                const int hi0 = ho * P.SH - P.PH, wi0 = wo * P.SW - P.PW;
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const int n = n0 + (wn * TN + j) * 32 + l32;
+                    f32x16 a2 = {};
+                    int r = 0, s = 0, c = half;
+#pragma nounroll
+                    for (int k = 0; k < P.K; k += 2) {
+                        const int hi = hi0 + r * P.DH, wi = wi0 + s * P.DW;
+                        const bool ok = m < P.M && (flat_rows || ((uint32_t)hi < (uint32_t)P.H && (uint32_t)wi < (uint32_t)P.W));
+                        const float av = buffer_load_x1(x_rsrc, ok ? (uint32_t)(b * P.xs_b + hi * P.xs_h + wi * P.xs_w + c) * 4u + x_bias : CONV_OOB);
+                        const float bv = packed_value(k + half, n);
+                        a2 = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, a2, 0, 0, 0);
+                        c += 2;
+                        if (c >= P.Cin) { c = half; if (++s == P.KW) { s = 0; ++r; } }
+                    }
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[i][j][v] = a2[v];
+                }
+            }
+        }
+    }
+
+    if (!c_contig) {
+        __syncthreads();
+        for (int r = tid; r < BM; r += NT) {
+            const int m = m0 + r;
+            const int b = m / HoWo, r2 = m - b * HoWo, ho = r2 / P.Wo, wo = r2 - ho * P.Wo;
+            Rs[r] = m < P.M ? b * P.os_b + ho * P.os_h + wo * P.os_w : -1;
+        }
+        __syncthreads();
+    }
+    auto sub_tile = [&](int i, int j, auto&& fn) {
+        const int n  = n0 + (wn * TN + j) * 32 + l32;
+        const int r0 = (wm * TM + i) * 32 + 4 * half;
+        if (c_contig) {
+            const uint32_t base = n < P.N ? (uint32_t)((m0 + r0) * P.N + n) * 4u : CONV_OOB;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) fn(v, base, (uint32_t)(8 * (v / 4) + (v % 4)) * rowb);
+        } else {
+            const int* ro = Rs + r0;
+            const int  cn = n < P.N ? n * P.os_n : -(1 << 30);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int r = ro[8 * (v / 4) + (v % 4)];
+                fn(v, (r >= 0 && cn >= 0) ? (uint32_t)(r + cn) * 4u : CONV_OOB, 0u);
+            }
+        }
+    };
+    const float* full_ptr = epi.p[0];
+#pragma unroll
+    for (int t = 1; t < CONV_MAX_EPI; ++t) full_ptr = epi_first_full == t ? epi.p[t] : full_ptr;
+    const __amdgpu_buffer_rsrc_t f_rsrc = make_rsrc(full_ptr, P.out_bytes);
+    const uint32_t slots = (P.flags >> 20) & 31u;
+    const int e_mul = __builtin_popcount(slots & 1u), e_add = __builtin_popcount(slots & 3u), e_max = __builtin_popcount(slots & 15u);
+    const int tap = (int)((P.flags >> 12) & 15u) - 1;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            float y[16], ov[16];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) y[v] = acc[i][j][v];
+            const int col = (wn * TN + j) * 32 + l32;
+            if (slots & 8u) sub_tile(i, j, [&](int v, uint32_t vo, uint32_t so) { ov[v] = buffer_load_x1_nt(f_rsrc, vo, so); });
+            auto tap_store = [&]() {
+                const __amdgpu_buffer_rsrc_t t_rsrc = make_rsrc(epi.p[CONV_MAX_EPI - 1], P.out_bytes);
+                sub_tile(i, j, [&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], t_rsrc, vo, so); });
+            };
+            if (tap == 0) tap_store();
+            if (slots & 1u) {
+                const float o = Es[col];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = y[v] - o;
+                if (tap == 1) tap_store();
+            }
+            if (slots & 2u) {
+                const float o = Es[e_mul * BN + col];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = y[v] * o;
+            }
+            if (slots & 4u) {
+                const float o = Es[e_add * BN + col];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = y[v] + o;
+            }
+            if (slots & 8u) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = y[v] + ov[v];
+            }
+            if (slots & 16u) {
+                const float o = Es[e_max * BN + col];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = (y[v] > o || y[v] != y[v]) ? y[v] : o;
+            }
+            sub_tile(i, j, [&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], o_rsrc, vo, so); });
+        }
+}
+
+#define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE)                                                                       \
+    extern "C" __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void name(             \
+        float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                                   \
+        float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) { \
+        __shared__ __attribute__((aligned(16))) u32x4 pool[24 * 32 * WGM * TM];                                              \
+        __shared__ float Es[CONV_MAX_EPI * 32 * WGN * TN];                                                                   \
+        __shared__ int Rs[32 * WGM * TM];                                                                                    \
+        conv_split_body<WGM, WGN, TM, TN>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);                        \
+    }
+// (2 x 2 waves of 64 x 64: 255 registers, two blocks per CU; 1 x 4 waves of 128 x 32, which load every column once, were 1 % slower)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128, 2, 2, 2, 2, 2)
+// for at most 64 columns, or where the smaller tile divides the rows better among the CUs: three blocks per CU
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64, 2, 2, 2, 1, 3)

@@ -369,13 +369,19 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                     while (p < pieces.size() && sorted_use[p] <= i) reached = (long)p++;
                     need[i] = reached;
                 }
-                // the first checkpoint lets the first launch go; behind it a handful, the distance doubling from
-                // CHECKPOINT_BYTES on (the first layers of a network read little and should not wait for much)
+                // the first checkpoint lets the first launch go (and one the launch that has an alternative form in parts);
+                // behind it a handful, the distance doubling from CHECKPOINT_BYTES on (the first layers of a network
+                // read little and should not wait for much)
                 if (need[0] >= 0 && (size_t)need[0] + 1 < pieces.size()) checkpoints.push_back((size_t)need[0]);
+                const long parts_end = s->early.empty() ? -1 : need[s->early_at];
                 size_t since = 0, step = CHECKPOINT_BYTES;
                 for (size_t q = (size_t)(need[0] + 1); q + 1 < pieces.size(); q++) {
                     since += pieces[q].nbytes;
-                    if (since >= step && (int)checkpoints.size() < Ctx::MAX_CHECKPOINTS - 1) { checkpoints.push_back(q); since = 0; step *= 2; }
+                    if (((long)q == parts_end || since >= step) && (int)checkpoints.size() < Ctx::MAX_CHECKPOINTS - 1) {
+                        checkpoints.push_back(q);
+                        since = 0;
+                        if ((long)q != parts_end) step *= 2;
+                    }
                 }
                 checkpoints.push_back(pieces.size() - 1);
             }
@@ -389,12 +395,13 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
             // The first launch in parts: a part goes to the side stream as soon as the chunks it reads have been
             // handed to the copy engines (both streams are in order: an event behind a chunk covers every chunk
             // before it), so the device computes while the rest of the argument is still on its way. Only with that
-            // argument as the last thing the first launch reads to be sent: whatever else it reads has then been sent.
+            // argument as the last thing that launch (and those recorded before it) reads to be sent: whatever else they
+            // read has then been sent. The launches recorded before it go in front of its first part.
             size_t early_piece = pieces.size(), next_part = 0;
             if (!s->early.empty() && !s->profiling && !s->want_graph && !s->uses_side) {
                 for (size_t p = 0; p < pieces.size(); p++)
                     if (piece_slot[p] == s->early_slot && pieces[p].nbytes >= s->early.back().bytes_needed) early_piece = p;
-                const size_t must_be = follow ? (size_t)(need[0] < 0 ? pieces.size() : need[0]) : pieces.size() - 1;
+                const size_t must_be = follow ? (size_t)(need[s->early_at] < 0 ? pieces.size() : need[s->early_at]) : pieces.size() - 1;
                 if (early_piece != must_be) early_piece = pieces.size();
             }
             hipError_t err = hipSuccess;
@@ -441,6 +448,8 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                     if ((err = hipEventRecord(part.ev_b, copy_odd)) != hipSuccess) return 1;
                     if ((err = hipStreamWaitEvent(parts_stream, part.ev_a, 0)) != hipSuccess) return 1;
                     if ((err = hipStreamWaitEvent(parts_stream, part.ev_b, 0)) != hipSuccess) return 1;
+                    while (next_launch < s->early_at)
+                        if ((launch_status = issue_launch(c, s->launches[next_launch++], parts_stream))) return 1;
                     if ((launch_status = issue_launch(c, part.launch, parts_stream))) return 1;
                 }
                 if (follow && next_checkpoint < checkpoints.size() && piece == checkpoints[next_checkpoint] && off + len == pieces[piece].nbytes) {
@@ -450,8 +459,8 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                     if ((err = hipEventRecord(ev_odd, copy_odd)) != hipSuccess) return 1;
                     if ((err = hipStreamWaitEvent(c->stream, ev_even, 0)) != hipSuccess) return 1;
                     if ((err = hipStreamWaitEvent(c->stream, ev_odd, 0)) != hipSuccess) return 1;
-                    // (every part of the first launch has been issued, on this stream: the last one needs no more than the whole argument)
-                    if (piece == early_piece && next_launch == 0) next_launch = 1;
+                    // (every part has been issued, on this stream: the last one needs no more than the whole argument)
+                    if (piece == early_piece && next_launch == s->early_at) next_launch = s->early_at + 1;
                     while (next_launch < nl && need[next_launch] <= (long)piece)
                         if ((launch_status = issue_launch(c, s->launches[next_launch++]))) return 1;
                 }
@@ -470,7 +479,7 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                     // (every part has been issued: the last one needs no more than the whole argument)
                     HIP_TRY(hipEventRecord(s->ev_early_done, c->side_stream));
                     HIP_TRY(hipStreamWaitEvent(c->stream, s->ev_early_done, 0));
-                    first_launch = 1;
+                    first_launch = s->early_at + 1;
                 }
             }
         } else {
@@ -1034,11 +1043,14 @@ int vkj_seq_record_early_part(vkj_handle sh, vkj_handle fh, const uint32_t grid[
                               const uint64_t* buf_byte_offsets, int nbufs, int upload_slot, size_t bytes_needed) {
     Seq* s = from_handle<Seq>(sh, MAGIC_SEQ);
     if (!s) return fail(VKJ_EINVAL, "vkj_seq_record_early_part: bad handle");
-    if (s->launches.empty()) return fail(VKJ_ESTATE, "vkj_seq_record_early_part: the launch the parts stand for is recorded first");
+    if (s->launches.empty()) return fail(VKJ_ESTATE, "vkj_seq_record_early_part: the launch the parts stand for has to be recorded before them");
     const Transfer* upload = nullptr;
     for (auto& t : s->uploads) if (t.slot == upload_slot) upload = &t;
     if (!upload || bytes_needed == 0 || bytes_needed > upload->nbytes)
         return fail(VKJ_EINVAL, "vkj_seq_record_early_part: no upload in slot %d, or it has fewer than %zu bytes", upload_slot, bytes_needed);
+    size_t at = 0;
+    while (at < s->launches.size() && std::find(s->launches[at].bufs.begin(), s->launches[at].bufs.end(), upload->buf) == s->launches[at].bufs.end()) at++;
+    if (at == s->launches.size()) return fail(VKJ_EINVAL, "vkj_seq_record_early_part: no launch reads the argument in slot %d", upload_slot);
     if (!s->early.empty() && (s->early_slot != upload_slot || bytes_needed < s->early.back().bytes_needed))
         return fail(VKJ_EINVAL, "vkj_seq_record_early_part: parts read one upload slot, in ascending order of what they need");
     if (int r = use(s->ctx)) return r;
@@ -1054,6 +1066,7 @@ int vkj_seq_record_early_part(vkj_handle sh, vkj_handle fh, const uint32_t grid[
     for (Buf* b : part.launch.bufs) b->seq_refs++;
     part.launch.fn->mod->seq_refs++;
     s->early_slot = upload_slot;
+    s->early_at = at;
     s->early.push_back(std::move(part));
     return 0;
 }

@@ -112,7 +112,7 @@ struct Launch {
                                                  // and waited for on this launch's lane before the launch is issued
 };
 
-// One part of the first launch's alternative form (vkj_seq_record_early_part): what it needs of the argument in
+// One part of a launch's alternative form (vkj_seq_record_early_part): what it needs of the argument in
 // upload slot Seq::early_slot, and the two events that tell its stream that those bytes have arrived.
 struct EarlyPart {
     Launch     launch;
@@ -137,8 +137,9 @@ struct Seq {
     bool                    graph_failed = false;   // capture did not work once: keep to plain launches
     hipGraphExec_t          graph_exec = nullptr;
     std::vector<std::pair<Slab*, void*>> slab_mirrors;   // pinned memory laid out like a slab: the staging of the uploads into its arrays
-    std::vector<EarlyPart>  early;                  // the first launch in parts, each issued while the rest of an argument is still on its way
+    std::vector<EarlyPart>  early;                  // a launch in parts, each issued while the rest of an argument is still on its way
     int                     early_slot = -1;
+    size_t                  early_at = 0;           // the recorded launch they stand for: the first that reads that argument
     hipEvent_t              ev_early_done = nullptr;
 };
 

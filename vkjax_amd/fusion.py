@@ -54,6 +54,8 @@ def _reads(op) -> tp.List:
             return [b for b, _ in op.launch.buffers[1:] if b is not None]
         if op.meta[0] == 'softmax':
             return [op.meta[2]]
+        if op.meta[0] == 'conv_pack':
+            return [op.meta[2].buffer]
     return [b for b, _ in op.launch.buffers if b is not None]
 
 
@@ -73,8 +75,8 @@ def _walks_densely(strides, shape) -> bool:
 def _through_copy(operand: EwOperand, copy: EwChain, shape) -> tp.Optional[EwOperand]:
     '''`operand` (of a chain over `shape`) reads the result of `copy`, a chain without steps, i.e. result[c] =
     source[offset + c . strides] over copy.shape. When every dimension the operand walks is one dimension of the
-    copy's result (a transposition, a slice, a broadcast of it, or the whole of it), the operand that reads the
-    copy's source directly is returned: the two index maps composed. None otherwise.'''
+    copy's result (a transposition, a slice, every n-th element, a broadcast of it, or the whole of it), the operand
+    that reads the copy's source directly is returned: the two index maps composed. None otherwise.'''
     src, cshape = copy.first, tuple(copy.shape)
     if operand.buffer.size != np_prod(cshape) or len(operand.strides) != len(shape):
         return None
@@ -90,11 +92,12 @@ def _through_copy(operand: EwOperand, copy: EwChain, shape) -> tp.Optional[EwOpe
         if n == 1 or s == 0:
             strides.append(0)
             continue
-        dims = [e for e in range(len(cshape)) if cshape[e] > 1 and dense[e] == s and e not in taken]
-        if len(dims) != 1 or start[dims[0]] + n > cshape[dims[0]]:
+        #the dimension with the largest pitch that divides the stride: the walk stays inside it or is none of one dimension
+        dims = [e for e in range(len(cshape)) if cshape[e] > 1 and s > 0 and s % dense[e] == 0 and e not in taken]
+        if not dims or start[dims[0]] + s // dense[dims[0]] * (n - 1) >= cshape[dims[0]]:
             return None
         taken.add(dims[0])
-        strides.append(src.strides[dims[0]])
+        strides.append(s // dense[dims[0]] * src.strides[dims[0]])
     return EwOperand(src.buffer, src.offset + sum(a * b for a, b in zip(start, src.strides)), tuple(strides))
 
 
@@ -223,8 +226,33 @@ def fuse_ops(all_ops, bufferpool, outvars):
         uses[pid] -= 1
         return fused
 
+    def fold_pack_source(op):
+        '''A kernel operand that is the result of a pure copy (the reversed kernel of an input gradient, a transposed
+        weight matrix) is packed straight from that copy's source.'''
+        _, packed, source, geom = op.meta
+        pid = id(source.buffer._placeholder)
+        prod = result[producer[pid]] if pid in producer else None
+        if prod is None or prod.chain is None or prod.chain.steps:
+            return op
+        through = _through_copy(source, prod.chain, (geom.KH, geom.KW, geom.Cin, geom.N))
+        if through is None:
+            return op
+        uses[pid] -= 1
+        uses[id(through.buffer._placeholder)] += 1
+        through.buffer.accesses.append(op.index)
+        if uses[pid] == 0:
+            uses[id(through.buffer._placeholder)] -= 1
+            _out(prod)._placeholder.elided = True
+            result[producer[pid]] = None
+            del producer[pid]
+        new = Op(op.equation, launch=K.conv_split_pack(packed, through, geom), meta=('conv_pack', packed, through, geom))
+        new.index = op.index
+        return new
+
     for op in all_ops:
         fused = None
+        if op.meta is not None and op.meta[0] == 'conv_pack':
+            op = fold_pack_source(op)
         if op.chain is not None:
             op = fold_copies(op)
             for cand in [o for o in op.chain.operands()[:2] if o is not None]:
@@ -259,6 +287,8 @@ def fuse_ops(all_ops, bufferpool, outvars):
                         continue
                     if K.conv_is_dense_rows(lhs, geom) and not K.dense_rows_epilogue_supported(list(epilogue) + extra):
                         continue                                  #the chain stays a launch of its own
+                    if geom.split is not None and not K.conv_split_epilogue_supported(list(epilogue) + extra):
+                        continue                                  #likewise
                     tap_at = [k for k, e in enumerate(epilogue) if e.op == K.CONV_TAP]
                     if tap_at and not K.conv_tap_supported(epilogue[:tap_at[0]], list(epilogue[tap_at[0] + 1:]) + extra):
                         continue
@@ -293,7 +323,7 @@ def fuse_ops(all_ops, bufferpool, outvars):
     ops = fold_index_wrap(ops, bufferpool, outvars)
     ops = fuse_dense_softmax(ops, bufferpool, outvars)
     ops = remove_dead_ops(ops, bufferpool, outvars)
-    return batch_small_chains(ops)
+    return batch_small_chains(batch_packs(ops))
 
 
 def fuse_softmax(ops, bufferpool, outvars):
@@ -977,7 +1007,7 @@ def _small_out(op):
 
 def _may_write(op) -> tp.List:
     '''Buffers an op may change: its result where the op's structure is known, else everything it touches.'''
-    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'reduce', 'softmax')):
+    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'reduce', 'softmax', 'conv_pack')):
         return _writes(op)
     return [b for b, _ in op.launch.buffers if b is not None]
 
@@ -986,6 +1016,43 @@ def _touched(op) -> tp.List:
     if op.chain is not None or op.conv is not None:
         return _reads(op) + _writes(op)
     return [b for b, _ in op.launch.buffers if b is not None]
+
+
+PACK_BATCH_ELEMENTS = 1 << 22          #weights that are packed by one launch, at least (16 MB)
+
+
+def batch_packs(ops):
+    '''Kernel operands that are packed for the matrix cores and depend on nothing the program computes (its weights) are
+    packed several layers at a time, in front of the first of those layers: one launch per 16 MB of weights instead of one
+    per layer, and not one for all of them, so that the first layers do not wait for weights of the last ones that are
+    still being uploaded.'''
+    from .ops import Op
+    written = set()
+    for op in ops:
+        written |= {id(b._placeholder) for b in _may_write(op)}
+    result, group, size, at = [], [], 0, None
+    def close():
+        if len(group) > 1:
+            batch = Op(_label(*group), launch=K.batch_launch([op.launch for op in group]))
+            batch.index = group[0].index
+            for op in group:
+                for b, _ in op.launch.buffers:
+                    b.accesses.append(batch.index)
+            result[at] = batch
+        group.clear()
+    for op in ops:
+        if op.meta is None or op.meta[0] != 'conv_pack' or id(op.meta[2].buffer._placeholder) in written:
+            result.append(op)
+            continue
+        if not group:
+            at, size = len(result), 0
+            result.append(op)
+        group.append(op)
+        size += op.meta[3].K * op.meta[3].N
+        if size >= PACK_BATCH_ELEMENTS:
+            close()
+    close()
+    return result
 
 
 BATCH_MIN_GAIN = 4          #launches a program must save before its small chains are moved and batched

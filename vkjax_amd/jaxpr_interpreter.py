@@ -153,31 +153,39 @@ class JaxprInterpreter:
     EARLY_PARTS_MIN_BYTES = 16 << 20
 
     def _early_parts_of_first_launch(self):
-        '''[(launch, upload slot, bytes of the argument the part needs)]: the program's first launch cut along the batch
+        '''[(launch, upload slot, bytes of the argument the part needs)]: the program's first product cut along the batch
         into parts that together compute what it computes, when it is a convolution or matrix product over a large
         argument whose images (rows) are computed independently by one kernel of the family in which a wave sums
         its contraction in one fixed order whatever the tiling (so every part's values are the whole launch's, bit for
         bit). The runtime issues a part as soon as the chunks of the argument it reads are on their way
         (vkj_seq_record_early_part); evaluations that do not upload that argument run the launch as it is.'''
-        if (not self.all_ops or self.profiling or self.graph or (self.lane_plan is not None and any(self.lane_plan.lane))
-                or self.all_ops[0].conv is None):
+        #(launches that pack weights for the matrix cores may stand in front of it)
+        at = next((i for i, l in enumerate(self.launches) if not l.kernel.startswith('conv_split_pack')), None)
+        if (at is None or self.profiling or self.graph or (self.lane_plan is not None and any(self.lane_plan.lane))
+                or self.all_ops[at].conv is None):
             return []
-        out, lhs, rhs, geom, epilogue = self.all_ops[0].conv
-        whole = self.launches[0]
+        out, lhs, rhs, geom, epilogue = self.all_ops[at].conv
+        whole = self.launches[at]
         k = next((i for i, b in enumerate(self.input_buffers) if b is lhs), None)
         if k is None or self._input_slots[k] is None or lhs.nbytes() < self.EARLY_PARTS_MIN_BYTES:
+            return []
+        if any(b is not None and b.tensor is lhs.tensor for l in self.launches[:at] for m in (l.members or (l,)) for b, _ in m.buffers):
             return []
         B = geom.batch
         nparts = 4 if B % 4 == 0 else 2 if B % 2 == 0 else 0
         plain = (whole.kernel.startswith('conv_gemm') and not any(tag in whole.kernel for tag in ('_mix', '_ks4')) and not whole.members)
-        if (not nparts or not plain or geom.k_splits > 1 or lhs.size % B or out.size % B or geom.xs[0] != lhs.size // B
+        if (not nparts or not plain or geom.k_splits > 1 or (geom.split is not None and geom.split.slices > 1) or lhs.size % B or out.size % B or geom.xs[0] != lhs.size // B
                 or geom.os[0] != out.size // B or any(e.kind == 3 or e.op in (K.CONV_TAP, K.CONV_SOFTMAX) for e in epilogue)):
             return []
         parts = []
         for p in range(nparts):
             try:
-                part = K.conv_gemm(out, lhs, rhs, geom._replace(batch=B // nparts), epilogue,
-                                   lhs_offset=p * (lhs.size // nparts), out_offset=p * (out.size // nparts))
+                sub = geom._replace(batch=B // nparts)
+                if geom.split is not None:
+                    tiles_m, tiles_n = K.conv_split_tiles(geom.split, sub)
+                    sub = sub._replace(split=geom.split._replace(whole=tiles_m * tiles_n))
+                part = K.conv_product(out, lhs, rhs, sub, epilogue,
+                                      lhs_offset=p * (lhs.size // nparts), out_offset=p * (out.size // nparts))
             except (ValueError, NotImplementedError):
                 return []
             if part.kernel != whole.kernel:

@@ -48,6 +48,8 @@ class _Choices:
         conv_dense_rows=None,            #the kernel for at most 16 output features: None = where it applies, False = never
         conv_mix=None,                   #mixed 64 x 64 / 32 x 32 tiling: None = by the heuristic, False = never, an int = that many M tiles stay 64 x 64
         conv_stem=None,                  #the patch kernel for few input features: False = never; None / True: where it applies; 64: its 64-position tiles only
+        conv_split=None,                 #the kernels on the bf16 matrix cores: None = where they pay, False = never, True or a tile's name = wherever they apply
+        conv_split_slices=None,          #blocks that share a tile behind the whole rounds (None: by the estimate)
         conv_k_splits=None,              #slices a contraction is cut into where that applies (None: by the heuristic, 1: never)
         conv_xcd_columns=0,              #four-waves-per-tile kernels: XCD columns over the tile grid (0: row-major ranges, None: least traffic)
         scatter_sort_threshold=1 << 18,  #update elements from which a row scatter-add sorts its updates instead of using atomics
@@ -332,10 +334,12 @@ REDUCE_BATCH_KERNELS = ('reduce_cols_fsum_v1', 'reduce_cols_fsum_v4')
 TRANSPOSE_BATCH_KERNELS = ('transpose_tiled_v4', 'transpose_tiled_v4_t128')
 BATCH_KERNELS        = {**{k: k.replace('ew_chain_', 'ew_chain_batch_') for k in EW_BATCH_KERNELS},
                         **{k: k.replace('fsum_', 'fsum_batch_') for k in REDUCE_BATCH_KERNELS},
-                        **{k: k.replace('tiled_', 'tiled_batch_') for k in TRANSPOSE_BATCH_KERNELS}}
+                        **{k: k.replace('tiled_', 'tiled_batch_') for k in TRANSPOSE_BATCH_KERNELS},
+                        'conv_split_pack': 'conv_split_pack_layers'}
 EW_BATCH_ENTRY_BYTES        = 432
 REDUCE_BATCH_ENTRY_BYTES    = 56
 TRANSPOSE_BATCH_ENTRY_BYTES = 48
+PACK_BATCH_ENTRY_BYTES      = 56
 BATCH_MAX_BLOCKS         = 4096        #launches of more workgroups than this keep a launch of their own
 REDUCE_NARROW_MAX_BLOCKS = 16          #column sums of at most this many workgroups trade block width for more blocks
 TRANSPOSE_BATCH_MAX_BLOCKS = 1024      #... tiled transposes (the kernels of a network, for its backward pass) up to this many
@@ -361,7 +365,8 @@ def batch_table(launch: Launch, device_address: tp.Callable[[Buffer], int]) -> n
     kind = launch.members[0].kernel
     is_chain, is_transpose = kind in EW_BATCH_KERNELS, kind in TRANSPOSE_BATCH_KERNELS
     entry_bytes, pointers = ((EW_BATCH_ENTRY_BYTES, 1 + EW_MAX_STEPS) if is_chain else
-                             (TRANSPOSE_BATCH_ENTRY_BYTES, 2) if is_transpose else (REDUCE_BATCH_ENTRY_BYTES, 2))
+                             (TRANSPOSE_BATCH_ENTRY_BYTES, 2) if is_transpose else
+                             (PACK_BATCH_ENTRY_BYTES, 2) if kind == 'conv_split_pack' else (REDUCE_BATCH_ENTRY_BYTES, 2))
     rows, first = [], 0
     for m in launch.members:
         assert len(m.buffers) == pointers, (m.kernel, len(m.buffers))
@@ -477,6 +482,8 @@ class ConvGeometry(tp.NamedTuple):
     #> 1: the contraction is cut into this many slices, each summed by blocks of its own into its own [M, N] matrix of
     #the result array (no epilogue); another launch adds the slices
     k_splits: int = 1
+    #how the kernels on the bf16 matrix cores share the product out, or None: the others compute it
+    split: tp.Optional['ConvSplit'] = None
 
     @property
     def M(self): return self.batch * self.Ho * self.Wo
@@ -979,6 +986,144 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
         kernel = f'conv_gemm_{tag}x{bk}_mix'
         blocks = split_tiles_m * tiles_n + _cdiv(M - split_tiles_m * 64, 32) * _cdiv(N, 32)
     return Launch(kernel, (blocks, 1, 1), (nt, 1, 1), buffers, params, bytes_moved=nbytes, flops=2 * M * N * K)
+
+
+# ------------------------------------------------- products on the bf16 matrix cores (csrc/kernels/conv_split.h)
+
+#tile -> (BM, BN, microseconds of a CU per k tile of 32: with several blocks on it, with one)
+CONV_SPLIT_TILES = {'128x128': (128, 128, 1.15, 1.15), '128x64': (128, 64, 0.65, 0.95)}
+#Products below these stay with the fp32 kernels. Rows: packing the kernel operand costs what about 250 rows' products cost,
+#and one launch. Contraction: with two k tiles of 32 a block is all start-up and stores (200704 x 64 x 256 with residual:
+#101 us here, 66 there, where a block walks several tiles; 50176 x 128 x 512: 59 against 61). Operations: launch latency.
+CONV_SPLIT_MIN_M, CONV_SPLIT_MIN_K, CONV_SPLIT_MIN_FLOPS = 2049, 128, 1e9
+CONV_SPLIT_MAX_SLICED = 4096       #tiles of one launch whose contraction is shared: counters set aside for them
+CONV_SPLIT_PACK_BYTES = 12288      #packed kernel operand: bytes per 32 columns and pair of k tiles of 32
+
+
+class ConvSplit(tp.NamedTuple):
+    '''How a product is shared out: the first `whole` tiles of the grid by one block each, the contraction of every tile
+    behind them by `slices` blocks. Those leave their sums in `partial`, and the one that finds at the tile's counter in
+    `arrivals` that it is the last adds them.'''
+    tile: str
+    whole: int
+    slices: int
+    partial: tp.Optional[Buffer] = None
+    arrivals: tp.Optional[Buffer] = None
+
+
+def conv_split_tiles(split: ConvSplit, g: ConvGeometry) -> tp.Tuple[int, int]:
+    bm, bn = CONV_SPLIT_TILES[split.tile][:2]
+    return _cdiv(g.M, bm), _cdiv(g.N, bn)
+
+
+def conv_split_partial_words(split: ConvSplit, g: ConvGeometry) -> int:
+    bm, bn = CONV_SPLIT_TILES[split.tile][:2]
+    tiles_m, tiles_n = conv_split_tiles(split, g)
+    return (tiles_m * tiles_n - split.whole) * split.slices * bm * bn
+
+
+def conv_split_packed_words(g: ConvGeometry) -> int:
+    return _cdiv(g.N, 32) * _cdiv(g.K, 64) * (CONV_SPLIT_PACK_BYTES // 4)
+
+
+def conv_split_plan(lhs: Buffer, g: ConvGeometry, lhs_offset: int = 0, compute_units: int = 256, sliceable: bool = True) -> tp.Optional[ConvSplit]:
+    '''The plan with the smallest estimated time, or None where these kernels do not apply or another one is faster.'''
+    if (CHOICES.conv_split is False or g.k_splits > 1 or _dense_rows_shape(lhs, g) or CHOICES.conv_general or CHOICES.conv_b_general
+            or any(v is not None for v in (CHOICES.conv_tile, CHOICES.conv_bk, CHOICES.conv_chunk, CHOICES.conv_ksplit, CHOICES.conv_k_splits, CHOICES.conv_mix))
+            or CHOICES.conv_stem not in (None, True)):
+        return None
+    g = _flatten_pointwise(g)
+    M, N, K = g.M, g.N, g.K
+    _, _, a_fast, _, _ = _conv_fast_paths(lhs, lhs, g, lhs_offset)
+    if not a_fast or (g.Cin % 32 != 0 and g.KH * g.KW != 1) or conv_split_packed_words(g) * 4 >= 2**31 or M * N == 0:
+        return None
+    if not (CHOICES.conv_split or CHOICES.conv_split_slices) and (M < CONV_SPLIT_MIN_M or K < CONV_SPLIT_MIN_K or 2 * M * N * K < CONV_SPLIT_MIN_FLOPS):
+        return None
+    #The whole tiles are dealt out in rounds of one per CU; the contraction of those of the last, incomplete round (or of all,
+    #if there are fewer tiles than CUs) may be cut into slices, of two k tiles at least. A block's start and end cost about
+    #three k tiles, a slice's partial sums five more.
+    ktiles, best = 2 * _cdiv(K, 64), None
+    for tile, (bm, bn, shared_step, lone_step) in CONV_SPLIT_TILES.items():
+        if CHOICES.conv_split not in (None, True, tile):
+            continue
+        tiles = _cdiv(M, bm) * _cdiv(N, bn)
+        for slices in range(1, 17):
+            whole = tiles if slices == 1 else tiles // compute_units * compute_units
+            if (slices > 1 and (ktiles < 2 * slices or not sliceable or whole == tiles or tiles - whole > CONV_SPLIT_MAX_SLICED)
+                    or CHOICES.conv_split_slices not in (None, slices)):
+                continue
+            blocks = whole + (tiles - whole) * slices
+            rounds = whole / compute_units if slices > 1 else _cdiv(tiles, compute_units)
+            time   = ((shared_step if blocks > compute_units else lone_step)
+                      * (rounds * (ktiles + 3) + _cdiv((tiles - whole) * slices, compute_units) * (ktiles / slices + 8)))
+            if best is None or time < best[0]:
+                best = (time, ConvSplit(tile, whole, slices))
+    return best[1] if best else None
+
+
+def conv_split_pack(packed: Buffer, source: EwOperand, g: ConvGeometry) -> Launch:
+    '''The kernel operand of a product, element (ky, kx, c, n) at source.offset + (ky, kx, c, n) . source.strides, taken
+    apart into three bf16 parts and laid out for the matrix cores.'''
+    assert packed.size == conv_split_packed_words(g)
+    params = _i32(g.N, g.K, g.Cin, g.KW, *source.strides)
+    blocks = _cdiv(g.N, 32) * _cdiv(g.K, 64)
+    return Launch('conv_split_pack', (blocks, 1, 1), (BLOCK, 1, 1), [(packed, 0), (source.buffer, source.offset * 4)], params,
+                  bytes_moved=4 * (packed.size + g.K * g.N))
+
+
+def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry, epilogue: tp.Sequence[ConvEpilogueStep] = (),
+                      lhs_offset: int = 0, out_offset: int = 0) -> Launch:
+    split, g = g.split, _flatten_pointwise(g)
+    M, N, K  = g.M, g.N, g.K
+    needs_masks, _, _, _, c_contig = _conv_fast_paths(lhs, lhs, g, lhs_offset)
+    flat_rows = g.batch == 1 and g.Wo == 1 and g.SH == 1 and g.PH == 0 and g.PW == 0 and not needs_masks
+    flags     = int(c_contig) | int(flat_rows) << 1 | int(needs_masks) << 2
+    taps = [(i, e.operand) for i, e in enumerate(epilogue) if e.op == CONV_TAP]
+    if taps:
+        (tap_position, tap_buffer), = taps
+        epilogue = [e for e in epilogue if e.op != CONV_TAP]
+        if not conv_tap_supported(epilogue[:tap_position], epilogue[tap_position:]) or out_offset or tap_buffer.size != out.size:
+            raise ValueError('a second result at this point of the epilogue is not supported')
+        flags |= (tap_position + 1) << 12
+    slots = _epilogue_template_slots(epilogue)
+    if epilogue and not slots:
+        raise ValueError('these kernels apply the straight-line epilogue only')
+    for name, extent in (('lhs', lhs.size), ('packed rhs', packed.size), ('out', out.size)):
+        if extent * 4 >= 2**31:
+            raise NotImplementedError(f'conv/dot {name} operand of {extent * 4} bytes exceeds the 2 GiB the kernel addresses')
+    kinds  = [e.kind for e in epilogue]
+    flags |= len(epilogue) << 8 | (kinds.index(3) + 1 if 3 in kinds else 0) << 16 | slots << 20
+    descs  = [0, 0]
+    for i, e in enumerate(epilogue):
+        descs[i // 3] |= ((e.op * 2 + int(e.operand_left)) | e.kind << 8) << (10 * (i % 3))
+    (tiles_m, tiles_n), kpairs = conv_split_tiles(split, g), _cdiv(K, 64)
+    shared = tiles_m * tiles_n - split.whole
+    params = (_i32(M, N, K, g.Ho, g.Wo, g.H, g.W, g.Cin, g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, *g.xs[:3], tiles_m, tiles_n)
+              + _u32(flags, *descs, (lhs.size - lhs_offset) * 4, packed.size * 4, (out.size - out_offset) * 4,
+                     *_magic_division(g.Ho * g.Wo), *_magic_division(g.Wo))
+              + _i32(g.LH, g.LW, g.xs[3], *g.ws, *g.os, split.whole, 0, split.slices, kpairs // split.slices, kpairs % split.slices))
+    derived_ptrs, derived_desc = _conv_derived(epilogue, N)
+    operand_slots = _pad([(e.operand, 0) for e in epilogue], CONV_MAX_EPI, (None, 0))
+    nbytes = 4 * (lhs.size + packed.size + out.size) + sum(4 * e.operand.size for e in epilogue if e.operand is not None)
+    if taps:
+        operand_slots[-1] = (tap_buffer, 0)
+        nbytes += 4 * tap_buffer.size
+    scratch = [(split.partial, 0), (split.arrivals, 0)] if shared else [(None, 0), (None, 0)]
+    return Launch(f'conv_gemm_split_{split.tile}', (split.whole + shared * split.slices, 1, 1), (256, 1, 1),
+                  [(out, out_offset * 4), (lhs, lhs_offset * 4), (packed, 0)] + scratch + operand_slots + derived_ptrs,
+                  params + derived_desc, bytes_moved=nbytes, flops=2 * M * N * K, written=(0, 3, 4) if shared else (0,))
+
+
+def conv_product(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: tp.Sequence[ConvEpilogueStep] = (), **offsets) -> Launch:
+    '''The launch of a product: `rhs` is its packed kernel operand where the geometry carries a plan for the bf16 matrix cores.'''
+    return (conv_split_launch if g.split is not None else conv_gemm)(out, lhs, rhs, g, epilogue, **offsets)
+
+
+def conv_split_epilogue_supported(epilogue: tp.Sequence[ConvEpilogueStep]) -> bool:
+    '''The kernels on the bf16 matrix cores apply the straight-line epilogue. A fusion pass leaves any other chain a launch of
+    its own instead of handing the product to a kernel that adds in another order than in the unfused program.'''
+    real = [e for e in epilogue if e.op != CONV_TAP]
+    return not real or _epilogue_template_slots(real) != 0
 
 
 # --------------------------------------------------------------------------- reductions

@@ -46,7 +46,7 @@ class Op:
                 self._launch = K.lower_ew_chain(self.chain)
             else:
                 out, lhs, rhs, geom, epilogue = self.conv
-                self._launch = K.conv_gemm(out, lhs, rhs, geom, epilogue)
+                self._launch = K.conv_product(out, lhs, rhs, geom, epilogue)
         return self._launch
 
     def invalidate(self):
@@ -563,6 +563,27 @@ def _wgrad_ops(bufferpool, equation, outbuf, x, cot, wg: 'K.WgradGeometry'):
     return [Op(equation, launch=l) for l in launches]
 
 
+def _split_ops(bufferpool, equation, outbuf, lhs: Buffer, rhs: Buffer, geom: 'K.ConvGeometry', rhs_offset: int = 0, out_offset: int = 0):
+    '''The launches of a product that the bf16 matrix cores compute: its kernel operand packed for them, and the product.
+    None where another kernel is to compute it.'''
+    plan = K.conv_split_plan(lhs, geom)
+    if plan is None:
+        return None
+    if plan.slices > 1:
+        plan = plan._replace(partial=bufferpool.shared_scratch(K.conv_split_partial_words(plan, geom), 'partial products'),
+                             arrivals=bufferpool.zeroed_scratch(K.CONV_SPLIT_MAX_SLICED, 'arrivals of partial products'))
+    geom     = geom._replace(split=plan)
+    position = bufferpool.op_counter
+    bufferpool.op_counter -= 1                  #the packed operand lives at the equation's own position
+    packed = bufferpool.new_temporary(np.uint32, (K.conv_split_packed_words(geom),))
+    bufferpool.op_counter = position
+    source = EwOperand(rhs, rhs_offset, tuple(geom.ws))
+    pack   = Op(equation, launch=K.conv_split_pack(packed, source, geom), meta=('conv_pack', packed, source, geom))
+    if out_offset or geom.os[1:] != (geom.Wo * geom.N, geom.N, 1) and geom.Ho * geom.Wo > 1:
+        return [pack, Op(equation, launch=K.conv_product(outbuf, lhs, packed, geom, out_offset=out_offset))]
+    return [pack, Op(equation, conv=(outbuf, lhs, packed, geom, []))]
+
+
 def _product_ops(bufferpool, equation, outbuf, lhs, rhs, geom: 'K.ConvGeometry'):
     '''The implicit-GEMM launch of a convolution or matrix product; for a product with very few output tiles and a
     long contraction, a launch that sums slices of the contraction into a temporary and an element-wise launch that
@@ -609,6 +630,9 @@ def dot_general(bufferpool, equation):
                           xs=(0, lst[1 - lc[0]], 0, lst[lc[0]]),
                           ws=(rst[rc[0]] * Kc, rst[rc[0]] * Kc, rst[rc[0]], rst[1 - rc[0]]),
                           os=(M * N, N, N, 1))
+    split = _split_ops(bufferpool, equation, outbuf, lhs, rhs, geom)
+    if split is not None:
+        return split
     ops, rhs, geom, _ = _with_dense_kernel(bufferpool, equation, rhs, geom, lhs, outbuf)
     return ops + _product_ops(bufferpool, equation, outbuf, lhs, rhs, geom)
 
@@ -650,6 +674,9 @@ def conv_general_dilated(bufferpool, equation):
         return _wgrad_ops(bufferpool, equation, outbuf, lhs, rhs, wg)
     if (geom.LH > 1 or geom.LW > 1) and geom.SH == geom.SW == 1 and geom.DH == geom.DW == 1:
         return _dilated_input_convolution(bufferpool, equation, outbuf, lhs, rhs, geom)
+    split = _split_ops(bufferpool, equation, outbuf, lhs, rhs, geom)
+    if split is not None:
+        return split
     ops, rhs, geom, _ = _with_dense_kernel(bufferpool, equation, rhs, geom, lhs, outbuf)
     return ops + _product_ops(bufferpool, equation, outbuf, lhs, rhs, geom)
 
@@ -697,6 +724,10 @@ def _dilated_input_convolution(bufferpool, equation, outbuf: Buffer, lhs: Buffer
             sub = g._replace(Ho=th, Wo=tw, KH=nh, KW=nw, PH=-ch, PW=-cw, LH=1, LW=1,
                              ws=(g.ws[0] * g.LH, g.ws[1] * g.LW, g.ws[2], g.ws[3]),
                              os=(g.os[0], g.os[1] * g.LH, g.os[2] * g.LW, g.os[3]))
+            split = _split_ops(bufferpool, equation, outbuf, lhs, rhs, sub, rh * g.ws[0] + rw * g.ws[1], ah * g.os[1] + aw * g.os[2])
+            if split is not None:
+                ops += split
+                continue
             copies, kernel, sub, kernel_offset = _with_dense_kernel(bufferpool, equation, rhs, sub, lhs, outbuf,
                                                                     rh * g.ws[0] + rw * g.ws[1])
             ops += copies
