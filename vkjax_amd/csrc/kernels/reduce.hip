@@ -500,81 +500,125 @@ SCALE_RELU_BACKWARD_KERNEL(scale_backward_v4, 4, false)
 
 // ---------------------------------------------------------------------------------------------
 // softmax over the rows of [outer, R] in one launch: out = exp(x - max(x)) / sum(exp(x - max(x))).
-// Takes the place of reduce_max -> (subtract, exp) -> reduce_sum -> divide. One wave per row; the
-// sum is accumulated in exactly the order reduce_rows uses (per-lane partial sums over the same
-// elements, combined pairwise, then the same butterfly), so the result has the same bits as the
-// four separate launches. For rows short enough to run unsplit there (the host checks R).
-struct SoftmaxParams { uint32_t outer, R; };
-
-template <int VEC, class F>
-__device__ __forceinline__ float row_sum_as_reduce_rows(F value_at, uint32_t R, uint32_t lane) {
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (VEC == 4) {
-        for (uint32_t r = lane * 4u; r < R; r += 256u)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[j] += value_at(r + j);
-    } else {
-        uint32_t r = lane;
-        for (int q = 0; r < R; r += 64u, q = (q + 1) & 3) {
-            const float v = value_at(r);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[j] += j == q ? v : 0.f;     // the sums are never -0, so adding 0 keeps them
-        }
-    }
-    float a = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) a = a + __shfl_xor(a, s, 64);
-    return a;
-}
-
+// Takes the place of reduce_max -> (subtract, exp) -> reduce_sum -> divide. The sum is accumulated in exactly the
+// order reduce_rows uses (per-lane partial sums over the same elements, combined pairwise, then the same butterfly),
+// so the result has the same bits as the four separate launches. For rows short enough to run unsplit there (the
+// host checks R).
+// A row is read once, all its loads in flight together, and stays in the wave's registers: NV vectors of VEC values
+// per lane (the host takes the smallest variant that holds the row), one exp per value. Rows of one vector per lane
+// take 2^lanes_log2 lanes each, the fewest that hold them, and a wave does several; the lanes that such a row would
+// leave idle only add zeros to its sum, so its bits do not depend on how many there are.
+// What bounds it: memory. 65536 rows of 1000 with labels: 79 us, 6.6 TB/s (one wave per row that read it three
+// times, two exps per value: 205 us). Replays of 65536 rows of 10 with one row per wave 35 us, with several 20 us; 20000
+// of 1001 76 -> 43 us, 16384 of 4092 223 -> 103 us.
 // `arg_out` (may be null): the index of each result row's largest value as reduce_rows_fargmax would report it
 // (first occurrence, a NaN wins), for programs that take the arg-max of the probabilities right away.
-template <int VEC>
+struct SoftmaxParams { uint32_t outer, R, lanes_log2; };
+
+template <int VEC, int NV>
 __device__ __forceinline__ void softmax_rows_body(float* __restrict__ out, const float* __restrict__ in, uint32_t* __restrict__ arg_out,
                                                   const SoftmaxParams& P) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
-    if (row >= P.outer) return;                                       // whole wave leaves together
-    const float* x = in + (uint64_t)row * P.R;
-    float* y = out + (uint64_t)row * P.R;
-    float m = -INFINITY;                                              // the maximum does not depend on the order; a NaN wins
-    for (uint32_t r = lane; r < P.R; r += 64u) { const float v = x[r]; m = (v > m || v != v) ? v : m; }
+    const uint32_t lane = threadIdx.x & 63u, outer = without_stream_bit(P.outer);
+    const uint32_t log2_lanes = NV == 1 ? P.lanes_log2 : 6u, lanes = 1u << log2_lanes, rows = 64u >> log2_lanes;
+    const uint32_t first = (blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * rows;
+    if (first >= outer) return;                                       // whole wave leaves together
+    const uint32_t sub = lane >> log2_lanes, l = lane & (lanes - 1u);
+    const uint32_t bytes = min(rows, outer - first) * P.R * 4u;       // rows beyond the last one lie outside the descriptors
+    const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(in + (uint64_t)first * P.R, bytes), y_rsrc = make_rsrc(out + (uint64_t)first * P.R, bytes);
+    uint32_t at[NV];                                                  // byte offset of a lane's vector i, none beyond the row
 #pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) { const float o = __shfl_xor(m, s, 64); m = (m > o || m != m) ? m : o; }
-    const float total = row_sum_as_reduce_rows<VEC>([&](uint32_t r) { return expf(x[r] - m); }, P.R, lane);
-    uint32_t best_v = 0, best_i = 0xFFFFFFFFu;
-    for (uint32_t r = lane; r < P.R; r += 64u) {
-        const float p = expf(x[r] - m) / total;
-        y[r] = p;
-        // a lane meets its elements in ascending order: on a tie the earlier one stays; a NaN replaces any number
-        const float q = u2f(best_v);
-        const bool better = p > q || (p != p && q == q) || best_i == 0xFFFFFFFFu;
-        best_v = better ? f2u(p) : best_v;
-        best_i = better ? r : best_i;
+    for (int i = 0; i < NV; ++i) {
+        const uint32_t r = (l + i * lanes) * VEC;
+        at[i] = r < P.R ? (sub * P.R + r) * 4u : 0x80000000u;
+    }
+    float v[NV][VEC];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        if constexpr (VEC == 4) {
+            const f32x4 t = buffer_load_x4(x_rsrc, at[i]);
+            v[i][0] = t.x; v[i][1] = t.y; v[i][2] = t.z; v[i][3] = t.w;
+        } else {
+            v[i][0] = buffer_load_x1(x_rsrc, at[i]);
+        }
+    }
+    float m = -INFINITY;                                              // the maximum does not depend on the order; a NaN wins
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) m = at[i] != 0x80000000u && (v[i][j] > m || v[i][j] != v[i][j]) ? v[i][j] : m;
+    for (uint32_t s = lanes >> 1; s >= 1; s >>= 1) { const float o = __shfl_xor(m, s, 64); m = (m > o || m != m) ? m : o; }
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+            v[i][j] = at[i] != 0x80000000u ? expf(v[i][j] - m) : 0.f;
+            acc[VEC == 4 ? j : i & 3] += v[i][j];                     // the sums are never -0, so adding 0 keeps them
+        }
+    float total = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    for (uint32_t s = lanes >> 1; s >= 1; s >>= 1) total = total + __shfl_xor(total, s, 64);
+    const bool stream = streams_result(P.outer);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) v[i][j] = v[i][j] / total;
+        if constexpr (VEC == 4) {
+            const u32x4 t = u32x4{f2u(v[i][0]), f2u(v[i][1]), f2u(v[i][2]), f2u(v[i][3])};
+            if (stream) __builtin_amdgcn_raw_buffer_store_b128(t, y_rsrc, at[i], 0, 2);
+            else __builtin_amdgcn_raw_buffer_store_b128(t, y_rsrc, at[i], 0, 0);
+        } else {
+            if (stream) __builtin_amdgcn_raw_buffer_store_b32(f2u(v[i][0]), y_rsrc, at[i], 0, 2);
+            else __builtin_amdgcn_raw_buffer_store_b32(f2u(v[i][0]), y_rsrc, at[i], 0, 0);
+        }
     }
     if (arg_out == nullptr) return;
+    uint32_t best_v = 0, best_i = 0xFFFFFFFFu;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+            // a lane meets its elements in ascending order: on a tie the earlier one stays; a NaN replaces any number
+            const float p = v[i][j], q = u2f(best_v);
+            const bool better = at[i] != 0x80000000u && (p > q || (p != p && q == q) || best_i == 0xFFFFFFFFu);
+            best_v = better ? f2u(p) : best_v;
+            best_i = better ? (l + i * lanes) * VEC + j : best_i;
+        }
     // across the lanes as in reduce_rows: the maximum of (rank of the value, complement of the index)
     const uint32_t zb      = best_v == 0x80000000u ? 0u : best_v;      // -0.0 ranks with +0.0
     const uint32_t flipped = zb ^ ((zb >> 31) ? 0xFFFFFFFFu : 0x80000000u);
     const float    bv      = u2f(best_v);
     uint64_t key = best_i == 0xFFFFFFFFu ? 0ull : ((uint64_t)(bv != bv ? 0xFFFFFFFFu : flipped) << 32 | (uint32_t)~best_i);
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) {
+    for (uint32_t s = lanes >> 1; s >= 1; s >>= 1) {
         const uint64_t other = __shfl_xor(key, s, 64);
         key = other > key ? other : key;
     }
-    if (lane == 0) arg_out[row] = key == 0ull ? 0u : ~(uint32_t)key;
+    if (l == 0 && first + sub < outer) arg_out[first + sub] = key == 0ull ? 0u : ~(uint32_t)key;
 }
 
-extern "C" __global__ __launch_bounds__(256) void softmax_rows_v1(float* __restrict__ out, const float* __restrict__ in, uint32_t* __restrict__ arg_out,
-                                                                  SoftmaxParams P) {
-    softmax_rows_body<1>(out, in, arg_out, P);
-}
-// R % 4 == 0: the summation order of the 16-byte reduce_rows kernel
-extern "C" __global__ __launch_bounds__(256) void softmax_rows_v4(float* __restrict__ out, const float* __restrict__ in, uint32_t* __restrict__ arg_out,
-                                                                  SoftmaxParams P) {
-    softmax_rows_body<4>(out, in, arg_out, P);
-}
+#define SOFTMAX_ROWS(name, VEC, NV)                                                                                         \
+    extern "C" __global__ __launch_bounds__(256) void name(                                                                 \
+        float* __restrict__ out, const float* __restrict__ in, uint32_t* __restrict__ arg_out, SoftmaxParams P) {           \
+        softmax_rows_body<VEC, NV>(out, in, arg_out, P);                                                                    \
+    }
+// _v4: R % 4 == 0, the summation order of the 16-byte reduce_rows kernel. _n<NV>: rows of more than 64 vectors
+SOFTMAX_ROWS(softmax_rows_v4, 4, 1)
+SOFTMAX_ROWS(softmax_rows_v4_n2, 4, 2)
+SOFTMAX_ROWS(softmax_rows_v4_n3, 4, 3)
+SOFTMAX_ROWS(softmax_rows_v4_n4, 4, 4)
+SOFTMAX_ROWS(softmax_rows_v4_n6, 4, 6)
+SOFTMAX_ROWS(softmax_rows_v4_n8, 4, 8)
+SOFTMAX_ROWS(softmax_rows_v4_n12, 4, 12)
+SOFTMAX_ROWS(softmax_rows_v4_n16, 4, 16)
+SOFTMAX_ROWS(softmax_rows_v1, 1, 1)
+SOFTMAX_ROWS(softmax_rows_v1_n2, 1, 2)
+SOFTMAX_ROWS(softmax_rows_v1_n4, 1, 4)
+SOFTMAX_ROWS(softmax_rows_v1_n8, 1, 8)
+SOFTMAX_ROWS(softmax_rows_v1_n12, 1, 12)
+SOFTMAX_ROWS(softmax_rows_v1_n16, 1, 16)
+SOFTMAX_ROWS(softmax_rows_v1_n24, 1, 24)
+SOFTMAX_ROWS(softmax_rows_v1_n32, 1, 32)
+SOFTMAX_ROWS(softmax_rows_v1_n48, 1, 48)
+SOFTMAX_ROWS(softmax_rows_v1_n64, 1, 64)
 
 struct ReduceGeneralParams {
     uint32_t n_out, n_red, op, type;

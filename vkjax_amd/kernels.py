@@ -1233,15 +1233,22 @@ def scale_relu_backward(column_sum: Launch, dx: Buffer, sum_m: Buffer, sum_mx: B
 
 
 SOFTMAX_MAX_ROW = 4096      #rows this short run unsplit in reduce_rows, whose summation order softmax_rows repeats
+#vectors per lane of the kernels' variants: a row stays in the registers of one wave
+SOFTMAX_VECTORS = {4: (1, 2, 3, 4, 6, 8, 12, 16), 1: (1, 2, 4, 8, 12, 16, 24, 32, 48, 64)}
 
 
 def softmax_rows(out: Buffer, inp: Buffer, outer: int, R: int, arg_out: tp.Optional[Buffer] = None) -> Launch:
     '''exp(x - max) / sum(exp(x - max)) over the rows of [outer, R]; see softmax_rows_body in reduce.hip.
     `arg_out`: also the arg-max of every result row (int32 [outer]).'''
     assert 0 < R < SOFTMAX_MAX_ROW and inp.size == out.size == outer * R and (arg_out is None or arg_out.size == outer)
-    vec = 4 if R % 4 == 0 else 1
-    return Launch(f'softmax_rows_v{vec}', (_cdiv(outer, 4), 1, 1), (BLOCK, 1, 1), [(out, 0), (inp, 0), (arg_out, 0)], _u32(outer, R),
-                  bytes_moved=8 * outer * R + (4 * outer if arg_out is not None else 0), written=(0, 2))
+    vec     = 4 if R % 4 == 0 else 1
+    vectors = next(n for n in SOFTMAX_VECTORS[vec] if n * 64 * vec >= R)
+    #short rows share a wave: as few lanes each as hold them
+    lanes   = _pow2_at_least(R // vec) if vectors == 1 else 64
+    kernel  = f'softmax_rows_v{vec}' + (f'_n{vectors}' if vectors > 1 else '')
+    return Launch(kernel, (_cdiv(outer, 4 * (64 // lanes)), 1, 1), (BLOCK, 1, 1), [(out, 0), (inp, 0), (arg_out, 0)],
+                  _u32(outer, R, lanes.bit_length() - 1), bytes_moved=8 * outer * R + (4 * outer if arg_out is not None else 0),
+                  streamable=True, written=(0, 2))
 
 
 def reduce_general(out: Buffer, inp: Buffer, kept, reduced, op: str) -> Launch:
