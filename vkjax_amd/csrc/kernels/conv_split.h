@@ -13,20 +13,8 @@
 // Measured against 64-bit sums (4096 x K x 128, normal data): an error of 0.88, 0.63 and 0.39 times that of
 // v_mfma_f32_32x32x2_f32 at K = 64, 576 and 2304 (which rounds after every second product, this after every sixteenth).
 #pragma once
+#include "split_bf16.h"
 
-typedef __bf16   bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16   bf16x2 __attribute__((ext_vector_type(2)));
-typedef float    f32x2  __attribute__((ext_vector_type(2)));
-
-// the two numbers' nearest bf16, the first in the low half
-__device__ __forceinline__ uint32_t to_bf16x2(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
-}
-// Consecutive workgroup ids go to the 8 XCDs in turn: renumbers [0, n) so that every XCD works through a contiguous range.
-__device__ __forceinline__ int xcd_range(int id, int n) {
-    const int per = n / 8;
-    return per > 0 && id < per * 8 ? (id & 7) * per + (id >> 3) : id;
-}
 // stores and loads that are seen by every workgroup of the GPU, whichever L2 it stands behind (agent scope)
 __device__ __forceinline__ void buffer_store_x4_agent(f32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, soff, 16);
@@ -410,8 +398,6 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                     }
     }
 
-    // An operand that is infinite, not a number, or beyond the largest bf16 leaves a sum that is not finite (infinity
-    // times the zero parts of the other operand): such sub-tiles are computed again with fp32 products.
     // An operand that is infinite, not a number, or beyond the largest bf16 leaves a sum that is not finite (infinity
     // times the zero parts of the other operand): such sub-tiles are computed again with fp32 products.
     {

@@ -26,6 +26,10 @@ struct WgradParams {
     uint32_t howo_magic, howo_shift, wo_magic, wo_shift, c_magic, c_shift, kw_magic, kw_shift;
     uint32_t x_bytes, g_bytes;
 };
+struct WgradSplitParams {
+    int32_t tiles_m, tiles_n;          // tiles of the result; every slice of the contraction has as many blocks
+    int32_t flat;                      // pixel p's features start at p * C: no taps, no strides
+};
 
 template <bool VEC_A, bool VEC_B>
 __device__ __forceinline__ void wgrad_body(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ g,
@@ -135,3 +139,5 @@ WGRAD_KERNEL(wgrad_gemm_64x64_aa, true, true)
 WGRAD_KERNEL(wgrad_gemm_64x64_as, true, false)
 WGRAD_KERNEL(wgrad_gemm_64x64_sa, false, true)
 WGRAD_KERNEL(wgrad_gemm_64x64_ss, false, false)
+
+#include "wgrad_split.h"

@@ -50,6 +50,8 @@ class _Choices:
         conv_stem=None,                  #the patch kernel for few input features: False = never; None / True: where it applies; 64: its 64-position tiles only
         conv_split=None,                 #the kernels on the bf16 matrix cores: None = where they pay, False = never, True or a tile's name = wherever they apply
         conv_split_slices=None,          #blocks that share a tile behind the whole rounds (None: by the estimate)
+        wgrad_split=None,                #kernel gradients on the bf16 matrix cores: None = where they pay, False = never, a tile's name = wherever it applies
+        wgrad_slices=None,               #slices of a kernel gradient's contraction (None: by the estimate)
         conv_k_splits=None,              #slices a contraction is cut into where that applies (None: by the heuristic, 1: never)
         conv_xcd_columns=0,              #four-waves-per-tile kernels: XCD columns over the tile grid (0: row-major ranges, None: least traffic)
         scatter_sort_threshold=1 << 18,  #update elements from which a row scatter-add sorts its updates instead of using atomics
@@ -512,8 +514,69 @@ def choose_wgrad_splits(g: WgradGeometry, compute_units: int = 256) -> int:
     return max(1, min(want, g.pixels // 128, 1024))
 
 
-def wgrad_gemm(out: Buffer, x: Buffer, cot: Buffer, g: WgradGeometry, splits: int) -> Launch:
-    '''`out` holds `splits` partial results of M * N elements each (the result itself when splits == 1).'''
+#Tiles of the kernel gradients on the bf16 matrix cores (csrc/kernels/wgrad_split.h): (BM, BN, blocks a CU holds, microseconds of such
+#a CU per block and k tile of 32 pixels, measured on ResNet-50's layers at batch 64, loads of X it is built for: 16 bytes / words)
+WGRAD_SPLIT_TILES = {'128x128': (128, 128, 2, 1.55, 'a'), '128x64': (128, 64, 3, 0.95, 'a'), '64x128': (64, 128, 3, 0.95, 'a'), '64x64': (64, 64, 4, 0.57, 'as')}
+#Below this many operations the fp32 kernels are as fast: 2000 x 1024 x 512 (2.1 GFLOP) takes 28 us there and 22 here, 1000 x 784 x 300
+#(0.5) 12.6 and 12.8, 3x3 on 4 x 14 x 14 x 256 (0.9) 18.4 and 18.8.
+WGRAD_SPLIT_MIN_FLOPS = 1.5e9
+WGRAD_SPLIT_MAX_SLICES = 1024
+
+
+class WgradPlan(tp.NamedTuple):
+    '''The tile of the kernel on the bf16 matrix cores, or None for the one on fp32 products; slices of the contraction.'''
+    tile:   tp.Optional[str]
+    splits: int
+
+
+def _wgrad_loads(g: WgradGeometry) -> str:
+    return ('a' if g.C % 4 == 0 else 's') + ('a' if g.N % 4 == 0 else 's')
+
+
+def wgrad_split_applies(tile: str, g: WgradGeometry) -> bool:
+    '''The kernels are built for G in 16-byte loads; a pixel's (y, x) and a tap's offset are added as 16-bit numbers, which
+    the bounds keep from running over.'''
+    if g.N % 4 != 0 or _wgrad_loads(g)[0] not in WGRAD_SPLIT_TILES[tile][4]:
+        return False
+    tap = lambda k, d, p: max(abs(p), abs((k - 1) * d - p))
+    return _wgrad_flat(g) or (max(g.H, g.W) <= 0x2000 and max(tap(g.KH, g.DH, g.PH), tap(g.KW, g.DW, g.PW)) < 0x1000
+                              and max((g.Ho - 1) * g.SH, (g.Wo - 1) * g.SW) < 0x3000)
+
+
+def wgrad_plan(g: WgradGeometry, compute_units: int = 256) -> WgradPlan:
+    '''The tile and the number of slices with the smallest estimated time: the k tiles of the CU with the most blocks (one alone on a
+    CU takes 1.3 times as long as one of as many as it holds), four microseconds to start and store, and the partial results written and added.'''
+    fp32 = WgradPlan(None, choose_wgrad_splits(g, compute_units))
+    if (CHOICES.wgrad_split is False or (CHOICES.wgrad_split is None and 2 * g.pixels * g.M * g.N < WGRAD_SPLIT_MIN_FLOPS)):
+        return fp32
+    ktiles, best = _cdiv(g.pixels, 32), None
+    for tile, (bm, bn, resident, step, _) in WGRAD_SPLIT_TILES.items():
+        if CHOICES.wgrad_split not in (None, tile) or not wgrad_split_applies(tile, g):
+            continue
+        tiles = _cdiv(g.M, bm) * _cdiv(g.N, bn)
+        if CHOICES.wgrad_slices is not None:
+            counts = {min(ktiles, CHOICES.wgrad_slices)}
+        else:                                         #those that fill a number of rounds of one block per CU
+            counts = {max(1, min(r * compute_units // tiles, ktiles // 4, WGRAD_SPLIT_MAX_SLICES)) for r in range(1, 9)}
+        for splits in sorted(counts):
+            per    = _cdiv(ktiles, splits)
+            splits = _cdiv(ktiles, per)
+            each   = _cdiv(tiles * splits, compute_units)
+            alone  = 0.3 * max(0, resident - each) / (resident - 1)
+            time   = each * per * step * (1 + alone) + 4 + (3 + splits * g.M * g.N * 8 / 8e6 if splits > 1 else 0)
+            if best is None or time < best[0]:
+                best = (time, WgradPlan(tile, splits))
+    return best[1] if best else fp32
+
+
+def _wgrad_flat(g: WgradGeometry) -> bool:
+    '''Pixel p's features start at p * C: a product of matrices, or a 1 x 1 window at a stride of 1 without padding.'''
+    return g.KH == g.KW == g.SH == g.SW == 1 and g.PH == g.PW == 0 and (g.H, g.W) == (g.Ho, g.Wo)
+
+
+def wgrad_gemm(out: Buffer, x: Buffer, cot: Buffer, g: WgradGeometry, splits: int, tile: tp.Optional[str] = None) -> Launch:
+    '''`out` holds `splits` partial results of M * N elements each (the result itself when splits == 1). `tile`: one of
+    WGRAD_SPLIT_TILES, for the kernel on the bf16 matrix cores.'''
     for name, b in (('input', x), ('cotangent', cot)):
         if b.size * 4 >= 2**31:
             raise NotImplementedError(f'kernel gradient: {name} of {b.size * 4} bytes exceeds the 2 GiB the kernel addresses')
@@ -523,9 +586,14 @@ def wgrad_gemm(out: Buffer, x: Buffer, cot: Buffer, g: WgradGeometry, splits: in
     magics = [v for d in (g.Ho * g.Wo, g.Wo, g.C, g.KW) for v in _magic_division(d)]
     params = _i32(g.pixels, g.M, g.N, g.Ho, g.Wo, g.H, g.W, g.C, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, per_split) \
            + _u32(*magics, x.size * 4, cot.size * 4)
-    kernel = 'wgrad_gemm_64x64_' + ('a' if g.C % 4 == 0 else 's') + ('a' if g.N % 4 == 0 else 's')
-    return Launch(kernel, (_cdiv(g.N, 64), _cdiv(g.M, 64), splits), (256, 1, 1), [(out, 0), (x, 0), (cot, 0)], params,
-                  bytes_moved=4 * (x.size + cot.size + out.size), flops=2 * g.pixels * g.M * g.N)
+    loads = _wgrad_loads(g)
+    work  = dict(bytes_moved=4 * (x.size + cot.size + out.size), flops=2 * g.pixels * g.M * g.N)
+    if tile is not None:
+        bm, bn = WGRAD_SPLIT_TILES[tile][:2]
+        tiles_m, tiles_n = _cdiv(g.M, bm), _cdiv(g.N, bn)
+        return Launch(f'wgrad_split_{tile}_{loads}', (tiles_m * tiles_n * splits, 1, 1), (256, 1, 1), [(out, 0), (x, 0), (cot, 0)],
+                      params + _i32(tiles_m, tiles_n, _wgrad_flat(g)), **work)
+    return Launch(f'wgrad_gemm_64x64_{loads}', (_cdiv(g.N, 64), _cdiv(g.M, 64), splits), (256, 1, 1), [(out, 0), (x, 0), (cot, 0)], params, **work)
 
 
 class ConvDerivedOperand(tp.NamedTuple):

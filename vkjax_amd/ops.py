@@ -552,14 +552,14 @@ WGRAD_MIN_PIXELS = 128
 
 def _wgrad_ops(bufferpool, equation, outbuf, x, cot, wg: 'K.WgradGeometry'):
     '''X^T G over the pixels, split over the contraction; the slices are added by a column reduction.'''
-    splits = K.choose_wgrad_splits(wg)
+    tile, splits = K.wgrad_plan(wg)
     if splits == 1:
-        return [Op(equation, launch=K.wgrad_gemm(outbuf, x, cot, wg, 1))]
+        return [Op(equation, launch=K.wgrad_gemm(outbuf, x, cot, wg, 1, tile))]
     position = bufferpool.op_counter
     bufferpool.op_counter -= 1                  #the temporary lives at the equation's own position
     partial = bufferpool.new_temporary(np.float32, (splits, wg.M * wg.N))
     bufferpool.op_counter = position
-    launches = [K.wgrad_gemm(partial, x, cot, wg, splits)] + K.reduce(outbuf, partial, 1, splits, wg.M * wg.N, 'reduce_sum')
+    launches = [K.wgrad_gemm(partial, x, cot, wg, splits, tile)] + K.reduce(outbuf, partial, 1, splits, wg.M * wg.N, 'reduce_sum')
     return [Op(equation, launch=l) for l in launches]
 
 
