@@ -229,7 +229,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         f32x4& v = x[q >> 1];
         const int e = 2 * (q & 1);
         const uint32_t w2 = to_bf16x2(v[e], v[e + 1]);
-        if (t < 2) { v[e] = v[e] - u2f(w2 << 16); v[e + 1] = v[e + 1] - u2f(w2 & 0xFFFF0000u); }
+        if (t < 2) { v[e] = minus_low(w2, v[e]); v[e + 1] = minus_high(w2, v[e + 1]); }
         return w2;
     };
     u32x4 part;
