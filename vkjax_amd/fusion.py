@@ -40,6 +40,7 @@ def _reads(op) -> tp.List:
         out, lhs, rhs, geom, epilogue = op.conv
         reads = [lhs, rhs] + [e.operand for e in epilogue if e.operand is not None and e.op not in (K.CONV_TAP, K.CONV_SOFTMAX)]
         for e in epilogue:
+            reads += e.bounds
             if e.derived is not None:
                 reads += [e.derived.first] + [st[1] for st in e.derived.steps if st[1] is not None]
         return reads
@@ -319,6 +320,7 @@ def fuse_ops(all_ops, bufferpool, outvars):
     ops = fuse_reduce_prologues(ops, bufferpool, outvars)
     ops = fuse_reduce_scales(ops, bufferpool, outvars)
     ops = fuse_derived_epilogue_operands(ops, bufferpool, outvars)
+    ops = fuse_relu_backward_epilogues(ops, bufferpool, outvars)
     ops = fuse_index_wrap(ops, bufferpool, outvars)
     ops = fold_index_wrap(ops, bufferpool, outvars)
     ops = fuse_dense_softmax(ops, bufferpool, outvars)
@@ -697,6 +699,83 @@ def fuse_scale_relu_backward(ops, bufferpool, outvars):
         removed |= set(involved) - {position}
         replacement[position] = fused
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
+
+
+def fuse_relu_backward_epilogues(ops, bufferpool, outvars):
+    '''The backward pass of a ReLU behind a product on the bf16 matrix cores (the gradient of a layer's input, to which another
+    branch's may have been added) and the scaling in front of that ReLU,
+
+        d = product (+ r) ; m = select(ans > t, d, z) ; dx = m * k
+
+    with d read by nothing else, become the product's epilogue. Where m is read elsewhere too it is the launch's second result.
+    The arithmetic and its order are unchanged. The merged launch stands where the select stood.'''
+    from .ops import Op
+    uses   = _use_counts(ops, bufferpool, outvars)
+    pid    = lambda b: id(b._placeholder)
+    single = lambda o: o is not None and o.buffer.size == 1 and o.offset == 0 and o.buffer.dtype == 'float32'
+    ops    = list(ops)
+    maker  = {pid(op.conv[0]): i for i, op in enumerate(ops) if op.conv is not None and op.conv[3].split is not None}
+    last_writer: tp.Dict[int, int] = {}
+    readers: tp.Dict[int, tp.List[int]] = {}
+    for i, op in enumerate(ops):
+        plain = op.chain is None and op.conv is None and op.meta is None
+        for b in ([op.launch.buffers[k][0] for k in op.launch.written] if plain else _may_write(op)):
+            if b is not None:
+                last_writer[pid(b)] = i
+        for b in _reads(op):
+            readers.setdefault(pid(b), []).append(i)
+
+    def scaling(chain, shape, geom):
+        '''(scaled buffer, epilogue step) of a chain that only multiplies by a value per feature.'''
+        if chain is None or [st.op for st in chain.steps] != [EW['MUL_F']] or tuple(chain.shape) != tuple(shape) or chain.steps[0].operand is None:
+            return None
+        for a, b in ((chain.first, chain.steps[0].operand), (chain.steps[0].operand, chain.first)):
+            step = _epilogue_steps([EwStep(EW['MUL_F'], b)], geom, shape)
+            if _is_full_contiguous(a, shape) and step is not None and step[0].kind == 2:
+                return a.buffer, step[0]
+        return None
+
+    for i, op in enumerate(ops):
+        ch = op.chain if op is not None else None
+        if (ch is None or [st.op for st in ch.steps[:3]] != [EW['GT_F'], EW['SEL_P'], EW['NOP']] or ch.steps[0].operand_left or len(ch.steps) > 4
+                or not single(ch.steps[0].operand) or not single(ch.steps[2].operand) or ch.out.dtype != 'float32' or ch.first.buffer.dtype != 'float32'
+                or not _is_full_contiguous(ch.first, ch.shape) or not _is_full_contiguous(ch.steps[1].operand, ch.shape)):
+            continue
+        d, activation = ch.steps[1].operand.buffer, ch.first.buffer
+        at = maker.get(pid(d))
+        if at is None or at >= i or uses[pid(d)] != 1 or ops[at] is None or pid(activation) == pid(d):
+            continue
+        out, lhs, rhs, geom, epilogue = ops[at].conv
+        if tuple(out.shape) != tuple(ch.shape) or ch.out.size != out.size or activation.size != out.size:
+            continue
+        #what the product reads still has to be there where the select stood
+        if any(last_writer.get(pid(b), -1) > at and pid(b) != pid(d) for b in _reads(ops[at])):
+            continue
+        steps = list(epilogue) + [K.ConvEpilogueStep(K.CONV_MASK, 3, activation, bounds=(ch.steps[0].operand.buffer, ch.steps[2].operand.buffer))]
+        result, involved = ch.out, [at, i]
+        if len(ch.steps) == 4:
+            vector = _epilogue_steps(ch.steps[3:], geom, ch.shape)
+            if vector is None:
+                continue
+            steps += vector
+        else:
+            for r in sorted(readers.get(pid(ch.out), [])):
+                scaled = scaling(ops[r].chain, ch.shape, geom) if r > i and ops[r] is not None else None
+                if scaled is not None and pid(scaled[0]) == pid(ch.out) and last_writer.get(pid(scaled[1].operand), -1) < i:
+                    steps += [K.ConvEpilogueStep(K.CONV_TAP, 3, ch.out), scaled[1]]
+                    result, involved = ops[r].chain.out, [at, i, r]
+                    break
+        if K.conv_masked_epilogue(steps) is None:
+            continue
+        fused = Op(_label(*[ops[j] for j in involved]), conv=(result, lhs, rhs, geom, steps))
+        fused.index = op.index
+        for b in _reads(fused) + _writes(fused):
+            b.accesses.append(fused.index)
+        d._placeholder.elided = True
+        for j in involved:
+            ops[j] = None
+        ops[i] = fused
+    return [op for op in ops if op is not None]
 
 
 def _is_full_contiguous_any_shape(operand: EwOperand, shape) -> bool:

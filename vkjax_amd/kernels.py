@@ -609,6 +609,7 @@ class ConvEpilogueStep(tp.NamedTuple):
     operand:      tp.Optional[Buffer]    #None when `derived` says how to compute it
     operand_left: bool = False
     derived:      tp.Optional[ConvDerivedOperand] = None
+    bounds:       tp.Tuple[Buffer, ...] = ()
 
 
 #A pseudo step: the value as it stands at this point of the epilogue is ALSO stored to `operand`, an array laid
@@ -618,6 +619,11 @@ CONV_TAP = -1
 #`operand`, if not None, is an int32 array [M] that receives each row's arg-max. Only the kernel for products with at
 #most 16 output features (dense_rows_n16) can do this.
 CONV_SOFTMAX = -2
+
+
+#A pseudo step: the value is kept where `operand` (an activation laid out like the result) lies above the first of `bounds` and
+#replaced by the second elsewhere (arrays of one float32 each): the backward pass of a ReLU
+CONV_MASK = -3
 
 
 def conv_tap_supported(steps_before: tp.Sequence[ConvEpilogueStep], steps_after: tp.Sequence[ConvEpilogueStep]) -> bool:
@@ -1147,23 +1153,30 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
     flat_rows = g.batch == 1 and g.Wo == 1 and g.SH == 1 and g.PH == 0 and g.PW == 0 and not needs_masks
     flags     = int(c_contig) | int(flat_rows) << 1 | int(needs_masks) << 2
     taps = [(i, e.operand) for i, e in enumerate(epilogue) if e.op == CONV_TAP]
-    if taps:
+    masked = any(e.op == CONV_MASK for e in epilogue)
+    if masked:
+        operands = conv_masked_epilogue(epilogue)
+        if operands is None or out_offset or any(e.operand.size != out.size for e in epilogue if e.kind == 3):
+            raise ValueError('an epilogue with a mask is: + full tensor, mask, second result, * vector')
+        flags   |= 1 << 25 | len(taps) << 12
+        epilogue = [e or ConvEpilogueStep(EW['NOP'], 0, None) for e in operands]
+    elif taps:
         (tap_position, tap_buffer), = taps
         epilogue = [e for e in epilogue if e.op != CONV_TAP]
         if not conv_tap_supported(epilogue[:tap_position], epilogue[tap_position:]) or out_offset or tap_buffer.size != out.size:
             raise ValueError('a second result at this point of the epilogue is not supported')
         flags |= (tap_position + 1) << 12
-    slots = _epilogue_template_slots(epilogue)
-    if epilogue and not slots:
+    slots = (8 if epilogue[0].operand is not None else 0) | (2 if epilogue[2].operand is not None else 0) if masked else _epilogue_template_slots(epilogue)
+    if epilogue and not slots and not masked:
         raise ValueError('these kernels apply the straight-line epilogue only')
     for name, extent in (('lhs', lhs.size), ('packed rhs', packed.size), ('out', out.size)):
         if extent * 4 >= 2**31:
             raise NotImplementedError(f'conv/dot {name} operand of {extent * 4} bytes exceeds the 2 GiB the kernel addresses')
     kinds  = [e.kind for e in epilogue]
-    flags |= len(epilogue) << 8 | (kinds.index(3) + 1 if 3 in kinds else 0) << 16 | slots << 20
+    flags |= len(epilogue) << 8 | ((int(bool(slots & 8)) if masked else kinds.index(3) + 1) if 3 in kinds else 0) << 16 | slots << 20
     descs  = [0, 0]
     for i, e in enumerate(epilogue):
-        descs[i // 3] |= ((e.op * 2 + int(e.operand_left)) | e.kind << 8) << (10 * (i % 3))
+        descs[i // 3] |= ((0 if masked else e.op * 2 + int(e.operand_left)) | e.kind << 8) << (10 * (i % 3))
     (tiles_m, tiles_n), kpairs = conv_split_tiles(split, g), _cdiv(K, 64)
     shared = tiles_m * tiles_n - split.whole
     params = (_i32(M, N, K, g.Ho, g.Wo, g.H, g.W, g.Cin, g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, *g.xs[:3], tiles_m, tiles_n)
@@ -1174,8 +1187,8 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
     operand_slots = _pad([(e.operand, 0) for e in epilogue], CONV_MAX_EPI, (None, 0))
     nbytes = 4 * (lhs.size + packed.size + out.size) + sum(4 * e.operand.size for e in epilogue if e.operand is not None)
     if taps:
-        operand_slots[-1] = (tap_buffer, 0)
-        nbytes += 4 * tap_buffer.size
+        operand_slots[-1] = (taps[0][1], 0)
+        nbytes += 4 * taps[0][1].size
     scratch = [(split.partial, 0), (split.arrivals, 0)] if shared else [(None, 0), (None, 0)]
     return Launch(f'conv_gemm_split_{split.tile}', (split.whole + shared * split.slices, 1, 1), (256, 1, 1),
                   [(out, out_offset * 4), (lhs, lhs_offset * 4), (packed, 0)] + scratch + operand_slots + derived_ptrs,
@@ -1185,6 +1198,20 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
 def conv_product(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: tp.Sequence[ConvEpilogueStep] = (), **offsets) -> Launch:
     '''The launch of a product: `rhs` is its packed kernel operand where the geometry carries a plan for the bf16 matrix cores.'''
     return (conv_split_launch if g.split is not None else conv_gemm)(out, lhs, rhs, g, epilogue, **offsets)
+
+
+def conv_masked_epilogue(epilogue: tp.Sequence[ConvEpilogueStep]) -> tp.Optional[tp.List[tp.Optional[ConvEpilogueStep]]]:
+    '''The operands of an epilogue with a mask by their places in the kernel's arguments (full tensor, activation, vector, limit,
+    constant; the second result has the last place), or None for one the kernel does not apply.'''
+    rest = list(epilogue)
+    take = lambda op, kind: rest.pop(0) if rest and rest[0].op == op and rest[0].kind == kind and rest[0].derived is None else None
+    full, mask = take(EW['ADD_F'], 3), take(CONV_MASK, 3)
+    take(CONV_TAP, 3)
+    vector = take(EW['MUL_F'], 2)
+    if mask is None or rest:
+        return None
+    limit, otherwise = (ConvEpilogueStep(EW['NOP'], 1, b) for b in mask.bounds)
+    return [full, mask, vector, limit, otherwise]
 
 
 def conv_split_epilogue_supported(epilogue: tp.Sequence[ConvEpilogueStep]) -> bool:
