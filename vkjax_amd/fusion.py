@@ -710,6 +710,8 @@ def fuse_relu_backward_epilogues(ops, bufferpool, outvars):
     with d read by nothing else, become the product's epilogue. Where m is read elsewhere too it is the launch's second result.
     The arithmetic and its order are unchanged. The merged launch stands where the select stood.'''
     from .ops import Op
+    if not any(op.conv is not None and op.conv[3].split is not None for op in ops):
+        return ops
     uses   = _use_counts(ops, bufferpool, outvars)
     pid    = lambda b: id(b._placeholder)
     single = lambda o: o is not None and o.buffer.size == 1 and o.offset == 0 and o.buffer.dtype == 'float32'
@@ -1106,6 +1108,8 @@ def batch_packs(ops):
     per layer, and not one for all of them, so that the first layers do not wait for weights of the last ones that are
     still being uploaded.'''
     from .ops import Op
+    if not any(op.meta is not None and op.meta[0] == 'conv_pack' for op in ops):
+        return ops
     written = set()
     for op in ops:
         written |= {id(b._placeholder) for b in _may_write(op)}
