@@ -144,3 +144,39 @@ def test_plans_and_packed_layout():
     assert each * slices + extra == 36 and product.grid[0] >= whole
     for m, k, n in ((2048, 4608, 512), (12544, 64, 256), (4096, 256, 32)):          #too few rows, too short a contraction, too little work
         assert all('split' not in l.kernel for l in plan(m, k, n).launches), (m, k, n)
+
+
+#input gradients of a strided 1x1 convolution whose result has one position: they write one element in four (or two) of the features'
+#array and zeros come from another launch, so what follows cannot be computed with the product
+ONE_POSITION = [(130, 2, 2, 64), (129, 1, 2, 64), (131, 2, 1, 64)]
+BEHIND = {'relu': lambda d, r, k: nn.relu(d), 'add': lambda d, r, k: d + r, 'scale': lambda d, r, k: d * k,
+          'relu backward': lambda d, r, k: jnp.where(r > 0, d, 0.0) * k}
+
+
+def gradient_of_one_position(behind):
+    loss = lambda x, w, ct: (lax.conv_general_dilated(x, w, (2, 2), 'VALID', dimension_numbers=DN) * ct).sum()
+    return lambda x, w, ct, r, k: behind(mj.grad(loss)(x, w, ct), r, k)
+
+
+@pytest.mark.parametrize('behind', list(BEHIND))
+@pytest.mark.parametrize('xs', ONE_POSITION)
+def test_a_product_that_writes_part_of_its_result_is_not_joined(xs, behind):
+    '''Plan only: the result of the program is written by a launch of its own, over all its elements.'''
+    args = [np.zeros(s, np.float32) for s in (xs, (1, 1, 64, 96), (xs[0], 1, 1, 96), xs, (64,))]
+    with K.overrides(conv_split=True):
+        program = JaxprInterpreter(mj.make_jaxpr(gradient_of_one_position(BEHIND[behind]))(*args), plan_only=True)
+    out = program.output_buffers[0]
+    writers = [l for l in program.launches if any(l.buffers[i][0] is out for i in l.written)]
+    assert len(writers) == 1 and writers[0].kernel.startswith('ew_chain'), [l.kernel for l in program.launches]
+    assert sum(l.kernel.startswith('conv_gemm_split') for l in program.launches) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('behind', list(BEHIND))
+@pytest.mark.parametrize('xs', ONE_POSITION)
+def test_values_behind_a_product_that_writes_part_of_its_result(xs, behind):
+    args = [ints(xs), ints((1, 1, 64, 96), -3, 4), ints((xs[0], 1, 1, 96)), ints(xs, -9, 10), ints((64,), 1, 4)]
+    print(f'case: {xs}, {behind}', flush=True)
+    with K.overrides(conv_split=True):
+        _, _, fn = check_against_oracle(gradient_of_one_position(BEHIND[behind]), args, exact=True)
+    assert len(split_kernels(fn)) == 1 and split_kernels(fn)[0].startswith('conv_gemm_split')

@@ -563,9 +563,11 @@ def _wgrad_ops(bufferpool, equation, outbuf, x, cot, wg: 'K.WgradGeometry'):
     return [Op(equation, launch=l) for l in launches]
 
 
-def _split_ops(bufferpool, equation, outbuf, lhs: Buffer, rhs: Buffer, geom: 'K.ConvGeometry', rhs_offset: int = 0, out_offset: int = 0):
+def _split_ops(bufferpool, equation, outbuf, lhs: Buffer, rhs: Buffer, geom: 'K.ConvGeometry', rhs_offset: int = 0,
+               part_at: tp.Optional[int] = None):
     '''The launches of a product that the bf16 matrix cores compute: its kernel operand packed for them, and the product.
-    None where another kernel is to compute it.'''
+    None where another kernel is to compute it. `part_at`: where in the result the product starts that writes only some of its
+    elements; nothing that follows may be joined to such a launch, since the other elements come from other launches.'''
     plan = K.conv_split_plan(lhs, geom)
     if plan is None:
         return None
@@ -579,8 +581,8 @@ def _split_ops(bufferpool, equation, outbuf, lhs: Buffer, rhs: Buffer, geom: 'K.
     bufferpool.op_counter = position
     source = EwOperand(rhs, rhs_offset, tuple(geom.ws))
     pack   = Op(equation, launch=K.conv_split_pack(packed, source, geom), meta=('conv_pack', packed, source, geom))
-    if out_offset or geom.os[1:] != (geom.Wo * geom.N, geom.N, 1) and geom.Ho * geom.Wo > 1:
-        return [pack, Op(equation, launch=K.conv_product(outbuf, lhs, packed, geom, out_offset=out_offset))]
+    if part_at is not None or geom.os[1:] != (geom.Wo * geom.N, geom.N, 1) and geom.Ho * geom.Wo > 1:
+        return [pack, Op(equation, launch=K.conv_product(outbuf, lhs, packed, geom, out_offset=part_at or 0))]
     return [pack, Op(equation, conv=(outbuf, lhs, packed, geom, []))]
 
 
