@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import vkjax_amd
-from vkjax_amd import lanes, minijax as mj, workloads as W
+from vkjax_amd import kernels as K, lanes, minijax as mj, workloads as W
 from vkjax_amd.jaxpr_interpreter import JaxprInterpreter
 from vkjax_amd.minijax import tree_util
 
@@ -51,6 +51,53 @@ def test_a_plan_that_misses_a_dependency_is_caught():
     #a wait covers what was issued on the other lane BEFORE it: a later launch there is not covered
     with pytest.raises(AssertionError, match='may overtake'):
         lanes.check(lanes.LanePlan(lane=[0, 1, 0, 1, 0], wait=[False, False, True, False, False], depends_on=[[], [], [1], [], [3]]))
+
+
+def products_with_shared_scratch(kind):
+    '''Independent products whose contractions are shared among blocks: their partial sums and counters lie in the same arrays.'''
+    dot = mj.numpy.dot
+    if kind == 'two products':
+        return lambda x, w, v: (dot(x, w), dot(x, v)), [(1024, 1024), (1024, 512), (1024, 512)]
+    return (lambda x, a, b, c, d: (lambda h: (dot(h, b), dot(h, c), dot(x, d)))(dot(x, a))), [(512, 2048), (2048, 1024), (1024, 512), (1024, 512), (2048, 512)]
+
+
+@pytest.mark.parametrize('kind', ('two products', 'four products'))
+def test_products_that_share_scratch_memory_are_ordered(kind):
+    fn, shapes = products_with_shared_scratch(kind)
+    with K.overrides(conv_split='128x128', conv_split_slices=2):
+        interp = JaxprInterpreter(mj.make_jaxpr(fn)(*[np.zeros(s, np.float32) for s in shapes]), plan_only=True, two_lanes=True)
+    plan, pairs = interp.lane_plan, 0
+    lanes.check(plan)
+    tensors = lambda buffers: {id(b.tensor) for b in buffers if b is not None and b.tensor is not None}
+    touched = [tensors(b for m in (l.members or (l,)) for b, _ in m.buffers) for l in interp.launches]
+    written = [tensors(m.buffers[i][0] for m in (l.members or (l,)) for i in m.written) for l in interp.launches]
+    for j in range(len(interp.launches)):
+        for i in range(j):
+            if written[i] & touched[j] or written[j] & touched[i]:
+                same_lane = plan.lane[i] == plan.lane[j]
+                waited = any(plan.wait[w] and plan.lane[w] == plan.lane[j] for w in range(i + 1, j + 1))
+                assert same_lane or waited, (i, j, [l.kernel for l in interp.launches])
+                pairs += bool(interp.launches[i].scratch and interp.launches[j].scratch)
+    assert any(plan.lane) and all(len(l.written) == 3 for l in interp.launches if l.kernel.startswith('conv_gemm_split'))
+    #what one lane's products leave half-way is not in the arrays of the other lane's
+    sets = [{id(l.buffers[i][0].tensor) for l, lane in zip(interp.launches, plan.lane) if lane == k for i in l.scratch} for k in (0, 1)]
+    assert len(sets[0]) == len(sets[1]) == 2 and not sets[0] & sets[1]
+    assert kind == 'two products' or pairs > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('kind', ('two products', 'four products'))
+def test_products_that_share_scratch_memory_give_the_bits_of_one_stream(kind):
+    fn, shapes = products_with_shared_scratch(kind)
+    rng  = np.random.RandomState(5)
+    args = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+    print(f'case: {kind}', flush=True)
+    with K.overrides(conv_split=True, conv_split_slices=2):
+        expected = vkjax_amd.wrap(fn, frontend='minijax')(*args)
+        two = vkjax_amd.wrap(fn, frontend='minijax', two_lanes=True)
+        for rep in range(3):
+            for a, b in zip(two(*args), expected):
+                assert np.array_equal(a, b), (kind, rep)
 
 
 def test_default_is_one_lane():

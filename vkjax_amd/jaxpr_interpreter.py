@@ -88,6 +88,8 @@ class JaxprInterpreter:
         #lower every op now so that unsupported layouts fail at build time, not at run time
         self.launches = self._stream_unread_results([op.launch for op in self.all_ops])
         self.lane_plan = lanes.plan(self.all_ops, self.launches) if self.two_lanes else None
+        if self.lane_plan is not None:
+            self.launches = lanes.with_scratch_of_their_lane(self.launches, self.lane_plan, self.bufferpool.second_set)
         self.early_parts = []
 
         if isinstance(self.mgr, PlanOnlyDevice):

@@ -98,6 +98,8 @@ class Launch(tp.NamedTuple):
     streamable: bool = False
     #which of `buffers` the kernel writes (positions); everything else it only reads
     written: tp.Tuple[int, ...] = (0,)
+    #which of `buffers` are scratch that other launches use too and that holds nothing (counters: zeros) between launches
+    scratch: tp.Tuple[int, ...] = ()
 
 
 def _u32(*values) -> bytes:
@@ -1193,7 +1195,8 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
     scratch = [(split.partial, 0), (split.arrivals, 0)] if shared else [(None, 0), (None, 0)]
     return Launch(f'conv_gemm_split_{split.tile}', (split.whole + shared * split.slices, 1, 1), (256, 1, 1),
                   [(out, out_offset * 4), (lhs, lhs_offset * 4), (packed, 0)] + scratch + operand_slots + derived_ptrs,
-                  params + derived_desc, bytes_moved=nbytes, flops=2 * M * N * K, written=(0, 3, 4) if shared else (0,))
+                  params + derived_desc, bytes_moved=nbytes, flops=2 * M * N * K,
+                  written=(0, 3, 4) if shared else (0,), scratch=(3, 4) if shared else ())
 
 
 def conv_product(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: tp.Sequence[ConvEpilogueStep] = (), **offsets) -> Launch:

@@ -59,18 +59,28 @@ def touched_and_written(op, launch) -> tp.Tuple[tp.Set[int], tp.Set[int]]:
         touched = tensors(b for m in launch.members for b, _ in m.buffers)
         written = tensors(m.buffers[0][0] for m in launch.members if m.buffers)
         return touched, written
-    #chains and convolutions know their results (a convolution may store a second one from its epilogue); every other
-    #kernel says which of its arrays it writes
+    #every launch says which of its arrays it writes (results, and scratch memory that launches may share: the partial sums and
+    #counters of products with a shared contraction); a convolution may store a second result from its epilogue besides
+    written = tensors(launch.buffers[i][0] for i in launch.written if i < len(launch.buffers))
     if op.chain is not None or op.conv is not None:
-        written = tensors(fusion._writes(op))
-    else:
-        written = tensors(launch.buffers[i][0] for i in launch.written if i < len(launch.buffers))
+        written |= tensors(fusion._writes(op))
     return tensors(b for b, _ in launch.buffers) | written, written
 
 
+def with_scratch_of_their_lane(launches, plan_: 'LanePlan', second_set: tp.Callable) -> tp.List:
+    '''The launches, those on the second lane with a second set of the scratch arrays that products with a shared contraction have in
+    common and that hold nothing from one launch to the next (kernels.Launch.scratch).'''
+    def moved(launch):
+        return launch._replace(buffers=[(second_set(b), offset) if i in launch.scratch else (b, offset)
+                                        for i, (b, offset) in enumerate(launch.buffers)])
+    return [moved(launch) if lane and launch.scratch else launch for launch, lane in zip(launches, plan_.lane)]
+
+
 def dependencies(ops, launches) -> tp.List[tp.List[int]]:
-    '''For every launch the earlier launches it must not overtake.'''
-    sets = [touched_and_written(op, launch) for op, launch in zip(ops, launches)]
+    '''For every launch the earlier launches it must not overtake. Launches on one lane never do; the scratch arrays that each
+    lane has a set of are left out.'''
+    own  = {id(launch.buffers[i][0].tensor) for launch in launches for i in launch.scratch}
+    sets = [tuple(s - own for s in touched_and_written(op, launch)) for op, launch in zip(ops, launches)]
     result = []
     for j, (touched_j, written_j) in enumerate(sets):
         deps = [i for i in range(j) if (sets[i][1] & touched_j) or (written_j & sets[i][0])]
