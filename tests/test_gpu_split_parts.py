@@ -58,3 +58,24 @@ def test_sums_of_few_terms_are_cut_off_once_per_product_behind_the_first(n):
         with K.overrides(wgrad_split=tile):
             y = vkjax_amd.wrap(lambda x, g: mj.lax.dot_general(x, g, (((0,), (0,)), ((), ()))), frontend='minijax')(np.ascontiguousarray(x.T), w)
         assert (np.abs(y - exact) <= limit).all(), (tile, np.max(np.abs(y - exact) / np.maximum(limit, 1e-300)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('value', (np.inf, np.nan, 3.4e38))
+def test_finite_sums_keep_their_bits_beside_others(value):
+    '''Data whose sums are rounded: an operand that is not finite (or beyond the largest bf16) in one row changes that row only.'''
+    x, w  = rng.standard_normal((200, 160)).astype(np.float32), rng.standard_normal((160, 96)).astype(np.float32)
+    other = x.copy()
+    other[37, 21] = value
+    rest  = np.arange(200) != 37
+    for tile in K.CONV_SPLIT_TILES:
+        for slices in (1, 2):
+            with K.overrides(conv_split=tile, conv_split_slices=slices):
+                fn = vkjax_amd.wrap(lambda x, w: jnp.dot(x, w), frontend='minijax')
+                before, after = fn(x, w), fn(other, w)
+            assert np.array_equal(before[rest], after[rest]) and not np.array_equal(before[37], after[37]), (tile, slices)
+    for tile in K.WGRAD_SPLIT_TILES:
+        with K.overrides(wgrad_split=tile):
+            fn = vkjax_amd.wrap(lambda x, g: mj.lax.dot_general(x, g, (((0,), (0,)), ((), ()))), frontend='minijax')
+            before, after = fn(np.ascontiguousarray(x.T), w), fn(np.ascontiguousarray(other.T), w)
+        assert np.array_equal(before[rest], after[rest]) and not np.array_equal(before[37], after[37]), tile

@@ -8,8 +8,8 @@
 // times as fast as fp32, so six products instead of one are still 2.6 times as fast at peak.
 //   - exact for numbers from 2^-109 up (below, lo loses what a bf16 cannot hold: an absolute error under 2^-134);
 //   - operands that are infinite, NaN or beyond the largest bf16 (3.39e38) leave sums that are not finite, because a part that is
-//     infinite meets parts that are zero: a wave whose results are not all finite computes its tile again with
-//     v_mfma_f32_32x32x2_f32 and fp32 operands, so that such results are what they always were.
+//     infinite meets parts that are zero: a wave whose results are not all finite computes those that are not again with
+//     v_mfma_f32_32x32x2_f32 and fp32 operands, so that such results are what fp32 products give.
 // Measured against 64-bit sums (4096 x K x 128, normal data): an error of 0.88, 0.63 and 0.39 times that of
 // v_mfma_f32_32x32x2_f32 at K = 64, 576 and 2304 (which rounds after every second product, this after every sixteenth).
 #pragma once
@@ -401,7 +401,8 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     }
 
     // An operand that is infinite, not a number, or beyond the largest bf16 leaves a sum that is not finite (infinity
-    // times the zero parts of the other operand): such sub-tiles are computed again with fp32 products.
+    // times the zero parts of the other operand): such sums are computed again with fp32 products. The finite ones beside them
+    // stay as they are, so a row's results do not depend on what the rows in its tile hold.
     {
         float t = 0.f;
 #pragma unroll
@@ -443,7 +444,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                         if (c >= P.Cin) { c = half; if (++s == P.KW) { s = 0; ++r; } }
                     }
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[i][j][v] = a2[v];
+                    for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_isfinite(acc[i][j][v]) ? acc[i][j][v] : a2[v];
                 }
             }
         }

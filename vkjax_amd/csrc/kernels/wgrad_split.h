@@ -201,7 +201,8 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
         __syncthreads();
     }
 
-    // Sums that are not finite (an operand that is infinite, not a number, or beyond the largest bf16): again, with fp32 products.
+    // Sums that are not finite (an operand that is infinite, not a number, or beyond the largest bf16): again, with fp32 products. The
+    // finite ones beside them stay as they are.
     float t = 0.f;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -230,7 +231,8 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
                     const float bv = buffer_load_x1(g_rsrc, p < kend && n < P.N ? (uint32_t)(p * P.N + n) * 4u : WG_OOB);
                     again = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, again, 0, 0, 0);
                 }
-                acc[i][j] = again;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_isfinite(acc[i][j][v]) ? acc[i][j][v] : again[v];
             }
         }
     }
