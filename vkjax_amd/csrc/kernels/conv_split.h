@@ -245,13 +245,13 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     // The small products of a k step come first, (A part, B part): a sum that begins there is cut off once at its full size and not four
     // times. (Of 512 terms 512, 16 and 1 that are not zero: errors of 1.22e-7, 7.6e-8 and 3.5e-8 of the results' 2-norm, with the largest
     // product first 1.36e-7, 8.9e-8 and 5.3e-8, through fp32 products 2.1e-7, 5.9e-8 and 2.5e-8; no slower.)
-    constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
+    constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
     constexpr int CH = TM * TN, NS = 6 * CH;
     float sign = kbeg & 2 ? -1.f : 1.f;
     auto k16_step = [&](auto step_, int kt) {
         constexpr int step = decltype(step_)::value, ks = step & 1, item = 1 - ks;   // step of the pair of k tiles, the second of its k tile
         u32x4 *const mine = As + (step >> 1) * 12 * BM, *const other = As + ((step >> 1) ^ 1) * 12 * BM;
-        constexpr int BARRIER = 6 * TN - 6;                                     // second step only: in front of the first part of the next tile
+        constexpr int BARRIER = 6 * TN - 4;                                     // second step only: in front of the first part of the next tile
         constexpr int SPLIT = ks == 0 ? 0 : BARRIER, EACH = (NS - SPLIT) / 6;   // an item's three parts, in halves, then its reload
         u32x4* const to = ks == 0 ? other : mine;                               // k tile kt + 1, or kt + 2
         FENCE();
@@ -268,7 +268,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                 for (int v = 4 * t - 8; v < 4 * t - 4; ++v) acc[pc / TN][pc % TN][v] = __builtin_fmaf(sum[pc][v], sign, acc[pc / TN][pc % TN][v]);
             }
             // parts of A that have met their last column are replaced by the next step's
-            if (j == TN - 1 && (t == 0 || t == 3 || t == 5)) read_a(ks == 1 ? other : mine, 1 - ks, t == 0 ? 2 : t == 3 ? 1 : 0, i);
+            if (j == TN - 1 && (t == 2 || t == 4 || t == 5)) read_a(ks == 1 ? other : mine, 1 - ks, t == 2 ? 2 : t == 4 ? 1 : 0, i);
             // an item of a later k tile
             if (n >= SPLIT && (n - SPLIT) % EACH == EACH - 1 && (n - SPLIT) / EACH < 6) {
                 const int h = (n - SPLIT) / EACH, pt = h / 2;
@@ -347,6 +347,10 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int t = 0; t < 3; ++t) read_a(As, 0, t, i);
+        // Everything requested so far has arrived when the loop begins: the compiler then counts in the loop which of its own loads it waits
+        // for. (Left alone it may wait for all of them once per pair of k tiles, where the paths into the loop differ in their order: 12544 x
+        // 2304 x 256, one block per CU, 95.5 us instead of 92.)
+        __builtin_amdgcn_s_waitcnt(0x0F70);
         for (int kt = kbeg; kt < kend; kt += 2) {
             k16_step(std::integral_constant<int, 0>{}, kt);
             k16_step(std::integral_constant<int, 1>{}, kt);

@@ -166,7 +166,7 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
     for (int j = 0; j < TN; ++j) b_from[j] = Bs + read_slot(wn * TN + j, BN);
 
     f32x16 acc[TM][TN] = {};
-    constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
+    constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
     if (nk > 0) load_tile(0);
     for (int kt = 0; kt < nk; ++kt) {
         park_tile(kt & 1);
