@@ -131,6 +131,25 @@ def test_infinite_and_huge_operands(slices):
     assert np.isnan(results[0]).any() and np.isinf(results[0]).any() and np.isfinite(results[0]).any()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize('tile', list(K.CONV_SPLIT_TILES))
+@pytest.mark.parametrize('desc,xs,ks,f', SHAPES, ids=[s[0] for s in SHAPES])
+def test_sums_computed_again_with_fp32_products(tile, desc, xs, ks, f):
+    '''Over the same shapes, with operands that are not finite (and one beyond the largest bf16) in images and kernel: the sums they reach are
+    computed again by another loop over the operands.'''
+    x, k = ints(xs), ints(ks, -3, 4)
+    k[:, :, -1] = np.sign(k[:, :, -1])                   #(a product beyond the largest number would be infinite or not by the order of its sum)
+    x.reshape(-1)[rng.permutation(x.size)[:3]] = np.inf, np.nan, -np.inf
+    k.reshape(-1)[rng.permutation(k.size)[:2]] = np.inf, -np.inf
+    x[-1, -1, -1, -1] = 3.4e38
+    results = []
+    print(f'case: {desc}, tile {tile}', flush=True)
+    for choice in (tile, False):
+        with K.overrides(conv_split=choice):
+            results.append(vkjax_amd.wrap(f, frontend='minijax')(x, k))
+    assert np.array_equal(results[0], results[1], equal_nan=True) and not np.isfinite(results[0]).all()
+
+
 def test_plans_and_packed_layout():
     '''Plan only: which products take these kernels, the argument block's tail, and the size of the packed operand.'''
     def plan(m, k, n):

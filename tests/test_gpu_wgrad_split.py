@@ -63,6 +63,25 @@ def test_tile_edges_and_slices(tile, desc, xs, ws, gyx, strides, padding, dilati
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('desc,xs,ws,gyx,strides,padding,dilation', SHAPES, ids=[s[0] for s in SHAPES])
+def test_sums_computed_again_with_fp32_products(desc, xs, ws, gyx, strides, padding, dilation):
+    '''Over the same shapes, with operands that are not finite in X and G.'''
+    x, w = rng.randint(-4, 5, size=xs).astype(np.float32), np.zeros(ws, np.float32)
+    g = rng.randint(-3, 4, size=(xs[0],) + gyx + ws[3:]).astype(np.float32)
+    x.reshape(-1)[rng.permutation(x.size)[:3]] = np.inf, np.nan, -np.inf
+    g.reshape(-1)[rng.permutation(g.size)[:2]] = np.inf, -np.inf
+    f = kernel_gradient(strides, padding, dilation)
+    results = {}
+    for tile in list(K.WGRAD_SPLIT_TILES) + [False]:
+        for slices in (1, 3):
+            print(f'case: {desc}, tile {tile}, {slices} slices', flush=True)
+            with K.overrides(wgrad_split=tile, wgrad_slices=slices):
+                results[tile, slices] = vkjax_amd.wrap(f, frontend='minijax')(x, w, g)
+    expected = results[False, 1]
+    assert not np.isfinite(expected).all() and all(np.array_equal(y, expected, equal_nan=True) for y in results.values())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('pixels,M,N', [(200, 40, 72), (2049, 132, 128), (12544, 256, 64)])
 def test_error_against_64_bit_sums_is_no_larger(pixels, M, N):
     x, g = rng.standard_normal((pixels, M)).astype(np.float32), rng.standard_normal((pixels, N)).astype(np.float32)
