@@ -79,3 +79,81 @@ def test_finite_sums_keep_their_bits_beside_others(value):
             fn = vkjax_amd.wrap(lambda x, g: mj.lax.dot_general(x, g, (((0,), (0,)), ((), ()))), frontend='minijax')
             before, after = fn(np.ascontiguousarray(x.T), w), fn(np.ascontiguousarray(other.T), w)
         assert np.array_equal(before[rest], after[rest]) and not np.array_equal(before[37], after[37]), tile
+
+
+def scaled(shape, factor):
+    return (rng.standard_normal(shape) * factor).astype(np.float32)
+
+
+#x, w by their factors: numbers whose parts a bf16 cannot hold (below 2^-102 = 2e-31), down to those with few bits themselves
+SMALL = [(1e-32, 1e30), (1e-36, 1e30), (1e-38, 1e20), (1e-42, 1e25), (1e30, 1e-36), (1e25, 1e-42), (1e-36, 1.0), (1e-20, 1e-17), (1e-19, 1e-19)]
+
+
+def assert_fp32_error(y, x, w):
+    '''At most two roundings per product of two k and one per 64 k, parts left out and cut sums below that: (K + K / 64 + 17) 2^-24 sum |x||w|;
+    numbers too small for 24 bits of their own are off by half of 2^-149 per rounding.'''
+    K_    = x.shape[1]
+    exact = x.astype(np.float64) @ w.astype(np.float64)
+    limit = (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64)) * (K_ + K_ / 64 + 17) * 2.0 ** -24 + (K_ + 1) * 2.0 ** -150
+    assert (np.abs(y - exact) <= limit).all(), np.max(np.abs(y - exact) / limit)
+    return np.linalg.norm(y - exact)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('fx,fw', SMALL)
+def test_small_operands_keep_their_bits(fx, fw):
+    '''Some rows (columns) of small numbers, some of zeros, some of ordinary ones; in the 2-norm no further off than fp32 products are.'''
+    K_, M, N = 320, 200, 72
+    x, w = scaled((M, K_), fx), scaled((K_, N), fw)
+    x[5], x[130:140], w[:, 3], w[:, 40:44] = 0, 0, 0, 0
+    x[7], x[150] = scaled((2, K_), 1.0)
+    x[9, :200], x[160, 1:] = 0, 0
+    dot = lambda x, w: jnp.dot(x, w)
+    wg  = lambda x, g: mj.lax.dot_general(x, g, (((0,), (0,)), ((), ())))
+    def result(f, a, b, **choice):
+        with K.overrides(**choice):
+            return vkjax_amd.wrap(f, frontend='minijax')(a, b)
+    fp32 = assert_fp32_error(result(dot, x, w, conv_split=False), x, w)
+    for tile in K.CONV_SPLIT_TILES:
+        for slices in (1, 3):
+            print(f'case: {fx} {fw}, tile {tile}, {slices} slices', flush=True)
+            assert assert_fp32_error(result(dot, x, w, conv_split=tile, conv_split_slices=slices), x, w) <= 1.05 * fp32
+    xt   = np.ascontiguousarray(x.T)
+    fp32 = assert_fp32_error(result(wg, xt, w, wgrad_split=False), x, w)
+    for tile in K.WGRAD_SPLIT_TILES:
+        for slices in (1, 3):
+            print(f'case: kernel gradient, {fx} {fw}, tile {tile}, {slices} slices', flush=True)
+            assert assert_fp32_error(result(wg, xt, w, wgrad_split=tile, wgrad_slices=slices), x, w) <= 1.05 * fp32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('tile', list(K.CONV_SPLIT_TILES))
+@pytest.mark.parametrize('stride,dilation,padding', [((1, 1), (1, 1), 'SAME'), ((2, 2), (1, 1), 'SAME'), ((1, 1), (2, 3), 'VALID')])
+def test_small_images(tile, stride, dilation, padding):
+    '''Rows that are windows of an image, parts of them outside it: powers of two below 2^-102, so that every product is exact.'''
+    f = lambda x, k: mj.lax.conv_general_dilated(x, k, stride, padding, rhs_dilation=dilation, dimension_numbers=('NHWC', 'HWIO', 'NHWC'))
+    x = (rng.randint(-4, 5, size=(2, 15, 14, 32)) * 2.0 ** -145).astype(np.float32)
+    x[1, 3:9] = 0
+    k = (rng.randint(-3, 4, size=(3, 3, 32, 40)) * 2.0 ** 100).astype(np.float32)
+    with K.overrides(conv_split=False):
+        expected = vkjax_amd.wrap(f, frontend='minijax')(x, k)
+    with K.overrides(conv_split=tile):
+        assert np.array_equal(vkjax_amd.wrap(f, frontend='minijax')(x, k), expected) and (expected != 0).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('large', (2.0 ** 48, 2.0 ** 49, 2.0 ** 103, 2.0 ** 104, 2.0 ** 120, 3.4e38))
+def test_large_kernel_operands(large):
+    '''Weights around the largest that are packed in three parts, and beyond: integers times powers of two, so that every result is exact.'''
+    x, w = rng.randint(-4, 5, size=(140, 160)).astype(np.float32), rng.randint(-3, 4, size=(160, 70)).astype(np.float32)
+    w[77, 5], w[100, 69], w[100, 68] = large, -large, large
+    x[:, 77], x[:, 100] = np.sign(x[:, 77]), np.sign(x[:, 100])
+    results = []
+    for choice in list(K.CONV_SPLIT_TILES) + [False]:
+        with K.overrides(conv_split=choice):
+            results.append(vkjax_amd.wrap(lambda x, w: jnp.dot(x, w), frontend='minijax')(x, w))
+    exact = x.astype(np.float64) @ w.astype(np.float64)
+    small = np.arange(70)[~np.isin(np.arange(70), (5, 68, 69))]
+    for y in results:
+        assert np.array_equal(y[:, small], exact[:, small])
+        assert np.allclose(y, exact, rtol=160 * 2.0 ** -24, atol=0)           #one rounding per term

@@ -6,12 +6,16 @@
 // products hi.hi, hi.mid, mid.hi, hi.lo, mid.mid, lo.hi, each exact in fp32 and added in fp32 accumulators; the three that are
 // left out are below 2^-24 of the product together, the rounding of an fp32 accumulation. The matrix cores run bf16 sixteen
 // times as fast as fp32, so six products instead of one are still 2.6 times as fast at peak.
-//   - exact for numbers from 2^-109 up (below, lo loses what a bf16 cannot hold: an absolute error under 2^-134);
+//   - a number below 2^-102 has parts that a bf16 holds with fewer bits, or not at all (an absolute error under 2^-125). The kernel operand is
+//     multiplied by 2^24 before it is taken apart, and the sums by 2^-24, so its smallest numbers have all their bits; of the rows' operand
+//     such numbers matter only to sums that are themselves below 2^-97 K times the largest weight. Those, if they exist, and if their
+//     row holds such a number, are computed again with fp32 products (below);
 //   - operands that are infinite, NaN or beyond the largest bf16 (3.39e38) leave sums that are not finite, because a part that is
 //     infinite meets parts that are zero: a wave whose results are not all finite computes those that are not again with
 //     v_mfma_f32_32x32x2_f32 and fp32 operands, so that such results are what fp32 products give.
-// Measured against 64-bit sums (4096 x K x 128, normal data): an error of 0.88, 0.63 and 0.39 times that of
-// v_mfma_f32_32x32x2_f32 at K = 64, 576 and 2304 (which rounds after every second product, this after every sixteenth).
+// Measured against 64-bit sums (4096 x K x 128, normal data): an error of 0.76, 0.56 and 0.30 times that of
+// v_mfma_f32_32x32x2_f32 at K = 64, 576 and 2304 (which rounds after every second product, this after every sixteenth). Sums of which less than
+// a fifth of the terms are not zero are further off than those: 1.3 times at 16 of 512, 1.4 times at one (which is cut off, not rounded).
 #pragma once
 #include "split_bf16.h"
 
@@ -40,11 +44,19 @@ struct ConvPackEntry {
     uint32_t first_block, pad;
     u32x4*       out;
     const float* w;
+    float*       largest;
     ConvPackParams P;
 };
-static_assert(sizeof(ConvPackEntry) == 56, "the host lays the table out with 56-byte entries");
+static_assert(sizeof(ConvPackEntry) == 64, "the host lays the table out with 64-byte entries");
 
-__device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const float* __restrict__ w, const ConvPackParams& P, int block) {
+// A number beyond CONV_PACK_MOST is stored as it is: a NaN of its own kind in front, which has the column's sums computed again with fp32
+// products, and its two halves behind it. `largest`: per workgroup (32 columns, 64 k), the largest of the others.
+constexpr float CONV_PACK_SCALE = 0x1p24f, CONV_PACK_MOST = 0x1p48f;
+constexpr uint32_t CONV_PACK_RAW = 0x7FC1u;
+
+__device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const float* __restrict__ w, float* __restrict__ largest, const ConvPackParams& P,
+                                               int block) {
+    __shared__ float wave_largest[4];
     const int id = block * 256 + (int)threadIdx.x, lane = id & 63, step = id >> 6, ksteps = (P.K + 63) / 64 * 4;
     const int nb = step / ksteps, s = step - nb * ksteps, o = 2 * (s & 1) + (lane >> 5), n = nb * 32 + (lane & 31);
     if (nb * 32 >= P.N) return;
@@ -61,32 +73,41 @@ __device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const fl
         }
     }
     u32x4 part[3];
+    float most = 0.f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        float a = x[2 * q], b = x[2 * q + 1];
+        float rest[2] = {x[2 * q] * CONV_PACK_SCALE, x[2 * q + 1] * CONV_PACK_SCALE};
+        uint32_t v[3];
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
-            uint32_t v = to_bf16x2(a, b);
-            if (t == 0) {
-                // a finite number beyond the largest bf16 keeps its leading bits instead of becoming infinite; behind an
-                // infinity or a NaN nothing is left: the three parts of any number add up to it
-                const bool fa = __builtin_isfinite(a), fb = __builtin_isfinite(b);
-                if (fa && (v & 0x7FFFu) == 0x7F80u) v = (v & 0xFFFF0000u) | (f2u(a) >> 16);
-                if (fb && (v & 0x7FFF0000u) == 0x7F800000u) v = (v & 0xFFFFu) | (f2u(b) & 0xFFFF0000u);
-                a = fa ? a - u2f(v << 16) : 0.f;
-                b = fb ? b - u2f(v & 0xFFFF0000u) : 0.f;
-            } else {
-                a = a - u2f(v << 16);
-                b = b - u2f(v & 0xFFFF0000u);
-            }
-            part[t][q] = v;
+            v[t] = to_bf16x2(rest[0], rest[1]);
+            rest[0] -= u2f(v[t] << 16);
+            rest[1] -= u2f(v[t] & 0xFFFF0000u);
         }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t shift = 16 * h, bits = f2u(x[2 * q + h]), keep = h ? 0xFFFFu : 0xFFFF0000u;
+            if (fabsf(x[2 * q + h]) <= CONV_PACK_MOST) { most = fmaxf(most, fabsf(x[2 * q + h])); continue; }
+            const bool raw = __builtin_isfinite(x[2 * q + h]);
+            const uint32_t front = raw ? CONV_PACK_RAW : bits << 1 > 0xFF000000u ? 0x7FC0u : bits >> 16;
+            v[0] = (v[0] & keep) | front << shift;
+            v[1] = (v[1] & keep) | (raw ? bits >> 16 : 0u) << shift;
+            v[2] = (v[2] & keep) | (raw ? bits & 0xFFFFu : 0u) << shift;
+        }
+#pragma unroll
+        for (int t = 0; t < 3; ++t) part[t][q] = v[t];
     }
 #pragma unroll
     for (int t = 0; t < 3; ++t) out[(size_t)step * 192 + t * 64 + lane] = part[t];
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) most = fmaxf(most, __shfl_xor(most, m, 64));
+    if (lane == 0) wave_largest[step & 3] = most;
+    __syncthreads();
+    if (threadIdx.x == 0) largest[block] = fmaxf(fmaxf(wave_largest[0], wave_largest[1]), fmaxf(wave_largest[2], wave_largest[3]));
 }
-extern "C" __global__ __launch_bounds__(256) void conv_split_pack(u32x4* __restrict__ out, const float* __restrict__ w, ConvPackParams P) {
-    conv_pack_body(out, w, P, blockIdx.x);
+extern "C" __global__ __launch_bounds__(256) void conv_split_pack(u32x4* __restrict__ out, const float* __restrict__ w, float* __restrict__ largest,
+                                                                  ConvPackParams P) {
+    conv_pack_body(out, w, largest, P, blockIdx.x);
 }
 // The weights of several layers in one launch: workgroup b belongs to the last entry of the table whose first_block is <= b.
 extern "C" __global__ __launch_bounds__(256) void conv_split_pack_layers(const ConvPackEntry* __restrict__ table, uint32_t entries) {
@@ -96,7 +117,7 @@ extern "C" __global__ __launch_bounds__(256) void conv_split_pack_layers(const C
         if (table[mid].first_block <= blockIdx.x) lo = mid; else hi = mid;
     }
     const ConvPackEntry& e = table[__builtin_amdgcn_readfirstlane(lo)];
-    conv_pack_body(e.out, e.w, e.P, (int)(blockIdx.x - e.first_block));
+    conv_pack_body(e.out, e.w, e.largest, e.P, (int)(blockIdx.x - e.first_block));
 }
 
 // ---- the product ------------------------------------------------------------------------------------------------------
@@ -125,11 +146,10 @@ template <int WGM, int WGN, int TM, int TN>
 __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float* __restrict__ Es, int* __restrict__ Rs,
                                                 float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                                                 float* __restrict__ partial, uint32_t* __restrict__ arrivals, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
-                                                const ConvParams& P, const ConvDerived& Dk) {
+                                                const float* __restrict__ largest, const ConvParams& P, const ConvDerived& Dk) {
     constexpr int BM = 32 * WGM * TM, BN = 32 * WGN * TN, NT = 64 * WGM * WGN, BK = 32;
     u32x4* const As = pool;                         // [2 buffers][3 parts][4 octets][BM rows]
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WGN, wn = wave % WGN, l32 = lane & 31, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / WGN, wn = wave % WGN;
     const bool c_contig = P.flags & 1u, flat_rows = P.flags & 2u, masked = P.flags & 4u;
     const int nepi = (P.flags >> 8) & 15u, epi_first_full = (int)((P.flags >> 16) & 15u) - 1;
     auto step_desc = [&](int e) -> uint32_t { return ((e < 3 ? P.epi_desc[0] : P.epi_desc[1]) >> (10 * (e < 3 ? e : e - 3))) & 1023u; };
@@ -154,6 +174,11 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(reinterpret_cast<const char*>(x) - x_bias, P.x_bytes + x_bias),
                                  w_rsrc = make_rsrc(w, P.w_bytes), o_rsrc = make_rsrc(out, P.out_bytes);
 
+    const uint32_t rowb = (uint32_t)P.N * 4u;
+    float acc[TM][TN][16];
+    uint32_t b_soff[TN];                             // the packed columns of this wave
+    {
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
     // ---- load assignment: A item = (row, octet of k); octet o holds k = 4o..4o+3 and 16+4o..16+4o+3 of the k tile
     constexpr int A_NI = BM * 4 / NT, A_RSTEP = NT / 4;
     const int a_o = tid & 3, a_r0 = tid >> 2;
@@ -180,8 +205,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                 a_inv[p] |= ((uint32_t)(hi0 + r * P.DH) >= (uint32_t)P.H ? wall : wbad) << (r * P.KW);
         }
     }
-    // the packed columns of this wave (blocks of columns beyond the last one lie outside the descriptor and read as zeros)
-    uint32_t b_soff[TN];
+    // (blocks of columns beyond the last one lie outside the descriptor and read as zeros)
 #pragma unroll
     for (int j = 0; j < TN; ++j) b_soff[j] = (uint32_t)(n0 / 32 + wn * TN + j) * (uint32_t)ktiles * 6144u;
     const uint32_t b_lane = (uint32_t)lane * 16u;
@@ -190,7 +214,6 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         const int rs = t_c / P.Cin;
         t_c -= rs * P.Cin; t_r = rs / P.KW; t_s = rs - t_r * P.KW;
     }
-    const uint32_t rowb = (uint32_t)P.N * 4u;
     static_assert(A_NI == 2 && TM == 2, "two items per thread, two rows of tiles per wave: the schedule below");
     f32x4 raw[2][2];
     // requests item p of k tile kt (beyond the contraction: zeros)
@@ -206,7 +229,6 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         const bool wrap_c = t_c >= P.Cin; t_c = wrap_c ? 0 : t_c; t_s += wrap_c ? 1 : 0;
         const bool wrap_s = t_s == P.KW; t_s = wrap_s ? 0 : t_s; t_r += wrap_s ? 1 : 0;
     };
-    float acc[TM][TN][16];
     f32x16 sum[TM * TN] = {};                        // the products of a pair of k tiles
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -247,7 +269,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     // product first 1.36e-7, 8.9e-8 and 5.3e-8, through fp32 products 2.1e-7, 5.9e-8 and 2.5e-8; no slower.)
     constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
     constexpr int CH = TM * TN, NS = 6 * CH;
-    float sign = kbeg & 2 ? -1.f : 1.f;
+    float sign = kbeg & 2 ? -1.f / CONV_PACK_SCALE : 1.f / CONV_PACK_SCALE;
     auto k16_step = [&](auto step_, int kt) {
         constexpr int step = decltype(step_)::value, ks = step & 1, item = 1 - ks;   // step of the pair of k tiles, the second of its k tile
         u32x4 *const mine = As + (step >> 1) * 12 * BM, *const other = As + ((step >> 1) ^ 1) * 12 * BM;
@@ -361,7 +383,11 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         for (int v = 0; v < 16; ++v) acc[TM - 1][TN - 1][v] = __builtin_fmaf(sum[CH - 1][v], sign, acc[TM - 1][TN - 1][v]);
         __syncthreads();
     }
+    }
 
+    // (behind the loop the lane's number is asked for again: kept over the loop, it and what depends on it would cost registers there)
+    const int tid = tid_again(wave), lane = tid & 63, l32 = lane & 31, half = lane >> 5;
+    const uint32_t b_lane = (uint32_t)lane * 16u;
     if (sliced) {
         // store this slice's sums; the block that arrives last adds all of them, in the order of the slices
         const int mine = tile - whole;
@@ -404,49 +430,155 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                     }
     }
 
-    // An operand that is infinite, not a number, or beyond the largest bf16 leaves a sum that is not finite (infinity
-    // times the zero parts of the other operand): such sums are computed again with fp32 products. The finite ones beside them
-    // stay as they are, so a row's results do not depend on what the rows in its tile hold.
+    // Sums that are computed again with fp32 products. The others beside them stay as they are, so a row's results do not depend on what
+    // the rows in its tile hold.
+    //   - An operand that is infinite, not a number, or beyond the largest bf16 leaves a sum that is not finite (infinity times the zero parts
+    //     of the other operand).
+    //   - Numbers of the rows below 2^-102 lose up to 2^-125 each, a sum up to 2^-125 K times its largest weight: less than 2^-28 of a sum from
+    //     2^-97 K times that weight up. Of smaller sums (zeros, nearly always: rows or columns of zeros) the row is looked through for such numbers.
     {
-        float t = 0.f;
+        float high = 0.f, low = __builtin_inff();
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) t = __builtin_fmaf(acc[i][j][v], 0.f, t);
-        if (__builtin_amdgcn_ballot_w64(t != t)) {
-            // In the order of the packed operand: lane l of a k16 step takes row l % 32, column l % 32 and the octet of its half of the wave,
-            // so both operands come in 16-byte loads, the next step's while this one's 8 TN products run. With NaN only, 12544 x 2304 x 256:
-            // 344 us (102 without any; 1560 with single words requested one after the other), 3x3x128x128 on 50176 rows 297 (91; 1350).
-            const int r0 = m0 + wm * TM * 32 + l32;
+                for (int v = 0; v < 16; v += 2) high = higher_of(high, acc[i][j][v], acc[i][j][v + 1]);
+        bool in_n[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) in_n[j] = n0 + (wn * TN + j) * 32 + l32 < P.N;
+        if (m0 + BM <= P.M && n0 + BN <= P.N) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; v += 2) low = lower_of(low, acc[i][j][v], acc[i][j][v + 1]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const bool in_m = m0 + (wm * TM + i) * 32 + 4 * half + 8 * (v / 4) + v % 4 < P.M;
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) low = lower_of(low, in_m && in_n[j] ? acc[i][j][v] : low, low);
+                }
+        }
+        // Rows' operand in the order of the packed one: lane l of a k16 step takes row l % 32 and the octet of its half of the wave, so both come
+        // in 16-byte loads.
+        int row_at[TM], row_y[TM], row_x[TM], tap_r, tap_s, tap_c;
+        auto start_rows = [&]() {
+            tap_r = tap_s = tap_c = 0;
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                const int m = r0 + i * 32;
+                const int m = m0 + (wm * TM + i) * 32 + l32;
                 const int b = flat_rows ? 0 : magic_div(m, P.howo_magic, P.howo_shift), r2 = m - b * HoWo;
                 const int ho = flat_rows ? 0 : magic_div(r2, P.wo_magic, P.wo_shift), wo = r2 - ho * P.Wo;
-                const int hi0 = ho * P.SH - P.PH, wi0 = wo * P.SW - P.PW;
-                const uint32_t row = (uint32_t)(flat_rows ? m * P.xs_h : b * P.xs_b + ho * P.SH * P.xs_h + wo * P.SW * P.xs_w) * 4u;
-                int r = 0, s = 0, c = 0;
+                row_at[i] = flat_rows ? m * P.xs_h : b * P.xs_b + ho * P.SH * P.xs_h + wo * P.SW * P.xs_w;
+                row_y[i]  = m < P.M ? ho * P.SH - P.PH : INT32_MIN / 2;      // (rows beyond the last one lie outside every image)
+                row_x[i]  = wo * P.SW - P.PW;
+            }
+        };
+        auto request_row = [&](f32x4 (&to)[2], int i, int step) {
+            const int y = row_y[i] + tap_r * P.DH, xx = row_x[i] + tap_s * P.DW, o = 2 * (step & 1) + half, k = (step >> 1) * BK + 4 * o;
+            const bool ok = flat_rows ? row_y[i] >= 0 : (uint32_t)y < (uint32_t)P.H && (uint32_t)xx < (uint32_t)P.W;
+            const uint32_t at = (uint32_t)(row_at[i] + tap_r * P.DH * P.xs_h + tap_s * P.DW * P.xs_w + tap_c + 4 * o) * 4u;
+            to[0] = buffer_load_x4(x_rsrc, ok && k < P.K ? at : CONV_OOB);
+            to[1] = buffer_load_x4(x_rsrc, ok && k + 16 < P.K ? at + 64u : CONV_OOB);
+        };
+        auto next_step = [&](int step) {
+            if (!(step & 1)) return;
+            tap_c += BK;
+            if (tap_c >= P.Cin) { tap_c = 0; if (++tap_s == P.KW) { tap_s = 0; ++tap_r; } }
+        };
+
+        float bound = 0.f;                                  // sums below it are looked at
+        uint32_t rows[TM] = {};                             // rows that hold numbers below 2^-102
+        if (__builtin_amdgcn_ballot_w64(low < 0x1p-97f * CONV_PACK_MOST * (float)P.K)) {
+            // (weights beyond CONV_PACK_MOST are stored as they are)
+            const int pairs = ktiles / 2;
+            const __amdgpu_buffer_rsrc_t l_rsrc = make_rsrc(largest, (uint32_t)((P.N + 31) / 32 * pairs) * 4u);
+            float most = 0.f;
+            for (int k = lane; k < pairs; k += 64)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) most = fmaxf(most, buffer_load_x1(l_rsrc, (uint32_t)((n0 / 32 + wn * TN + j) * pairs + k) * 4u));
+#pragma unroll
+            for (int m = 32; m >= 1; m >>= 1) most = fmaxf(most, __shfl_xor(most, m, 64));
+            bound = 0x1p-97f * most * (float)P.K;
+        }
+        if (__builtin_amdgcn_ballot_w64(low < bound)) {
+            start_rows();
+            constexpr int U = 4 * TN;                       // steps whose loads are in flight together
+            uint32_t least[TM];                             // (a number's magnitude in bits, doubled) - 1: zero is the largest
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                least[i] = 0xFFFFFFFFu;
+                uint32_t wanted = 0;                        // rows with such sums; the others are not loaded
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    bool small = false;
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) small |= fabsf(acc[i][j][v]) < bound && in_n[j];
+                    const uint64_t lanes = __builtin_amdgcn_ballot_w64(small);
+                    wanted |= ((uint32_t)lanes ? 1u : 0u) << (8 * (v / 4) + v % 4) | (lanes >> 32 ? 16u : 0u) << (8 * (v / 4) + v % 4);
+                }
+                if (!(wanted >> l32 & 1u)) row_y[i] = INT32_MIN / 2;
+            }
+#pragma nounroll
+            for (int step = 0; step < 2 * ktiles; step += U) {
+                f32x4 x8[U][TM][2];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) request_row(x8[u][i], i, step + u);
+                    next_step(step + u);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) least[i] = min(least[i], (f2u(x8[u][i][e >> 2][e & 3]) << 1) - 1u);
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const uint64_t small = __builtin_amdgcn_ballot_w64(least[i] < (f2u(0x1p-102f) << 1) - 1u);
+                rows[i] = (uint32_t)small | (uint32_t)(small >> 32);
+            }
+        }
+        // 12544 x 2304 x 256 as an example (102 us, through the fp32 kernels 140): NaN only 456 us (1560 with single words requested one after the
+        // other), numbers of 1e-36 only 530, every third row zero 129, zeros only 163; 3x3x128x128 on 50176 rows 91, NaN only 351. Data without any
+        // of these: 0 to 2 % for the look at the sums.
+        uint32_t looked = __builtin_amdgcn_ballot_w64(!(high < __builtin_inff())) != 0;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) looked |= rows[i];
+        if (looked) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                uint32_t flags = 0;                         // bit 16 j + v: that sum
+                const uint32_t small_rows = rows[i] >> (4 * half);
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const uint32_t bits = f2u(acc[i][j][v]) << 1, at = 8 * (v / 4) + v % 4;
+                        const uint32_t small = (small_rows >> at & 1u) && bits < f2u(bound) << 1 && in_n[j];
+                        flags |= (bits >= 0xFF000000u ? 1u : small) << (16 * j + v);
+                    }
+                if (!__builtin_amdgcn_ballot_w64(flags != 0)) continue;
+                start_rows();
                 f32x4 a_next[2];
                 u32x4 b_next[TN][3];
                 auto request = [&](int step) {
-                    const int hi = hi0 + r * P.DH, wi = wi0 + s * P.DW, o = 2 * (step & 1) + half, k = (step >> 1) * BK + 4 * o;
-                    const bool ok = m < P.M && (flat_rows || ((uint32_t)hi < (uint32_t)P.H && (uint32_t)wi < (uint32_t)P.W));
-                    const uint32_t at = row + (uint32_t)(r * P.DH * P.xs_h + s * P.DW * P.xs_w + c + 4 * o) * 4u;
-                    a_next[0] = buffer_load_x4(x_rsrc, ok && k < P.K ? at : CONV_OOB);
-                    a_next[1] = buffer_load_x4(x_rsrc, ok && k + 16 < P.K ? at + 64u : CONV_OOB);
+                    request_row(a_next, i, step);
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
 #pragma unroll
                         for (int q = 0; q < 3; ++q)
                             b_next[j][q] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, b_lane, b_soff[j] + (uint32_t)step * 3072u + (uint32_t)q * 1024u, 0);
-                    if (step & 1) {
-                        c += BK;
-                        if (c >= P.Cin) { c = 0; if (++s == P.KW) { s = 0; ++r; } }
-                    }
+                    next_step(step);
                 };
-                f32x16 again[TN] = {};
+                f32x16 again[TN] = {}, total[TN] = {};      // (summed by 64 k, as rounded as in the loop above)
                 request(0);
 #pragma nounroll
                 for (int step = 0; step < 2 * ktiles; ++step) {
@@ -457,10 +589,11 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                         av[e] = a_next[e >> 2][e & 3];
 #pragma unroll
                         for (int j = 0; j < TN; ++j) {
-                            float part_e[3];
+                            uint32_t part_e[3];
 #pragma unroll
-                            for (int q = 0; q < 3; ++q) part_e[q] = u2f(e & 1 ? b_next[j][q][e >> 1] & 0xFFFF0000u : b_next[j][q][e >> 1] << 16);
-                            bv[j][e] = ((part_e[2] + part_e[1]) + part_e[0]) * sign_k;
+                            for (int q = 0; q < 3; ++q) part_e[q] = e & 1 ? b_next[j][q][e >> 1] & 0xFFFF0000u : b_next[j][q][e >> 1] << 16;
+                            const float value = ((u2f(part_e[2]) + u2f(part_e[1])) + u2f(part_e[0])) * (1.f / CONV_PACK_SCALE);
+                            bv[j][e] = (part_e[0] == CONV_PACK_RAW << 16 ? u2f(part_e[1] | part_e[2] >> 16) : value) * sign_k;
                         }
                     }
                     request(step + 1);                      // (behind the last step: zeros, or the next columns' first, unused)
@@ -468,11 +601,17 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                     for (int e = 0; e < 8; ++e)
 #pragma unroll
                         for (int j = 0; j < TN; ++j) again[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], bv[j][e], again[j], 0, 0, 0);
+                    if ((step & 3) == 3) {
+#pragma unroll
+                        for (int j = 0; j < TN; ++j)
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) { total[j][v] += again[j][v]; again[j][v] = 0.f; }
+                    }
                 }
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_isfinite(acc[i][j][v]) ? acc[i][j][v] : again[j][v];
+                    for (int v = 0; v < 16; ++v) acc[i][j][v] = flags >> (16 * j + v) & 1u ? total[j][v] : acc[i][j][v];
             }
         }
     }
@@ -579,11 +718,12 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
 #define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE)                                                                       \
     extern "C" __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void name(             \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                                   \
-        float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) { \
+        float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp,                   \
+        const float* __restrict__ largest, ConvParams P, ConvDerived D) {                                                    \
         __shared__ __attribute__((aligned(16))) u32x4 pool[24 * 32 * WGM * TM];                                              \
         __shared__ float Es[CONV_MAX_EPI * 32 * WGN * TN];                                                                   \
         __shared__ int Rs[32 * WGM * TM];                                                                                    \
-        conv_split_body<WGM, WGN, TM, TN>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);                        \
+        conv_split_body<WGM, WGN, TM, TN>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, largest, P, D);           \
     }
 // (2 x 2 waves of 64 x 64: 255 registers, two blocks per CU; 1 x 4 waves of 128 x 32, which load every column once, were 1 % slower)
 CONV_SPLIT_KERNEL(conv_gemm_split_128x128, 2, 2, 2, 2, 2)

@@ -30,3 +30,24 @@ __device__ __forceinline__ int xcd_range(int id, int n) {
     const int per = n / 8;
     return per > 0 && id < per * 8 ? (id & 7) * per + (id >> 3) : id;
 }
+// min(low, |a|, |b|), numbers that are not ones left out
+__device__ __forceinline__ float lower_of(float low, float a, float b) {
+    asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(low) : "v"(a), "v"(b));
+    return low;
+}
+// max(high, |a|, |b|), numbers that are not ones left out
+__device__ __forceinline__ float largest_of(float high, float a, float b) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(high) : "v"(a), "v"(b));
+    return high;
+}
+// the same; NaN if one of them is
+__device__ __forceinline__ float higher_of(float high, float a, float b) {
+    asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(high) : "v"(a), "v"(b));
+    return high;
+}
+// threadIdx.x of a one-dimensional block, from the wave's number
+__device__ __forceinline__ int tid_again(int wave) {
+    int lane;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+    return wave * 64 + lane;
+}

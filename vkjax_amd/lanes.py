@@ -55,9 +55,9 @@ def touched_and_written(op, launch) -> tp.Tuple[tp.Set[int], tp.Set[int]]:
     def tensors(buffers):
         return {id(b.tensor) for b in buffers if b is not None and b.tensor is not None}
     if launch.members:
-        #a batch of small launches: every member's kernel writes its first array and reads the others
+        #a batch of small launches: every member says which of its arrays it writes
         touched = tensors(b for m in launch.members for b, _ in m.buffers)
-        written = tensors(m.buffers[0][0] for m in launch.members if m.buffers)
+        written = tensors(m.buffers[i][0] for m in launch.members for i in m.written if i < len(m.buffers))
         return touched, written
     #every launch says which of its arrays it writes (results, and scratch memory that launches may share: the partial sums and
     #counters of products with a shared contraction); a convolution may store a second result from its epilogue besides
