@@ -157,3 +157,20 @@ def test_large_kernel_operands(large):
     for y in results:
         assert np.array_equal(y[:, small], exact[:, small])
         assert np.allclose(y, exact, rtol=160 * 2.0 ** -24, atol=0)           #one rounding per term
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('k', (16, 40, 64, 200))
+def test_the_largest_weight_is_found_wherever_it_is(k):
+    '''Rows of numbers whose last bits no bf16 part holds against weights of 1, one of them 2^48: its column's sums, 2^-64, would pass for right if
+    that weight were overlooked. They are the one number times 2^48, all others together are below the half of the last bit.'''
+    x = (2.0 ** -112 * (1 + (2 * rng.randint(0, 2 ** 22, size=(130, k)) + 1) * 2.0 ** -23)).astype(np.float32)
+    for at in sorted({0, 1, k // 2, k - 1}):
+        for n in (0, 31, 32, 70):
+            w = np.ones((k, 71), np.float32)
+            w[at, n] = 2.0 ** 48
+            for tile in K.CONV_SPLIT_TILES:
+                with K.overrides(conv_split=tile):
+                    y = vkjax_amd.wrap(lambda x, w: jnp.dot(x, w), frontend='minijax')(x, w)
+                assert np.array_equal(y[:, n], x[:, at] * np.float32(2.0 ** 48)), (tile, at, n)
+                assert_fp32_error(y, x, w)

@@ -50,13 +50,12 @@ struct ConvPackEntry {
 static_assert(sizeof(ConvPackEntry) == 64, "the host lays the table out with 64-byte entries");
 
 // A number beyond CONV_PACK_MOST is stored as it is: a NaN of its own kind in front, which has the column's sums computed again with fp32
-// products, and its two halves behind it. `largest`: per workgroup (32 columns, 64 k), the largest of the others.
+// products, and its two halves behind it. `largest`: per wave (32 columns, 16 k), the largest of the others.
 constexpr float CONV_PACK_SCALE = 0x1p24f, CONV_PACK_MOST = 0x1p48f;
 constexpr uint32_t CONV_PACK_RAW = 0x7FC1u;
 
 __device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const float* __restrict__ w, float* __restrict__ largest, const ConvPackParams& P,
                                                int block) {
-    __shared__ float wave_largest[4];
     const int id = block * 256 + (int)threadIdx.x, lane = id & 63, step = id >> 6, ksteps = (P.K + 63) / 64 * 4;
     const int nb = step / ksteps, s = step - nb * ksteps, o = 2 * (s & 1) + (lane >> 5), n = nb * 32 + (lane & 31);
     if (nb * 32 >= P.N) return;
@@ -99,11 +98,11 @@ __device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const fl
     }
 #pragma unroll
     for (int t = 0; t < 3; ++t) out[(size_t)step * 192 + t * 64 + lane] = part[t];
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) most = fmaxf(most, __shfl_xor(most, m, 64));
-    if (lane == 0) wave_largest[step & 3] = most;
-    __syncthreads();
-    if (threadIdx.x == 0) largest[block] = fmaxf(fmaxf(wave_largest[0], wave_largest[1]), fmaxf(wave_largest[2], wave_largest[3]));
+    // (the last lane of the wave ends with all lanes' largest: shifts by 1, 2, 4, 8 within rows of 16 lanes, then row by row)
+#define WITH_LANES(control, rows) most = fmaxf(most, u2f(__builtin_amdgcn_update_dpp(0, f2u(most), control, rows, 0xF, true)))
+    WITH_LANES(0x111, 0xF); WITH_LANES(0x112, 0xF); WITH_LANES(0x114, 0xF); WITH_LANES(0x118, 0xF); WITH_LANES(0x142, 0xA); WITH_LANES(0x143, 0xC);
+#undef WITH_LANES
+    if (lane == 63) largest[step] = most;
 }
 extern "C" __global__ __launch_bounds__(256) void conv_split_pack(u32x4* __restrict__ out, const float* __restrict__ w, float* __restrict__ largest,
                                                                   ConvPackParams P) {
@@ -496,12 +495,12 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         uint32_t rows[TM] = {};                             // rows that hold numbers below 2^-102
         if (__builtin_amdgcn_ballot_w64(low < 0x1p-97f * CONV_PACK_MOST * (float)P.K)) {
             // (weights beyond CONV_PACK_MOST are stored as they are)
-            const int pairs = ktiles / 2;
-            const __amdgpu_buffer_rsrc_t l_rsrc = make_rsrc(largest, (uint32_t)((P.N + 31) / 32 * pairs) * 4u);
+            const int steps = 2 * ktiles;
+            const __amdgpu_buffer_rsrc_t l_rsrc = make_rsrc(largest, (uint32_t)((P.N + 31) / 32 * steps) * 4u);
             float most = 0.f;
-            for (int k = lane; k < pairs; k += 64)
+            for (int k = lane; k < steps; k += 64)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) most = fmaxf(most, buffer_load_x1(l_rsrc, (uint32_t)((n0 / 32 + wn * TN + j) * pairs + k) * 4u));
+                for (int j = 0; j < TN; ++j) most = fmaxf(most, buffer_load_x1(l_rsrc, (uint32_t)((n0 / 32 + wn * TN + j) * steps + k) * 4u));
 #pragma unroll
             for (int m = 32; m >= 1; m >>= 1) most = fmaxf(most, __shfl_xor(most, m, 64));
             bound = 0x1p-97f * most * (float)P.K;

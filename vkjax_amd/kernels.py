@@ -1086,7 +1086,7 @@ class ConvSplit(tp.NamedTuple):
     slices: int
     partial: tp.Optional[Buffer] = None
     arrivals: tp.Optional[Buffer] = None
-    largest: tp.Optional[Buffer] = None          #of the packed kernel operand, per workgroup of the launch that packs it
+    largest: tp.Optional[Buffer] = None          #of the packed kernel operand, per wave of the launch that packs it
 
 
 def conv_split_tiles(split: ConvSplit, g: ConvGeometry) -> tp.Tuple[int, int]:
@@ -1100,12 +1100,12 @@ def conv_split_partial_words(split: ConvSplit, g: ConvGeometry) -> int:
     return (tiles_m * tiles_n - split.whole) * split.slices * bm * bn
 
 
-def conv_split_pack_blocks(g: ConvGeometry) -> int:
-    return _cdiv(g.N, 32) * _cdiv(g.K, 64)
-
-
 def conv_split_packed_words(g: ConvGeometry) -> int:
-    return conv_split_pack_blocks(g) * (CONV_SPLIT_PACK_BYTES // 4)
+    return _cdiv(g.N, 32) * _cdiv(g.K, 64) * (CONV_SPLIT_PACK_BYTES // 4)
+
+
+def conv_split_largest_words(g: ConvGeometry) -> int:
+    return _cdiv(g.N, 32) * _cdiv(g.K, 64) * 4
 
 
 def conv_split_plan(lhs: Buffer, g: ConvGeometry, lhs_offset: int = 0, compute_units: int = 256, sliceable: bool = True) -> tp.Optional[ConvSplit]:
@@ -1145,9 +1145,9 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry, lhs_offset: int = 0, compute_u
 
 def conv_split_pack(packed: Buffer, largest: Buffer, source: EwOperand, g: ConvGeometry) -> Launch:
     '''The kernel operand of a product, element (ky, kx, c, n) at source.offset + (ky, kx, c, n) . source.strides, taken
-    apart into three bf16 parts and laid out for the matrix cores; `largest`: its largest element per 32 columns and 64 k.'''
-    blocks = conv_split_pack_blocks(g)
-    assert packed.size == conv_split_packed_words(g) and largest.size == blocks
+    apart into three bf16 parts and laid out for the matrix cores; `largest`: its largest element per 32 columns and 16 k.'''
+    assert packed.size == conv_split_packed_words(g) and largest.size == conv_split_largest_words(g)
+    blocks = _cdiv(g.N, 32) * _cdiv(g.K, 64)
     params = _i32(g.N, g.K, g.Cin, g.KW, *source.strides)
     return Launch('conv_split_pack', (blocks, 1, 1), (BLOCK, 1, 1), [(packed, 0), (source.buffer, source.offset * 4), (largest, 0)], params,
                   bytes_moved=4 * (packed.size + g.K * g.N), written=(0, 2))

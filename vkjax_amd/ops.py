@@ -577,7 +577,7 @@ def _split_ops(bufferpool, equation, outbuf, lhs: Buffer, rhs: Buffer, geom: 'K.
     position = bufferpool.op_counter
     bufferpool.op_counter -= 1                  #the packed operand lives at the equation's own position
     packed  = bufferpool.new_temporary(np.uint32, (K.conv_split_packed_words(geom),))
-    largest = bufferpool.new_temporary(np.float32, (K.conv_split_pack_blocks(geom),))
+    largest = bufferpool.new_temporary(np.float32, (K.conv_split_largest_words(geom),))
     bufferpool.op_counter = position
     geom   = geom._replace(split=plan._replace(largest=largest))
     source = EwOperand(rhs, rhs_offset, tuple(geom.ws))
