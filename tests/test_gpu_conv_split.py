@@ -66,8 +66,7 @@ def test_tile_edges_and_slices(tile, desc, xs, ks, f):
 @pytest.mark.gpu
 @pytest.mark.parametrize('slices', (1, 3))
 def test_epilogues_and_second_results(slices):
-    '''Batch norm, residual and ReLU in the launch, a centred result stored beside it, and an epilogue the kernels do not apply
-    (it stays a launch of its own).'''
+    '''Batch norm, residual and ReLU in the launch, a centred result stored beside it, and an epilogue in another order.'''
     x, k, r = ints([2, 14, 13, 64]), ints([3, 3, 64, 72], -3, 4), ints([2, 14, 13, 72], -50, 50)
     mean, scale, beta = ints([72]), ints([72], 1, 4), ints([72], -9, 9)
     def bn_residual(x, k, mean, scale, beta, r):
@@ -81,6 +80,38 @@ def test_epilogues_and_second_results(slices):
         with K.overrides(conv_split=True, conv_split_slices=slices):
             _, _, fn = check_against_oracle(f, [x, k, mean, scale, beta, r], exact=True)
         assert len(split_kernels(fn)) == 1 and split_kernels(fn)[0].startswith('conv_gemm_split_')
+
+
+#epilogues other than (- vector, * vector, + vector, + full tensor, max with a scalar) in this order
+STEPS = {'relu6': lambda y, r, v: jnp.minimum(nn.relu(y), 6.0), 'scalar': lambda y, r, v: 0.5 - (y + 2.0) * 0.25, 'quotient': lambda y, r, v: y / v,
+         'reciprocal': lambda y, r, v: v / (y * y + 1.0), 'bias, scale': lambda y, r, v: (y + v) * v, 'behind the relu': lambda y, r, v: nn.relu(y) + r,
+         'residual, bias': lambda y, r, v: y + r + v, 'difference': lambda y, r, v: y - r, 'difference, left': lambda y, r, v: r - y,
+         'two residuals': lambda y, r, v: jnp.maximum((y + r) * r, v - r), 'six steps': lambda y, r, v: (((y + v) * v - r) * 0.5 + r) * v}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('tile', list(K.CONV_SPLIT_TILES))
+@pytest.mark.parametrize('name', list(STEPS))
+def test_other_epilogues(name, tile):
+    x, k, r = ints([2, 14, 13, 64]), ints([3, 3, 64, 72], -3, 4), ints([2, 14, 13, 72], -50, 50)
+    v = 2.0 ** ints([72], -2, 3)
+    for slices in (1, 3):
+        print(f'case: {name}, tile {tile}, {slices} slices', flush=True)
+        with K.overrides(conv_split=tile, conv_split_slices=slices):
+            #(a quotient by more than a power of two is rounded, by both sides to the nearest)
+            check_against_oracle(lambda x, k, r, v: STEPS[name](conv()(x, k), r, v), [x, k, r, v], exact=True)
+
+
+@pytest.mark.parametrize('name', list(STEPS))
+def test_other_epilogues_are_part_of_the_product(name):
+    '''Plan only: as behind the fp32 kernels, no launch besides the product and the packing for those that are one chain behind it.'''
+    args = [np.zeros(s, np.float32) for s in ((8, 28, 28, 128), (1, 1, 128, 512), (8, 28, 28, 512), (512,))]
+    f = lambda x, k, r, v: STEPS[name](conv()(x, k), r, v)
+    def launches(choice):
+        with K.overrides(conv_split=choice):
+            return [l.kernel for l in JaxprInterpreter(mj.make_jaxpr(f)(*args), plan_only=True).launches]
+    here, fp32 = launches(True), launches(False)
+    assert any(k.startswith('conv_gemm_split') for k in here) and len(here) == len(fp32) + 1, (here, fp32)
 
 
 @pytest.mark.gpu

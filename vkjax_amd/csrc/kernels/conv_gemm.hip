@@ -135,6 +135,26 @@ __device__ __forceinline__ float conv_derived_value(const float (&in)[CONV_MAX_D
     return v;
 }
 
+// one step of an epilogue on a sub-tile's 16 values of a lane, operand(v) beside them; code: opcode * 2 + (operand on the left)
+template <class Operand>
+__device__ __forceinline__ void conv_epilogue_step(uint32_t code, float (&y)[16], Operand&& operand) {
+#define EPI_LOOP(expr) _Pragma("unroll") for (int v = 0; v < 16; ++v) { const float a = y[v], o = operand(v); y[v] = (expr); }
+    switch (code) {
+        case CEW_ADD_F * 2: case CEW_ADD_F * 2 + 1: EPI_LOOP(a + o) break;
+        case CEW_MUL_F * 2: case CEW_MUL_F * 2 + 1: EPI_LOOP(a * o) break;
+        case CEW_SUB_F * 2:     EPI_LOOP(a - o) break;
+        case CEW_SUB_F * 2 + 1: EPI_LOOP(o - a) break;
+        case CEW_DIV_F * 2:     EPI_LOOP(a / o) break;
+        case CEW_DIV_F * 2 + 1: EPI_LOOP(o / a) break;
+        case CEW_MAX_F * 2:     EPI_LOOP((a > o || a != a) ? a : o) break;
+        case CEW_MAX_F * 2 + 1: EPI_LOOP((o > a || o != o) ? o : a) break;
+        case CEW_MIN_F * 2:     EPI_LOOP((a < o || a != a) ? a : o) break;
+        case CEW_MIN_F * 2 + 1: EPI_LOOP((o < a || o != o) ? o : a) break;
+        default: __builtin_unreachable();                    // the host fuses no other operation
+    }
+#undef EPI_LOOP
+}
+
 // LEAN: the variant for the common case, with the rarely needed paths compiled out (they cost
 // registers, and with them resident waves, even when not taken): both operands on the 16-byte
 // path, k tiles that never straddle kernel taps, a row-major result, an epilogue that fits the
@@ -715,23 +735,6 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
                 }
         } else if constexpr (!LEAN) {
             // any other chain: one uniform branch per step and sub-tile, not per element
-            auto apply = [&](uint32_t code, float (&y)[16], auto&& operand) {
-#define EPI_LOOP(expr) _Pragma("unroll") for (int v = 0; v < 16; ++v) { const float a = y[v], o = operand(v); y[v] = (expr); }
-                switch (code) {                                          // bit0: operand on the left
-                    case CEW_ADD_F * 2: case CEW_ADD_F * 2 + 1: EPI_LOOP(a + o) break;
-                    case CEW_MUL_F * 2: case CEW_MUL_F * 2 + 1: EPI_LOOP(a * o) break;
-                    case CEW_SUB_F * 2:     EPI_LOOP(a - o) break;
-                    case CEW_SUB_F * 2 + 1: EPI_LOOP(o - a) break;
-                    case CEW_DIV_F * 2:     EPI_LOOP(a / o) break;
-                    case CEW_DIV_F * 2 + 1: EPI_LOOP(o / a) break;
-                    case CEW_MAX_F * 2:     EPI_LOOP((a > o || a != a) ? a : o) break;
-                    case CEW_MAX_F * 2 + 1: EPI_LOOP((o > a || o != o) ? o : a) break;
-                    case CEW_MIN_F * 2:     EPI_LOOP((a < o || a != a) ? a : o) break;
-                    case CEW_MIN_F * 2 + 1: EPI_LOOP((o < a || o != o) ? o : a) break;
-                    default: __builtin_unreachable();                    // the host fuses no other operation
-                }
-#undef EPI_LOOP
-            };
             // The step loop stays rolled: one copy of the step code keeps the kernel small.
 #pragma nounroll
             for (int e = 0; e < nepi; ++e) {
@@ -743,7 +746,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
                     for (int j = 0; j < TN; ++j) {
                         if (kind == 3) {
                             if (PREFETCH_FULL && e == first_full) {
-                                apply(code, c[i][j], [&](int v) { return full[PREFETCH_FULL ? i : 0][PREFETCH_FULL ? j : 0][v]; });
+                                conv_epilogue_step(code, c[i][j], [&](int v) { return full[PREFETCH_FULL ? i : 0][PREFETCH_FULL ? j : 0][v]; });
                             } else {
                                 float ov[16];
                                 // (the pointer table is re-read from the argument block: indexing the by-value
@@ -752,12 +755,12 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
                                     reinterpret_cast<const char*>(__builtin_amdgcn_kernarg_segment_ptr()) + 24);
                                 const __amdgpu_buffer_rsrc_t g_rsrc = make_rsrc(table[e], P.out_bytes);
                                 sub_tile(m0, i, j, [&](int v, uint32_t vo, uint32_t so) { ov[v] = buffer_load_x1(g_rsrc, vo, so); });
-                                apply(code, c[i][j], [&](int v) { return ov[v]; });
+                                conv_epilogue_step(code, c[i][j], [&](int v) { return ov[v]; });
                             }
                         } else {
                             // one value per column: used straight from its register
                             const float o1 = Es[e * BN + (wn * TN + j) * 32 + l32];
-                            apply(code, c[i][j], [&](int) { return o1; });
+                            conv_epilogue_step(code, c[i][j], [&](int) { return o1; });
                         }
                     }
             }

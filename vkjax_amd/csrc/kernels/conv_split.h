@@ -141,7 +141,8 @@ extern "C" __global__ __launch_bounds__(256) void conv_split_pack_layers(const C
 // last at the tile's counter adds all slices in their order and applies the epilogue: no block waits for another. The
 // counters are left at zero for the next launch.
 
-template <int WGM, int WGN, int TM, int TN>
+// STEPS: an epilogue other than the straight-line one, step by step (ReLU6, a scalar or a vector in another place, a residual that is subtracted).
+template <int WGM, int WGN, int TM, int TN, bool STEPS>
 __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float* __restrict__ Es, int* __restrict__ Rs,
                                                 float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                                                 float* __restrict__ partial, uint32_t* __restrict__ arrivals, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
@@ -641,6 +642,34 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
             }
         }
     };
+    if constexpr (STEPS) {
+        // (the pointer table is read from the argument block: indexing the by-value argument with a run-time value would make the compiler copy
+        // it to scratch memory)
+        const float* const* table = reinterpret_cast<const float* const*>(reinterpret_cast<const char*>(__builtin_amdgcn_kernarg_segment_ptr()) + 40);
+#pragma nounroll
+        for (int e = 0; e < nepi; ++e) {
+            const uint32_t kind = step_desc(e) >> 8, code = step_desc(e) & 255u;
+            const __amdgpu_buffer_rsrc_t e_rsrc = make_rsrc(table[e], kind == 3 ? P.out_bytes : 0u);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    if (kind == 3) {
+                        float ov[16];
+                        sub_tile(i, j, [&](int v, uint32_t vo, uint32_t so) { ov[v] = buffer_load_x1_nt(e_rsrc, vo, so); });
+                        conv_epilogue_step(code, acc[i][j], [&](int v) { return ov[v]; });
+                    } else {
+                        const float o = Es[e * BN + (wn * TN + j) * 32 + l32];
+                        conv_epilogue_step(code, acc[i][j], [&](int) { return o; });
+                    }
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) sub_tile(i, j, [&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(acc[i][j][v], o_rsrc, vo, so); });
+        return;
+    }
     const float* full_ptr = epi.p[0];
 #pragma unroll
     for (int t = 1; t < CONV_MAX_EPI; ++t) full_ptr = epi_first_full == t ? epi.p[t] : full_ptr;
@@ -714,7 +743,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         }
 }
 
-#define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE)                                                                       \
+#define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE, STEPS)                                                                \
     extern "C" __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void name(             \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                                   \
         float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp,                   \
@@ -722,9 +751,13 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         __shared__ __attribute__((aligned(16))) u32x4 pool[24 * 32 * WGM * TM];                                              \
         __shared__ float Es[CONV_MAX_EPI * 32 * WGN * TN];                                                                   \
         __shared__ int Rs[32 * WGM * TM];                                                                                    \
-        conv_split_body<WGM, WGN, TM, TN>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, largest, P, D);           \
+        conv_split_body<WGM, WGN, TM, TN, STEPS>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, largest, P, D);    \
     }
+// _steps: 50176 x 128 x 512 with a ReLU6 65 us, with a scalar 57, with `relu(y) + r` 76 (each as launches of its own behind the product: 83, 82, 94;
+// in the fp32 kernels 70, 68, 73).
 // (2 x 2 waves of 64 x 64: 255 registers, two blocks per CU; 1 x 4 waves of 128 x 32, which load every column once, were 1 % slower)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x128, 2, 2, 2, 2, 2)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128, 2, 2, 2, 2, 2, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128_steps, 2, 2, 2, 2, 2, true)
 // for at most 64 columns, or where the smaller tile divides the rows better among the CUs: three blocks per CU
-CONV_SPLIT_KERNEL(conv_gemm_split_128x64, 2, 2, 2, 1, 3)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64, 2, 2, 2, 1, 3, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_steps, 2, 2, 2, 1, 3, true)

@@ -290,8 +290,6 @@ def fuse_ops(all_ops, bufferpool, outvars):
                         continue
                     if K.conv_is_dense_rows(lhs, geom) and not K.dense_rows_epilogue_supported(list(epilogue) + extra):
                         continue                                  #the chain stays a launch of its own
-                    if geom.split is not None and not K.conv_split_epilogue_supported(list(epilogue) + extra):
-                        continue                                  #likewise
                     tap_at = [k for k, e in enumerate(epilogue) if e.op == K.CONV_TAP]
                     if tap_at and not K.conv_tap_supported(epilogue[:tap_at[0]], list(epilogue[tap_at[0] + 1:]) + extra):
                         continue

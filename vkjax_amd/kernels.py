@@ -1175,8 +1175,9 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
             raise ValueError('a second result at this point of the epilogue is not supported')
         flags |= (tap_position + 1) << 12
     slots = (8 if epilogue[0].operand is not None else 0) | (2 if epilogue[2].operand is not None else 0) if masked else _epilogue_template_slots(epilogue)
-    if epilogue and not slots and not masked:
-        raise ValueError('these kernels apply the straight-line epilogue only')
+    steps = bool(epilogue) and not slots and not masked           #any other chain: the kernel that walks through its steps
+    if steps and taps:
+        raise ValueError('a second result at this point of the epilogue is not supported')
     for name, extent in (('lhs', lhs.size), ('packed rhs', packed.size), ('out', out.size)):
         if extent * 4 >= 2**31:
             raise NotImplementedError(f'conv/dot {name} operand of {extent * 4} bytes exceeds the 2 GiB the kernel addresses')
@@ -1198,7 +1199,7 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
         operand_slots[-1] = (taps[0][1], 0)
         nbytes += 4 * taps[0][1].size
     scratch = [(split.partial, 0), (split.arrivals, 0)] if shared else [(None, 0), (None, 0)]
-    return Launch(f'conv_gemm_split_{split.tile}', (split.whole + shared * split.slices, 1, 1), (256, 1, 1),
+    return Launch(f'conv_gemm_split_{split.tile}' + ('_steps' if steps else ''), (split.whole + shared * split.slices, 1, 1), (256, 1, 1),
                   [(out, out_offset * 4), (lhs, lhs_offset * 4), (packed, 0)] + scratch + operand_slots + derived_ptrs + [(split.largest, 0)],
                   params + derived_desc, bytes_moved=nbytes, flops=2 * M * N * K,
                   written=(0, 3, 4) if shared else (0,), scratch=(3, 4) if shared else ())
@@ -1221,13 +1222,6 @@ def conv_masked_epilogue(epilogue: tp.Sequence[ConvEpilogueStep]) -> tp.Optional
         return None
     limit, otherwise = (ConvEpilogueStep(EW['NOP'], 1, b) for b in mask.bounds)
     return [full, mask, vector, limit, otherwise]
-
-
-def conv_split_epilogue_supported(epilogue: tp.Sequence[ConvEpilogueStep]) -> bool:
-    '''The kernels on the bf16 matrix cores apply the straight-line epilogue. A fusion pass leaves any other chain a launch of
-    its own instead of handing the product to a kernel that adds in another order than in the unfused program.'''
-    real = [e for e in epilogue if e.op != CONV_TAP]
-    return not real or _epilogue_template_slots(real) != 0
 
 
 # --------------------------------------------------------------------------- reductions
