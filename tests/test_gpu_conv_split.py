@@ -114,6 +114,49 @@ def test_other_epilogues_are_part_of_the_product(name):
     assert any(k.startswith('conv_gemm_split') for k in here) and len(here) == len(fp32) + 1, (here, fp32)
 
 
+LAYOUTS = ('NCHW', 'HWNC', 'CHWN', 'NHWC')
+
+
+def conv_laid_out(layout):
+    return lambda x, k: lax.conv_general_dilated(x, k, (1, 1), 'SAME', dimension_numbers=('NHWC', 'HWIO', layout))
+
+
+def laid_out(layout):
+    per_feature = [72 if d == 'C' else 1 for d in layout]
+    return lambda x, k, r, v: nn.relu((conv_laid_out(layout)(x, k) - v.reshape(per_feature)) + r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('tile', list(K.CONV_SPLIT_TILES))
+@pytest.mark.parametrize('layout', LAYOUTS)
+def test_results_in_other_layouts(layout, tile):
+    size = dict(N=3, H=9, W=11, C=72)
+    args = [ints([3, 9, 11, 32]), ints([3, 3, 32, 72], -3, 4), ints([size[d] for d in layout], -50, 50), ints([72])]
+    for slices in (1, 3):
+        print(f'case: {layout}, tile {tile}, {slices} slices', flush=True)
+        with K.overrides(conv_split=tile, conv_split_slices=slices):
+            _, _, fn = check_against_oracle(laid_out(layout), args, exact=True)
+        assert len(split_kernels(fn)) == 1 and split_kernels(fn)[0].startswith('conv_gemm_split')
+        #the backward pass of a ReLU: a second result, both laid out like the activation
+        def masked(x, k, r, v):
+            m = jnp.where(r > 0, conv_laid_out(layout)(x, k), 0.0)
+            return m, m * v.reshape([72 if d == 'C' else 1 for d in layout])
+        with K.overrides(conv_split=tile, conv_split_slices=slices):
+            check_against_oracle(masked, args, exact=True)
+
+
+@pytest.mark.parametrize('layout', LAYOUTS)
+def test_epilogues_join_products_of_every_layout(layout):
+    '''Plan only: the same launches behind the product as with the fp32 kernels.'''
+    size = dict(N=8, H=28, W=28, C=72)
+    args = [np.zeros(s, np.float32) for s in ([8, 28, 28, 256], [3, 3, 256, 72], [size[d] for d in layout], [72])]
+    def launches(choice):
+        with K.overrides(conv_split=choice):
+            return [l.kernel for l in JaxprInterpreter(mj.make_jaxpr(laid_out(layout))(*args), plan_only=True).launches]
+    here, fp32 = launches(True), launches(False)
+    assert any(k.startswith('conv_gemm_split') for k in here) and len(here) == len(fp32) + 1, (here, fp32)
+
+
 @pytest.mark.gpu
 def test_gradients_pack_transposed_and_reversed_kernels():
     '''Input gradients of strided and unit-stride convolutions: the kernel operand is packed straight from the forward

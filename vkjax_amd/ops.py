@@ -582,8 +582,8 @@ def _split_ops(bufferpool, equation, outbuf, lhs: Buffer, rhs: Buffer, geom: 'K.
     geom   = geom._replace(split=plan._replace(largest=largest))
     source = EwOperand(rhs, rhs_offset, tuple(geom.ws))
     pack   = Op(equation, launch=K.conv_split_pack(packed, largest, source, geom), meta=('conv_pack', packed, source, geom))
-    if part_at is not None or geom.os[1:] != (geom.Wo * geom.N, geom.N, 1) and geom.Ho * geom.Wo > 1:
-        return [pack, Op(equation, launch=K.conv_product(outbuf, lhs, packed, geom, out_offset=part_at or 0))]
+    if part_at is not None:
+        return [pack, Op(equation, launch=K.conv_product(outbuf, lhs, packed, geom, out_offset=part_at))]
     return [pack, Op(equation, conv=(outbuf, lhs, packed, geom, []))]
 
 
