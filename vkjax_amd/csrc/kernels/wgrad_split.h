@@ -23,6 +23,11 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // 64-bit sums 0.3 to 0.65 times that of the fp32 products (3136 to 50176 pixels).
 // Sums: the twelve products of a k tile are chained from zero and added to the accumulators by fp32 operations, G's sign changed in
 // every other k tile (the matrix cores cut sums off, see conv_split.h).
+// Scale: both operands are multiplied by 2^24 before they are taken apart and the sums by 2^-48, so the smallest numbers have all their bits
+// (a bf16 part of a number below 2^-102 would not). It costs 1 to 2 % of the kernel. (Looking behind the loop for sums that such numbers could matter
+// to, as conv_split.h does, costs as much for the columns' largest numbers and far more where it finds some: sums of nothing but zeros are
+// everywhere behind a ReLU, ResNet-50's training step took 17.7 ms instead of 12.6.)
+constexpr float WGRAD_SCALE = 0x1p24f;
 template <int TM, int TN, bool VEC_A, bool VEC_B>
 __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2* __restrict__ table, float* __restrict__ out,
                                                  const float* __restrict__ x, const float* __restrict__ g, const WgradParams& P, const WgradSplitParams& Q) {
@@ -126,21 +131,13 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
     };
     u32x4* const to = (is_a ? As : Bs) + oct * (is_a ? BM : BN);
     const int part_step = 4 * (is_a ? BM : BN);
-    // The largest number of each of this thread's columns, for the check behind the loop; it costs 2 to 4 % of the kernel (12544 pixels, 2304 x
-    // 256: 90 -> 93 us).
-    float most[4] = {0.f, 0.f, 0.f, 0.f};
-    auto park_tile = [&](bool negate) {
+    auto park_tile = [&](bool odd) {
         if (!is_a && !is_b) return;
+        const float scale = odd && is_b ? -WGRAD_SCALE : WGRAD_SCALE;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int q = 0; q < 8; ++q)
 #pragma unroll
-            for (int q = 0; q < 8; q += 2) most[e] = largest_of(most[e], raw[q][e], raw[q + 1][e]);
-        if (negate && is_b) {
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) raw[q][e] = -raw[q][e];
-        }
+            for (int e = 0; e < 4; ++e) raw[q][e] *= scale;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             u32x4* const slot = to + e * cols4 + (cg ^ ((e * 8) & (cols4 - 1)));
@@ -179,7 +176,7 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
         park_tile(kt & 1);
         __syncthreads();
         if (kt + 1 < nk) load_tile(kt + 1);
-        const float sign = kt & 1 ? -1.f : 1.f;
+        const float sign = kt & 1 ? -1.f / (WGRAD_SCALE * WGRAD_SCALE) : 1.f / (WGRAD_SCALE * WGRAD_SCALE);
         bf16x8 af[TM][2][3];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -208,50 +205,20 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
         __syncthreads();
     }
 
-    // Sums that are computed again with fp32 products; the others beside them stay as they are.
-    //   - Sums that are not finite (an operand that is infinite, not a number, or beyond the largest bf16).
-    //   - Numbers below 2^-102 lose up to 2^-125 each, a sum up to 2^-125 K times what they meet: less than 2^-27 of a sum from 2^-97 K
-    //     times the largest numbers of its two columns up; what the matrix cores may lose of products below 2^-126, less than that of a sum
-    //     from 2^-102 K up. Of smaller sums whose columns are not zeros the columns are looked through for such numbers.
-    const int columns = BM + BN;
-    float* const most_of = reinterpret_cast<float*>(lds);         // [4 octets of pixels][columns of X, then of G]
-    if (is_a || is_b) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) most_of[oct * columns + (is_a ? 0 : BM) + 4 * cg + e] = most[e];
-    }
-    __syncthreads();
-    const float terms = (float)max(kend - kbeg, 1);
-    float high = 0.f, low = __builtin_inff(), operand = 0.f;
+    // Sums that are not finite (an operand that is infinite, not a number, or beyond 2^104; a sum beyond 2^80): again, with fp32 products. The
+    // finite ones beside them stay as they are.
+    float high = 0.f;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; v += 2) { high = higher_of(high, acc[i][j][v], acc[i][j][v + 1]); low = lower_of(low, acc[i][j][v], acc[i][j][v + 1]); }
-    for (int c = lane; c < columns; c += 64) {                    // (4 octets side by side: any order does)
-        const f32x4 q = reinterpret_cast<const f32x4*>(most_of)[c];
-        operand = fmaxf(fmaxf(operand, fmaxf(q.x, q.y)), fmaxf(q.z, q.w));
-    }
-    const uint32_t not_finite = __builtin_amdgcn_ballot_w64(!(high < __builtin_inff())) != 0;
-    if (not_finite || __builtin_amdgcn_ballot_w64(low < 0x1p-49f * terms || operand > 0x1p48f)) {
-        auto most_at = [&](int c) { return fmaxf(fmaxf(most_of[c], most_of[columns + c]), fmaxf(most_of[2 * columns + c], most_of[3 * columns + c])); };
-        uint32_t flags[TN];                                       // bit 16 i + v: that sum
-        bool tiny = false;
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const float most_g = most_at(BM + (wn * TN + j) * 32 + 4 * (l32 & 7) + (l32 >> 3));
-            flags[j] = 0;
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const float most_x = most_at((wm * TM + i) * 32 + 4 * (4 * half + v % 4) + v / 4);
-                    const bool  small  = fabsf(acc[i][j][v]) < (0x1p-97f * (most_x + most_g) + 0x1p-102f) * terms && most_x > 0.f && most_g > 0.f;
-                    flags[j] |= (uint32_t)small << (16 * i + v);
-                    tiny |= small;
-                }
-        }
-        int dy[TM], dx[TM], n[TN];
+            for (int v = 0; v < 16; v += 2) high = higher_of(high, acc[i][j][v], acc[i][j][v + 1]);
+    if (__builtin_amdgcn_ballot_w64(!(high < __builtin_inff()))) {
+        // Steps of eight pixels per half of the wave, the next step's words requested before this one's products. 12544 pixels, 2304 x 256 with NaN
+        // only: 465 us (95 without; 868 with the words requested one after the other), through the fp32 kernels 160.
+        constexpr int U = 8;
+        int dy[TM], dx[TM];
         uint32_t x_at[TM];
         bool in_m[TM];
 #pragma unroll
@@ -263,73 +230,29 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
             in_m[i] = m < P.M;
         }
 #pragma unroll
-        for (int j = 0; j < TN; ++j) n[j] = n0 + (wn * TN + j) * 32 + 4 * (l32 & 7) + (l32 >> 3);
-        auto x_word = [&](int p, int i) {
-            const int img = magic_div(p, P.howo_magic, P.howo_shift), r = p - img * (P.Ho * P.Wo);
-            const int ho  = magic_div(r, P.wo_magic, P.wo_shift), y0 = ho * P.SH, x0 = (r - ho * P.Wo) * P.SW;
-            const bool ok = p < kend && in_m[i] && (uint32_t)(y0 + dy[i]) < (uint32_t)P.H && (uint32_t)(x0 + dx[i]) < (uint32_t)P.W;
-            return buffer_load_x1(x_rsrc, ok ? (uint32_t)(((img * P.H + y0) * P.W + x0) * P.C) * 4u + x_at[i] : WG_OOB);
-        };
-        auto g_word = [&](int p, int j) { return buffer_load_x1(g_rsrc, p < kend && n[j] < P.N ? (uint32_t)(p * P.N + n[j]) * 4u : WG_OOB); };
-        constexpr int U = 8;                                      // pixels per half of the wave whose words are requested together
-        if (__builtin_amdgcn_ballot_w64(tiny)) {
-            uint32_t least_x[TM], least_g[TN];                    // (a number's magnitude in bits, doubled) - 1: zero is the largest
-#pragma unroll
-            for (int i = 0; i < TM; ++i) least_x[i] = 0xFFFFFFFFu;
-#pragma unroll
-            for (int j = 0; j < TN; ++j) least_g[j] = 0xFFFFFFFFu;
-#pragma nounroll
-            for (int p0 = kbeg; p0 < kend; p0 += 2 * U) {
-                float xv[TM][U], gv[TN][U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) xv[i][u] = x_word(p0 + 2 * u + half, i);
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) gv[j][u] = g_word(p0 + 2 * u + half, j);
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) least_x[i] = min(least_x[i], (f2u(xv[i][u]) << 1) - 1u);
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) least_g[j] = min(least_g[j], (f2u(gv[j][u]) << 1) - 1u);
-                }
-            }
-            auto number = [](uint32_t least) { return u2f((min(least, (uint32_t)__shfl_xor((int)least, 32, 64)) + 1u) >> 1); };
-            float x_least[TM];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) x_least[i] = number(least_x[i]);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const float g_least = number(least_g[j]);
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const float least = __shfl(x_least[i], 8 * (v / 4) + 4 * half + v % 4, 64);
-                        const bool  lossy = least < 0x1p-102f || g_least < 0x1p-102f || least * g_least < 0x1p-102f;
-                        flags[j] &= ~((uint32_t)!lossy << (16 * i + v));
-                    }
-            }
-        }
-        // 12544 pixels, 2304 x 256 as an example (97 us, through the fp32 kernels 168): NaN only 405 us (868 with the words requested one after the
-        // other), numbers of 1e-36 only 546.
-#pragma unroll
         for (int j = 0; j < TN; ++j) {
+            bool any = false;
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) flags[j] |= (uint32_t)!__builtin_isfinite(acc[i][j][v]) << (16 * i + v);
-            if (!__builtin_amdgcn_ballot_w64(flags[j] != 0)) continue;
+                for (int v = 0; v < 16; ++v) any |= !__builtin_isfinite(acc[i][j][v]);
+            if (!__builtin_amdgcn_ballot_w64(any)) continue;
+            const int n = n0 + (wn * TN + j) * 32 + 4 * (l32 & 7) + (l32 >> 3);
             f32x16 again[TM] = {}, total[TM] = {};                // (summed by 64 pixels)
             float x_next[TM][U], g_next[U];
             auto request = [&](int p0) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
+                    const int p   = p0 + 2 * u + half;
+                    const int img = magic_div(p, P.howo_magic, P.howo_shift), r = p - img * (P.Ho * P.Wo);
+                    const int ho  = magic_div(r, P.wo_magic, P.wo_shift), y0 = ho * P.SH, x0 = (r - ho * P.Wo) * P.SW;
+                    const uint32_t px = (uint32_t)(((img * P.H + y0) * P.W + x0) * P.C) * 4u;
 #pragma unroll
-                    for (int i = 0; i < TM; ++i) x_next[i][u] = x_word(p0 + 2 * u + half, i);
-                    g_next[u] = g_word(p0 + 2 * u + half, j);
+                    for (int i = 0; i < TM; ++i) {
+                        const bool ok = p < kend && in_m[i] && (uint32_t)(y0 + dy[i]) < (uint32_t)P.H && (uint32_t)(x0 + dx[i]) < (uint32_t)P.W;
+                        x_next[i][u] = buffer_load_x1(x_rsrc, ok ? px + x_at[i] : WG_OOB);
+                    }
+                    g_next[u] = buffer_load_x1(g_rsrc, p < kend && n < P.N ? (uint32_t)(p * P.N + n) * 4u : WG_OOB);
                 }
             };
             request(kbeg);
@@ -357,7 +280,7 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = flags[j] >> (16 * i + v) & 1u ? total[i][v] : acc[i][j][v];
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_isfinite(acc[i][j][v]) ? acc[i][j][v] : total[i][v];
         }
     }
     float* const result = out + (size_t)slice * P.M * P.N;
