@@ -161,9 +161,9 @@ def test_large_kernel_operands(large):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('k', (16, 40, 64, 200))
-def test_the_largest_weight_is_found_wherever_it_is(k):
-    '''Rows of numbers whose last bits no bf16 part holds against weights of 1, one of them 2^48: its column's sums, 2^-64, would pass for right if
-    that weight were overlooked. They are the one number times 2^48, all others together are below the half of the last bit.'''
+def test_last_bits_of_small_rows(k):
+    '''Rows of numbers whose last bits no bf16 part holds unless it is scaled, against weights of 1, one of them 2^48: that column's sums are the one
+    number times 2^48, all others together are below the half of the last bit.'''
     x = (2.0 ** -112 * (1 + (2 * rng.randint(0, 2 ** 22, size=(130, k)) + 1) * 2.0 ** -23)).astype(np.float32)
     for at in sorted({0, 1, k // 2, k - 1}):
         for n in (0, 31, 32, 70):

@@ -6,13 +6,11 @@
 // products hi.hi, hi.mid, mid.hi, hi.lo, mid.mid, lo.hi, each exact in fp32 and added in fp32 accumulators; the three that are
 // left out are below 2^-24 of the product together, the rounding of an fp32 accumulation. The matrix cores run bf16 sixteen
 // times as fast as fp32, so six products instead of one are still 2.6 times as fast at peak.
-//   - a number below 2^-102 has parts that a bf16 holds with fewer bits, or not at all (an absolute error under 2^-125). The kernel operand is
-//     multiplied by 2^24 before it is taken apart, and the sums by 2^-24, so its smallest numbers have all their bits; of the rows' operand
-//     such numbers matter only to sums that are themselves below 2^-97 K times the largest weight. Those, if they exist, and if their
-//     row holds such a number, are computed again with fp32 products (below);
-//   - operands that are infinite, NaN or beyond the largest bf16 (3.39e38) leave sums that are not finite, because a part that is
-//     infinite meets parts that are zero: a wave whose results are not all finite computes those that are not again with
-//     v_mfma_f32_32x32x2_f32 and fp32 operands, so that such results are what fp32 products give.
+//   - a number below 2^-102 has parts that a bf16 holds with fewer bits, or not at all: both operands are multiplied by 2^24 before they are
+//     taken apart, and the sums by 2^-48, so the smallest numbers have all their bits (which costs 1 to 2 % of the kernel);
+//   - operands that are infinite, NaN or beyond 2^104 (then beyond the largest bf16) leave sums that are not finite, because a part that is
+//     infinite meets parts that are zero, and so do sums beyond 2^80: a wave whose results are not all finite computes those that are not again
+//     with v_mfma_f32_32x32x2_f32 and fp32 operands, so that such results are what fp32 products give.
 // Measured against 64-bit sums (4096 x K x 128, normal data): an error of 0.76, 0.56 and 0.30 times that of
 // v_mfma_f32_32x32x2_f32 at K = 64, 576 and 2304 (which rounds after every second product, this after every sixteenth). Sums of which less than
 // a fifth of the terms are not zero are further off than those: 1.3 times at 16 of 512, 1.4 times at one (which is cut off, not rounded).
@@ -44,18 +42,16 @@ struct ConvPackEntry {
     uint32_t first_block, pad;
     u32x4*       out;
     const float* w;
-    float*       largest;
     ConvPackParams P;
 };
-static_assert(sizeof(ConvPackEntry) == 64, "the host lays the table out with 64-byte entries");
+static_assert(sizeof(ConvPackEntry) == 56, "the host lays the table out with 56-byte entries");
 
-// A number beyond CONV_PACK_MOST is stored as it is: a NaN of its own kind in front, which has the column's sums computed again with fp32
-// products, and its two halves behind it. `largest`: per wave (32 columns, 16 k), the largest of the others.
-constexpr float CONV_PACK_SCALE = 0x1p24f, CONV_PACK_MOST = 0x1p48f;
+// A number that the scale takes beyond the largest bf16 is stored as it is: a NaN of its own kind in front, which has the column's sums computed
+// again with fp32 products, and its two halves behind it.
+constexpr float CONV_SPLIT_SCALE = 0x1p24f;
 constexpr uint32_t CONV_PACK_RAW = 0x7FC1u;
 
-__device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const float* __restrict__ w, float* __restrict__ largest, const ConvPackParams& P,
-                                               int block) {
+__device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const float* __restrict__ w, const ConvPackParams& P, int block) {
     const int id = block * 256 + (int)threadIdx.x, lane = id & 63, step = id >> 6, ksteps = (P.K + 63) / 64 * 4;
     const int nb = step / ksteps, s = step - nb * ksteps, o = 2 * (s & 1) + (lane >> 5), n = nb * 32 + (lane & 31);
     if (nb * 32 >= P.N) return;
@@ -72,10 +68,9 @@ __device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const fl
         }
     }
     u32x4 part[3];
-    float most = 0.f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        float rest[2] = {x[2 * q] * CONV_PACK_SCALE, x[2 * q + 1] * CONV_PACK_SCALE};
+        float rest[2] = {x[2 * q] * CONV_SPLIT_SCALE, x[2 * q + 1] * CONV_SPLIT_SCALE};
         uint32_t v[3];
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
@@ -86,7 +81,7 @@ __device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const fl
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const uint32_t shift = 16 * h, bits = f2u(x[2 * q + h]), keep = h ? 0xFFFFu : 0xFFFF0000u;
-            if (fabsf(x[2 * q + h]) <= CONV_PACK_MOST) { most = fmaxf(most, fabsf(x[2 * q + h])); continue; }
+            if ((v[0] >> shift & 0x7F80u) != 0x7F80u) continue;
             const bool raw = __builtin_isfinite(x[2 * q + h]);
             const uint32_t front = raw ? CONV_PACK_RAW : bits << 1 > 0xFF000000u ? 0x7FC0u : bits >> 16;
             v[0] = (v[0] & keep) | front << shift;
@@ -98,15 +93,9 @@ __device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const fl
     }
 #pragma unroll
     for (int t = 0; t < 3; ++t) out[(size_t)step * 192 + t * 64 + lane] = part[t];
-    // (the last lane of the wave ends with all lanes' largest: shifts by 1, 2, 4, 8 within rows of 16 lanes, then row by row)
-#define WITH_LANES(control, rows) most = fmaxf(most, u2f(__builtin_amdgcn_update_dpp(0, f2u(most), control, rows, 0xF, true)))
-    WITH_LANES(0x111, 0xF); WITH_LANES(0x112, 0xF); WITH_LANES(0x114, 0xF); WITH_LANES(0x118, 0xF); WITH_LANES(0x142, 0xA); WITH_LANES(0x143, 0xC);
-#undef WITH_LANES
-    if (lane == 63) largest[step] = most;
 }
-extern "C" __global__ __launch_bounds__(256) void conv_split_pack(u32x4* __restrict__ out, const float* __restrict__ w, float* __restrict__ largest,
-                                                                  ConvPackParams P) {
-    conv_pack_body(out, w, largest, P, blockIdx.x);
+extern "C" __global__ __launch_bounds__(256) void conv_split_pack(u32x4* __restrict__ out, const float* __restrict__ w, ConvPackParams P) {
+    conv_pack_body(out, w, P, blockIdx.x);
 }
 // The weights of several layers in one launch: workgroup b belongs to the last entry of the table whose first_block is <= b.
 extern "C" __global__ __launch_bounds__(256) void conv_split_pack_layers(const ConvPackEntry* __restrict__ table, uint32_t entries) {
@@ -116,7 +105,7 @@ extern "C" __global__ __launch_bounds__(256) void conv_split_pack_layers(const C
         if (table[mid].first_block <= blockIdx.x) lo = mid; else hi = mid;
     }
     const ConvPackEntry& e = table[__builtin_amdgcn_readfirstlane(lo)];
-    conv_pack_body(e.out, e.w, e.largest, e.P, (int)(blockIdx.x - e.first_block));
+    conv_pack_body(e.out, e.w, e.P, (int)(blockIdx.x - e.first_block));
 }
 
 // ---- the product ------------------------------------------------------------------------------------------------------
@@ -146,7 +135,7 @@ template <int WGM, int WGN, int TM, int TN, bool STEPS>
 __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float* __restrict__ Es, int* __restrict__ Rs,
                                                 float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                                                 float* __restrict__ partial, uint32_t* __restrict__ arrivals, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
-                                                const float* __restrict__ largest, const ConvParams& P, const ConvDerived& Dk) {
+                                                const ConvParams& P, const ConvDerived& Dk) {
     constexpr int BM = 32 * WGM * TM, BN = 32 * WGN * TN, NT = 64 * WGM * WGN, BK = 32;
     u32x4* const As = pool;                         // [2 buffers][3 parts][4 octets][BM rows]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / WGN, wn = wave % WGN;
@@ -250,6 +239,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     auto split_word = [&](f32x4 (&x)[2], int t, int q) {
         f32x4& v = x[q >> 1];
         const int e = 2 * (q & 1);
+        if (t == 0) { v[e] *= CONV_SPLIT_SCALE; v[e + 1] *= CONV_SPLIT_SCALE; }
         const uint32_t w2 = to_bf16x2(v[e], v[e + 1]);
         if (t < 2) { v[e] = minus_low(w2, v[e]); v[e + 1] = minus_high(w2, v[e + 1]); }
         return w2;
@@ -269,7 +259,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     // product first 1.36e-7, 8.9e-8 and 5.3e-8, through fp32 products 2.1e-7, 5.9e-8 and 2.5e-8; no slower.)
     constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
     constexpr int CH = TM * TN, NS = 6 * CH;
-    float sign = kbeg & 2 ? -1.f / CONV_PACK_SCALE : 1.f / CONV_PACK_SCALE;
+    float sign = kbeg & 2 ? -1.f / (CONV_SPLIT_SCALE * CONV_SPLIT_SCALE) : 1.f / (CONV_SPLIT_SCALE * CONV_SPLIT_SCALE);
     auto k16_step = [&](auto step_, int kt) {
         constexpr int step = decltype(step_)::value, ks = step & 1, item = 1 - ks;   // step of the pair of k tiles, the second of its k tile
         u32x4 *const mine = As + (step >> 1) * 12 * BM, *const other = As + ((step >> 1) ^ 1) * 12 * BM;
@@ -430,189 +420,86 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                     }
     }
 
-    // Sums that are computed again with fp32 products. The others beside them stay as they are, so a row's results do not depend on what
-    // the rows in its tile hold.
-    //   - An operand that is infinite, not a number, or beyond the largest bf16 leaves a sum that is not finite (infinity times the zero parts
-    //     of the other operand).
-    //   - Numbers of the rows below 2^-102 lose up to 2^-125 each, a sum up to 2^-125 K times its largest weight: less than 2^-28 of a sum from
-    //     2^-97 K times that weight up. Of smaller sums (zeros, nearly always: rows or columns of zeros) the row is looked through for such numbers.
-    {
-        float high = 0.f, low = __builtin_inff();
+    // Sums that are not finite are computed again with fp32 products. The others beside them stay as they are, so a row's results do not
+    // depend on what the rows in its tile hold.
+    float high = 0.f;
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; v += 2) high = higher_of(high, acc[i][j][v], acc[i][j][v + 1]);
+    if (__builtin_amdgcn_ballot_w64(!(high < __builtin_inff()))) {
+        // In the order of the packed operand: lane l of a k16 step takes row l % 32, column l % 32 and the octet of its half of the wave,
+        // so both operands come in 16-byte loads, the next step's while this one's 8 TN products run. 12544 x 2304 x 256 with NaN only: 454 us
+        // (102 without; 1560 with single words requested one after the other), 3x3x128x128 on 50176 rows 356 (91; 1350), through the fp32
+        // kernels 131 and 132.
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            bool any = false;
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; v += 2) high = higher_of(high, acc[i][j][v], acc[i][j][v + 1]);
-        bool in_n[TN];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) in_n[j] = n0 + (wn * TN + j) * 32 + l32 < P.N;
-        if (m0 + BM <= P.M && n0 + BN <= P.N) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
+                for (int v = 0; v < 16; ++v) any |= !__builtin_isfinite(acc[i][j][v]);
+            if (!__builtin_amdgcn_ballot_w64(any)) continue;
+            const int m = m0 + (wm * TM + i) * 32 + l32;
+            const int b = flat_rows ? 0 : magic_div(m, P.howo_magic, P.howo_shift), r2 = m - b * HoWo;
+            const int ho = flat_rows ? 0 : magic_div(r2, P.wo_magic, P.wo_shift), wo = r2 - ho * P.Wo;
+            const int hi0 = ho * P.SH - P.PH, wi0 = wo * P.SW - P.PW;
+            const uint32_t row = (uint32_t)(flat_rows ? m * P.xs_h : b * P.xs_b + ho * P.SH * P.xs_h + wo * P.SW * P.xs_w) * 4u;
+            int r = 0, s = 0, c = 0;
+            f32x4 a_next[2];
+            u32x4 b_next[TN][3];
+            auto request = [&](int step) {
+                const int hi = hi0 + r * P.DH, wi = wi0 + s * P.DW, o = 2 * (step & 1) + half, k = (step >> 1) * BK + 4 * o;
+                const bool ok = m < P.M && (flat_rows || ((uint32_t)hi < (uint32_t)P.H && (uint32_t)wi < (uint32_t)P.W));
+                const uint32_t at = row + (uint32_t)(r * P.DH * P.xs_h + s * P.DW * P.xs_w + c + 4 * o) * 4u;
+                a_next[0] = buffer_load_x4(x_rsrc, ok && k < P.K ? at : CONV_OOB);
+                a_next[1] = buffer_load_x4(x_rsrc, ok && k + 16 < P.K ? at + 64u : CONV_OOB);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
-                    for (int v = 0; v < 16; v += 2) low = lower_of(low, acc[i][j][v], acc[i][j][v + 1]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const bool in_m = m0 + (wm * TM + i) * 32 + 4 * half + 8 * (v / 4) + v % 4 < P.M;
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) low = lower_of(low, in_m && in_n[j] ? acc[i][j][v] : low, low);
+                    for (int q = 0; q < 3; ++q)
+                        b_next[j][q] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, b_lane, b_soff[j] + (uint32_t)step * 3072u + (uint32_t)q * 1024u, 0);
+                if (step & 1) {
+                    c += BK;
+                    if (c >= P.Cin) { c = 0; if (++s == P.KW) { s = 0; ++r; } }
                 }
-        }
-        // Rows' operand in the order of the packed one: lane l of a k16 step takes row l % 32 and the octet of its half of the wave, so both come
-        // in 16-byte loads.
-        int row_at[TM], row_y[TM], row_x[TM], tap_r, tap_s, tap_c;
-        auto start_rows = [&]() {
-            tap_r = tap_s = tap_c = 0;
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const int m = m0 + (wm * TM + i) * 32 + l32;
-                const int b = flat_rows ? 0 : magic_div(m, P.howo_magic, P.howo_shift), r2 = m - b * HoWo;
-                const int ho = flat_rows ? 0 : magic_div(r2, P.wo_magic, P.wo_shift), wo = r2 - ho * P.Wo;
-                row_at[i] = flat_rows ? m * P.xs_h : b * P.xs_b + ho * P.SH * P.xs_h + wo * P.SW * P.xs_w;
-                row_y[i]  = m < P.M ? ho * P.SH - P.PH : INT32_MIN / 2;      // (rows beyond the last one lie outside every image)
-                row_x[i]  = wo * P.SW - P.PW;
-            }
-        };
-        auto request_row = [&](f32x4 (&to)[2], int i, int step) {
-            const int y = row_y[i] + tap_r * P.DH, xx = row_x[i] + tap_s * P.DW, o = 2 * (step & 1) + half, k = (step >> 1) * BK + 4 * o;
-            const bool ok = flat_rows ? row_y[i] >= 0 : (uint32_t)y < (uint32_t)P.H && (uint32_t)xx < (uint32_t)P.W;
-            const uint32_t at = (uint32_t)(row_at[i] + tap_r * P.DH * P.xs_h + tap_s * P.DW * P.xs_w + tap_c + 4 * o) * 4u;
-            to[0] = buffer_load_x4(x_rsrc, ok && k < P.K ? at : CONV_OOB);
-            to[1] = buffer_load_x4(x_rsrc, ok && k + 16 < P.K ? at + 64u : CONV_OOB);
-        };
-        auto next_step = [&](int step) {
-            if (!(step & 1)) return;
-            tap_c += BK;
-            if (tap_c >= P.Cin) { tap_c = 0; if (++tap_s == P.KW) { tap_s = 0; ++tap_r; } }
-        };
-
-        float bound = 0.f;                                  // sums below it are looked at
-        uint32_t rows[TM] = {};                             // rows that hold numbers below 2^-102
-        if (__builtin_amdgcn_ballot_w64(low < 0x1p-97f * CONV_PACK_MOST * (float)P.K)) {
-            // (weights beyond CONV_PACK_MOST are stored as they are)
-            const int steps = 2 * ktiles;
-            const __amdgpu_buffer_rsrc_t l_rsrc = make_rsrc(largest, (uint32_t)((P.N + 31) / 32 * steps) * 4u);
-            float most = 0.f;
-            for (int k = lane; k < steps; k += 64)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) most = fmaxf(most, buffer_load_x1(l_rsrc, (uint32_t)((n0 / 32 + wn * TN + j) * steps + k) * 4u));
-#pragma unroll
-            for (int m = 32; m >= 1; m >>= 1) most = fmaxf(most, __shfl_xor(most, m, 64));
-            bound = 0x1p-97f * most * (float)P.K;
-        }
-        if (__builtin_amdgcn_ballot_w64(low < bound)) {
-            start_rows();
-            constexpr int U = 4 * TN;                       // steps whose loads are in flight together
-            uint32_t least[TM];                             // (a number's magnitude in bits, doubled) - 1: zero is the largest
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                least[i] = 0xFFFFFFFFu;
-                uint32_t wanted = 0;                        // rows with such sums; the others are not loaded
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    bool small = false;
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) small |= fabsf(acc[i][j][v]) < bound && in_n[j];
-                    const uint64_t lanes = __builtin_amdgcn_ballot_w64(small);
-                    wanted |= ((uint32_t)lanes ? 1u : 0u) << (8 * (v / 4) + v % 4) | (lanes >> 32 ? 16u : 0u) << (8 * (v / 4) + v % 4);
-                }
-                if (!(wanted >> l32 & 1u)) row_y[i] = INT32_MIN / 2;
-            }
+            };
+            f32x16 again[TN] = {}, total[TN] = {};          // (summed by 64 k, as rounded as in the loop above)
+            request(0);
 #pragma nounroll
-            for (int step = 0; step < 2 * ktiles; step += U) {
-                f32x4 x8[U][TM][2];
+            for (int step = 0; step < 2 * ktiles; ++step) {
+                float av[8], bv[TN][8];
+                const float sign_k = step & 4 ? -1.f : 1.f;
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
+                for (int e = 0; e < 8; ++e) {
+                    av[e] = a_next[e >> 2][e & 3];
 #pragma unroll
-                    for (int i = 0; i < TM; ++i) request_row(x8[u][i], i, step + u);
-                    next_step(step + u);
-                }
+                    for (int j = 0; j < TN; ++j) {
+                        uint32_t part_e[3];
 #pragma unroll
-                for (int u = 0; u < U; ++u)
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) least[i] = min(least[i], (f2u(x8[u][i][e >> 2][e & 3]) << 1) - 1u);
-            }
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const uint64_t small = __builtin_amdgcn_ballot_w64(least[i] < (f2u(0x1p-102f) << 1) - 1u);
-                rows[i] = (uint32_t)small | (uint32_t)(small >> 32);
-            }
-        }
-        // 12544 x 2304 x 256 as an example (102 us, through the fp32 kernels 140): NaN only 456 us (1560 with single words requested one after the
-        // other), numbers of 1e-36 only 530, every third row zero 129, zeros only 163; 3x3x128x128 on 50176 rows 91, NaN only 351. Data without any
-        // of these: 0 to 2 % for the look at the sums.
-        uint32_t looked = __builtin_amdgcn_ballot_w64(!(high < __builtin_inff())) != 0;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) looked |= rows[i];
-        if (looked) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                uint32_t flags = 0;                         // bit 16 j + v: that sum
-                const uint32_t small_rows = rows[i] >> (4 * half);
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const uint32_t bits = f2u(acc[i][j][v]) << 1, at = 8 * (v / 4) + v % 4;
-                        const uint32_t small = (small_rows >> at & 1u) && bits < f2u(bound) << 1 && in_n[j];
-                        flags |= (bits >= 0xFF000000u ? 1u : small) << (16 * j + v);
+                        for (int q = 0; q < 3; ++q) part_e[q] = e & 1 ? b_next[j][q][e >> 1] & 0xFFFF0000u : b_next[j][q][e >> 1] << 16;
+                        const float value = ((u2f(part_e[2]) + u2f(part_e[1])) + u2f(part_e[0])) * (1.f / CONV_SPLIT_SCALE);
+                        bv[j][e] = (part_e[0] == CONV_PACK_RAW << 16 ? u2f(part_e[1] | part_e[2] >> 16) : value) * sign_k;
                     }
-                if (!__builtin_amdgcn_ballot_w64(flags != 0)) continue;
-                start_rows();
-                f32x4 a_next[2];
-                u32x4 b_next[TN][3];
-                auto request = [&](int step) {
-                    request_row(a_next, i, step);
+                }
+                request(step + 1);                          // (behind the last step: zeros, or the next columns' first, unused)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) again[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], bv[j][e], again[j], 0, 0, 0);
+                if ((step & 3) == 3) {
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
 #pragma unroll
-                        for (int q = 0; q < 3; ++q)
-                            b_next[j][q] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, b_lane, b_soff[j] + (uint32_t)step * 3072u + (uint32_t)q * 1024u, 0);
-                    next_step(step);
-                };
-                f32x16 again[TN] = {}, total[TN] = {};      // (summed by 64 k, as rounded as in the loop above)
-                request(0);
-#pragma nounroll
-                for (int step = 0; step < 2 * ktiles; ++step) {
-                    float av[8], bv[TN][8];
-                    const float sign_k = step & 4 ? -1.f : 1.f;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        av[e] = a_next[e >> 2][e & 3];
-#pragma unroll
-                        for (int j = 0; j < TN; ++j) {
-                            uint32_t part_e[3];
-#pragma unroll
-                            for (int q = 0; q < 3; ++q) part_e[q] = e & 1 ? b_next[j][q][e >> 1] & 0xFFFF0000u : b_next[j][q][e >> 1] << 16;
-                            const float value = ((u2f(part_e[2]) + u2f(part_e[1])) + u2f(part_e[0])) * (1.f / CONV_PACK_SCALE);
-                            bv[j][e] = (part_e[0] == CONV_PACK_RAW << 16 ? u2f(part_e[1] | part_e[2] >> 16) : value) * sign_k;
-                        }
-                    }
-                    request(step + 1);                      // (behind the last step: zeros, or the next columns' first, unused)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j) again[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], bv[j][e], again[j], 0, 0, 0);
-                    if ((step & 3) == 3) {
-#pragma unroll
-                        for (int j = 0; j < TN; ++j)
-#pragma unroll
-                            for (int v = 0; v < 16; ++v) { total[j][v] += again[j][v]; again[j][v] = 0.f; }
-                    }
+                        for (int v = 0; v < 16; ++v) { total[j][v] += again[j][v]; again[j][v] = 0.f; }
                 }
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[i][j][v] = flags >> (16 * j + v) & 1u ? total[j][v] : acc[i][j][v];
             }
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = __builtin_isfinite(acc[i][j][v]) ? acc[i][j][v] : total[j][v];
         }
     }
 
@@ -746,12 +633,11 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
 #define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE, STEPS)                                                                \
     extern "C" __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void name(             \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                                   \
-        float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp,                   \
-        const float* __restrict__ largest, ConvParams P, ConvDerived D) {                                                    \
+        float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) { \
         __shared__ __attribute__((aligned(16))) u32x4 pool[24 * 32 * WGM * TM];                                              \
         __shared__ float Es[CONV_MAX_EPI * 32 * WGN * TN];                                                                   \
         __shared__ int Rs[32 * WGM * TM];                                                                                    \
-        conv_split_body<WGM, WGN, TM, TN, STEPS>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, largest, P, D);    \
+        conv_split_body<WGM, WGN, TM, TN, STEPS>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);             \
     }
 // _steps: 50176 x 128 x 512 with a ReLU6 65 us, with a scalar 57, with `relu(y) + r` 76 (each as launches of its own behind the product: 83, 82, 94;
 // in the fp32 kernels 70, 68, 73).

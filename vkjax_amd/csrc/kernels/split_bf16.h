@@ -30,11 +30,6 @@ __device__ __forceinline__ int xcd_range(int id, int n) {
     const int per = n / 8;
     return per > 0 && id < per * 8 ? (id & 7) * per + (id >> 3) : id;
 }
-// min(low, |a|, |b|), numbers that are not ones left out
-__device__ __forceinline__ float lower_of(float low, float a, float b) {
-    asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(low) : "v"(a), "v"(b));
-    return low;
-}
 // max(high, |a|, |b|); NaN if one of them is
 __device__ __forceinline__ float higher_of(float high, float a, float b) {
     asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(high) : "v"(a), "v"(b));

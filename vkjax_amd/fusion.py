@@ -39,8 +39,6 @@ def _reads(op) -> tp.List:
     if op.conv is not None:
         out, lhs, rhs, geom, epilogue = op.conv
         reads = [lhs, rhs] + [e.operand for e in epilogue if e.operand is not None and e.op not in (K.CONV_TAP, K.CONV_SOFTMAX)]
-        if geom.split is not None:
-            reads.append(geom.split.largest)
         for e in epilogue:
             reads += e.bounds
             if e.derived is not None:
@@ -248,7 +246,7 @@ def fuse_ops(all_ops, bufferpool, outvars):
             _out(prod)._placeholder.elided = True
             result[producer[pid]] = None
             del producer[pid]
-        new = Op(op.equation, launch=K.conv_split_pack(packed, geom.split.largest, through, geom), meta=('conv_pack', packed, through, geom))
+        new = Op(op.equation, launch=K.conv_split_pack(packed, through, geom), meta=('conv_pack', packed, through, geom))
         new.index = op.index
         return new
 
@@ -910,8 +908,6 @@ def _writes(op) -> tp.List:
         return [op.meta[1]]
     if op.meta is not None and op.meta[0] in ('threefry', 'softmax'):
         return list(op.meta[1])
-    if op.meta is not None and op.meta[0] == 'conv_pack':
-        return [op.meta[1], op.meta[3].split.largest]
     return [b for b, _ in op.launch.buffers[:1] if b is not None]      #kernels write their first argument
 
 

@@ -343,7 +343,7 @@ BATCH_KERNELS        = {**{k: k.replace('ew_chain_', 'ew_chain_batch_') for k in
 EW_BATCH_ENTRY_BYTES        = 432
 REDUCE_BATCH_ENTRY_BYTES    = 56
 TRANSPOSE_BATCH_ENTRY_BYTES = 48
-PACK_BATCH_ENTRY_BYTES      = 64
+PACK_BATCH_ENTRY_BYTES      = 56
 BATCH_MAX_BLOCKS         = 4096        #launches of more workgroups than this keep a launch of their own
 REDUCE_NARROW_MAX_BLOCKS = 16          #column sums of at most this many workgroups trade block width for more blocks
 TRANSPOSE_BATCH_MAX_BLOCKS = 1024      #... tiled transposes (the kernels of a network, for its backward pass) up to this many
@@ -370,7 +370,7 @@ def batch_table(launch: Launch, device_address: tp.Callable[[Buffer], int]) -> n
     is_chain, is_transpose = kind in EW_BATCH_KERNELS, kind in TRANSPOSE_BATCH_KERNELS
     entry_bytes, pointers = ((EW_BATCH_ENTRY_BYTES, 1 + EW_MAX_STEPS) if is_chain else
                              (TRANSPOSE_BATCH_ENTRY_BYTES, 2) if is_transpose else
-                             (PACK_BATCH_ENTRY_BYTES, 3) if kind == 'conv_split_pack' else (REDUCE_BATCH_ENTRY_BYTES, 2))
+                             (PACK_BATCH_ENTRY_BYTES, 2) if kind == 'conv_split_pack' else (REDUCE_BATCH_ENTRY_BYTES, 2))
     rows, first = [], 0
     for m in launch.members:
         assert len(m.buffers) == pointers, (m.kernel, len(m.buffers))
@@ -1086,7 +1086,6 @@ class ConvSplit(tp.NamedTuple):
     slices: int
     partial: tp.Optional[Buffer] = None
     arrivals: tp.Optional[Buffer] = None
-    largest: tp.Optional[Buffer] = None          #of the packed kernel operand, per wave of the launch that packs it
 
 
 def conv_split_tiles(split: ConvSplit, g: ConvGeometry) -> tp.Tuple[int, int]:
@@ -1102,10 +1101,6 @@ def conv_split_partial_words(split: ConvSplit, g: ConvGeometry) -> int:
 
 def conv_split_packed_words(g: ConvGeometry) -> int:
     return _cdiv(g.N, 32) * _cdiv(g.K, 64) * (CONV_SPLIT_PACK_BYTES // 4)
-
-
-def conv_split_largest_words(g: ConvGeometry) -> int:
-    return _cdiv(g.N, 32) * _cdiv(g.K, 64) * 4
 
 
 def conv_split_plan(lhs: Buffer, g: ConvGeometry, lhs_offset: int = 0, compute_units: int = 256, sliceable: bool = True) -> tp.Optional[ConvSplit]:
@@ -1143,14 +1138,14 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry, lhs_offset: int = 0, compute_u
     return best[1] if best else None
 
 
-def conv_split_pack(packed: Buffer, largest: Buffer, source: EwOperand, g: ConvGeometry) -> Launch:
+def conv_split_pack(packed: Buffer, source: EwOperand, g: ConvGeometry) -> Launch:
     '''The kernel operand of a product, element (ky, kx, c, n) at source.offset + (ky, kx, c, n) . source.strides, taken
-    apart into three bf16 parts and laid out for the matrix cores; `largest`: its largest element per 32 columns and 16 k.'''
-    assert packed.size == conv_split_packed_words(g) and largest.size == conv_split_largest_words(g)
-    blocks = _cdiv(g.N, 32) * _cdiv(g.K, 64)
+    apart into three bf16 parts and laid out for the matrix cores.'''
+    assert packed.size == conv_split_packed_words(g)
     params = _i32(g.N, g.K, g.Cin, g.KW, *source.strides)
-    return Launch('conv_split_pack', (blocks, 1, 1), (BLOCK, 1, 1), [(packed, 0), (source.buffer, source.offset * 4), (largest, 0)], params,
-                  bytes_moved=4 * (packed.size + g.K * g.N), written=(0, 2))
+    blocks = _cdiv(g.N, 32) * _cdiv(g.K, 64)
+    return Launch('conv_split_pack', (blocks, 1, 1), (BLOCK, 1, 1), [(packed, 0), (source.buffer, source.offset * 4)], params,
+                  bytes_moved=4 * (packed.size + g.K * g.N))
 
 
 def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry, epilogue: tp.Sequence[ConvEpilogueStep] = (),
@@ -1200,7 +1195,7 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
         nbytes += 4 * taps[0][1].size
     scratch = [(split.partial, 0), (split.arrivals, 0)] if shared else [(None, 0), (None, 0)]
     return Launch(f'conv_gemm_split_{split.tile}' + ('_steps' if steps else ''), (split.whole + shared * split.slices, 1, 1), (256, 1, 1),
-                  [(out, out_offset * 4), (lhs, lhs_offset * 4), (packed, 0)] + scratch + operand_slots + derived_ptrs + [(split.largest, 0)],
+                  [(out, out_offset * 4), (lhs, lhs_offset * 4), (packed, 0)] + scratch + operand_slots + derived_ptrs,
                   params + derived_desc, bytes_moved=nbytes, flops=2 * M * N * K,
                   written=(0, 3, 4) if shared else (0,), scratch=(3, 4) if shared else ())
 
