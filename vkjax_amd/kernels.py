@@ -1073,7 +1073,7 @@ CONV_SPLIT_TILES = {'128x128': (128, 128, 1.15, 1.15), '128x64': (128, 64, 0.65,
 #and one launch. Contraction: with two k tiles of 32 a block is all start-up and stores (200704 x 64 x 256 with residual:
 #101 us here, 66 there, where a block walks several tiles; 50176 x 128 x 512: 59 against 61). Operations: launch latency.
 CONV_SPLIT_MIN_M, CONV_SPLIT_MIN_K, CONV_SPLIT_MIN_FLOPS = 2049, 128, 1e9
-CONV_SPLIT_MAX_SLICED = 4096       #tiles of one launch whose contraction is shared: counters set aside for them
+CONV_SPLIT_ROUND = 256             #tiles of a whole round, one per CU; only those behind the last whole round are shared, fewer than this many
 CONV_SPLIT_PACK_BYTES = 12288      #packed kernel operand: bytes per 32 columns and pair of k tiles of 32
 
 
@@ -1103,7 +1103,7 @@ def conv_split_packed_words(g: ConvGeometry) -> int:
     return _cdiv(g.N, 32) * _cdiv(g.K, 64) * (CONV_SPLIT_PACK_BYTES // 4)
 
 
-def conv_split_plan(lhs: Buffer, g: ConvGeometry, lhs_offset: int = 0, compute_units: int = 256, sliceable: bool = True) -> tp.Optional[ConvSplit]:
+def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
     '''The plan with the smallest estimated time, or None where these kernels do not apply or another one is faster.'''
     if (CHOICES.conv_split is False or g.k_splits > 1 or _dense_rows_shape(lhs, g) or CHOICES.conv_general or CHOICES.conv_b_general
             or any(v is not None for v in (CHOICES.conv_tile, CHOICES.conv_bk, CHOICES.conv_chunk, CHOICES.conv_ksplit, CHOICES.conv_k_splits, CHOICES.conv_mix))
@@ -1111,7 +1111,7 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry, lhs_offset: int = 0, compute_u
         return None
     g = _flatten_pointwise(g)
     M, N, K = g.M, g.N, g.K
-    _, _, a_fast, _, _ = _conv_fast_paths(lhs, lhs, g, lhs_offset)
+    _, _, a_fast, _, _ = _conv_fast_paths(lhs, lhs, g, 0)
     if not a_fast or (g.Cin % 32 != 0 and g.KH * g.KW != 1) or conv_split_packed_words(g) * 4 >= 2**31 or M * N == 0:
         return None
     if not (CHOICES.conv_split or CHOICES.conv_split_slices) and (M < CONV_SPLIT_MIN_M or K < CONV_SPLIT_MIN_K or 2 * M * N * K < CONV_SPLIT_MIN_FLOPS):
@@ -1125,14 +1125,13 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry, lhs_offset: int = 0, compute_u
             continue
         tiles = _cdiv(M, bm) * _cdiv(N, bn)
         for slices in range(1, 17):
-            whole = tiles if slices == 1 else tiles // compute_units * compute_units
-            if (slices > 1 and (ktiles < 2 * slices or not sliceable or whole == tiles or tiles - whole > CONV_SPLIT_MAX_SLICED)
-                    or CHOICES.conv_split_slices not in (None, slices)):
+            whole = tiles if slices == 1 else tiles // CONV_SPLIT_ROUND * CONV_SPLIT_ROUND
+            if slices > 1 and (ktiles < 2 * slices or whole == tiles) or CHOICES.conv_split_slices not in (None, slices):
                 continue
             blocks = whole + (tiles - whole) * slices
-            rounds = whole / compute_units if slices > 1 else _cdiv(tiles, compute_units)
-            time   = ((shared_step if blocks > compute_units else lone_step)
-                      * (rounds * (ktiles + 3) + _cdiv((tiles - whole) * slices, compute_units) * (ktiles / slices + 8)))
+            rounds = whole / CONV_SPLIT_ROUND if slices > 1 else _cdiv(tiles, CONV_SPLIT_ROUND)
+            time   = ((shared_step if blocks > CONV_SPLIT_ROUND else lone_step)
+                      * (rounds * (ktiles + 3) + _cdiv((tiles - whole) * slices, CONV_SPLIT_ROUND) * (ktiles / slices + 8)))
             if best is None or time < best[0]:
                 best = (time, ConvSplit(tile, whole, slices))
     return best[1] if best else None

@@ -573,7 +573,7 @@ def _split_ops(bufferpool, equation, outbuf, lhs: Buffer, rhs: Buffer, geom: 'K.
         return None
     if plan.slices > 1:
         plan = plan._replace(partial=bufferpool.shared_scratch(K.conv_split_partial_words(plan, geom), 'partial products'),
-                             arrivals=bufferpool.zeroed_scratch(K.CONV_SPLIT_MAX_SLICED, 'arrivals of partial products'))
+                             arrivals=bufferpool.zeroed_scratch(K.CONV_SPLIT_ROUND, 'arrivals of partial products'))
     position = bufferpool.op_counter
     bufferpool.op_counter -= 1                  #the packed operand lives at the equation's own position
     packed = bufferpool.new_temporary(np.uint32, (K.conv_split_packed_words(geom),))
