@@ -85,6 +85,15 @@ struct ConvParams {
                                     // m_extra = tiles_m % m_blocks blocks one more; the M tiles per block in the flags are then
                                     // ignored. For grids sized to what the GPU holds at once.
     int32_t m_each, m_extra;
+    // The kernels on the bf16 matrix cores (conv_split.h) read some of these words in a way of their own:
+    //   flags bit 25 (CONV_SPLIT_MASKED): the epilogue is the backward pass of a ReLU, (+ full tensor), mask, (second result), (* vector), its
+    //     operands at fixed places of the pointer table: full tensor, activation, vector, limit, constant; bits 12-15 are then 0 or 1 (there is
+    //     a second result, behind the mask), bits 20-24 say which of full tensor (bit 23) and vector (bit 21) are there. Bits 26-31 are 0.
+    //   flags bits 20-24 without it: all zero with steps in bits 8-11 is an epilogue walked through step by step (kernels named _steps)
+    //   w_bytes: the packed kernel operand's size; ws_*, LH, LW, xs_c, k_split_steps: unused
+    //   split_tiles_m: the first tiles of the grid (tiles_m x tiles_n, row by row), computed by one block each
+    //   m_blocks: the slices that the contraction of every tile behind those is cut into, of m_each pairs of k tiles of 32 each, the first
+    //     m_extra of them one more
 };
 
 // The part of the output a block's tile number refers to: a grid of tiles_m x tiles_n tiles whose first row is

@@ -51,6 +51,8 @@ static_assert(sizeof(ConvPackEntry) == 56, "the host lays the table out with 56-
 constexpr float CONV_SPLIT_SCALE = 0x1p24f;
 constexpr uint32_t CONV_PACK_RAW = 0x7FC1u;
 
+constexpr uint32_t CONV_SPLIT_MASKED = 1u << 25;      // ConvParams::flags; the host has it under the same name
+
 __device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const float* __restrict__ w, const ConvPackParams& P, int block) {
     const int id = block * 256 + (int)threadIdx.x, lane = id & 63, step = id >> 6, ksteps = (P.K + 63) / 64 * 4;
     const int nb = step / ksteps, s = step - nb * ksteps, o = 2 * (s & 1) + (lane >> 5), n = nb * 32 + (lane & 31);
@@ -567,7 +569,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     // The epilogue of a backward pass: + full tensor (operand 0), kept where an activation (operand 1) lies above a limit (3) and
     // replaced by a constant (4) elsewhere, stored as a second result, * vector (2). The launches it replaces moved four to six times
     // the result; ResNet-50's training step at batch 64: 13.31 -> 12.11 ms.
-    const bool masked_form = P.flags & (1u << 25);
+    const bool masked_form = P.flags & CONV_SPLIT_MASKED;
     const __amdgpu_buffer_rsrc_t m_rsrc = make_rsrc(epi.p[1], masked_form ? P.out_bytes : 0u);
 #pragma unroll
     for (int i = 0; i < TM; ++i)

@@ -1074,6 +1074,7 @@ CONV_SPLIT_TILES = {'128x128': (128, 128, 1.15, 1.15), '128x64': (128, 64, 0.65,
 #101 us here, 66 there, where a block walks several tiles; 50176 x 128 x 512: 59 against 61). Operations: launch latency.
 CONV_SPLIT_MIN_M, CONV_SPLIT_MIN_K, CONV_SPLIT_MIN_FLOPS = 2049, 128, 1e9
 CONV_SPLIT_ROUND = 256             #tiles of a whole round, one per CU; only those behind the last whole round are shared, fewer than this many
+CONV_SPLIT_MASKED = 1 << 25        #ConvParams.flags: the epilogue has a mask (conv_masked_epilogue)
 CONV_SPLIT_PACK_BYTES = 12288      #packed kernel operand: bytes per 32 columns and pair of k tiles of 32
 
 
@@ -1160,7 +1161,7 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
         operands = conv_masked_epilogue(epilogue)
         if operands is None or out_offset or any(e.operand.size != out.size for e in epilogue if e.kind == 3):
             raise ValueError('an epilogue with a mask is: + full tensor, mask, second result, * vector')
-        flags   |= 1 << 25 | len(taps) << 12
+        flags   |= CONV_SPLIT_MASKED | len(taps) << 12
         epilogue = [e or ConvEpilogueStep(EW['NOP'], 0, None) for e in operands]
     elif taps:
         (tap_position, tap_buffer), = taps
