@@ -24,9 +24,9 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // Sums: the twelve products of a k tile are chained from zero and added to the accumulators by fp32 operations, G's sign changed in
 // every other k tile (the matrix cores cut sums off, see conv_split.h).
 // Scale: both operands are multiplied by 2^24 before they are taken apart and the sums by 2^-48, so the smallest numbers have all their bits
-// (a bf16 part of a number below 2^-102 would not). It costs 1 to 2 % of the kernel. (Looking behind the loop for sums that such numbers could matter
-// to, as conv_split.h does, costs as much for the columns' largest numbers and far more where it finds some: sums of nothing but zeros are
-// everywhere behind a ReLU, ResNet-50's training step took 17.7 ms instead of 12.6.)
+// (a bf16 part of a number below 2^-102 would not). It costs 1 to 2 % of the kernel. (Looking behind the loop for sums that such numbers could
+// matter to, and through their columns, costs as much for the columns' largest numbers and far more where it finds some: sums of nothing but
+// zeros are everywhere behind a ReLU, ResNet-50's training step took 17.7 ms instead of 12.6.)
 constexpr float WGRAD_SCALE = 0x1p24f;
 template <int TM, int TN, bool VEC_A, bool VEC_B>
 __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2* __restrict__ table, float* __restrict__ out,
