@@ -239,6 +239,17 @@ def test_plans_and_packed_layout():
         assert all('split' not in l.kernel for l in plan(m, k, n).launches), (m, k, n)
 
 
+@pytest.mark.parametrize('m,k,n,bf16', [
+    (65536, 1024, 32, False), (16384, 4096, 32, False), (50176, 4096, 20, False), (200704, 512, 32, False), (65536, 1024, 33, True),  #columns
+    (20000, 2048, 32, True), (32768, 2048, 32, True), (32800, 2048, 32, False), (20000, 1024, 32, False),                             #... up to 1024 tiles of 32 rows
+    (4096, 1024, 128, False), (8192, 2048, 64, False), (3136, 3072, 128, False), (4096, 4096, 64, True), (8224, 2048, 64, True),      #few tiles
+    (3136, 1024, 256, True), (12544, 512, 128, True), (12544, 64, 1024, False)])                                                       #layers of a network
+def test_products_that_the_fp32_kernels_compute_faster_stay_with_them(m, k, n, bf16):
+    '''Plan only: sizes that were measured on both sides of every line of the rule, and those beside the lines.'''
+    program = JaxprInterpreter(mj.make_jaxpr(jnp.dot)(np.broadcast_to(np.float32(0), (m, k)), np.broadcast_to(np.float32(0), (k, n))), plan_only=True)
+    assert any('split' in l.kernel for l in program.launches) == bf16, [l.kernel for l in program.launches]
+
+
 #input gradients of a strided 1x1 convolution whose result has one position: they write one element in four (or two) of the features'
 #array and zeros come from another launch, so what follows cannot be computed with the product
 ONE_POSITION = [(130, 2, 2, 64), (129, 1, 2, 64), (131, 2, 1, 64)]

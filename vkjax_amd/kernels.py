@@ -1071,7 +1071,11 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
 CONV_SPLIT_TILES = {'128x128': (128, 128, 1.15, 1.15), '128x64': (128, 64, 0.65, 0.95)}
 #Products below these stay with the fp32 kernels. Rows: packing the kernel operand costs what about 250 rows' products cost,
 #and one launch. Contraction: with two k tiles of 32 a block is all start-up and stores (200704 x 64 x 256 with residual:
-#101 us here, 66 there, where a block walks several tiles; 50176 x 128 x 512: 59 against 61). Operations: launch latency.
+#101 us here, 66 there, where a block walks several tiles; 50176 x 128 x 512: 59 against 61). Operations: start and end of two launches. A
+#product alone is slower up to 2 GFLOP (8188 x 880 x 98, 1.4: 28.9 against 23.9; 20000 x 512 x 64, 1.3: 23.4, 21.6; 8192 x 512 x 256, 2.1: 23.0,
+#23.4), by the packing launch; in a network, where several layers' weights are packed by one launch, it is faster from 1 on, more so where
+#the backward pass of a ReLU is its epilogue (ResNet-50 with the line at 1, at 1.5 and at 2: batch 16 1566, 1583, 1623 us, batch 8 at 200 x 200 1092, 1119,
+#1120; its training step at batch 16 5603, 5577, 5976, at batch 24 on 160 x 160 5099, 5407, 5408).
 CONV_SPLIT_MIN_M, CONV_SPLIT_MIN_K, CONV_SPLIT_MIN_FLOPS = 2049, 128, 1e9
 CONV_SPLIT_ROUND = 256             #tiles of a whole round, one per CU; only those behind the last whole round are shared, fewer than this many
 CONV_SPLIT_MASKED = 1 << 25        #ConvParams.flags: the epilogue has a mask (conv_masked_epilogue)
@@ -1104,6 +1108,21 @@ def conv_split_packed_words(g: ConvGeometry) -> int:
     return _cdiv(g.N, 32) * _cdiv(g.K, 64) * (CONV_SPLIT_PACK_BYTES // 4)
 
 
+def _conv_split_pays(g: ConvGeometry, c_contig: bool) -> bool:
+    '''Where the kernels on the bf16 matrix cores are faster than the fp32 kernels that would compute the product otherwise.'''
+    M, N, K = g.M, g.N, g.K
+    if M < CONV_SPLIT_MIN_M or K < CONV_SPLIT_MIN_K or 2 * M * N * K < CONV_SPLIT_MIN_FLOPS:
+        return False
+    #(times in microseconds, here and there)
+    if N <= 32:
+        #half of a tile is columns that do not exist: 65536 x 1024 x 32 58, 48; 16384 x 4096 x 32 70, 49; 50176 x 4096 x 32 202, 185. Except where
+        #the fp32 tiles are more than four waves share and fewer than the SIMDs: 20000 x 2048 x 32 42, 55; 30000 x 4096 x 32 122, 161
+        return K >= 2048 and 2 * CONV_SPLIT_ROUND < _cdiv(M, 32) <= 4 * CONV_SPLIT_ROUND
+    #few tiles: the fp32 kernel whose four waves share a tile is ahead until the contraction is long (K = 2048, 4096 and 8192: 4096 x 64 22, 16;
+    #31, 27; 46, 48. 4096 x 128 31, 24; 42, 43; 64, 80. 3136 x 128 33, 24; 44, 41; 59, 76)
+    return K >= 4096 or not _four_waves_per_tile(g, True, c_contig, CONV_SPLIT_ROUND)
+
+
 def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
     '''The plan with the smallest estimated time, or None where these kernels do not apply or another one is faster.'''
     if (CHOICES.conv_split is False or g.k_splits > 1 or _dense_rows_shape(lhs, g) or CHOICES.conv_general or CHOICES.conv_b_general
@@ -1112,10 +1131,10 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
         return None
     g = _flatten_pointwise(g)
     M, N, K = g.M, g.N, g.K
-    _, _, a_fast, _, _ = _conv_fast_paths(lhs, lhs, g, 0)
+    _, _, a_fast, _, c_contig = _conv_fast_paths(lhs, lhs, g, 0)
     if not a_fast or (g.Cin % 32 != 0 and g.KH * g.KW != 1) or conv_split_packed_words(g) * 4 >= 2**31 or M * N == 0:
         return None
-    if not (CHOICES.conv_split or CHOICES.conv_split_slices) and (M < CONV_SPLIT_MIN_M or K < CONV_SPLIT_MIN_K or 2 * M * N * K < CONV_SPLIT_MIN_FLOPS):
+    if not (CHOICES.conv_split or CHOICES.conv_split_slices) and not _conv_split_pays(g, c_contig):
         return None
     #The whole tiles are dealt out in rounds of one per CU; the contraction of those of the last, incomplete round (or of all,
     #if there are fewer tiles than CUs) may be cut into slices, of two k tiles at least. A block's start and end cost about
