@@ -85,6 +85,30 @@ def test_products_that_share_scratch_memory_are_ordered(kind):
     assert kind == 'two products' or pairs > 0
 
 
+def unordered_pairs(interp):
+    '''Pairs of launches on different lanes that touch one allocation, one of them writing it, with no wait between them.'''
+    plan = interp.lane_plan
+    sets = [lanes.touched_and_written(op, launch) for op, launch in zip(interp.all_ops, interp.launches)]
+    waited = lambda i, j: any(plan.wait[w] and plan.lane[w] == plan.lane[j] for w in range(i + 1, j + 1))
+    return [(i, j) for j in range(len(sets)) for i in range(j) if plan.lane[i] != plan.lane[j]
+            and (sets[i][1] & sets[j][0] or sets[j][1] & sets[i][0]) and not waited(i, j)]
+
+
+#programs whose batched launches have given the partial sums' storage to other arrays too, before and behind the products
+POOLED = {'mlp_train': (W.mlp_train_step, lambda: W.mlp_train_inputs(0, 4096, (512, 512, 256, 10)), {}),
+          'resnet50_train': (W.resnet50_train_step, lambda: W.resnet50_train_inputs(batch=4, size=64), dict(conv_split='128x128', conv_split_slices=2))}
+
+
+@pytest.mark.parametrize('name', list(POOLED))
+def test_arrays_that_lie_in_scratch_storage_are_ordered(name):
+    fn, inputs, choices = POOLED[name]
+    with K.overrides(**choices):
+        interp = JaxprInterpreter(mj.make_jaxpr(fn)(*inputs()), plan_only=True, two_lanes=True)
+    lanes.check(interp.lane_plan)
+    assert any(interp.lane_plan.lane) and any(l.scratch for l in interp.launches)
+    assert not unordered_pairs(interp)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize('kind', ('two products', 'four products'))
 def test_products_that_share_scratch_memory_give_the_bits_of_one_stream(kind):

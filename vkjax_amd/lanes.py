@@ -77,10 +77,13 @@ def with_scratch_of_their_lane(launches, plan_: 'LanePlan', second_set: tp.Calla
 
 
 def dependencies(ops, launches) -> tp.List[tp.List[int]]:
-    '''For every launch the earlier launches it must not overtake. Launches on one lane never do; the scratch arrays that each
-    lane has a set of are left out.'''
-    own  = {id(launch.buffers[i][0].tensor) for launch in launches for i in launch.scratch}
-    sets = [tuple(s - own for s in touched_and_written(op, launch)) for op, launch in zip(ops, launches)]
+    '''For every launch the earlier launches it must not overtake. Launches on one lane never do; scratch arrays that each
+    lane has a set of are left out, unless the pool has given their storage to other buffers as well.'''
+    sets  = [touched_and_written(op, launch) for op, launch in zip(ops, launches)]
+    other = {id(b.tensor) for launch in launches for m in (launch.members or (launch,)) for i, (b, _) in enumerate(m.buffers)
+             if b is not None and i not in m.scratch}
+    own   = {id(launch.buffers[i][0].tensor) for launch in launches for i in launch.scratch} - other
+    sets  = [tuple(s - own for s in pair) for pair in sets]
     result = []
     for j, (touched_j, written_j) in enumerate(sets):
         deps = [i for i in range(j) if (sets[i][1] & touched_j) or (written_j & sets[i][0])]
