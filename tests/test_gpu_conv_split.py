@@ -243,6 +243,7 @@ def test_plans_and_packed_layout():
     (65536, 1024, 32, False), (16384, 4096, 32, False), (50176, 4096, 20, False), (200704, 512, 32, False), (65536, 1024, 33, True),  #columns
     (20000, 2048, 32, True), (32768, 2048, 32, True), (32800, 2048, 32, False), (20000, 1024, 32, False),                             #... up to 1024 tiles of 32 rows
     (4096, 1024, 128, False), (8192, 2048, 64, False), (3136, 3072, 128, False), (4096, 4096, 64, True), (8224, 2048, 64, True),      #few tiles
+    (200704, 128, 64, False), (200704, 192, 64, True), (200704, 128, 68, True),                                                        #short and narrow
     (3136, 1024, 256, True), (12544, 512, 128, True), (12544, 64, 1024, False)])                                                       #layers of a network
 def test_products_that_the_fp32_kernels_compute_faster_stay_with_them(m, k, n, bf16):
     '''Plan only: sizes that were measured on both sides of every line of the rule, and those beside the lines.'''

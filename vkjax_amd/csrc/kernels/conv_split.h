@@ -122,10 +122,10 @@ extern "C" __global__ __launch_bounds__(256) void conv_split_pack_layers(const C
 // alone, the compiler gathers loads and splitting in front of or behind the MFMAs (a 128 x 128 x 4608 tile alone on a CU:
 // 273 us with one stage after the other, 193 without a branch in the loop, 147 with the order written down).
 //
-// What bounds it: power. On 8192 x 2048 x 8192 the matrix cores are busy 73 to 79 % of the time at 1.64 to 1.71 GHz, 207 to 221
+// What bounds it: power. On 8192 x 2048 x 8192 the matrix cores are busy 73 to 79 % of the time at 1.64 to 1.71 GHz, 200 to 221
 // TFLOP/s of fp32 products (133 through v_mfma_f32_32x32x2_f32, which cannot exceed 157); a loop of these MFMAs and nothing
 // else runs at 1.8 to 1.9 GHz. So what moves less data is faster: 128 x 64 tiles reach 0.88 of the 128 x 128 tiles' rate. The
-// layers of a network are shorter: start, stores and the last round of blocks count (12544 x 2304 x 256: 163 TFLOP/s).
+// layers of a network are shorter: start, stores and the last round of blocks count (12544 x 2304 x 256: 147 to 163 TFLOP/s, by the card).
 //
 // Sharing out: the first P.split_tiles_m tiles of the grid are computed by one block each, the contraction of every tile behind
 // them by P.m_blocks blocks (slices of P.m_each or one more pairs of k tiles). A slice's sums go to `partial`, and whichever block arrives
@@ -641,8 +641,9 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         __shared__ int Rs[32 * WGM * TM];                                                                                    \
         conv_split_body<WGM, WGN, TM, TN, STEPS>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);             \
     }
-// _steps: 50176 x 128 x 512 with a ReLU6 65 us, with a scalar 57, with `relu(y) + r` 76 (each as launches of its own behind the product: 83, 82, 94;
-// in the fp32 kernels 70, 68, 73).
+// _steps: 50176 x 128 x 512 with a ReLU6 68 us, with a scalar 62, with `relu(y) + r` 82 (each as launches of its own behind the product: 83, 82, 94;
+// in the fp32 kernels 73, 71, 73); 50176 x 256 x 512 97, 89, 108 (127, 120, 130). (Words of a full tensor requested for two tiles at a time
+// instead of one: 80 instead of 82, not kept; for four: registers spill.)
 // (2 x 2 waves of 64 x 64: 255 registers, two blocks per CU; 1 x 4 waves of 128 x 32, which load every column once, were 1 % slower)
 CONV_SPLIT_KERNEL(conv_gemm_split_128x128, 2, 2, 2, 2, 2, false)
 CONV_SPLIT_KERNEL(conv_gemm_split_128x128_steps, 2, 2, 2, 2, 2, true)

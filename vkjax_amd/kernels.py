@@ -1118,6 +1118,10 @@ def _conv_split_pays(g: ConvGeometry, c_contig: bool) -> bool:
         #half of a tile is columns that do not exist: 65536 x 1024 x 32 58, 48; 16384 x 4096 x 32 70, 49; 50176 x 4096 x 32 202, 185. Except where
         #the fp32 tiles are more than four waves share and fewer than the SIMDs: 20000 x 2048 x 32 42, 55; 30000 x 4096 x 32 122, 161
         return K >= 2048 and 2 * CONV_SPLIT_ROUND < _cdiv(M, 32) <= 4 * CONV_SPLIT_ROUND
+    #short and narrow: bound by HBM on both sides, start and end of a block count (65536 x 128 x 64 18, 15; 157776 x 136 x 63 39, 36; 200704 x 128 x 64
+    #40, 41, with a residual behind its ReLU 51, 45; 65536 x 192 x 64 22, 20; 200704 x 192 x 64 47, 49)
+    if N <= 64 and K < 192:
+        return False
     #few tiles: the fp32 kernel whose four waves share a tile is ahead until the contraction is long (K = 2048, 4096 and 8192: 4096 x 64 22, 16;
     #31, 27; 46, 48. 4096 x 128 31, 24; 42, 43; 64, 80. 3136 x 128 33, 24; 44, 41; 59, 76)
     return K >= 4096 or not _four_waves_per_tile(g, True, c_contig, CONV_SPLIT_ROUND)
