@@ -51,11 +51,11 @@ OTHER_CONFIGS = ('affine', 'mlp', 'conv_block', 'rng_uniform', 'gather_scatter')
 
 #kernel families whose launches compute their results from their operands alone, so that replaying one changes nothing
 REPEATABLE = ('conv_gemm', 'dense_rows', 'softmax_rows', 'ew_chain', 'ew_affine', 'threefry2x32', 'gather_rows', 'pool', 'reduce_rows',
-              'reduce_cols', 'transpose_tiled', 'pad_nd')
+              'reduce_cols', 'transpose_tiled', 'pad_nd', 'rows_')
 
 
 def kernel_family(name: str) -> str:
-    for prefix in ('conv_gemm', 'conv_split_pack', 'wgrad_gemm', 'wgrad_split', 'dense_rows', 'softmax_rows', 'ew_chain', 'ew_affine', 'threefry2x32', 'gather_rows', 'pool', 'reduce_rows', 'reduce_cols', 'scatter_rows',
+    for prefix in ('conv_gemm', 'conv_split_pack', 'wgrad_gemm', 'wgrad_split', 'dense_rows', 'softmax_rows', 'ew_chain', 'ew_affine', 'threefry2x32', 'gather_rows', 'pool', 'reduce_rows', 'reduce_cols', 'scatter_rows', 'rows_',
                    'select_window', 'scatter_selected', 'pad_nd', 'scale_relu_backward', 'scale_backward', 'transpose_tiled'):
         if name.startswith(prefix):
             return prefix

@@ -652,3 +652,47 @@ def test_stream_in_flight_hands_out_results_in_order_whatever_the_lanes_do():
     assert [next(it) for _ in range(5)] == [0, 10, 20, 30, 40]
     it.close()
     assert not lane_threads() and state['taken'] < 40
+
+
+def test_row_programs_leave_what_they_cannot_hold_to_the_separate_launches():
+    '''Which runs of row-wise ops become one launch: rows of 2 to 1024 values, two of them at least; what reads a result in
+    the middle of the run moves behind the launch; slots are handed on within the LDS of a block.'''
+    from vkjax_amd import fusion, workloads as W
+    def plan(rows, cols):
+        x, y = np.zeros((rows, cols), np.float32), np.zeros((rows, cols), np.float32)
+        return JaxprInterpreter(mj.make_jaxpr(mj.value_and_grad(W.softmax_cross_entropy))(x, y), plan_only=True)
+    for rows, cols, fused in ((2, 2, True), (1000, 10, True), (64, 1000, True), (4097, 1024, True), (64, 1025, False), (64, 1, False), (1, 64, False)):
+        interp  = plan(rows, cols)
+        kernels = [l.kernel for l in interp.launches]
+        assert sum(k.startswith('rows_v') for k in kernels) == int(fused), (rows, cols, kernels)
+        for op, l in zip(interp.all_ops, interp.launches):
+            if l.kernel.startswith('rows_v'):
+                assert l.lds <= K.ROWS_LDS and l.lds % (l.block[0] * 4) == 0 and l.written == (0, 1)
+                #the loss is summed from what the launch stores
+                at = interp.launches.index(l)
+                assert any(any(b is not None and b.tensor is l.buffers[0][0].tensor for b, _ in m.buffers[1:])
+                           for later in interp.launches[at + 1:] for m in (later.members or (later,)))
+    assert len(K.row_program([], [], [], 8, 10).params) == 4 * (5 + 5 * 8 + 2 * K.ROWS_MAX_CODE)
+
+
+def test_a_run_of_row_ops_keeps_clear_of_what_reads_it_on_the_way():
+    '''An op between two members that reads a member's result and feeds a later op: neither it nor what it feeds is a member.'''
+    jnp = mj.numpy
+    def f(x, w):
+        e = mj.lax.exp(x - jnp.max(x, axis=1, keepdims=True))
+        s = jnp.sum(e, axis=1, keepdims=True)
+        h = jnp.dot(e / s, w)                                     #a product over the rows' values
+        return jnp.sum(h * e, axis=1), jnp.sum(e * e, axis=1) / s[:, 0]
+    args   = [np.zeros((30, 12), np.float32), np.zeros((12, 12), np.float32)]
+    interp = JaxprInterpreter(mj.make_jaxpr(f)(*args), plan_only=True)
+    kernels = [l.kernel for l in interp.launches]
+    first   = next(i for i, k in enumerate(kernels) if k.startswith('rows_v'))
+    product = next(i for i, k in enumerate(kernels) if k.startswith(('dense_rows', 'conv_gemm')))
+    assert first < product < len(kernels) - 1, kernels
+    made = set()
+    for l in interp.launches:                                      #every launch reads inputs, constants or what has been made before it
+        for i, (b, _) in enumerate(l.buffers):
+            if b is not None and i not in l.written:
+                assert id(b.tensor) in made or any(b.tensor is x.tensor for x in interp.input_buffers) or b.constant_value is not None \
+                    or getattr(b.tensor, 'initial_value', None) is not None, l.kernel
+        made |= {id(l.buffers[i][0].tensor) for i in l.written if l.buffers[i][0] is not None}

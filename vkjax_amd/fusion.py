@@ -18,6 +18,8 @@ to that position, and the skipped intermediates get no storage.
 import collections
 import typing as tp
 
+import numpy as np
+
 from . import kernels as K
 from .kernels import EW, EwChain, EwOperand, EwStep
 
@@ -55,6 +57,8 @@ def _reads(op) -> tp.List:
             return [b for b, _ in op.launch.buffers[1:] if b is not None]
         if op.meta[0] == 'softmax':
             return [op.meta[2]]
+        if op.meta[0] == 'rows':
+            return list(op.meta[2])
         if op.meta[0] == 'conv_pack':
             return [op.meta[2].buffer]
     return [b for b, _ in op.launch.buffers if b is not None]
@@ -314,6 +318,7 @@ def fuse_ops(all_ops, bufferpool, outvars):
     ops = fuse_random_streams([op for op in result if op is not None], bufferpool, outvars)
     ops = fuse_stream_chains(ops, bufferpool, outvars)
     ops = fuse_softmax(ops, bufferpool, outvars)
+    ops = fuse_row_programs(remove_dead_ops(ops, bufferpool, outvars), bufferpool, outvars)
     ops = fuse_scale_relu_backward(ops, bufferpool, outvars)
     ops = fuse_reduce_prologues(ops, bufferpool, outvars)
     ops = fuse_reduce_scales(ops, bufferpool, outvars)
@@ -382,6 +387,199 @@ def fuse_softmax(ops, bufferpool, outvars):
         removed |= {i, i + 1, i + 2}
         replacement[i + 3 + (arg_out is not None)] = fused
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
+
+
+#From three ops on a launch is saved whatever else the step needs. There is no upper line to the array's size: a loss and its
+#gradient on rows of 10, 64, 100, 256, 1000 and 1001 were faster in one launch on 50 to 262144 rows, where they take 36 to 838 us
+#through the separate launches (1000 x 10: 39 -> 16 us, 65536 x 64: 120 -> 56, 65536 x 1000: 838 -> 462).
+ROW_PROGRAM_MIN_OPS = 3
+
+
+def _row_walk(operand: EwOperand, shape, outer: int, R: int):
+    '''(element of row 0, row stride, column stride, one value per row) of an operand of a chain over `shape`, an array of
+    [outer, R] or of `outer` values, or None where its rows do not lie at one stride.'''
+    full = len(shape) > 0 and shape[-1] == R and np_prod(shape) == outer * R
+    if not full and np_prod(shape) != outer:
+        return None
+    walk  = list(zip(shape, operand.strides))
+    outer_dims = [(n, s) for n, s in (walk[:-1] if full else walk) if n != 1]
+    for (_, s), (m, t) in zip(outer_dims, outer_dims[1:]):
+        if s != t * m:
+            return None
+    return operand.offset, outer_dims[-1][1] if outer_dims else 0, walk[-1][1] if full else 0, not full
+
+
+class _RowProgram:
+    '''The instructions of a run of row-wise ops (`members`, in order), or no `launch` where they do not fit the kernel.'''
+
+    def __init__(self, members, outer: int, R: int, needed_outside):
+        pid = lambda b: id(b._placeholder)
+        self.inputs, self.outs, self.steps, self.inside, self.launch = [], [], [], {}, None
+        result_of = lambda op: op.meta[1] if op.chain is None else op.chain.out
+        made      = {pid(result_of(op)): n for n, op in enumerate(members)}
+        self.inside = {pid(result_of(op)): result_of(op) for op in members}
+        singles, number, in_acc, in_slots = {}, {}, None, set()
+
+        def operand(o: EwOperand, shape):
+            '''(slot, one value per row) an operand is read from; None: it is not read as the kernel reads.'''
+            walk = _row_walk(o, shape, outer, R)
+            if walk is None:
+                return None
+            base, row, column, whole_row = walk
+            if pid(o.buffer) in made:
+                single = singles.get(pid(o.buffer))
+                if single is None or (base, row, column) != (0, 1 if single else R, 0 if single or whole_row else 1) or (whole_row and not single):
+                    return None
+                return ('value', pid(o.buffer)), single
+            i = K.RowsInput(o.buffer, base, row, column, column == 0)
+            if i not in self.inputs:
+                self.inputs.append(i)
+            return ('in', self.inputs.index(i)), i.single
+
+        #values that a later member reads otherwise than from the accumulator the moment they are made
+        reads = []
+        for op in members:
+            o = [EwOperand(op.meta[2], 0, (R, 1))] if op.chain is None else op.chain.operands()
+            reads.append([None if x is None else pid(x.buffer) for x in o])
+        keep = set()
+        for n, r in enumerate(reads):
+            for k, b in enumerate(r):
+                if b in made and not (k == 0 and made[b] == n - 1):
+                    keep.add(b)
+
+        def load(o, shape):
+            nonlocal in_acc
+            where = operand(o, shape)
+            if where is None:
+                return False
+            if where[0] != ('value', in_acc):
+                self.steps.append(K.RowsStep('load', slot=where[0], single=where[1]))
+            return True
+
+        for op in members:
+            if op.chain is None:
+                _, out, source, _, _, _, name, _, _ = op.meta
+                if not load(EwOperand(source, 0, (R, 1)), (outer, R)):
+                    return
+                self.steps.append(K.RowsStep(name))
+                single = True
+            else:
+                chain = op.chain
+                out   = chain.out
+                if any(s.op in _SELECTS for s in chain.steps) or not load(chain.first, chain.shape):
+                    return
+                for s in chain.steps:
+                    where = (None, False)
+                    if s.operand is not None:
+                        where = operand(s.operand, chain.shape)
+                        if where is None:
+                            return
+                    self.steps.append(K.RowsStep('apply', s.op, s.operand_left, where[0], where[1], s.imm))
+                single = np_prod(chain.shape) != outer * R
+            singles[pid(out)] = single
+            in_acc = pid(out)
+            if pid(out) in keep:
+                self.steps.append(K.RowsStep('put', slot=('value', pid(out)), single=single))
+            if pid(out) in needed_outside:
+                self.steps.append(K.RowsStep('out', slot=('out', len(self.outs)), single=single))
+                self.outs.append(out)
+        self.launch = K.row_program(self.outs, self.inputs, self.steps, outer, R)
+
+
+def fuse_row_programs(ops, bufferpool, outvars):
+    '''Element-wise chains and row reductions over the rows of one [outer, R] array that feed each other - a classifier's
+    loss and its gradient - become one launch (rows.hip), values bit for bit. What stands between them and reads
+    their results moves behind it.'''
+    from .ops import Op
+    pid  = lambda b: id(b._placeholder)
+    done = set()
+    while True:
+        seed = next((i for i, op in enumerate(ops) if id(op) not in done and _is_row_reduction(op)), None)
+        if seed is None:
+            return ops
+        done.add(id(ops[seed]))
+        _, _, _, outer, R, _, _, _, _ = ops[seed].meta
+        program, members, behind = _row_program_around(ops, seed, outer, R, bufferpool, outvars)
+        if program is None:
+            continue
+        last  = members[-1]
+        fused = Op(_label(*[ops[i] for i in members]), launch=program.launch, meta=('rows', program.outs, [i.buffer for i in program.inputs]))
+        fused.index = ops[last].index
+        for b in [i.buffer for i in program.inputs] + program.outs:
+            b.accesses.append(fused.index)
+        for key, b in program.inside.items():
+            if not any(pid(o) == key for o in program.outs):
+                b._placeholder.elided = True
+        #what moves gets a place of its own between the launch and whatever followed it
+        for n, i in enumerate(behind):
+            ops[i].index = fused.index + (n + 1) / (len(behind) + 1)
+            for b in _touched(ops[i]) + [b for b, _ in ops[i].launch.buffers if b is not None]:
+                b.accesses.append(ops[i].index)
+        taken = set(members) | set(behind)
+        ops = ([op for i, op in enumerate(ops[:last]) if i not in taken] + [fused] + [ops[i] for i in behind] + list(ops[last + 1:]))
+
+
+def _is_row_reduction(op) -> bool:
+    if op.meta is None or op.meta[0] != 'reduce' or op.chain is not None or op.conv is not None:
+        return False
+    _, _, source, outer, R, inner, name, _, nsplit = op.meta
+    return (inner == 1 and nsplit == 1 and name in ('reduce_sum', 'reduce_max') and source.dtype == np.float32
+            and 2 <= R <= K.ROWS_MAX_ROW and outer >= 2 and outer * R < 2**30)
+
+
+def _row_program_around(ops, seed: int, outer: int, R: int, bufferpool, outvars):
+    '''(program, positions of its members, positions of the ops among them that move behind it) for the largest run of ops
+    connected to the reduction at `seed`, or (None, ...).'''
+    pid = lambda b: id(b._placeholder)
+
+    def candidate(op) -> bool:
+        if _is_row_reduction(op):
+            return op.meta[3:5] == (outer, R)
+        if op.chain is None or op.meta is not None or np_prod(op.chain.shape) not in (outer, outer * R):
+            return False
+        return all(o is None or (o.buffer.size < 2**30 and _row_walk(o, op.chain.shape, outer, R) is not None) for o in op.chain.operands())
+
+    result_of  = lambda op: op.meta[1] if op.chain is None else op.chain.out
+    candidates = [i for i, op in enumerate(ops) if candidate(op)]
+    #connected through the values they make
+    maker, group = {pid(result_of(ops[i])): i for i in candidates}, {seed}
+    while True:
+        more = {i for i in candidates if i not in group
+                and (any(maker.get(pid(b)) in group for b in _reads(ops[i])) or any(maker.get(pid(b)) == i for g in group for b in _reads(ops[g])))}
+        if not more:
+            break
+        group |= more
+    members = sorted(group)
+    counts  = collections.Counter(pid(b) for op in ops for b in _writes(op))
+    while len(members) >= ROW_PROGRAM_MIN_OPS:
+        inside, tainted, taken, behind = set(), set(), [], []
+        for i in range(members[0], members[-1] + 1):
+            op = ops[i]
+            if i in members and not any(pid(b) in tainted for b in _reads(op)) and counts[pid(result_of(op))] == 1:
+                taken.append(i)
+                inside.add(pid(result_of(op)))
+            elif any(pid(b) in tainted or pid(b) in inside for b in _touched(op)):
+                behind.append(i)
+                tainted |= {pid(b) for b in _may_write(op)}
+        if len(taken) < ROW_PROGRAM_MIN_OPS or seed not in taken:
+            return None, [], []
+        if taken != members:
+            members = taken
+            continue
+        #nothing that stands behind a member and in front of the launch may change what the member reads
+        read = set()
+        for i in range(members[0], members[-1] + 1):
+            if i in members:
+                read |= {pid(b) for b in _reads(ops[i])}
+            elif any(pid(b) in read or pid(b) in inside for b in _may_write(ops[i])):
+                return None, [], []
+        uses = _use_counts(ops, bufferpool, outvars)
+        own  = collections.Counter(pid(b) for i in members for b in _reads(ops[i]))
+        program = _RowProgram([ops[i] for i in members], outer, R, {k for k in inside if uses[k] > own[k]})
+        if program.launch is not None:
+            return program, members, [i for i in behind if i < members[-1]]
+        members = members[:-1] if members[-1] != seed else members[1:]
+    return None, [], []
 
 
 def fuse_index_wrap(ops, bufferpool, outvars):
@@ -906,7 +1104,7 @@ def _writes(op) -> tp.List:
         return [_out(op)]
     if op.meta is not None and op.meta[0] in ('iota', 'concat_part'):
         return [op.meta[1]]
-    if op.meta is not None and op.meta[0] in ('threefry', 'softmax'):
+    if op.meta is not None and op.meta[0] in ('threefry', 'softmax', 'rows'):
         return list(op.meta[1])
     return [b for b, _ in op.launch.buffers[:1] if b is not None]      #kernels write their first argument
 
@@ -1086,7 +1284,7 @@ def _small_out(op):
 
 def _may_write(op) -> tp.List:
     '''Buffers an op may change: its result where the op's structure is known, else everything it touches.'''
-    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'reduce', 'softmax', 'conv_pack')):
+    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'reduce', 'softmax', 'rows', 'conv_pack')):
         return _writes(op)
     return [b for b, _ in op.launch.buffers if b is not None]
 

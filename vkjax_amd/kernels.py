@@ -1367,6 +1367,95 @@ def softmax_rows(out: Buffer, inp: Buffer, outer: int, R: int, arg_out: tp.Optio
                   streamable=True, written=(0, 2))
 
 
+# ---------------------------------------------------------------- row programs (rows.hip)
+
+ROWS_MAX_IN, ROWS_MAX_OUT, ROWS_MAX_CODE = 8, 6, 48
+ROWS_OPS     = dict(load=0, apply=1, reduce_sum=2, reduce_max=3, put=4, out=5)
+ROWS_MAX_ROW = 1024                 #a row stays in the registers of one wave, 16 values per lane
+#(values per vector, vectors per lane) of the kernels' variants
+ROWS_VARIANTS = ((4, 1), (4, 4), (1, 1), (1, 4), (1, 16))
+ROWS_LDS     = 64 << 10
+
+
+class RowsInput(tp.NamedTuple):
+    '''An array a row program reads: element base + row * row_stride + column * column_stride; `single`: one value per row.'''
+    buffer:        Buffer
+    base:          int
+    row_stride:    int
+    column_stride: int
+    single:        bool
+
+
+class RowsStep(tp.NamedTuple):
+    '''One instruction: `slot` is a pair (kind, number) - ('in', input), ('value', number of a value put away) or
+    ('out', output) - or None; `single`: one value per row.'''
+    what:   str
+    op:     int = 0
+    left:   bool = False
+    slot:   tp.Optional[tp.Tuple[str, int]] = None
+    single: bool = False
+    imm:    int = 0
+
+
+def rows_variant(R: int) -> tp.Tuple[int, int]:
+    '''The order of additions is that of reduce_rows: 16-byte vectors where the row has a multiple of 4 values.'''
+    vec = 4 if R % 4 == 0 else 1
+    return vec, next(n for v, n in ROWS_VARIANTS if v == vec and 64 * v * n >= R)
+
+
+def _rows_slots(steps: tp.Sequence[RowsStep], inputs: tp.Sequence[RowsInput], width: int) -> tp.Tuple[tp.Dict, int]:
+    '''First word of every slot and the number of words: a slot is handed on once what it holds is not read any more.'''
+    sizes, last = {('in', k): 1 if i.single else width for k, i in enumerate(inputs)}, {}
+    for at, s in enumerate(steps):
+        if s.slot is not None and s.slot[0] != 'out':
+            sizes.setdefault(s.slot, 1 if s.single else width)
+            last[s.slot] = at
+    place, free, words = {}, {1: [], width: []}, 0
+
+    def give(slot):
+        nonlocal words
+        n = sizes[slot]
+        if free[n]:
+            place[slot] = free[n].pop()
+        else:
+            place[slot] = words
+            words += n
+
+    for k in range(len(inputs)):
+        give(('in', k))
+    for at, s in enumerate(steps):
+        if s.what == 'put':
+            give(s.slot)
+        for slot in [x for x, end in last.items() if end == at]:
+            free[sizes[slot]].append(place[slot])
+    return place, words
+
+
+def row_program(outs: tp.Sequence[Buffer], inputs: tp.Sequence[RowsInput], steps: tp.Sequence[RowsStep], outer: int, R: int) -> tp.Optional[Launch]:
+    '''One launch for element-wise steps and reductions over the rows of [outer, R]; see rows.hip. None where the program
+    does not fit the kernel.'''
+    vec, vectors = rows_variant(R)
+    place, words = _rows_slots(steps, inputs, vec * vectors)
+    waves = next((w for w in (4, 2, 1) if words * 4 * 64 * w <= ROWS_LDS), None)
+    if waves is None or len(inputs) > ROWS_MAX_IN or len(outs) > ROWS_MAX_OUT or len(steps) > ROWS_MAX_CODE:
+        return None
+    lanes = min(64, _pow2_at_least(R // vec)) if vectors == 1 else 64
+    flags = [place['in', k] | (i.single << 16)
+             | ((vec == 4 and i.column_stride == 1 and i.row_stride % 4 == 0 and i.base % 4 == 0) << 17) for k, i in enumerate(inputs)]
+    code = []
+    for s in steps:
+        slot = 0 if s.slot is None else s.slot[1] if s.slot[0] == 'out' else place[s.slot]
+        code += [ROWS_OPS[s.what] | s.op << 4 | bool(s.left) << 16 | bool(s.single) << 17 | (s.slot is not None) << 18 | slot << 20, s.imm]
+    params = (_u32(outer, R, lanes.bit_length() - 1, len(inputs), len(steps), *_pad([i.buffer.size * 4 for i in inputs], ROWS_MAX_IN),
+                   *_pad([i.base for i in inputs], ROWS_MAX_IN))
+              + _i32(*_pad([i.row_stride for i in inputs], ROWS_MAX_IN), *_pad([i.column_stride for i in inputs], ROWS_MAX_IN))
+              + _u32(*_pad(flags, ROWS_MAX_IN), *_pad(code, 2 * ROWS_MAX_CODE)))
+    nbytes = sum(4 * min(b.size, outer * R) for b in [i.buffer for i in inputs] + list(outs))
+    return Launch(f'rows_v{vec}_n{vectors}', (_cdiv(outer, waves * (64 // lanes)), 1, 1), (64 * waves, 1, 1),
+                  _pad([(b, 0) for b in outs], ROWS_MAX_OUT, (None, 0)) + _pad([(i.buffer, 0) for i in inputs], ROWS_MAX_IN, (None, 0)),
+                  params, lds=4 * words * 64 * waves, bytes_moved=nbytes, written=tuple(range(len(outs))))
+
+
 def reduce_general(out: Buffer, inp: Buffer, kept, reduced, op: str) -> Launch:
     '''kept / reduced: lists of (size, stride) in row-major order of the output / of the reduce index.'''
     if len(kept) > 4 or len(reduced) > 4:
