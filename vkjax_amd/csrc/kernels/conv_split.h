@@ -34,8 +34,10 @@ __device__ __forceinline__ f32x4 buffer_load_x4_agent(__amdgpu_buffer_rsrc_t r, 
 // 16+4o .. 16+4o+3 (the order in which four lanes that share a row of the other operand load 64 contiguous bytes each time).
 // The kernel operand may lie in any order (strides, negative ones too), which makes the transposed and reversed kernels of a
 // backward pass no work of their own.
+// For the kernels that hold a patch of the input in LDS (PATCH below) a step is 16 input features under one tap of a 3 x 3 window, the nine taps
+// one after the other: [block of 32 columns][16 features][tap][part][lane], lane l: features 4o .. 4o+3 and 8+4o .. of them for o = l / 32.
 struct ConvPackParams {
-    int32_t N, K, Cin, KW;               // k = (ky * KW + kx) * Cin + c
+    int32_t N, K, Cin, KW;               // k = (ky * KW + kx) * Cin + c; K below 0: -K, in the order for a patch
     int32_t ws_r, ws_s, ws_c, ws_n;      // element strides of ky, kx, c, n
 };
 struct ConvPackEntry {
@@ -54,18 +56,22 @@ constexpr uint32_t CONV_PACK_RAW = 0x7FC1u;
 constexpr uint32_t CONV_SPLIT_MASKED = 1u << 25;      // ConvParams::flags; the host has it under the same name
 
 __device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const float* __restrict__ w, const ConvPackParams& P, int block) {
-    const int id = block * 256 + (int)threadIdx.x, lane = id & 63, step = id >> 6, ksteps = (P.K + 63) / 64 * 4;
+    const bool patch = P.K < 0;
+    const int K = patch ? -P.K : P.K;
+    const int id = block * 256 + (int)threadIdx.x, lane = id & 63, step = id >> 6, ksteps = patch ? K / 16 : (K + 63) / 64 * 4;
     const int nb = step / ksteps, s = step - nb * ksteps, o = 2 * (s & 1) + (lane >> 5), n = nb * 32 + (lane & 31);
     if (nb * 32 >= P.N) return;
+    const int sixteen = s / 9, tap = s - 9 * sixteen;
+    const bool negative = patch ? s / 3 & 1 : s & 4;        // every other group of steps: see the product's sums
     float x[8];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const int k0 = (s >> 1) * 32 + h * 16 + 4 * o, rs = k0 / P.Cin;
+        const int k0 = patch ? tap * P.Cin + 16 * sixteen + 8 * h + 4 * (lane >> 5) : (s >> 1) * 32 + h * 16 + 4 * o, rs = k0 / P.Cin;
         int c = k0 - rs * P.Cin, ky = rs / P.KW, kx = rs - ky * P.KW;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const float v = (k0 + q < P.K && n < P.N) ? w[(int64_t)ky * P.ws_r + (int64_t)kx * P.ws_s + (int64_t)c * P.ws_c + (int64_t)n * P.ws_n] : 0.f;
-            x[4 * h + q] = s & 4 ? -v : v;                  // every other pair of k tiles: see the product's sums
+            const float v = (k0 + q < K && n < P.N) ? w[(int64_t)ky * P.ws_r + (int64_t)kx * P.ws_s + (int64_t)c * P.ws_c + (int64_t)n * P.ws_n] : 0.f;
+            x[4 * h + q] = negative ? -v : v;
             if (++c == P.Cin) { c = 0; if (++kx == P.KW) { kx = 0; ++ky; } }
         }
     }
@@ -110,6 +116,53 @@ extern "C" __global__ __launch_bounds__(256) void conv_split_pack_layers(const C
     conv_pack_body(e.out, e.w, e.P, (int)(blockIdx.x - e.first_block));
 }
 
+__device__ __forceinline__ uint32_t conv_split_step_desc(const ConvParams& P, int e) {
+    return ((e < 3 ? P.epi_desc[0] : P.epi_desc[1]) >> (10 * (e < 3 ? e : e - 3))) & 1023u;
+}
+// The epilogue's scalars and per-column vectors, to LDS
+template <int BN>
+__device__ __forceinline__ void conv_split_epilogue_operands(float* __restrict__ Es, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp, const ConvParams& P,
+                                                             const ConvDerived& Dk, int tid, int n0) {
+    if (tid < BN) {
+        float e_reg[CONV_MAX_EPI], d_in[CONV_MAX_DERIVED + 1];
+#pragma unroll
+        for (int e = 0; e < CONV_MAX_EPI; ++e) {
+            const uint32_t kind = conv_split_step_desc(P, e) >> 8;
+            const uint32_t present = epi.p[e] != nullptr ? 1u : 0u;
+            e_reg[e] = buffer_load_x1(make_rsrc(epi.p[e], kind == 1 ? 4u * present : kind == 2 ? (uint32_t)P.N * 4u * present : 0u),
+                                      kind == 2 ? (uint32_t)(n0 + tid) * 4u : 0u);
+        }
+        if (Dk.nsteps) {
+#pragma unroll
+            for (int k = 0; k <= CONV_MAX_DERIVED; ++k) {
+                const bool vec = (Dk.vector_mask >> k) & 1u;
+                d_in[k] = buffer_load_x1(make_rsrc(Dp.p[k], Dp.p[k] == nullptr ? 0u : vec ? (uint32_t)P.N * 4u : 4u),
+                                         vec ? (uint32_t)(n0 + tid) * 4u : 0u);
+            }
+            const float v = conv_derived_value(d_in, Dk);
+#pragma unroll
+            for (int e = 0; e < CONV_MAX_EPI; ++e)
+                if (e == (int)Dk.step) e_reg[e] = v;
+        }
+#pragma unroll
+        for (int e = 0; e < CONV_MAX_EPI; ++e)
+            if (e < (int)((P.flags >> 8) & 15u)) Es[e * BN + tid] = e_reg[e];
+    }
+}
+
+#define FENCE() __builtin_amdgcn_sched_barrier(0)
+// The next part of two neighbouring numbers of an item's eight, and what is left of them: their nearest bf16
+__device__ __forceinline__ uint32_t conv_split_word(f32x4 (&x)[2], int t, int q) {
+    f32x4& v = x[q >> 1];
+    const int e = 2 * (q & 1);
+    if (t == 0) { v[e] *= CONV_SPLIT_SCALE; v[e + 1] *= CONV_SPLIT_SCALE; }
+    const uint32_t w2 = to_bf16x2(v[e], v[e + 1]);
+    if (t < 2) { v[e] = minus_low(w2, v[e]); v[e + 1] = minus_high(w2, v[e + 1]); }
+    return w2;
+}
+// (A part, B part) of the six products of a k16 step, in their order
+__device__ constexpr int CONV_SPLIT_PA[6] = {2, 1, 1, 0, 0, 0}, CONV_SPLIT_PB[6] = {0, 0, 1, 1, 2, 0};
+
 // ---- the product ------------------------------------------------------------------------------------------------------
 // Block = WGM x WGN waves, each with TM x TN tiles of 32 x 32; k tile 32, i.e. two k16 steps, taken in pairs. A tile of the
 // rows' operand is loaded as fp32 (two items per thread, each a row's octet in two 16-byte vectors), taken apart in registers and
@@ -132,8 +185,184 @@ extern "C" __global__ __launch_bounds__(256) void conv_split_pack_layers(const C
 // last at the tile's counter adds all slices in their order and applies the epilogue: no block waits for another. The
 // counters are left at zero for the next launch.
 
+// ---- the sums of a tile, from a patch of the input in LDS ----------------------------------------------------------------
+// 3 x 3 windows at a stride of 1 over an input with a border of one: the rows of a tile are consecutive positions m of the images laid end to
+// end, and under tap (r, s) position m sees position m + (r - 1) W + s - 1. So the 128 + 2 W + 2 positions m0 - W - 1 .. of 16 input features
+// are loaded, taken apart and put into LDS once and serve nine k16 steps, where the kernel above loads and takes apart 128 positions in each
+// of them. A tap that lies outside the image for some rows (their neighbour belongs to another row or image there) has those lanes read zeros
+// that stand behind the patch.
+//   LDS: [2 buffers][3 parts][2 octets][264 positions] x 8 bf16; octet o: features 4o .. 4o+3 and 8+4o .. of the 16; positions 256 .. 258 are zeros;
+//     264: neither the writes nor the reads of lanes that go together meet in a bank.
+// While one buffer serves its nine steps, the next 16 features' two items per thread are taken apart into the other one, in the first
+// eight steps, and requested again for the 16 features behind them. One barrier per nine steps, in the last. The products of three steps, not
+// four, are summed from zero before they are added to the accumulators: errors against 64-bit sums of 1.06e-7 and 1.28e-7 of the 2-norm for 64 and 512
+// features where every tap is loaded anew 1.24e-7 and 1.37e-7.
+// What bounds it: power, as below; what it saves is vector instructions, LDS writes and loads, which take their share of it. Products alone, before and after:
+// 64 x 56 x 56 x 64 x 64 91.5 -> 78.0 us, 28 x 28 x 128 x 128 88.1 -> 74.2, 14 x 14 x 256 x 256 87.5 -> 73.5, 7 x 7 x 512 x 512 88.3 -> 79.0 (187 to 201 TFLOP/s);
+// 32 x 56 x 56 x 64 x 64 52.5 -> 44.9, 50 x 24 x 24 x 128 x 64 38.3 -> 25.6. ResNet-50 at batch 64 3.94 -> 3.83 ms, its training step 13.10 -> 12.82.
+// (The body of the loop has no branch: skipping the second item where a patch is short cost more in spilled registers than it saved.)
+constexpr int CONV_PATCH_ROWS = 264, CONV_PATCH_ZEROS = 256;
+
+template <int WGM, int WGN, int TM, int TN>
+__device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* __restrict__ Es, float (&acc)[TM][TN][16], const uint32_t (&b_soff)[TN],
+                                                const float* __restrict__ x, __amdgpu_buffer_rsrc_t w_rsrc, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
+                                                const ConvParams& P, const ConvDerived& Dk, int wave, int m0, int n0, int kbeg, int kend) {
+    constexpr int BN = 32 * WGN * TN, NT = 64 * WGM * WGN, ROWS = CONV_PATCH_ROWS;
+    static_assert(WGM * TM == 4 && NT == 256, "tiles of 128 rows, two items per thread");
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5, wm = wave / WGN;
+    const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(x, P.x_bytes);
+    // ---- items: (position of the patch, octet)
+    const int p_octet = tid & 1, p_row = tid >> 1;                      // item p: position p_row + 128 p
+    uint32_t p_voff[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int at = m0 - P.W - 1 + p_row + 128 * p;
+        p_voff[p] = at >= 0 && at < P.M && p_row + 128 * p < 130 + 2 * P.W ? (uint32_t)(at * P.xs_w + 4 * p_octet) * 4u : CONV_OOB;
+    }
+    const int p_slot = p_octet * ROWS + p_row;
+    constexpr int RAWS = TN == 1 ? 2 : 1;                               // items in registers: there is no room for two beside 128 columns
+    f32x4 raw[RAWS][2];
+    auto load_item = [&](f32x4 (&to)[2], int sixteen, int p) {
+        to[0] = buffer_load_x4(x_rsrc, p_voff[p], (uint32_t)sixteen * 64u);
+        to[1] = buffer_load_x4(x_rsrc, p_voff[p], (uint32_t)sixteen * 64u + 32u);
+    };
+    u32x4 part;
+    auto park = [&](u32x4* to, int p, int t) { to[t * 2 * ROWS + p_slot + 128 * p] = part; };
+    // ---- the rows of this wave's tiles, and which of their neighbours lie outside the image
+    const int a_zero = (half * ROWS + CONV_PATCH_ZEROS) * 16, row_bytes = P.W * 16;
+    int a_slot[TM];
+    uint64_t above[TM], below[TM], before[TM], behind[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int row = (wm * TM + i) * 32 + l32, m = m0 + row;
+        const int b = magic_div(m, P.howo_magic, P.howo_shift), r2 = m - b * P.Ho * P.Wo;
+        const int ho = magic_div(r2, P.wo_magic, P.wo_shift), wo = r2 - ho * P.Wo;
+        a_slot[i] = (half * ROWS + row) * 16;
+        above[i]  = __builtin_amdgcn_ballot_w64(ho == 0);
+        below[i]  = __builtin_amdgcn_ballot_w64(ho == P.H - 1);
+        before[i] = __builtin_amdgcn_ballot_w64(wo == 0);
+        behind[i] = __builtin_amdgcn_ballot_w64(wo == P.W - 1);
+    }
+    u32x4 bf[2][TN][3], af[TM][3];
+    // where tile i's rows lie under tap (r, s), and their part t from there (s is in the read's own offset)
+    int a_at[TM];
+    auto find_a = [&](int r, int s, int i) {
+        const uint64_t outside = (r == 0 ? above[i] : r == 2 ? below[i] : 0u) | (s == 0 ? before[i] : s == 2 ? behind[i] : 0u);
+        a_at[i] = a_slot[i] + r * row_bytes;
+        if (r != 1 || s != 1) asm volatile("v_cndmask_b32_e64 %0, %0, %1, %2" : "+v"(a_at[i]) : "v"(a_zero), "s"(outside));
+    };
+    auto read_a = [&](const u32x4* from, int s, int t, int i) {
+        af[i][t] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(from + t * 2 * ROWS + s) + a_at[i]);
+    };
+    const uint32_t b_lane = (uint32_t)lane * 16u;
+    auto load_b = [&](int step, int parity, int t, int j) {
+        bf[parity][j][t] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, b_lane, b_soff[j] + (uint32_t)step * 3072u + t * 1024u, 0);
+    };
+    f32x16 sum[TM * TN] = {};
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    constexpr int CH = TM * TN, NS = 6 * CH, BARRIER = 6 * TN - 4;
+    // which of the two items' twelve pieces follows a product of the nine steps, -1: none. One item in registers: the second is requested when
+    // the first has been taken apart, and has a step and a half to arrive.
+    constexpr auto item_piece = [](int place) {
+        for (int e = 0; e < 12; ++e) {
+            const int at = RAWS == 2 ? (e + 1) * 8 * NS / 12 - 1 : (e < 6 ? 3 * NS / 2 : 11 * NS / 2) + (e % 6 + 1) * 5 * NS / 12 - 1;
+            if (place == at) return e;
+        }
+        return -1;
+    };
+    float sign = 1.f / (CONV_SPLIT_SCALE * CONV_SPLIT_SCALE);            // (six groups of three steps per turn of the loop)
+    auto nine_steps = [&](auto buffer_, int sixteen) {
+        constexpr int buffer = decltype(buffer_)::value;
+        u32x4 *const mine = As + buffer * 6 * ROWS, *const other = As + (buffer ^ 1) * 6 * ROWS;
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) {
+            const int parity = (tap + buffer) & 1, next = tap == 8 ? 0 : tap + 1;
+            FENCE();
+#pragma unroll
+            for (int n = 0; n < NS; ++n) {
+                const int c = n / 6, t = n % 6, i = c / TN, j = c % TN;
+                if (tap == 8 && n == BARRIER) { __syncthreads(); FENCE(); }
+                sum[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i][CONV_SPLIT_PA[t]]), __builtin_bit_cast(bf16x8, bf[parity][j][CONV_SPLIT_PB[t]]),
+                                                                 tap % 3 == 0 && t == 0 ? f32x16{} : sum[c], 0, 0, 0);
+                // the chain before has seen its last product
+                if (tap % 3 == (c > 0 ? 2 : 0) && t >= 2) {
+                    const int pc = (c + CH - 1) % CH;
+#pragma unroll
+                    for (int v = 4 * t - 8; v < 4 * t - 4; ++v) acc[pc / TN][pc % TN][v] = __builtin_fmaf(sum[pc][v], sign, acc[pc / TN][pc % TN][v]);
+                }
+                // parts of A that have met their last column are replaced by the next step's
+                if (j == TN - 1 && t == 2) find_a(next / 3, next % 3, i);
+                if (j == TN - 1 && (t == 2 || t == 4 || t == 5)) read_a(tap == 8 ? other : mine, next % 3, t == 2 ? 2 : t == 4 ? 1 : 0, i);
+                // an item of the next 16 features: its three parts, in halves, then the request of a later one
+                const int place = tap * NS + n, e = item_piece(place), h = e % 6, item = e / 6;
+                if (e >= 0) {
+                    f32x4 (&numbers)[2] = raw[item % RAWS];
+                    part[2 * (h & 1)] = conv_split_word(numbers, h / 2, 2 * (h & 1));
+                    part[2 * (h & 1) + 1] = conv_split_word(numbers, h / 2, 2 * (h & 1) + 1);
+                    if (h & 1) park(other, item, h / 2);
+                    if (h == 5) load_item(numbers, sixteen + (RAWS == 2 || item == 1 ? 2 : 1), RAWS == 2 ? item : item ^ 1);
+                }
+                // the columns' parts of the next step but one
+#pragma unroll
+                for (int q = 0; q < TN; ++q)
+                    if (q < TN - 1 ? n == (CH - TN + q + 1) * 6 + 1 : n == NS - 1) {
+#pragma unroll
+                        for (int t2 = 0; t2 < 3; ++t2) load_b(9 * sixteen + tap + 2, parity, t2, q);
+                    }
+                FENCE();
+            }
+            if (tap % 3 == 0 && (tap > 0 || sixteen > kbeg)) sign = -sign;
+        }
+    };
+
+    f32x4 first[2][2];
+    load_item(first[0], kbeg, 0);
+    load_item(first[1], kbeg, 1);
+    FENCE();
+#pragma unroll
+    for (int p = 0; p < RAWS; ++p) load_item(raw[p], kbeg + 1, p);
+    FENCE();
+#pragma unroll
+    for (int parity = 0; parity < 2; ++parity)
+#pragma unroll
+        for (int q = 0; q < TN; ++q)
+#pragma unroll
+            for (int t = 0; t < 3; ++t) { load_b(9 * kbeg + parity, parity, t, q); FENCE(); }
+    conv_split_epilogue_operands<BN>(Es, epi, Dp, P, Dk, tid, n0);
+    if (tid < 36) As[(tid / 3) * ROWS + CONV_PATCH_ZEROS + tid % 3] = u32x4{0u, 0u, 0u, 0u};      // (no item lies there)
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) part[q] = conv_split_word(first[f], t, q);
+            park(As, f, t);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        find_a(0, 0, i);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) read_a(As, 0, t, i);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);                                  // (as in the kernel below)
+    for (int sixteen = kbeg; sixteen < kend; sixteen += 2) {             // (no branch inside: registers would spill)
+        nine_steps(std::integral_constant<int, 0>{}, sixteen);
+        nine_steps(std::integral_constant<int, 1>{}, sixteen + 1);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[TM - 1][TN - 1][v] = __builtin_fmaf(sum[CH - 1][v], sign, acc[TM - 1][TN - 1][v]);
+    __syncthreads();
+}
+
 // STEPS: an epilogue other than the straight-line one, step by step (ReLU6, a scalar or a vector in another place, a residual that is subtracted).
-template <int WGM, int WGN, int TM, int TN, bool STEPS>
+template <int WGM, int WGN, int TM, int TN, bool STEPS, bool PATCH>
 __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float* __restrict__ Es, int* __restrict__ Rs,
                                                 float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                                                 float* __restrict__ partial, uint32_t* __restrict__ arrivals, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
@@ -143,10 +372,11 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / WGN, wn = wave % WGN;
     const bool c_contig = P.flags & 1u, flat_rows = P.flags & 2u, masked = P.flags & 4u;
     const int nepi = (P.flags >> 8) & 15u, epi_first_full = (int)((P.flags >> 16) & 15u) - 1;
-    auto step_desc = [&](int e) -> uint32_t { return ((e < 3 ? P.epi_desc[0] : P.epi_desc[1]) >> (10 * (e < 3 ? e : e - 3))) & 1023u; };
+    auto step_desc = [&](int e) -> uint32_t { return conv_split_step_desc(P, e); };
 
-    const int ktiles = (P.K + 2 * BK - 1) / (2 * BK) * 2, slices = P.m_blocks, whole = P.split_tiles_m;
-    int work = (int)blockIdx.x, tile, slice = 0, kbeg = 0, kend = ktiles;
+    // k16 steps; what a slice is made of: k tiles, in pairs, or (PATCH) groups of nine steps, in pairs too
+    const int ktiles = (P.K + 2 * BK - 1) / (2 * BK) * 2, ksteps = PATCH ? P.K / 16 : 2 * ktiles, slices = P.m_blocks, whole = P.split_tiles_m;
+    int work = (int)blockIdx.x, tile, slice = 0, kbeg = 0, kend = PATCH ? ksteps / 9 : ktiles;
     if (work < whole) {
         tile = xcd_range(work, whole);
     } else {
@@ -168,7 +398,12 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     const uint32_t rowb = (uint32_t)P.N * 4u;
     float acc[TM][TN][16];
     uint32_t b_soff[TN];                             // the packed columns of this wave
-    {
+    // (blocks of columns beyond the last one lie outside the descriptor and read as zeros)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) b_soff[j] = (uint32_t)(n0 / 32 + wn * TN + j) * (uint32_t)ksteps * 3072u;
+    if constexpr (PATCH) {
+        conv_patch_sums<WGM, WGN, TM, TN>(pool, Es, acc, b_soff, x, w_rsrc, epi, Dp, P, Dk, wave, m0, n0, kbeg, kend);
+    } else {
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
     // ---- load assignment: A item = (row, octet of k); octet o holds k = 4o..4o+3 and 16+4o..16+4o+3 of the k tile
     constexpr int A_NI = BM * 4 / NT, A_RSTEP = NT / 4;
@@ -196,9 +431,6 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                 a_inv[p] |= ((uint32_t)(hi0 + r * P.DH) >= (uint32_t)P.H ? wall : wbad) << (r * P.KW);
         }
     }
-    // (blocks of columns beyond the last one lie outside the descriptor and read as zeros)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) b_soff[j] = (uint32_t)(n0 / 32 + wn * TN + j) * (uint32_t)ktiles * 6144u;
     const uint32_t b_lane = (uint32_t)lane * 16u;
     int t_r = 0, t_s = 0, t_c = kbeg * BK;          // kernel tap and first feature of the next k tile to load
     if (kbeg > 0 && P.KH * P.KW > 1) {
@@ -235,17 +467,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
 #pragma unroll
     for (int i = 0; i < TM; ++i) a_slot[i] = half * BM + (((wm * TM + i) * 32 + l32) ^ (half * 2));
     auto read_a = [&](const u32x4* from, int ks, int t, int i) { af[i][t] = from[(t * 4 + 2 * ks) * BM + (a_slot[i] ^ (ks * 4))]; };
-#define FENCE() __builtin_amdgcn_sched_barrier(0)
-    // An item's next part, and what is left of it: the eight numbers' nearest bf16, to LDS at `to`
     const int p_slot = a_o * BM + (a_r0 ^ (a_o * 2));
-    auto split_word = [&](f32x4 (&x)[2], int t, int q) {
-        f32x4& v = x[q >> 1];
-        const int e = 2 * (q & 1);
-        if (t == 0) { v[e] *= CONV_SPLIT_SCALE; v[e + 1] *= CONV_SPLIT_SCALE; }
-        const uint32_t w2 = to_bf16x2(v[e], v[e + 1]);
-        if (t < 2) { v[e] = minus_low(w2, v[e]); v[e + 1] = minus_high(w2, v[e + 1]); }
-        return w2;
-    };
     u32x4 part;
     auto park = [&](u32x4* to, int p, int t) { to[t * 4 * BM + (p_slot ^ (p * A_RSTEP))] = part; };
 
@@ -259,7 +481,6 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     // The small products of a k step come first, (A part, B part): a sum that begins there is cut off once at its full size and not four
     // times. (Of 512 terms 512, 16 and 1 that are not zero: errors of 1.22e-7, 7.6e-8 and 3.5e-8 of the results' 2-norm, with the largest
     // product first 1.36e-7, 8.9e-8 and 5.3e-8, through fp32 products 2.1e-7, 5.9e-8 and 2.5e-8; no slower.)
-    constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
     constexpr int CH = TM * TN, NS = 6 * CH;
     float sign = kbeg & 2 ? -1.f / (CONV_SPLIT_SCALE * CONV_SPLIT_SCALE) : 1.f / (CONV_SPLIT_SCALE * CONV_SPLIT_SCALE);
     auto k16_step = [&](auto step_, int kt) {
@@ -273,7 +494,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         for (int n = 0; n < NS; ++n) {
             const int c = n / 6, t = n % 6, i = c / TN, j = c % TN;
             if (ks == 1 && n == BARRIER) { __syncthreads(); FENCE(); }
-            sum[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i][PA[t]]), __builtin_bit_cast(bf16x8, bf[ks][j][PB[t]]),
+            sum[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i][CONV_SPLIT_PA[t]]), __builtin_bit_cast(bf16x8, bf[ks][j][CONV_SPLIT_PB[t]]),
                                                              step == 0 && t == 0 ? f32x16{} : sum[c], 0, 0, 0);
             // the chain before has seen its last product
             if (step == (c > 0 ? 3 : 0) && t >= 2) {
@@ -286,8 +507,8 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
             // an item of a later k tile
             if (n >= SPLIT && (n - SPLIT) % EACH == EACH - 1 && (n - SPLIT) / EACH < 6) {
                 const int h = (n - SPLIT) / EACH, pt = h / 2;
-                part[2 * (h & 1)] = split_word(raw[item], pt, 2 * (h & 1));
-                part[2 * (h & 1) + 1] = split_word(raw[item], pt, 2 * (h & 1) + 1);
+                part[2 * (h & 1)] = conv_split_word(raw[item], pt, 2 * (h & 1));
+                part[2 * (h & 1) + 1] = conv_split_word(raw[item], pt, 2 * (h & 1) + 1);
                 if (h & 1) park(to, item, pt);
                 if (h == 5) load_item(raw[item], kt + (ks == 0 ? 2 : 3), item);
             }
@@ -319,32 +540,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
 #pragma unroll
             for (int t = 0; t < 3; ++t) { load_b(kbeg, ks, t, q); FENCE(); }
         }
-    // ---- epilogue operands
-    if (tid < BN) {
-        float e_reg[CONV_MAX_EPI], d_in[CONV_MAX_DERIVED + 1];
-#pragma unroll
-        for (int e = 0; e < CONV_MAX_EPI; ++e) {
-            const uint32_t kind = step_desc(e) >> 8;
-            const uint32_t present = epi.p[e] != nullptr ? 1u : 0u;
-            e_reg[e] = buffer_load_x1(make_rsrc(epi.p[e], kind == 1 ? 4u * present : kind == 2 ? (uint32_t)P.N * 4u * present : 0u),
-                                      kind == 2 ? (uint32_t)(n0 + tid) * 4u : 0u);
-        }
-        if (Dk.nsteps) {
-#pragma unroll
-            for (int k = 0; k <= CONV_MAX_DERIVED; ++k) {
-                const bool vec = (Dk.vector_mask >> k) & 1u;
-                d_in[k] = buffer_load_x1(make_rsrc(Dp.p[k], Dp.p[k] == nullptr ? 0u : vec ? (uint32_t)P.N * 4u : 4u),
-                                         vec ? (uint32_t)(n0 + tid) * 4u : 0u);
-            }
-            const float v = conv_derived_value(d_in, Dk);
-#pragma unroll
-            for (int e = 0; e < CONV_MAX_EPI; ++e)
-                if (e == (int)Dk.step) e_reg[e] = v;
-        }
-#pragma unroll
-        for (int e = 0; e < CONV_MAX_EPI; ++e)
-            if (e < nepi) Es[e * BN + tid] = e_reg[e];
-    }
+    conv_split_epilogue_operands<BN>(Es, epi, Dp, P, Dk, tid, n0);
 
     {
 #pragma unroll
@@ -352,7 +548,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
 #pragma unroll
             for (int t = 0; t < 3; ++t) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) part[q] = split_word(first[f], t, q);
+                for (int q = 0; q < 4; ++q) part[q] = conv_split_word(first[f], t, q);
                 park(As + f / 2 * 12 * BM, f & 1, t);
             }
         }
@@ -453,27 +649,29 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
             f32x4 a_next[2];
             u32x4 b_next[TN][3];
             auto request = [&](int step) {
-                const int hi = hi0 + r * P.DH, wi = wi0 + s * P.DW, o = 2 * (step & 1) + half, k = (step >> 1) * BK + 4 * o;
+                const int hi = hi0 + r * P.DH, wi = wi0 + s * P.DW, o = PATCH ? half : 2 * (step & 1) + half, k = PATCH ? 16 * step : (step >> 1) * BK + 4 * o;
                 const bool ok = m < P.M && (flat_rows || ((uint32_t)hi < (uint32_t)P.H && (uint32_t)wi < (uint32_t)P.W));
                 const uint32_t at = row + (uint32_t)(r * P.DH * P.xs_h + s * P.DW * P.xs_w + c + 4 * o) * 4u;
                 a_next[0] = buffer_load_x4(x_rsrc, ok && k < P.K ? at : CONV_OOB);
-                a_next[1] = buffer_load_x4(x_rsrc, ok && k + 16 < P.K ? at + 64u : CONV_OOB);
+                a_next[1] = buffer_load_x4(x_rsrc, ok && k + (PATCH ? 8 : 16) < P.K ? at + (PATCH ? 32u : 64u) : CONV_OOB);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
                     for (int q = 0; q < 3; ++q)
                         b_next[j][q] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, b_lane, b_soff[j] + (uint32_t)step * 3072u + (uint32_t)q * 1024u, 0);
-                if (step & 1) {
+                if constexpr (PATCH) {
+                    if (++s == 3) { s = 0; if (++r == 3) { r = 0; c += 16; } }
+                } else if (step & 1) {
                     c += BK;
                     if (c >= P.Cin) { c = 0; if (++s == P.KW) { s = 0; ++r; } }
                 }
             };
-            f32x16 again[TN] = {}, total[TN] = {};          // (summed by 64 k, as rounded as in the loop above)
+            f32x16 again[TN] = {}, total[TN] = {};          // (summed by as many k, as rounded as in the loop above)
             request(0);
 #pragma nounroll
-            for (int step = 0; step < 2 * ktiles; ++step) {
+            for (int step = 0; step < ksteps; ++step) {
                 float av[8], bv[TN][8];
-                const float sign_k = step & 4 ? -1.f : 1.f;
+                const float sign_k = (PATCH ? step / 3 & 1 : step & 4) ? -1.f : 1.f;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     av[e] = a_next[e >> 2][e & 3];
@@ -491,7 +689,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                 for (int e = 0; e < 8; ++e)
 #pragma unroll
                     for (int j = 0; j < TN; ++j) again[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], bv[j][e], again[j], 0, 0, 0);
-                if ((step & 3) == 3) {
+                if (PATCH ? step % 3 == 2 : (step & 3) == 3) {
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -632,21 +830,25 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         }
 }
 
-#define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE, STEPS)                                                                \
+#define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE, STEPS, PATCH)                                                         \
     extern "C" __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void name(             \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                                   \
         float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) { \
-        __shared__ __attribute__((aligned(16))) u32x4 pool[24 * 32 * WGM * TM];                                              \
+        __shared__ __attribute__((aligned(16))) u32x4 pool[PATCH ? 12 * CONV_PATCH_ROWS : 24 * 32 * WGM * TM];               \
         __shared__ float Es[CONV_MAX_EPI * 32 * WGN * TN];                                                                   \
         __shared__ int Rs[32 * WGM * TM];                                                                                    \
-        conv_split_body<WGM, WGN, TM, TN, STEPS>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);             \
+        conv_split_body<WGM, WGN, TM, TN, STEPS, PATCH>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);          \
     }
 // _steps: 50176 x 128 x 512 with a ReLU6 68 us, with a scalar 62, with `relu(y) + r` 82 (each as launches of its own behind the product: 83, 82, 94;
 // in the fp32 kernels 73, 71, 73); 50176 x 256 x 512 97, 89, 108 (127, 120, 130). (Words of a full tensor requested for two tiles at a time
 // instead of one: 80 instead of 82, not kept; for four: registers spill.)
 // (2 x 2 waves of 64 x 64: 255 registers, two blocks per CU; 1 x 4 waves of 128 x 32, which load every column once, were 1 % slower)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x128, 2, 2, 2, 2, 2, false)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x128_steps, 2, 2, 2, 2, 2, true)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128, 2, 2, 2, 2, 2, false, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128_patch, 2, 2, 2, 2, 2, false, true)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128_steps, 2, 2, 2, 2, 2, true, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128_patch_steps, 2, 2, 2, 2, 2, true, true)
 // for at most 64 columns, or where the smaller tile divides the rows better among the CUs: three blocks per CU
-CONV_SPLIT_KERNEL(conv_gemm_split_128x64, 2, 2, 2, 1, 3, false)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x64_steps, 2, 2, 2, 1, 3, true)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64, 2, 2, 2, 1, 3, false, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch, 2, 2, 2, 1, 3, false, true)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_steps, 2, 2, 2, 1, 3, true, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_steps, 2, 2, 2, 1, 3, true, true)

@@ -50,6 +50,7 @@ class _Choices:
         conv_stem=None,                  #the patch kernel for few input features: False = never; None / True: where it applies; 64: its 64-position tiles only
         conv_split=None,                 #the kernels on the bf16 matrix cores: None = where they pay, False = never, True or a tile's name = wherever they apply
         conv_split_slices=None,          #blocks that share a tile behind the whole rounds (None: by the estimate)
+        conv_patch=None,                 #the bf16 kernels that hold a patch of the input in LDS: None = wherever they apply (a pinned conv_split: never), True = wherever they apply, False = never
         wgrad_split=None,                #kernel gradients on the bf16 matrix cores: None = where they pay, False = never, a tile's name = wherever it applies
         wgrad_slices=None,               #slices of a kernel gradient's contraction (None: by the estimate)
         conv_k_splits=None,              #slices a contraction is cut into where that applies (None: by the heuristic, 1: never)
@@ -1069,6 +1070,10 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
 
 #tile -> (BM, BN, microseconds of a CU per k tile of 32: with several blocks on it, with one)
 CONV_SPLIT_TILES = {'128x128': (128, 128, 1.15, 1.15), '128x64': (128, 64, 0.65, 0.95)}
+#tile -> microseconds of a CU per k tile of 32 for the kernels that hold a patch of the input in LDS, and what a block's start and end cost, and those
+#of a slice, in k tiles. (Products alone, 128x64 and 128x128: 64 x 28 x 28 x 128 x 128 74.7 in 832 blocks and 75.9, 64 x 14 x 14 x 256 x 256 78.7, 75.2, 64 x 7 x 7
+#x 512 x 512 80.1, 78.1 in 200 blocks, 16 x 7 x 7 x 512 x 512 73.9 in 56 blocks, 41.8 in 112, 29.2 in 224; 119, 66, 41.)
+CONV_PATCH_STEP, CONV_PATCH_START, CONV_PATCH_SLICE = {'128x128': 0.88, '128x64': 0.5}, 8, 16
 #Products below these stay with the fp32 kernels. Rows: packing the kernel operand costs what about 250 rows' products cost,
 #and one launch. Contraction: with two k tiles of 32 a block is all start-up and stores (200704 x 64 x 256 with residual:
 #101 us here, 66 there, where a block walks several tiles; 50176 x 128 x 512: 59 against 61). Operations: start and end of two launches. A
@@ -1091,6 +1096,7 @@ class ConvSplit(tp.NamedTuple):
     slices: int
     partial: tp.Optional[Buffer] = None
     arrivals: tp.Optional[Buffer] = None
+    patch: bool = False               #by the kernels that hold a patch of the input in LDS (conv_patch_applies)
 
 
 def conv_split_tiles(split: ConvSplit, g: ConvGeometry) -> tp.Tuple[int, int]:
@@ -1105,7 +1111,29 @@ def conv_split_partial_words(split: ConvSplit, g: ConvGeometry) -> int:
 
 
 def conv_split_packed_words(g: ConvGeometry) -> int:
+    if g.split is not None and g.split.patch:
+        return _cdiv(g.N, 32) * (g.K // 64) * (CONV_SPLIT_PACK_BYTES // 4) + _cdiv(g.N, 32) * (g.K % 64) * (CONV_SPLIT_PACK_BYTES // 4 // 64)
     return _cdiv(g.N, 32) * _cdiv(g.K, 64) * (CONV_SPLIT_PACK_BYTES // 4)
+
+
+def conv_patch_applies(g: ConvGeometry) -> bool:
+    '''3 x 3 windows at a stride of 1 over dense images with a border of one: the positions of a tile and their neighbours are
+    consecutive in memory. A patch has room for 256 positions (128 + 2 W + 2).'''
+    return ((g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, g.LH, g.LW) == (3, 3) + (1,) * 8
+            and g.Ho == g.H and g.Wo == g.W and g.W <= 63 and g.Cin % 32 == 0 and g.xs[2] >= g.Cin
+            and g.xs[1] == g.W * g.xs[2] and g.xs[0] == g.H * g.xs[1])
+
+
+def _conv_patch_pays(g: ConvGeometry, c_contig: bool) -> bool:
+    '''Where the kernels that hold a patch are faster, packing included, than the fp32 kernels (images x H x W x features x columns: there, here).'''
+    flops = 2 * g.M * g.N * g.K
+    if _four_waves_per_tile(g, True, c_contig, CONV_SPLIT_ROUND):
+        #4 x 28 x 28 x 128 x 128 (0.9 GFLOP) 17.6, 19.1; 8 x 14 x 14 x 256 x 256 (1.8) 28.8, 25.1; 8 x 7 x 7 x 512 x 512 32.2, 29.9; 16 x 7 x 7 x 512 x 512 51.4, 36.9
+        return flops >= 1.8e9
+    #one wave walks the whole contraction there: 1 x 7 x 7 x 96 x 96 21.4, 14.9; 1 x 10 x 10 x 160 x 40 33.4, 15.5; 1 x 7 x 7 x 480 x 480 93, 28; 4 x 56 x 56 x 64 x 64 17.2,
+    #16.9; 64 x 56 x 56 x 64 x 32 114, 71. The shortest, 32 features: 9 x 30 x 30 x 100 columns (0.47 GFLOP) 11.0, 12.7; 20 x 30 x 30 x 64 (0.66) 16.6, 12.8; 8 x 56 x 56 x 48
+    #(0.69) 15.8, 13.0; of at most 32 columns 64 x 28 x 28 x 24 16.4, 17.2; 32 x 56 x 56 x 32 26.6, 27.5
+    return g.K >= 576 or (g.N > 32 and flops >= 0.6e9)
 
 
 def _conv_split_pays(g: ConvGeometry, c_contig: bool) -> bool:
@@ -1138,26 +1166,30 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
     _, _, a_fast, _, c_contig = _conv_fast_paths(lhs, lhs, g, 0)
     if not a_fast or (g.Cin % 32 != 0 and g.KH * g.KW != 1) or conv_split_packed_words(g) * 4 >= 2**31 or M * N == 0:
         return None
-    if not (CHOICES.conv_split or CHOICES.conv_split_slices) and not _conv_split_pays(g, c_contig):
+    #(pinned to other kernels of this family, a product is theirs)
+    wanted = CHOICES.conv_split is None and CHOICES.conv_split_slices is None if CHOICES.conv_patch is None else CHOICES.conv_patch
+    patch  = bool(wanted) and conv_patch_applies(g)
+    if not (CHOICES.conv_split or CHOICES.conv_split_slices) and not (_conv_patch_pays if patch else _conv_split_pays)(g, c_contig):
         return None
     #The whole tiles are dealt out in rounds of one per CU; the contraction of those of the last, incomplete round (or of all,
     #if there are fewer tiles than CUs) may be cut into slices, of two k tiles at least. A block's start and end cost about
-    #three k tiles, a slice's partial sums five more.
-    ktiles, best = 2 * _cdiv(K, 64), None
+    #three k tiles, a slice's partial sums five more (a patch has to be complete before the first product: eight).
+    ktiles, best = K // 32 if patch else 2 * _cdiv(K, 64), None
     for tile, (bm, bn, shared_step, lone_step) in CONV_SPLIT_TILES.items():
         if CHOICES.conv_split not in (None, True, tile):
             continue
         tiles = _cdiv(M, bm) * _cdiv(N, bn)
         for slices in range(1, 17):
             whole = tiles if slices == 1 else tiles // CONV_SPLIT_ROUND * CONV_SPLIT_ROUND
-            if slices > 1 and (ktiles < 2 * slices or whole == tiles) or CHOICES.conv_split_slices not in (None, slices):
+            if slices > 1 and (ktiles < (9 if patch else 2) * slices or whole == tiles) or CHOICES.conv_split_slices not in (None, slices):
                 continue
             blocks = whole + (tiles - whole) * slices
             rounds = whole / CONV_SPLIT_ROUND if slices > 1 else _cdiv(tiles, CONV_SPLIT_ROUND)
-            time   = ((shared_step if blocks > CONV_SPLIT_ROUND else lone_step)
-                      * (rounds * (ktiles + 3) + _cdiv((tiles - whole) * slices, CONV_SPLIT_ROUND) * (ktiles / slices + 8)))
+            step   = CONV_PATCH_STEP[tile] if patch else shared_step if blocks > CONV_SPLIT_ROUND else lone_step
+            start, slice_start = (CONV_PATCH_START, CONV_PATCH_SLICE) if patch else (3, 8)
+            time   = step * (rounds * (ktiles + start) + _cdiv((tiles - whole) * slices, CONV_SPLIT_ROUND) * (ktiles / slices + slice_start))
             if best is None or time < best[0]:
-                best = (time, ConvSplit(tile, whole, slices))
+                best = (time, ConvSplit(tile, whole, slices, patch=patch))
     return best[1] if best else None
 
 
@@ -1165,8 +1197,9 @@ def conv_split_pack(packed: Buffer, source: EwOperand, g: ConvGeometry) -> Launc
     '''The kernel operand of a product, element (ky, kx, c, n) at source.offset + (ky, kx, c, n) . source.strides, taken
     apart into three bf16 parts and laid out for the matrix cores.'''
     assert packed.size == conv_split_packed_words(g)
-    params = _i32(g.N, g.K, g.Cin, g.KW, *source.strides)
-    blocks = _cdiv(g.N, 32) * _cdiv(g.K, 64)
+    patch  = g.split is not None and g.split.patch
+    params = _i32(g.N, -g.K if patch else g.K, g.Cin, g.KW, *source.strides)
+    blocks = _cdiv(_cdiv(g.N, 32) * (g.K // 16), 4) if patch else _cdiv(g.N, 32) * _cdiv(g.K, 64)
     return Launch('conv_split_pack', (blocks, 1, 1), (BLOCK, 1, 1), [(packed, 0), (source.buffer, source.offset * 4)], params,
                   bytes_moved=4 * (packed.size + g.K * g.N))
 
@@ -1204,7 +1237,8 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
     descs  = [0, 0]
     for i, e in enumerate(epilogue):
         descs[i // 3] |= ((0 if masked else e.op * 2 + int(e.operand_left)) | e.kind << 8) << (10 * (i % 3))
-    (tiles_m, tiles_n), kpairs = conv_split_tiles(split, g), _cdiv(K, 64)
+    (tiles_m, tiles_n), kpairs = conv_split_tiles(split, g), g.Cin // 32 if split.patch else _cdiv(K, 64)
+    assert not split.patch or conv_patch_applies(g)
     shared = tiles_m * tiles_n - split.whole
     params = (_i32(M, N, K, g.Ho, g.Wo, g.H, g.W, g.Cin, g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, *g.xs[:3], tiles_m, tiles_n)
               + _u32(flags, *descs, (lhs.size - lhs_offset) * 4, packed.size * 4, (out.size - out_offset) * 4,
@@ -1217,7 +1251,7 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
         operand_slots[-1] = (taps[0][1], 0)
         nbytes += 4 * taps[0][1].size
     scratch = [(split.partial, 0), (split.arrivals, 0)] if shared else [(None, 0), (None, 0)]
-    return Launch(f'conv_gemm_split_{split.tile}' + ('_steps' if steps else ''), (split.whole + shared * split.slices, 1, 1), (256, 1, 1),
+    return Launch(f'conv_gemm_split_{split.tile}' + ('_patch' if split.patch else '') + ('_steps' if steps else ''), (split.whole + shared * split.slices, 1, 1), (256, 1, 1),
                   [(out, out_offset * 4), (lhs, lhs_offset * 4), (packed, 0)] + scratch + operand_slots + derived_ptrs,
                   params + derived_desc, bytes_moved=nbytes, flops=2 * M * N * K,
                   written=(0, 3, 4) if shared else (0,), scratch=(3, 4) if shared else ())

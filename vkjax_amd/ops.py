@@ -576,9 +576,9 @@ def _split_ops(bufferpool, equation, outbuf, lhs: Buffer, rhs: Buffer, geom: 'K.
                              arrivals=bufferpool.zeroed_scratch(K.CONV_SPLIT_ROUND, 'arrivals of partial products'))
     position = bufferpool.op_counter
     bufferpool.op_counter -= 1                  #the packed operand lives at the equation's own position
+    geom   = geom._replace(split=plan)
     packed = bufferpool.new_temporary(np.uint32, (K.conv_split_packed_words(geom),))
     bufferpool.op_counter = position
-    geom   = geom._replace(split=plan)
     source = EwOperand(rhs, rhs_offset, tuple(geom.ws))
     pack   = Op(equation, launch=K.conv_split_pack(packed, source, geom), meta=('conv_pack', packed, source, geom))
     if part_at is not None:
