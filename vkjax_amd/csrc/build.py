@@ -1,11 +1,12 @@
-'''Build the native parts in-tree: the C-ABI runtime (libvkjax_hip.so) and the gfx950 code
-objects with the kernels (one .hsaco per kernels/*.hip). Needs only hipcc; no GPU.
+'''Build the native parts in-tree: the C-ABI runtime (libvkjax_hip.so), the extension module that makes
+calls natively (vkjax_call.so) and the gfx950 code objects with the kernels (one .hsaco per kernels/*.hip). Needs only hipcc; no GPU.
 
     python -m vkjax_amd.csrc.build [--force]
 '''
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 CSRC    = os.path.dirname(os.path.abspath(__file__))
@@ -65,6 +66,16 @@ def build_shim(force=True):
     return out
 
 
+def build_call(force=True):
+    '''vkjax_call.so: the extension module that makes calls of wrapped functions natively (host only).'''
+    import numpy
+    src, out = os.path.join(CSRC, 'call.cpp'), os.path.join(LIBDIR, 'vkjax_call.so')
+    if not force and _newer(out, [src]):
+        return out
+    _run(['g++', '-O2', '-fPIC', '-shared', '-std=c++17', f'-I{sysconfig.get_paths()["include"]}', f'-I{numpy.get_include()}', src, '-o', out])
+    return out
+
+
 def build_kernel(name, force=True):
     src  = os.path.join(CSRC, 'kernels', f'{name}.hip')
     deps = [src] + [os.path.join(CSRC, 'kernels', h) for h in ('common.h', 'ew_opcodes.h', 'ew_apply.h', 'conv_split.h', 'split_bf16.h', 'wgrad_split.h')]
@@ -79,7 +90,7 @@ def build_all(force=True, jobs=None):
     os.makedirs(LIBDIR, exist_ok=True)
     jobs = jobs or min(8, os.cpu_count() or 1)
     with ThreadPoolExecutor(jobs) as pool:
-        futures = [pool.submit(build_shim, force)] + [pool.submit(build_kernel, k, force) for k in KERNEL_SOURCES]
+        futures = [pool.submit(build_shim, force), pool.submit(build_call, force)] + [pool.submit(build_kernel, k, force) for k in KERNEL_SOURCES]
         return [f.result() for f in futures]
 
 

@@ -93,13 +93,25 @@ class Function:
         self.jaxpr_function      = make_jaxpr(function, static_argnums, return_shape=True)
         self._jaxpr_interpreters = dict()
         self._output_shapes      = dict()
+        #(native plan of a call, its sequence's attributes) per signature, the newest first
+        self._plans              = []
         self._profiling          = profiling
         self._static_argnums     = tuple(static_argnums)
         kwargs['profiling']      = profiling
         kwargs['static_argnums'] = static_argnums
         self._interpreter_args   = (args, kwargs)
 
+    #signatures whose calls are made natively; those of older ones take the general path
+    MAX_PLANS = 16
+
     def __call__(self, *args: tp.Any, **kwargs: tp.Any) -> tp.Any:
+        if not kwargs:
+            for plan, sequence in self._plans:
+                #(an evaluation that something has been put in front of is made by the general path, which goes through it)
+                if 'eval' not in sequence:
+                    output = plan(args)
+                    if output is not NotImplemented:
+                        return output
         if self._tree is tree_util and not kwargs:
             #the arguments are flattened once, for the cache key and for the run
             leaves, structure = tree_util.tree_flatten(args)
@@ -340,6 +352,12 @@ class Function:
                 iargs, ikwargs       = self._interpreter_args
                 self._jaxpr_interpreters[shape_structure] = JaxprInterpreter(jaxpr, *iargs, **ikwargs)
                 self._output_shapes[shape_structure]      = output_shapes
+                if self._tree is tree_util and not self._profiling:
+                    interpreter = self._jaxpr_interpreters[shape_structure]
+                    leaves      = (flattened or tree_util.tree_flatten(args))[0]
+                    plan        = interpreter.call_plan(leaves, shape_structure[2].children, tree_util.tree_structure(output_shapes))
+                    if plan is not None:
+                        self._plans = [(plan, interpreter.sequence.__dict__)] + self._plans[:self.MAX_PLANS - 1]
         return self._jaxpr_interpreters[shape_structure], self._output_shapes[shape_structure]
 
     def _restore_shapes(self, x, targetshapes):

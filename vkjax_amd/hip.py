@@ -7,6 +7,7 @@ if the library or the code objects are missing, or no GPU is present, constructi
 raises.
 '''
 import ctypes as C
+import importlib.util
 import os
 import threading
 import typing as tp
@@ -75,6 +76,7 @@ _PROTOTYPES = {
 }
 
 _lib      = None
+_call_module = None
 _lib_lock = threading.Lock()
 
 
@@ -97,14 +99,37 @@ def load_library() -> C.CDLL:
     return _lib
 
 
+def function_address(name: str) -> int:
+    return C.cast(getattr(load_library(), name), C.c_void_p).value
+
+
+def load_call_module():
+    '''The extension module whose plans make calls natively (csrc/call.cpp). Raises if it has not been built.'''
+    global _call_module
+    with _lib_lock:
+        if _call_module is None:
+            path = os.path.join(LIBDIR, 'vkjax_call.so')
+            if not os.path.exists(path):
+                raise RuntimeError(f'{path} is missing: build it with `python -m vkjax_amd.csrc.build`')
+            spec   = importlib.util.spec_from_file_location('vkjax_call', path)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            _call_module = module
+    return _call_module
+
+
 class HipError(RuntimeError):
     pass
 
 
+def last_error(status: int, what: str) -> HipError:
+    msg = load_library().vkj_last_error().decode('utf8', 'replace')
+    return HipError(f'{what} failed with status {status}: {msg}')
+
+
 def _check(status: int, what: str):
     if status != 0:
-        msg = load_library().vkj_last_error().decode('utf8', 'replace')
-        raise HipError(f'{what} failed with status {status}: {msg}')
+        raise last_error(status, what)
 
 
 def device_count() -> int:

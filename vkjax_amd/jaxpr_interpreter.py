@@ -283,16 +283,55 @@ class JaxprInterpreter:
         try:
             self.sequence.eval(host, flags=hip.EVAL_NULL_IS_RESIDENT, next_host_arrays=next_host_arrays)
         except BaseException:
-            self._resident_leaves.clear()                       #nothing is known about what reached HBM
-            for key, b in self.bufferpool.buffers.items():
-                if isinstance(key, tuple) and key[:1] == ('zeroed',):
-                    try:
-                        b.tensor.upload(np.zeros(b.size, np.uint32))
-                    except Exception:                            #a device that is gone reports the first error
-                        pass
+            self._recover()
             raise
         finally:
             self._evaluations += 1
+
+    def _recover(self):
+        self._resident_leaves.clear()                           #nothing is known about what reached HBM
+        for key, b in self.bufferpool.buffers.items():
+            if isinstance(key, tuple) and key[:1] == ('zeroed',):
+                try:
+                    b.tensor.upload(np.zeros(b.size, np.uint32))
+                except Exception:                                #a device that is gone reports the first error
+                    pass
+
+    def _evaluated(self, status: int):
+        '''What `evaluate` does around an evaluation, for one that a call's native plan has made (csrc/call.cpp).'''
+        self._evaluations += 1
+        if status:
+            error = hip.last_error(status, 'vkj_seq_eval')       #(recovering may leave another message)
+            self._recover()
+            raise error
+
+    def call_plan(self, leaves, argument_structures, result_structure):
+        '''The native plan of calls with arguments like these (`leaves` in containers of these structures, minijax.tree_util) and
+        results of that structure, or None where the general path has something to do that a plan does not: arguments converted
+        or checked on the host, results that are.'''
+        plain = {np.dtype(np.float32): 'f', np.dtype(np.int32): 'i', np.dtype(np.uint32): 'u'}
+        avals, outs = [v.aval for v in self.jaxpr.jaxpr.invars], [v.aval for v in self.jaxpr.jaxpr.outvars]
+        if (self.sequence is None or self.profiling or self.static_argnums or self.resident_argnums
+                or any(core.is_key_dtype(a.dtype) or np.dtype(a.dtype) not in plain for a in avals + outs)
+                or any(b is None for b in self.output_buffers) or any(np.dtype(b.dtype) not in plain for b in self.output_buffers)
+                or len(leaves) != len(avals) or result_structure.num_leaves != len(outs)
+                or any(type(x) is not np.ndarray or x.dtype != a.dtype or x.shape != tuple(a.shape) for x, a in zip(leaves, avals))):
+            return None
+
+        def specification(structure, leaves):
+            if structure.kind == 'leaf':
+                aval, slot = next(leaves)
+                return ('a', tuple(int(n) for n in aval.shape), plain[np.dtype(aval.dtype)], -1 if slot is None else slot)
+            if structure.kind == 'none':
+                return ('n',)
+            children = [specification(c, leaves) for c in structure.children]
+            return ('d', list(structure.meta), children) if structure.kind == 'dict' else (structure.kind[0], children)
+
+        inputs    = iter(zip(avals, self._input_slots))
+        arguments = [specification(c, inputs) for c in argument_structures]
+        result    = specification(result_structure, iter(zip(outs, self._output_slots)))
+        return hip.load_call_module().Plan(self, self._resident_leaves, hip.function_address('vkj_seq_eval'), self.sequence.handle, self.sequence.n_slots,
+                                           hip.EVAL_NULL_IS_RESIDENT, arguments, result)
 
     def run_leaves(self, per_argument):
         '''`run` for a caller that has flattened the arguments already: one list of leaves per argument.'''
