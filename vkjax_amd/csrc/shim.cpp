@@ -223,6 +223,11 @@ int issue_launch(Ctx* c, Launch& l, hipStream_t stream = nullptr) {
     return 0;
 }
 
+// whether the kernel that carries ranges takes this one: it copies words
+bool carried(const void* device, const void* staging, size_t nbytes) {
+    return (((uintptr_t)device | (uintptr_t)staging | nbytes) & 3u) == 0;
+}
+
 void drop_graph(Seq* s) {
     if (s->graph_exec) { hipGraphExecDestroy(s->graph_exec); s->graph_exec = nullptr; }
     s->graph_failed = false;
@@ -482,6 +487,35 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                     first_launch = s->early_at + 1;
                 }
             }
+        } else if (c->carry) {
+            // (neighbours in HBM that are neighbours in their staging memory: one range, with what lies between them)
+            Carry what;
+            const Slab* slab = nullptr;                  // of the last range
+            for (auto& t : s->uploads) {
+                if (!t.nbytes || !host_ptrs[t.slot]) continue;
+                memcpy(t.staging, host_ptrs[t.slot], t.nbytes);
+                char* device = (char*)t.buf->dptr + t.offset;
+                if (!carried(device, t.staging, t.nbytes)) {
+                    HIP_TRY(hipMemcpyAsync(device, t.staging, t.nbytes, hipMemcpyHostToDevice, c->stream));
+                    continue;
+                }
+                if (what.count && t.staging_mirrors_slab && t.buf->slab == slab) {
+                    auto& last = what.range[what.count - 1];
+                    const size_t step = (uintptr_t)device - (uintptr_t)last.dst;
+                    if ((uintptr_t)device > (uintptr_t)last.dst && step == (uintptr_t)t.staging - (uintptr_t)last.src && step >= last.nbytes
+                            && step < last.nbytes + PACKED_ALIGN) {
+                        last.nbytes = step + t.nbytes;
+                        continue;
+                    }
+                }
+                slab = t.staging_mirrors_slab ? t.buf->slab : nullptr;
+                if (what.count == Carry::MAX) {
+                    if (int r = c->carry(what, false, c->stream)) return r;
+                    what.count = 0;
+                }
+                what.range[what.count++] = {device, t.staging, t.nbytes};
+            }
+            if (int r = c->carry(what, false, c->stream)) return r;
         } else {
             for (auto& t : s->uploads) {
                 if (!t.nbytes || !host_ptrs[t.slot]) continue;
@@ -553,8 +587,20 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
     // queue in order, and a download queued first waits there for the launches, with every upload
     // behind it, even one from the other stream, waiting as well.
     size_t nchunk_events = 0;
+    if (down && c->carry) {
+        Carry what;
+        for (auto& t : s->downloads) {
+            if (!t.nbytes || t.nbytes > CARRY_OUT_MAX || !carried((char*)t.buf->dptr + t.offset, t.staging, t.nbytes)) continue;
+            if (what.count == Carry::MAX) {
+                if (int r = c->carry(what, true, c->stream)) return r;
+                what.count = 0;
+            }
+            what.range[what.count++] = {t.staging, (char*)t.buf->dptr + t.offset, t.nbytes};
+        }
+        if (int r = c->carry(what, true, c->stream)) return r;
+    }
     if (down) for (auto& t : s->downloads) {
-        if (!t.nbytes) continue;
+        if (!t.nbytes || (c->carry && t.nbytes <= CARRY_OUT_MAX && carried((char*)t.buf->dptr + t.offset, t.staging, t.nbytes))) continue;
         if (t.nbytes < STAGE_MIN) {
             HIP_TRY(hipMemcpyAsync(t.staging, (char*)t.buf->dptr + t.offset, t.nbytes, hipMemcpyDeviceToHost, c->stream));
             continue;

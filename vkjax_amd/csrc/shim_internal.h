@@ -38,6 +38,16 @@ struct Slab {
 };
 constexpr size_t SLAB_BYTES = 1u << 20, PACKED_MAX_BYTES = 64u << 10, PACKED_ALIGN = 256;
 
+// Ranges copied between HBM and pinned host memory by one kernel launch (static_landing.hip): small arguments on their way in, small
+// results on their way out. A transfer command each costs 3 us of the call and of the stream, and more time on the way: from pinned
+// memory to HBM 64 KB take 19.7 us with the launch and the wait behind them, by the kernel 14.9; 784 KB 32.7, 28.4; 8 MB 165.7, 161.8.
+struct Carry {
+    static constexpr int MAX = 16;
+    struct { void* dst; const void* src; uint64_t nbytes; } range[MAX];      // addresses and sizes are multiples of 4
+    int count = 0;
+};
+constexpr size_t CARRY_OUT_MAX = 256u << 10;       // larger results leave with a transfer of their own
+
 struct Ctx {
     uint64_t    handle = 0;
     uint32_t    magic = MAGIC_CTX;
@@ -59,6 +69,7 @@ struct Ctx {
     hipEvent_t  ev_checkpoint[2 * MAX_CHECKPOINTS] = {};
     std::vector<Slab*> slabs;            // those with live arrays; the last one is the one being filled
     void*       static_landing = nullptr;   // this device's copy of the static landing array (static_landing.hip)
+    int       (*carry)(const Carry& what, bool to_host, hipStream_t stream) = nullptr;      // null: there is no kernel for it (the host-only test build)
 };
 
 // A buffer recorded into sequences stays allocated until the last of them is destroyed:

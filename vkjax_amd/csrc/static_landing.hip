@@ -17,6 +17,7 @@
 // refusals, so that the host-only test build exercises them).
 #include "shim_internal.h"
 
+#include <algorithm>
 #include <cstring>
 
 using namespace vkj;
@@ -39,6 +40,41 @@ __global__ __launch_bounds__(256) void move_landed(unsigned char* __restrict__ d
     } else {
         for (; i < nbytes; i += stride) dst[i] = src[i];
     }
+}
+
+// Every range of the table; block (x, y) copies its share of range y. Host memory is read and written at system scope, past the caches: what
+// an earlier launch found there is not what the host has put there since.
+__global__ __launch_bounds__(256) void carry_ranges(Carry what, int to_host) {
+    const auto r = what.range[blockIdx.y];
+    const uint32_t stride = gridDim.x * 256u, first = blockIdx.x * 256u + threadIdx.x;
+    const bool vectors = (((uintptr_t)r.dst | (uintptr_t)r.src) & 15u) == 0;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    // (a range is below 2 GiB: larger evaluations are staged and sent in chunks)
+    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(r.src), 0, (int)r.nbytes, 0x00020000),
+                                 to   = __builtin_amdgcn_make_buffer_rsrc(r.dst, 0, (int)r.nbytes, 0x00020000);
+    constexpr int SYSTEM = 17;                                          // sc0 sc1
+    const uint32_t whole = vectors ? (uint32_t)(r.nbytes / 16u) : 0u;
+    for (uint32_t v = first; v < whole; v += stride) {
+        if (to_host) __builtin_amdgcn_raw_buffer_store_b128(__builtin_amdgcn_raw_buffer_load_b128(from, v * 16u, 0, 0), to, v * 16u, 0, SYSTEM);
+        else         __builtin_amdgcn_raw_buffer_store_b128(__builtin_amdgcn_raw_buffer_load_b128(from, v * 16u, 0, SYSTEM), to, v * 16u, 0, 0);
+    }
+    for (uint32_t w = whole * 4u + first; w < (uint32_t)(r.nbytes / 4u); w += stride) {
+        if (to_host) __builtin_amdgcn_raw_buffer_store_b32(__builtin_amdgcn_raw_buffer_load_b32(from, w * 4u, 0, 0), to, w * 4u, 0, SYSTEM);
+        else         __builtin_amdgcn_raw_buffer_store_b32(__builtin_amdgcn_raw_buffer_load_b32(from, w * 4u, 0, SYSTEM), to, w * 4u, 0, 0);
+    }
+}
+
+int carry_on(const Carry& what, bool to_host, hipStream_t stream) {
+    if (!what.count) return 0;
+    uint64_t most = 0;
+    for (int k = 0; k < what.count; k++) most = std::max<uint64_t>(most, what.range[k].nbytes);
+    // 32 blocks keep the link busy (784 KB in 32, 128 and 512 blocks: 28.4, 29.9, 31.8 us)
+    const uint64_t blocks = std::min<uint64_t>(32u, (most + 4095u) / 4096u);
+    Carry table = what;
+    int out = to_host;
+    void* args[] = {&table, &out};
+    HIP_TRY(hipLaunchKernel((const void*)carry_ranges, dim3((unsigned)blocks, (unsigned)what.count), dim3(256), args, 0, stream));
+    return 0;
 }
 
 int move_on(void* dst, const void* src, size_t nbytes, hipStream_t stream) {
@@ -66,6 +102,7 @@ int vkj::static_landing_init(Ctx* c) {
     HIP_TRY(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
     if (!p) return fail(VKJ_ENODEV, "vkj_ctx_create: the static landing array has no address on device %d", c->device);
     c->static_landing = p;
+    c->carry = carry_on;
     return 0;
 }
 
