@@ -9,17 +9,28 @@ struct ThreefryParams { uint32_t n, key_is_scalar; };
 
 __device__ __forceinline__ uint32_t rotl32(uint32_t v, uint32_t d) { return (v << d) | (v >> (32u - d)); }
 
+// on the scalar unit, for a value that is the same in the whole wave (it has no rotation; left alone the compiler moves all that depends on
+// one to the vector unit)
+__device__ __forceinline__ uint32_t rotl32_scalar(uint32_t v, int d) {
+    uint32_t high, low;
+    asm("s_lshl_b32 %0, %2, %3\n\ts_lshr_b32 %1, %2, %4\n\ts_or_b32 %0, %0, %1" : "=&s"(high), "=&s"(low) : "s"(v), "i"(d), "i"(32 - d) : "scc");
+    return high;
+}
+
+template <bool SCALAR = false>
 __device__ __forceinline__ void threefry_block(uint32_t k0, uint32_t k1, uint32_t& x0, uint32_t& x1) {
     const uint32_t ks[3] = {k0, k1, k0 ^ k1 ^ 0x1BD11BDAu};
-    const uint32_t rot[2][4] = {{13, 15, 26, 6}, {17, 29, 16, 24}};
+    constexpr int rot[2][4] = {{13, 15, 26, 6}, {17, 29, 16, 24}};
     x0 += ks[0];
     x1 += ks[1];
+    // (in a loop the compiler would carry the part of x0 that is the same in every turn beside the rest, and add the two in every round)
+    if constexpr (!SCALAR) asm("" : "+v"(x0), "+v"(x1));
 #pragma unroll
     for (uint32_t i = 0; i < 5; ++i) {
 #pragma unroll
         for (uint32_t r = 0; r < 4; ++r) {
             x0 += x1;
-            x1 = rotl32(x1, rot[i & 1][r]);
+            x1 = SCALAR ? rotl32_scalar(x1, rot[i & 1][r]) : rotl32(x1, (uint32_t)rot[i & 1][r]);
             x1 ^= x0;
         }
         x0 += ks[(i + 1) % 3];
@@ -97,6 +108,9 @@ struct ThreefryStreamParams {
     uint32_t flags[TF_MAX_STEPS];      // bit0: the step has an operand (a single value); bit1: it is the LEFT argument
     uint32_t imm[TF_MAX_STEPS];        // immediate of step k (integer_pow exponent)
     uint32_t n;                        // halves layout: elements of the output (2h, or 2h - 1 for an odd-sized draw)
+    // 0: the key words lie at key0, key1. Else they are words key_word[0], key_word[1] of a key split, i.e. of what a launch without steps would
+    // store in layout key_split - 1 (HALVES or PAIRS) with the key at key0, key1 and these counters: every wave computes the two itself
+    uint32_t key_split, key_h, key_c0, key_c1, key_n, key_word[2];
 };
 
 struct ThreefryStreamPtrs { const uint32_t* p[TF_MAX_STEPS]; };
@@ -156,12 +170,27 @@ __device__ __forceinline__ void threefry_uniform_steps(uint32_t (&y)[NV], const 
     }
 }
 
+// Word i of a key split. Everything is the same for the whole wave, so this is scalar arithmetic beside the other waves' vector instructions.
+__device__ __forceinline__ uint32_t threefry_split_word(uint32_t k0, uint32_t k1, const ThreefryStreamParams& P, uint32_t i) {
+    const bool pairs = P.key_split - 1u == TF_PAIRS, second = pairs ? i & 1u : i >= P.key_h;
+    const uint32_t j = pairs ? i >> 1 : second ? i - P.key_h : i;
+    uint32_t x0 = pairs ? P.key_c0 : P.key_c0 + j, x1 = P.key_c1 + j;
+    if (!pairs && P.key_h + j >= P.key_n) x1 = 0u;                  // the padding counter of an odd-sized draw
+    threefry_block<true>(k0, k1, x0, x1);
+    return second ? x1 : x0;
+}
+
+// A draw whose key was split off another one just before is one launch: the split was one of a single workgroup, 2.4 us and the gap behind it
+// (single replays: 16 M uniform numbers 36.4 -> 34.3 us, 1 M 20.4 -> 17.2, 4096 19.3 -> 16.6). Its threads take several vectors each, so that the two blocks
+// of the split stay beside the work (16 M in 8192, 4096, 2048, 1024 workgroups: 24.7, 21.3, 21.1, 20.8 us among others; 33 M: 36.4, 35.8, 35.1, 35.8).
 template <int VEC, int MODE, bool UNIFORM = false>
 __device__ __forceinline__ void threefry_stream_body(uint32_t* __restrict__ out, const uint32_t* __restrict__ key0,
                                                      const uint32_t* __restrict__ key1, const ThreefryStreamParams& P) {
-    const uint32_t j0 = (blockIdx.x * 256u + threadIdx.x) * VEC;
-    if (j0 >= P.h) return;
-    const uint32_t k0 = key0[0], k1 = key1[0];
+    uint32_t k0 = key0[0], k1 = key1[0];
+    if (P.key_split) {
+        const uint32_t s0 = threefry_split_word(k0, k1, P, P.key_word[0]), s1 = threefry_split_word(k0, k1, P, P.key_word[1]);
+        k0 = s0; k1 = s1;
+    }
     uint32_t o[6] = {};
     if constexpr (UNIFORM) {
         const char* const args = reinterpret_cast<const char*>(__builtin_amdgcn_kernarg_segment_ptr());
@@ -169,49 +198,53 @@ __device__ __forceinline__ void threefry_stream_body(uint32_t* __restrict__ out,
 #pragma unroll
         for (int k = 0; k < 6; ++k) o[k] = op_ptr[k][0];
     }
-    if constexpr (MODE == TF_HALVES) {
-        uint32_t y[2 * VEC];                         // [0, VEC): first results, [VEC, 2 VEC): second results
+#pragma nounroll
+    for (uint64_t at = (blockIdx.x * 256ull + threadIdx.x) * VEC; at < P.h; at += gridDim.x * 256ull * VEC) {
+        const uint32_t j0 = (uint32_t)at;
+        if constexpr (MODE == TF_HALVES) {
+            uint32_t y[2 * VEC];                         // [0, VEC): first results, [VEC, 2 VEC): second results
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-            y[j]       = P.c0 + j0 + j;
-            y[VEC + j] = P.c1 + j0 + j;
-            if (VEC == 1 && P.h + j0 >= P.n) y[VEC] = 0u;           // the padding counter of an odd-sized draw
-            threefry_block(k0, k1, y[j], y[VEC + j]);
-        }
-        if constexpr (UNIFORM) threefry_uniform_steps<2 * VEC>(y, o);
-        else threefry_stream_steps<2 * VEC>(y, P.nsteps);
-        if constexpr (VEC == 4) {
-            u32x4 va, vb;
-            va.x = y[0]; va.y = y[1]; va.z = y[2]; va.w = y[3];
-            vb.x = y[4]; vb.y = y[5]; vb.z = y[6]; vb.w = y[7];
-            *reinterpret_cast<u32x4*>(out + j0) = va;
-            *reinterpret_cast<u32x4*>(out + P.h + j0) = vb;
-        } else {
-            out[j0] = y[0];
-            if (P.h + j0 < P.n) out[P.h + j0] = y[1];
-        }
-    } else {
-        uint32_t y[VEC], z[VEC];
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-            y[j] = P.c0;
-            z[j] = P.c1 + j0 + j;
-            threefry_block(k0, k1, y[j], z[j]);
-        }
-        if constexpr (MODE == TF_PAIRS) {
-            static_assert(VEC == 1, "pairs are written one block per thread");
-            out[2 * j0] = y[0]; out[2 * j0 + 1] = z[0];
-        } else {
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) y[j] ^= z[j];
-            if constexpr (UNIFORM) threefry_uniform_steps<VEC>(y, o);
-            else threefry_stream_steps<VEC>(y, P.nsteps);
+            for (int j = 0; j < VEC; ++j) {
+                y[j]       = P.c0 + j0 + j;
+                y[VEC + j] = P.c1 + j0 + j;
+                if (VEC == 1 && P.h + j0 >= P.n) y[VEC] = 0u;           // the padding counter of an odd-sized draw
+                threefry_block(k0, k1, y[j], y[VEC + j]);
+            }
+            if constexpr (UNIFORM) threefry_uniform_steps<2 * VEC>(y, o);
+            else threefry_stream_steps<2 * VEC>(y, P.nsteps);
             if constexpr (VEC == 4) {
-                u32x4 va;
+                u32x4 va, vb;
                 va.x = y[0]; va.y = y[1]; va.z = y[2]; va.w = y[3];
+                vb.x = y[4]; vb.y = y[5]; vb.z = y[6]; vb.w = y[7];
                 *reinterpret_cast<u32x4*>(out + j0) = va;
+                *reinterpret_cast<u32x4*>(out + P.h + j0) = vb;
             } else {
                 out[j0] = y[0];
+                if (P.h + j0 < P.n) out[P.h + j0] = y[1];
+            }
+        } else {
+            uint32_t y[VEC], z[VEC];
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) {
+                y[j] = P.c0;
+                z[j] = P.c1 + j0 + j;
+                threefry_block(k0, k1, y[j], z[j]);
+            }
+            if constexpr (MODE == TF_PAIRS) {
+                static_assert(VEC == 1, "pairs are written one block per thread");
+                out[2 * j0] = y[0]; out[2 * j0 + 1] = z[0];
+            } else {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) y[j] ^= z[j];
+                if constexpr (UNIFORM) threefry_uniform_steps<VEC>(y, o);
+                else threefry_stream_steps<VEC>(y, P.nsteps);
+                if constexpr (VEC == 4) {
+                    u32x4 va;
+                    va.x = y[0]; va.y = y[1]; va.z = y[2]; va.w = y[3];
+                    *reinterpret_cast<u32x4*>(out + j0) = va;
+                } else {
+                    out[j0] = y[0];
+                }
             }
         }
     }

@@ -316,7 +316,7 @@ def fuse_ops(all_ops, bufferpool, outvars):
             for b in _writes(new):
                 producer.pop(id(b._placeholder), None)
     ops = fuse_random_streams([op for op in result if op is not None], bufferpool, outvars)
-    ops = fuse_stream_chains(ops, bufferpool, outvars)
+    ops = fuse_key_splits(remove_dead_ops(fuse_stream_chains(ops, bufferpool, outvars), bufferpool, outvars), bufferpool, outvars)
     ops = fuse_softmax(ops, bufferpool, outvars)
     ops = fuse_row_programs(remove_dead_ops(ops, bufferpool, outvars), bufferpool, outvars)
     ops = fuse_scale_relu_backward(ops, bufferpool, outvars)
@@ -995,8 +995,8 @@ def fuse_stream_chains(ops, bufferpool, outvars):
     for si, S in enumerate(ops):
         if S.meta is None or S.meta[0] != 'random_stream':
             continue
-        _, out, layout, key0, key1, h, c0, c1, n = S.meta
-        if layout == 'pairs' or uses[pid(out)] != 1:
+        _, out, layout, key0, key1, h, c0, c1, n, steps = S.meta[:10]
+        if layout == 'pairs' or uses[pid(out)] != 1 or steps:
             continue
         for i in range(si + 1, len(ops)):
             op = ops[i]
@@ -1011,7 +1011,7 @@ def fuse_stream_chains(ops, bufferpool, outvars):
                     and all(st.op not in _SELECTS and st.op != EW['NOP'] and
                             (st.operand is None or (st.operand.buffer.size == 1 and st.operand.offset == 0)) for st in ch.steps)):
                 fused = Op(_label(S, op), launch=K.threefry_stream(ch.out, key0, key1, h, c0, c1, list(ch.steps), layout=layout, n=n),
-                           meta=('random_stream', ch.out, layout, key0, key1, h, c0, c1, n))
+                           meta=('random_stream', ch.out, layout, key0, key1, h, c0, c1, n, list(ch.steps)))
                 fused.index = op.index
                 for b in [key0[0], key1[0]] + [st.operand.buffer for st in ch.steps if st.operand is not None]:
                     b.accesses.append(fused.index)
@@ -1020,6 +1020,62 @@ def fuse_stream_chains(ops, bufferpool, outvars):
                 replacement[i] = fused
             break
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
+
+
+def fuse_key_splits(ops, bufferpool, outvars):
+    '''A key split (a launch of random words without steps) whose words nothing but the keys of other draws read: those draws
+    compute their two words of it themselves. Same bits; the split's launch goes.'''
+    from .ops import Op
+    uses = _use_counts(ops, bufferpool, outvars)
+    pid  = lambda b: id(b._placeholder)
+    writers = collections.defaultdict(list)
+    for i, op in enumerate(ops):
+        for b in _may_write(op):
+            writers[pid(b)].append(i)
+    result, gone = list(ops), set()
+    #(from the end: a split that a draw has taken over may itself read the words of another)
+    for si in reversed(range(len(ops))):
+        S = result[si]
+        if S.meta is None or S.meta[0] != 'random_stream' or si in gone:
+            continue
+        if len(S.meta) > 10:
+            continue
+        _, out, layout, key0, key1, h, c0, c1, n, steps = S.meta
+        if steps or layout == 'xor':
+            continue
+        reading = lambda b: [i for i in range(len(ops)) if i != si and i not in gone and any(r._placeholder is b._placeholder for r in _reads(result[i]))]
+        #where the words are read: from the split's result itself, or from a copy of one key of it
+        places, copies = [(out, 0, 1)], []
+        for i in reading(out):
+            ch = result[i].chain
+            if ch is not None and not ch.steps and ch.out.size == 2 and max(ch.shape) == 2 and len(writers[pid(ch.out)]) == 1:
+                places.append((ch.out, ch.first.offset, ch.first.strides[list(ch.shape).index(2)]))
+                copies.append(i)
+        takes = lambda op, b: (op.meta is not None and op.meta[0] == 'random_stream' and len(op.meta) == 10
+                               and all(k[0]._placeholder is b._placeholder for k in op.meta[3:5])
+                               and sum(r._placeholder is b._placeholder for r in _reads(op)) == 2)
+        draws = [(i, first, step) for b, first, step in places for i in reading(b) if i not in copies]
+        if (not draws or min(i for i, _, _ in draws) < si or len(writers[pid(out)]) != 1
+                or not all(takes(result[i], b) for b, _, _ in places for i in reading(b) if i not in copies)
+                or any(uses[pid(b)] != 2 * len([i for i in reading(b) if i not in copies]) + (len(copies) if b is out else 0) for b, _, _ in places)
+                or any(writers[pid(k[0])] and max(writers[pid(k[0])]) > si for k in (key0, key1))):
+            continue
+        for i, first, step in draws:
+            op = result[i]
+            _, out2, layout2, (_, w0), (_, w1), h2, d0, d1, n2, steps2 = op.meta
+            split = K.KeySplit(layout, h, c0, c1, 2 * h if layout == 'pairs' else n, (first + w0 * step, first + w1 * step))
+            fused = Op(_label(S, op), launch=K.threefry_stream(out2, key0, key1, h2, d0, d1, steps2, layout=layout2, n=n2, key_split=split),
+                       meta=('random_stream', out2, layout2, key0, key1, h2, d0, d1, n2, steps2, split))
+            fused.index = op.index
+            for b in (key0[0], key1[0]):
+                b.accesses.append(fused.index)
+            result[i] = fused
+        for i in copies:
+            result[i].chain.out._placeholder.elided = True
+            gone.add(i)
+        out._placeholder.elided = True
+        gone.add(si)
+    return [op for i, op in enumerate(result) if i not in gone]
 
 
 def fuse_derived_epilogue_operands(ops, bufferpool, outvars):
@@ -1246,7 +1302,8 @@ def fuse_random_streams(ops, bufferpool, outvars):
             else:
                 keys.append((kb, 0))
         fused = Op(_label(*[ops[i] for i in sorted(members)]),
-                   launch=K.threefry_stream(out, keys[0], keys[1], h, sources[0][1], sources[1][1], steps))
+                   launch=K.threefry_stream(out, keys[0], keys[1], h, sources[0][1], sources[1][1], steps),
+                   meta=('random_stream', out, 'halves', keys[0], keys[1], h, sources[0][1], sources[1][1], 2 * h, steps))
         fused.index = ops[last].index
         for b in [keys[0][0], keys[1][0]] + [st.operand.buffer for st in steps if st.operand is not None]:
             b.accesses.append(fused.index)
@@ -1284,7 +1341,7 @@ def _small_out(op):
 
 def _may_write(op) -> tp.List:
     '''Buffers an op may change: its result where the op's structure is known, else everything it touches.'''
-    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'reduce', 'softmax', 'rows', 'conv_pack')):
+    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'random_stream', 'reduce', 'softmax', 'rows', 'conv_pack')):
         return _writes(op)
     return [b for b, _ in op.launch.buffers if b is not None]
 

@@ -441,15 +441,31 @@ TF_MAX_STEPS = 8
 _UNIFORM_CHAIN_OPS = [EW[name] for name in ('SHR_L', 'OR_X', 'SUB_F', 'MUL_F', 'ADD_F', 'MAX_F')]
 
 
+class KeySplit(tp.NamedTuple):
+    '''Two words of what a stream without steps would store: its layout (halves or pairs), blocks, counters and size.'''
+    layout: str
+    h:      int
+    c0:     int
+    c1:     int
+    n:      int
+    words:  tp.Tuple[int, int]
+
+
+#blocks of a launch that splits its key itself: eight per CU, every thread on several vectors
+KEY_SPLIT_BLOCKS = 2048
+
+
 def threefry_stream(out: Buffer, key0: tp.Tuple[Buffer, int], key1: tp.Tuple[Buffer, int], h: int, c0: int, c1: int,
-                    steps: tp.Sequence[EwStep], layout: str = 'halves', n: tp.Optional[int] = None) -> Launch:
+                    steps: tp.Sequence[EwStep], layout: str = 'halves', n: tp.Optional[int] = None,
+                    key_split: tp.Optional[KeySplit] = None) -> Launch:
     '''Random words from counters generated in registers, the element-wise `steps` (operands: single
     values) applied before the only store. `h` blocks are run; the key words are given as
     (buffer, element offset). Layouts:
       halves  out[j], out[h + j] = steps(threefry2x32(key, c0 + j, c1 + j)); `n` (2h or 2h - 1) is the
               number of elements stored, and with n == 2h - 1 the last x1 counter is 0
       xor     out[j] = steps(y0 ^ y1) with y = threefry2x32(key, c0, c1 + j)
-      pairs   out[2j], out[2j + 1] = threefry2x32(key, c0, c1 + j)  (no steps)'''
+      pairs   out[2j], out[2j + 1] = threefry2x32(key, c0, c1 + j)  (no steps)
+    `key_split`: key0 and key1 are the key that was split, and the key words two words of that split.'''
     if len(steps) > TF_MAX_STEPS:
         raise ValueError('too many steps')
     if layout == 'pairs' and steps:
@@ -464,12 +480,16 @@ def threefry_stream(out: Buffer, key0: tp.Tuple[Buffer, int], key1: tp.Tuple[Buf
         buffers.append((s.operand.buffer if s.operand is not None else None, 0))
     vec = 4 if h % 4 == 0 and (n == 2 * h if layout == 'halves' else layout == 'xor') else 1
     params = _u32(h, c0, c1, len(steps), *_pad([s.op for s in steps], TF_MAX_STEPS), *_pad(flags, TF_MAX_STEPS),
-                  *_pad([s.imm for s in steps], TF_MAX_STEPS), n)
+                  *_pad([s.imm for s in steps], TF_MAX_STEPS), n,
+                  *(({'halves': 1, 'pairs': 3}[key_split.layout], *key_split[1:5], *key_split.words) if key_split else (0,) * 7))
     kernel = {'halves': 'threefry2x32_stream', 'xor': 'threefry2x32_stream_xor', 'pairs': 'threefry2x32_stream_pairs'}[layout]
     #jax.random.uniform's chain has a kernel of its own with the steps compiled in
     if vec == 4 and [s.op for s in steps] == _UNIFORM_CHAIN_OPS and flags == [1, 1, 1, 1, 1, 3] and all(s.imm == 0 for s in steps):
         kernel += '_uniform'
-    return Launch(f'{kernel}_v{vec}', (_cdiv(_cdiv(h, vec), BLOCK), 1, 1), (BLOCK, 1, 1),
+    blocks = _cdiv(_cdiv(h, vec), BLOCK)
+    if key_split and layout != 'pairs':
+        blocks = min(blocks, KEY_SPLIT_BLOCKS)
+    return Launch(f'{kernel}_v{vec}', (blocks, 1, 1), (BLOCK, 1, 1),
                   [(out, 0), (key0[0], key0[1] * 4), (key1[0], key1[1] * 4)] + _pad(buffers, TF_MAX_STEPS, (None, 0)), params,
                   bytes_moved=4 * (h if layout == 'xor' else n))
 

@@ -1075,7 +1075,7 @@ def _single_key(bufferpool, equation) -> Buffer:
 def _stream_op(equation, outbuf, layout, key, h, c0, c1, n):
     k0, k1 = (key, 0), (key, 1)
     return Op(equation, launch=K.threefry_stream(outbuf, k0, k1, h, c0, c1, [], layout=layout, n=n),
-              meta=('random_stream', outbuf, layout, k0, k1, h, c0, c1, n))
+              meta=('random_stream', outbuf, layout, k0, k1, h, c0, c1, n, []))
 
 
 def random_bits(bufferpool, equation):
