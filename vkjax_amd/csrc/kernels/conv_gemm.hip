@@ -164,6 +164,45 @@ __device__ __forceinline__ void conv_epilogue_step(uint32_t code, float (&y)[16]
 #undef EPI_LOOP
 }
 
+// The usual chain behind a product, (- vector, * vector, + vector, + full tensor, max with a scalar), each step optional, on the NV values a lane
+// holds of one column; `tap_store` stores them as they stand before or after the first step (tap 0 or 1).
+template <int NV, class TapStore>
+__device__ __forceinline__ void conv_straight_steps(float (&y)[NV], const float (&full)[NV], uint32_t slots, int tap, const float* Es, int BN, int col, TapStore&& tap_store) {
+    const int e_mul = __builtin_popcount(slots & 1u), e_add = __builtin_popcount(slots & 3u), e_max = __builtin_popcount(slots & 15u);
+    if (tap == 0) tap_store();
+    if (slots & 1u) {
+        const float o = Es[col];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) y[v] = y[v] - o;
+        if (tap == 1) tap_store();
+    }
+    if (slots & 2u) {
+        const float o = Es[e_mul * BN + col];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) y[v] = y[v] * o;
+    }
+    if (slots & 4u) {
+        const float o = Es[e_add * BN + col];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) y[v] = y[v] + o;
+    }
+    if (slots & 8u) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) y[v] = y[v] + full[v];
+    }
+    if (slots & 16u) {
+        const float o = Es[e_max * BN + col];          // the same value in every lane
+        if (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, o != o ? 1.f : 0.f)) == 0) {
+            // max(y, o) that returns a NaN y, for o known not to be NaN: one compare
+#pragma unroll
+            for (int v = 0; v < NV; ++v) y[v] = !(y[v] <= o) ? y[v] : o;
+        } else {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) y[v] = (y[v] > o || y[v] != y[v]) ? y[v] : o;
+        }
+    }
+}
+
 // LEAN: the variant for the common case, with the rarely needed paths compiled out (they cost
 // registers, and with them resident waves, even when not taken): both operands on the 16-byte
 // path, k tiles that never straddle kernel taps, a row-major result, an epilogue that fits the
@@ -543,10 +582,22 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
         }
     };
 
+    // the same for a wave's quarter of the one tile of a block whose four waves share it (the result is a row-major matrix there)
+    auto quarter_tile = [&](auto&& fn) {
+        const int n = n0 + l32, first = 8 * __builtin_amdgcn_readfirstlane(kw);
+        const uint32_t base = n < P.N ? (uint32_t)((region.m_base + tile_m0 * BM + 4 * half) * P.N + n) * 4u : CONV_OOB, rowb = (uint32_t)P.N * 4u;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) fn(v, base, (uint32_t)(first + v) * rowb);
+    };
+
     float full[PREFETCH_FULL ? TM : 1][PREFETCH_FULL ? TN : 1][16];
+    float quarter[4] = {0.f, 0.f, 0.f, 0.f};                     // ... and of its residual, requested before the product is computed
     setup_rows(region.m_base + tile_m0 * BM);
     load_tiles(kbase * BK);
     if constexpr (EPI_BEHIND_TILES) request_epilogue_operands();
+    if constexpr (KSW > 1) {
+        if (P.flags & (8u << 20)) quarter_tile([&](int v, uint32_t vo, uint32_t so) { quarter[v] = buffer_load_x1_nt(f_rsrc, vo, so); });
+    }
     if (tid < BN) {
         if (Dk.nsteps) {
             const float v = conv_derived_value(d_in, Dk);
@@ -658,6 +709,25 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
             }
             __syncthreads();
         }
+        if constexpr (KSW > 1) {
+            // The k slices meet in LDS (the A and B tiles are done with), and every wave finishes a quarter of the tile: rows 8 kw + 4 half ..
+            // + 3 of its column. (The first wave finishing all of it, with the residual requested
+            // only then: the launches of ResNet-50 on one image 516 us, so 502.)
+            static_assert(KSW == 4 && WGM * WGN * TM * TN == 1 && KSW * 16 * 64 <= BM * LDA + BK * LDB, "sixteen values per lane of each of four waves, in the A and B tiles (B follows A)");
+            f32x4* const red = reinterpret_cast<f32x4*>(As);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) red[(kw * 4 + q) * 64 + lane] = f32x4{acc[0][0][4 * q], acc[0][0][4 * q + 1], acc[0][0][4 * q + 2], acc[0][0][4 * q + 3]};
+            __syncthreads();
+            f32x4 sum = red[kw * 64 + lane];
+#pragma unroll
+            for (int s = 1; s < KSW; ++s) sum += red[(s * 4 + kw) * 64 + lane];
+            float y[4] = {sum[0], sum[1], sum[2], sum[3]};
+            conv_straight_steps<4>(y, quarter, (P.flags >> 20) & 31u, (int)((P.flags >> 12) & 15u) - 1, Es, BN, l32, [&]() {
+                quarter_tile([&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], make_rsrc(epi.p[CONV_MAX_EPI - 1], P.out_bytes), vo, so); });
+            });
+            quarter_tile([&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], o_rsrc, vo, so); });
+            return;                                               // one M tile per block, a row-major result
+        }
         // From here on the accumulators are handled as separate scalars: element-wise updates of a
         // 16-register MFMA tuple make the compiler copy the whole tuple at every step.
         float c[TM][TN][16];
@@ -667,27 +737,10 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
             for (int j = 0; j < TN; ++j)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) c[i][j][v] = acc[i][j][v];
-        if constexpr (KSW > 1) {
-            // the k slices meet in the first group of waves (the LDS space of the A and B tiles is free after the last step)
-            static_assert((KSW - 1) * WGM * WGN * 16 * 64 <= BM * LDA + BK * LDB, "reduction buffer does not fit the A and B tiles (B follows A)");
-            float* red = As + ((kw - 1) * WGM * WGN + wm * WGN + wn) * 16 * 64 + lane;
-            if (kw > 0) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v) red[v * 64] = c[0][0][v];
-            }
-            __syncthreads();
-            if (kw > 0) continue;                                 // nsub == 1 for these kernels: the wave is done
-#pragma unroll
-            for (int s = 1; s < KSW; ++s)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) c[0][0][v] += As[((s - 1) * WGM * WGN + wm * WGN + wn) * 16 * 64 + v * 64 + lane];
-        }
         const uint32_t slots = (P.flags >> 20) & 31u;
         if (LEAN || slots) {
             // The usual chains (bias, batch norm, residual add, ReLU in that order, each optional) run
             // as straight-line code: every step is one pass over a sub-tile's 16 values, in place.
-            const int e_mul = __builtin_popcount(slots & 1u), e_add = __builtin_popcount(slots & 3u),
-                      e_max = __builtin_popcount(slots & 15u);
             const int tap = (int)((P.flags >> 12) & 15u) - 1;          // -1: no second result
 #pragma unroll
             for (int i = 0; i < TM; ++i)
@@ -700,47 +753,14 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
                     float ov[16];
                     if ((slots & 8u) && !(PREFETCH_FULL && first_full >= 0))
                         sub_tile(m0, i, j, [&](int v, uint32_t vo, uint32_t so) { ov[v] = buffer_load_x1_nt(f_rsrc, vo, so); });   // read once: kept out of the caches (-0.8 % on ResNet-50's step)
-                    // a second result: the value as it stands before or after the first step
-#define CONV_TAP_STORE() sub_tile(m0, i, j, [&](int v, uint32_t vo, uint32_t so) {                                   \
-                            buffer_store_x1(y[v], make_rsrc(epi.p[CONV_MAX_EPI - 1], P.out_bytes), vo, so); })
-                    if (tap == 0) CONV_TAP_STORE();
-                    if (slots & 1u) {
-                        const float o = Es[col];
+                    const bool prefetched = PREFETCH_FULL && first_full >= 0;
+                    if (prefetched) {
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) y[v] = y[v] - o;
-                        if (tap == 1) CONV_TAP_STORE();
+                        for (int v = 0; v < 16; ++v) ov[v] = full[PREFETCH_FULL ? i : 0][PREFETCH_FULL ? j : 0][v];
                     }
-#undef CONV_TAP_STORE
-                    if (slots & 2u) {
-                        const float o = Es[e_mul * BN + col];
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) y[v] = y[v] * o;
-                    }
-                    if (slots & 4u) {
-                        const float o = Es[e_add * BN + col];
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) y[v] = y[v] + o;
-                    }
-                    if (slots & 8u) {
-                        if (PREFETCH_FULL && first_full >= 0) {
-#pragma unroll
-                            for (int v = 0; v < 16; ++v) y[v] = y[v] + full[PREFETCH_FULL ? i : 0][PREFETCH_FULL ? j : 0][v];
-                        } else {
-#pragma unroll
-                            for (int v = 0; v < 16; ++v) y[v] = y[v] + ov[v];
-                        }
-                    }
-                    if (slots & 16u) {
-                        const float o = Es[e_max * BN + col];          // the same value in every lane
-                        if (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, o != o ? 1.f : 0.f)) == 0) {
-                            // max(y, o) that returns a NaN y, for o known not to be NaN: one compare
-#pragma unroll
-                            for (int v = 0; v < 16; ++v) y[v] = !(y[v] <= o) ? y[v] : o;
-                        } else {
-#pragma unroll
-                            for (int v = 0; v < 16; ++v) y[v] = (y[v] > o || y[v] != y[v]) ? y[v] : o;
-                        }
-                    }
+                    conv_straight_steps<16>(y, ov, slots, tap, Es, BN, col, [&]() {
+                        sub_tile(m0, i, j, [&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], make_rsrc(epi.p[CONV_MAX_EPI - 1], P.out_bytes), vo, so); });
+                    });
                 }
         } else if constexpr (!LEAN) {
             // any other chain: one uniform branch per step and sub-tile, not per element
