@@ -53,7 +53,7 @@ def _reads(op) -> tp.List:
             return [op.meta[2]]
         if op.meta[0] == 'threefry':
             return list(op.meta[2])
-        if op.meta[0] in ('random_stream', 'reduce'):
+        if op.meta[0] in ('random_stream', 'reduce', 'update'):
             return [b for b, _ in op.launch.buffers[1:] if b is not None]
         if op.meta[0] == 'softmax':
             return [op.meta[2]]
@@ -322,6 +322,7 @@ def fuse_ops(all_ops, bufferpool, outvars):
     ops = fuse_scale_relu_backward(ops, bufferpool, outvars)
     ops = fuse_reduce_prologues(ops, bufferpool, outvars)
     ops = fuse_reduce_scales(ops, bufferpool, outvars)
+    ops = fuse_reduce_updates(ops, bufferpool, outvars)
     ops = fuse_derived_epilogue_operands(ops, bufferpool, outvars)
     ops = fuse_relu_backward_epilogues(ops, bufferpool, outvars)
     ops = fuse_index_wrap(ops, bufferpool, outvars)
@@ -785,6 +786,51 @@ def fuse_reduce_scales(ops, bufferpool, outvars):
         for b in (inp, o.buffer):
             b.accesses.append(ops[C].index)
         out._placeholder.elided = True
+        removed.add(i)
+        replacement[C] = fused
+    return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
+
+
+def fuse_reduce_updates(ops, bufferpool, outvars):
+    '''A float column sum (of the slices of a kernel gradient, of the rows of a bias gradient) whose result is read once, by
+    `p - rate * sum` with a single value `rate` - a step of gradient descent - stores that difference itself. Same
+    operands and roundings as the element-wise launch behind it, which goes away. There is no lower or upper line: it is one
+    launch, one write and one read of the gradient less at every size (a training step of a 784-300-100-10 network over 1000
+    rows 145 -> 128 us together with its weight gradients in the layout of the weights, ResNet-50's 12.82 -> 12.74 ms).'''
+    from .ops import Op
+    uses = _use_counts(ops, bufferpool, outvars)
+    pid  = lambda b: id(b._placeholder)
+    sums = {pid(op.launch.buffers[0][0]): i for i, op in enumerate(ops)
+            if op.chain is None and op.conv is None and op.launch.kernel in K.REDUCE_BATCH_KERNELS}
+    removed, replacement = set(), {}
+    for C, op in enumerate(ops):
+        ch = op.chain
+        if ch is None or [st.op for st in ch.steps] != [EW['MUL_F'], EW['SUB_F']] or not ch.steps[1].operand_left:
+            continue
+        total, rate, before = ch.first, ch.steps[0].operand, ch.steps[1].operand
+        if pid(total.buffer) not in sums:
+            total, rate = rate, total                           #rate * sum: the product is the same number
+        i = sums.get(pid(total.buffer))
+        if i is None or i in removed or i > C:
+            continue
+        #(a launch without a record of its structure counts among the readers of its own result)
+        if uses[pid(total.buffer)] - sum(b._placeholder is total.buffer._placeholder for b in _reads(ops[i])) != 1:
+            continue
+        n = total.buffer.size
+        if (rate.buffer.size != 1 or rate.offset != 0 or ch.out.size != n or before.buffer.size != n or before.buffer.dtype != 'float32'
+                or ch.out.dtype != 'float32' or not all(_is_full_contiguous_any_shape(o, ch.shape) for o in (total, before))):
+            continue
+        source = ops[i].launch.buffers[1][0]
+        #the sum is taken where the update stood: its operand must still hold the same values there
+        if any(w._placeholder is source._placeholder for j in range(i + 1, C) for w in _may_write(ops[j])):
+            continue
+        launch = K.column_sum_update(ops[i].launch, ch.out, before.buffer, rate.buffer)
+        if launch is None:
+            continue
+        fused = Op(_label(ops[i], op), launch=launch, meta=('update',))
+        fused.index = op.index
+        source.accesses.append(op.index)
+        total.buffer._placeholder.elided = True
         removed.add(i)
         replacement[C] = fused
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
@@ -1322,7 +1368,7 @@ def fuse_random_streams(ops, bufferpool, outvars):
 
 def _is_small(op) -> bool:
     '''An element-wise chain or a plain float column sum of a few workgroups, of a kind that has a batch kernel.'''
-    if op.chain is None and not (op.conv is None and op.launch.kernel in K.REDUCE_BATCH_KERNELS):
+    if op.chain is None and not (op.conv is None and op.launch.kernel in K.REDUCE_BATCH_KERNELS + K.UPDATE_BATCH_KERNELS):
         return False
     if op.launch.kernel in K.TRANSPOSE_BATCH_KERNELS:
         #a tiled copy that swaps two dimensions (a network's kernels, transposed for its backward pass): batched up to a
@@ -1341,7 +1387,7 @@ def _small_out(op):
 
 def _may_write(op) -> tp.List:
     '''Buffers an op may change: its result where the op's structure is known, else everything it touches.'''
-    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'random_stream', 'reduce', 'softmax', 'rows', 'conv_pack')):
+    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'random_stream', 'reduce', 'update', 'softmax', 'rows', 'conv_pack')):
         return _writes(op)
     return [b for b, _ in op.launch.buffers if b is not None]
 
@@ -1391,7 +1437,9 @@ def batch_packs(ops):
     return result
 
 
-BATCH_MIN_GAIN = 4          #launches a program must save before its small chains are moved and batched
+#launches a program must save before its small chains are moved and batched (3: the four updates of a network of two
+#convolutions; their chains and sums apart used to save 6)
+BATCH_MIN_GAIN = 3
 
 
 def batch_small_chains(ops):

@@ -52,7 +52,7 @@ class JaxprInterpreter:
         #different contexts, each driven by a thread of its own, run side by side on the GPU)
         self.mgr            = PlanOnlyDevice() if plan_only else (device if device is not None else hip.Device.get())
         self.workgroup_size = get_maximum_workgroup_size(self.mgr)
-        self.bufferpool     = BufferPool(self.mgr, self.workgroup_size, reuse_buffers)
+        self.bufferpool     = BufferPool(self.mgr, self.workgroup_size, reuse_buffers, fuse)
         self.sequence       = None
         #counts evaluations: a suspended stream sees from it whether something else has used the argument buffers
         self._evaluations   = 0

@@ -336,9 +336,10 @@ def _as_affine_chain(chain: EwChain, n: int, dims, strides) -> tp.Optional[Launc
 
 EW_BATCH_KERNELS     = ('ew_chain_v1_s2', 'ew_chain_v1_s4', 'ew_chain_v4_s2', 'ew_chain_v4_s4')
 REDUCE_BATCH_KERNELS = ('reduce_cols_fsum_v1', 'reduce_cols_fsum_v4')
+UPDATE_BATCH_KERNELS = ('reduce_cols_fsum_update_v1', 'reduce_cols_fsum_update_v4')
 TRANSPOSE_BATCH_KERNELS = ('transpose_tiled_v4', 'transpose_tiled_v4_t128')
 BATCH_KERNELS        = {**{k: k.replace('ew_chain_', 'ew_chain_batch_') for k in EW_BATCH_KERNELS},
-                        **{k: k.replace('fsum_', 'fsum_batch_') for k in REDUCE_BATCH_KERNELS},
+                        **{k: k.replace('fsum_', 'fsum_batch_') for k in REDUCE_BATCH_KERNELS + UPDATE_BATCH_KERNELS},
                         **{k: k.replace('tiled_', 'tiled_batch_') for k in TRANSPOSE_BATCH_KERNELS},
                         'conv_split_pack': 'conv_split_pack_layers'}
 EW_BATCH_ENTRY_BYTES        = 432
@@ -371,7 +372,7 @@ def batch_table(launch: Launch, device_address: tp.Callable[[Buffer], int]) -> n
     is_chain, is_transpose = kind in EW_BATCH_KERNELS, kind in TRANSPOSE_BATCH_KERNELS
     entry_bytes, pointers = ((EW_BATCH_ENTRY_BYTES, 1 + EW_MAX_STEPS) if is_chain else
                              (TRANSPOSE_BATCH_ENTRY_BYTES, 2) if is_transpose else
-                             (PACK_BATCH_ENTRY_BYTES, 2) if kind == 'conv_split_pack' else (REDUCE_BATCH_ENTRY_BYTES, 2))
+                             (PACK_BATCH_ENTRY_BYTES, 2) if kind == 'conv_split_pack' else (REDUCE_BATCH_ENTRY_BYTES, 4 if kind in UPDATE_BATCH_KERNELS else 2))
     rows, first = [], 0
     for m in launch.members:
         assert len(m.buffers) == pointers, (m.kernel, len(m.buffers))
@@ -1383,6 +1384,19 @@ def reduce(out: Buffer, inp: Buffer, outer: int, R: int, inner: int, op: str,
     assert partial.size >= outer * nsplit * inner and partial.dtype == inp.dtype
     second = _reduce_launch(out, partial, outer, nsplit, inner, op, 1)[0]
     return [first, second]
+
+
+def column_sum_update(column_sum: Launch, out: Buffer, minuend: Buffer, rate: Buffer) -> tp.Optional[Launch]:
+    '''out = minuend - rate * (what `column_sum` writes), in the order of its additions; None where `column_sum` is not an
+    unsplit float column sum of one [R, inner] array.'''
+    if column_sum.kernel not in REDUCE_BATCH_KERNELS:
+        return None
+    outer, R, inner, _, _, _, nsplit, TI = (int(v) for v in np.frombuffer(column_sum.params, dtype=np.uint32))
+    if (outer, nsplit) != (1, 1):
+        return None
+    assert out.size == minuend.size == inner and rate.size == 1
+    return Launch(column_sum.kernel.replace('fsum_', 'fsum_update_'), column_sum.grid, column_sum.block,
+                  [(out, 0), column_sum.buffers[1], (minuend, 0), (rate, 0)], _u32(R, inner, TI), bytes_moved=column_sum.bytes_moved + 4 * inner)
 
 
 def scale_relu_backward(column_sum: Launch, dx: Buffer, sum_m: Buffer, sum_mx: Buffer, x: Buffer, scale: Buffer, cotangent: Buffer,

@@ -14,6 +14,7 @@ can later be merged into one launch; broadcasts, slices, transposes and reversal
 through strides inside that kernel and never materialised on their own unless they are the
 whole op.
 '''
+import collections
 import typing as tp
 
 import numpy as np
@@ -71,7 +72,7 @@ class Op:
 def analyze_jaxpr(bufferpool: BufferPool, jaxpr) -> tp.List[Op]:
     '''Analyzes (possibly inner) jaxprs'''
     all_ops = []
-    for eq in jaxpr.eqns:
+    for eq in _without_transposed_gradients(jaxpr) if bufferpool.fuse else jaxpr.eqns:
         if all(core.is_dropped(v) for v in eq.outvars):
             continue
         if all(core.is_dropped(v) or 0 in core.physical(v.aval)[0] for v in eq.outvars):
@@ -93,6 +94,30 @@ def analyze_jaxpr(bufferpool: BufferPool, jaxpr) -> tp.List[Op]:
                 op.index = position
         all_ops += method_ops
     return all_ops
+
+
+def _without_transposed_gradients(jaxpr) -> tp.List:
+    '''The equations, with a dense layer's weight gradient as autodiff spells it - the transposition of the product of cotangent
+    and activations, contracted over their rows - replaced by the product of activations and cotangent: the same sums, laid
+    out like the weights. The copy goes away, and with it what kept the gradient's sum from storing the updated weights itself
+    (see fusion.fuse_reduce_updates, where the measurements of both stand). A product that anything else reads keeps its layout.'''
+    from .buffers import hashable
+    uses = collections.Counter(hashable(v) for eq in jaxpr.eqns for v in eq.invars)
+    uses.update(hashable(v) for v in jaxpr.outvars)
+    products, eqns = {}, list(jaxpr.eqns)
+    for i, eq in enumerate(eqns):
+        if eq.primitive.name == 'dot_general' and len(eq.outvars) == 1 and len(eq.outvars[0].aval.shape) == 2:
+            (lc, rc), (lb, rb) = eq.params['dimension_numbers']
+            if (tuple(lc), tuple(rc), tuple(lb), tuple(rb)) == ((0,), (0,), (), ()) and uses[hashable(eq.outvars[0])] == 1:
+                products[hashable(eq.outvars[0])] = i
+        elif (eq.primitive.name == 'transpose' and tuple(eq.params['permutation']) == (1, 0)
+              and hashable(eq.invars[0]) in products and not core.is_dropped(eq.outvars[0])):
+            at      = products.pop(hashable(eq.invars[0]))
+            product = eqns[at]
+            #(this package's equations are named tuples, jax's have a method of their own)
+            changed = getattr(product, '_replace', None) or product.replace
+            eqns[at], eqns[i] = changed(invars=list(reversed(product.invars)), outvars=list(eq.outvars)), None
+    return [eq for eq in eqns if eq is not None]
 
 
 def _reuse_equal_equation(bufferpool: BufferPool, eq) -> bool:
