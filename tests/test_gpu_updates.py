@@ -35,8 +35,8 @@ def test_updates_are_planned():
     for shape in SHAPES:
         kernels = kernels_of(sums_step, sums_args([shape]), plan_only=True)
         assert kernels[-1].startswith('reduce_cols_fsum_update_v') and not any(k.startswith('ew_chain') for k in kernels), (shape, kernels)
-    kernels = kernels_of(sums_step, sums_args([(7, 64), (20, 100), (9, 8), (30, 12), (63, 1000)]), plan_only=True)
-    assert kernels == ['reduce_cols_fsum_batch_update_v4'], kernels
+    kernels = kernels_of(sums_step, sums_args([(7, 64), (20, 100), (9, 7), (30, 10), (63, 1000)]), plan_only=True)
+    assert kernels == ['reduce_cols_fsum_batch_update'], kernels
     #a gradient that is returned or read again, other signs, a rate per column and a sum over the leading of three dimensions' rows
     kept = [lambda p, a: (lambda g: (p - RATE * g, g))(jnp.sum(a, axis=0)), lambda p, a: (lambda g: (p - RATE * g) * g)(jnp.sum(a, axis=0)),
             lambda p, a: RATE * jnp.sum(a, axis=0) - p, lambda p, a: p + RATE * jnp.sum(a, axis=0), lambda p, a: p - p * jnp.sum(a, axis=0)]
@@ -102,3 +102,78 @@ def test_weight_gradients(rows, n_in, n_out):
         assert got.shape == (n_in, n_out) and np.all(np.abs(got - exact) <= bound), fuse
         new = vkjax_amd.wrap(weight_step, frontend='minijax', fuse=fuse)(w, x, cot)
         assert np.all(np.abs(new - (w - float(RATE) * exact)) <= float(RATE) * bound + 3 * 2.0**-24 * (np.abs(w) + float(RATE) * np.abs(exact))), fuse
+
+
+def relu_backward(pre, g):
+    '''The gradient through a ReLU and of the bias in front of it, with the gradient read again.'''
+    m = jnp.where(pre > np.float32(0.25), g, np.float32(0))
+    return m, jnp.sum(m, axis=0)
+
+
+#unsplit sums end at 127 rows; blocks of 256 columns, of 8 vectors or values, and what lies beside them
+RELU_SHAPES = [(2, 2), (3, 4), (17, 10), (63, 64), (64, 65), (127, 100), (127, 256), (128, 256), (129, 257), (1000, 300), (1000, 7), (4099, 8), (700, 1028)]
+
+
+def test_relu_backward_with_its_sum_is_planned():
+    for shape in RELU_SHAPES:
+        x = np.ones(shape, np.float32)
+        kernels = kernels_of(relu_backward, (x, x), plan_only=True)
+        assert kernels[0].startswith('relu_backward_v') and len(kernels) == (2 if shape[0] >= 128 else 1), (shape, kernels)
+    #values of the mask per column, or sums along the other dimension: the launches stay apart
+    other = [lambda x, g: (lambda m: (m, jnp.sum(m, axis=0)))(jnp.where(x > x[0], g, np.float32(0))),
+             lambda x, g: (lambda m: (m, jnp.sum(m, axis=1)))(jnp.where(x > np.float32(0), g, np.float32(0)))]
+    for f in other:
+        assert not any(k.startswith('relu_backward') for k in kernels_of(f, (np.ones((9, 12), np.float32),) * 2, plan_only=True))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('shape', RELU_SHAPES, ids=str)
+def test_relu_backward_keeps_every_bit(shape):
+    print('relu backward', shape, flush=True)
+    rng  = np.random.default_rng(shape[0])
+    x, g = (rng.standard_normal(shape).astype(np.float32) for _ in range(2))
+    x[0, 0], g[1, 1], x[1, 0], g[0, 1] = np.nan, np.inf, np.float32(0.25), -0.0
+    got, expected = (vkjax_amd.wrap(relu_backward, frontend='minijax', fuse=fuse)(x, g) for fuse in (True, False))
+    for a, b in zip(got, expected):
+        assert np.array_equal(a, b, equal_nan=True)
+    assert np.array_equal(got[0], np.where(x > np.float32(0.25), g, np.float32(0)), equal_nan=True)
+
+
+def scaled_sums(x, c):
+    '''A change of sign behind a mean: of rows, of columns, of everything, with values known before and with one that is not.'''
+    n = np.float32(x.shape[0])
+    return [-(jnp.sum(x, axis=1) / c), -(jnp.sum(x, axis=0) / n), -(jnp.sum(x) / np.float32(x.size)), jnp.sum(x, axis=0) / c, c * jnp.sum(x)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('shape', [(2, 3), (5, 64), (127, 12), (128, 10), (1000, 10), (3, 8192), (4, 40000), (5000, 33)], ids=str)
+def test_scaled_sums_keep_every_bit(shape):
+    x, c = np.random.default_rng(1).standard_normal(shape).astype(np.float32), np.float32(7)
+    x[0, 0], x[1, 1] = 0, -0.0
+    got, expected = (vkjax_amd.wrap(scaled_sums, frontend='minijax', fuse=fuse)(x, c) for fuse in (True, False))
+    kernels = kernels_of(scaled_sums, (x, c), plan_only=True)
+    assert shape[0] > 127 or x.size > 4096 or not any(k.startswith('ew_chain') for k in kernels), kernels       #(split sums keep theirs)
+    for a, b in zip(got, expected):
+        assert np.array_equal(a, b)
+
+
+def known_scalars(x):
+    '''Values that are known before anything runs, and one that is not: quotients that need rounding, signed zeros, an overflow and
+    an underflow (which the device computes).'''
+    neg, div, mul = lax.neg, lax.div, lax.mul
+    f = np.float32
+    values = [div(neg(f(1)), f(1000)), div(f(1), f(3)), mul(div(f(2), f(3)), f(0.1)), neg(f(0)), div(neg(f(0)), f(5)), mul(f(3e38), f(10)), div(f(1e-38), f(10))]
+    return [x * v for v in values] + [values[0]]
+
+
+def test_known_scalars_cost_no_launch():
+    kernels = kernels_of(lambda x: x * lax.div(lax.neg(np.float32(1)), np.float32(1000)), (np.ones(64, np.float32),), plan_only=True)
+    assert len(kernels) == 1, kernels
+
+
+@pytest.mark.gpu
+def test_known_scalars_keep_every_bit():
+    x = np.linspace(-3, 3, 65).astype(np.float32)
+    got, expected = (vkjax_amd.wrap(known_scalars, frontend='minijax', fuse=fuse)(x) for fuse in (True, False))
+    for a, b in zip(got, expected):
+        assert np.array_equal(np.asarray(a, np.float32).view(np.uint32), np.asarray(b, np.float32).view(np.uint32))

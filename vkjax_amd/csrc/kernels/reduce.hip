@@ -82,6 +82,7 @@ template <int POST>
 __device__ __forceinline__ uint32_t reduce_post(uint32_t sum, const uint32_t* __restrict__ post) {
     if constexpr (POST == 1) return f2u(u2f(sum) / u2f(post[0]));
     else if constexpr (POST == 2) return f2u(u2f(sum) * u2f(post[0]));
+    else if constexpr (POST == 4) return f2u(u2f(sum) / u2f(post[0])) ^ 0x80000000u;
     else return sum;
 }
 
@@ -330,7 +331,8 @@ __device__ __forceinline__ void reduce_cols_body(uint32_t* __restrict__ out, con
 #define REDUCE_COLS_PROLOGUE_KERNELS(tag, PRO)                                                                                 \
     extern "C" __global__ __launch_bounds__(256) void reduce_cols_fsum_##tag##_v1(uint32_t* out, const uint32_t* in, const uint32_t* in2, ReduceParams P) { reduce_cols_body<1, 0, PRO>(out, in, P, in2); } \
     extern "C" __global__ __launch_bounds__(256) void reduce_cols_fsum_##tag##_v4(uint32_t* out, const uint32_t* in, const uint32_t* in2, ReduceParams P) { reduce_cols_body<4, 0, PRO>(out, in, P, in2); }
-// float sums followed by a division or a multiplication by one value (a mean): unsplit reductions only
+// float sums followed by a division or a multiplication by one value (a mean), or by a division and a change of sign (a mean
+// negative log-likelihood): unsplit reductions only
 #define REDUCE_POST_KERNELS(tag, POST)                                                                                         \
     extern "C" __global__ __launch_bounds__(256) void reduce_rows_fsum_##tag##_v1(uint32_t* out, const uint32_t* in, const uint32_t* post, ReduceParams P) { reduce_rows_body<1, 0, POST>(out, in, P, post); } \
     extern "C" __global__ __launch_bounds__(256) void reduce_rows_fsum_##tag##_v4(uint32_t* out, const uint32_t* in, const uint32_t* post, ReduceParams P) { reduce_rows_body<4, 0, POST>(out, in, P, post); } \
@@ -389,8 +391,10 @@ __device__ __forceinline__ void reduce_cols_update_body(uint32_t* out, const uin
     const ReduceParams P = {1u, U.R, U.inner, RED_SUM, RT_F32, U.R, 1u, U.TI};
     reduce_cols_body<VEC, 0, PRO_NONE, POST_UPDATE>(out, in, P, nullptr, block, rate, minuend);
 }
-template <int VEC>
-__device__ __forceinline__ void reduce_cols_update_batch_body(const ReduceUpdateEntry* __restrict__ table, uint32_t entries) {
+extern "C" __global__ __launch_bounds__(256) void reduce_cols_fsum_update_v1(uint32_t* out, const uint32_t* in, const uint32_t* minuend, const uint32_t* rate, ReduceUpdateParams P) { reduce_cols_update_body<1>(out, in, minuend, rate, P, blockIdx.x); }
+extern "C" __global__ __launch_bounds__(256) void reduce_cols_fsum_update_v4(uint32_t* out, const uint32_t* in, const uint32_t* minuend, const uint32_t* rate, ReduceUpdateParams P) { reduce_cols_update_body<4>(out, in, minuend, rate, P, blockIdx.x); }
+// (sums over both kinds of column counts share the launch: which body a workgroup takes is the same for all of it)
+extern "C" __global__ __launch_bounds__(256) void reduce_cols_fsum_batch_update(const ReduceUpdateEntry* __restrict__ table, uint32_t entries) {
     uint32_t lo = 0, hi = entries;
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
@@ -398,12 +402,9 @@ __device__ __forceinline__ void reduce_cols_update_batch_body(const ReduceUpdate
     }
     lo = __builtin_amdgcn_readfirstlane(lo);
     const ReduceUpdateEntry& e = table[lo];
-    reduce_cols_update_body<VEC>(e.out, e.in, e.minuend, e.rate, e.P, blockIdx.x - e.first_block);
+    if (e.P.inner % 4u == 0) reduce_cols_update_body<4>(e.out, e.in, e.minuend, e.rate, e.P, blockIdx.x - e.first_block);
+    else                     reduce_cols_update_body<1>(e.out, e.in, e.minuend, e.rate, e.P, blockIdx.x - e.first_block);
 }
-extern "C" __global__ __launch_bounds__(256) void reduce_cols_fsum_update_v1(uint32_t* out, const uint32_t* in, const uint32_t* minuend, const uint32_t* rate, ReduceUpdateParams P) { reduce_cols_update_body<1>(out, in, minuend, rate, P, blockIdx.x); }
-extern "C" __global__ __launch_bounds__(256) void reduce_cols_fsum_update_v4(uint32_t* out, const uint32_t* in, const uint32_t* minuend, const uint32_t* rate, ReduceUpdateParams P) { reduce_cols_update_body<4>(out, in, minuend, rate, P, blockIdx.x); }
-extern "C" __global__ __launch_bounds__(256) void reduce_cols_fsum_batch_update_v1(const ReduceUpdateEntry* __restrict__ table, uint32_t entries) { reduce_cols_update_batch_body<1>(table, entries); }
-extern "C" __global__ __launch_bounds__(256) void reduce_cols_fsum_batch_update_v4(const ReduceUpdateEntry* __restrict__ table, uint32_t entries) { reduce_cols_update_batch_body<4>(table, entries); }
 
 // the _v4 variants need R % 4 == 0, r_chunk % 4 == 0 (rows) or inner % 4 == 0 (cols) and 16-byte aligned pointers
 REDUCE_COLS_PROLOGUE_KERNELS(mul, PRO_MUL)
@@ -411,6 +412,7 @@ REDUCE_COLS_PROLOGUE_KERNELS(mulv, PRO_MULV)
 REDUCE_COLS_PROLOGUE_KERNELS(neg, PRO_NEG)
 REDUCE_POST_KERNELS(div, 1)
 REDUCE_POST_KERNELS(times, 2)
+REDUCE_POST_KERNELS(negdiv, 4)
 REDUCE_KERNELS(fsum, 0)
 REDUCE_KERNELS(fmax, 1)
 // Any other combination of operation and element type. The combine is selected once per launch: every case calls the
@@ -446,14 +448,14 @@ REDUCE_KERNELS(fargmin, 4)
 // sums over rows r_lo + tr, + TR, ..., then the same tree over tr in LDS), so sum_m and sum_mx hold
 // the bits the separate launches would have produced, partial results per row range included.
 // SELECT = false: m is g itself (no activation between the scale and what follows; ans, thr and alt unused).
-template <int VEC, bool SELECT>
+template <int VEC, bool SELECT, bool SCALED>
 __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx, float* __restrict__ sum_m, float* __restrict__ sum_mx,
                                                          const float* __restrict__ ans, const float* __restrict__ thr,
                                                          const float* __restrict__ g, const float* __restrict__ alt,
                                                          const float* __restrict__ x, const float* __restrict__ kvec,
                                                          const ReduceParams& P) {
     __shared__ float s_m[256 * VEC];
-    __shared__ float s_x[256 * VEC];
+    __shared__ float s_x[SCALED ? 256 * VEC : 1];
     const uint32_t TI = P.TI, TR = 256u / TI;
     const uint32_t tid = threadIdx.x, ti = tid % TI, tr = tid / TI;
     const uint32_t tiles_i = (P.inner + TI * VEC - 1u) / (TI * VEC);
@@ -469,19 +471,23 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
         const uint64_t base = (uint64_t)o * P.R * P.inner + i;
         float kv[VEC];
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) kv[j] = kvec[i + j];
+        for (int j = 0; j < VEC; ++j) kv[j] = SCALED ? kvec[i + j] : 0.f;
         auto fetch = [&](uint32_t row, float (&a)[VEC], float (&c)[VEC], float (&v)[VEC]) {
             const uint64_t off = base + (uint64_t)row * P.inner;
             if constexpr (VEC == 4) {
-                const f32x4 tc = *reinterpret_cast<const f32x4*>(g + off), tv = *reinterpret_cast<const f32x4*>(x + off);
+                const f32x4 tc = *reinterpret_cast<const f32x4*>(g + off);
                 c[0] = tc.x; c[1] = tc.y; c[2] = tc.z; c[3] = tc.w;
-                v[0] = tv.x; v[1] = tv.y; v[2] = tv.z; v[3] = tv.w;
+                if constexpr (SCALED) {
+                    const f32x4 tv = *reinterpret_cast<const f32x4*>(x + off);
+                    v[0] = tv.x; v[1] = tv.y; v[2] = tv.z; v[3] = tv.w;
+                }
                 if constexpr (SELECT) {
                     const f32x4 ta = *reinterpret_cast<const f32x4*>(ans + off);
                     a[0] = ta.x; a[1] = ta.y; a[2] = ta.z; a[3] = ta.w;
                 }
             } else {
-                c[0] = g[off]; v[0] = x[off];
+                c[0] = g[off];
+                if constexpr (SCALED) v[0] = x[off];
                 if constexpr (SELECT) a[0] = ans[off];
             }
         };
@@ -490,9 +496,9 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
 #pragma unroll
             for (int j = 0; j < VEC; ++j) {
                 m[j] = SELECT ? (a[j] > t ? c[j] : z) : c[j];
-                d[j] = m[j] * kv[j];
+                d[j] = SCALED ? m[j] * kv[j] : m[j];
                 acc_m[j] = acc_m[j] + m[j];
-                acc_x[j] = acc_x[j] + m[j] * v[j];
+                if constexpr (SCALED) acc_x[j] = acc_x[j] + m[j] * v[j];
             }
             const uint64_t off = base + (uint64_t)row * P.inner;
             if constexpr (VEC == 4) *reinterpret_cast<f32x4*>(dx + off) = f32x4{d[0], d[1], d[2], d[3]};
@@ -517,7 +523,7 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
         }
     }
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) { s_m[tid * VEC + j] = acc_m[j]; s_x[tid * VEC + j] = acc_x[j]; }
+    for (int j = 0; j < VEC; ++j) { s_m[tid * VEC + j] = acc_m[j]; if constexpr (SCALED) s_x[tid * VEC + j] = acc_x[j]; }
     __syncthreads();
     for (uint32_t s = TR >> 1; s >= 1; s >>= 1) {
         if (tr < s) {
@@ -525,7 +531,7 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
             for (int j = 0; j < VEC; ++j) {
                 const uint32_t mine = tid * VEC + j, other = (tid + s * TI) * VEC + j;
                 s_m[mine] = s_m[mine] + s_m[other];
-                s_x[mine] = s_x[mine] + s_x[other];
+                if constexpr (SCALED) s_x[mine] = s_x[mine] + s_x[other];
             }
         }
         __syncthreads();
@@ -533,7 +539,7 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
     if (tr == 0 && i < P.inner) {
         const uint64_t dst = ((uint64_t)o * P.nsplit + sp) * P.inner + i;
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) { sum_m[dst + j] = s_m[tid * VEC + j]; sum_mx[dst + j] = s_x[tid * VEC + j]; }
+        for (int j = 0; j < VEC; ++j) { sum_m[dst + j] = s_m[tid * VEC + j]; if constexpr (SCALED) sum_mx[dst + j] = s_x[tid * VEC + j]; }
     }
 }
 
@@ -541,13 +547,24 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
     extern "C" __global__ __launch_bounds__(256) void name(float* dx, float* sum_m, float* sum_mx, const float* ans,   \
                                                            const float* thr, const float* g, const float* alt,        \
                                                            const float* x, const float* kvec, ReduceParams P) {       \
-        scale_relu_backward_body<VEC, SELECT>(dx, sum_m, sum_mx, ans, thr, g, alt, x, kvec, P);                              \
+        scale_relu_backward_body<VEC, SELECT, true>(dx, sum_m, sum_mx, ans, thr, g, alt, x, kvec, P);                        \
     }
 // _v4 needs inner % 4 == 0 and 16-byte aligned arrays
 SCALE_RELU_BACKWARD_KERNEL(scale_relu_backward_v1, 1, true)
 SCALE_RELU_BACKWARD_KERNEL(scale_relu_backward_v4, 4, true)
 SCALE_RELU_BACKWARD_KERNEL(scale_backward_v1, 1, false)
 SCALE_RELU_BACKWARD_KERNEL(scale_backward_v4, 4, false)
+// m itself and its column sums (a dense layer's ReLU: the sums are its bias gradient). Memory bounds it from some MB on: 65536 x 256
+// 52 us as two launches, 43 as one. Below that the launches do; the step of a 784-300-100-10 network over 1000 rows has two of
+// these, and with them, the sign behind its loss's mean, its known scalars and one batch for all its updates it takes 114 us
+// in 16 launches (128 us in 21).
+#define RELU_BACKWARD_KERNEL(name, VEC)                                                                                     \
+    extern "C" __global__ __launch_bounds__(256) void name(float* m, float* sum_m, const float* ans, const float* thr,     \
+                                                           const float* g, const float* alt, ReduceParams P) {             \
+        scale_relu_backward_body<VEC, true, false>(m, sum_m, nullptr, ans, thr, g, alt, nullptr, nullptr, P);                \
+    }
+RELU_BACKWARD_KERNEL(relu_backward_v1, 1)
+RELU_BACKWARD_KERNEL(relu_backward_v4, 4)
 
 // ---------------------------------------------------------------------------------------------
 // softmax over the rows of [outer, R] in one launch: out = exp(x - max(x)) / sum(exp(x - max(x))).

@@ -53,6 +53,8 @@ def _reads(op) -> tp.List:
             return [op.meta[2]]
         if op.meta[0] == 'threefry':
             return list(op.meta[2])
+        if op.meta[0] == 'relu_backward':
+            return [b for b, _ in op.launch.buffers[2:]]
         if op.meta[0] in ('random_stream', 'reduce', 'update'):
             return [b for b, _ in op.launch.buffers[1:] if b is not None]
         if op.meta[0] == 'softmax':
@@ -158,6 +160,7 @@ def _epilogue_steps(steps: tp.Sequence[EwStep], geom: K.ConvGeometry, out_shape)
 
 def fuse_ops(all_ops, bufferpool, outvars):
     from .ops import Op
+    all_ops = fold_scalar_constants(all_ops, bufferpool, outvars)
     uses = collections.Counter()
     for op in all_ops:
         for b in _reads(op):
@@ -325,6 +328,7 @@ def fuse_ops(all_ops, bufferpool, outvars):
     ops = fuse_reduce_updates(ops, bufferpool, outvars)
     ops = fuse_derived_epilogue_operands(ops, bufferpool, outvars)
     ops = fuse_relu_backward_epilogues(ops, bufferpool, outvars)
+    ops = fuse_relu_backward_sums(ops, bufferpool, outvars)
     ops = fuse_index_wrap(ops, bufferpool, outvars)
     ops = fold_index_wrap(ops, bufferpool, outvars)
     ops = fuse_dense_softmax(ops, bufferpool, outvars)
@@ -746,46 +750,53 @@ def fuse_reduce_prologues(ops, bufferpool, outvars):
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
 
 
+def _is_float_sum(op) -> bool:
+    '''A launch that writes finished float sums: an unsplit reduction, or the second launch of one that is split (of the
+    slices of a kernel gradient too).'''
+    return (op.chain is None and op.conv is None and (op.meta is None or op.meta[0] == 'reduce')
+            and op.launch.kernel.startswith(('reduce_rows_fsum_v', 'reduce_cols_fsum_v')))
+
+
+def _sole_reader_takes(ops, i, C, uses) -> bool:
+    '''The sum ops[i], which ops[C] reads, is read by nothing else and could be taken where ops[C] stands: its operand still
+    holds the same values there.'''
+    out, source = ops[i].launch.buffers[0][0], ops[i].launch.buffers[1][0]
+    #(a launch without a record of its structure counts among the readers of its own result)
+    own = sum(b._placeholder is out._placeholder for b in _reads(ops[i]))
+    return (i < C and uses[id(out._placeholder)] - own == 1
+            and not any(w._placeholder is source._placeholder for j in range(i + 1, C) for w in _may_write(ops[j])))
+
+
 def fuse_reduce_scales(ops, bufferpool, outvars):
-    '''A float sum (one launch: not split into ranges) whose result is read once, by `sum / c` or `sum * c` with a
-    single value c - a mean - stores the quotient / product itself: the element-wise launch behind it goes away. The
-    division is the one the element-wise kernel would have made (same operands, same rounding).'''
+    '''A float sum (one launch: not split into ranges) whose result is read once, by `sum / c`, `sum * c` or `-(sum / c)` with a single value c - a mean, a mean
+    negative log-likelihood - stores that itself: the element-wise launch behind it goes away. The division is the one
+    the element-wise kernel would have made (same operands, same rounding).'''
     from .ops import Op
     uses = _use_counts(ops, bufferpool, outvars)
     pid  = lambda b: id(b._placeholder)
+    sums = {pid(op.launch.buffers[0][0]): i for i, op in enumerate(ops) if _is_float_sum(op) and op.meta is not None and op.meta[8] == 1}
     removed, replacement = set(), {}
-    for i, R in enumerate(ops):
-        if R.meta is None or R.meta[0] != 'reduce' or i + 1 >= len(ops):
+    for C, op in enumerate(ops):
+        ch = op.chain
+        if ch is None or not ch.steps or ch.steps[0].operand is None:
             continue
-        _, out, inp, outer, rows, inner, name, partial, nsplit = R.meta
-        if name != 'reduce_sum' or nsplit != 1 or inp.dtype != 'float32' or uses[pid(out)] != 1:
-            continue
-        #the reader: the next launch that reads the sum (nothing in between touches it, it has one use)
-        C = next((j for j in range(i + 1, len(ops)) if any(b._placeholder is out._placeholder for b in _reads(ops[j]))), None)
-        if C is None or ops[C].chain is None:
-            continue
-        #the sum is taken where its reader stood: its operand must still hold the same values there
-        if any(w._placeholder is inp._placeholder for j in range(i + 1, C) for w in _may_write(ops[j])):
-            continue
-        ch = ops[C].chain
-        if len(ch.steps) != 1 or ch.steps[0].operand is None:
-            continue
-        step = ch.steps[0]
-        total, o = ch.first, step.operand
-        if step.op == EW['MUL_F'] and o.buffer._placeholder is out._placeholder:
+        kind = {(EW['DIV_F'],): 'div', (EW['MUL_F'],): 'times', (EW['DIV_F'], EW['NEG_F']): 'negdiv'}.get(tuple(st.op for st in ch.steps))
+        total, o = ch.first, ch.steps[0].operand
+        if kind == 'times' and pid(total.buffer) not in sums:
             total, o = o, ch.first                              #c * sum: the product is the same number
-        elif step.op == EW['DIV_F'] and step.operand_left:
-            continue                                            #c / sum
-        kind = 'div' if step.op == EW['DIV_F'] else 'times' if step.op == EW['MUL_F'] else None
-        if (kind is None or total.buffer._placeholder is not out._placeholder or not _is_full_contiguous_any_shape(total, ch.shape)
-                or o.buffer.size != 1 or o.offset != 0 or ch.out.size != out.size):
+        i = sums.get(pid(total.buffer))
+        if (kind is None or (kind != 'times' and ch.steps[0].operand_left) or i is None or not _sole_reader_takes(ops, i, C, uses)
+                or not _is_full_contiguous_any_shape(total, ch.shape) or o.buffer.size != 1 or o.offset != 0
+                or o.buffer.dtype != 'float32' or ch.out.dtype != 'float32' or ch.out.size != total.buffer.size):
             continue
-        launch = K.reduce(ch.out, inp, outer, rows, inner, name, None, 1, post=(kind, o.buffer))[0]
-        fused  = Op(_label(R, ops[C]), launch=launch, meta=None)
-        fused.index = ops[C].index
-        for b in (inp, o.buffer):
-            b.accesses.append(ops[C].index)
-        out._placeholder.elided = True
+        launch = K.sum_with_post(ops[i].launch, ch.out, kind, o.buffer)
+        if launch is None:
+            continue
+        fused = Op(_label(ops[i], op), launch=launch, meta=None)
+        fused.index = op.index
+        for b in (ops[i].launch.buffers[1][0], o.buffer):
+            b.accesses.append(op.index)
+        total.buffer._placeholder.elided = True
         removed.add(i)
         replacement[C] = fused
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
@@ -800,8 +811,7 @@ def fuse_reduce_updates(ops, bufferpool, outvars):
     from .ops import Op
     uses = _use_counts(ops, bufferpool, outvars)
     pid  = lambda b: id(b._placeholder)
-    sums = {pid(op.launch.buffers[0][0]): i for i, op in enumerate(ops)
-            if op.chain is None and op.conv is None and op.launch.kernel in K.REDUCE_BATCH_KERNELS}
+    sums = {pid(op.launch.buffers[0][0]): i for i, op in enumerate(ops) if _is_float_sum(op)}
     removed, replacement = set(), {}
     for C, op in enumerate(ops):
         ch = op.chain
@@ -811,25 +821,18 @@ def fuse_reduce_updates(ops, bufferpool, outvars):
         if pid(total.buffer) not in sums:
             total, rate = rate, total                           #rate * sum: the product is the same number
         i = sums.get(pid(total.buffer))
-        if i is None or i in removed or i > C:
-            continue
-        #(a launch without a record of its structure counts among the readers of its own result)
-        if uses[pid(total.buffer)] - sum(b._placeholder is total.buffer._placeholder for b in _reads(ops[i])) != 1:
+        if i is None or not _sole_reader_takes(ops, i, C, uses):
             continue
         n = total.buffer.size
         if (rate.buffer.size != 1 or rate.offset != 0 or ch.out.size != n or before.buffer.size != n or before.buffer.dtype != 'float32'
                 or ch.out.dtype != 'float32' or not all(_is_full_contiguous_any_shape(o, ch.shape) for o in (total, before))):
-            continue
-        source = ops[i].launch.buffers[1][0]
-        #the sum is taken where the update stood: its operand must still hold the same values there
-        if any(w._placeholder is source._placeholder for j in range(i + 1, C) for w in _may_write(ops[j])):
             continue
         launch = K.column_sum_update(ops[i].launch, ch.out, before.buffer, rate.buffer)
         if launch is None:
             continue
         fused = Op(_label(ops[i], op), launch=launch, meta=('update',))
         fused.index = op.index
-        source.accesses.append(op.index)
+        ops[i].launch.buffers[1][0].accesses.append(op.index)
         total.buffer._placeholder.elided = True
         removed.add(i)
         replacement[C] = fused
@@ -1022,6 +1025,96 @@ def fuse_relu_backward_epilogues(ops, bufferpool, outvars):
     return [op for op in ops if op is not None]
 
 
+def _select_by_threshold(chain) -> bool:
+    '''`chain` is select(ans > t, g, z) of two whole float arrays and two single values.'''
+    single = lambda o: o is not None and o.offset == 0 and o.buffer.size == 1 and o.buffer.dtype == 'float32'
+    return (chain is not None and [st.op for st in chain.steps] == [EW['GT_F'], EW['SEL_P'], EW['NOP']] and not chain.steps[0].operand_left
+            and single(chain.steps[0].operand) and single(chain.steps[2].operand)
+            and all(_is_full_contiguous_any_shape(o, chain.shape) and o.buffer.dtype == 'float32' for o in (chain.first, chain.steps[1].operand))
+            and chain.out.dtype == 'float32' and chain.out.size == np_prod(chain.shape))
+
+
+def fuse_relu_backward_sums(ops, bufferpool, outvars):
+    '''The backward pass of a dense layer's ReLU and the gradient of the bias in front of it,
+
+        m = select(ans > t, g, z) ; db = sum_rows(m)
+
+    become ONE launch that writes m and the column sums (their first stage, when they are split over row ranges), in the order
+    of the launch it replaces. It runs behind the passes that take the select into a product's epilogue. No line by size: the
+    launch has the grid of the sum, and replays of the pair took as long or longer at every size that was timed (127 x 256
+    14.6 -> 5.4 us, 1000 x 300 18.4 -> 15.3, 1000 x 7 15.2 -> 15.4, 65536 x 256 52.4 -> 42.9, 100000 x 33 30.4 -> 29.4).'''
+    from .ops import Op
+    pid = lambda b: id(b._placeholder)
+    selects = {pid(op.chain.out): i for i, op in enumerate(ops) if _select_by_threshold(op.chain)}
+    removed, replacement = set(), {}
+    for i, R in enumerate(ops):
+        if R.meta is None or R.meta[0] != 'reduce' or R.launch.kernel not in K.REDUCE_BATCH_KERNELS:
+            continue
+        _, _, m, outer, rows, inner, _, _, _ = R.meta
+        M = selects.get(pid(m))
+        if M is None or M > i or M in replacement or outer != 1 or rows * inner != m.size:
+            continue
+        ch, sums = ops[M].chain, R.launch.buffers[0][0]
+        #the sums are written where the select stood, and m must not change between there and the launch that summed it
+        if any(pid(b) in (pid(m), pid(sums)) for op in ops[M + 1:i] for b in _may_write(op)):
+            continue
+        launch = K.relu_backward(R.launch, ch.out, sums, ch.steps[1].operand.buffer, (ch.first.buffer, ch.steps[0].operand.buffer, ch.steps[2].operand.buffer))
+        fused  = Op(_label(ops[M], R), launch=launch, meta=('relu_backward', [ch.out, sums]))
+        fused.index = ops[M].index
+        for b, _ in launch.buffers:
+            b.accesses.append(fused.index)
+        removed.add(i)
+        replacement[M] = fused
+    return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
+
+
+def fold_scalar_constants(ops, bufferpool, outvars):
+    '''Arithmetic on single floats that are known when the program is built (-1 / 1000, the factor of a mean's gradient) is done
+    then, with the device's rounding, and its result is a constant like the ones it came from: one launch less per value
+    (4 us in a chain of small launches). Results that are no normal number or zero are left to the device.'''
+    from .buffers import to_device_words
+    operations = {EW['NEG_F']: lambda a, b: -a, EW['ADD_F']: lambda a, b: a + b, EW['SUB_F']: lambda a, b: a - b,
+                  EW['MUL_F']: lambda a, b: a * b, EW['DIV_F']: lambda a, b: a / b}
+    returned = set()
+    for v in outvars:
+        b = bufferpool.get_buffer(v)
+        if b is not None:
+            returned.add(id(b._placeholder))
+            b.accesses.pop()                       #the lookup above is not a device access
+    normal   = lambda v: v == 0 or (np.isfinite(v) and abs(v) >= np.finfo(np.float32).tiny)
+
+    def known(operand):
+        b = operand.buffer
+        if b.size != 1 or b.dtype != 'float32' or operand.offset != 0 or b.constant_value is None:
+            return None
+        value = np.asarray(b.constant_value)
+        return np.float32(value.reshape(())) if value.size == 1 and value.dtype in (np.float32, np.float64) else None
+
+    kept = []
+    for op in ops:
+        ch = op.chain
+        if (ch is None or ch.out.size != 1 or ch.out.dtype != 'float32' or not ch.steps or ch.out.tensor is not None
+                or id(ch.out._placeholder) in returned or any(st.op not in operations for st in ch.steps)):
+            kept.append(op)
+            continue
+        value = known(ch.first)
+        for st in ch.steps:
+            other = known(st.operand) if st.operand is not None else np.float32(0)
+            if value is None or other is None:
+                value = None
+                break
+            with np.errstate(all='ignore'):
+                value = operations[st.op](*((other, value) if st.operand_left else (value, other)))
+            value = value if normal(value) else None
+        if value is None:
+            kept.append(op)
+            continue
+        ch.out.tensor         = bufferpool.device.tensor(to_device_words(value.reshape(1)))
+        ch.out.constant_value = value
+        ch.out.accesses      += [0, np.inf]
+    return kept
+
+
 def _is_full_contiguous_any_shape(operand: EwOperand, shape) -> bool:
     '''The operand covers `shape` densely in row-major order (its buffer may carry another shape of the same size).'''
     size = 1
@@ -1206,7 +1299,7 @@ def _writes(op) -> tp.List:
         return [_out(op)]
     if op.meta is not None and op.meta[0] in ('iota', 'concat_part'):
         return [op.meta[1]]
-    if op.meta is not None and op.meta[0] in ('threefry', 'softmax', 'rows'):
+    if op.meta is not None and op.meta[0] in ('threefry', 'softmax', 'rows', 'relu_backward'):
         return list(op.meta[1])
     return [b for b, _ in op.launch.buffers[:1] if b is not None]      #kernels write their first argument
 
@@ -1387,7 +1480,7 @@ def _small_out(op):
 
 def _may_write(op) -> tp.List:
     '''Buffers an op may change: its result where the op's structure is known, else everything it touches.'''
-    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'random_stream', 'reduce', 'update', 'softmax', 'rows', 'conv_pack')):
+    if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'random_stream', 'reduce', 'update', 'relu_backward', 'softmax', 'rows', 'conv_pack')):
         return _writes(op)
     return [b for b, _ in op.launch.buffers if b is not None]
 
@@ -1506,7 +1599,7 @@ def batch_small_chains(ops):
             by_kernel: tp.Dict[str, list] = {}
             for k, op in enumerate(run):
                 if level[k] == lv:
-                    by_kernel.setdefault(op.launch.kernel, []).append(op)
+                    by_kernel.setdefault(K.BATCH_KERNELS[op.launch.kernel], []).append(op)
             for group in by_kernel.values():
                 if len(group) == 1:
                     result.append(group[0])

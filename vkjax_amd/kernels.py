@@ -339,7 +339,8 @@ REDUCE_BATCH_KERNELS = ('reduce_cols_fsum_v1', 'reduce_cols_fsum_v4')
 UPDATE_BATCH_KERNELS = ('reduce_cols_fsum_update_v1', 'reduce_cols_fsum_update_v4')
 TRANSPOSE_BATCH_KERNELS = ('transpose_tiled_v4', 'transpose_tiled_v4_t128')
 BATCH_KERNELS        = {**{k: k.replace('ew_chain_', 'ew_chain_batch_') for k in EW_BATCH_KERNELS},
-                        **{k: k.replace('fsum_', 'fsum_batch_') for k in REDUCE_BATCH_KERNELS + UPDATE_BATCH_KERNELS},
+                        **{k: k.replace('fsum_', 'fsum_batch_') for k in REDUCE_BATCH_KERNELS},
+                        **{k: 'reduce_cols_fsum_batch_update' for k in UPDATE_BATCH_KERNELS},
                         **{k: k.replace('tiled_', 'tiled_batch_') for k in TRANSPOSE_BATCH_KERNELS},
                         'conv_split_pack': 'conv_split_pack_layers'}
 EW_BATCH_ENTRY_BYTES        = 432
@@ -356,11 +357,11 @@ def _blocks(launch: Launch) -> int:
 
 
 def batch_launch(members: tp.Sequence[Launch]) -> Launch:
-    '''One launch for several small launches of the same kernel (element-wise chains or float column sums)
+    '''One launch for several small launches of one batch kernel (element-wise chains or float column sums)
     that do not depend on one another.'''
-    kernel = members[0].kernel
-    assert kernel in BATCH_KERNELS and all(m.kernel == kernel and not m.members for m in members), [m.kernel for m in members]
-    return Launch(BATCH_KERNELS[kernel], (sum(_blocks(m) for m in members), 1, 1), (BLOCK, 1, 1), [],
+    kernel = BATCH_KERNELS[members[0].kernel]
+    assert all(BATCH_KERNELS[m.kernel] == kernel and not m.members for m in members), [m.kernel for m in members]
+    return Launch(kernel, (sum(_blocks(m) for m in members), 1, 1), (BLOCK, 1, 1), [],
                   _u32(len(members)), bytes_moved=sum(m.bytes_moved for m in members), members=tuple(members))
 
 
@@ -1327,21 +1328,14 @@ def plan_reduce_splits(outer: int, R: int, inner: int, op: str, compute_units: i
 
 
 def _reduce_launch(out: Buffer, inp: Buffer, outer: int, R: int, inner: int, op: str, nsplit: int, in_offset_ok=True,
-                   prologue: tp.Optional[tp.Tuple[str, tp.Optional[Buffer]]] = None,
-                   post: tp.Optional[tp.Tuple[str, Buffer]] = None) -> Launch:
+                   prologue: tp.Optional[tp.Tuple[str, tp.Optional[Buffer]]] = None) -> Launch:
     ty   = _RTYPE[inp.dtype]
     mode = {('reduce_sum', 0): 'fsum', ('reduce_max', 0): 'fmax', ('argmax', 0): 'fargmax', ('argmin', 0): 'fargmin'}.get((op, ty), 'any')
     r_chunk = _cdiv(_cdiv(R, nsplit), 4) * 4
     nsplit  = _cdiv(R, r_chunk)
-    if post is not None:
-        #('div' | 'times', one value): applied to every finished float sum of an unsplit reduction
-        assert mode == 'fsum' and nsplit == 1 and prologue is None and post[0] in ('div', 'times') and post[1].size == 1
     if inner == 1:
         vec = 4 if R % 4 == 0 else 1
         params = _u32(outer, R, 1, RED[op], ty, r_chunk, nsplit, 0)
-        if post is not None:
-            return Launch(f'reduce_rows_fsum_{post[0]}_v{vec}', (_cdiv(outer * nsplit, 4), 1, 1), (BLOCK, 1, 1), [(out, 0), (inp, 0), (post[1], 0)],
-                          params, bytes_moved=4 * (outer * R + outer * nsplit)), nsplit
         return Launch(f'reduce_rows_{mode}_v{vec}', (_cdiv(outer * nsplit, 4), 1, 1), (BLOCK, 1, 1), [(out, 0), (inp, 0)], params,
                       bytes_moved=4 * (outer * R + outer * nsplit)), nsplit
     vec = 4 if inner % 4 == 0 else 1
@@ -1364,20 +1358,16 @@ def _reduce_launch(out: Buffer, inp: Buffer, outer: int, R: int, inner: int, op:
         extra = 0 if second is None else second.size
         return Launch(f'reduce_cols_fsum_{kind}_v{vec}', (blocks, 1, 1), (BLOCK, 1, 1), [(out, 0), (inp, 0), (second, 0)], params,
                       bytes_moved=4 * (outer * R * inner + outer * nsplit * inner + extra)), nsplit
-    if post is not None:
-        return Launch(f'reduce_cols_fsum_{post[0]}_v{vec}', (blocks, 1, 1), (BLOCK, 1, 1), [(out, 0), (inp, 0), (post[1], 0)], params,
-                      bytes_moved=4 * (outer * R * inner + outer * nsplit * inner)), nsplit
     return Launch(f'reduce_cols_{mode}_v{vec}', (blocks, 1, 1), (BLOCK, 1, 1), [(out, 0), (inp, 0)], params,
                   bytes_moved=4 * (outer * R * inner + outer * nsplit * inner)), nsplit
 
 
 def reduce(out: Buffer, inp: Buffer, outer: int, R: int, inner: int, op: str,
-           partial: tp.Optional[Buffer] = None, nsplit: int = 1, prologue=None, post=None) -> tp.List[Launch]:
+           partial: tp.Optional[Buffer] = None, nsplit: int = 1, prologue=None) -> tp.List[Launch]:
     '''[outer, R, inner] -> [outer, inner]. With nsplit > 1, `partial` (outer * nsplit * inner words) receives
-    the per-range results of a first launch and a second launch reduces them. `prologue`, `post`: see _reduce_launch.'''
+    the per-range results of a first launch and a second launch reduces them. `prologue`: see _reduce_launch.'''
     if nsplit <= 1:
-        return [_reduce_launch(out, inp, outer, R, inner, op, 1, prologue=prologue, post=post)[0]]
-    assert post is None
+        return [_reduce_launch(out, inp, outer, R, inner, op, 1, prologue=prologue)[0]]
     first, nsplit = _reduce_launch(partial, inp, outer, R, inner, op, nsplit, prologue=prologue)
     if nsplit == 1:
         return [_reduce_launch(out, inp, outer, R, inner, op, 1, prologue=prologue)[0]]
@@ -1414,6 +1404,28 @@ def scale_relu_backward(column_sum: Launch, dx: Buffer, sum_m: Buffer, sum_mx: B
     return Launch(name + column_sum.kernel[-2:], column_sum.grid, column_sum.block,
                   [(dx, 0), (sum_m, 0), (sum_mx, 0), (ans, 0), (threshold, 0), (cotangent, 0), (otherwise, 0), (x, 0), (scale, 0)],
                   column_sum.params, bytes_moved=4 * ((4 if select is not None else 3) * n + 2 * scale.size), written=(0, 1, 2))
+
+
+def relu_backward(column_sum: Launch, m: Buffer, sum_m: Buffer, cotangent: Buffer, select: tp.Tuple[Buffer, Buffer, Buffer]) -> Launch:
+    '''m = ans > threshold ? cotangent : otherwise with select = (ans, threshold, otherwise), and sum_m receives what
+    `column_sum` would write for m.'''
+    assert column_sum.kernel in REDUCE_BATCH_KERNELS, column_sum.kernel
+    ans, threshold, otherwise = select
+    assert ans.size == cotangent.size == m.size and threshold.size == otherwise.size == 1
+    return Launch('relu_backward_' + column_sum.kernel[-2:], column_sum.grid, column_sum.block,
+                  [(m, 0), (sum_m, 0), (ans, 0), (threshold, 0), (cotangent, 0), (otherwise, 0)], column_sum.params,
+                  bytes_moved=12 * m.size + 4 * sum_m.size, written=(0, 1))
+
+
+def sum_with_post(total: Launch, out: Buffer, kind: str, value: Buffer) -> tp.Optional[Launch]:
+    '''An unsplit float sum that stores sum / value, sum * value or -(sum / value) (kind 'div', 'times', 'negdiv'; one value).'''
+    if total.kernel not in ('reduce_rows_fsum_v1', 'reduce_rows_fsum_v4') + REDUCE_BATCH_KERNELS:
+        return None
+    if np.frombuffer(total.params, dtype=np.uint32)[6] != 1:
+        return None
+    assert kind in ('div', 'times', 'negdiv') and value.size == 1 and out.size == total.buffers[0][0].size
+    return Launch(total.kernel.replace('fsum_', f'fsum_{kind}_'), total.grid, total.block, [(out, 0), total.buffers[1], (value, 0)], total.params,
+                  bytes_moved=total.bytes_moved)
 
 
 SOFTMAX_MAX_ROW = 4096      #rows this short run unsplit in reduce_rows, whose summation order softmax_rows repeats
