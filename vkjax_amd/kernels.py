@@ -944,14 +944,30 @@ def _conv_fast_paths(lhs: Buffer, rhs: Buffer, g: ConvGeometry, lhs_offset: int 
     return needs_masks, x_bias, a_fast, b_fast, c_contig
 
 
-def _four_waves_per_tile(g: ConvGeometry, a_fast: bool, c_contig: bool, compute_units: int) -> bool:
+def _four_waves_per_tile(g: ConvGeometry, a_fast: bool, c_contig: bool, compute_units: int, b_fast: bool = True) -> bool:
     '''A product with so few 32 x 32 tiles that one wave per tile leaves most MFMA units idle: four waves per tile,
     each taking a quarter of every (128-long) k step.'''
     want = (CHOICES.conv_ksplit if CHOICES.conv_ksplit is not None else
-            (_cdiv(g.M, 32) * _cdiv(g.N, 32) <= 2 * compute_units and g.K >= 256 and CHOICES.conv_tile is None and CHOICES.conv_bk is None))
+            (CHOICES.conv_tile is None and CHOICES.conv_bk is None and _four_waves_pay(g, b_fast, compute_units)))
     return bool(want) and a_fast and c_contig and (g.Cin % 64 == 0 or g.KH * g.KW == 1) and not CHOICES.conv_general
 
 
+def _four_waves_pay(g: ConvGeometry, b_fast: bool, compute_units: int) -> bool:
+    '''By the rounds of one 32 x 32 tile per CU, against 64 x 64 tiles with a k step of 32 (us for M x K x N, alone):
+    up to one, always (1000 x 32 x 100: 4.1 against 4.4, 196 x 64 x 512 4.1, 5.0, 196 x 224 x 512 4.8, 8.1); up to two, from a
+    contraction of 64 on (784 x 32 x 512 5.1, 4.5, x 64 5.1, 5.2, x 128 5.1, 6.4, x 160 6.7, 7.1, x 256 6.7, 9.0); up to three, where
+    a step of 128 that is only partly used does not cost more than it saves: 2.1 us against 0.65 for one of 32 (784 x 128 x 768 6.1,
+    6.7, x 192 8.3, 8.0, x 256 8.3, 9.4, x 1024 19.6, 26.4); up to four, only long contractions (784 x 256 x 1024 9.8, 9.6, x 512
+    14.6, 14.6, x 1024 23.7, 29.4). Without 16-byte loads of the kernel operand up to two
+    rounds, from a contraction of 64 (200 x 16 x 1000 5.1, 4.3, x 64 5.1, 5.9, x 200 7.8, 12.2) and 128 (255 x 64 x 2048 6.7, 6.0, x 128
+    8.0, 8.5). Windows from 256 on and up to two rounds, as they were measured in networks.'''
+    rounds = _cdiv(_cdiv(g.M, 32) * _cdiv(g.N, 32), compute_units)
+    if g.KH * g.KW != 1:
+        return rounds <= 2 and g.K >= 256
+    if not b_fast:
+        return rounds <= 2 and g.K >= 64 * rounds
+    return (rounds <= 1 or (rounds == 2 and g.K >= 64) or (rounds == 3 and 3.2 * _cdiv(g.K, 128) < _cdiv(g.K, 32))
+            or (rounds == 4 and g.K >= 1024))
 
 
 def conv_k_splits(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int = 256) -> int:
@@ -965,8 +981,8 @@ def conv_k_splits(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int 
     g = _flatten_pointwise(g)
     if g.K * g.N * 4 >= 2**31 or lhs.size * 4 >= 2**31 or g.M * g.N == 0:
         return 1
-    _, _, a_fast, _, c_contig = _conv_fast_paths(lhs, rhs, g)
-    if not _four_waves_per_tile(g, a_fast, c_contig, compute_units) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
+    _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g)
+    if not _four_waves_per_tile(g, a_fast, c_contig, compute_units, b_fast) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
         return 1
     tiles, ksteps = _cdiv(g.M, 32) * _cdiv(g.N, 32), _cdiv(g.K, 128)
     if CHOICES.conv_k_splits is not None:
@@ -1022,7 +1038,7 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
     flat_rows = g.batch == 1 and g.Wo == 1 and g.SH == 1 and g.PH == 0 and g.PW == 0 and not needs_masks
     #a product with so few 32 x 32 tiles that one wave per tile leaves most MFMA units idle: four waves per
     #tile, each taking a quarter of every (128-long) k step
-    ksplit = _four_waves_per_tile(g, a_fast, c_contig, compute_units) and (not epilogue or slots != 0)
+    ksplit = _four_waves_per_tile(g, a_fast, c_contig, compute_units, b_fast) and (not epilogue or slots != 0)
     #(windows over 64 input features take a 64-long k step, with 16-byte loads of the kernel operand only)
     short_step = ksplit and g.Cin % 128 != 0 and g.KH * g.KW != 1
     if short_step and not b_fast:
@@ -1174,7 +1190,7 @@ def _conv_split_pays(g: ConvGeometry, c_contig: bool) -> bool:
         return False
     #few tiles: the fp32 kernel whose four waves share a tile is ahead until the contraction is long (K = 2048, 4096 and 8192: 4096 x 64 22, 16;
     #31, 27; 46, 48. 4096 x 128 31, 24; 42, 43; 64, 80. 3136 x 128 33, 24; 44, 41; 59, 76)
-    return K >= 4096 or not _four_waves_per_tile(g, True, c_contig, CONV_SPLIT_ROUND)
+    return K >= 4096 or _cdiv(M, 32) * _cdiv(N, 32) > 2 * CONV_SPLIT_ROUND or not _four_waves_per_tile(g, True, c_contig, CONV_SPLIT_ROUND)
 
 
 def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
