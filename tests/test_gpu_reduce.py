@@ -149,3 +149,20 @@ def test_means_store_the_quotient_from_the_summing_launch():
         print(f'case: {name}', flush=True)
         _, _, fn = check_against_oracle(f, args, rtol=1e-5, atol=0)
         assert len(list(fn._jaxpr_interpreters.values())[0].launches) == launches
+
+
+@pytest.mark.parametrize('shape', [(127, 1728), (128, 1728), (129, 4100), (300, 9408), (128, 30001), (937, 16380)], ids=str)
+def test_unsplit_sums_of_many_rows_take_narrow_blocks(shape, monkeypatch):
+    '''Sums of at least 128 rows by one launch (a kernel gradient's slices): blocks as narrow as leave one per CU.'''
+    import vkjax_amd
+    from vkjax_amd import kernels as K
+    monkeypatch.setattr(K, 'plan_reduce_splits', lambda *args: 1)
+    x = rng.standard_normal(shape).astype(np.float32)
+    f = vkjax_amd.wrap(lambda x: jnp.sum(x, axis=0), frontend='minijax')
+    y = f(x)
+    launch, = list(f._jaxpr_interpreters.values())[0].launches
+    width  = np.frombuffer(launch.params, np.uint32)[7]
+    assert width == 64 or (launch.grid[0] <= 256 and shape[0] >= 128)
+    assert width == 8 or shape[0] < 128 or 2 * launch.grid[0] > 256
+    #a sum of n terms in fp32 is off by at most n roundings of the sum of their magnitudes
+    assert np.all(np.abs(y - x.astype(np.float64).sum(axis=0)) <= shape[0] * 2.0**-24 * np.abs(x).astype(np.float64).sum(axis=0))

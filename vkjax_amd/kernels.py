@@ -348,7 +348,10 @@ REDUCE_BATCH_ENTRY_BYTES    = 56
 TRANSPOSE_BATCH_ENTRY_BYTES = 48
 PACK_BATCH_ENTRY_BYTES      = 56
 BATCH_MAX_BLOCKS         = 4096        #launches of more workgroups than this keep a launch of their own
-REDUCE_NARROW_MAX_BLOCKS = 16          #column sums of at most this many workgroups trade block width for more blocks
+#column sums of up to a workgroup per CU trade the width of a block for more blocks. Sums of R rows alone, at 16 and at 256
+#workgroups: 937 x 1728 7.0, 3.8 us; 256 x 4096 4.6, 2.8; 2000 x 4096 23.4, 6.6; 128 x 9408 3.5, 2.7; 937 x 30000 25.1, 19.1; at 512
+#workgroups 937 x 9408 takes 6.1 instead of 8.3 and 937 x 30000 20.7
+REDUCE_NARROW_MAX_BLOCKS = 256
 TRANSPOSE_BATCH_MAX_BLOCKS = 1024      #... tiled transposes (the kernels of a network, for its backward pass) up to this many
 
 
@@ -1358,7 +1361,6 @@ def _reduce_launch(out: Buffer, inp: Buffer, outer: int, R: int, inner: int, op:
     TI  = min(64, _pow2_at_least(_cdiv(inner, vec)))
     #few blocks with many rows each (the second stage of a split sum): narrower blocks, more of them, more thread rows
     #walking the rows side by side
-    #(up to the number of blocks below which small sums are batched with their neighbours into one launch)
     while TI > 8 and 2 * _cdiv(inner, TI * vec) * nsplit * outer <= REDUCE_NARROW_MAX_BLOCKS and _cdiv(R, nsplit) >= 128:
         TI //= 2
     params = _u32(outer, R, inner, RED[op], ty, r_chunk, nsplit, TI)
