@@ -413,13 +413,13 @@ def _scale_shift_relu_step(params, x):
 
 
 def test_convnet_step_keeps_its_batched_launches():
-    '''The conv-net SGD step at its benchmark size: 23 launches, one of them a batch of column sums
+    '''The conv-net SGD step at its benchmark size: 19 launches, one of them a batch of column sums
     (the sums of the kernel gradients' slices, with the parameter updates, wait for the end of the step and share a
     launch).'''
     from vkjax_amd.jaxpr_interpreter import JaxprInterpreter
     closed = mj.make_jaxpr(W.convnet_train_step)(*W.convnet_train_inputs())
     kernels = [l.kernel for l in JaxprInterpreter(closed, plan_only=True).launches]
-    assert len(kernels) == 23 and sum('batch' in k for k in kernels) == 1, kernels
+    assert len(kernels) == 19 and sum('batch' in k for k in kernels) == 1, kernels
 
 
 def test_scale_relu_backward_and_small_chain_batches_are_planned():

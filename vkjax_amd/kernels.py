@@ -1598,6 +1598,34 @@ def pool(out: Buffer, inp: Buffer, op: str, window, strides, pad_low, dilation) 
                   bytes_moved=4 * (inp.size + out.size))
 
 
+POOL_SUM_STEPS = {'div': 1, 'times': 2, 'select': 3}
+
+
+def pool_sum(out: Buffer, source: EwOperand, source_extent, low, spread, window, strides, dilation, before=None, after=None) -> tp.Optional[Launch]:
+    '''Float sums under windows over y and x of [batch, y, x, channels], out = after(sum(before(source) on a grid of zeros)); None where the kernel
+    does not apply. `source` reads [batch, *source_extent, channels] through its strides; its elements lie `spread` apart behind `low`
+    zeros (a negative number cuts none off: the padding of the windows). `before`, `after`: None, ('div' | 'times', one value), and
+    for `after` ('select', threshold, otherwise, compared array): compared > threshold ? sum : otherwise.'''
+    if len(out.shape) != 4 or tuple(window) not in ((3, 3), (2, 2)) or out.size == 0:
+        return None
+    batch, Ho, Wo, C = out.shape
+    sb, sy, sx, sc = source.strides
+    if (C % 4 or sc != 1 or source.offset % 4 or any(st % 4 or st < 0 for st in (sb, sy, sx)) or source.buffer.size * 4 >= 2**31 or out.size * 4 >= 2**31
+            or min(spread) < 1 or max(*spread, *strides, *dilation, *source_extent, Ho, Wo, abs(low[0]), abs(low[1])) >= 1 << 14):
+        return None
+    words = source.buffer.size - source.offset
+    params = (_u32(out.size, Ho, Wo, C, *source_extent, sb, sy, sx, words) + _i32(-low[0], -low[1]) + _u32(*strides, *dilation, *spread,
+              POOL_SUM_STEPS[before[0]] if before else 0, POOL_SUM_STEPS[after[0]] if after else 0) + _pool_divisions(out.shape))
+    compared = otherwise = None
+    if after is not None and after[0] == 'select':
+        otherwise, compared = after[2:]
+        assert compared.size == out.size
+    buffers = [(out, 0), (source.buffer, source.offset * 4)] + [(b, 0) for b in (before[1] if before else None, after[1] if after else None, compared, otherwise)]
+    spreading = 'pad_nd_' if tuple(spread) != (1, 1) else ''
+    return Launch(f'{spreading}pool2d_sum_{window[0]}x{window[1]}_v4', (_cdiv(out.size // 4, BLOCK), 1, 1), (BLOCK, 1, 1), buffers, params,
+                  bytes_moved=4 * (min(source.buffer.size, batch * int(np.prod(source_extent)) * C) + out.size * (2 if compared is not None else 1)))
+
+
 def select_scatter_add(out: Buffer, source: Buffer, operand: Buffer, selected: Buffer, op: str, window, strides, pad_low) -> tp.List[Launch]:
     '''Gradient of a max (`op` = 'reduce_max': select with ge) or min pooling in two launches: the selected tap
     of every window into `selected` (uint32, source's shape), then the per-element sums; see reduce.hip.'''
