@@ -28,7 +28,7 @@ def sums_args(shapes, seed=0):
 
 
 #one row and one step of 4 thread rows more or less, one vector and one lane's width more or less, split and unsplit sums
-SHAPES = [(2, 2), (2, 3), (3, 4), (4, 5), (5, 8), (16, 10), (17, 64), (63, 100), (64, 256), (65, 257), (127, 260), (1000, 10), (1000, 300), (5000, 1000)]
+SHAPES = [(2, 2), (2, 3), (3, 4), (4, 5), (5, 8), (16, 10), (17, 64), (63, 100), (64, 256), (65, 257), (127, 260), (1000, 10), (1000, 300), (1536, 64), (1537, 64), (5000, 1000)]
 
 
 def test_updates_are_planned():
@@ -110,15 +110,15 @@ def relu_backward(pre, g):
     return m, jnp.sum(m, axis=0)
 
 
-#unsplit sums end at 127 rows; blocks of 256 columns, of 8 vectors or values, and what lies beside them
-RELU_SHAPES = [(2, 2), (3, 4), (17, 10), (63, 64), (64, 65), (127, 100), (127, 256), (128, 256), (129, 257), (1000, 300), (1000, 7), (4099, 8), (700, 1028)]
+#unsplit sums end at 1536 rows; blocks of 256 columns, of 8 vectors or values, and what lies beside them
+RELU_SHAPES = [(2, 2), (3, 4), (17, 10), (63, 64), (64, 65), (127, 100), (127, 256), (128, 256), (129, 257), (1000, 300), (1000, 7), (1536, 40), (1537, 40), (4099, 8), (700, 1028)]
 
 
 def test_relu_backward_with_its_sum_is_planned():
     for shape in RELU_SHAPES:
         x = np.ones(shape, np.float32)
         kernels = kernels_of(relu_backward, (x, x), plan_only=True)
-        assert kernels[0].startswith('relu_backward_v') and len(kernels) == (2 if shape[0] >= 128 else 1), (shape, kernels)
+        assert kernels[0].startswith('relu_backward_v') and len(kernels) == (2 if shape[0] > 1536 else 1), (shape, kernels)
     #values of the mask per column, or sums along the other dimension: the launches stay apart
     other = [lambda x, g: (lambda m: (m, jnp.sum(m, axis=0)))(jnp.where(x > x[0], g, np.float32(0))),
              lambda x, g: (lambda m: (m, jnp.sum(m, axis=1)))(jnp.where(x > np.float32(0), g, np.float32(0)))]
@@ -152,7 +152,7 @@ def test_scaled_sums_keep_every_bit(shape):
     x[0, 0], x[1, 1] = 0, -0.0
     got, expected = (vkjax_amd.wrap(scaled_sums, frontend='minijax', fuse=fuse)(x, c) for fuse in (True, False))
     kernels = kernels_of(scaled_sums, (x, c), plan_only=True)
-    assert shape[0] > 127 or x.size > 4096 or not any(k.startswith('ew_chain') for k in kernels), kernels       #(split sums keep theirs)
+    assert shape[0] > 1536 or x.size > 4096 or not any(k.startswith('ew_chain') for k in kernels), kernels       #(split sums keep theirs)
     for a, b in zip(got, expected):
         assert np.array_equal(a, b)
 

@@ -223,10 +223,16 @@ __device__ __forceinline__ void reduce_cols_body(uint32_t* __restrict__ out, con
     const uint32_t r_lo = sp * P.r_chunk, r_hi = min(P.R, r_lo + P.r_chunk);
     const bool is_arg = MODE >= 3 || (MODE == 2 && P.op >= RED_ARGMAX), is_max = MODE == 3 || (MODE == 2 && P.op == RED_ARGMAX);
     const uint32_t ident = MODE == 0 ? 0u : MODE == 1 ? 0xFF800000u : red_identity(P.op, P.type);
-    uint32_t acc[VEC], best_i[VEC], best_v[VEC];
+    // float sums keep one accumulator per load in flight: a chain of rows a quarter as long, and its rounding errors with it
+    constexpr int CHAINS = MODE == 0 ? 4 : 1;
+    uint32_t acc[CHAINS][VEC], best_i[VEC], best_v[VEC];
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) { acc[j] = ident; best_i[j] = 0xFFFFFFFFu; best_v[j] = 0; }
-    auto take = [&](uint32_t v, uint32_t r, int j) {
+    for (int j = 0; j < VEC; ++j) {
+#pragma unroll
+        for (int q = 0; q < CHAINS; ++q) acc[q][j] = ident;
+        best_i[j] = 0xFFFFFFFFu; best_v[j] = 0;
+    }
+    auto take = [&](uint32_t v, uint32_t r, int j, int q) {
         if constexpr (MODE >= 3) {
             const float x = u2f(v), y = u2f(best_v[j]);
             const bool better = (MODE == 3 ? x > y : x < y) || (x != x && y == y) || best_i[j] == 0xFFFFFFFFu;
@@ -235,7 +241,7 @@ __device__ __forceinline__ void reduce_cols_body(uint32_t* __restrict__ out, con
         } else if (is_arg) {
             if (best_i[j] == 0xFFFFFFFFu || arg_better(is_max, P.type, v, r, best_v[j], best_i[j])) { best_v[j] = v; best_i[j] = r; }
         } else {
-            acc[j] = red_step<MODE>(P.op, P.type, acc[j], v);
+            acc[q % CHAINS][j] = red_step<MODE>(P.op, P.type, acc[q % CHAINS][j], v);
         }
     };
     uint32_t before[VEC], rate = 0;                                   // POST_UPDATE: requested ahead of the rows
@@ -280,7 +286,7 @@ __device__ __forceinline__ void reduce_cols_body(uint32_t* __restrict__ out, con
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
-                for (int j = 0; j < VEC; ++j) take(v[q][j], r + q * TR, j);
+                for (int j = 0; j < VEC; ++j) take(v[q][j], r + q * TR, j, q);
         }
         if (first < r_hi) {
             uint32_t v[4][VEC];
@@ -290,12 +296,16 @@ __device__ __forceinline__ void reduce_cols_body(uint32_t* __restrict__ out, con
             for (int q = 0; q < 4; ++q)
                 if (r + q * TR < r_hi) {
 #pragma unroll
-                    for (int j = 0; j < VEC; ++j) take(v[q][j], r + q * TR, j);
+                    for (int j = 0; j < VEC; ++j) take(v[q][j], r + q * TR, j, q);
                 }
         }
     }
+    if constexpr (CHAINS == 4) {
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) { s_val[tid * VEC + j] = is_arg ? best_v[j] : acc[j]; s_idx[tid * VEC + j] = best_i[j]; }
+        for (int j = 0; j < VEC; ++j) acc[0][j] = f2u((u2f(acc[0][j]) + u2f(acc[1][j])) + (u2f(acc[2][j]) + u2f(acc[3][j])));
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) { s_val[tid * VEC + j] = is_arg ? best_v[j] : acc[0][j]; s_idx[tid * VEC + j] = best_i[j]; }
     __syncthreads();
     for (uint32_t s = TR >> 1; s >= 1; s >>= 1) {
         if (tr < s) {
@@ -444,8 +454,8 @@ REDUCE_KERNELS(fargmin, 4)
 // as two element-wise launches, two more that only feed the column sums, and the two sums: nine
 // passes over arrays of the activation's size. Here every element of ans, g and x is read once, dx
 // written once, and both sums accumulated on the way: four passes. The sums run over exactly the
-// rows, in exactly the order, of reduce_cols_body with the same ReduceParams (per-thread running
-// sums over rows r_lo + tr, + TR, ..., then the same tree over tr in LDS), so sum_m and sum_mx hold
+// rows, in exactly the order, of reduce_cols_body with the same ReduceParams (four running sums
+// per thread over its rows r_lo + tr, + TR, ..., then the same tree over tr in LDS), so sum_m and sum_mx hold
 // the bits the separate launches would have produced, partial results per row range included.
 // SELECT = false: m is g itself (no activation between the scale and what follows; ans, thr and alt unused).
 template <int VEC, bool SELECT, bool SCALED>
@@ -463,9 +473,11 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
     const uint32_t sp = rest % P.nsplit, o = rest / P.nsplit;
     const uint32_t i = (it * TI + ti) * VEC;
     const uint32_t r_lo = sp * P.r_chunk, r_hi = min(P.R, r_lo + P.r_chunk);
-    float acc_m[VEC], acc_x[VEC];
+    float acc_m[4][VEC], acc_x[4][VEC];                               // a chain per load in flight, as in reduce_cols_body
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) { acc_m[j] = 0.f; acc_x[j] = 0.f; }
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) { acc_m[q][j] = 0.f; acc_x[q][j] = 0.f; }
     if (i < P.inner) {                                                // inner is a multiple of VEC
         const float t = SELECT ? thr[0] : 0.f, z = SELECT ? alt[0] : 0.f;
         const uint64_t base = (uint64_t)o * P.R * P.inner + i;
@@ -491,14 +503,14 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
                 if constexpr (SELECT) a[0] = ans[off];
             }
         };
-        auto take = [&](uint32_t row, const float (&a)[VEC], const float (&c)[VEC], const float (&v)[VEC]) {
+        auto take = [&](uint32_t row, const float (&a)[VEC], const float (&c)[VEC], const float (&v)[VEC], int q) {
             float m[VEC], d[VEC];
 #pragma unroll
             for (int j = 0; j < VEC; ++j) {
                 m[j] = SELECT ? (a[j] > t ? c[j] : z) : c[j];
                 d[j] = SCALED ? m[j] * kv[j] : m[j];
-                acc_m[j] = acc_m[j] + m[j];
-                if constexpr (SCALED) acc_x[j] = acc_x[j] + m[j] * v[j];
+                acc_m[q][j] = acc_m[q][j] + m[j];
+                if constexpr (SCALED) acc_x[q][j] = acc_x[q][j] + m[j] * v[j];
             }
             const uint64_t off = base + (uint64_t)row * P.inner;
             if constexpr (VEC == 4) *reinterpret_cast<f32x4*>(dx + off) = f32x4{d[0], d[1], d[2], d[3]};
@@ -512,18 +524,21 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
 #pragma unroll
             for (int q = 0; q < 4; ++q) fetch(r + q * TR, a[q], c[q], v[q]);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) take(r + q * TR, a[q], c[q], v[q]);
+            for (int q = 0; q < 4; ++q) take(r + q * TR, a[q], c[q], v[q], q);
         }
         if (first < r_hi) {
             float a[4][VEC], c[4][VEC], v[4][VEC];
 #pragma unroll
             for (int q = 0; q < 4; ++q) if (r + q * TR < r_hi) fetch(r + q * TR, a[q], c[q], v[q]);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) if (r + q * TR < r_hi) take(r + q * TR, a[q], c[q], v[q]);
+            for (int q = 0; q < 4; ++q) if (r + q * TR < r_hi) take(r + q * TR, a[q], c[q], v[q], q);
         }
     }
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) { s_m[tid * VEC + j] = acc_m[j]; if constexpr (SCALED) s_x[tid * VEC + j] = acc_x[j]; }
+    for (int j = 0; j < VEC; ++j) {
+        s_m[tid * VEC + j] = (acc_m[0][j] + acc_m[1][j]) + (acc_m[2][j] + acc_m[3][j]);
+        if constexpr (SCALED) s_x[tid * VEC + j] = (acc_x[0][j] + acc_x[1][j]) + (acc_x[2][j] + acc_x[3][j]);
+    }
     __syncthreads();
     for (uint32_t s = TR >> 1; s >= 1; s >>= 1) {
         if (tr < s) {

@@ -765,7 +765,7 @@ def _sole_reader_takes(ops, i, C, uses) -> bool:
     #(a launch without a record of its structure counts among the readers of its own result)
     own = sum(b._placeholder is out._placeholder for b in _reads(ops[i]))
     return (i < C and uses[id(out._placeholder)] - own == 1
-            and not any(w._placeholder is source._placeholder for j in range(i + 1, C) for w in _may_write(ops[j])))
+            and not any(w._placeholder is source._placeholder for j in range(i + 1, C) for w in _written(ops[j])))
 
 
 def fuse_reduce_scales(ops, bufferpool, outvars):
@@ -966,10 +966,8 @@ def fuse_relu_backward_epilogues(ops, bufferpool, outvars):
     last_writer: tp.Dict[int, int] = {}
     readers: tp.Dict[int, tp.List[int]] = {}
     for i, op in enumerate(ops):
-        plain = op.chain is None and op.conv is None and op.meta is None
-        for b in ([op.launch.buffers[k][0] for k in op.launch.written] if plain else _may_write(op)):
-            if b is not None:
-                last_writer[pid(b)] = i
+        for b in _written(op):
+            last_writer[pid(b)] = i
         for b in _reads(op):
             readers.setdefault(pid(b), []).append(i)
 
@@ -1602,6 +1600,13 @@ def _may_write(op) -> tp.List:
     if op.chain is not None or op.conv is not None or (op.meta is not None and op.meta[0] in ('iota', 'concat_part', 'threefry', 'random_stream', 'reduce', 'update', 'window_sum', 'relu_backward', 'softmax', 'rows', 'conv_pack')):
         return _writes(op)
     return [b for b, _ in op.launch.buffers if b is not None]
+
+
+def _written(op) -> tp.List:
+    '''Buffers an op changes, by its launch's own record where its structure is not known otherwise.'''
+    if op.chain is None and op.conv is None and op.meta is None:
+        return [op.launch.buffers[k][0] for k in op.launch.written if op.launch.buffers[k][0] is not None]
+    return _may_write(op)
 
 
 def _touched(op) -> tp.List:

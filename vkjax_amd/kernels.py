@@ -1330,6 +1330,25 @@ def _pow2_at_least(x: int) -> int:
     return p
 
 
+def _column_block_width(outer: int, R: int, inner: int, nsplit: int) -> int:
+    '''Threads side by side along the columns (of four columns each, where their number is a multiple of four) of a block of a column
+    reduction. Few blocks with many rows each (the sum of a kernel gradient's slices): narrower blocks, more of them, more
+    thread rows walking the rows side by side.'''
+    vec = 4 if inner % 4 == 0 else 1
+    TI  = min(64, _pow2_at_least(_cdiv(inner, vec)))
+    while TI > 8 and 2 * _cdiv(inner, TI * vec) * nsplit * outer <= REDUCE_NARROW_MAX_BLOCKS and _cdiv(R, nsplit) >= 128:
+        TI //= 2
+    return TI
+
+
+#Columns of at most this many rows are summed by one launch: a second one costs about 2.3 us. Sums of R x columns in two launches, in one:
+#128 x 100 4.6, 2.5 us; 1000 x 10 4.7, 3.2; 1000 x 100 5.1, 3.9; 1536 x 64 5.1, 4.2; 1536 x 1000 5.9, 4.8; 1000 x 9408 9.1, 8.8; 1536 x 5000 8.4, 9.6;
+#1536 x 30000 34, 29; 2000 x 100 5.2, 5.4; 4096 x 100 5.3, 8.7. A number of columns that is no multiple of four is read a word at a time,
+#and up to eight steps of four rows per thread pay: 1000 x 1001 5.7, 3.7; 512 x 4095 (8 steps) 5.7, 3.6; 1000 x 4095 (16) 6.4, 10.0; 1536 x 1001 (12) 6.0, 6.3;
+#512 x 9407 (32) 7.4, 12.7
+REDUCE_UNSPLIT_ROWS, REDUCE_UNSPLIT_STEPS = 1536, 8
+
+
 def plan_reduce_splits(outer: int, R: int, inner: int, op: str, compute_units: int = 256) -> int:
     '''Into how many ranges R is cut so that outer x inner x splits fills the GPU (1 = a single launch).'''
     if op in ('argmax', 'argmin'):
@@ -1337,6 +1356,8 @@ def plan_reduce_splits(outer: int, R: int, inner: int, op: str, compute_units: i
     if inner == 1:
         want  = 32 * compute_units                 #waves
         split = min(_cdiv(want, outer), R // 4096)         #at least 16 KB per wave
+    elif R <= REDUCE_UNSPLIT_ROWS and (inner % 4 == 0 or _cdiv(R, 4 * (BLOCK // _column_block_width(outer, R, inner, 1))) <= REDUCE_UNSPLIT_STEPS):
+        return 1
     else:
         tiles = _cdiv(inner, 256)
         #blocks: several per CU for arrays that stream from HBM for a while; one per CU for smaller ones, whose
@@ -1358,11 +1379,7 @@ def _reduce_launch(out: Buffer, inp: Buffer, outer: int, R: int, inner: int, op:
         return Launch(f'reduce_rows_{mode}_v{vec}', (_cdiv(outer * nsplit, 4), 1, 1), (BLOCK, 1, 1), [(out, 0), (inp, 0)], params,
                       bytes_moved=4 * (outer * R + outer * nsplit)), nsplit
     vec = 4 if inner % 4 == 0 else 1
-    TI  = min(64, _pow2_at_least(_cdiv(inner, vec)))
-    #few blocks with many rows each (the second stage of a split sum): narrower blocks, more of them, more thread rows
-    #walking the rows side by side
-    while TI > 8 and 2 * _cdiv(inner, TI * vec) * nsplit * outer <= REDUCE_NARROW_MAX_BLOCKS and _cdiv(R, nsplit) >= 128:
-        TI //= 2
+    TI  = _column_block_width(outer, R, inner, nsplit)
     params = _u32(outer, R, inner, RED[op], ty, r_chunk, nsplit, TI)
     blocks = _cdiv(inner, TI * vec) * nsplit * outer
     if blocks >= 2**31:
