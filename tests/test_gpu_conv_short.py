@@ -1,0 +1,83 @@
+'''The kernels for dense rows of at most 64 features (conv_short_body in csrc/kernels/conv_split.h): integer-valued data make every product and
+sum exact, and on any data their bits are those of the kernels that compute a tile per block.'''
+import numpy as np
+import pytest
+
+import vkjax_amd
+from vkjax_amd import kernels as K, minijax as mj
+from vkjax_amd.jaxpr_interpreter import JaxprInterpreter
+
+from .common import check_against_oracle
+
+nn, jnp = mj.nn, mj.numpy
+rng = np.random.RandomState(31)
+
+
+def ints(shape, low=-4, high=5):
+    return rng.randint(low, high, size=shape).astype(np.float32)
+
+
+def kernels_of(fn):
+    return [l.kernel for l in list(fn._jaxpr_interpreters.values())[0].launches if l.kernel.startswith('conv_gemm')]
+
+
+#rows around one tile, a wave's second tile (256 blocks of 12 waves: from 98304 on) and none; features that fill a vector, a k tile, not all of
+#two; columns around a block of 32, of 256, and groups of blocks that are not equally wide
+SHAPES = [(33, 4, 17), (31, 64, 256), (32, 36, 32), (65, 60, 257), (1000, 64, 300), (98400, 32, 33), (40, 44, 1100), (8200, 64, 8200)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('m,k,n', SHAPES)
+def test_tile_edges(m, k, n):
+    x, w = ints((m, k)), ints((k, n), -3, 4)
+    with K.overrides(conv_short=True):
+        fn = vkjax_amd.wrap(jnp.dot, frontend='minijax')
+        y  = np.asarray(fn(x, w))
+    assert kernels_of(fn) == ['conv_gemm_split_short']
+    assert np.array_equal(y, x @ w)                            #(sums of at most 64 products of at most 12: exact in any order)
+
+
+@pytest.mark.gpu
+def test_epilogues():
+    x, w, r, a, v = ints((530, 64)), ints((64, 288), -3, 4), ints((530, 288), -50, 50), ints((530, 288)), 2.0 ** ints((288,), -2, 3)
+    bn     = lambda x, w, r, a, v: nn.relu((jnp.dot(x, w) - v) * v + v + r)
+    two    = lambda x, w, r, a, v: (lambda c: (nn.relu(c * v), c))(jnp.dot(x, w) - v)
+    steps  = lambda x, w, r, a, v: (((jnp.dot(x, w) + v) * v - r) * 0.5 + r) * v
+    masked = lambda x, w, r, a, v: jnp.where(a > 0.0, jnp.dot(x, w) + r, 0.0) * v
+    both   = lambda x, w, r, a, v: (lambda m: (m, m * v))(jnp.where(a > 0.0, jnp.dot(x, w), 0.0))
+    for f, name in ((bn, ''), (two, ''), (steps, '_steps'), (masked, ''), (both, '')):
+        with K.overrides(conv_short=True):
+            _, _, fn = check_against_oracle(f, [x, w, r, a, v], exact=True)
+        assert kernels_of(fn) == ['conv_gemm_split_short' + name]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('kind', ('normal', 'small', 'not finite', 'large'))
+def test_the_bits_are_those_of_the_tiled_kernels(kind):
+    '''Sums that are not finite are computed again with fp32 products, as there.'''
+    x, w = rng.standard_normal((999, 60)).astype(np.float32), rng.standard_normal((60, 288)).astype(np.float32)
+    if kind == 'small':
+        x, w = x * np.float32(1e-36), w * np.float32(1e30)
+    if kind == 'not finite':
+        x[0, 3], x[40, 59], x[998, 0], x[500, 7], w[5, 287], w[9, 32] = np.inf, np.nan, -np.inf, 1e37, np.inf, np.nan
+    if kind == 'large':
+        x, w = x * np.float32(1e30), w * np.float32(1e7)
+    def of(**choice):
+        with K.overrides(**choice):
+            return np.asarray(vkjax_amd.wrap(jnp.dot, frontend='minijax')(x, w))
+    assert np.array_equal(of(conv_short=True), of(conv_split='128x64'), equal_nan=True)
+
+
+def test_where_they_apply():
+    '''Plan only.'''
+    def kernels(m, k, n, f=jnp.dot, x=None, **choice):
+        zeros = lambda *s: np.broadcast_to(np.float32(0), s)
+        with K.overrides(**choice):
+            return [l.kernel for l in JaxprInterpreter(mj.make_jaxpr(f)(zeros(*(x or (m, k))), zeros(k, n)), plan_only=True).launches if l.kernel.startswith('conv_gemm')]
+    short = lambda *a, **c: kernels(*a, **c) == ['conv_gemm_split_short']
+    assert short(200704, 64, 256) and short(131072, 64, 128) and short(200704, 40, 256)
+    assert not short(131071, 64, 128) and not short(200704, 32, 256) and not short(200704, 68, 256)                   #results, features
+    assert not short(400000, 64, 64) and not short(200704, 64, 250)                                                    #columns
+    assert not short(200704, 64, 256, conv_split='128x64') and not short(200704, 64, 256, conv_short=False) and not short(200704, 64, 256, conv_split=False)
+    image = lambda stride: lambda x, w: mj.lax.conv_general_dilated(x, w.reshape((1, 1) + w.shape), (stride, stride), 'VALID', dimension_numbers=('NHWC', 'HWIO', 'NHWC'))
+    assert short(0, 64, 256, f=image(1), x=(64, 56, 56, 64)) and not short(0, 64, 256, f=image(2), x=(64, 112, 112, 64))

@@ -94,6 +94,7 @@ struct ConvParams {
     //   split_tiles_m: the first tiles of the grid (tiles_m x tiles_n, row by row), computed by one block each
     //   m_blocks: the slices that the contraction of every tile behind those is cut into, of m_each pairs of k tiles of 32 each, the first
     //     m_extra of them one more
+    //   (kernels named _short: tiles_m tiles of 32 rows, tiles_n groups of m_each blocks of 32 columns; split_tiles_m and m_blocks unused)
 };
 
 // The part of the output a block's tile number refers to: a grid of tiles_m x tiles_n tiles whose first row is

@@ -852,3 +852,206 @@ CONV_SPLIT_KERNEL(conv_gemm_split_128x64, 2, 2, 2, 1, 3, false, false)
 CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch, 2, 2, 2, 1, 3, false, true)
 CONV_SPLIT_KERNEL(conv_gemm_split_128x64_steps, 2, 2, 2, 1, 3, true, false)
 CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_steps, 2, 2, 2, 1, 3, true, true)
+
+// ---- short contractions -------------------------------------------------------------------------------------------------
+// Dense rows [M, K] with K <= 64: a product whose time is that of its result, and of the arrays its epilogue reads. A block holds the packed
+// kernel operand of 256 columns in LDS (96 KB) for good; its 12 waves take 32 rows each, by themselves, keep their parts in registers and walk
+// the columns. No barrier behind the first, nothing loaded twice, and while some waves of a SIMD wait for memory others multiply. The products
+// of a sum and their order are those of the kernels above: the same bits.
+// What bounds it: HBM, at 0.8 to 0.9 of a copy's rate. 200704 x 64 x 256 alone (replays, packing included) 86 -> 72 us, with a residual 113 -> 93 (67 us
+// of memory time; the fp32 tiles and those above load the rows once per 64 or 128 columns, and start and end a block for two k tiles), and with the
+// backward pass of a ReLU, which the fp32 tiles leave to a launch of its own, 189 -> 93. Holding the next tile's rows in registers too, with 8 waves
+// of 256 registers: 71, 97 and 95.
+constexpr int CONV_SHORT_ROWS = 32, CONV_SHORT_COLS = 256, CONV_SHORT_WAVES = 12;
+
+template <bool STEPS>
+__device__ __forceinline__ void conv_short_body(u32x4* __restrict__ Bs, float* __restrict__ Es, float* __restrict__ out, const float* __restrict__ x,
+                                                const float* __restrict__ w, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp, const ConvParams& P,
+                                                const ConvDerived& Dk) {
+    constexpr int COLS = CONV_SHORT_COLS, KSTEPS = 4, WAVES = CONV_SHORT_WAVES, NT = 64 * WAVES;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // blocks that share rows stand behind the same L2
+    const int work = xcd_range((int)blockIdx.x, (int)gridDim.x), walkers = (int)gridDim.x / P.tiles_n;
+    const int walker = work / P.tiles_n, n0 = (work - walker * P.tiles_n) * P.m_each * 32;         // (m_each blocks of 32 columns per block, 8 at most)
+    const int blocks_here = min(P.m_each, (P.N - n0 + 31) / 32);
+    const uint32_t out_bytes = min(P.out_bytes, (uint32_t)P.M * (uint32_t)P.N * 4u), rowb = (uint32_t)P.N * 4u;
+    const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(x, P.x_bytes), w_rsrc = make_rsrc(w, P.w_bytes), o_rsrc = make_rsrc(out, out_bytes);
+    const int nepi = (P.flags >> 8) & 15u, epi_first_full = (int)((P.flags >> 16) & 15u) - 1;
+    const uint32_t slots = (P.flags >> 20) & 31u;
+    const int e_mul = __builtin_popcount(slots & 1u), e_add = __builtin_popcount(slots & 3u), e_max = __builtin_popcount(slots & 15u);
+    const int tap = (int)((P.flags >> 12) & 15u) - 1;
+    const bool masked_form = P.flags & CONV_SPLIT_MASKED;
+    const float* full_ptr = epi.p[0];
+#pragma unroll
+    for (int t = 1; t < CONV_MAX_EPI; ++t) full_ptr = epi_first_full == t ? epi.p[t] : full_ptr;
+    const __amdgpu_buffer_rsrc_t f_rsrc = make_rsrc(full_ptr, slots & 8u ? out_bytes : 0u),
+                                 m_rsrc = make_rsrc(epi.p[1], masked_form ? out_bytes : 0u),
+                                 t_rsrc = make_rsrc(epi.p[CONV_MAX_EPI - 1], tap >= 0 ? out_bytes : 0u);
+
+    auto request_rows = [&](f32x4 (&raw)[KSTEPS][2], int tile) {                     // (rows and features that do not exist: zeros)
+        const int m = tile * CONV_SHORT_ROWS + l32;
+        const uint32_t row = m < P.M ? (uint32_t)(m * P.xs_h) * 4u : CONV_OOB;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int k = (s >> 1) * 32 + 16 * h + 4 * (2 * (s & 1) + half);
+                raw[s][h] = buffer_load_x4(x_rsrc, k < P.K ? row + (uint32_t)k * 4u : CONV_OOB);
+            }
+    };
+    const int tiles = (P.M + CONV_SHORT_ROWS - 1) / CONV_SHORT_ROWS;
+    for (int i = tid; i < blocks_here * KSTEPS * 192; i += NT)
+        Bs[i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (uint32_t)i * 16u, (uint32_t)(n0 / 32 * KSTEPS) * 3072u, 0);
+    conv_split_epilogue_operands<COLS>(Es, epi, Dp, P, Dk, tid, n0);
+    __syncthreads();
+
+    for (int tile = wave * walkers + walker; tile < tiles; tile += WAVES * walkers) {
+        f32x4 raw[KSTEPS][2];
+        request_rows(raw, tile);
+        u32x4 af[KSTEPS][3];
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) af[s][t][q] = conv_split_word(raw[s], t, q);
+        const int m0 = tile * CONV_SHORT_ROWS;
+#pragma nounroll
+        for (int cb = 0; cb < blocks_here; ++cb) {
+            const int col = cb * 32 + l32, n = n0 + col;
+            const uint32_t base = n < P.N ? (uint32_t)((m0 + 4 * half) * P.N + n) * 4u : CONV_OOB;
+            auto at = [&](int v) { return (uint32_t)(8 * (v / 4) + (v % 4)) * rowb; };
+            float y[16], ov[16], av[16];
+            if constexpr (!STEPS) {
+                if (slots & 8u) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) ov[v] = buffer_load_x1_nt(f_rsrc, base, at(v));
+                }
+                if (masked_form) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) av[v] = buffer_load_x1_nt(m_rsrc, base, at(v));
+                }
+            }
+            const u32x4* b_at = Bs + cb * KSTEPS * 192 + lane;
+            f32x16 sum = {};
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                u32x4 bf[3];
+#pragma unroll
+                for (int t = 0; t < 3; ++t) bf[t] = b_at[s * 192 + t * 64];
+                if (s & 1) FENCE();                         // (all of the columns' parts at once: registers would spill)
+#pragma unroll
+                for (int t = 0; t < 6; ++t)
+                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[s][CONV_SPLIT_PA[t]]), __builtin_bit_cast(bf16x8, bf[CONV_SPLIT_PB[t]]), sum, 0, 0, 0);
+            }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) y[v] = sum[v] * (1.f / (CONV_SPLIT_SCALE * CONV_SPLIT_SCALE));
+            // sums that are not finite: again with fp32 products, as above
+            float high = 0.f;
+#pragma unroll
+            for (int v = 0; v < 16; v += 2) high = higher_of(high, y[v], y[v + 1]);
+            if (__builtin_amdgcn_ballot_w64(!(high < __builtin_inff()))) {
+                f32x16 again = {};
+                const int m = m0 + l32;
+                const uint32_t row = m < P.M ? (uint32_t)(m * P.xs_h) * 4u : CONV_OOB;
+#pragma nounroll
+                for (int s = 0; s < KSTEPS; ++s) {
+                    const int k = (s >> 1) * 32 + 4 * (2 * (s & 1) + half);
+                    f32x4 a[2] = {buffer_load_x4(x_rsrc, k < P.K ? row + (uint32_t)k * 4u : CONV_OOB),
+                                  buffer_load_x4(x_rsrc, k + 16 < P.K ? row + (uint32_t)(k + 16) * 4u : CONV_OOB)};
+                    u32x4 b[3];
+#pragma unroll
+                    for (int t = 0; t < 3; ++t) b[t] = b_at[s * 192 + t * 64];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        uint32_t part_e[3];
+#pragma unroll
+                        for (int t = 0; t < 3; ++t) part_e[t] = e & 1 ? b[t][e >> 1] & 0xFFFF0000u : b[t][e >> 1] << 16;
+                        const float value = ((u2f(part_e[2]) + u2f(part_e[1])) + u2f(part_e[0])) * (1.f / CONV_SPLIT_SCALE);
+                        const float bv = part_e[0] == CONV_PACK_RAW << 16 ? u2f(part_e[1] | part_e[2] >> 16) : value;
+                        again = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e >> 2][e & 3], bv, again, 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = __builtin_isfinite(y[v]) ? y[v] : again[v];
+            }
+            auto store = [&](__amdgpu_buffer_rsrc_t to) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) buffer_store_x1(y[v], to, base, at(v));
+            };
+            if constexpr (STEPS) {
+                // (the pointer table is read from the argument block, as above)
+                const float* const* table = reinterpret_cast<const float* const*>(reinterpret_cast<const char*>(__builtin_amdgcn_kernarg_segment_ptr()) + 40);
+#pragma nounroll
+                for (int e = 0; e < nepi; ++e) {
+                    const uint32_t desc = conv_split_step_desc(P, e);
+                    if (desc >> 8 == 3) {
+                        const __amdgpu_buffer_rsrc_t e_rsrc = make_rsrc(table[e], out_bytes);
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) ov[v] = buffer_load_x1_nt(e_rsrc, base, at(v));
+                        conv_epilogue_step(desc & 255u, y, [&](int v) { return ov[v]; });
+                    } else {
+                        const float o = Es[e * COLS + col];
+                        conv_epilogue_step(desc & 255u, y, [&](int) { return o; });
+                    }
+                }
+                store(o_rsrc);
+                continue;
+            }
+            if (masked_form) {
+                const float limit = Es[3 * COLS + col], otherwise = Es[4 * COLS + col], o = Es[2 * COLS + col];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    if (slots & 8u) y[v] = y[v] + ov[v];
+                    y[v] = av[v] > limit ? y[v] : otherwise;
+                }
+                if (tap >= 0) store(t_rsrc);
+                if (slots & 2u) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) y[v] = y[v] * o;
+                }
+                store(o_rsrc);
+                continue;
+            }
+            if (tap == 0) store(t_rsrc);
+            if (slots & 1u) {
+                const float o = Es[col];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = y[v] - o;
+                if (tap == 1) store(t_rsrc);
+            }
+            if (slots & 2u) {
+                const float o = Es[e_mul * COLS + col];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = y[v] * o;
+            }
+            if (slots & 4u) {
+                const float o = Es[e_add * COLS + col];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = y[v] + o;
+            }
+            if (slots & 8u) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = y[v] + ov[v];
+            }
+            if (slots & 16u) {
+                const float o = Es[e_max * COLS + col];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) y[v] = (y[v] > o || y[v] != y[v]) ? y[v] : o;
+            }
+            store(o_rsrc);
+        }
+    }
+}
+
+#define CONV_SHORT_KERNEL(name, STEPS)                                                                                       \
+    extern "C" __global__ __launch_bounds__(64 * CONV_SHORT_WAVES) __attribute__((amdgpu_waves_per_eu(CONV_SHORT_WAVES / 4, CONV_SHORT_WAVES / 4))) void name( \
+        float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                                   \
+        float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) { \
+        __shared__ __attribute__((aligned(16))) u32x4 Bs[CONV_SHORT_COLS / 32 * 4 * 192];                                    \
+        __shared__ float Es[CONV_MAX_EPI * CONV_SHORT_COLS];                                                                 \
+        conv_short_body<STEPS>(Bs, Es, out, x, w, epi, dp, P, D);                                                            \
+    }
+CONV_SHORT_KERNEL(conv_gemm_split_short, false)
+CONV_SHORT_KERNEL(conv_gemm_split_short_steps, true)

@@ -51,6 +51,7 @@ class _Choices:
         conv_split=None,                 #the kernels on the bf16 matrix cores: None = where they pay, False = never, True or a tile's name = wherever they apply
         conv_split_slices=None,          #blocks that share a tile behind the whole rounds (None: by the estimate)
         conv_patch=None,                 #the bf16 kernels that hold a patch of the input in LDS: None = wherever they apply (a pinned conv_split: never), True = wherever they apply, False = never
+        conv_short=None,                 #the bf16 kernels for dense rows of at most 64 features: None = where they pay (a pinned conv_split: never), True = wherever they apply, False = never
         wgrad_split=None,                #kernel gradients on the bf16 matrix cores: None = where they pay, False = never, a tile's name = wherever it applies
         wgrad_slices=None,               #slices of a kernel gradient's contraction (None: by the estimate)
         conv_k_splits=None,              #slices a contraction is cut into where that applies (None: by the heuristic, 1: never)
@@ -1116,8 +1117,8 @@ CONV_SPLIT_TILES = {'128x128': (128, 128, 1.15, 1.15), '128x64': (128, 64, 0.65,
 #x 512 x 512 80.1, 78.1 in 200 blocks, 16 x 7 x 7 x 512 x 512 73.9 in 56 blocks, 41.8 in 112, 29.2 in 224; 119, 66, 41.)
 CONV_PATCH_STEP, CONV_PATCH_START, CONV_PATCH_SLICE = {'128x128': 0.88, '128x64': 0.5}, 8, 16
 #Products below these stay with the fp32 kernels. Rows: packing the kernel operand costs what about 250 rows' products cost,
-#and one launch. Contraction: with two k tiles of 32 a block is all start-up and stores (200704 x 64 x 256 with residual:
-#101 us here, 66 there, where a block walks several tiles; 50176 x 128 x 512: 59 against 61). Operations: start and end of two launches. A
+#and one launch. Contraction: with two k tiles of 32 a block is all start-up and stores (12544 x 64 x 256 with residual 29
+#us here, 25 there; 200704 x 64 x 256 115, 113, and 93 where a block holds the kernel operand, _conv_short_pays; 50176 x 128 x 512: 59 against 61). Operations: start and end of two launches. A
 #product alone is slower up to 2 GFLOP (8188 x 880 x 98, 1.4: 28.9 against 23.9; 20000 x 512 x 64, 1.3: 23.4, 21.6; 8192 x 512 x 256, 2.1: 23.0,
 #23.4), by the packing launch; in a network, where several layers' weights are packed by one launch, it is faster from 1 on, more so where
 #the backward pass of a ReLU is its epilogue (ResNet-50 with the line at 1, at 1.5 and at 2: batch 16 1566, 1583, 1623 us, batch 8 at 200 x 200 1092, 1119,
@@ -1138,6 +1139,7 @@ class ConvSplit(tp.NamedTuple):
     partial: tp.Optional[Buffer] = None
     arrivals: tp.Optional[Buffer] = None
     patch: bool = False               #by the kernels that hold a patch of the input in LDS (conv_patch_applies)
+    short: bool = False               #by the kernels that hold the kernel operand in LDS (conv_short_applies)
 
 
 def conv_split_tiles(split: ConvSplit, g: ConvGeometry) -> tp.Tuple[int, int]:
@@ -1163,6 +1165,21 @@ def conv_patch_applies(g: ConvGeometry) -> bool:
     return ((g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, g.LH, g.LW) == (3, 3) + (1,) * 8
             and g.Ho == g.H and g.Wo == g.W and g.W <= 63 and g.Cin % 32 == 0 and g.xs[2] >= g.Cin
             and g.xs[1] == g.W * g.xs[2] and g.xs[0] == g.H * g.xs[1])
+
+
+def conv_short_applies(g: ConvGeometry, c_contig: bool) -> bool:
+    '''Dense rows of at most 64 features (a flattened geometry), the result's rows dense too.'''
+    return (c_contig and 0 < g.K <= 64 and (g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.LH, g.LW) == (1,) * 4 + (0,) * 2 + (1,) * 2
+            and g.batch == 1 and g.Wo == 1 and g.Ho == g.H)
+
+
+def _conv_short_pays(g: ConvGeometry) -> bool:
+    '''Where those kernels are faster than any other.'''
+    #(times of replays of a product with a residual behind its ReLU in microseconds, packing included, fp32 and here.) Columns: half lines of a width
+    #that is no multiple of 32 are requested twice (100000 x 48 x 300 92, 90, but 43000 x 64 x 300 49, 54; 1000000 x 64 x 65 in 128 x 128 tiles 244, 307), and
+    #below 96 there is little to walk (200704 x 64 x 64 46, 49). Features: 200704 x 40 x 256 112, 92, but without an epilogue 200704 x 32 x 256 60, 63.
+    #Results: 11.5 M 60000 x 64 x 192 41.5, 42.3; 12.8 M 100352 x 64 x 128 44, 46, 50176 x 64 x 256 43, 41; 19 M 150000 x 64 x 128 58, 55, 200704 x 64 x 96 78, 56
+    return g.N % 32 == 0 and g.N >= 96 and g.K > 32 and g.M * g.N >= 1 << 24
 
 
 def _conv_patch_pays(g: ConvGeometry, c_contig: bool) -> bool:
@@ -1210,6 +1227,9 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
     #(pinned to other kernels of this family, a product is theirs)
     wanted = CHOICES.conv_split is None and CHOICES.conv_split_slices is None if CHOICES.conv_patch is None else CHOICES.conv_patch
     patch  = bool(wanted) and conv_patch_applies(g)
+    wanted = CHOICES.conv_split is None and CHOICES.conv_split_slices is None if CHOICES.conv_short is None else CHOICES.conv_short
+    if wanted and conv_short_applies(g, c_contig) and (CHOICES.conv_short or _conv_short_pays(g)):
+        return ConvSplit('128x64', _cdiv(M, 128) * _cdiv(N, 64), 1, short=True)
     if not (CHOICES.conv_split or CHOICES.conv_split_slices) and not (_conv_patch_pays if patch else _conv_split_pays)(g, c_contig):
         return None
     #The whole tiles are dealt out in rounds of one per CU; the contraction of those of the last, incomplete round (or of all,
@@ -1281,10 +1301,18 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
     (tiles_m, tiles_n), kpairs = conv_split_tiles(split, g), g.Cin // 32 if split.patch else _cdiv(K, 64)
     assert not split.patch or conv_patch_applies(g)
     shared = tiles_m * tiles_n - split.whole
+    blocks, threads, kernel = split.whole + shared * split.slices, 256, f'conv_gemm_split_{split.tile}' + ('_patch' if split.patch else '')
+    if split.short:
+        assert conv_short_applies(g, c_contig) and flat_rows
+        #one block per CU for at most 256 columns, its waves walk the tiles of 32 rows
+        tiles_m, tiles_n = _cdiv(M, 32), _cdiv(N, 256)
+        column_blocks    = _cdiv(_cdiv(N, 32), tiles_n)
+        tiles_n          = _cdiv(_cdiv(N, 32), column_blocks)
+        blocks, threads, kernel, shared = max(1, min(CONV_SPLIT_ROUND // tiles_n, tiles_m)) * tiles_n, 768, 'conv_gemm_split_short', 0
     params = (_i32(M, N, K, g.Ho, g.Wo, g.H, g.W, g.Cin, g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, *g.xs[:3], tiles_m, tiles_n)
               + _u32(flags, *descs, (lhs.size - lhs_offset) * 4, packed.size * 4, (out.size - out_offset) * 4,
                      *_magic_division(g.Ho * g.Wo), *_magic_division(g.Wo))
-              + _i32(g.LH, g.LW, g.xs[3], *g.ws, *g.os, split.whole, 0, split.slices, kpairs // split.slices, kpairs % split.slices))
+              + _i32(g.LH, g.LW, g.xs[3], *g.ws, *g.os, split.whole, 0, split.slices, column_blocks if split.short else kpairs // split.slices, kpairs % split.slices))
     derived_ptrs, derived_desc = _conv_derived(epilogue, N)
     operand_slots = _pad([(e.operand, 0) for e in epilogue], CONV_MAX_EPI, (None, 0))
     nbytes = 4 * (lhs.size + packed.size + out.size) + sum(4 * e.operand.size for e in epilogue if e.operand is not None)
@@ -1292,7 +1320,7 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
         operand_slots[-1] = (taps[0][1], 0)
         nbytes += 4 * taps[0][1].size
     scratch = [(split.partial, 0), (split.arrivals, 0)] if shared else [(None, 0), (None, 0)]
-    return Launch(f'conv_gemm_split_{split.tile}' + ('_patch' if split.patch else '') + ('_steps' if steps else ''), (split.whole + shared * split.slices, 1, 1), (256, 1, 1),
+    return Launch(kernel + ('_steps' if steps else ''), (blocks, 1, 1), (threads, 1, 1),
                   [(out, out_offset * 4), (lhs, lhs_offset * 4), (packed, 0)] + scratch + operand_slots + derived_ptrs,
                   params + derived_desc, bytes_moved=nbytes, flops=2 * M * N * K,
                   written=(0, 3, 4) if shared else (0,), scratch=(3, 4) if shared else ())
