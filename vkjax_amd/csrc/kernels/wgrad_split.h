@@ -6,7 +6,7 @@
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-// Block = 2 x 2 waves, each with TM x TN tiles of 32 x 32; k tile: 32 pixels. The matrix cores want eight consecutive pixels of one
+// Block = 2 x 2 waves (twice as many where PAIR, below), each with TM x TN tiles of 32 x 32; k tile: 32 pixels. The matrix cores want eight consecutive pixels of one
 // column per lane where memory has consecutive columns of one pixel, so a thread loads eight pixels of four columns (16 bytes each)
 // and finds every column's eight numbers in its own registers: taken apart they are 16 bytes of LDS per column and part,
 // [part][octet of pixels][column]. Columns lie by their number modulo 4 first (what 32 threads of a wave write at once is contiguous),
@@ -28,19 +28,32 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // matter to, and through their columns, costs as much for the columns' largest numbers and far more where it finds some: sums of nothing but
 // zeros are everywhere behind a ReLU, ResNet-50's training step took 17.7 ms instead of 12.6.)
 constexpr float WGRAD_SCALE = 0x1p24f;
-template <int TM, int TN, bool VEC_A, bool VEC_B>
+//
+// PAIR: a block is two such groups of four waves, each with LDS of its own and half of the slice's k tiles; they take turns, the one
+// takes its tile apart while the other one multiplies, and add their sums up in LDS in the end: half as many partial results are written, and
+// read by the sum behind, as by two blocks per CU that each have a slice. ResNet-50's training step at batch 64: 12.59 -> 12.40 ms, the
+// launch that adds the partial results 288 -> 185 us.
+template <int TM, int TN, bool VEC_A, bool VEC_B, bool PAIR>
 __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2* __restrict__ table, float* __restrict__ out,
                                                  const float* __restrict__ x, const float* __restrict__ g, const WgradParams& P, const WgradSplitParams& Q) {
     constexpr int BM = 64 * TM, BN = 64 * TN, BK = 32;
+    const int tid = threadIdx.x, lane = tid & 63, wave_of_block = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = wave_of_block & 3, group = PAIR ? wave_of_block >> 2 : 0;
+    float* const exchange = reinterpret_cast<float*>(lds);
+    lds += group * 12 * (BM + BN);
+    table += group * 4 * 32;
     u32x4 *const As = lds, *const Bs = lds + 12 * BM;             // [3 parts][4 octets][columns]
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1, l32 = lane & 31, half = lane >> 5;
     // the blocks of one slice read the same pixels: neighbours on one XCD
     const int work = xcd_range((int)blockIdx.x, (int)gridDim.x), tiles = Q.tiles_m * Q.tiles_n;
     const int slice = work / tiles, tile = work - slice * tiles, tile_m = tile / Q.tiles_n, tile_n = tile - tile_m * Q.tiles_n;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
-    const int kbeg = slice * P.pix_per_split, kend = min(P.pixels, kbeg + P.pix_per_split);
-    const int nk = kbeg < kend ? (kend - kbeg + BK - 1) / BK : 0;
+    int kbeg = slice * P.pix_per_split, kend = min(P.pixels, kbeg + P.pix_per_split), nk = kbeg < kend ? (kend - kbeg + BK - 1) / BK : 0, turns = nk;
+    if constexpr (PAIR) {                                         // the first group has the odd k tile
+        turns = (nk + 1) / 2;
+        if (group == 0) { kend = min(kend, kbeg + turns * BK); nk = turns; }
+        else            { kbeg += turns * BK; nk -= turns; }
+    }
     const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(x, P.x_bytes), g_rsrc = make_rsrc(g, P.g_bytes);
     const bool flat = Q.flat != 0;
 
@@ -172,9 +185,11 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
     f32x16 acc[TM][TN] = {};
     constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 0, 1, 1, 2, 0};
     if (nk > 0) load_tile(0);
-    for (int kt = 0; kt < nk; ++kt) {
-        park_tile(kt & 1);
+    if (PAIR && group == 1) __syncthreads();
+    for (int kt = 0; kt < turns; ++kt) {
+        if (!PAIR || kt < nk) park_tile(kt & 1);
         __syncthreads();
+        if (PAIR && kt >= nk) { __syncthreads(); continue; }
         if (kt + 1 < nk) load_tile(kt + 1);
         const float sign = kt & 1 ? -1.f / (WGRAD_SCALE * WGRAD_SCALE) : 1.f / (WGRAD_SCALE * WGRAD_SCALE);
         bf16x8 af[TM][2][3];
@@ -204,6 +219,7 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
         }
         __syncthreads();
     }
+    if (PAIR && group == 0) __syncthreads();
 
     // Sums that are not finite (an operand that is infinite, not a number, or beyond 2^104; a sum beyond 2^80): again, with fp32 products. The
     // finite ones beside them stay as they are.
@@ -284,8 +300,8 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
         }
     }
     float* const result = out + (size_t)slice * P.M * P.N;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
+    auto store_row_of_tiles = [&](auto i_) {
+        constexpr int i = decltype(i_)::value;
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const int col = n0 + (wn * TN + j) * 32 + 4 * (l32 & 7) + (l32 >> 3);
@@ -295,17 +311,45 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
                 if (row < P.M && col < P.N) result[(size_t)row * P.N + col] = acc[i][j][v];
             }
         }
+    };
+    if constexpr (PAIR) {
+        // group i finishes row i of its waves' tiles, with the other group's sums of it
+        static_assert(TM == 2, "a row of tiles for each group");
+        auto hand_over = [&](auto i_) {
+            constexpr int i = decltype(i_)::value;
+            float* const to = exchange + i * (4 * TN * 16 * 64) + wave * (TN * 16 * 64) + lane;
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) to[(j * 16 + v) * 64] = acc[i][j][v];
+        };
+        auto finish = [&](auto i_) {
+            constexpr int i = decltype(i_)::value;
+            const float* const from = exchange + i * (4 * TN * 16 * 64) + wave * (TN * 16 * 64) + lane;
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] += from[(j * 16 + v) * 64];
+            store_row_of_tiles(i_);
+        };
+        if (group == 0) hand_over(std::integral_constant<int, 1>{}); else hand_over(std::integral_constant<int, 0>{});
+        __syncthreads();
+        if (group == 0) finish(std::integral_constant<int, 0>{}); else finish(std::integral_constant<int, 1>{});
+    } else {
+        store_row_of_tiles(std::integral_constant<int, 0>{});
+        if constexpr (TM == 2) store_row_of_tiles(std::integral_constant<int, 1>{});
+    }
 }
 
-#define WGRAD_SPLIT_KERNEL(name, TM, TN, VA, VB, WPE)                                                                         \
-    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void name(                         \
+#define WGRAD_SPLIT_KERNEL(name, TM, TN, VA, VB, WPE, PAIR)                                                                         \
+    extern "C" __global__ __launch_bounds__(PAIR ? 512 : 256) __attribute__((amdgpu_waves_per_eu(WPE))) void name(                         \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ g, WgradParams P, WgradSplitParams Q) { \
-        __shared__ __attribute__((aligned(16))) u32x4 lds[12 * 64 * (TM + TN)];                                               \
-        __shared__ __attribute__((aligned(16))) u32x2 table[4 * 32];                                                          \
-        wgrad_split_body<TM, TN, VA, VB>(lds, table, out, x, g, P, Q);                                                        \
+        __shared__ __attribute__((aligned(16))) u32x4 lds[(PAIR ? 2 : 1) * 12 * 64 * (TM + TN)];                                               \
+        __shared__ __attribute__((aligned(16))) u32x2 table[(PAIR ? 2 : 1) * 4 * 32];                                                          \
+        wgrad_split_body<TM, TN, VA, VB, PAIR>(lds, table, out, x, g, P, Q);                                                        \
     }
-WGRAD_SPLIT_KERNEL(wgrad_split_128x128_aa, 2, 2, true, true, 2)
-WGRAD_SPLIT_KERNEL(wgrad_split_128x64_aa, 2, 1, true, true, 3)
-WGRAD_SPLIT_KERNEL(wgrad_split_64x128_aa, 1, 2, true, true, 3)
-WGRAD_SPLIT_KERNEL(wgrad_split_64x64_aa, 1, 1, true, true, 4)
-WGRAD_SPLIT_KERNEL(wgrad_split_64x64_sa, 1, 1, false, true, 4)
+WGRAD_SPLIT_KERNEL(wgrad_split_128x128_aa, 2, 2, true, true, 2, true)
+WGRAD_SPLIT_KERNEL(wgrad_split_128x64_aa, 2, 1, true, true, 3, false)
+WGRAD_SPLIT_KERNEL(wgrad_split_64x128_aa, 1, 2, true, true, 3, false)
+WGRAD_SPLIT_KERNEL(wgrad_split_64x64_aa, 1, 1, true, true, 4, false)
+WGRAD_SPLIT_KERNEL(wgrad_split_64x64_sa, 1, 1, false, true, 4, false)

@@ -543,9 +543,10 @@ def choose_wgrad_splits(g: WgradGeometry, compute_units: int = 256) -> int:
     return max(1, min(want, g.pixels // 128, 1024))
 
 
-#Tiles of the kernel gradients on the bf16 matrix cores (csrc/kernels/wgrad_split.h): (BM, BN, blocks a CU holds, microseconds of such
+#Tiles of the kernel gradients on the bf16 matrix cores (csrc/kernels/wgrad_split.h): (BM, BN, blocks a CU holds (one of 128 x 128: of
+#two groups of four waves, the others have one), microseconds of such
 #a CU per block and k tile of 32 pixels, measured on ResNet-50's layers at batch 64, loads of X it is built for: 16 bytes / words)
-WGRAD_SPLIT_TILES = {'128x128': (128, 128, 2, 1.55, 'a'), '128x64': (128, 64, 3, 0.95, 'a'), '64x128': (64, 128, 3, 0.95, 'a'), '64x64': (64, 64, 4, 0.57, 'as')}
+WGRAD_SPLIT_TILES = {'128x128': (128, 128, 1, 1.55, 'a'), '128x64': (128, 64, 3, 0.95, 'a'), '64x128': (64, 128, 3, 0.95, 'a'), '64x64': (64, 64, 4, 0.57, 'as')}
 #Below this many operations the fp32 kernels are as fast: 2000 x 1024 x 512 (2.1 GFLOP) takes 28 us there and 22 here, 1000 x 784 x 300
 #(0.5) 12.6 and 12.8, 3x3 on 4 x 14 x 14 x 256 (0.9) 18.4 and 18.8.
 WGRAD_SPLIT_MIN_FLOPS = 1.5e9
@@ -592,7 +593,7 @@ def wgrad_plan(g: WgradGeometry, compute_units: int = 256) -> WgradPlan:
             per    = _cdiv(ktiles, splits)
             splits = _cdiv(ktiles, per)
             each   = _cdiv(tiles * splits, compute_units)
-            alone  = 0.3 * max(0, resident - each) / (resident - 1)
+            alone  = 0.3 * max(0, resident - each) / max(1, resident - 1)
             time   = each * per * step * (1 + alone) + 4 + (3 + splits * g.M * g.N * 8 / 8e6 if splits > 1 else 0)
             if best is None or time < best[0]:
                 best = (time, WgradPlan(tile, splits))
@@ -621,7 +622,7 @@ def wgrad_gemm(out: Buffer, x: Buffer, cot: Buffer, g: WgradGeometry, splits: in
     if tile is not None:
         bm, bn = WGRAD_SPLIT_TILES[tile][:2]
         tiles_m, tiles_n = _cdiv(g.M, bm), _cdiv(g.N, bn)
-        return Launch(f'wgrad_split_{tile}_{loads}', (tiles_m * tiles_n * splits, 1, 1), (256, 1, 1), [(out, 0), (x, 0), (cot, 0)],
+        return Launch(f'wgrad_split_{tile}_{loads}', (tiles_m * tiles_n * splits, 1, 1), (512 if tile == '128x128' else 256, 1, 1), [(out, 0), (x, 0), (cot, 0)],
                       params + _i32(tiles_m, tiles_n, _wgrad_flat(g)), **work)
     return Launch(f'wgrad_gemm_64x64_{loads}', (_cdiv(g.N, 64), _cdiv(g.M, 64), splits), (256, 1, 1), [(out, 0), (x, 0), (cot, 0)], params, **work)
 
