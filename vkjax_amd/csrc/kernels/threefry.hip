@@ -263,4 +263,8 @@ TF_STREAM_KERNEL(threefry2x32_stream_pairs_v1, 1, TF_PAIRS)
 // the steps are exactly jax.random.uniform's chain, every step with an operand (see threefry_uniform_steps)
 TF_STREAM_KERNEL(threefry2x32_stream_uniform_v4, 4, TF_HALVES, true)
 TF_STREAM_KERNEL(threefry2x32_stream_xor_uniform_v4, 4, TF_XOR, true)
+// where the blocks are no multiple of four. Draws of an odd number of words were thirteen launches before the host saw one in them: 4095 x 8191 uniform
+// numbers 710 -> 54 us a replay, 1001 x 1001 64 -> 22; bound by the integer ALUs as the others are (4096 x 8191, four blocks per thread: 50).
+TF_STREAM_KERNEL(threefry2x32_stream_v1_uniform, 1, TF_HALVES, true)
+TF_STREAM_KERNEL(threefry2x32_stream_xor_v1_uniform, 1, TF_XOR, true)
 

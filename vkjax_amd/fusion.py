@@ -1463,7 +1463,8 @@ def fuse_random_streams(ops, bufferpool, outvars):
     shift / or / bitcast / sub / mul / add / max). The fused kernel generates the counters in
     registers and applies the chain before its only store, so of the iota, the two slices, the
     block function, the two concatenate copies and the chain only one write of the result remains.
-    The arithmetic per element is unchanged.'''
+    The arithmetic per element is unchanged. A draw of an odd number of words n = 2h - 1 has c = concatenate(iota(n), 0) and drops
+    the last of the bits, which the kernel does itself.'''
     from .ops import Op
     uses = _use_counts(ops, bufferpool, outvars)
     pid  = lambda b: id(b._placeholder)
@@ -1482,6 +1483,16 @@ def fuse_random_streams(ops, bufferpool, outvars):
             for b, _ in op.launch.buffers[:1]:       #kernels write their first argument
                 if b is not None:
                     writers[pid(b)].append(i)
+    def padded(ws, counters) -> bool:
+        '''Whether the two launches at `ws` write an iota of 2h - 1 words and a zero behind it.'''
+        if len(ws) != 2 or len(counters.shape) != 1 or counters.dtype != 'uint32' or any(ops[i].meta is None or ops[i].meta[0] != 'concat_part' for i in ws):
+            return False
+        (_, _, words, d0, at0, *_), (_, _, pad, d1, at1, *_) = sorted((ops[i].meta for i in ws), key=lambda m: m[4])
+        source = writers.get(pid(words), [])
+        return ((d0, at0, d1, at1) == (0, 0, 0, words.size) and pad.size == 1 and counters.size == words.size + 1 and words.size > 1 and words.dtype == 'uint32'
+                and pad.dtype == 'uint32' and pad.constant_value is not None and int(np.asarray(pad.constant_value).reshape(())) == 0 and not writers.get(pid(pad))
+                and len(source) == 1 and ops[source[0]].meta is not None and ops[source[0]].meta[0] == 'iota' and len(words.shape) == 1)
+
     removed = set()
     replacement = {}
     for ti, T in enumerate(ops):
@@ -1502,11 +1513,19 @@ def fuse_random_streams(ops, bufferpool, outvars):
                 break
             S  = C.chain.first.buffer
             ws = writers.get(pid(S), [])
+            if padded(ws, S):
+                sources.append((w[0], C.chain.first.offset, ws, S))
+                continue
             if len(ws) != 1 or ops[ws[0]].meta is None or ops[ws[0]].meta[0] != 'iota' or len(S.shape) != 1 or S.dtype != 'uint32':
                 break
             sources.append((w[0], C.chain.first.offset, ws[0], S))
         if len(sources) != 2:
             continue
+        odd = [isinstance(ws, list) for _, _, ws, _ in sources]
+        if any(odd) and not (all(odd) and sources[0][3]._placeholder is sources[1][3]._placeholder and uses[pid(sources[0][3])] == 2
+                             and sources[0][3].size == 2 * h and (sources[0][1], sources[1][1]) == (0, h)):
+            continue
+        count = 2 * h - 1 if any(odd) else 2 * h
         #results: concatenated in order into one array
         if uses[pid(aa)] != 1 or uses[pid(ab)] != 1:
             continue
@@ -1532,13 +1551,15 @@ def fuse_random_streams(ops, bufferpool, outvars):
                     n  = 1
                     for d in (ch.shape if ch is not None else ()):
                         n *= d
-                    if (ch is not None and ch.first.buffer._placeholder is AC._placeholder and ch.first.offset == 0 and n == 2 * h
+                    if (ch is not None and ch.first.buffer._placeholder is AC._placeholder and ch.first.offset == 0 and n == count
                             and tuple(ch.first.strides) == K.row_major_strides(ch.shape) and len(ch.steps) <= K.TF_MAX_STEPS
                             and all(st.op not in _SELECTS and st.op != EW['NOP'] and
                                     (st.operand is None or (st.operand.buffer.size == 1 and st.operand.offset == 0)) for st in ch.steps)):
                         chain_pos = i
                     break
-        members = [sources[0][0], sources[1][0], ti] + cats + ([chain_pos] if chain_pos is not None else [])
+        if any(odd) and chain_pos is None:
+            continue
+        members = [sources[0][0], sources[1][0], ti] + cats + ([chain_pos] if chain_pos is not None else []) + (sources[0][2] if any(odd) else [])
         if removed & set(members):
             continue
         last  = max(members)
@@ -1558,8 +1579,8 @@ def fuse_random_streams(ops, bufferpool, outvars):
             else:
                 keys.append((kb, 0))
         fused = Op(_label(*[ops[i] for i in sorted(members)]),
-                   launch=K.threefry_stream(out, keys[0], keys[1], h, sources[0][1], sources[1][1], steps),
-                   meta=('random_stream', out, 'halves', keys[0], keys[1], h, sources[0][1], sources[1][1], 2 * h, steps))
+                   launch=K.threefry_stream(out, keys[0], keys[1], h, sources[0][1], sources[1][1], steps, n=count),
+                   meta=('random_stream', out, 'halves', keys[0], keys[1], h, sources[0][1], sources[1][1], count, steps))
         fused.index = ops[last].index
         for b in [keys[0][0], keys[1][0]] + [st.operand.buffer for st in steps if st.operand is not None]:
             b.accesses.append(fused.index)
@@ -1567,6 +1588,10 @@ def fuse_random_streams(ops, bufferpool, outvars):
             b._placeholder.elided = True
         removed |= set(members)
         replacement[last] = fused
+        if any(odd):
+            sources[0][3]._placeholder.elided = True
+            part    = next(ops[i].meta[2] for i in sources[0][2] if ops[i].meta[2].size != 1)
+            sources = [(None, 0, writers[pid(part)][0], part)]
         #an iota nobody reads any more goes too
         for _, _, si, S in sources:
             uses[pid(S)] -= 1

@@ -489,13 +489,14 @@ def threefry_stream(out: Buffer, key0: tp.Tuple[Buffer, int], key1: tp.Tuple[Buf
                   *_pad([s.imm for s in steps], TF_MAX_STEPS), n,
                   *(({'halves': 1, 'pairs': 3}[key_split.layout], *key_split[1:5], *key_split.words) if key_split else (0,) * 7))
     kernel = {'halves': 'threefry2x32_stream', 'xor': 'threefry2x32_stream_xor', 'pairs': 'threefry2x32_stream_pairs'}[layout]
-    #jax.random.uniform's chain has a kernel of its own with the steps compiled in
-    if vec == 4 and [s.op for s in steps] == _UNIFORM_CHAIN_OPS and flags == [1, 1, 1, 1, 1, 3] and all(s.imm == 0 for s in steps):
-        kernel += '_uniform'
+    kernel += f'_v{vec}'
+    #jax.random.uniform's chain has kernels of its own with the steps compiled in
+    if [s.op for s in steps] == _UNIFORM_CHAIN_OPS and flags == [1, 1, 1, 1, 1, 3] and all(s.imm == 0 for s in steps) and layout != 'pairs':
+        kernel = kernel.replace('_v4', '_uniform_v4') if vec == 4 else kernel + '_uniform'
     blocks = _cdiv(_cdiv(h, vec), BLOCK)
     if key_split and layout != 'pairs':
         blocks = min(blocks, KEY_SPLIT_BLOCKS)
-    return Launch(f'{kernel}_v{vec}', (blocks, 1, 1), (BLOCK, 1, 1),
+    return Launch(kernel, (blocks, 1, 1), (BLOCK, 1, 1),
                   [(out, 0), (key0[0], key0[1] * 4), (key1[0], key1[1] * 4)] + _pad(buffers, TF_MAX_STEPS, (None, 0)), params,
                   bytes_moved=4 * (h if layout == 'xor' else n))
 
