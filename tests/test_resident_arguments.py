@@ -1,0 +1,105 @@
+'''What stays in HBM between calls: an evaluation computes with the arguments of its own call, whatever was held there before
+(CPU: the evaluation is a stand-in that keeps what it is handed; on the GPU, the results).'''
+import numpy as np
+import pytest
+
+import vkjax_amd
+from vkjax_amd import minijax as mj
+from vkjax_amd.jaxpr_interpreter import JaxprInterpreter
+
+
+def frozen(x):
+    x = x.copy()
+    x.flags.writeable = False
+    return x
+
+
+class Sequence:
+    '''Keeps what is uploaded, slot by slot, and notes what every evaluation computes with.'''
+    def __init__(self, n_inputs):
+        self.n_slots, self.hbm, self.computed_with = n_inputs + 1, [None] * n_inputs, []
+
+    def eval(self, host, flags, next_host_arrays=None):
+        for these, last in ((host, False), (next_host_arrays or [None] * self.n_slots, True)):
+            for slot in range(len(self.hbm)):
+                if these[slot] is not None:
+                    self.hbm[slot] = these[slot].copy()
+            if not last:
+                self.computed_with.append([float(x[0]) if x is not None else None for x in (np.asarray(h).view(np.float32) for h in self.hbm)])
+
+
+def interpreter(**kwargs):
+    '''The program w * x on two arrays of 20, on the stand-in.'''
+    args = [np.zeros(20, np.float32)] * 2
+    interp = JaxprInterpreter(mj.make_jaxpr(lambda w, x: w * x)(*args), plan_only=True, **kwargs)
+    interp.sequence, interp._input_slots, interp._input_specs = Sequence(2), [0, 1], [(20, np.dtype(np.float32))] * 2
+    interp._output_slots, interp._output_sizes = [2], [20]
+    return interp
+
+
+def full(value, kind=np.copy):
+    return kind(np.full(20, value, np.float32))
+
+
+X = full(0)
+
+
+@pytest.mark.parametrize('resident', [(), (0,)])
+def test_an_array_held_before_another_took_its_place(resident):
+    interp = interpreter(resident_argnums=resident)
+    a, b = full(1, frozen), full(2)
+    for w in (a, a, b, a, b, b, a, full(3, frozen), a):
+        interp.run(w, X)
+        assert interp.sequence.computed_with[-1][0] == w[0]
+
+
+def test_one_array_made_writeable_changed_and_made_read_only_again():
+    interp = interpreter()
+    a = full(1, frozen)
+    for value in (1, 3, 5):
+        interp.run(a, X)
+        assert interp.sequence.computed_with[-1][0] == value
+        a.flags.writeable = True
+        a += 1
+        interp.run(a, X)
+        assert interp.sequence.computed_with[-1][0] == value + 1
+        a += 1
+        a.flags.writeable = False
+
+
+def test_streams():
+    interp = interpreter()
+    a, b = full(1, frozen), full(2)
+    order = [a, b, a, a, b, b, a]
+    for _ in interp.run_stream([(w, X) for w in order]):
+        pass
+    assert [w[0] for w in interp.sequence.computed_with] == [w[0] for w in order]
+    #a call in between takes the place of what the stream had sent ahead
+    interp, seen = interpreter(), []
+    for _ in interp.run_stream([(w, X) for w in order]):
+        seen.append(interp.sequence.computed_with[-1][0])
+        interp.run(full(5), X)
+        interp.run(a, X)
+    assert seen == [w[0] for w in order]
+
+
+# ------------------------------------------------------------------ on the GPU
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('way', ['plan', 'general', 'stream'])
+def test_results_of_calls_in_turn(way):
+    f = vkjax_amd.wrap(lambda w, x: w * x + np.float32(1), frontend='minijax')
+    rng = np.random.default_rng(5)
+    x = rng.random(300, dtype=np.float32)
+    a, b, c = frozen(rng.random(300, dtype=np.float32)), rng.random(300, dtype=np.float32), frozen(rng.random(300, dtype=np.float32))
+    order = [a, b, a, a, c, b, c, a]
+    if way == 'stream':
+        results = list(f.stream([(w, x) for w in order]))
+    else:
+        results = []
+        for w in order:
+            results.append(f(w, x))
+            if way == 'general':
+                f._plans = []
+    for w, y in zip(order, results):
+        assert np.array_equal(y, w * x + np.float32(1))

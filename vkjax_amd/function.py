@@ -377,7 +377,8 @@ def wrap(function: tp.Callable, *args, **kwargs) -> Function:
     Arguments are copied to the device on every call, as the reference does, with two exceptions that save the
     copy of weights and tables: leaves that cannot change while the caller holds them (numpy arrays with
     `flags.writeable == False`, jax arrays) are uploaded once and again only when another object is passed in their
-    place; and `resident_argnums=(i, ...)` declares the same for every leaf of those arguments, writeable or not -
+    place (so pass a new object for an array that was made writeable, changed and made read-only again between two
+    calls); and `resident_argnums=(i, ...)` declares the same for every leaf of those arguments, writeable or not -
     an in-place change of such a writeable array is noticed only if it touches its first or last 64 bytes, so pass a
     new array for new values. Further keyword arguments: `frontend` ('jax', 'minijax', default:
     jax where importable), `fuse`, `reuse_buffers`, `graph`.'''

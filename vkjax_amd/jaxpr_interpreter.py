@@ -246,8 +246,9 @@ class JaxprInterpreter:
 
     def _select_uploads(self, converted) -> tp.List[tp.Optional[np.ndarray]]:
         '''One entry per transfer slot: the device words of every leaf that has to be copied. A resident leaf is
-        copied when the object passed for it is not the one its buffer holds, and is noted as held from here on:
-        to be called only when the evaluation that uploads these arguments follows at once.'''
+        copied when the object passed for it is not the one its buffer holds, and is noted as held from here on; any
+        other leaf takes the place of what was held. To be called only when the evaluation that uploads these
+        arguments follows at once.'''
         host = [None] * self.sequence.n_slots
         for k, slot, x, words, is_resident in converted:
             if is_resident:
@@ -256,6 +257,8 @@ class JaxprInterpreter:
                 if held is not None and held[0] is x and held[1] == mark:
                     continue                                    #already in HBM
                 self._resident_leaves[k] = (x, mark)
+            else:
+                self._resident_leaves.pop(k, None)
             host[slot] = words if words is not None else self._device_words(k, x)
         return host
 
