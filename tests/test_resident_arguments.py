@@ -1,10 +1,12 @@
 '''What stays in HBM between calls: an evaluation computes with the arguments of its own call, whatever was held there before
 (CPU: the evaluation is a stand-in that keeps what it is handed; on the GPU, the results).'''
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import vkjax_amd
-from vkjax_amd import minijax as mj
+from vkjax_amd import hip, minijax as mj
 from vkjax_amd.jaxpr_interpreter import JaxprInterpreter
 
 
@@ -81,6 +83,34 @@ def test_streams():
         interp.run(full(5), X)
         interp.run(a, X)
     assert seen == [w[0] for w in order]
+
+
+def test_native_calls():
+    '''The same through a call's native plan.'''
+    hbm, computed_with = [None, None], []
+    def evaluate(sequence, pointers, n, flags):
+        for slot in range(2):
+            if pointers[slot]:
+                hbm[slot] = (C.c_float * 20).from_address(pointers[slot])[0]
+        computed_with.append(hbm[0])
+        return 0
+    class Interpreter:
+        def _evaluated(self, status):
+            assert status == 0
+    callback, resident, leaf = C.CFUNCTYPE(C.c_int, C.c_uint64, C.POINTER(C.c_void_p), C.c_int, C.c_uint32)(evaluate), {}, lambda slot: ('a', (20,), 'f', slot)
+    plan = hip.load_call_module().Plan(Interpreter(), resident, C.cast(callback, C.c_void_p).value, 1, 3, 0, [leaf(0), leaf(1)], leaf(2))
+    a, b = full(1, frozen), full(2)
+    for w in (a, a, b, a, b, b, a, full(3, frozen), a):
+        assert plan((w, X)) is not NotImplemented and computed_with[-1] == w[0]
+        assert list(resident) == ([] if w is b else [0])
+    for value in (3, 5):
+        a.flags.writeable = True
+        a[:] = value
+        plan((a, X))
+        a += 1
+        a.flags.writeable = False
+        plan((a, X))
+        assert computed_with[-2:] == [value, value + 1]
 
 
 # ------------------------------------------------------------------ on the GPU

@@ -204,6 +204,9 @@ PyObject* run(Plan* plan, PyObject* args) {
             PyObject* note = PyTuple_Pack(2, leaf, Py_None);
             if (!note || PyDict_SetItem(plan->resident, key, note)) { Py_XDECREF(note); PyDict_Clear(plan->resident); return nullptr; }
             Py_DECREF(note);
+        } else if (PyDict_GET_SIZE(plan->resident)) {   // takes the place of what its buffer held
+            const int noted = PyDict_Contains(plan->resident, (*plan->numbers)[k]);
+            if (noted < 0 || (noted && PyDict_DelItem(plan->resident, (*plan->numbers)[k]))) { PyDict_Clear(plan->resident); return nullptr; }
         }
         Py_INCREF(leaf);                            // (another thread may take it out of its container meanwhile)
         uploads.objects.push_back(leaf);
