@@ -85,6 +85,28 @@ def test_streams():
     assert seen == [w[0] for w in order]
 
 
+def test_uploads_between_calls():
+    '''upload_inputs takes the place of held arrays and of what a stream has sent ahead, as a call does.'''
+    class Storage:
+        size = 20
+        def __init__(self, slot):
+            self.slot, self.tensor = slot, self
+        def upload(self, words):
+            interp.sequence.hbm[self.slot] = words.copy()
+    interp = interpreter()
+    interp.input_buffers = [Storage(0), Storage(1)]
+    a, b = full(1, frozen), full(2, frozen)
+    interp.run(a, X)
+    interp.upload_inputs(b, X)
+    interp.run(a, X)
+    assert interp.sequence.computed_with[-1][0] == 1
+    seen = []
+    for _ in interp.run_stream([(a, X), (a, X), (b, X), (a, X)]):
+        seen.append(interp.sequence.computed_with[-1][0])
+        interp.upload_inputs(full(7), X)
+    assert seen == [1, 1, 2, 1]
+
+
 def test_native_calls():
     '''The same through a call's native plan.'''
     hbm, computed_with = [None, None], []

@@ -54,7 +54,7 @@ class JaxprInterpreter:
         self.workgroup_size = get_maximum_workgroup_size(self.mgr)
         self.bufferpool     = BufferPool(self.mgr, self.workgroup_size, reuse_buffers, fuse)
         self.sequence       = None
-        #counts evaluations: a suspended stream sees from it whether something else has used the argument buffers
+        #counts evaluations and uploads: a suspended stream sees from it whether something else has used the argument buffers
         self._evaluations   = 0
         self.analyze_closed_jaxpr(jaxpr)
 
@@ -383,6 +383,9 @@ class JaxprInterpreter:
     def upload_inputs(self, *X):
         '''Copy arguments into their HBM buffers without running (for measurements with resident inputs).'''
         X = self._flatten_args(X)
+        #neither held arrays nor what a suspended stream has sent ahead are there any more
+        self._resident_leaves.clear()
+        self._evaluations += 1
         for b, x, var in zip(self.input_buffers, X, self.jaxpr.jaxpr.invars):
             if b is not None and b.size:
                 b.tensor.upload(_device_words_of_argument(x, var.aval))
