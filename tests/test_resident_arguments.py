@@ -107,6 +107,37 @@ def test_uploads_between_calls():
     assert seen == [1, 1, 2, 1]
 
 
+def test_arguments_whose_evaluation_never_came():
+    '''An argument is held only once the evaluation that uploads it has been made.'''
+    a, x, wrong = full(1, frozen), full(2, frozen), np.zeros(3, np.float32)
+    wrong.flags.writeable = False
+    def runs(interp):
+        interp.run(a, x)
+        return interp.sequence.computed_with[-1]
+    interp = interpreter()
+    with pytest.raises(TypeError):
+        interp.run(a, wrong)
+    assert runs(interp) == [1, 2]
+    def raises(then):
+        yield a, x
+        if then is not None:
+            yield a, then
+        raise KeyError
+    for then, error in ((None, KeyError), (wrong, TypeError)):
+        interp = interpreter()
+        with pytest.raises(error):
+            list(interp.run_stream(raises(then)))
+        assert runs(interp) == [1, 2]
+    #the iterable makes a call of its own
+    interp = interpreter()
+    def calls():
+        for w in (a, full(3, frozen), full(4)):
+            yield w, x
+            interp.run(full(9), X)
+    for _, w in zip(interp.run_stream(calls()), (1, 3, 4)):
+        assert interp.sequence.computed_with[-1] == [w, 2]
+
+
 def test_native_calls():
     '''The same through a call's native plan.'''
     hbm, computed_with = [None, None], []
@@ -136,6 +167,20 @@ def test_native_calls():
 
 
 # ------------------------------------------------------------------ on the GPU
+
+@pytest.mark.gpu
+def test_a_stream_that_ends_in_an_error():
+    f = vkjax_amd.wrap(lambda w, x: w * x, frontend='minijax')
+    rng = np.random.default_rng(6)
+    a, b = frozen(rng.random(300, dtype=np.float32)), frozen(rng.random(300, dtype=np.float32))
+    f(b, b)
+    def raises():
+        yield a, b
+        raise KeyError
+    with pytest.raises(KeyError):
+        list(f.stream(raises()))
+    assert np.array_equal(f(a, b), a * b)
+
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('way', ['plan', 'general', 'stream'])

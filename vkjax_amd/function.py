@@ -320,10 +320,11 @@ class Function:
             in_place = False                                     #current's arguments were uploaded by the previous evaluation
             while current is not None:
                 interpreter, output_shapes, converted = current
+                #(taking the next tuple may raise: from the selection on the evaluation follows)
+                following = resolved(next(items, None))
                 if in_place and interpreter._evaluations != stamp:
                     in_place = False                             #something else used the argument buffers in between
                 host      = [None] * interpreter.sequence.n_slots if in_place else interpreter._select_uploads(converted)
-                following = resolved(next(items, None))
                 overlap   = following is not None and following[0] is interpreter
                 next_host = interpreter._select_uploads(following[2]) if overlap else None
                 fresh     = interpreter._fresh_outputs(host)

@@ -250,16 +250,20 @@ class JaxprInterpreter:
         other leaf takes the place of what was held. To be called only when the evaluation that uploads these
         arguments follows at once.'''
         host = [None] * self.sequence.n_slots
-        for k, slot, x, words, is_resident in converted:
-            if is_resident:
-                held = self._resident_leaves.get(k)
-                mark = _fingerprint(x, words) if is_resident == RESIDENT_CHECKED else None
-                if held is not None and held[0] is x and held[1] == mark:
-                    continue                                    #already in HBM
-                self._resident_leaves[k] = (x, mark)
-            else:
-                self._resident_leaves.pop(k, None)
-            host[slot] = words if words is not None else self._device_words(k, x)
+        try:
+            for k, slot, x, words, is_resident in converted:
+                if is_resident:
+                    held = self._resident_leaves.get(k)
+                    mark = _fingerprint(x, words) if is_resident == RESIDENT_CHECKED else None
+                    if held is not None and held[0] is x and held[1] == mark:
+                        continue                                #already in HBM
+                    self._resident_leaves[k] = (x, mark)
+                else:
+                    self._resident_leaves.pop(k, None)
+                host[slot] = words if words is not None else self._device_words(k, x)
+        except BaseException:
+            self._resident_leaves.clear()                       #no evaluation follows
+            raise
         return host
 
     def _host_inputs(self, X, per_argument=None) -> tp.List[tp.Optional[np.ndarray]]:
@@ -267,7 +271,11 @@ class JaxprInterpreter:
 
     def _fresh_outputs(self, host) -> tp.List[tp.Optional[np.ndarray]]:
         #every call hands out fresh arrays: the runtime copies the results straight into them
-        fresh = [np.empty(n, np.uint32) if n is not None else None for n in self._output_sizes]
+        try:
+            fresh = [np.empty(n, np.uint32) if n is not None else None for n in self._output_sizes]
+        except BaseException:
+            self._resident_leaves.clear()                       #no evaluation follows
+            raise
         for slot, arr in zip(self._output_slots, fresh):
             if slot is not None:
                 host[slot] = arr
@@ -369,9 +377,14 @@ class JaxprInterpreter:
         while True:
             if in_place and self._evaluations != stamp:
                 in_place = False                                 #something else used the argument buffers in between
-            host      = [None] * self.sequence.n_slots if in_place else self._host_inputs(tuple(current))
+            #(what may raise, or call the function itself, comes first: from the selection on the evaluation follows)
+            words     = None if in_place else self._convert_inputs(tuple(current))
             following = next(iterator, end)
-            next_host = self._host_inputs(tuple(following)) if following is not end else None
+            if in_place and self._evaluations != stamp:
+                in_place, words = False, self._convert_inputs(tuple(current))
+            next_words = self._convert_inputs(tuple(following)) if following is not end else None
+            host      = [None] * self.sequence.n_slots if in_place else self._select_uploads(words)
+            next_host = self._select_uploads(next_words) if following is not end else None
             fresh     = self._fresh_outputs(host)
             self.evaluate(host, next_host)
             stamp, in_place = self._evaluations, following is not end
