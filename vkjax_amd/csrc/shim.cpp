@@ -228,6 +228,12 @@ bool carried(const void* device, const void* staging, size_t nbytes) {
     return (((uintptr_t)device | (uintptr_t)staging | nbytes) & 3u) == 0;
 }
 
+// Whether one range of a slab may cover both uploads, the second of which begins `gap` bytes behind the first's end: what lies
+// between them belongs to no array, i.e. is the padding behind the first one's.
+bool only_padding_between(const Transfer& first, const Transfer& second, size_t gap) {
+    return gap == 0 || (gap < PACKED_ALIGN && second.offset == 0 && first.offset + first.nbytes == first.buf->nbytes);
+}
+
 void drop_graph(Seq* s) {
     if (s->graph_exec) { hipGraphExecDestroy(s->graph_exec); s->graph_exec = nullptr; }
     s->graph_failed = false;
@@ -321,11 +327,11 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
             // all arguments as one stream of chunks: a few threads stage them, this one hands each chunk to the
             // DMA engine as soon as it is staged
             std::vector<UploadPiece> pieces;
-            std::vector<int> piece_slot;
+            std::vector<const Transfer*> transfer;
             for (auto& t : s->uploads)
                 if (t.nbytes && host_ptrs[t.slot]) {
                     pieces.push_back({(char*)t.staging, (const char*)host_ptrs[t.slot], (char*)t.buf->dptr + t.offset, t.nbytes});
-                    piece_slot.push_back(t.slot);
+                    transfer.push_back(&t);
                 }
             const size_t nl = s->launches.size();
             // Launches that follow the uploads: a program that brings all its weights with every call need not wait for
@@ -362,11 +368,11 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                     return first_use[a] != first_use[b] ? first_use[a] < first_use[b] : pieces[a].nbytes < pieces[b].nbytes;
                 });
                 std::vector<UploadPiece> sorted_pieces;
-                std::vector<int> sorted_slot;
+                std::vector<const Transfer*> sorted_transfer;
                 std::vector<size_t> sorted_use;
-                for (size_t p : order) { sorted_pieces.push_back(pieces[p]); sorted_slot.push_back(piece_slot[p]); sorted_use.push_back(first_use[p]); }
+                for (size_t p : order) { sorted_pieces.push_back(pieces[p]); sorted_transfer.push_back(transfer[p]); sorted_use.push_back(first_use[p]); }
                 pieces.swap(sorted_pieces);
-                piece_slot.swap(sorted_slot);
+                transfer.swap(sorted_transfer);
                 // (sorted by first use: the pieces a launch needs end where the pieces first read by a later launch begin)
                 size_t p = 0;
                 long reached = -1;
@@ -405,7 +411,7 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
             size_t early_piece = pieces.size(), next_part = 0;
             if (!s->early.empty() && !s->profiling && !s->want_graph && !s->uses_side) {
                 for (size_t p = 0; p < pieces.size(); p++)
-                    if (piece_slot[p] == s->early_slot && pieces[p].nbytes >= s->early.back().bytes_needed) early_piece = p;
+                    if (transfer[p]->slot == s->early_slot && pieces[p].nbytes >= s->early.back().bytes_needed) early_piece = p;
                 const size_t must_be = follow ? (size_t)(need[s->early_at] < 0 ? pieces.size() : need[s->early_at]) : pieces.size() - 1;
                 if (early_piece != must_be) early_piece = pieces.size();
             }
@@ -417,10 +423,10 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                 if ((launch_status = issue_launch(c, s->launches[next_launch++]))) return launch_status;
             }
             // Small arrays that lie next to each other in HBM and in their staging memory alike (vkj_buf_alloc_packed) are
-            // sent as one transfer: the run is extended while the next array starts within the alignment step behind it,
+            // sent as one transfer: the run is extended while the next array starts behind it with nothing but padding between them,
             // by the same distance on both sides. Hundreds of transfers of a few KB each would cost more host time than
             // the bytes take to travel.
-            struct { uintptr_t device = 0, staging = 0; size_t len = 0; hipStream_t stream = nullptr; } run;
+            struct { uintptr_t device = 0, staging = 0; size_t len = 0; hipStream_t stream = nullptr; const Transfer* last = nullptr; } run;
             auto flush_run = [&]() {
                 if (run.len) err = hipMemcpyAsync((void*)run.device, (const void*)run.staging, run.len, hipMemcpyHostToDevice, run.stream);
                 run.len = 0;
@@ -431,13 +437,14 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                 hipStream_t to = (k & 1) ? copy_odd : copy_even;
                 if (pieces[piece].nbytes <= PACKED_MAX_BYTES) {
                     const size_t step = device - run.device;
-                    if (run.len && device > run.device && step == staging - run.staging && step >= run.len && step < run.len + PACKED_ALIGN
-                            && step + len <= UPLOAD_CHUNK) {
+                    if (run.len && device > run.device && step == staging - run.staging && step >= run.len
+                            && only_padding_between(*run.last, *transfer[piece], step - run.len) && step + len <= UPLOAD_CHUNK) {
                         run.len = step + len;
                     } else {
                         if (!flush_run()) return 1;
                         run.device = device; run.staging = staging; run.len = len; run.stream = to;
                     }
+                    run.last = transfer[piece];
                 } else {
                     if (!flush_run()) return 1;
                     err = hipMemcpyAsync((void*)device, (const void*)staging, len, hipMemcpyHostToDevice, to);
@@ -488,9 +495,9 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                 }
             }
         } else if (c->carry) {
-            // (neighbours in HBM that are neighbours in their staging memory: one range, with what lies between them)
+            // (neighbours in HBM that are neighbours in their staging memory: one range, with the padding between them)
             Carry what;
-            const Slab* slab = nullptr;                  // of the last range
+            const Transfer* before = nullptr;            // the last one in the last range, where that lies in a slab
             for (auto& t : s->uploads) {
                 if (!t.nbytes || !host_ptrs[t.slot]) continue;
                 memcpy(t.staging, host_ptrs[t.slot], t.nbytes);
@@ -499,16 +506,17 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                     HIP_TRY(hipMemcpyAsync(device, t.staging, t.nbytes, hipMemcpyHostToDevice, c->stream));
                     continue;
                 }
-                if (what.count && t.staging_mirrors_slab && t.buf->slab == slab) {
+                if (what.count && before && t.staging_mirrors_slab && t.buf->slab == before->buf->slab) {
                     auto& last = what.range[what.count - 1];
                     const size_t step = (uintptr_t)device - (uintptr_t)last.dst;
                     if ((uintptr_t)device > (uintptr_t)last.dst && step == (uintptr_t)t.staging - (uintptr_t)last.src && step >= last.nbytes
-                            && step < last.nbytes + PACKED_ALIGN) {
+                            && only_padding_between(*before, t, step - last.nbytes)) {
                         last.nbytes = step + t.nbytes;
+                        before = &t;
                         continue;
                     }
                 }
-                slab = t.staging_mirrors_slab ? t.buf->slab : nullptr;
+                before = t.staging_mirrors_slab ? &t : nullptr;
                 if (what.count == Carry::MAX) {
                     if (int r = c->carry(what, false, c->stream)) return r;
                     what.count = 0;
