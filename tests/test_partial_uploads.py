@@ -32,6 +32,11 @@ CASES = {
     'one inside another':      ([300], [(0, 0, 300), (0, 100, 8)]),
     'one around another':      ([300], [(0, 100, 8), (0, 0, 300)]),
     'two in their middle':     ([300], [(0, 0, 200), (0, 100, 200)]),
+    'inside, unpacked':        ([100000], [(0, 0, 100000), (0, 4096, 8)]),
+    'around, unpacked':        ([100000], [(0, 4096, 8), (0, 0, 100000)]),
+    'odd inside, unpacked':    ([100000], [(0, 0, 100000), (0, 4097, 2)]),
+    'many':                    ([100000], [(0, 4 * k, 400) for k in range(0, 1000, 25)]),
+    'inside, large':           ([9 << 20], [(0, 0, 9 << 20), (0, 5 << 20, 8)]),
 }
 
 

@@ -323,7 +323,8 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
     if (up) {
         size_t total = 0;
         for (auto& t : s->uploads) if (t.nbytes && host_ptrs[t.slot]) total += t.nbytes;
-        if (total >= STAGE_MIN) {
+        // (uploads that overlap arrive in the order they were recorded in: one after the other, on the stream)
+        if (total >= STAGE_MIN && !s->uploads_overlap) {
             // all arguments as one stream of chunks: a few threads stage them, this one hands each chunk to the
             // DMA engine as soon as it is staged
             std::vector<UploadPiece> pieces;
@@ -494,7 +495,7 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
                     first_launch = s->early_at + 1;
                 }
             }
-        } else if (c->carry) {
+        } else if (c->carry && !s->uploads_overlap) {
             // (neighbours in HBM that are neighbours in their staging memory: one range, with the padding between them)
             Carry what;
             const Transfer* before = nullptr;            // the last one in the last range, where that lies in a slab
@@ -1021,7 +1022,13 @@ static int record_transfer(const char* who, std::vector<Transfer>& list, Seq* s,
 int vkj_seq_record_upload(vkj_handle sh, vkj_handle bh, size_t offset, int slot, size_t nbytes) {
     Seq* s = from_handle<Seq>(sh, MAGIC_SEQ);
     if (!s) return fail(VKJ_EINVAL, "vkj_seq_record_upload: bad sequence handle");
-    return record_transfer("vkj_seq_record_upload", s->uploads, s, bh, offset, slot, nbytes);
+    if (int r = record_transfer("vkj_seq_record_upload", s->uploads, s, bh, offset, slot, nbytes)) return r;
+    const Transfer& t = s->uploads.back();
+    for (size_t k = 0; k + 1 < s->uploads.size(); k++) {
+        const Transfer& u = s->uploads[k];
+        if (u.buf == t.buf && u.offset < t.offset + t.nbytes && t.offset < u.offset + u.nbytes) s->uploads_overlap = true;
+    }
+    return 0;
 }
 
 int vkj_seq_record_download(vkj_handle sh, vkj_handle bh, size_t offset, int slot, size_t nbytes) {

@@ -137,6 +137,7 @@ struct Seq {
     Ctx*                    ctx = nullptr;
     bool                    profiling = false;
     std::vector<Transfer>   uploads, downloads;
+    bool                    uploads_overlap = false;    // two of them write the same bytes
     std::vector<Launch>     launches;
     std::vector<hipEvent_t> chunk_events;   // one behind every chunk of a large download
     std::vector<hipEvent_t> stamps;         // profiling: 1 + number of steps
