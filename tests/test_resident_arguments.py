@@ -1,6 +1,7 @@
 '''What stays in HBM between calls: an evaluation computes with the arguments of its own call, whatever was held there before
 (CPU: the evaluation is a stand-in that keeps what it is handed; on the GPU, the results).'''
 import ctypes as C
+import weakref
 
 import numpy as np
 import pytest
@@ -164,6 +165,33 @@ def test_native_calls():
         a.flags.writeable = False
         plan((a, X))
         assert computed_with[-2:] == [value, value + 1]
+
+
+def test_arguments_live_until_a_native_call_ends():
+    '''The last reference to an array that was held goes inside a call, and what runs then empties the call's own list.'''
+    alive, values = [], []
+    def evaluate(sequence, pointers, n, flags):
+        alive.append(second() is not None)
+        values.append((C.c_float * 20).from_address(pointers[1])[19])
+        return 0
+    class Interpreter:
+        def _evaluated(self, status):
+            pass
+    callback, resident, leaf = C.CFUNCTYPE(C.c_int, C.c_uint64, C.POINTER(C.c_void_p), C.c_int, C.c_uint32)(evaluate), {}, lambda slot: ('a', (20,), 'f', slot)
+    plan = hip.load_call_module().Plan(Interpreter(), resident, C.cast(callback, C.c_void_p).value, 1, 3, 0, [('l', [leaf(0), leaf(1)])], leaf(2))
+    for kind in (frozen, np.copy):
+        old = full(1, frozen)
+        arguments = [old, full(3)]
+        second = weakref.ref(arguments[1])
+        plan((arguments,))
+        weakref.finalize(old, lambda: following.clear())
+        #the note of `old` gives way to another one, or goes
+        following = [full(4, kind), full(5)]
+        second = weakref.ref(following[1])
+        del old, arguments
+        plan((following,))
+        assert following == [] and alive[-1] and values[-1] == 5
+        assert second() is None
 
 
 # ------------------------------------------------------------------ on the GPU

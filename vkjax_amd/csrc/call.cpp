@@ -75,9 +75,15 @@ bool parse(PyObject* spec, Node& node, Py_ssize_t& leaves) {
     return true;
 }
 
-// Whether x is what the signature says; its leaves are added to `found` (borrowed). Exact types only: anything else may mean
-// something else to the general path. -1: an exception is set.
-int match(const Node& node, PyObject* x, std::vector<PyArrayObject*>& found) {
+struct Held {                                       // references that go when the call ends, whichever way
+    std::vector<PyObject*> objects;
+    ~Held() { for (PyObject* o : objects) Py_XDECREF(o); }
+};
+
+// Whether x is what the signature says; its leaves are added to `found`, with a reference each: what runs between here and the
+// evaluation (the end of an array that was held, the cycle collector, another thread) may take them out of their containers.
+// Exact types only: anything else may mean something else to the general path. -1: an exception is set.
+int match(const Node& node, PyObject* x, Held& found) {
     switch (node.kind) {
     case Node::LEAF: {
         if (!PyArray_CheckExact(x)) return 0;
@@ -85,7 +91,8 @@ int match(const Node& node, PyObject* x, std::vector<PyArrayObject*>& found) {
         if (PyArray_TYPE(a) != node.type || PyArray_ISBYTESWAPPED(a) || PyArray_NDIM(a) != (int)node.shape.size()) return 0;
         for (size_t d = 0; d < node.shape.size(); d++) if (PyArray_DIM(a, (int)d) != node.shape[d]) return 0;
         if (node.slot >= 0 && !PyArray_IS_C_CONTIGUOUS(a)) return 0;
-        found.push_back(a);
+        found.objects.push_back(x);
+        Py_INCREF(x);
         return 1;
     }
     case Node::NONE:
@@ -167,39 +174,33 @@ void leaf_slots(const Node& node, std::vector<int>& slots) {
     for (const Node& c : node.children) leaf_slots(c, slots);
 }
 
-struct Held {                                       // references that go when the call ends, whichever way
-    std::vector<PyObject*> objects;
-    ~Held() { for (PyObject* o : objects) Py_XDECREF(o); }
-};
-
 PyObject* run(Plan* plan, PyObject* args) {
     if (!PyTuple_CheckExact(args) || PyTuple_GET_SIZE(args) != (Py_ssize_t)plan->arguments->size()) Py_RETURN_NOTIMPLEMENTED;
-    std::vector<PyArrayObject*> found;
-    found.reserve(plan->numbers->size());
+    Held found;
+    found.objects.reserve(plan->numbers->size());
     for (size_t i = 0; i < plan->arguments->size(); i++) {
         const int r = match((*plan->arguments)[i], PyTuple_GET_ITEM(args, (Py_ssize_t)i), found);
         if (r < 0) return nullptr;
         if (r == 0) Py_RETURN_NOTIMPLEMENTED;
     }
     std::vector<int> slots;
-    slots.reserve(found.size());
+    slots.reserve(found.objects.size());
     for (const Node& n : *plan->arguments) leaf_slots(n, slots);
     std::vector<void*> host((size_t)plan->nslots, nullptr);
-    Held results, uploads;
+    Held results;
     results.objects.reserve((size_t)plan->nresults);
-    uploads.objects.reserve(found.size());
     if (!new_results(*plan->result, results.objects)) return nullptr;
     size_t next = 0;
     result_pointers(*plan->result, results.objects, next, host);
     // Which leaves have to be copied: all that may have changed, and those that are not what their buffers hold. From here on
     // the evaluation follows at once, so what is noted as held is held.
-    for (size_t k = 0; k < found.size(); k++) {
+    for (size_t k = 0; k < found.objects.size(); k++) {
         if (slots[k] < 0) continue;
-        PyObject* leaf = (PyObject*)found[k];
+        PyObject* leaf = found.objects[k];
         if (immutable(leaf)) {
             PyObject* key  = (*plan->numbers)[k];
             PyObject* held = PyDict_GetItemWithError(plan->resident, key);
-            if (!held && PyErr_Occurred()) return nullptr;
+            if (!held && PyErr_Occurred()) { PyDict_Clear(plan->resident); return nullptr; }
             if (held && PyTuple_CheckExact(held) && PyTuple_GET_SIZE(held) == 2 && PyTuple_GET_ITEM(held, 0) == leaf && PyTuple_GET_ITEM(held, 1) == Py_None) continue;
             PyObject* note = PyTuple_Pack(2, leaf, Py_None);
             if (!note || PyDict_SetItem(plan->resident, key, note)) { Py_XDECREF(note); PyDict_Clear(plan->resident); return nullptr; }
@@ -208,9 +209,7 @@ PyObject* run(Plan* plan, PyObject* args) {
             const int noted = PyDict_Contains(plan->resident, (*plan->numbers)[k]);
             if (noted < 0 || (noted && PyDict_DelItem(plan->resident, (*plan->numbers)[k]))) { PyDict_Clear(plan->resident); return nullptr; }
         }
-        Py_INCREF(leaf);                            // (another thread may take it out of its container meanwhile)
-        uploads.objects.push_back(leaf);
-        host[(size_t)slots[k]] = PyArray_DATA(found[k]);
+        host[(size_t)slots[k]] = PyArray_DATA((PyArrayObject*)leaf);
     }
     int status;
     Py_BEGIN_ALLOW_THREADS
