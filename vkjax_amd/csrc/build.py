@@ -1,5 +1,6 @@
 '''Build the native parts in-tree: the C-ABI runtime (libvkjax_hip.so), the extension module that makes
 calls natively (vkjax_call.so) and the gfx950 code objects with the kernels (one .hsaco per kernels/*.hip). Needs only hipcc; no GPU.
+Without the headers of Python and numpy the extension module is left out: calls take the general path then.
 
     python -m vkjax_amd.csrc.build [--force]
 '''
@@ -72,7 +73,12 @@ def build_call(force=True):
     src, out = os.path.join(CSRC, 'call.cpp'), os.path.join(LIBDIR, 'vkjax_call.so')
     if not force and _newer(out, [src]):
         return out
-    _run(['g++', '-O2', '-fPIC', '-shared', '-std=c++17', f'-I{sysconfig.get_paths()["include"]}', f'-I{numpy.get_include()}', src, '-o', out])
+    headers = {'Python.h': sysconfig.get_paths()['include'], 'numpy/arrayobject.h': numpy.get_include()}
+    missing = [f'{name} in {path}' for name, path in headers.items() if not os.path.exists(os.path.join(path, name))]
+    if missing:
+        print(f'not built: vkjax_call.so (no {", no ".join(missing)}); calls of wrapped functions take the general path')
+        return None
+    _run([HIPCC, '-no-hip-rt', '-x', 'c++', '-O2', '-fPIC', '-shared', '-std=c++17'] + [f'-I{path}' for path in headers.values()] + [src, '-o', out])
     return out
 
 
@@ -91,7 +97,7 @@ def build_all(force=True, jobs=None):
     jobs = jobs or min(8, os.cpu_count() or 1)
     with ThreadPoolExecutor(jobs) as pool:
         futures = [pool.submit(build_shim, force), pool.submit(build_call, force)] + [pool.submit(build_kernel, k, force) for k in KERNEL_SOURCES]
-        return [f.result() for f in futures]
+        return [path for path in (f.result() for f in futures) if path is not None]
 
 
 if __name__ == '__main__':

@@ -11,6 +11,7 @@ import importlib.util
 import os
 import threading
 import typing as tp
+import warnings
 
 import numpy as np
 
@@ -76,7 +77,7 @@ _PROTOTYPES = {
 }
 
 _lib      = None
-_call_module = None
+_call_module = None             #False: it could not be loaded
 _lib_lock = threading.Lock()
 
 
@@ -107,7 +108,7 @@ def load_call_module():
     '''The extension module whose plans make calls natively (csrc/call.cpp). Raises if it has not been built.'''
     global _call_module
     with _lib_lock:
-        if _call_module is None:
+        if not _call_module:
             path = os.path.join(LIBDIR, 'vkjax_call.so')
             if not os.path.exists(path):
                 raise RuntimeError(f'{path} is missing: build it with `python -m vkjax_amd.csrc.build`')
@@ -116,6 +117,18 @@ def load_call_module():
             spec.loader.exec_module(module)
             _call_module = module
     return _call_module
+
+
+def call_module():
+    '''load_call_module(), or None - with a warning, once - where it cannot be loaded: the general path makes the same calls.'''
+    global _call_module
+    if _call_module is None:
+        try:
+            load_call_module()
+        except (RuntimeError, ImportError) as error:
+            warnings.warn(f'calls of wrapped functions take the general path: {error}', RuntimeWarning, stacklevel=2)
+            _call_module = False
+    return _call_module or None
 
 
 class HipError(RuntimeError):

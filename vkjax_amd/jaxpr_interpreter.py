@@ -319,7 +319,7 @@ class JaxprInterpreter:
     def call_plan(self, leaves, argument_structures, result_structure):
         '''The native plan of calls with arguments like these (`leaves` in containers of these structures, minijax.tree_util) and
         results of that structure, or None where the general path has something to do that a plan does not: arguments converted
-        or checked on the host, results that are.'''
+        or checked on the host, results that are. None also where the extension module has not been built.'''
         plain = {np.dtype(np.float32): 'f', np.dtype(np.int32): 'i', np.dtype(np.uint32): 'u'}
         avals, outs = [v.aval for v in self.jaxpr.jaxpr.invars], [v.aval for v in self.jaxpr.jaxpr.outvars]
         if (self.sequence is None or self.profiling or self.static_argnums or self.resident_argnums
@@ -327,6 +327,9 @@ class JaxprInterpreter:
                 or any(b is None for b in self.output_buffers) or any(np.dtype(b.dtype) not in plain for b in self.output_buffers)
                 or len(leaves) != len(avals) or result_structure.num_leaves != len(outs)
                 or any(type(x) is not np.ndarray or x.dtype != a.dtype or x.shape != tuple(a.shape) for x, a in zip(leaves, avals))):
+            return None
+        module = hip.call_module()
+        if module is None:
             return None
 
         def specification(structure, leaves):
@@ -341,8 +344,8 @@ class JaxprInterpreter:
         inputs    = iter(zip(avals, self._input_slots))
         arguments = [specification(c, inputs) for c in argument_structures]
         result    = specification(result_structure, iter(zip(outs, self._output_slots)))
-        return hip.load_call_module().Plan(self, self._resident_leaves, hip.function_address('vkj_seq_eval'), self.sequence.handle, self.sequence.n_slots,
-                                           hip.EVAL_NULL_IS_RESIDENT, arguments, result)
+        return module.Plan(self, self._resident_leaves, hip.function_address('vkj_seq_eval'), self.sequence.handle, self.sequence.n_slots,
+                           hip.EVAL_NULL_IS_RESIDENT, arguments, result)
 
     def run_leaves(self, per_argument):
         '''`run` for a caller that has flattened the arguments already: one list of leaves per argument.'''
