@@ -558,15 +558,17 @@ def _row_program_around(ops, seed: int, outer: int, R: int, bufferpool, outvars)
     members = sorted(group)
     counts  = collections.Counter(pid(b) for op in ops for b in _writes(op))
     while len(members) >= ROW_PROGRAM_MIN_OPS:
-        inside, tainted, taken, behind = set(), set(), [], []
+        inside, tainted, wanted, taken, behind = set(), set(), set(), [], []
         for i in range(members[0], members[-1] + 1):
             op = ops[i]
             if i in members and not any(pid(b) in tainted for b in _reads(op)) and counts[pid(result_of(op))] == 1:
                 taken.append(i)
                 inside.add(pid(result_of(op)))
-            elif any(pid(b) in tainted or pid(b) in inside for b in _touched(op)):
+            elif any(pid(b) in tainted or pid(b) in inside for b in _touched(op)) or any(pid(b) in wanted for b in _written(op)):
+                #(what it reads may not be written in front of it either)
                 behind.append(i)
                 tainted |= {pid(b) for b in _may_write(op)}
+                wanted  |= {pid(b) for b in _reads(op)}
         if len(taken) < ROW_PROGRAM_MIN_OPS or seed not in taken:
             return None, [], []
         if taken != members:
