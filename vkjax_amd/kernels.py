@@ -1372,11 +1372,25 @@ def _column_block_width(outer: int, R: int, inner: int, nsplit: int) -> int:
 
 
 #Columns of at most this many rows are summed by one launch: a second one costs about 2.3 us. Sums of R x columns in two launches, in one:
-#128 x 100 4.6, 2.5 us; 1000 x 10 4.7, 3.2; 1000 x 100 5.1, 3.9; 1536 x 64 5.1, 4.2; 1536 x 1000 5.9, 4.8; 1000 x 9408 9.1, 8.8; 1536 x 5000 8.4, 9.6;
+#128 x 100 4.6, 2.5 us; 1000 x 10 4.7, 3.2; 1000 x 100 5.1, 3.9; 1536 x 64 5.1, 4.2; 1536 x 1000 5.9, 4.8; 1000 x 9408 9.1, 8.8;
 #1536 x 30000 34, 29; 2000 x 100 5.2, 5.4; 4096 x 100 5.3, 8.7. A number of columns that is no multiple of four is read a word at a time,
 #and up to eight steps of four rows per thread pay: 1000 x 1001 5.7, 3.7; 512 x 4095 (8 steps) 5.7, 3.6; 1000 x 4095 (16) 6.4, 10.0; 1536 x 1001 (12) 6.0, 6.3;
 #512 x 9407 (32) 7.4, 12.7
 REDUCE_UNSPLIT_ROWS, REDUCE_UNSPLIT_STEPS = 1536, 8
+#Two launches are faster on arrays of some size in two cases (of 368 sums of 256 to 1536 rows and 64 to 80000 columns, one launch always costs 1.5 % more
+#than the better of the two on average and up to 25 %, this rule 0.3 % and up to 14). The narrowest blocks read 128 bytes of every row, two lines of memory
+#where rows do not begin at a line: 1536 x 4316 7.6 us in two, 9.5 in one, 1536 x 5000 8.4, 9.6, 1400 x 5860 8.8, 10.7, 1100 x 7640 8.8, 10.3; below that
+#size 1024 x 5000 (20 MB) 6.8, 6.2, 1536 x 3372 (21) 7.5, 7.6; at whole lines 1536 x 4096 5.8, 4.6. And large arrays for which one launch has too few blocks, as where a
+#block more per CU would make them narrower: 900 x 33216 (130 blocks, 120 MB) 20.9, 24.6, 1536 x 36864 (144) 35.1, 39.4; but 1536 x 9408 (147, 58 MB) 12.7, 12.2,
+#1536 x 24576 (192) 26.5, 22.7
+REDUCE_NARROW_UNSPLIT_BYTES, REDUCE_UNSPLIT_BYTES, REDUCE_UNSPLIT_BLOCKS = 24 << 20, 64 << 20, 160
+
+
+def _column_sum_starves(outer: int, R: int, inner: int) -> bool:
+    '''Whether columns read four at a time are summed faster by two launches although there are few rows.'''
+    width, nbytes = _column_block_width(outer, R, inner, 1), 4 * outer * R * inner
+    return ((width == 8 and inner % 32 != 0 and nbytes >= REDUCE_NARROW_UNSPLIT_BYTES)
+            or (outer * _cdiv(inner, 4 * width) <= REDUCE_UNSPLIT_BLOCKS and nbytes >= REDUCE_UNSPLIT_BYTES))
 
 
 def plan_reduce_splits(outer: int, R: int, inner: int, op: str, compute_units: int = 256) -> int:
@@ -1386,7 +1400,8 @@ def plan_reduce_splits(outer: int, R: int, inner: int, op: str, compute_units: i
     if inner == 1:
         want  = 32 * compute_units                 #waves
         split = min(_cdiv(want, outer), R // 4096)         #at least 16 KB per wave
-    elif R <= REDUCE_UNSPLIT_ROWS and (inner % 4 == 0 or _cdiv(R, 4 * (BLOCK // _column_block_width(outer, R, inner, 1))) <= REDUCE_UNSPLIT_STEPS):
+    elif R <= REDUCE_UNSPLIT_ROWS and (not _column_sum_starves(outer, R, inner) if inner % 4 == 0 else
+                                       _cdiv(R, 4 * (BLOCK // _column_block_width(outer, R, inner, 1))) <= REDUCE_UNSPLIT_STEPS):
         return 1
     else:
         tiles = _cdiv(inner, 256)
