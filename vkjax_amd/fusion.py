@@ -1681,8 +1681,9 @@ def batch_packs(ops):
     return result
 
 
-#launches a program must save before its small chains are moved and batched (3: the four updates of a network of two
-#convolutions; their chains and sums apart used to save 6)
+#launches a program must save before its small chains are moved and batched. Replays of training steps, not batched and batched: two
+#dense layers over 1000 rows, which save three, 78.4 and 69.0 us; programs that would save two, and are left as they are: two dense layers
+#over 200 rows 61.5, 57.2, over 128 rows 55.8, 52.1, two convolutions on four images 88.0, 82.2, three dense layers over 61 rows 75.2, 72.5
 BATCH_MIN_GAIN = 3
 
 
