@@ -16,6 +16,7 @@ the position of its last member, so the lifetimes of the earlier members' inputs
 to that position, and the skipped intermediates get no storage.
 '''
 import collections
+import functools
 import typing as tp
 
 import numpy as np
@@ -156,6 +157,24 @@ def _epilogue_steps(steps: tp.Sequence[EwStep], geom: K.ConvGeometry, out_shape)
             return None
         result.append(K.ConvEpilogueStep(s.op, kind, o.buffer, s.operand_left))
     return result
+
+
+def _where(occurs):
+    '''A pass that is entered only where an op it is about occurs, and hands the list it was given back where it changes
+    nothing (what is known about a list of ops is kept with the list: _use_counts, remove_dead_ops).'''
+    def only(fuse):
+        @functools.wraps(fuse)
+        def entered(ops, bufferpool, outvars):
+            if not any(map(occurs, ops)):
+                return ops
+            result = fuse(ops, bufferpool, outvars)
+            return ops if len(result) == len(ops) and all(a is b for a, b in zip(result, ops)) else result
+        return entered
+    return only
+
+
+def _is(kind):
+    return lambda op: op.meta is not None and op.meta[0] == kind
 
 
 def fuse_ops(all_ops, bufferpool, outvars):
@@ -334,9 +353,11 @@ def fuse_ops(all_ops, bufferpool, outvars):
     ops = fold_index_wrap(ops, bufferpool, outvars)
     ops = fuse_dense_softmax(ops, bufferpool, outvars)
     ops = remove_dead_ops(ops, bufferpool, outvars)
+    bufferpool.use_counts, bufferpool.without_dead = (None, None), None
     return batch_small_chains(batch_packs(ops))
 
 
+@_where(_is('reduce'))
 def fuse_softmax(ops, bufferpool, outvars):
     '''softmax over the last dimension as jax.nn.softmax spells it,
 
@@ -492,6 +513,7 @@ class _RowProgram:
         self.launch = K.row_program(self.outs, self.inputs, self.steps, outer, R)
 
 
+@_where(lambda op: _is_row_reduction(op))
 def fuse_row_programs(ops, bufferpool, outvars):
     '''Element-wise chains and row reductions over the rows of one [outer, R] array that feed each other - a classifier's
     loss and its gradient - become one launch (rows.hip), values bit for bit. What stands between them and reads
@@ -590,6 +612,7 @@ def _row_program_around(ops, seed: int, outer: int, R: int, bufferpool, outvars)
     return None, [], []
 
 
+@_where(lambda op: op.chain is not None and len(op.chain.steps) == 3 and op.chain.steps[0].op == EW['LT_I'])
 def fuse_index_wrap(ops, bufferpool, outvars):
     '''`select(x < 0, x + n, x)` on int32, the way tracing normalises an index that may count from the end, is two
     launches after chain fusion (x + n, and the comparison with the select, which needs x + n as a second full-size
@@ -626,6 +649,7 @@ def fuse_index_wrap(ops, bufferpool, outvars):
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
 
 
+@_where(lambda op: op.chain is not None and len(op.chain.steps) == 1 and op.chain.steps[0].op == EW['WRAP_I'])
 def fold_index_wrap(ops, bufferpool, outvars):
     '''The normalised copy of an index array, `select(i < 0, i + n, i)` (one launch after fuse_index_wrap), is not made
     when everything that reads it is a row gather or a sorted row scatter-add: those kernels read the indices as they
@@ -668,6 +692,7 @@ def fold_index_wrap(ops, bufferpool, outvars):
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
 
 
+@_where(_is('softmax'))
 def fuse_dense_softmax(ops, bufferpool, outvars):
     '''A classifier's last layer: a product with at most 16 output features, read by nothing but the softmax launch
     right behind it, computes the softmax (and the arg-max that launch carries) on the row before it is stored
@@ -705,6 +730,7 @@ def np_prod(values) -> int:
     return out
 
 
+@_where(_is('reduce'))
 def fuse_reduce_prologues(ops, bufferpool, outvars):
     '''A float column sum whose operand is, and is only, the result of `a * b` (b of the same shape or a
     vector over the columns) or of `-a` reads a (and b) itself and applies the step while loading: the
@@ -770,6 +796,7 @@ def _sole_reader_takes(ops, i, C, uses) -> bool:
             and not any(w._placeholder is source._placeholder for j in range(i + 1, C) for w in _written(ops[j])))
 
 
+@_where(_is('reduce'))
 def fuse_reduce_scales(ops, bufferpool, outvars):
     '''A float sum (one launch: not split into ranges) whose result is read once, by `sum / c`, `sum * c` or `-(sum / c)` with a single value c - a mean, a mean
     negative log-likelihood - stores that itself: the element-wise launch behind it goes away. The division is the one
@@ -805,6 +832,7 @@ def fuse_reduce_scales(ops, bufferpool, outvars):
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
 
 
+@_where(lambda op: _is_float_sum(op))
 def fuse_reduce_updates(ops, bufferpool, outvars):
     '''A float column sum (of the slices of a kernel gradient, of the rows of a bias gradient) whose result is read once, by
     `p - rate * sum` with a single value `rate` - a step of gradient descent - stores that difference itself. Same
@@ -842,6 +870,7 @@ def fuse_reduce_updates(ops, bufferpool, outvars):
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
 
 
+@_where(_is('reduce'))
 def fuse_scale_relu_backward(ops, bufferpool, outvars):
     '''The backward pass of a per-channel scale and shift followed by ReLU (a batch norm with fixed statistics
     and its activation), as reverse-mode differentiation emits it:
@@ -1035,6 +1064,7 @@ def _select_by_threshold(chain) -> bool:
             and chain.out.dtype == 'float32' and chain.out.size == np_prod(chain.shape))
 
 
+@_where(_is('reduce'))
 def fuse_relu_backward_sums(ops, bufferpool, outvars):
     '''The backward pass of a dense layer's ReLU and the gradient of the bias in front of it,
 
@@ -1187,6 +1217,7 @@ def fuse_window_sums(ops, bufferpool, outvars):
     return [op for op in ops if op is not None]
 
 
+@_where(lambda op: op.chain is not None and op.chain.out.size == 1 and op.chain.out.tensor is None)
 def fold_scalar_constants(ops, bufferpool, outvars):
     '''Arithmetic on single floats that are known when the program is built (-1 / 1000, the factor of a mean's gradient) is done
     then, with the device's rounding, and its result is a constant like the ones it came from: one launch less per value
@@ -1242,6 +1273,7 @@ def _is_full_contiguous_any_shape(operand: EwOperand, shape) -> bool:
     return operand.offset == 0 and operand.buffer.size == size and _walks_densely(operand.strides, shape)
 
 
+@_where(_is('random_stream'))
 def fuse_stream_chains(ops, bufferpool, outvars):
     '''A launch that generates random words (random_bits lowered directly) followed by an
     element-wise chain over exactly those words whose operands are single values: the chain is
@@ -1280,6 +1312,7 @@ def fuse_stream_chains(ops, bufferpool, outvars):
     return [replacement.get(i, op) for i, op in enumerate(ops) if i not in removed]
 
 
+@_where(_is('random_stream'))
 def fuse_key_splits(ops, bufferpool, outvars):
     '''A key split (a launch of random words without steps) whose words nothing but the keys of other draws read: those draws
     compute their two words of it themselves. Same bits; the split's launch goes.'''
@@ -1336,6 +1369,7 @@ def fuse_key_splits(ops, bufferpool, outvars):
     return [op for i, op in enumerate(result) if i not in gone]
 
 
+@_where(lambda op: op.conv is not None and any(e.kind == 2 and e.derived is None for e in op.conv[4]))
 def fuse_derived_epilogue_operands(ops, bufferpool, outvars):
     '''A per-feature operand of a convolution epilogue that is itself the result of a short chain over
     per-feature vectors and single values (the batch-norm scale gamma * rsqrt(var + eps)) is computed
@@ -1427,23 +1461,29 @@ def remove_dead_ops(ops, bufferpool, outvars):
     '''Drops launches none of whose results is read by a later launch or returned (the unused half
     of a PRNG key split, for instance). The reference runs every equation; the values returned
     are the same.'''
-    ops = list(ops)
-    while True:
+    while bufferpool.without_dead is not ops:
         uses = _use_counts(ops, bufferpool, outvars)
         #an accumulating kernel (scatter-add) also reads what it writes: such a use does not keep it alive
-        dead = [i for i, op in enumerate(ops)
+        dead = {i for i, op in enumerate(ops)
                 if _writes(op) and all(uses[id(b._placeholder)] - sum(1 for r in _reads(op) if r._placeholder is b._placeholder) == 0
                                        for b in _writes(op))
-                and not any(sum(1 for o in ops if any(w._placeholder is b._placeholder for w in _writes(o))) > 1 for b in _writes(op))]
+                and not any(sum(1 for o in ops if any(w._placeholder is b._placeholder for w in _writes(o))) > 1 for b in _writes(op))}
         if not dead:
-            return ops
+            bufferpool.without_dead = ops
+            break
         for i in dead:
             for b in _writes(ops[i]):
                 b._placeholder.elided = True
-        ops = [op for i, op in enumerate(ops) if i not in set(dead)]
+        ops = [op for i, op in enumerate(ops) if i not in dead]
+    return ops
 
 
 def _use_counts(ops, bufferpool, outvars):
+    '''How often every array is read by the ops of this list, two more for results of the program; not to be changed. Kept
+    until another list is asked about: the passes do not change the lists they are given.'''
+    counted, uses = bufferpool.use_counts
+    if counted is ops:
+        return uses
     uses = collections.Counter()
     for op in ops:
         for b in _reads(op):
@@ -1453,9 +1493,11 @@ def _use_counts(ops, bufferpool, outvars):
         if b is not None:
             uses[id(b._placeholder)] += 2
             b.accesses.pop()
+    bufferpool.use_counts = (ops, uses)
     return uses
 
 
+@_where(_is('threefry'))
 def fuse_random_streams(ops, bufferpool, outvars):
     '''Collapses the random-bits pipeline into one launch:
 
@@ -1468,7 +1510,7 @@ def fuse_random_streams(ops, bufferpool, outvars):
     The arithmetic per element is unchanged. A draw of an odd number of words n = 2h - 1 has c = concatenate(iota(n), 0) and drops
     the last of the bits, which the kernel does itself.'''
     from .ops import Op
-    uses = _use_counts(ops, bufferpool, outvars)
+    uses = collections.Counter(_use_counts(ops, bufferpool, outvars))      #(counted down below)
     pid  = lambda b: id(b._placeholder)
     writers = collections.defaultdict(list)          #placeholder id -> positions of the ops that write it
     for i, op in enumerate(ops):

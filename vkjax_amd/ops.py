@@ -102,6 +102,9 @@ def _without_transposed_gradients(jaxpr) -> tp.List:
     out like the weights. The copy goes away, and with it what kept the gradient's sum from storing the updated weights itself
     (see fusion.fuse_reduce_updates, where the measurements of both stand). A product that anything else reads keeps its layout.'''
     from .buffers import hashable
+    transposes = lambda eq: eq.primitive.name == 'transpose' and tuple(eq.params['permutation']) == (1, 0)
+    if not any(transposes(eq) for eq in jaxpr.eqns):
+        return jaxpr.eqns
     uses = collections.Counter(hashable(v) for eq in jaxpr.eqns for v in eq.invars)
     uses.update(hashable(v) for v in jaxpr.outvars)
     products, eqns = {}, list(jaxpr.eqns)
@@ -110,8 +113,7 @@ def _without_transposed_gradients(jaxpr) -> tp.List:
             (lc, rc), (lb, rb) = eq.params['dimension_numbers']
             if (tuple(lc), tuple(rc), tuple(lb), tuple(rb)) == ((0,), (0,), (), ()) and uses[hashable(eq.outvars[0])] == 1:
                 products[hashable(eq.outvars[0])] = i
-        elif (eq.primitive.name == 'transpose' and tuple(eq.params['permutation']) == (1, 0)
-              and hashable(eq.invars[0]) in products and not core.is_dropped(eq.outvars[0])):
+        elif transposes(eq) and hashable(eq.invars[0]) in products and not core.is_dropped(eq.outvars[0]):
             at      = products.pop(hashable(eq.invars[0]))
             product = eqns[at]
             #(this package's equations are named tuples, jax's have a method of their own)
