@@ -856,13 +856,19 @@ CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_steps, 2, 2, 2, 1, 3, true, true)
 // ---- short contractions -------------------------------------------------------------------------------------------------
 // Dense rows [M, K] with K <= 64: a product whose time is that of its result, and of the arrays its epilogue reads. A block holds the packed
 // kernel operand of 256 columns in LDS (96 KB) for good; its 12 waves take 32 rows each, by themselves, keep their parts in registers and walk
-// the columns. No barrier behind the first, nothing loaded twice, and while some waves of a SIMD wait for memory others multiply. The products
-// of a sum and their order are those of the kernels above: the same bits.
-// What bounds it: HBM, at 0.8 to 0.9 of a copy's rate. 200704 x 64 x 256 alone (replays, packing included) 86 -> 72 us, with a residual 113 -> 93 (67 us
+// the columns. No barrier behind the first, nothing loaded twice, and while some waves of a SIMD wait for memory others multiply.
+// Eight products of parts, not six (all but lo.lo, which is 2^-36 of the whole), and those of the two largest parts in a sum of their own: they are 16
+// bits long, so few of them are cut off where they are added, and the other seven are a 256th of them. The two sums meet in one addition that is
+// rounded. Errors against 64-bit sums, as a multiple of those of v_mfma_f32_32x32x2_f32, 64 terms of which 1, 2, 4, 16 and 64 are not zero: 1.00,
+// 0.83, 0.66, 0.45, 0.34 (all of six products in one sum: 1.37, 1.56, 1.65, 1.36, 0.76, and 1.04 for activations of which half are zero; six in
+// two sums: 1.03, 0.85, 0.68, 0.45, 0.35).
+// What bounds it: HBM, at 0.7 to 0.85 of a copy's rate. 200704 x 64 x 256 alone (replays, packing included) 77 -> 60 us, with a residual 103 -> 83 (67 us
 // of memory time; the fp32 tiles and those above load the rows once per 64 or 128 columns, and start and end a block for two k tiles), and with the
-// backward pass of a ReLU, which the fp32 tiles leave to a launch of its own, 189 -> 93. Holding the next tile's rows in registers too, with 8 waves
-// of 256 registers: 71, 97 and 95.
+// backward pass of a ReLU, which the fp32 tiles leave to a launch of its own, 179 -> 82. (Six products in one sum: 52, 80 and 79; six in two sums: 53, 81, 80.
+// Holding the next tile's rows in registers too, with 8 waves of 256 registers, was slower by 4 us with a residual.)
 constexpr int CONV_SHORT_ROWS = 32, CONV_SHORT_COLS = 256, CONV_SHORT_WAVES = 12;
+// (A part, B part) of the seven products beside the largest, the smallest first
+__device__ constexpr int CONV_SHORT_PA[7] = {2, 1, 2, 1, 1, 0, 0}, CONV_SHORT_PB[7] = {1, 2, 0, 0, 1, 1, 2};
 
 template <bool STEPS>
 __device__ __forceinline__ void conv_short_body(u32x4* __restrict__ Bs, float* __restrict__ Es, float* __restrict__ out, const float* __restrict__ x,
@@ -934,7 +940,7 @@ __device__ __forceinline__ void conv_short_body(u32x4* __restrict__ Bs, float* _
                 }
             }
             const u32x4* b_at = Bs + cb * KSTEPS * 192 + lane;
-            f32x16 sum = {};
+            f32x16 sum = {}, large = {};
 #pragma unroll
             for (int s = 0; s < KSTEPS; ++s) {
                 u32x4 bf[3];
@@ -942,11 +948,12 @@ __device__ __forceinline__ void conv_short_body(u32x4* __restrict__ Bs, float* _
                 for (int t = 0; t < 3; ++t) bf[t] = b_at[s * 192 + t * 64];
                 if (s & 1) FENCE();                         // (all of the columns' parts at once: registers would spill)
 #pragma unroll
-                for (int t = 0; t < 6; ++t)
-                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[s][CONV_SPLIT_PA[t]]), __builtin_bit_cast(bf16x8, bf[CONV_SPLIT_PB[t]]), sum, 0, 0, 0);
+                for (int t = 0; t < 7; ++t)
+                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[s][CONV_SHORT_PA[t]]), __builtin_bit_cast(bf16x8, bf[CONV_SHORT_PB[t]]), sum, 0, 0, 0);
+                large = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[s][0]), __builtin_bit_cast(bf16x8, bf[0]), large, 0, 0, 0);
             }
 #pragma unroll
-            for (int v = 0; v < 16; ++v) y[v] = sum[v] * (1.f / (CONV_SPLIT_SCALE * CONV_SPLIT_SCALE));
+            for (int v = 0; v < 16; ++v) y[v] = (sum[v] + large[v]) * (1.f / (CONV_SPLIT_SCALE * CONV_SPLIT_SCALE));
             // sums that are not finite: again with fp32 products, as above
             float high = 0.f;
 #pragma unroll

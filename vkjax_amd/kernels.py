@@ -1120,7 +1120,7 @@ CONV_SPLIT_TILES = {'128x128': (128, 128, 1.15, 1.15), '128x64': (128, 64, 0.65,
 CONV_PATCH_STEP, CONV_PATCH_START, CONV_PATCH_SLICE = {'128x128': 0.88, '128x64': 0.5}, 8, 16
 #Products below these stay with the fp32 kernels. Rows: packing the kernel operand costs what about 250 rows' products cost,
 #and one launch. Contraction: with two k tiles of 32 a block is all start-up and stores (12544 x 64 x 256 with residual 29
-#us here, 25 there; 200704 x 64 x 256 115, 113, and 93 where a block holds the kernel operand, _conv_short_pays; 50176 x 128 x 512: 59 against 61). Operations: start and end of two launches. A
+#us here, 25 there; 200704 x 64 x 256 115, 113, and 0.8 times that where a block holds the kernel operand, _conv_short_pays; 50176 x 128 x 512: 59 against 61). Operations: start and end of two launches. A
 #product alone is slower up to 2 GFLOP (8188 x 880 x 98, 1.4: 28.9 against 23.9; 20000 x 512 x 64, 1.3: 23.4, 21.6; 8192 x 512 x 256, 2.1: 23.0,
 #23.4), by the packing launch; in a network, where several layers' weights are packed by one launch, it is faster from 1 on, more so where
 #the backward pass of a ReLU is its epilogue (ResNet-50 with the line at 1, at 1.5 and at 2: batch 16 1566, 1583, 1623 us, batch 8 at 200 x 200 1092, 1119,
@@ -1178,9 +1178,9 @@ def conv_short_applies(g: ConvGeometry, c_contig: bool) -> bool:
 def _conv_short_pays(g: ConvGeometry) -> bool:
     '''Where those kernels are faster than any other.'''
     #(times of replays of a product with a residual behind its ReLU in microseconds, packing included, fp32 and here.) Columns: half lines of a width
-    #that is no multiple of 32 are requested twice (100000 x 48 x 300 92, 90, but 43000 x 64 x 300 49, 54; 1000000 x 64 x 65 in 128 x 128 tiles 244, 307), and
-    #below 96 there is little to walk (200704 x 64 x 64 46, 49). Features: 200704 x 40 x 256 112, 92, but without an epilogue 200704 x 32 x 256 60, 63.
-    #Results: 11.5 M 60000 x 64 x 192 41.5, 42.3; 12.8 M 100352 x 64 x 128 44, 46, 50176 x 64 x 256 43, 41; 19 M 150000 x 64 x 128 58, 55, 200704 x 64 x 96 78, 56
+    #that is no multiple of 32 are requested twice (43000 x 64 x 300 35, 41; 100000 x 48 x 300 80, 76), and below 96 there is little to walk (200704 x 64 x 64 32, 34). Features: 200704 x 36 x 256 101, 79, but without an epilogue 200704
+    #x 32 x 256 50, 57. Results: 10 M 40000 x 64 x 256 26, 29; 12.8 M 100352 x 64 x 128 31, 32; 17 M 65536 x 64 x 256 41, 34, 131072 x 64 x 128 40, 34, 8200 x
+    #64 x 2048 40, 36 (without an epilogue 30, 30); 19 M 200704 x 64 x 96 66, 42. With the backward pass of a ReLU half as long from 12 M on
     return g.N % 32 == 0 and g.N >= 96 and g.K > 32 and g.M * g.N >= 1 << 24
 
 
