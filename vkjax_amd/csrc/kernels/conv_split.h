@@ -162,6 +162,10 @@ __device__ __forceinline__ uint32_t conv_split_word(f32x4 (&x)[2], int t, int q)
 }
 // (A part, B part) of the six products of a k16 step, in their order
 __device__ constexpr int CONV_SPLIT_PA[6] = {2, 1, 1, 0, 0, 0}, CONV_SPLIT_PB[6] = {0, 0, 1, 1, 2, 0};
+// Where sums of few terms have to be as close to 64 bits as fp32 products give them: the seven products beside the largest, the smallest first. The largest,
+// of the two parts of 8 bits that come first, is summed for itself: such products are 16 bits long, so few bits are cut off where they are added,
+// and the others are a 256th of them. (Without the first two a sum of one term is 1.03 times as far off as its fp32 product.)
+__device__ constexpr int CONV_FINE_PA[7] = {2, 1, 2, 1, 1, 0, 0}, CONV_FINE_PB[7] = {1, 2, 0, 0, 1, 1, 2};
 
 // ---- the product ------------------------------------------------------------------------------------------------------
 // Block = WGM x WGN waves, each with TM x TN tiles of 32 x 32; k tile 32, i.e. two k16 steps, taken in pairs. A tile of the
@@ -201,10 +205,15 @@ __device__ constexpr int CONV_SPLIT_PA[6] = {2, 1, 1, 0, 0, 0}, CONV_SPLIT_PB[6]
 // 64 x 56 x 56 x 64 x 64 91.5 -> 78.0 us, 28 x 28 x 128 x 128 88.1 -> 74.2, 14 x 14 x 256 x 256 87.5 -> 73.5, 7 x 7 x 512 x 512 88.3 -> 79.0 (187 to 201 TFLOP/s);
 // 32 x 56 x 56 x 64 x 64 52.5 -> 44.9, 50 x 24 x 24 x 128 x 64 38.3 -> 25.6. ResNet-50 at batch 64 3.94 -> 3.83 ms, its training step 13.10 -> 12.82.
 // (The body of the loop has no branch: skipping the second item where a patch is short cost more in spilled registers than it saved.)
+// FINE: the eight products and two sums of CONV_FINE_PA, each sum with accumulators of its own, which meet behind the last slice. For products that the
+// fp32 kernels would compute: errors of 0.3 to 0.96 times theirs however few terms are not zero, 1.00 for sums of one term (with six products in one sum 1.2 to
+// 1.3 times where less than a tenth of the terms are not zero). A third more products and twice the accumulators, two blocks per CU: 64 x 56 x 56 x 64 x 32 68
+// -> 86 us (fp32 114), 33 x 7 x 7 x 512 x 512 55 -> 67 (101), 1 x 7 x 7 x 480 x 480 27 -> 32 (93).
 constexpr int CONV_PATCH_ROWS = 264, CONV_PATCH_ZEROS = 256;
 
-template <int WGM, int WGN, int TM, int TN>
-__device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* __restrict__ Es, float (&acc)[TM][TN][16], const uint32_t (&b_soff)[TN],
+template <int WGM, int WGN, int TM, int TN, bool FINE>
+__device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* __restrict__ Es, float (&acc)[TM][TN][16],
+                                                float (&acc_large)[FINE ? TM : 1][FINE ? TN : 1][16], const uint32_t (&b_soff)[TN],
                                                 const float* __restrict__ x, __amdgpu_buffer_rsrc_t w_rsrc, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
                                                 const ConvParams& P, const ConvDerived& Dk, int wave, int m0, int n0, int kbeg, int kend) {
     constexpr int BN = 32 * WGN * TN, NT = 64 * WGM * WGN, ROWS = CONV_PATCH_ROWS;
@@ -258,14 +267,21 @@ __device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* _
     auto load_b = [&](int step, int parity, int t, int j) {
         bf[parity][j][t] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, b_lane, b_soff[j] + (uint32_t)step * 3072u + t * 1024u, 0);
     };
-    f32x16 sum[TM * TN] = {};
+    f32x16 sum[TM * TN] = {}, large[FINE ? TM * TN : 1] = {};
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-    constexpr int CH = TM * TN, NS = 6 * CH, BARRIER = 6 * TN - 4;
+            for (int v = 0; v < 16; ++v) {
+                acc[i][j][v] = 0.f;
+                if constexpr (FINE) acc_large[i][j][v] = 0.f;
+            }
+    // products of a step, and behind which of them the parts 2, 1 and 0 of A have met their last
+    constexpr int NP = FINE ? 8 : 6, LAST[3] = {NP - 1, FINE ? 5 : 4, FINE ? 3 : 2};
+    constexpr int CH = TM * TN, NS = NP * CH, BARRIER = NP * (TN - 1) + LAST[2];
+    constexpr auto pa = [](int t) { return FINE ? t < 7 ? CONV_FINE_PA[t] : 0 : CONV_SPLIT_PA[t]; };
+    constexpr auto pb = [](int t) { return FINE ? t < 7 ? CONV_FINE_PB[t] : 0 : CONV_SPLIT_PB[t]; };
     // which of the two items' twelve pieces follows a product of the nine steps, -1: none. One item in registers: the second is requested when
     // the first has been taken apart, and has a step and a half to arrive.
     constexpr auto item_piece = [](int place) {
@@ -285,19 +301,25 @@ __device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* _
             FENCE();
 #pragma unroll
             for (int n = 0; n < NS; ++n) {
-                const int c = n / 6, t = n % 6, i = c / TN, j = c % TN;
+                const int c = n / NP, t = n % NP, i = c / TN, j = c % TN;
                 if (tap == 8 && n == BARRIER) { __syncthreads(); FENCE(); }
-                sum[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i][CONV_SPLIT_PA[t]]), __builtin_bit_cast(bf16x8, bf[parity][j][CONV_SPLIT_PB[t]]),
-                                                                 tap % 3 == 0 && t == 0 ? f32x16{} : sum[c], 0, 0, 0);
+                f32x16& to = FINE && t == NP - 1 ? large[FINE ? c : 0] : sum[c];
+                to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[i][pa(t)]), __builtin_bit_cast(bf16x8, bf[parity][j][pb(t)]),
+                                                             tap % 3 == 0 && (t == 0 || (FINE && t == NP - 1)) ? f32x16{} : to, 0, 0, 0);
                 // the chain before has seen its last product
-                if (tap % 3 == (c > 0 ? 2 : 0) && t >= 2) {
-                    const int pc = (c + CH - 1) % CH;
+                if (tap % 3 == (c > 0 ? 2 : 0) && t >= NP - 4) {
+                    const int pc = (c + CH - 1) % CH, v0 = 4 * (t - NP + 4);
 #pragma unroll
-                    for (int v = 4 * t - 8; v < 4 * t - 4; ++v) acc[pc / TN][pc % TN][v] = __builtin_fmaf(sum[pc][v], sign, acc[pc / TN][pc % TN][v]);
+                    for (int v = v0; v < v0 + 4; ++v) {
+                        acc[pc / TN][pc % TN][v] = __builtin_fmaf(sum[pc][v], sign, acc[pc / TN][pc % TN][v]);
+                        if constexpr (FINE) acc_large[pc / TN][pc % TN][v] = __builtin_fmaf(large[pc][v], sign, acc_large[pc / TN][pc % TN][v]);
+                    }
                 }
                 // parts of A that have met their last column are replaced by the next step's
-                if (j == TN - 1 && t == 2) find_a(next / 3, next % 3, i);
-                if (j == TN - 1 && (t == 2 || t == 4 || t == 5)) read_a(tap == 8 ? other : mine, next % 3, t == 2 ? 2 : t == 4 ? 1 : 0, i);
+                if (j == TN - 1 && t == LAST[2]) find_a(next / 3, next % 3, i);
+#pragma unroll
+                for (int q = 2; q >= 0; --q)
+                    if (j == TN - 1 && t == LAST[q]) read_a(tap == 8 ? other : mine, next % 3, q, i);
                 // an item of the next 16 features: its three parts, in halves, then the request of a later one
                 const int place = tap * NS + n, e = item_piece(place), h = e % 6, item = e / 6;
                 if (e >= 0) {
@@ -310,7 +332,7 @@ __device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* _
                 // the columns' parts of the next step but one
 #pragma unroll
                 for (int q = 0; q < TN; ++q)
-                    if (q < TN - 1 ? n == (CH - TN + q + 1) * 6 + 1 : n == NS - 1) {
+                    if (q < TN - 1 ? n == (CH - TN + q + 1) * NP + 1 : n == NS - 1) {
 #pragma unroll
                         for (int t2 = 0; t2 < 3; ++t2) load_b(9 * sixteen + tap + 2, parity, t2, q);
                     }
@@ -357,12 +379,16 @@ __device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* _
         nine_steps(std::integral_constant<int, 1>{}, sixteen + 1);
     }
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[TM - 1][TN - 1][v] = __builtin_fmaf(sum[CH - 1][v], sign, acc[TM - 1][TN - 1][v]);
+    for (int v = 0; v < 16; ++v) {
+        acc[TM - 1][TN - 1][v] = __builtin_fmaf(sum[CH - 1][v], sign, acc[TM - 1][TN - 1][v]);
+        if constexpr (FINE) acc_large[TM - 1][TN - 1][v] = __builtin_fmaf(large[CH - 1][v], sign, acc_large[TM - 1][TN - 1][v]);
+    }
     __syncthreads();
 }
 
 // STEPS: an epilogue other than the straight-line one, step by step (ReLU6, a scalar or a vector in another place, a residual that is subtracted).
-template <int WGM, int WGN, int TM, int TN, bool STEPS, bool PATCH>
+// FINE: products and sums of CONV_FINE_PA; a slice leaves both its sums.
+template <int WGM, int WGN, int TM, int TN, bool STEPS, bool PATCH, bool FINE>
 __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float* __restrict__ Es, int* __restrict__ Rs,
                                                 float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                                                 float* __restrict__ partial, uint32_t* __restrict__ arrivals, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
@@ -396,14 +422,15 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                                  w_rsrc = make_rsrc(w, P.w_bytes), o_rsrc = make_rsrc(out, P.out_bytes);
 
     const uint32_t rowb = (uint32_t)P.N * 4u;
-    float acc[TM][TN][16];
+    float acc[TM][TN][16], acc_large[FINE ? TM : 1][FINE ? TN : 1][16];
     uint32_t b_soff[TN];                             // the packed columns of this wave
     // (blocks of columns beyond the last one lie outside the descriptor and read as zeros)
 #pragma unroll
     for (int j = 0; j < TN; ++j) b_soff[j] = (uint32_t)(n0 / 32 + wn * TN + j) * (uint32_t)ksteps * 3072u;
     if constexpr (PATCH) {
-        conv_patch_sums<WGM, WGN, TM, TN>(pool, Es, acc, b_soff, x, w_rsrc, epi, Dp, P, Dk, wave, m0, n0, kbeg, kend);
+        conv_patch_sums<WGM, WGN, TM, TN, FINE>(pool, Es, acc, acc_large, b_soff, x, w_rsrc, epi, Dp, P, Dk, wave, m0, n0, kbeg, kend);
     } else {
+    static_assert(!FINE, "only with a patch");
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
     // ---- load assignment: A item = (row, octet of k); octet o holds k = 4o..4o+3 and 16+4o..16+4o+3 of the k tile
     constexpr int A_NI = BM * 4 / NT, A_RSTEP = NT / 4;
@@ -579,16 +606,23 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     if (sliced) {
         // store this slice's sums; the block that arrives last adds all of them, in the order of the slices
         const int mine = tile - whole;
-        const uint32_t tile_bytes = BM * BN * 4;
+        constexpr int SUMS = FINE ? 2 : 1;
+        const uint32_t tile_bytes = BM * BN * 4 * SUMS;
         const __amdgpu_buffer_rsrc_t p_rsrc = make_rsrc(reinterpret_cast<char*>(partial) + (size_t)mine * slices * tile_bytes, (uint32_t)slices * tile_bytes);
+        auto each = [&](auto&& fn) {                              // fn(four of this lane's sums, their place in a slice)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+                for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; v += 4)
-                    buffer_store_x4_agent(f32x4{acc[i][j][v], acc[i][j][v + 1], acc[i][j][v + 2], acc[i][j][v + 3]}, p_rsrc,
-                                          (uint32_t)tid * 16u, (uint32_t)slice * tile_bytes + (uint32_t)((i * TN + j) * 4 + v / 4) * (NT * 16u));
+                    for (int v = 0; v < 16; v += 4) {
+                        fn(&acc[i][j][v], (uint32_t)((i * TN + j) * 4 + v / 4) * (NT * 16u));
+                        if constexpr (FINE) fn(&acc_large[i][j][v], (uint32_t)((TM * TN + i * TN + j) * 4 + v / 4) * (NT * 16u));
+                    }
+        };
+        each([&](float* four, uint32_t place) {
+            buffer_store_x4_agent(f32x4{four[0], four[1], four[2], four[3]}, p_rsrc, (uint32_t)tid * 16u, (uint32_t)slice * tile_bytes + place);
+        });
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the stores above have reached memory
         __syncthreads();
         if (tid == 0) {
@@ -598,24 +632,25 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         }
         __syncthreads();
         if (Rs[0] + 1 != slices) return;
+        each([&](float* four, uint32_t) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) four[u] = 0.f;
+        });
+#pragma nounroll
+        for (int s = 0; s < slices; ++s)
+            each([&](float* four, uint32_t place) {
+                const f32x4 q = buffer_load_x4_agent(p_rsrc, (uint32_t)tid * 16u, (uint32_t)s * tile_bytes + place);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) four[u] += q[u];
+            });
+    }
+    if constexpr (FINE) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-#pragma nounroll
-        for (int s = 0; s < slices; ++s)
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int v = 0; v < 16; v += 4) {
-                        const f32x4 q = buffer_load_x4_agent(p_rsrc, (uint32_t)tid * 16u, (uint32_t)s * tile_bytes + (uint32_t)((i * TN + j) * 4 + v / 4) * (NT * 16u));
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) acc[i][j][v + u] += q[u];
-                    }
+                for (int v = 0; v < 16; ++v) acc[i][j][v] += acc_large[i][j][v];
     }
 
     // Sums that are not finite are computed again with fp32 products. The others beside them stay as they are, so a row's results do not
@@ -830,28 +865,31 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         }
 }
 
-#define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE, STEPS, PATCH)                                                         \
+#define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE, STEPS, PATCH, FINE)                                                   \
     extern "C" __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void name(             \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                                   \
         float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) { \
         __shared__ __attribute__((aligned(16))) u32x4 pool[PATCH ? 12 * CONV_PATCH_ROWS : 24 * 32 * WGM * TM];               \
         __shared__ float Es[CONV_MAX_EPI * 32 * WGN * TN];                                                                   \
         __shared__ int Rs[32 * WGM * TM];                                                                                    \
-        conv_split_body<WGM, WGN, TM, TN, STEPS, PATCH>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);          \
+        conv_split_body<WGM, WGN, TM, TN, STEPS, PATCH, FINE>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);    \
     }
 // _steps: 50176 x 128 x 512 with a ReLU6 68 us, with a scalar 62, with `relu(y) + r` 82 (each as launches of its own behind the product: 83, 82, 94;
 // in the fp32 kernels 73, 71, 73); 50176 x 256 x 512 97, 89, 108 (127, 120, 130). (Words of a full tensor requested for two tiles at a time
 // instead of one: 80 instead of 82, not kept; for four: registers spill.)
 // (2 x 2 waves of 64 x 64: 255 registers, two blocks per CU; 1 x 4 waves of 128 x 32, which load every column once, were 1 % slower)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x128, 2, 2, 2, 2, 2, false, false)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x128_patch, 2, 2, 2, 2, 2, false, true)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x128_steps, 2, 2, 2, 2, 2, true, false)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x128_patch_steps, 2, 2, 2, 2, 2, true, true)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128, 2, 2, 2, 2, 2, false, false, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128_patch, 2, 2, 2, 2, 2, false, true, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128_steps, 2, 2, 2, 2, 2, true, false, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x128_patch_steps, 2, 2, 2, 2, 2, true, true, false)
 // for at most 64 columns, or where the smaller tile divides the rows better among the CUs: three blocks per CU
-CONV_SPLIT_KERNEL(conv_gemm_split_128x64, 2, 2, 2, 1, 3, false, false)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch, 2, 2, 2, 1, 3, false, true)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x64_steps, 2, 2, 2, 1, 3, true, false)
-CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_steps, 2, 2, 2, 1, 3, true, true)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64, 2, 2, 2, 1, 3, false, false, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch, 2, 2, 2, 1, 3, false, true, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_steps, 2, 2, 2, 1, 3, true, false, false)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_steps, 2, 2, 2, 1, 3, true, true, false)
+// (242 registers: two blocks per CU)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_fine, 2, 2, 2, 1, 2, false, true, true)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_fine_steps, 2, 2, 2, 1, 2, true, true, true)
 
 // ---- short contractions -------------------------------------------------------------------------------------------------
 // Dense rows [M, K] with K <= 64: a product whose time is that of its result, and of the arrays its epilogue reads. A block holds the packed
@@ -867,8 +905,6 @@ CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_steps, 2, 2, 2, 1, 3, true, true)
 // backward pass of a ReLU, which the fp32 tiles leave to a launch of its own, 179 -> 82. (Six products in one sum: 52, 80 and 79; six in two sums: 53, 81, 80.
 // Holding the next tile's rows in registers too, with 8 waves of 256 registers, was slower by 4 us with a residual.)
 constexpr int CONV_SHORT_ROWS = 32, CONV_SHORT_COLS = 256, CONV_SHORT_WAVES = 12;
-// (A part, B part) of the seven products beside the largest, the smallest first
-__device__ constexpr int CONV_SHORT_PA[7] = {2, 1, 2, 1, 1, 0, 0}, CONV_SHORT_PB[7] = {1, 2, 0, 0, 1, 1, 2};
 
 template <bool STEPS>
 __device__ __forceinline__ void conv_short_body(u32x4* __restrict__ Bs, float* __restrict__ Es, float* __restrict__ out, const float* __restrict__ x,
@@ -949,7 +985,7 @@ __device__ __forceinline__ void conv_short_body(u32x4* __restrict__ Bs, float* _
                 if (s & 1) FENCE();                         // (all of the columns' parts at once: registers would spill)
 #pragma unroll
                 for (int t = 0; t < 7; ++t)
-                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[s][CONV_SHORT_PA[t]]), __builtin_bit_cast(bf16x8, bf[CONV_SHORT_PB[t]]), sum, 0, 0, 0);
+                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[s][CONV_FINE_PA[t]]), __builtin_bit_cast(bf16x8, bf[CONV_FINE_PB[t]]), sum, 0, 0, 0);
                 large = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[s][0]), __builtin_bit_cast(bf16x8, bf[0]), large, 0, 0, 0);
             }
 #pragma unroll

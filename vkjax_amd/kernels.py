@@ -50,7 +50,7 @@ class _Choices:
         conv_stem=None,                  #the patch kernel for few input features: False = never; None / True: where it applies; 64: its 64-position tiles only
         conv_split=None,                 #the kernels on the bf16 matrix cores: None = where they pay, False = never, True or a tile's name = wherever they apply
         conv_split_slices=None,          #blocks that share a tile behind the whole rounds (None: by the estimate)
-        conv_patch=None,                 #the bf16 kernels that hold a patch of the input in LDS: None = wherever they apply (a pinned conv_split: never), True = wherever they apply, False = never
+        conv_patch=None,                 #the bf16 kernels that hold a patch of the input in LDS: None = wherever they pay (a pinned conv_split: never), True = wherever they apply, 'fine' = wherever they apply, with their two sums, False = never
         conv_short=None,                 #the bf16 kernels for dense rows of at most 64 features: None = where they pay (a pinned conv_split: never), True = wherever they apply, False = never
         wgrad_split=None,                #kernel gradients on the bf16 matrix cores: None = where they pay, False = never, a tile's name = wherever it applies
         wgrad_slices=None,               #slices of a kernel gradient's contraction (None: by the estimate)
@@ -1117,7 +1117,7 @@ CONV_SPLIT_TILES = {'128x128': (128, 128, 1.15, 1.15), '128x64': (128, 64, 0.65,
 #tile -> microseconds of a CU per k tile of 32 for the kernels that hold a patch of the input in LDS, and what a block's start and end cost, and those
 #of a slice, in k tiles. (Products alone, 128x64 and 128x128: 64 x 28 x 28 x 128 x 128 74.7 in 832 blocks and 75.9, 64 x 14 x 14 x 256 x 256 78.7, 75.2, 64 x 7 x 7
 #x 512 x 512 80.1, 78.1 in 200 blocks, 16 x 7 x 7 x 512 x 512 73.9 in 56 blocks, 41.8 in 112, 29.2 in 224; 119, 66, 41.)
-CONV_PATCH_STEP, CONV_PATCH_START, CONV_PATCH_SLICE = {'128x128': 0.88, '128x64': 0.5}, 8, 16
+CONV_PATCH_STEP, CONV_PATCH_START, CONV_PATCH_SLICE = {'128x128': 0.88, '128x64': 0.5, 'fine': 0.65}, 8, 16
 #Products below these stay with the fp32 kernels. Rows: packing the kernel operand costs what about 250 rows' products cost,
 #and one launch. Contraction: with two k tiles of 32 a block is all start-up and stores (12544 x 64 x 256 with residual 29
 #us here, 25 there; 200704 x 64 x 256 115, 113, and 0.8 times that where a block holds the kernel operand, _conv_short_pays; 50176 x 128 x 512: 59 against 61). Operations: start and end of two launches. A
@@ -1141,6 +1141,7 @@ class ConvSplit(tp.NamedTuple):
     partial: tp.Optional[Buffer] = None
     arrivals: tp.Optional[Buffer] = None
     patch: bool = False               #by the kernels that hold a patch of the input in LDS (conv_patch_applies)
+    fine: bool = False                #... by the one with two sums (_conv_patch_pays)
     short: bool = False               #by the kernels that hold the kernel operand in LDS (conv_short_applies)
 
 
@@ -1152,7 +1153,7 @@ def conv_split_tiles(split: ConvSplit, g: ConvGeometry) -> tp.Tuple[int, int]:
 def conv_split_partial_words(split: ConvSplit, g: ConvGeometry) -> int:
     bm, bn = CONV_SPLIT_TILES[split.tile][:2]
     tiles_m, tiles_n = conv_split_tiles(split, g)
-    return (tiles_m * tiles_n - split.whole) * split.slices * bm * bn
+    return (tiles_m * tiles_n - split.whole) * split.slices * bm * bn * (2 if split.fine else 1)
 
 
 def conv_split_packed_words(g: ConvGeometry) -> int:
@@ -1185,15 +1186,19 @@ def _conv_short_pays(g: ConvGeometry) -> bool:
 
 
 def _conv_patch_pays(g: ConvGeometry, c_contig: bool) -> bool:
-    '''Where the kernels that hold a patch are faster, packing included, than the fp32 kernels (images x H x W x features x columns: there, here).'''
+    '''Products that stay with the fp32 kernels otherwise: where the kernel that holds a patch and keeps two sums, whose errors are no larger than
+    theirs however few of a sum's terms are not zero, is faster than they are, packing included (images x H x W x features x columns: there, here).'''
     flops = 2 * g.M * g.N * g.K
+    #16 x 7 x 7 x 512 x 512 (3.7 GFLOP) 48, 45; 33 x 7 x 7 x 512 x 512 101, 67; 64 x 56 x 56 x 64 x 32 114, 86; but 18 x 6 x 6 x 512 x 512 (3.1) 48, 49; 8 x 7 x 7 x 512
+    #x 512 (1.9) 31, 38; of 32 features 32 x 56 x 56 x 32 x 32 26, 32
+    if flops >= 3.5e9:
+        return g.K >= 576
+    #four waves that share a contraction are as fast or faster: 4 x 28 x 28 x 128 x 128 16, 23; 8 x 14 x 14 x 256 x 256 27, 32; 10 x 10 x 10 x 320 x 320 33, 35
     if _four_waves_per_tile(g, True, c_contig, CONV_SPLIT_ROUND):
-        #4 x 28 x 28 x 128 x 128 (0.9 GFLOP) 17.6, 19.1; 8 x 14 x 14 x 256 x 256 (1.8) 28.8, 25.1; 8 x 7 x 7 x 512 x 512 32.2, 29.9; 16 x 7 x 7 x 512 x 512 51.4, 36.9
-        return flops >= 1.8e9
-    #one wave walks the whole contraction there: 1 x 7 x 7 x 96 x 96 21.4, 14.9; 1 x 10 x 10 x 160 x 40 33.4, 15.5; 1 x 7 x 7 x 480 x 480 93, 28; 4 x 56 x 56 x 64 x 64 17.2,
-    #16.9; 64 x 56 x 56 x 64 x 32 114, 71. The shortest, 32 features: 9 x 30 x 30 x 100 columns (0.47 GFLOP) 11.0, 12.7; 20 x 30 x 30 x 64 (0.66) 16.6, 12.8; 8 x 56 x 56 x 48
-    #(0.69) 15.8, 13.0; of at most 32 columns 64 x 28 x 28 x 24 16.4, 17.2; 32 x 56 x 56 x 32 26.6, 27.5
-    return g.K >= 576 or (g.N > 32 and flops >= 0.6e9)
+        return False
+    #one wave walks the whole contraction there: 1 x 7 x 7 x 480 x 480 93, 32; 3 x 13 x 13 x 224 x 224 45, 25; 1 x 10 x 10 x 160 x 40 33, 18; 1519 rows x 160 x 308 35, 32;
+    #of 96 features 1 x 7 x 7 x 96 x 96 21, 17; 2673 rows x 96 x 97 (84 tiles) 22, 20, 3600 x 96 x 96 (114) 22, 22, 16200 x 96 x 32 22, 26; of 64 4 x 56 x 56 x 64 x 64 16, 21
+    return g.K >= 1440 or (g.K >= 864 and _cdiv(g.M, 64) * _cdiv(g.N, 64) <= 96)
 
 
 def _conv_split_pays(g: ConvGeometry, c_contig: bool) -> bool:
@@ -1232,14 +1237,16 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
     wanted = CHOICES.conv_split is None and CHOICES.conv_split_slices is None if CHOICES.conv_short is None else CHOICES.conv_short
     if wanted and conv_short_applies(g, c_contig) and (CHOICES.conv_short or _conv_short_pays(g)):
         return ConvSplit('128x64', _cdiv(M, 128) * _cdiv(N, 64), 1, short=True)
-    if not (CHOICES.conv_split or CHOICES.conv_split_slices) and not (_conv_patch_pays if patch else _conv_split_pays)(g, c_contig):
+    pays  = _conv_split_pays(g, c_contig)
+    fine  = patch and (CHOICES.conv_patch == 'fine' or (CHOICES.conv_patch is None and not pays))
+    if not (CHOICES.conv_split or CHOICES.conv_split_slices or CHOICES.conv_patch == 'fine') and not (_conv_patch_pays(g, c_contig) if fine else pays):
         return None
     #The whole tiles are dealt out in rounds of one per CU; the contraction of those of the last, incomplete round (or of all,
     #if there are fewer tiles than CUs) may be cut into slices, of two k tiles at least. A block's start and end cost about
     #three k tiles, a slice's partial sums five more (a patch has to be complete before the first product: eight).
     ktiles, best = K // 32 if patch else 2 * _cdiv(K, 64), None
     for tile, (bm, bn, shared_step, lone_step) in CONV_SPLIT_TILES.items():
-        if CHOICES.conv_split not in (None, True, tile):
+        if CHOICES.conv_split not in (None, True, tile) or (fine and tile != '128x64'):
             continue
         tiles = _cdiv(M, bm) * _cdiv(N, bn)
         for slices in range(1, 17):
@@ -1248,11 +1255,11 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
                 continue
             blocks = whole + (tiles - whole) * slices
             rounds = whole / CONV_SPLIT_ROUND if slices > 1 else _cdiv(tiles, CONV_SPLIT_ROUND)
-            step   = CONV_PATCH_STEP[tile] if patch else shared_step if blocks > CONV_SPLIT_ROUND else lone_step
+            step   = CONV_PATCH_STEP['fine' if fine else tile] if patch else shared_step if blocks > CONV_SPLIT_ROUND else lone_step
             start, slice_start = (CONV_PATCH_START, CONV_PATCH_SLICE) if patch else (3, 8)
             time   = step * (rounds * (ktiles + start) + _cdiv((tiles - whole) * slices, CONV_SPLIT_ROUND) * (ktiles / slices + slice_start))
             if best is None or time < best[0]:
-                best = (time, ConvSplit(tile, whole, slices, patch=patch))
+                best = (time, ConvSplit(tile, whole, slices, patch=patch, fine=fine))
     return best[1] if best else None
 
 
@@ -1303,7 +1310,7 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
     (tiles_m, tiles_n), kpairs = conv_split_tiles(split, g), g.Cin // 32 if split.patch else _cdiv(K, 64)
     assert not split.patch or conv_patch_applies(g)
     shared = tiles_m * tiles_n - split.whole
-    blocks, threads, kernel = split.whole + shared * split.slices, 256, f'conv_gemm_split_{split.tile}' + ('_patch' if split.patch else '')
+    blocks, threads, kernel = split.whole + shared * split.slices, 256, f'conv_gemm_split_{split.tile}' + ('_patch' if split.patch else '') + ('_fine' if split.fine else '')
     if split.short:
         assert conv_short_applies(g, c_contig) and flat_rows
         #one block per CU for at most 256 columns, its waves walk the tiles of 32 rows
