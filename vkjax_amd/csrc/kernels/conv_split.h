@@ -797,7 +797,6 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
     for (int t = 1; t < CONV_MAX_EPI; ++t) full_ptr = epi_first_full == t ? epi.p[t] : full_ptr;
     const __amdgpu_buffer_rsrc_t f_rsrc = make_rsrc(full_ptr, P.out_bytes);
     const uint32_t slots = (P.flags >> 20) & 31u;
-    const int e_mul = __builtin_popcount(slots & 1u), e_add = __builtin_popcount(slots & 3u), e_max = __builtin_popcount(slots & 15u);
     const int tap = (int)((P.flags >> 12) & 15u) - 1;
     // The epilogue of a backward pass: + full tensor (operand 0), kept where an activation (operand 1) lies above a limit (3) and
     // replaced by a constant (4) elsewhere, stored as a second result, * vector (2). The launches it replaces moved four to six times
@@ -835,32 +834,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                 sub_tile(i, j, [&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], o_rsrc, vo, so); });
                 continue;
             }
-            if (tap == 0) tap_store();
-            if (slots & 1u) {
-                const float o = Es[col];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = y[v] - o;
-                if (tap == 1) tap_store();
-            }
-            if (slots & 2u) {
-                const float o = Es[e_mul * BN + col];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = y[v] * o;
-            }
-            if (slots & 4u) {
-                const float o = Es[e_add * BN + col];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = y[v] + o;
-            }
-            if (slots & 8u) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = y[v] + ov[v];
-            }
-            if (slots & 16u) {
-                const float o = Es[e_max * BN + col];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = (y[v] > o || y[v] != y[v]) ? y[v] : o;
-            }
+            conv_straight_steps<16>(y, ov, slots, tap, Es, BN, col, tap_store);
             sub_tile(i, j, [&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], o_rsrc, vo, so); });
         }
 }
@@ -921,7 +895,6 @@ __device__ __forceinline__ void conv_short_body(u32x4* __restrict__ Bs, float* _
     const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(x, P.x_bytes), w_rsrc = make_rsrc(w, P.w_bytes), o_rsrc = make_rsrc(out, out_bytes);
     const int nepi = (P.flags >> 8) & 15u, epi_first_full = (int)((P.flags >> 16) & 15u) - 1;
     const uint32_t slots = (P.flags >> 20) & 31u;
-    const int e_mul = __builtin_popcount(slots & 1u), e_add = __builtin_popcount(slots & 3u), e_max = __builtin_popcount(slots & 15u);
     const int tap = (int)((P.flags >> 12) & 15u) - 1;
     const bool masked_form = P.flags & CONV_SPLIT_MASKED;
     const float* full_ptr = epi.p[0];
@@ -1057,32 +1030,7 @@ __device__ __forceinline__ void conv_short_body(u32x4* __restrict__ Bs, float* _
                 store(o_rsrc);
                 continue;
             }
-            if (tap == 0) store(t_rsrc);
-            if (slots & 1u) {
-                const float o = Es[col];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = y[v] - o;
-                if (tap == 1) store(t_rsrc);
-            }
-            if (slots & 2u) {
-                const float o = Es[e_mul * COLS + col];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = y[v] * o;
-            }
-            if (slots & 4u) {
-                const float o = Es[e_add * COLS + col];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = y[v] + o;
-            }
-            if (slots & 8u) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = y[v] + ov[v];
-            }
-            if (slots & 16u) {
-                const float o = Es[e_max * COLS + col];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = (y[v] > o || y[v] != y[v]) ? y[v] : o;
-            }
+            conv_straight_steps<16>(y, ov, slots, tap, Es, COLS, col, [&]() { store(t_rsrc); });
             store(o_rsrc);
         }
     }
