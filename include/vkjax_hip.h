@@ -101,7 +101,8 @@ int vkj_buf_download(vkj_handle ctx, vkj_handle buf, size_t offset, void* host, 
 int vkj_seq_create(vkj_handle ctx, int profiling, vkj_handle* seq);
 int vkj_seq_destroy(vkj_handle seq);
 /* seq.record(kp.OpTensorSyncDevice([...]))  reference: vkjax/kompute_jaxpr_interpreter.py:51-53
- * `slot` indexes the host_ptrs array given to vkj_seq_eval. */
+ * `slot` indexes the host_ptrs array given to vkj_seq_eval. Bytes of a buffer that no upload of an evaluation
+ * covers keep their contents; of two uploads that overlap, the one recorded last stays. */
 int vkj_seq_record_upload(vkj_handle seq, vkj_handle buf, size_t offset, int slot, size_t nbytes);
 /* mgr.algorithm(tensors, spirv, workgroup) + seq.record(kp.OpAlgoDispatch(algo))
  *                                     reference: vkjax/kompute_jaxpr_interpreter.py:55-60

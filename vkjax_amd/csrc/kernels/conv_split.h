@@ -14,6 +14,7 @@
 // Measured against 64-bit sums (4096 x K x 128, normal data): an error of 0.76, 0.56 and 0.30 times that of
 // v_mfma_f32_32x32x2_f32 at K = 64, 576 and 2304 (which rounds after every second product, this after every sixteenth). Sums of which less than
 // a fifth of the terms are not zero are further off than those: 1.3 times at 16 of 512, 1.4 times at one (which is cut off, not rounded).
+// The kernels that serve products the fp32 kernels would be nearly as fast at (_short, _fine) are not: see CONV_FINE_PA.
 #pragma once
 #include "split_bf16.h"
 

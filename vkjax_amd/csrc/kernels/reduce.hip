@@ -570,9 +570,9 @@ SCALE_RELU_BACKWARD_KERNEL(scale_relu_backward_v4, 4, true)
 SCALE_RELU_BACKWARD_KERNEL(scale_backward_v1, 1, false)
 SCALE_RELU_BACKWARD_KERNEL(scale_backward_v4, 4, false)
 // m itself and its column sums (a dense layer's ReLU: the sums are its bias gradient). Memory bounds it from some MB on: 65536 x 256
-// 52 us as two launches, 43 as one. Below that the launches do; the step of a 784-300-100-10 network over 1000 rows has two of
-// these, and with them, the sign behind its loss's mean, its known scalars and one batch for all its updates it takes 114 us
-// in 16 launches (128 us in 21).
+// 52 us as two launches, 43 as one; below that the launches do (127 x 256 14.6, 5.4). For gradients that are results, and for sums of more rows than one
+// launch takes: the sums of a training step over at most 1536 rows store the updated biases (reduce_cols_fsum_update), and the select in front of
+// them is a launch of its own.
 #define RELU_BACKWARD_KERNEL(name, VEC)                                                                                     \
     extern "C" __global__ __launch_bounds__(256) void name(float* m, float* sum_m, const float* ans, const float* thr,     \
                                                            const float* g, const float* alt, ReduceParams P) {             \

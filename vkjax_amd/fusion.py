@@ -1071,9 +1071,11 @@ def fuse_relu_backward_sums(ops, bufferpool, outvars):
         m = select(ans > t, g, z) ; db = sum_rows(m)
 
     become ONE launch that writes m and the column sums (their first stage, when they are split over row ranges), in the order
-    of the launch it replaces. It runs behind the passes that take the select into a product's epilogue. No line by size: the
-    launch has the grid of the sum, and replays of the pair took as long or longer at every size that was timed (127 x 256
-    14.6 -> 5.4 us, 1000 x 300 18.4 -> 15.3, 1000 x 7 15.2 -> 15.4, 65536 x 256 52.4 -> 42.9, 100000 x 33 30.4 -> 29.4).'''
+    of the launch it replaces. It runs behind the passes that take the select into a product's epilogue and those that let an
+    unsplit sum store an updated parameter: what is left are gradients that are results of the program and, in a training step, sums of
+    more rows than one launch takes. No line by size: the launch has the grid of the sum, and replays of the pair alone took as long or
+    longer at every size that was timed (127 x 256 14.6 -> 5.4 us, 1000 x 300 18.4 -> 15.3, 1000 x 7 15.2 -> 15.4, 65536 x 256 52.4 ->
+    42.9, 100000 x 33 30.4 -> 29.4).'''
     from .ops import Op
     pid = lambda b: id(b._placeholder)
     selects = {pid(op.chain.out): i for i, op in enumerate(ops) if _select_by_threshold(op.chain)}
