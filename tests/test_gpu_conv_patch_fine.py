@@ -97,3 +97,15 @@ def test_where_it_is_taken(xs, columns, kernel):
     interp = JaxprInterpreter(mj.make_jaxpr(conv)(zeros(*xs), zeros(3, 3, xs[3], columns)), plan_only=True)
     names  = [l.kernel for l in interp.launches if l.kernel.startswith('conv_gemm')]
     assert names == [kernel] if kernel else '_split' not in names[0], names
+
+
+def test_pinned_to_the_patch_kernels():
+    '''Plan only: wherever they apply, and nowhere else.'''
+    zeros = lambda *s: np.broadcast_to(np.float32(0), s)
+    pointwise = lambda x, k: lax.conv_general_dilated(x, k, (1, 1), 'VALID', dimension_numbers=('NHWC', 'HWIO', 'NHWC'))
+    for choice, kernel in ((True, '_patch'), ('fine', '_patch_fine')):
+        with K.overrides(conv_patch=choice):
+            for f, window, expected in ((conv, 3, kernel), (pointwise, 1, None)):
+                interp = JaxprInterpreter(mj.make_jaxpr(f)(zeros(2, 14, 14, 64), zeros(window, window, 64, 64)), plan_only=True)
+                name,  = [l.kernel for l in interp.launches if l.kernel.startswith('conv_gemm')]
+                assert name.endswith(expected) if expected else '_split' not in name, name

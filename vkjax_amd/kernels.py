@@ -1239,7 +1239,7 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
         return ConvSplit('128x64', _cdiv(M, 128) * _cdiv(N, 64), 1, short=True)
     pays  = _conv_split_pays(g, c_contig)
     fine  = patch and (CHOICES.conv_patch == 'fine' or (CHOICES.conv_patch is None and not pays))
-    if not (CHOICES.conv_split or CHOICES.conv_split_slices or CHOICES.conv_patch == 'fine') and not (_conv_patch_pays(g, c_contig) if fine else pays):
+    if not (CHOICES.conv_split or CHOICES.conv_split_slices or (patch and CHOICES.conv_patch)) and not (_conv_patch_pays(g, c_contig) if fine else pays):
         return None
     #The whole tiles are dealt out in rounds of one per CU; the contraction of those of the last, incomplete round (or of all,
     #if there are fewer tiles than CUs) may be cut into slices, of two k tiles at least. A block's start and end cost about
