@@ -35,6 +35,7 @@
 #include "common.h"
 
 #define CONV_MAX_EPI 6
+#define CONV_MAX_SHARES 8        // blocks that share a tile of the four-waves-per-tile kernels and add their sums themselves
 #define CONV_OOB 0x80000000u     // byte offset beyond any descriptor: loads give 0, stores are dropped
 
 enum EwOpConv : uint32_t {
@@ -77,9 +78,10 @@ struct ConvParams {
     int32_t os_b, os_h, os_w, os_n; // out strides
     int32_t split_tiles_m;          // mixed kernels only: the first split_tiles_m M tiles (of 64 rows) are computed as 64 x 64
                                     // tiles, the rows behind them as 32 x 32 tiles by the blocks that follow in the grid
-    int32_t k_split_steps;          // four-waves-per-tile kernels only: 0, or the k steps (of 128) one block sums. The grid then holds
+    int32_t k_split_steps;          // four-waves-per-tile kernels only: 0, or the k steps one block sums. The grid then holds
                                     // ceil(k steps / k_split_steps) blocks per tile; those of slice s store their sums, without an
-                                    // epilogue, to the s-th [M, N] matrix behind out, and a later launch adds the slices
+                                    // epilogue, to the s-th [M, N] matrix behind out, and a later launch adds the slices (kernels named
+                                    // _shared: to `partial`, and the block that arrives last adds them)
     int32_t m_blocks;               // lean kernels: 0, or the number of blocks that share the M tiles of one N tile as evenly as whole
                                     // tiles allow: every block takes m_each = tiles_m / m_blocks consecutive tiles, the first
                                     // m_extra = tiles_m % m_blocks blocks one more; the M tiles per block in the flags are then
@@ -96,6 +98,14 @@ struct ConvParams {
     //     m_extra of them one more
     //   (kernels named _short: tiles_m tiles of 32 rows, tiles_n groups of m_each blocks of 32 columns; split_tiles_m and m_blocks unused)
 };
+
+// stores and loads that are seen by every workgroup of the GPU, whichever L2 it stands behind (agent scope)
+__device__ __forceinline__ void buffer_store_x4_agent(f32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, soff, 16);
+}
+__device__ __forceinline__ f32x4 buffer_load_x4_agent(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 16));
+}
 
 // The part of the output a block's tile number refers to: a grid of tiles_m x tiles_n tiles whose first row is
 // m_base, handed to the blocks from first_block on.
@@ -208,10 +218,11 @@ __device__ __forceinline__ void conv_straight_steps(float (&y)[NV], const float 
 // registers, and with them resident waves, even when not taken): both operands on the 16-byte
 // path, k tiles that never straddle kernel taps, a row-major result, an epilogue that fits the
 // straight-line template.
-template <int WGM, int WGN, int TM, int TN, int BK, bool A_FAST, bool B_FAST, bool LEAN, int KSW = 1>
+template <int WGM, int WGN, int TM, int TN, int BK, bool A_FAST, bool B_FAST, bool LEAN, int KSW = 1, bool SHARED = false>
 __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const ConvRegion region, float* __restrict__ out, const float* __restrict__ x,
                                                const float* __restrict__ w, const ConvEpiPtrs& epi,
-                                               const ConvDerivedPtrs& Dp, const ConvParams& Pk, const ConvDerived& Dk) {
+                                               const ConvDerivedPtrs& Dp, const ConvParams& Pk, const ConvDerived& Dk,
+                                               float* __restrict__ partial = nullptr, uint32_t* __restrict__ arrivals = nullptr) {
     // KSW > 1: KSW groups of WGM x WGN waves share one block tile, each taking a 1/KSW slice of every k
     // step; their accumulators are added through LDS before the epilogue. For products whose handful of
     // tiles would otherwise leave most of a CU's four MFMA units idle (a wave can drive only one).
@@ -279,15 +290,19 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
     // K_SPLIT kernels can share a tile's contraction among several blocks (for products with so few tiles that most
     // CUs would stay idle while a few fetch all the weights): slice s sums k steps [kbase, kbase + ktiles)
     constexpr bool K_SPLIT = KSW > 1 && BK == 128;
+    static_assert(!SHARED || K_SPLIT, "shared are tiles whose k steps four waves take");
     int kbase = 0, ktiles = max(1, (P.K + BK - 1) / BK);       // K = 0 runs as one k step whose loads are all out of range
+    int slice = 0, slices = 1;
     if constexpr (K_SPLIT) {
         const int per = Pk.k_split_steps;
         if (per > 0) {
-            const int tiles = chunks_m * region.tiles_n, slice = work / tiles;
+            const int tiles = chunks_m * region.tiles_n;
+            slice = work / tiles;
             work -= slice * tiles;
             kbase = slice * per;
+            slices = (ktiles + per - 1) / per;
             ktiles = min(per, ktiles - kbase);
-            out += (size_t)slice * (size_t)P.M * (size_t)P.N;
+            if constexpr (!SHARED) out += (size_t)slice * (size_t)P.M * (size_t)P.N;
         }
     }
     // Four-waves-per-tile kernels (products with few tiles, often with the kernel operand as the large one): the host may
@@ -722,6 +737,30 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
             f32x4 sum = red[kw * 64 + lane];
 #pragma unroll
             for (int s = 1; s < KSW; ++s) sum += red[(s * 4 + kw) * 64 + lane];
+            if constexpr (SHARED) {
+                // A slice leaves its sums in memory; the block that arrives last at the tile's counter, which it sets back, adds all of them in
+                // their order. No block waits for another.
+                constexpr uint32_t TILE = BM * BN * 4u;
+                const int tile = chunk_m * region.tiles_n + tile_n;
+                const __amdgpu_buffer_rsrc_t p_rsrc = make_rsrc(reinterpret_cast<const char*>(partial) + (size_t)tile * (size_t)slices * TILE, (uint32_t)slices * TILE);
+                buffer_store_x4_agent(sum, p_rsrc, (uint32_t)tid * 16u, (uint32_t)slice * TILE);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the sums have reached memory
+                __syncthreads();
+                if (tid == 0) {
+                    const uint32_t n = __hip_atomic_fetch_add(arrivals + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (n + 1u == (uint32_t)slices) __hip_atomic_store(arrivals + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    Rs[0] = (int)n;
+                }
+                __syncthreads();
+                if (Rs[0] + 1 != slices) return;
+                f32x4 q[CONV_MAX_SHARES];                              // requested together; beyond the last slice the loads read zeros, which are not added
+#pragma unroll
+                for (int s = 0; s < CONV_MAX_SHARES; ++s) q[s] = buffer_load_x4_agent(p_rsrc, (uint32_t)tid * 16u, (uint32_t)s * TILE);
+                sum = q[0];
+#pragma unroll
+                for (int s = 1; s < CONV_MAX_SHARES; ++s)
+                    if (s < slices) sum += q[s];
+            }
             float y[4] = {sum[0], sum[1], sum[2], sum[3]};
             conv_straight_steps<4>(y, quarter, (P.flags >> 20) & 31u, (int)((P.flags >> 12) & 15u) - 1, Es, BN, l32, [&]() {
                 quarter_tile([&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], make_rsrc(epi.p[CONV_MAX_EPI - 1], P.out_bytes), vo, so); });
@@ -832,6 +871,21 @@ CONV_KERNEL(conv_gemm_32x32x128_ks4, 1, 1, 1, 1, 128, true, true, true, 4)
 CONV_KERNEL(conv_gemm_32x32x128_ks4g, 1, 1, 1, 1, 128, true, false, true, 4)
 // the same with a 64-long k step, for windows over 64 (or 192, ...) input features, whose taps a 128-long step would straddle
 CONV_KERNEL(conv_gemm_32x32x64_ks4, 1, 1, 1, 1, 64, true, true, true, 4)
+// The first two with several blocks per tile, each summing a slice of the contraction (k_split_steps): one block alone on its CU waits for its loads and
+// LDS reads between its matrix instructions (0.8 us per k step, 0.43 at the rate of the matrix cores; two together 1.36), and few tiles leave
+// CUs idle. A slice's sums make a round trip to memory and the counter another, 2 us for 32 x 32 numbers; a launch that adds them takes 3.2 and a start.
+// 196 x 2304 x 256 11.8 -> 10.8 us, 784 x 1152 x 128 11.6 -> 10.4, 196 x 1024 x 256 9.5 -> 7.5 (before: that launch), 588 x 4608 x 512 48.6 -> 34.8.
+#define CONV_SHARED_KERNEL(name, BF)                                                                         \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void name(          \
+        float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
+        float* __restrict__ partial, uint32_t* __restrict__ arrivals,                                        \
+        ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
+        __shared__ __attribute__((aligned(16))) float pool[conv_pool_floats<1, 1, 1, 1, 128>()];             \
+        const ConvRegion all{0, P.tiles_m, P.tiles_n, 0};                                                    \
+        conv_gemm_body<1, 1, 1, 1, 128, true, BF, true, 4, true>(pool, all, out, x, w, epi, dp, P, D, partial, arrivals); \
+    }
+CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4_shared, true)
+CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4g_shared, false)
 // Mixed tiling for layers whose 64 x 64 tiles do not divide evenly among the CUs (784 tiles on 256 CUs: a CU
 // with four tiles sets the time, the average is 3.06). The first P.split_tiles_m M tiles are computed as 64 x 64
 // tiles, as many as fill every CU equally; the rows behind them as 32 x 32 tiles of a quarter of the work each

@@ -18,14 +18,6 @@
 #pragma once
 #include "split_bf16.h"
 
-// stores and loads that are seen by every workgroup of the GPU, whichever L2 it stands behind (agent scope)
-__device__ __forceinline__ void buffer_store_x4_agent(f32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, soff, 16);
-}
-__device__ __forceinline__ f32x4 buffer_load_x4_agent(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 16));
-}
-
 // ---- the kernel operand, taken apart and laid out for the matrix cores ----------------------------------------------
 // A program's weights serve every row of a product: a launch of this kernel takes them apart once, instead of every tile of
 // rows doing it again, and lays them out in the order in which the lanes of a wave want them, so that the product's waves

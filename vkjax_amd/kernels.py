@@ -55,6 +55,7 @@ class _Choices:
         wgrad_split=None,                #kernel gradients on the bf16 matrix cores: None = where they pay, False = never, a tile's name = wherever it applies
         wgrad_slices=None,               #slices of a kernel gradient's contraction (None: by the estimate)
         conv_k_splits=None,              #slices a contraction is cut into where that applies (None: by the heuristic, 1: never)
+        conv_shares=None,                #blocks that share a tile of the four-waves-per-tile kernels and add its slices themselves (None: by the estimate, or where conv_k_splits is pinned, 1: never)
         conv_xcd_columns=0,              #four-waves-per-tile kernels: XCD columns over the tile grid (0: row-major ranges, None: least traffic)
         scatter_sort_threshold=1 << 18,  #update elements from which a row scatter-add sorts its updates instead of using atomics
         reuse_equal_equations=True,      #an equation that repeats an earlier one is bound to that one's buffer
@@ -516,6 +517,8 @@ class ConvGeometry(tp.NamedTuple):
     k_splits: int = 1
     #how the kernels on the bf16 matrix cores share the product out, or None: the others compute it
     split: tp.Optional['ConvSplit'] = None
+    #how blocks share the tiles of a four-waves-per-tile kernel, or None: one block per tile
+    shares: tp.Optional['ConvShares'] = None
 
     @property
     def M(self): return self.batch * self.Ho * self.Wo
@@ -803,6 +806,10 @@ def _epilogue_template_slots(epilogue: tp.Sequence[ConvEpilogueStep]) -> int:
     return slots
 
 
+def conv_straight_epilogue(epilogue: tp.Sequence[ConvEpilogueStep]) -> bool:
+    return _epilogue_template_slots([e for e in epilogue if e.op != CONV_TAP]) != 0
+
+
 def _magic_division(d: int) -> tp.Tuple[int, int]:
     '''(magic, shift) with n // d == (n * magic >> 32) >> shift for every 0 <= n < 2**31; magic 0 stands for d == 1.'''
     if d <= 1:
@@ -976,6 +983,12 @@ def _four_waves_pay(g: ConvGeometry, b_fast: bool, compute_units: int) -> bool:
             or (rounds == 4 and g.K >= 1024))
 
 
+#Up to here slices are added by a launch of their own, which also takes over chains longer than an epilogue; more tiles are shared by blocks that add them
+#themselves (conv_share_count). (Shared by eight blocks, 32 tiles x 36 k steps would take 11.2 us instead of 14.4, 32 x 16 7.9 instead of 9.5; but these
+#products are promised two launches: test_long_contractions_of_few_tiles_are_sliced, test_sliced_contractions.)
+CONV_SLICED_MAX_TILES = 32
+
+
 def conv_k_splits(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int = 256) -> int:
     '''Into how many slices the contraction of a product with very few tiles is cut (1: not at all). With 32 blocks on
     256 CUs, a layer whose kernel operand is megabytes long (the 3 x 3 layers of a network's last stages at batch 1)
@@ -990,15 +1003,69 @@ def conv_k_splits(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int 
     _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g)
     if not _four_waves_per_tile(g, a_fast, c_contig, compute_units, b_fast) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
         return 1
-    tiles, ksteps = _cdiv(g.M, 32) * _cdiv(g.N, 32), _cdiv(g.K, 128)
+    tiles, ksteps = conv_shared_tiles(g), _cdiv(g.K, 128)
     if CHOICES.conv_k_splits is not None:
         want = CHOICES.conv_k_splits
     else:
-        want = min(4, compute_units // tiles, ksteps // 4)
+        want = 1 if tiles > CONV_SLICED_MAX_TILES else min(4, compute_units // tiles, ksteps // 4)
     if want <= 1 or ksteps < 2:
         return 1
     per = _cdiv(ksteps, min(want, ksteps))
     return _cdiv(ksteps, per)
+
+
+class ConvShares(tp.NamedTuple):
+    '''`count` blocks per tile, each with a slice of the contraction: they leave their sums in `partial`, and the one that finds at
+    the tile's counter in `arrivals` that it is the last adds them in their order and applies the epilogue.'''
+    count: int
+    partial: Buffer
+    arrivals: Buffer
+
+
+CONV_MAX_SHARES = 8                #(of the same name in the kernel source)
+CONV_MAX_SHARED_TILES = 2048
+
+
+def conv_shared_tiles(g: ConvGeometry) -> int:
+    return _cdiv(g.M, 32) * _cdiv(g.N, 32)
+
+
+def choose_conv_shares(tiles: int, ksteps: int, compute_units: int = 256) -> int:
+    '''The number of blocks per tile with the smallest estimated time. A CU holds four blocks; a k step of 128 takes 0.8 us alone on one, 1.36 us
+    beside one other, 1.85 beside two and 2.3 beside three. A block starts in about a step; leaving, counting and
+    adding slices takes 2.2 us and 2.5 ns per block. Measured (tiles x k steps: one block per tile, and with the chosen number): 56 x 18 17.7, 10.8 us;
+    56 x 8 9.1, 7.5; 100 x 9 11.4, 10.4; 104 x 18 18.0, 13.7; 112 x 36 30.6, 19.1; 160 x 36 31.9, 23.4; 296 x 18 27.9, 22.2; 304 x 36 48.6, 34.8;
+    400 x 36 50.9, 44.9; where it stays at one, more take as long or longer: 100 x 4 6.5, 7.1; 56 x 4 6.2, 6.8; 200 x 18 18.8, 19.1; 400 x 16 25.4, 26.3. (The
+    partial sums in a launch of their own: 56 x 18 11.8 with four slices, 56 x 8 9.5, 100 x 9 11.6, 112 x 36 22.3.)'''
+    together = (0.8, 1.36, 1.85, 2.3)
+    def time(count):
+        per    = _cdiv(ksteps, count)
+        blocks = tiles * _cdiv(ksteps, per)
+        on_cu  = _cdiv(blocks, compute_units)
+        each   = together[on_cu - 1] if on_cu <= 4 else 2.3 + 0.57 * (on_cu - 4)
+        return 2.5 + each * (per + 0.8) + (2.2 + 0.0025 * blocks if count > 1 else 0.0)
+    alone = time(1)
+    count = min(range(1, min(ksteps, CONV_MAX_SHARES) + 1), key=time)
+    return count if time(count) < 0.95 * alone else 1
+
+
+def conv_share_count(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int = 256) -> int:
+    '''How many blocks share a tile where the four-waves-per-tile kernels compute the product (1: no sharing).'''
+    if (CHOICES.conv_shares == 1 or (CHOICES.conv_shares is None and CHOICES.conv_k_splits is not None) or g.k_splits > 1 or g.split is not None
+            or _dense_rows_shape(lhs, g)):
+        return 1
+    g = _flatten_pointwise(g)
+    if g.K * g.N * 4 >= 2**31 or lhs.size * 4 >= 2**31 or g.M * g.N == 0:
+        return 1
+    _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g)
+    #(not the 64-long step: 196 x 9 of those 7.8 us, by two blocks each 9.3)
+    if not _four_waves_per_tile(g, a_fast, c_contig, compute_units, b_fast) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
+        return 1
+    tiles, ksteps = conv_shared_tiles(g), _cdiv(g.K, 128)
+    if tiles > CONV_MAX_SHARED_TILES or (CHOICES.conv_shares is None and tiles <= CONV_SLICED_MAX_TILES):
+        return 1
+    want = min(CHOICES.conv_shares, ksteps, CONV_MAX_SHARES) if CHOICES.conv_shares is not None else choose_conv_shares(tiles, ksteps, compute_units)
+    return _cdiv(ksteps, _cdiv(ksteps, want))
 
 
 def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: tp.Sequence[ConvEpilogueStep] = (),
@@ -1058,6 +1125,9 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
         if (not ksplit or short_step or epilogue or taps or out_offset or out.size != g.k_splits * M * N
                 or _cdiv(_cdiv(K, 128), k_split_steps) != g.k_splits):
             raise ValueError('a sliced contraction needs the four-waves-per-tile kernel, no epilogue and one [M, N] matrix per non-empty slice')
+    elif g.shares is not None and ksplit and not short_step:
+        k_split_steps = _cdiv(_cdiv(K, bk), g.shares.count)
+        assert _cdiv(_cdiv(K, bk), k_split_steps) == g.shares.count and tiles_m * tiles_n <= g.shares.arrivals.size and not out_offset
     chunk = (CHOICES.conv_chunk or choose_conv_chunk(tiles_m, tiles_n, compute_units)) if lean and not ksplit else 1
     m_blocks = 0
     if lean and not ksplit and CHOICES.conv_chunk is None:
@@ -1095,19 +1165,23 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
     derived_ptrs, derived_desc = _conv_derived(epilogue, N)
     params += derived_desc
     buffers = [(out, out_offset * 4), (lhs, lhs_offset * 4), (rhs, rhs_offset * 4)]
+    shared  = k_split_steps > 0 and g.k_splits == 1
+    if shared:
+        buffers += [(g.shares.partial, 0), (g.shares.arrivals, 0)]
     operand_slots = _pad([(e.operand, 0) for e in epilogue], CONV_MAX_EPI, (None, 0))
     if taps:
         assert operand_slots[-1] == (None, 0)
         operand_slots[-1] = (tap_buffer, 0)
     buffers += operand_slots + derived_ptrs
-    kernel  = f'conv_gemm_{tag}x{bk}_' + (('ks4' if b_fast else 'ks4g') if ksplit else 'lean' if lean else ('f' if a_fast else 'g') + ('f' if b_fast else 'g'))
+    kernel  = f'conv_gemm_{tag}x{bk}_' + (('ks4' if b_fast else 'ks4g') + ('_shared' if shared else '') if ksplit else 'lean' if lean else ('f' if a_fast else 'g') + ('f' if b_fast else 'g'))
     nbytes  = 4 * (lhs.size + rhs.size + out.size) + sum(4 * e.operand.size for e in epilogue if e.operand is not None)
     nbytes += 4 * tap_buffer.size if taps else 0
-    blocks = (m_blocks or _cdiv(tiles_m, chunk)) * tiles_n * max(1, g.k_splits)
+    blocks = (m_blocks or _cdiv(tiles_m, chunk)) * tiles_n * (g.shares.count if shared else g.k_splits)
     if split_tiles_m:
         kernel = f'conv_gemm_{tag}x{bk}_mix'
         blocks = split_tiles_m * tiles_n + _cdiv(M - split_tiles_m * 64, 32) * _cdiv(N, 32)
-    return Launch(kernel, (blocks, 1, 1), (nt, 1, 1), buffers, params, bytes_moved=nbytes, flops=2 * M * N * K)
+    return Launch(kernel, (blocks, 1, 1), (nt, 1, 1), buffers, params, bytes_moved=nbytes, flops=2 * M * N * K,
+                  written=(0, 3, 4) if shared else (0,), scratch=(3, 4) if shared else ())
 
 
 # ------------------------------------------------- products on the bf16 matrix cores (csrc/kernels/conv_split.h)
