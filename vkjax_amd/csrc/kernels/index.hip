@@ -126,8 +126,8 @@ extern "C" __global__ __launch_bounds__(256) void scatter_add_rows(uint32_t* __r
 //
 // Buckets. A counting sort proper needs the bucket starts - a prefix sum over all counters, i.e. a launch of
 // its own between counting and placing, and a third one to place. Instead every row owns `cap` slots of a
-// table `fixed` (the host picks cap a few times the average number of updates per row, at most 64; 0: no
-// such table): update number i for row r takes k = count[r]++ and, if k < cap, goes to fixed[r * cap + k].
+// table `fixed` (the host picks cap a few times the average number of updates per row; 0: no
+// such table; see choose_scatter_bucket_cap): update number i for row r takes k = count[r]++ and, if k < cap, goes to fixed[r * cap + k].
 // The others go to an overflow table of at least twice as many slots as there are updates, open addressing:
 // the entry (r + 1) << 32 | i is put into the first free slot from hash(r) + (k - cap) on, so that the
 // overflow of one row lies in a run the row's wave later scans with coalesced loads, and entries of a row
@@ -137,7 +137,7 @@ extern "C" __global__ __launch_bounds__(256) void scatter_add_rows(uint32_t* __r
 // Counters and overflow slots are zero before and after an evaluation: the wave that reads them clears them.
 // Scratch: count (n_rows + 1 words: the counters, then the cursor, which the first launch resets), fixed
 // (n_rows * cap), table (2 words for each of table_mask + 1 slots), gathered and sorted (n_idx words each:
-// room for the buckets of rows with more than cap updates).
+// room for the buckets of rows with more than cap, or more than 64, updates).
 #define SCATTER_SORTED_MAX 4096u
 struct ScatterSortParams { uint32_t n_idx, row_len, n_rows, idx_stride, operand_is_scalar, clip, wrap, cap, table_mask; };   // clip: as in ScatterRowsParams; wrap: as in GatherRowsParams
 
@@ -199,7 +199,7 @@ __device__ __forceinline__ uint32_t wave_sort_first(uint32_t e, uint32_t n, uint
 // through the L2 (relaxed device-scope accesses). Out of line, like sort_bucket: crowded rows only.
 __device__ __attribute__((noinline)) uint32_t gather_bucket(uint32_t* gathered, const uint32_t* fixed_row, unsigned long long* table,
                                                             uint32_t table_mask, uint32_t row, uint32_t n, uint32_t cap, uint32_t lane) {
-    if (lane < cap) store_word(gathered + lane, load_word(fixed_row + lane));               // cap <= 64
+    for (uint32_t k = lane; k < cap; k += 64u) store_word(gathered + k, load_word(fixed_row + k));
     uint32_t found = cap;
     const uint32_t h0 = scatter_hash(row);
     // 64 consecutive slots a step, every slot of the table at most once (the table has at least 64 slots)
@@ -259,14 +259,17 @@ __device__ __forceinline__ void scatter_rows_sum_body(uint32_t* __restrict__ out
     if (lane == 0u) n_lane0 = count[row];
     uint32_t n = __builtin_amdgcn_readfirstlane(n_lane0);
     if (lane == 0u && n != 0u) count[row] = 0u;
-    // the row's bucket: its fixed slots, or - more updates than slots - a piece of `gathered` that holds all of them
+    // the row's bucket: its fixed slots, or - more updates than slots - a piece of `gathered` that holds all of them. More than the wave
+    // has lanes take a piece of `sorted` (numbered alike) as well
     const uint32_t* bucket = fixed + (uint64_t)row * P.cap;
-    if (n > P.cap) {
+    if (n > min(P.cap, 64u)) {
         uint32_t piece_lane0 = 0;
         if (lane == 0u) piece_lane0 = atomicAdd(count + P.n_rows, n);     // (the counters add up to at most n_idx)
         const uint32_t piece = __builtin_amdgcn_readfirstlane(piece_lane0);
-        n = gather_bucket(gathered + piece, bucket, table, P.table_mask, row, n, P.cap, lane);
-        bucket = gathered + piece;
+        if (n > P.cap) {
+            n = gather_bucket(gathered + piece, bucket, table, P.table_mask, row, n, P.cap, lane);
+            bucket = gathered + piece;
+        }
         sorted += piece;
     }
     auto add = [](vec_t a, vec_t b) -> vec_t {

@@ -1900,21 +1900,27 @@ def scatter_add_rows(out: Buffer, idx: Buffer, updates: Buffer, n_idx: int, row_
                   bytes_moved=4 * (total + n_idx + out.size))
 
 
+SCATTER_MAX_CAP = 1024
+
+
 def choose_scatter_bucket_cap(n_idx: int, n_rows: int, row_len: int) -> int:
     '''How many slots every table row gets in the sorted scatter-add's table of fixed-capacity buckets (0: none, every
     update goes through the overflow table): four times the average number of updates per row, as a power of two
-    between 4 and 64 - with indices spread evenly a row with more than that is a rarity - as long as the slots take at
-    most an eighth of the table's own size and eight words per update.'''
+    between 8 and 1024 - with indices spread evenly a row with more than that is a rarity - as long as the slots take at
+    most eight words per update, or 64 MB. Updates beyond the slots cost a hash table's insertion and a search each (rows x row length,
+    updates: us of gather and scatter-add with 0, 8, 16, 32, 64, 128, 256 slots): 100000 x 16, 262144 1104, 65, 64, 64, 64, 64, 64; 20000 x 16, 262144
+    427, 259, 76, 42, 42, 42, 42; 100000 x 24, 32000 330, 30, 30, 30, 30, 30, 31; 5000 x 200, 90000 116, 109, 81, 42, 41, 41, 41; 1000 x 256,
+    262144 5340, 4496, 3724, 2440, 685, 199, 194; 65536 x 256, 262144 869, 150, 148, 148, 148, 148, 148.'''
     if CHOICES.scatter_bucket_cap is not None:
         cap = int(CHOICES.scatter_bucket_cap)
-        assert 0 <= cap <= 64
+        assert 0 <= cap <= SCATTER_MAX_CAP
         return cap
     if n_rows == 0 or n_idx == 0:
         return 0
-    cap = 4
-    while cap < 64 and cap * n_rows < 4 * n_idx:
+    cap = 8
+    while cap < SCATTER_MAX_CAP and cap * n_rows < 4 * n_idx:
         cap *= 2
-    while cap >= 4 and (cap * 8 > row_len or cap * n_rows > 8 * n_idx):
+    while cap >= 4 and cap * n_rows > max(8 * n_idx, 1 << 24):
         cap //= 2
     return cap if cap >= 4 else 0
 
@@ -1936,7 +1942,7 @@ def scatter_add_rows_sorted(out: Buffer, operand: Buffer, idx: Buffer, updates: 
     value.'''
     slots = scatter_table_slots(n_idx)
     assert count.size == n_rows + 1 and table.size == 2 * slots and gathered.size == n_idx and sorted_.size == n_idx
-    assert 0 <= cap <= 64 and (cap == 0 or (fixed is not None and fixed.size == n_rows * cap))
+    assert 0 <= cap <= SCATTER_MAX_CAP and (cap == 0 or (fixed is not None and fixed.size == n_rows * cap))
     if fixed is None:
         fixed = gathered                 #(never touched: no update's number within its row is below 0)
     params = _u32(n_idx, row_len, n_rows, idx_stride, int(operand_is_scalar), int(clip), 0, cap, slots - 1)
