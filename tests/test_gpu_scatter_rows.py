@@ -1,9 +1,10 @@
-'''Sorted scatter-adds: more slots per row than a wave has lanes. The sums have the bits of a sequential loop.'''
+'''Sorted scatter-adds: more slots per row than a wave has lanes, and several short rows per wave. The sums have the bits of a sequential loop.'''
 import numpy as np
 import pytest
 
 import vkjax_amd
 from vkjax_amd import kernels as K, minijax as mj
+from vkjax_amd.jaxpr_interpreter import JaxprInterpreter
 
 pytestmark = pytest.mark.gpu
 
@@ -43,15 +44,30 @@ def check(rows, cols, idx, dtype, kernel, **choices):
             assert np.array_equal(vkjax_amd.wrap(onto_zeros(table.shape), frontend='minijax')(idx, updates), want)
 
 
+#rows that do not fill the last wave, rows of one number up to 32 lanes; buckets of none up to beyond the 16 that are sorted together, up to the slots and beyond
+@pytest.mark.parametrize('cols,vec', [(1, 1), (3, 1), (4, 4), (16, 4), (17, 1), (31, 1), (36, 4), (60, 4), (64, 4), (128, 4)])
+@pytest.mark.parametrize('dtype', [np.float32, np.int32])
+def test_several_rows_per_wave(cols, vec, dtype):
+    print('short rows:', cols, dtype.__name__, flush=True)
+    rng = np.random.default_rng(cols)
+    for rows, cap in ((1, 8), (67, 8), (131, 32), (300, 128)):
+        idx = indices(rng, rows, (0, 1, 2, 15, 16, 17, 32, 33, 64, 65, 130, 3, 4, 5)[:rows], 500)
+        check(rows, cols, idx, dtype, f'scatter_rows_sum_short_{"f" if dtype == np.float32 else "i"}_v{vec}', scatter_short_rows=True, scatter_bucket_cap=cap)
+
+
 @pytest.mark.parametrize('cap', (65, 128, 1024))
 @pytest.mark.parametrize('cols', (5, 256))
 def test_more_slots_than_lanes(cols, cap):
     print('slots:', cols, cap, flush=True)
     idx = indices(np.random.default_rng(cap), 40, (0, 63, 64, 65, 66, 127, 128, 129, 1023, 1024, 1025, 4096, 5), 9000)
-    check(40, cols, idx, np.float32, f'scatter_rows_sum_f_v{4 if cols % 4 == 0 else 1}', scatter_bucket_cap=cap)
+    check(40, cols, idx, np.float32, f'scatter_rows_sum_f_v{4 if cols % 4 == 0 else 1}', scatter_short_rows=False, scatter_bucket_cap=cap)
 
 
 def test_slots_by_the_rule():
+    plan = lambda rows, cols, n: [l.kernel for l in JaxprInterpreter(mj.make_jaxpr(scatter)(*[np.zeros(s, t) for s, t in (((rows, cols), np.float32), ((n,), np.int32), ((n, cols), np.float32))]),
+                                                                     plan_only=True).launches]
+    assert plan(20000, 16, 60000)[-1] == 'scatter_rows_sum_short_f_v4' and plan(20000, 128, 60000)[-1] == 'scatter_rows_sum_f_v4'
+    assert plan(20000, 16, 200000)[-1] == 'scatter_rows_sum_f_v4' and plan(2000, 16, 20000)[-1] == 'scatter_rows_sum_f_v4'
     caps = [K.choose_scatter_bucket_cap(n, rows, cols) for n, rows, cols in ((262144, 65536, 256), (32000, 100000, 24), (262144, 1000, 256), (90000, 5000, 200), (1000, 3000000, 16), (5, 2**27, 4))]
     assert caps == [16, 8, 1024, 128, 4, 0]
     assert all(cap * rows <= max(8 * n, 1 << 24) for cap, (n, rows) in zip(caps, ((262144, 65536), (32000, 100000), (262144, 1000), (90000, 5000), (1000, 3000000), (5, 2**27))))

@@ -58,6 +58,7 @@ class _Choices:
         conv_shares=None,                #blocks that share a tile of the four-waves-per-tile kernels and add its slices themselves (None: by the estimate, or where conv_k_splits is pinned, 1: never)
         conv_xcd_columns=0,              #four-waves-per-tile kernels: XCD columns over the tile grid (0: row-major ranges, None: least traffic)
         scatter_sort_threshold=1 << 18,  #update elements from which a row scatter-add sorts its updates instead of using atomics
+        scatter_short_rows=None,         #several table rows per wave in the sorted scatter-add: None = where it pays, True = wherever rows are short enough, False = never
         reuse_equal_equations=True,      #an equation that repeats an earlier one is bound to that one's buffer
     )
 
@@ -1935,7 +1936,7 @@ def scatter_add_rows_sorted(out: Buffer, operand: Buffer, idx: Buffer, updates: 
                             sorted_: Buffer, n_idx: int, row_len: int, n_rows: int, operand_is_scalar: bool = False,
                             idx_stride: int = 1, clip: bool = False, fixed: tp.Optional[Buffer] = None, cap: int = 0) -> tp.List[Launch]:
     '''out = operand; out[idx[i], :] += updates[i, :] without atomics on the data: the first launch buckets the updates by
-    row, then one wave per row sums its bucket. `count`: n_rows + 1 words, `table`: two words per slot of the overflow
+    row, then one wave per row, or for several short ones, sums their buckets. `count`: n_rows + 1 words, `table`: two words per slot of the overflow
     table (scatter_table_slots), both zero before and after; `fixed`: n_rows * cap words, the first `cap` updates of
     every row (cap = 0: no such table); `gathered`, `sorted_`: n_idx words each, room for the buckets of rows with
     more than cap updates. `operand` is the table, or one word when the table is a constant filled with a single
@@ -1949,11 +1950,18 @@ def scatter_add_rows_sorted(out: Buffer, operand: Buffer, idx: Buffer, updates: 
     vec    = 4 if row_len % 4 == 0 else 1
     kind   = 'f' if out.dtype == np.float32 else 'i'
     table_passes = 1 if operand_is_scalar else 2
+    lanes = max(4, _pow2_at_least(row_len // vec))
+    #Several rows per wave where there are more rows than waves the chip holds and few updates for each (us of gather and scatter-add, one row per
+    #wave and several; rows x row length, updates: 100000 x 16, 262144 63.6, 37.9; 100000 x 24, 32000 30.0, 15.9; 20000 x 24, 100000 25.5, 21.2; 40000 x 31, 131072 39.7, 35.8;
+    #but 5000 x 24, 32000 12.8, 15.2; 12000 x 40, 96000 25.4, 28.8; 20000 x 16, 262144 42.3, 65.9; 30000 x 128, 60000 32.6, 33.4)
+    short = (cap >= 8 and lanes <= 32 and
+             (CHOICES.scatter_short_rows if CHOICES.scatter_short_rows is not None else row_len <= 64 and n_rows >= 8192 and n_idx <= 6 * n_rows))
     return [
         Launch('scatter_rows_rank', (_cdiv(n_idx, BLOCK), 1, 1), (BLOCK, 1, 1), [(count, 0), (fixed, 0), (table, 0), (idx, 0)], params,
                bytes_moved=8 * n_idx, written=(0, 1, 2)),
-        Launch(f'scatter_rows_sum_{kind}_v{vec}', (_cdiv(n_rows, 4), 1, 1), (BLOCK, 1, 1),      #one wave per row
-               [(out, 0), (operand, 0), (updates, 0), (count, 0), (fixed, 0), (table, 0), (gathered, 0), (sorted_, 0)], params,
+        Launch(f'scatter_rows_sum_{"short_" if short else ""}{kind}_v{vec}', (_cdiv(n_rows, 4 * (64 // lanes if short else 1)), 1, 1), (BLOCK, 1, 1),
+               [(out, 0), (operand, 0), (updates, 0), (count, 0), (fixed, 0), (table, 0), (gathered, 0), (sorted_, 0)],
+               params + (_u32(lanes.bit_length() - 1) if short else b''),
                bytes_moved=4 * (n_idx * row_len + n_idx + n_rows + table_passes * n_rows * row_len), written=(0, 3, 5, 6, 7)),
     ]
 
