@@ -55,7 +55,7 @@ class _Choices:
         wgrad_split=None,                #kernel gradients on the bf16 matrix cores: None = where they pay, False = never, a tile's name = wherever it applies
         wgrad_slices=None,               #slices of a kernel gradient's contraction (None: by the estimate)
         conv_k_splits=None,              #slices a contraction is cut into where that applies (None: by the heuristic, 1: never)
-        conv_shares=None,                #blocks that share a tile of the four-waves-per-tile kernels and add its slices themselves (None: by the estimate, or where conv_k_splits is pinned, 1: never)
+        conv_shares=None,                #blocks that share a tile of the four-waves-per-tile kernels and add its slices themselves (None: by the estimate; a pinned conv_k_splits or conv_split: never, 1: never)
         conv_xcd_columns=0,              #four-waves-per-tile kernels: XCD columns over the tile grid (0: row-major ranges, None: least traffic)
         scatter_sort_threshold=1 << 18,  #update elements from which a row scatter-add sorts its updates instead of using atomics
         scatter_short_rows=None,         #several table rows per wave in the sorted scatter-add: None = where it pays, True = wherever rows are short enough, False = never
@@ -1052,7 +1052,8 @@ def choose_conv_shares(tiles: int, ksteps: int, compute_units: int = 256) -> int
 
 def conv_share_count(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int = 256) -> int:
     '''How many blocks share a tile where the four-waves-per-tile kernels compute the product (1: no sharing).'''
-    if (CHOICES.conv_shares == 1 or (CHOICES.conv_shares is None and CHOICES.conv_k_splits is not None) or g.k_splits > 1 or g.split is not None
+    pinned = CHOICES.conv_k_splits is not None or CHOICES.conv_split is not None          #(to the kernels themselves: one block per tile)
+    if (CHOICES.conv_shares == 1 or (CHOICES.conv_shares is None and pinned) or g.k_splits > 1 or g.split is not None
             or _dense_rows_shape(lhs, g)):
         return 1
     g = _flatten_pointwise(g)
