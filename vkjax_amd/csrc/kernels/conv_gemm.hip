@@ -544,8 +544,16 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
         }
     };
 
-    auto store_tiles = [&](int st = 0) {
+    auto store_tiles = [&](int k0, int st = 0) {
         if constexpr (A_FAST) {
+            // A contraction that ends within a vector (only with a single tap): what lies behind it is the next row's. The kernel operand's rows
+            // there read as zeros, which a value that is not finite would not leave alone.
+            if ((P.K & 3) != 0 && k0 + BK > P.K) {
+#pragma unroll
+                for (int p = 0; p < A_NV; ++p)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) a_reg[st][p][q] = k0 + a_kv * 4 + q < P.K ? a_reg[st][p][q] : 0.f;
+            }
 #pragma unroll
             for (int p = 0; p < A_NV; ++p) {
                 const int row = a_r0 + p * A_RSTEP, kv = a_kv;
@@ -670,13 +678,13 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
             // publishes the epilogue operands parked in LDS, and again before the reduction reuses the tiles.
             if (ktiles > 1) load_tiles((kbase + 1) * BK, 1);
             for (int kt = 0; kt < ktiles; kt += 2) {
-                store_tiles(0);
+                store_tiles((kbase + kt) * BK, 0);
                 if (kt == 0) __syncthreads(); else tile_barrier();
                 if (kt + 2 < ktiles) load_tiles((kbase + kt + 2) * BK, 0);
                 compute();
                 tile_barrier();
                 if (kt + 1 < ktiles) {
-                    store_tiles(1);
+                    store_tiles((kbase + kt + 1) * BK, 1);
                     tile_barrier();
                     if (kt + 3 < ktiles) load_tiles((kbase + kt + 3) * BK, 1);
                     compute();
@@ -687,7 +695,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
         } else {
             // all k steps but the last: the next step's loads are in flight during the MFMAs
             for (int kt = 1; kt < ktiles; ++kt) {
-                store_tiles();
+                store_tiles((kbase + kt - 1) * BK);
                 tile_barrier();
                 load_tiles((kbase + kt) * BK);
                 compute();
@@ -695,7 +703,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
             }
             // last k step: the loads in flight are those of the next M tile's first step and of
             // the residual operand
-            store_tiles();
+            store_tiles((kbase + ktiles - 1) * BK);
             __syncthreads();                 // (also where wave-private tiles publish the epilogue operands parked in LDS)
             if (sub + 1 < nsub) {
                 setup_rows(m0 + BM);
@@ -1179,6 +1187,12 @@ __device__ __forceinline__ void dense_rows_body(float* __restrict__ out, const f
             xv[u] = buffer_load_x4(x_rsrc, in ? xrow + (uint32_t)k4 * 4u : CONV_OOB);
 #pragma unroll
             for (int j = 0; j < N; ++j) wv[u][j] = buffer_load_x4(w_rsrc, in ? (uint32_t)(k4 * N + 4 * j) * 4u : CONV_OOB);
+        }
+        if ((P.K & 3) != 0) {                                              // (the next row's values, against rows of w that read as zeros)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) xv[u][q] = k0 + u * 256 + lane * 4 + q < P.K ? xv[u][q] : 0.f;
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u)

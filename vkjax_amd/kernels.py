@@ -871,6 +871,10 @@ def _conv_stem_launch(out, lhs, rhs, g: 'ConvGeometry', epilogue, taps, compute_
 
 
 DENSE_ROWS_MAX_N = 16
+#Rows x features up to which a wave per row serves contractions that are no multiple of four: a tile for 32 rows is faster beyond (us there and by tiles: 1024 x 511 x 8 4.6, 6.3;
+#5017 x 249 x 14 12.9, 5.0; 16384 x 511 x 8 36, 10; 131072 x 511 x 8 270, 57), and is as fast with multiples of four, whose sums are 2 to 3 times as far from 64 bits there
+#(4096 x 256 x 10 1.5e-7, here 7.7e-8; the others came from tiles with 64-wide steps, 3.9e-7 for 64 x 511 x 8, where they are 8.8e-8)
+DENSE_ROWS_MAX_RESULTS = 20480
 
 
 def _dense_rows_shape(lhs: Buffer, g: 'ConvGeometry') -> bool:
@@ -881,8 +885,8 @@ def _dense_rows_shape(lhs: Buffer, g: 'ConvGeometry') -> bool:
         return False
     M, N, K = g.M, g.N, g.K
     flat = (g.batch == 1 and g.Wo == 1 and g.KH == g.KW == 1 and g.SH == 1 and g.PH == g.PW == 0 and g.LH == 1 and g.H == g.Ho
-            and g.xs[3] == 1 and g.xs[1] % 4 == 0 and g.xs[1] >= K)
-    return (flat and 1 <= N <= DENSE_ROWS_MAX_N and K % 4 == 0 and K > 0 and tuple(g.ws[2:]) == (N, 1) and tuple(g.os[1:]) == (N, N, 1)
+            and g.xs[3] == 1 and g.xs[1] >= K)
+    return (flat and 1 <= N <= DENSE_ROWS_MAX_N and (K % 4 == 0 or M * N <= DENSE_ROWS_MAX_RESULTS) and K > 0 and tuple(g.ws[2:]) == (N, 1) and tuple(g.os[1:]) == (N, N, 1)
             and lhs.size * 4 < 2**31 and M * N * 4 < 2**31)
 
 
@@ -902,7 +906,7 @@ def dense_rows_epilogue_supported(epilogue: tp.Sequence[ConvEpilogueStep]) -> bo
 def _dense_rows_launch(out, lhs, rhs, g: 'ConvGeometry', epilogue, taps, lhs_offset, rhs_offset, out_offset,
                        softmax: bool, arg_out: tp.Optional[Buffer]) -> tp.Optional[Launch]:
     '''dense_rows_n16 where it applies: a matrix product (or 1x1 convolution over a dense array) with at most 16 output
-    features, a contraction that is a multiple of 4, dense operands, and an epilogue of per-feature and single-value
+    features and few rows, dense operands, and an epilogue of per-feature and single-value
     template steps; see the kernel.'''
     if taps or lhs_offset or rhs_offset or out_offset or g.k_splits > 1:
         return None
@@ -936,6 +940,11 @@ def _conv_derived(epilogue, N):
     return derived_ptrs, derived_desc
 
 
+def _features_in_vectors(g: ConvGeometry) -> bool:
+    '''Every position's features are whole, aligned vectors of four.'''
+    return g.Cin % 4 == 0 and all(s % 4 == 0 for s in g.xs[:3])
+
+
 def _conv_fast_paths(lhs: Buffer, rhs: Buffer, g: ConvGeometry, lhs_offset: int = 0, rhs_offset: int = 0):
     '''(needs_masks, x_bias, a_fast, b_fast, c_contig) of a flattened geometry: which loaders and stores apply.'''
     N = g.N
@@ -946,8 +955,9 @@ def _conv_fast_paths(lhs: Buffer, rhs: Buffer, g: ConvGeometry, lhs_offset: int 
     #input from (PH, PW) positions before its start
     x_bias = (g.PH * g.xs[1] + g.PW * g.xs[2]) * 4
     #(negative padding, i.e. cropping, goes through the generic loader's coordinate checks)
-    a_fast = (g.xs[3] == 1 and g.Cin % 4 == 0 and g.LH == 1 and g.LW == 1 and lhs_offset % 4 == 0 and g.PH >= 0 and g.PW >= 0
-              and all(s % 4 == 0 and s >= 0 for s in g.xs[:3]) and (not needs_masks or g.KH * g.KW <= 32)
+    #(a vector has to start at a word only; with several taps it must not straddle two of them)
+    a_fast = (g.xs[3] == 1 and (_features_in_vectors(g) or g.KH * g.KW == 1) and g.LH == 1 and g.LW == 1 and lhs_offset % 4 == 0 and g.PH >= 0 and g.PW >= 0
+              and all(s >= 0 for s in g.xs[:3]) and (not needs_masks or g.KH * g.KW <= 32)
               and (lhs.size - lhs_offset) * 4 + x_bias <= 2**31)
     #16-byte loads of the kernel operand need a dense [ky, kx, in, out] array, not an output width that is a multiple of 4:
     #a buffer load of four words only has to start at a word (verified on gfx950 with integer-exact products of odd
@@ -1305,7 +1315,7 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
     g = _flatten_pointwise(g)
     M, N, K = g.M, g.N, g.K
     _, _, a_fast, _, c_contig = _conv_fast_paths(lhs, lhs, g, 0)
-    if not a_fast or (g.Cin % 32 != 0 and g.KH * g.KW != 1) or conv_split_packed_words(g) * 4 >= 2**31 or M * N == 0:
+    if not a_fast or not _features_in_vectors(g) or (g.Cin % 32 != 0 and g.KH * g.KW != 1) or conv_split_packed_words(g) * 4 >= 2**31 or M * N == 0:
         return None
     #(pinned to other kernels of this family, a product is theirs)
     wanted = CHOICES.conv_split is None and CHOICES.conv_split_slices is None if CHOICES.conv_patch is None else CHOICES.conv_patch
