@@ -59,13 +59,15 @@ __device__ __forceinline__ void conv_pack_body(u32x4* __restrict__ out, const fl
     float x[8];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const int k0 = patch ? tap * P.Cin + 16 * sixteen + 8 * h + 4 * (lane >> 5) : (s >> 1) * 32 + h * 16 + 4 * o, rs = k0 / P.Cin;
-        int c = k0 - rs * P.Cin, ky = rs / P.KW, kx = rs - ky * P.KW;
+        const int c_patch = 16 * sixteen + 8 * h + 4 * (lane >> 5), k0 = (s >> 1) * 32 + h * 16 + 4 * o, rs = patch ? tap : k0 / P.Cin;
+        int c = patch ? c_patch : k0 - rs * P.Cin, ky = rs / P.KW, kx = rs - ky * P.KW;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const float v = (k0 + q < K && n < P.N) ? w[(int64_t)ky * P.ws_r + (int64_t)kx * P.ws_s + (int64_t)c * P.ws_c + (int64_t)n * P.ws_n] : 0.f;
+            // (the last vector of a patch, where features are left for a part of one only, ends with the last feature: it begins with ones that were there before)
+            if (patch) c = c_patch + 4 > P.Cin && c_patch < P.Cin ? P.Cin - 4 + q : c_patch + q;
+            const float v = ((patch ? c >= c_patch && c < P.Cin : k0 + q < K) && n < P.N) ? w[(int64_t)ky * P.ws_r + (int64_t)kx * P.ws_s + (int64_t)c * P.ws_c + (int64_t)n * P.ws_n] : 0.f;
             x[4 * h + q] = negative ? -v : v;
-            if (++c == P.Cin) { c = 0; if (++kx == P.KW) { kx = 0; ++ky; } }
+            if (++c == P.Cin && !patch) { c = 0; if (++kx == P.KW) { kx = 0; ++ky; } }
         }
     }
     u32x4 part[3];
@@ -204,7 +206,7 @@ __device__ constexpr int CONV_FINE_PA[7] = {2, 1, 2, 1, 1, 0, 0}, CONV_FINE_PB[7
 // -> 86 us (fp32 114), 33 x 7 x 7 x 512 x 512 55 -> 67 (101), 1 x 7 x 7 x 480 x 480 27 -> 32 (93).
 constexpr int CONV_PATCH_ROWS = 264, CONV_PATCH_ZEROS = 256;
 
-template <int WGM, int WGN, int TM, int TN, bool FINE>
+template <int WGM, int WGN, int TM, int TN, bool FINE, bool RAGGED>
 __device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* __restrict__ Es, float (&acc)[TM][TN][16],
                                                 float (&acc_large)[FINE ? TM : 1][FINE ? TN : 1][16], const uint32_t (&b_soff)[TN],
                                                 const float* __restrict__ x, __amdgpu_buffer_rsrc_t w_rsrc, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
@@ -224,9 +226,17 @@ __device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* _
     const int p_slot = p_octet * ROWS + p_row;
     constexpr int RAWS = TN == 1 ? 2 : 1;                               // items in registers: there is no room for two beside 128 columns
     f32x4 raw[RAWS][2];
+    // RAGGED: the vectors of the last eight features that are not all there; those of one octet behind the last feature are not, and those that reach beyond it begin earlier
+    const int last_eight = RAGGED ? (P.Cin - 1) >> 3 : 0, into = RAGGED ? P.Cin - 8 * last_eight - 4 * p_octet : 4;
+    const uint32_t p_last = into <= 0 ? CONV_OOB : (uint32_t)(8 * last_eight + min(into - 4, 0)) * 4u;      // (all in the lane's offset, which must not be negative)
+    auto load_eight = [&](int eight, int p) {
+        if constexpr (!RAGGED) return buffer_load_x4(x_rsrc, p_voff[p], (uint32_t)eight * 32u);
+        const uint32_t v = p_voff[p] + (eight == last_eight ? p_last : 0u);
+        return buffer_load_x4(x_rsrc, p_voff[p] == CONV_OOB ? CONV_OOB : v, eight > last_eight ? CONV_OOB : eight == last_eight ? 0u : (uint32_t)eight * 32u);
+    };
     auto load_item = [&](f32x4 (&to)[2], int sixteen, int p) {
-        to[0] = buffer_load_x4(x_rsrc, p_voff[p], (uint32_t)sixteen * 64u);
-        to[1] = buffer_load_x4(x_rsrc, p_voff[p], (uint32_t)sixteen * 64u + 32u);
+        to[0] = load_eight(2 * sixteen, p);
+        to[1] = load_eight(2 * sixteen + 1, p);
     };
     u32x4 part;
     auto park = [&](u32x4* to, int p, int t) { to[t * 2 * ROWS + p_slot + 128 * p] = part; };
@@ -381,7 +391,10 @@ __device__ __forceinline__ void conv_patch_sums(u32x4* __restrict__ As, float* _
 
 // STEPS: an epilogue other than the straight-line one, step by step (ReLU6, a scalar or a vector in another place, a residual that is subtracted).
 // FINE: products and sums of CONV_FINE_PA; a slice leaves both its sums.
-template <int WGM, int WGN, int TM, int TN, bool STEPS, bool PATCH, bool FINE>
+// RAGGED (with a patch): any number of features from four on. The kernel operand is laid out for a multiple of 32 of them, with zeros behind the last. A
+// vector of the input that would reach beyond a position's last feature ends there instead and begins with features of the vector in front, which meet zeros:
+// nothing of another position is read, so sums are what they are whatever their neighbours hold.
+template <int WGM, int WGN, int TM, int TN, bool STEPS, bool PATCH, bool FINE, bool RAGGED = false>
 __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float* __restrict__ Es, int* __restrict__ Rs,
                                                 float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                                                 float* __restrict__ partial, uint32_t* __restrict__ arrivals, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp,
@@ -421,7 +434,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
 #pragma unroll
     for (int j = 0; j < TN; ++j) b_soff[j] = (uint32_t)(n0 / 32 + wn * TN + j) * (uint32_t)ksteps * 3072u;
     if constexpr (PATCH) {
-        conv_patch_sums<WGM, WGN, TM, TN, FINE>(pool, Es, acc, acc_large, b_soff, x, w_rsrc, epi, Dp, P, Dk, wave, m0, n0, kbeg, kend);
+        conv_patch_sums<WGM, WGN, TM, TN, FINE, RAGGED>(pool, Es, acc, acc_large, b_soff, x, w_rsrc, epi, Dp, P, Dk, wave, m0, n0, kbeg, kend);
     } else {
     static_assert(!FINE, "only with a patch");
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
@@ -675,13 +688,16 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
             const uint32_t row = (uint32_t)(flat_rows ? m * P.xs_h : b * P.xs_b + ho * P.SH * P.xs_h + wo * P.SW * P.xs_w) * 4u;
             int r = 0, s = 0, c = 0;
             f32x4 a_next[2];
+            int c_next = 0;                                      // (RAGGED) the first feature of the vectors in a_next
             u32x4 b_next[TN][3];
             auto request = [&](int step) {
                 const int hi = hi0 + r * P.DH, wi = wi0 + s * P.DW, o = PATCH ? half : 2 * (step & 1) + half, k = PATCH ? 16 * step : (step >> 1) * BK + 4 * o;
+                c_next = RAGGED ? c + 4 * half : 0;
                 const bool ok = m < P.M && (flat_rows || ((uint32_t)hi < (uint32_t)P.H && (uint32_t)wi < (uint32_t)P.W));
                 const uint32_t at = row + (uint32_t)(r * P.DH * P.xs_h + s * P.DW * P.xs_w + c + 4 * o) * 4u;
-                a_next[0] = buffer_load_x4(x_rsrc, ok && k < P.K ? at : CONV_OOB);
-                a_next[1] = buffer_load_x4(x_rsrc, ok && k + (PATCH ? 8 : 16) < P.K ? at + (PATCH ? 32u : 64u) : CONV_OOB);
+                const int over0 = RAGGED ? max(0, c_next + 4 - P.Cin) : 0, over1 = RAGGED ? max(0, c_next + 12 - P.Cin) : 0;      // (4 or more: nothing is left)
+                a_next[0] = buffer_load_x4(x_rsrc, ok && k < P.K && over0 < 4 ? at - (uint32_t)over0 * 4u : CONV_OOB);
+                a_next[1] = buffer_load_x4(x_rsrc, ok && k + (PATCH ? 8 : 16) < P.K && over1 < 4 ? at + (PATCH ? 32u : 64u) - (uint32_t)over1 * 4u : CONV_OOB);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -702,7 +718,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
                 const float sign_k = (PATCH ? step / 3 & 1 : step & 4) ? -1.f : 1.f;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    av[e] = a_next[e >> 2][e & 3];
+                    av[e] = !RAGGED || (e & 3) >= c_next + 8 * (e >> 2) + 4 - P.Cin ? a_next[e >> 2][e & 3] : 0.f;      // (not the features that were there before)
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
                         uint32_t part_e[3];
@@ -832,14 +848,14 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         }
 }
 
-#define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE, STEPS, PATCH, FINE)                                                   \
+#define CONV_SPLIT_KERNEL(name, WGM, WGN, TM, TN, WPE, STEPS, PATCH, FINE, ...)                                              \
     extern "C" __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(WPE))) void name(             \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                                   \
         float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) { \
         __shared__ __attribute__((aligned(16))) u32x4 pool[PATCH ? 12 * CONV_PATCH_ROWS : 24 * 32 * WGM * TM];               \
         __shared__ float Es[CONV_MAX_EPI * 32 * WGN * TN];                                                                   \
         __shared__ int Rs[32 * WGM * TM];                                                                                    \
-        conv_split_body<WGM, WGN, TM, TN, STEPS, PATCH, FINE>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);    \
+        conv_split_body<WGM, WGN, TM, TN, STEPS, PATCH, FINE, ##__VA_ARGS__>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);    \
     }
 // _steps: 50176 x 128 x 512 with a ReLU6 68 us, with a scalar 62, with `relu(y) + r` 82 (each as launches of its own behind the product: 83, 82, 94;
 // in the fp32 kernels 73, 71, 73); 50176 x 256 x 512 97, 89, 108 (127, 120, 130). (Words of a full tensor requested for two tiles at a time
@@ -857,6 +873,9 @@ CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_steps, 2, 2, 2, 1, 3, true, true,
 // (242 registers: two blocks per CU)
 CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_fine, 2, 2, 2, 1, 2, false, true, true)
 CONV_SPLIT_KERNEL(conv_gemm_split_128x64_patch_fine_steps, 2, 2, 2, 1, 2, true, true, true)
+// (11 x 31 x 31 x 397 x 397 589 -> 209 us, 4 x 37 x 37 x 191 x 191 186 -> 44, 9 x 62 x 62 x 152 x 152 169 -> 115, 1 x 11 x 11 x 105 x 105 57 -> 18; before: the fp32 kernels)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_ragged, 2, 2, 2, 1, 2, false, true, true, true)
+CONV_SPLIT_KERNEL(conv_gemm_split_128x64_ragged_steps, 2, 2, 2, 1, 2, true, true, true, true)
 
 // ---- short contractions -------------------------------------------------------------------------------------------------
 // Dense rows [M, K] with K <= 64: a product whose time is that of its result, and of the arrays its epilogue reads. A block holds the packed

@@ -51,6 +51,7 @@ class _Choices:
         conv_split=None,                 #the kernels on the bf16 matrix cores: None = where they pay, False = never, True or a tile's name = wherever they apply
         conv_split_slices=None,          #blocks that share a tile behind the whole rounds (None: by the estimate)
         conv_patch=None,                 #the bf16 kernels that hold a patch of the input in LDS: None = wherever they pay (a pinned conv_split: never), True = wherever they apply, 'fine' = wherever they apply, with their two sums, False = never
+        conv_ragged=None,                #the bf16 kernel for 3 x 3 windows over any number of features: None = where it pays (a pinned conv_split: never), True = wherever no other patch kernel applies, False = never
         conv_short=None,                 #the bf16 kernels for dense rows of at most 64 features: None = where they pay (a pinned conv_split: never), True = wherever they apply, False = never
         wgrad_split=None,                #kernel gradients on the bf16 matrix cores: None = where they pay, False = never, a tile's name = wherever it applies
         wgrad_slices=None,               #slices of a kernel gradient's contraction (None: by the estimate)
@@ -1227,6 +1228,7 @@ class ConvSplit(tp.NamedTuple):
     partial: tp.Optional[Buffer] = None
     arrivals: tp.Optional[Buffer] = None
     patch: bool = False               #by the kernels that hold a patch of the input in LDS (conv_patch_applies)
+    ragged: bool = False              #... of any number of features, with two sums (conv_ragged_applies)
     fine: bool = False                #... by the one with two sums (_conv_patch_pays)
     short: bool = False               #by the kernels that hold the kernel operand in LDS (conv_short_applies)
 
@@ -1244,16 +1246,25 @@ def conv_split_partial_words(split: ConvSplit, g: ConvGeometry) -> int:
 
 def conv_split_packed_words(g: ConvGeometry) -> int:
     if g.split is not None and g.split.patch:
-        return _cdiv(g.N, 32) * (g.K // 64) * (CONV_SPLIT_PACK_BYTES // 4) + _cdiv(g.N, 32) * (g.K % 64) * (CONV_SPLIT_PACK_BYTES // 4 // 64)
+        return _cdiv(g.N, 32) * (conv_patch_k(g) // 32) * (CONV_SPLIT_PACK_BYTES // 8)
     return _cdiv(g.N, 32) * _cdiv(g.K, 64) * (CONV_SPLIT_PACK_BYTES // 4)
 
 
-def conv_patch_applies(g: ConvGeometry) -> bool:
+def conv_patch_k(g: ConvGeometry) -> int:
+    '''The contraction as the kernels that hold a patch walk it: features in pairs of sixteens.'''
+    return g.KH * g.KW * _cdiv(g.Cin, 32) * 32
+
+
+def conv_ragged_applies(g: ConvGeometry) -> bool:
     '''3 x 3 windows at a stride of 1 over dense images with a border of one: the positions of a tile and their neighbours are
     consecutive in memory. A patch has room for 256 positions (128 + 2 W + 2).'''
     return ((g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, g.LH, g.LW) == (3, 3) + (1,) * 8
-            and g.Ho == g.H and g.Wo == g.W and g.W <= 63 and g.Cin % 32 == 0 and g.xs[2] >= g.Cin
+            and g.Ho == g.H and g.Wo == g.W and g.W <= 63 and g.Cin >= 4 and g.xs[2] >= g.Cin and g.xs[3] == 1
             and g.xs[1] == g.W * g.xs[2] and g.xs[0] == g.H * g.xs[1])
+
+
+def conv_patch_applies(g: ConvGeometry) -> bool:
+    return conv_ragged_applies(g) and g.Cin % 32 == 0
 
 
 def conv_short_applies(g: ConvGeometry, c_contig: bool) -> bool:
@@ -1269,6 +1280,21 @@ def _conv_short_pays(g: ConvGeometry) -> bool:
     #x 32 x 256 50, 57. Results: 10 M 40000 x 64 x 256 26, 29; 12.8 M 100352 x 64 x 128 31, 32; 17 M 65536 x 64 x 256 41, 34, 131072 x 64 x 128 40, 34, 8200 x
     #64 x 2048 40, 36 (without an epilogue 30, 30); 19 M 200704 x 64 x 96 66, 42. With the backward pass of a ReLU half as long from 12 M on
     return g.N % 32 == 0 and g.N >= 96 and g.K > 32 and g.M * g.N >= 1 << 24
+
+
+def _conv_ragged_pays(g: ConvGeometry) -> bool:
+    '''3 x 3 windows over a number of features that is no multiple of 32, for which the fp32 kernels look every vector's tap up (or, without whole
+    vectors, every word's): where the kernel that holds a patch, whose errors are no larger, is faster, its packing launch included (us there and here).'''
+    #loads of words, images x size, features: 1 x 8, 22 15.8, 13.1; 60 x 40, 22 37.7, 27.8; 30 x 14, 41 25.3, 18.2; 11 x 31, 397 589, 209; 3 x 22, 417 219, 55; but 4 x 14, 17
+    #12.5, 13.5; 60 x 40, 9 18.5, 26.7
+    if g.Cin % 4 != 0:
+        return g.Cin >= 20
+    #of vectors: a long contraction in few tiles (1 x 8, 104 27.7, 18.3; 64 x 7, 200 50, 39; 16 x 14, 136 35, 29; but of 100 for 17 columns 60 x 28 43.5, 47.6), ...
+    if g.Cin >= 100 and (g.N >= 24 or g.M <= 8192):
+        return True
+    #... very few of them (4 x 14, 60 18.1, 16.9; 4 x 14, 80 22.6, 18.3; but 30 x 14, 72 21.7, 25.3), or many operations (60 x 40, 36 47.8, 43.5; 60 x 40, 60 71.9, 53.2; 8 x 30, 44 for
+    #300 columns 32.2, 30.5; but 10 x 40, 60 20.0, 25.0; 8 x 30, 36 for 300 28.5, 30.3)
+    return (g.Cin >= 60 and g.M <= 1024) or 2 * g.M * g.N * g.K >= 1.5e9
 
 
 def _conv_patch_pays(g: ConvGeometry, c_contig: bool) -> bool:
@@ -1315,7 +1341,9 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
     g = _flatten_pointwise(g)
     M, N, K = g.M, g.N, g.K
     _, _, a_fast, _, c_contig = _conv_fast_paths(lhs, lhs, g, 0)
-    if not a_fast or not _features_in_vectors(g) or (g.Cin % 32 != 0 and g.KH * g.KW != 1) or conv_split_packed_words(g) * 4 >= 2**31 or M * N == 0:
+    #(features that k tiles of 32 divide, or a single tap; one of the kernels that hold a patch takes any number)
+    tiled = a_fast and _features_in_vectors(g) and (g.Cin % 32 == 0 or g.KH * g.KW == 1)
+    if M * N == 0 or _cdiv(N, 32) * g.KH * g.KW * _cdiv(g.Cin, 32) * (CONV_SPLIT_PACK_BYTES // 2) >= 2**31:
         return None
     #(pinned to other kernels of this family, a product is theirs)
     wanted = CHOICES.conv_split is None and CHOICES.conv_split_slices is None if CHOICES.conv_patch is None else CHOICES.conv_patch
@@ -1323,14 +1351,20 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
     wanted = CHOICES.conv_split is None and CHOICES.conv_split_slices is None if CHOICES.conv_short is None else CHOICES.conv_short
     if wanted and conv_short_applies(g, c_contig) and (CHOICES.conv_short or _conv_short_pays(g)):
         return ConvSplit('128x64', _cdiv(M, 128) * _cdiv(N, 64), 1, short=True)
-    pays  = _conv_split_pays(g, c_contig)
-    fine  = patch and (CHOICES.conv_patch == 'fine' or (CHOICES.conv_patch is None and not pays))
-    if not (CHOICES.conv_split or CHOICES.conv_split_slices or (patch and CHOICES.conv_patch)) and not (_conv_patch_pays(g, c_contig) if fine else pays):
+    ragged = (conv_ragged_applies(g) and not patch and CHOICES.conv_split is None and CHOICES.conv_split_slices is None
+              and (CHOICES.conv_ragged if CHOICES.conv_ragged is not None else _conv_ragged_pays(g)))
+    if not tiled and not ragged:
+        return None
+    if ragged:
+        patch = True
+    pays  = tiled and _conv_split_pays(g, c_contig)
+    fine  = ragged or patch and (CHOICES.conv_patch == 'fine' or (CHOICES.conv_patch is None and not pays))
+    if not (ragged or CHOICES.conv_split or CHOICES.conv_split_slices or (patch and CHOICES.conv_patch)) and not (_conv_patch_pays(g, c_contig) if fine else pays):
         return None
     #The whole tiles are dealt out in rounds of one per CU; the contraction of those of the last, incomplete round (or of all,
     #if there are fewer tiles than CUs) may be cut into slices, of two k tiles at least. A block's start and end cost about
     #three k tiles, a slice's partial sums five more (a patch has to be complete before the first product: eight).
-    ktiles, best = K // 32 if patch else 2 * _cdiv(K, 64), None
+    ktiles, best = conv_patch_k(g) // 32 if patch else 2 * _cdiv(K, 64), None
     for tile, (bm, bn, shared_step, lone_step) in CONV_SPLIT_TILES.items():
         if CHOICES.conv_split not in (None, True, tile) or (fine and tile != '128x64'):
             continue
@@ -1345,7 +1379,7 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
             start, slice_start = (CONV_PATCH_START, CONV_PATCH_SLICE) if patch else (3, 8)
             time   = step * (rounds * (ktiles + start) + _cdiv((tiles - whole) * slices, CONV_SPLIT_ROUND) * (ktiles / slices + slice_start))
             if best is None or time < best[0]:
-                best = (time, ConvSplit(tile, whole, slices, patch=patch, fine=fine))
+                best = (time, ConvSplit(tile, whole, slices, patch=patch, ragged=ragged, fine=fine))
     return best[1] if best else None
 
 
@@ -1354,8 +1388,8 @@ def conv_split_pack(packed: Buffer, source: EwOperand, g: ConvGeometry) -> Launc
     apart into three bf16 parts and laid out for the matrix cores.'''
     assert packed.size == conv_split_packed_words(g)
     patch  = g.split is not None and g.split.patch
-    params = _i32(g.N, -g.K if patch else g.K, g.Cin, g.KW, *source.strides)
-    blocks = _cdiv(_cdiv(g.N, 32) * (g.K // 16), 4) if patch else _cdiv(g.N, 32) * _cdiv(g.K, 64)
+    params = _i32(g.N, -conv_patch_k(g) if patch else g.K, g.Cin, g.KW, *source.strides)
+    blocks = _cdiv(_cdiv(g.N, 32) * (conv_patch_k(g) // 16), 4) if patch else _cdiv(g.N, 32) * _cdiv(g.K, 64)
     return Launch('conv_split_pack', (blocks, 1, 1), (BLOCK, 1, 1), [(packed, 0), (source.buffer, source.offset * 4)], params,
                   bytes_moved=4 * (packed.size + g.K * g.N))
 
@@ -1393,10 +1427,10 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
     descs  = [0, 0]
     for i, e in enumerate(epilogue):
         descs[i // 3] |= ((0 if masked else e.op * 2 + int(e.operand_left)) | e.kind << 8) << (10 * (i % 3))
-    (tiles_m, tiles_n), kpairs = conv_split_tiles(split, g), g.Cin // 32 if split.patch else _cdiv(K, 64)
-    assert not split.patch or conv_patch_applies(g)
+    (tiles_m, tiles_n), kpairs = conv_split_tiles(split, g), _cdiv(g.Cin, 32) if split.patch else _cdiv(K, 64)
+    assert not split.patch or (conv_ragged_applies if split.ragged else conv_patch_applies)(g)
     shared = tiles_m * tiles_n - split.whole
-    blocks, threads, kernel = split.whole + shared * split.slices, 256, f'conv_gemm_split_{split.tile}' + ('_patch' if split.patch else '') + ('_fine' if split.fine else '')
+    blocks, threads, kernel = split.whole + shared * split.slices, 256, f'conv_gemm_split_{split.tile}' + ('_ragged' if split.ragged else ('_patch' if split.patch else '') + ('_fine' if split.fine else ''))
     if split.short:
         assert conv_short_applies(g, c_contig) and flat_rows
         #one block per CU for at most 256 columns, its waves walk the tiles of 32 rows
@@ -1404,7 +1438,7 @@ def conv_split_launch(out: Buffer, lhs: Buffer, packed: Buffer, g: ConvGeometry,
         column_blocks    = _cdiv(_cdiv(N, 32), tiles_n)
         tiles_n          = _cdiv(_cdiv(N, 32), column_blocks)
         blocks, threads, kernel, shared = max(1, min(CONV_SPLIT_ROUND // tiles_n, tiles_m)) * tiles_n, 768, 'conv_gemm_split_short', 0
-    params = (_i32(M, N, K, g.Ho, g.Wo, g.H, g.W, g.Cin, g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, *g.xs[:3], tiles_m, tiles_n)
+    params = (_i32(M, N, conv_patch_k(g) if split.patch else K, g.Ho, g.Wo, g.H, g.W, g.Cin, g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW, *g.xs[:3], tiles_m, tiles_n)
               + _u32(flags, *descs, (lhs.size - lhs_offset) * 4, packed.size * 4, (out.size - out_offset) * 4,
                      *_magic_division(g.Ho * g.Wo), *_magic_division(g.Wo))
               + _i32(g.LH, g.LW, g.xs[3], *g.ws, *g.os, split.whole, 0, split.slices, column_blocks if split.short else kpairs // split.slices, kpairs % split.slices))
