@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 typedef float    f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -12,11 +13,43 @@ typedef float    f32x16 __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ uint32_t f2u(float x) { return __float_as_uint(x); }
 __device__ __forceinline__ float    u2f(uint32_t x) { return __uint_as_float(x); }
 
-// Butterfly reductions across the 64 lanes of a wave.
+// The value of lane ^ S, in vector instructions: __shfl_xor goes through LDS, a round trip of some 100 cycles, of which a butterfly makes six in a row.
+// (Needs the lanes it reads to be active, like __shfl_xor.)
+template <int S>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+    static_assert(S == 1 || S == 2 || S == 4 || S == 8 || S == 16 || S == 32, "a step of a butterfly");
+    if constexpr (S == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);           // quads: 1 0 3 2
+    else if constexpr (S == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);      // quads: 2 3 0 1
+    else if constexpr (S == 4) {                                        // quads 0 and 2 of a row of 16 lanes take the next quad, 1 and 3 the one before
+        const int up = __builtin_amdgcn_update_dpp((int)v, (int)v, 0x104, 0xF, 0x5, false);
+        return (uint32_t)__builtin_amdgcn_update_dpp(up, (int)v, 0x114, 0xF, 0xA, false);
+    }
+    else if constexpr (S == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);     // a row turned by 8
+    else {                                                              // [0]: the even rows (the lower half) twice, [1]: the odd ones (the upper half) twice
+        const bool second = (__lane_id() & (uint32_t)S) != 0u;
+        if constexpr (S == 16) { const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false); return second ? r[0] : r[1]; }
+        else                   { const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false); return second ? r[0] : r[1]; }
+    }
+}
+template <int S> __device__ __forceinline__ float lane_xor(float v) { return u2f(lane_xor<S>(f2u(v))); }
+template <int S> __device__ __forceinline__ uint64_t lane_xor(uint64_t v) {
+    return (uint64_t)lane_xor<S>((uint32_t)(v >> 32)) << 32 | lane_xor<S>((uint32_t)v);
+}
+// step(std::integral_constant<int, S>) for S = 32, 16 .. 1
+template <class F>
+__device__ __forceinline__ void wave_butterfly(F step) {
+    step(std::integral_constant<int, 32>{}); step(std::integral_constant<int, 16>{}); step(std::integral_constant<int, 8>{});
+    step(std::integral_constant<int, 4>{});  step(std::integral_constant<int, 2>{});  step(std::integral_constant<int, 1>{});
+}
+// Butterfly across groups of `lanes` lanes (a power of two, the same in the whole wave), the widest step first.
 template <class T, class F>
-__device__ __forceinline__ T wave_allreduce(T v, F f) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = f(v, __shfl_xor(v, off, VKJ_WAVE));
+__device__ __forceinline__ T lanes_allreduce(T v, uint32_t lanes, F f) {
+    if (lanes > 32u) v = f(v, lane_xor<32>(v));
+    if (lanes > 16u) v = f(v, lane_xor<16>(v));
+    if (lanes > 8u)  v = f(v, lane_xor<8>(v));
+    if (lanes > 4u)  v = f(v, lane_xor<4>(v));
+    if (lanes > 2u)  v = f(v, lane_xor<2>(v));
+    if (lanes > 1u)  v = f(v, lane_xor<1>(v));
     return v;
 }
 

@@ -1201,14 +1201,13 @@ __device__ __forceinline__ void dense_rows_body(float* __restrict__ out, const f
 #pragma unroll
                 for (int n = 0; n < N; ++n) acc[n] = __builtin_fmaf(xv[u][q], wv[u][(q * N + n) / 4][(q * N + n) % 4], acc[n]);
     }
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) {
+    wave_butterfly([&](auto step) {
         float o[N];
 #pragma unroll
-        for (int n = 0; n < N; ++n) o[n] = __shfl_xor(acc[n], s, 64);
+        for (int n = 0; n < N; ++n) o[n] = lane_xor<decltype(step)::value>(acc[n]);
 #pragma unroll
         for (int n = 0; n < N; ++n) acc[n] = acc[n] + o[n];
-    }
+    });
     float y[N];
 #pragma unroll
     for (int n = 0; n < N; ++n) {

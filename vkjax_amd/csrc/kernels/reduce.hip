@@ -178,23 +178,19 @@ __device__ __forceinline__ void reduce_rows_body(uint32_t* __restrict__ out, con
         const float    x    = u2f(bits);
         const uint32_t rank = x != x ? 0xFFFFFFFFu : (MODE == 3 ? flipped : ~flipped);
         uint64_t key = best_i == 0xFFFFFFFFu ? 0ull : ((uint64_t)rank << 32 | (uint32_t)~best_i);   // no rank of a value is 0
-#pragma unroll
-        for (int s = 32; s >= 1; s >>= 1) {
-            const uint64_t other = __shfl_xor(key, s, 64);
-            key = other > key ? other : key;
-        }
+        key = lanes_allreduce(key, 64u, [](uint64_t a, uint64_t b) { return b > a ? b : a; });
         if (lane == 0) out[unit] = key == 0ull ? 0u : ~(uint32_t)key;
         return;
     }
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) {
+    wave_butterfly([&](auto step) {
+        constexpr int S = decltype(step)::value;
         if (is_arg) {
-            const uint32_t vi = __shfl_xor(best_i, s, 64), vv = __shfl_xor(best_v, s, 64);
+            const uint32_t vi = lane_xor<S>(best_i), vv = lane_xor<S>(best_v);
             if (vi != 0xFFFFFFFFu && (best_i == 0xFFFFFFFFu || arg_better(is_max, P.type, vv, vi, best_v, best_i))) { best_v = vv; best_i = vi; }
         } else {
-            a = red_step<MODE>(P.op, P.type, a, __shfl_xor(a, s, 64));
+            a = red_step<MODE>(P.op, P.type, a, lane_xor<S>(a));
         }
-    }
+    });
     if (lane == 0) out[unit] = is_arg ? (best_i == 0xFFFFFFFFu ? 0u : best_i) : reduce_post<POST>(a, post);
 }
 
@@ -629,7 +625,7 @@ __device__ __forceinline__ void softmax_rows_body(float* __restrict__ out, const
     for (int i = 0; i < NV; ++i)
 #pragma unroll
         for (int j = 0; j < VEC; ++j) m = at[i] != 0x80000000u && (v[i][j] > m || v[i][j] != v[i][j]) ? v[i][j] : m;
-    for (uint32_t s = lanes >> 1; s >= 1; s >>= 1) { const float o = __shfl_xor(m, s, 64); m = (m > o || m != m) ? m : o; }
+    m = lanes_allreduce(m, lanes, [](float a, float b) { return (a > b || a != a) ? a : b; });
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < NV; ++i)
@@ -639,7 +635,7 @@ __device__ __forceinline__ void softmax_rows_body(float* __restrict__ out, const
             acc[VEC == 4 ? j : i & 3] += v[i][j];                     // the sums are never -0, so adding 0 keeps them
         }
     float total = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-    for (uint32_t s = lanes >> 1; s >= 1; s >>= 1) total = total + __shfl_xor(total, s, 64);
+    total = lanes_allreduce(total, lanes, [](float a, float b) { return a + b; });
     const bool stream = streams_result(P.outer);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -671,10 +667,7 @@ __device__ __forceinline__ void softmax_rows_body(float* __restrict__ out, const
     const uint32_t flipped = zb ^ ((zb >> 31) ? 0xFFFFFFFFu : 0x80000000u);
     const float    bv      = u2f(best_v);
     uint64_t key = best_i == 0xFFFFFFFFu ? 0ull : ((uint64_t)(bv != bv ? 0xFFFFFFFFu : flipped) << 32 | (uint32_t)~best_i);
-    for (uint32_t s = lanes >> 1; s >= 1; s >>= 1) {
-        const uint64_t other = __shfl_xor(key, s, 64);
-        key = other > key ? other : key;
-    }
+    key = lanes_allreduce(key, lanes, [](uint64_t a, uint64_t b) { return b > a ? b : a; });
     if (l == 0 && first + sub < outer) arg_out[first + sub] = key == 0ull ? 0u : ~(uint32_t)key;
 }
 
@@ -732,15 +725,15 @@ extern "C" __global__ __launch_bounds__(256) void reduce_general(uint32_t* __res
             acc = red_combine(P.op, P.type, acc, v);
         }
     }
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) {
+    wave_butterfly([&](auto step) {
+        constexpr int S = decltype(step)::value;
         if (is_arg) {
-            const uint32_t vi = __shfl_xor(best_i, s, 64), vv = __shfl_xor(best_v, s, 64);
+            const uint32_t vi = lane_xor<S>(best_i), vv = lane_xor<S>(best_v);
             if (vi != 0xFFFFFFFFu && (best_i == 0xFFFFFFFFu || arg_better(is_max, P.type, vv, vi, best_v, best_i))) { best_v = vv; best_i = vi; }
         } else {
-            acc = red_combine(P.op, P.type, acc, __shfl_xor(acc, s, 64));
+            acc = red_combine(P.op, P.type, acc, lane_xor<S>(acc));
         }
-    }
+    });
     if (lane == 0) out[o] = is_arg ? (best_i == 0xFFFFFFFFu ? 0u : best_i) : acc;
 }
 

@@ -123,7 +123,7 @@ __device__ __forceinline__ void rows_body(const RowsOut& out, const RowsIn& in, 
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) s[VEC == 4 ? j : i & 3] += ok[i] ? u2f(acc[i * VEC + j]) : 0.f;
             float total = (s[0] + s[1]) + (s[2] + s[3]);
-            for (uint32_t d = lanes >> 1; d >= 1; d >>= 1) total = total + __shfl_xor(total, d, 64);
+            total = lanes_allreduce(total, lanes, [](float a, float b) { return a + b; });
 #pragma unroll
             for (int e = 0; e < W; ++e) acc[e] = f2u(total);
         } else if (kind == ROWS_MAX) {
@@ -134,7 +134,7 @@ __device__ __forceinline__ void rows_body(const RowsOut& out, const RowsIn& in, 
 #pragma unroll
                 for (int j = 0; j < VEC; ++j) s[VEC == 4 ? j : i & 3] = higher(s[VEC == 4 ? j : i & 3], ok[i] ? u2f(acc[i * VEC + j]) : -INFINITY);
             float top = higher(higher(s[0], s[1]), higher(s[2], s[3]));
-            for (uint32_t d = lanes >> 1; d >= 1; d >>= 1) top = higher(top, __shfl_xor(top, d, 64));
+            top = lanes_allreduce(top, lanes, higher);
             top = __shfl(top, lane & ~(lanes - 1u), 64);              // (the first lane's, as reduce_rows stores it)
 #pragma unroll
             for (int e = 0; e < W; ++e) acc[e] = f2u(top);
