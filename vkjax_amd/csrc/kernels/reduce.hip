@@ -587,11 +587,12 @@ RELU_BACKWARD_KERNEL(relu_backward_v4, 4)
 // per lane (the host takes the smallest variant that holds the row), one exp per value. Rows of one vector per lane
 // take 2^lanes_log2 lanes each, the fewest that hold them, and a wave does several; the lanes that such a row would
 // leave idle only add zeros to its sum, so its bits do not depend on how many there are.
-// What bounds it: memory. 65536 rows of 1000 with labels: 79 us, 6.6 TB/s (one wave per row that read it three
-// times, two exps per value: 205 us). Replays of 65536 rows of 10 with one row per wave 35 us, with several 20 us; 20000
-// of 1001 76 -> 43 us, 16384 of 4092 223 -> 103 us.
+// What bounds it: memory for long rows, next to it the instructions of exp and division, some 25 a value now. Replays of 65536 rows of 1000 with labels
+// 83.9 -> 77.2 us (6.8 TB/s), 45179 of 163 20.7 -> 16.8, 30544 of 562 30.0 -> 24.7, 171 of 2038 7.9 -> 5.3 (before: each value divided by itself,
+// every value compared as reduce_rows_fargmax does). One wave per row that read it three times, two exps per value: 205 us; 65536 rows of 10 with one
+// row per wave 35 us, with several 20.
 // `arg_out` (may be null): the index of each result row's largest value as reduce_rows_fargmax would report it
-// (first occurrence, a NaN wins), for programs that take the arg-max of the probabilities right away.
+// (first occurrence; of a row of NaN the first), for programs that take the arg-max of the probabilities right away.
 struct SoftmaxParams { uint32_t outer, R, lanes_log2; };
 
 template <int VEC, int NV>
@@ -620,27 +621,51 @@ __device__ __forceinline__ void softmax_rows_body(float* __restrict__ out, const
             v[i][0] = buffer_load_x1(x_rsrc, at[i]);
         }
     }
-    float m = -INFINITY;                                              // the maximum does not depend on the order; a NaN wins
+    // beyond the row: values whose exponentials are 0 and which are never the largest
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) m = at[i] != 0x80000000u && (v[i][j] > m || v[i][j] != v[i][j]) ? v[i][j] : m;
-    m = lanes_allreduce(m, lanes, [](float a, float b) { return (a > b || a != a) ? a : b; });
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < VEC; ++j) v[i][j] = at[i] != 0x80000000u ? v[i][j] : -INFINITY;
+    float m = -INFINITY;                                              // (does not depend on the order; rows with a NaN have sums that are NaN whatever it is)
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) m = fmaxf(m, v[i][j]);
+    m = lanes_allreduce(m, lanes, [](float a, float b) { return fmaxf(a, b); });
+    float acc[4] = {0.f, 0.f, 0.f, 0.f}, least = 1.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
         for (int j = 0; j < VEC; ++j) {
-            v[i][j] = at[i] != 0x80000000u ? expf(v[i][j] - m) : 0.f;
+            v[i][j] = expf(v[i][j] - m);
             acc[VEC == 4 ? j : i & 3] += v[i][j];                     // the sums are never -0, so adding 0 keeps them
+            least = fminf(least, v[i][j] == 0.f ? 1.f : v[i][j]);
         }
     float total = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     total = lanes_allreduce(total, lanes, [](float a, float b) { return a + b; });
+    // Every value of a row has the same divisor: its reciprocal once, then three instructions a value instead of ten. With r the rounded reciprocal of t, q = e r
+    // and the exact remainder e - q t, q + (e - q t) r is the rounded quotient (P. Markstein, IBM J. Res. Dev. 34, 1990). r is rounded where one Newton step has
+    // been taken from v_rcp_f32, unless all bits of t's fraction are set; t is 1 or more (the largest value's exponential is 1), so the remainder is exact where e is
+    // not so small that its bits are lost. Rows beyond that, and those with a NaN, are divided value by value.
+    const bool plain = total < 0x1p60f && (f2u(total) & 0x7FFFFFu) != 0x7FFFFFu && least >= 0x1p-90f;
+    if (__builtin_amdgcn_ballot_w64(!plain) == 0) {
+        const float r0 = __builtin_amdgcn_rcpf(total), r = __builtin_fmaf(__builtin_fmaf(-total, r0, 1.f), r0, r0);
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) {
+                const float q = v[i][j] * r;
+                v[i][j] = __builtin_fmaf(__builtin_fmaf(-total, q, v[i][j]), r, q);
+            }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) v[i][j] = v[i][j] / total;
+    }
     const bool stream = streams_result(P.outer);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) v[i][j] = v[i][j] / total;
         if constexpr (VEC == 4) {
             const u32x4 t = u32x4{f2u(v[i][0]), f2u(v[i][1]), f2u(v[i][2]), f2u(v[i][3])};
             if (stream) __builtin_amdgcn_raw_buffer_store_b128(t, y_rsrc, at[i], 0, 2);
@@ -651,24 +676,20 @@ __device__ __forceinline__ void softmax_rows_body(float* __restrict__ out, const
         }
     }
     if (arg_out == nullptr) return;
-    uint32_t best_v = 0, best_i = 0xFFFFFFFFu;
+    // the first of the largest: results are at least 0, so none beyond the row is larger, and a row of NaN has its first value's number
+    float top = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-            // a lane meets its elements in ascending order: on a tie the earlier one stays; a NaN replaces any number
-            const float p = v[i][j], q = u2f(best_v);
-            const bool better = at[i] != 0x80000000u && (p > q || (p != p && q == q) || best_i == 0xFFFFFFFFu);
-            best_v = better ? f2u(p) : best_v;
-            best_i = better ? (l + i * lanes) * VEC + j : best_i;
-        }
-    // across the lanes as in reduce_rows: the maximum of (rank of the value, complement of the index)
-    const uint32_t zb      = best_v == 0x80000000u ? 0u : best_v;      // -0.0 ranks with +0.0
-    const uint32_t flipped = zb ^ ((zb >> 31) ? 0xFFFFFFFFu : 0x80000000u);
-    const float    bv      = u2f(best_v);
-    uint64_t key = best_i == 0xFFFFFFFFu ? 0ull : ((uint64_t)(bv != bv ? 0xFFFFFFFFu : flipped) << 32 | (uint32_t)~best_i);
-    key = lanes_allreduce(key, lanes, [](uint64_t a, uint64_t b) { return b > a ? b : a; });
-    if (l == 0 && first + sub < outer) arg_out[first + sub] = key == 0ull ? 0u : ~(uint32_t)key;
+        for (int j = 0; j < VEC; ++j) top = fmaxf(top, v[i][j]);
+    top = lanes_allreduce(top, lanes, [](float a, float b) { return fmaxf(a, b); });
+    uint32_t best = 0xFFFFFFFFu;
+#pragma unroll
+    for (int i = NV - 1; i >= 0; --i)
+#pragma unroll
+        for (int j = VEC - 1; j >= 0; --j) best = v[i][j] == top ? (l + i * lanes) * VEC + j : best;
+    best = lanes_allreduce(best, lanes, [](uint32_t a, uint32_t b) { return min(a, b); });
+    if (l == 0 && first + sub < outer) arg_out[first + sub] = total == total ? best : 0u;
 }
 
 #define SOFTMAX_ROWS(name, VEC, NV)                                                                                         \
@@ -687,7 +708,9 @@ SOFTMAX_ROWS(softmax_rows_v4_n12, 4, 12)
 SOFTMAX_ROWS(softmax_rows_v4_n16, 4, 16)
 SOFTMAX_ROWS(softmax_rows_v1, 1, 1)
 SOFTMAX_ROWS(softmax_rows_v1_n2, 1, 2)
+SOFTMAX_ROWS(softmax_rows_v1_n3, 1, 3)
 SOFTMAX_ROWS(softmax_rows_v1_n4, 1, 4)
+SOFTMAX_ROWS(softmax_rows_v1_n6, 1, 6)
 SOFTMAX_ROWS(softmax_rows_v1_n8, 1, 8)
 SOFTMAX_ROWS(softmax_rows_v1_n12, 1, 12)
 SOFTMAX_ROWS(softmax_rows_v1_n16, 1, 16)

@@ -1637,7 +1637,7 @@ def sum_with_post(total: Launch, out: Buffer, kind: str, value: Buffer) -> tp.Op
 
 SOFTMAX_MAX_ROW = 4096      #rows this short run unsplit in reduce_rows, whose summation order softmax_rows repeats
 #vectors per lane of the kernels' variants: a row stays in the registers of one wave
-SOFTMAX_VECTORS = {4: (1, 2, 3, 4, 6, 8, 12, 16), 1: (1, 2, 4, 8, 12, 16, 24, 32, 48, 64)}
+SOFTMAX_VECTORS = {4: (1, 2, 3, 4, 6, 8, 12, 16), 1: (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64)}
 
 
 def softmax_rows(out: Buffer, inp: Buffer, outer: int, R: int, arg_out: tp.Optional[Buffer] = None) -> Launch:
