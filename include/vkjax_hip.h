@@ -183,8 +183,8 @@ int vkj_seq_eval_next(vkj_handle seq, void* const* host_ptrs, int nslots, uint32
 #define VKJ_STATIC_LANDING_BYTES (64u << 20)
 int vkj_seq_eval_next_static(vkj_handle seq, void* const* host_ptrs, int nslots, uint32_t flags,
                              void* const* next_host_ptrs);
-/* Launches only, `iters` times back to back, bracketed by two events on the context's
- * stream; *ms_total receives the elapsed device time of all iterations. Used for
+/* Launches only, `iters` times back to back, between two readings of the GPU's clock on the
+ * context's stream; *ms_total receives the elapsed device time of all iterations. Used for
  * measurement with inputs resident in HBM. No counterpart in the reference. */
 int vkj_seq_replay(vkj_handle seq, int iters, float* ms_total);
 /* Makes vkj_seq_eval and vkj_seq_replay issue the launches of this sequence as ONE captured HIP

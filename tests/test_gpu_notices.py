@@ -1,0 +1,99 @@
+'''The end of an evaluation, told by its last launch: results are all there when it is seen, call after call, from several threads, and for readers on other streams.'''
+import ctypes
+import threading
+import time
+
+import numpy as np
+import pytest
+import torch
+
+import vkjax_amd
+from vkjax_amd import minijax as mj
+from vkjax_amd.jaxpr_interpreter import JaxprInterpreter
+
+pytestmark = pytest.mark.gpu
+jnp = mj.numpy
+
+
+def steps(x, w):
+    y = jnp.dot(x, w)
+    return y + 1.0, jnp.sum(y, axis=1), y * 2.0
+
+
+def numbers(seed, *shape):
+    return np.random.default_rng(seed).integers(-9, 10, size=shape).astype(np.float32)
+
+
+@pytest.mark.parametrize('rows', (1, 7, 300))
+def test_every_call_has_its_own_results(rows):
+    '''More calls than are made between two synchronisations of the stream; results of one block and of several.'''
+    print('calls:', rows, flush=True)
+    f, w = vkjax_amd.wrap(steps, frontend='minijax'), numbers(1, 24, 40)
+    for k in range(150):
+        x = numbers(k + 2, rows, 24)
+        y = x @ w
+        for got, want in zip(f(x, w), (y + 1, y.sum(axis=1), y * 2)):
+            assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize('count', (16, 17, 40))
+def test_more_results_than_one_launch_carries(count):
+    f = vkjax_amd.wrap(lambda x: tuple(x * float(k + 1) for k in range(count)), frontend='minijax')
+    for seed in range(5):
+        x = numbers(seed, 3, 5)
+        for k, got in enumerate(f(x)):
+            assert np.array_equal(got, x * (k + 1))
+
+
+def test_results_larger_than_what_is_carried():
+    f = vkjax_amd.wrap(lambda x: (x + 1.0, jnp.sum(x)), frontend='minijax')
+    for seed in range(3):
+        x = numbers(seed, 300, 400)
+        got, total = f(x)
+        assert np.array_equal(got, x + 1) and total == x.sum()
+
+
+class InHBM:
+    def __init__(self, buffer):
+        self.__cuda_array_interface__ = dict(shape=buffer.shape, typestr='<f4', data=(buffer.tensor.device_ptr(), False), version=2)
+
+
+def test_a_replay_is_over_when_it_returns():
+    '''Read on another stream right behind it; the elapsed time is that of the device.'''
+    program = JaxprInterpreter(mj.make_jaxpr(steps)(numbers(0, 2000, 24), numbers(1, 24, 40)))
+    ctypes.CDLL('libamdhip64.so.7').hipGetLastError()       #(what looking kernels up has left: torch's next call would report it)
+    outputs = [torch.as_tensor(InHBM(b), device='cuda') for b in program.output_buffers]
+    w, other = numbers(1, 24, 40), torch.cuda.Stream()
+    for k in range(100):
+        x = numbers(k + 2, 2000, 24)
+        program.upload_inputs(x, w)
+        begun = time.perf_counter()
+        ms    = program.replay(1 + k % 3)
+        wall  = (time.perf_counter() - begun) * 1e3
+        with torch.cuda.stream(other):
+            seen = [o.clone() for o in outputs]
+        other.synchronize()
+        y = x @ w
+        assert all(np.array_equal(a.cpu().numpy(), b) for a, b in zip(seen, (y + 1, y.sum(axis=1), y * 2)))
+        assert 0 < ms <= wall
+
+
+def test_threads_with_programs_of_their_own():
+    failures = []
+    def work(seed):
+        try:
+            f, w = vkjax_amd.wrap(lambda x, w: steps(x, w)[:1 + seed % 3], frontend='minijax'), numbers(seed, 24, 40)
+            for k in range(60):
+                x = numbers(100 * seed + k, 1 + 50 * (seed % 2), 24)
+                y = x @ w
+                got = f(x, w)
+                got = got if isinstance(got, tuple) else (got,)
+                for a, b in zip(got, (y + 1, y.sum(axis=1), y * 2)):
+                    if not np.array_equal(a, b):
+                        failures.append((seed, k))
+        except BaseException as e:
+            failures.append((seed, repr(e)))
+    threads = [threading.Thread(target=work, args=(seed,)) for seed in range(4)]
+    for t in threads: t.start()
+    for t in threads: t.join()
+    assert not failures, failures[:5]

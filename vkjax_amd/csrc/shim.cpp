@@ -5,6 +5,7 @@
 #include "shim_internal.h"
 
 #include <atomic>
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -175,6 +176,8 @@ int use(Ctx* c) {
 }
 
 void destroy_ctx_objects(Ctx* c) {
+    if (c->carry_count) hipFree(c->carry_count);
+    c->carry_count = nullptr;
     if (c->ev_begin)    hipEventDestroy(c->ev_begin);
     if (c->ev_end)      hipEventDestroy(c->ev_end);
     if (c->ev_landed)   hipEventDestroy(c->ev_landed);
@@ -292,6 +295,26 @@ int issue_all(Ctx* c, Seq* s, size_t first = 0) {
     }
     HIP_TRY(hipEventRecord(s->ev_join, c->side_stream));
     HIP_TRY(hipStreamWaitEvent(c->stream, s->ev_join, 0));
+    return 0;
+}
+
+// Waits until the launch that announces `number` has, and with it everything in front of it on the stream
+int wait_for(Ctx* c, Seq* s, uint64_t number) {
+    const auto started = std::chrono::steady_clock::now();
+    for (;;) {
+        for (int k = 0; k < 64; k++) {
+            if (__atomic_load_n(&s->mailbox->done, __ATOMIC_ACQUIRE) == number) {
+                if (++c->polls < POLLS_IN_A_ROW) return 0;
+                c->polls = 0;
+                HIP_TRY(hipStreamSynchronize(c->stream));
+                return 0;
+            }
+            __builtin_ia32_pause();
+        }
+        if (std::chrono::duration<double>(std::chrono::steady_clock::now() - started).count() > POLL_SECONDS) break;
+    }
+    c->polls = 0;
+    HIP_TRY(hipStreamSynchronize(c->stream));
     return 0;
 }
 
@@ -596,8 +619,11 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
     // queue in order, and a download queued first waits there for the launches, with every upload
     // behind it, even one from the other stream, waiting as well.
     size_t nchunk_events = 0;
+    uint64_t number = 0;                         // not 0: the last launch tells the host under this number that everything is over
     if (down && c->carry) {
         Carry what;
+        bool all = s->mailbox && !s->profiling && !landed;
+        for (auto& t : s->downloads) all = all && (!t.nbytes || (t.nbytes <= CARRY_OUT_MAX && carried((char*)t.buf->dptr + t.offset, t.staging, t.nbytes)));
         for (auto& t : s->downloads) {
             if (!t.nbytes || t.nbytes > CARRY_OUT_MAX || !carried((char*)t.buf->dptr + t.offset, t.staging, t.nbytes)) continue;
             if (what.count == Carry::MAX) {
@@ -606,7 +632,8 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
             }
             what.range[what.count++] = {t.staging, (char*)t.buf->dptr + t.offset, t.nbytes};
         }
-        if (int r = c->carry(what, true, c->stream)) return r;
+        if (all && what.count) number = ++s->evaluations;
+        if (int r = number ? c->carry_out(what, Notice{c->carry_count, &s->mailbox->done, number}, c->stream) : c->carry(what, true, c->stream)) return r;
     }
     if (down) for (auto& t : s->downloads) {
         if (!t.nbytes || (c->carry && t.nbytes <= CARRY_OUT_MAX && carried((char*)t.buf->dptr + t.offset, t.staging, t.nbytes))) continue;
@@ -649,7 +676,11 @@ int vkj::seq_eval(Seq* s, void* const* host_ptrs, int nslots, uint32_t flags, vo
             first_event += (t.nbytes + STAGE_CHUNK - 1) / STAGE_CHUNK;
         }
     }
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (number) {
+        if (int r = wait_for(c, s, number)) return r;
+    } else {
+        HIP_TRY(hipStreamSynchronize(c->stream));
+    }
     if (down) for (auto& t : s->downloads)
         if (t.nbytes && t.nbytes < STAGE_MIN) memcpy(host_ptrs[t.slot], t.staging, t.nbytes);
     if (s->profiling) s->stamps_valid = (int)nstamps;
@@ -949,6 +980,15 @@ int vkj_seq_create(vkj_handle h, int profiling, vkj_handle* out) {
     if (!s) return fail(VKJ_ENOMEM, "vkj_seq_create: out of host memory");
     s->ctx = c;
     s->profiling = profiling != 0;
+    if (c->stamp) {
+        hipError_t e = hipSetDevice(c->device);
+        if (e == hipSuccess) e = hipHostMalloc((void**)&s->mailbox, sizeof(Mailbox), hipHostMallocDefault);
+        if (e != hipSuccess) {
+            delete s;
+            return hip_fail(e, "hipHostMalloc (mailbox)");
+        }
+        *s->mailbox = Mailbox{0, 0, 0};
+    }
     *out = to_handle(s);
     return 0;
 }
@@ -959,6 +999,7 @@ int vkj_seq_destroy(vkj_handle sh) {
     if (int r = use(s->ctx)) return r;
     hipStreamSynchronize(s->ctx->stream);
     hipStreamSynchronize(s->ctx->copy_stream);
+    if (s->mailbox) hipHostFree(s->mailbox);
     for (auto& m : s->slab_mirrors) hipHostFree(m.second);
     for (auto& t : s->uploads) {
         if (t.staging && !t.staging_mirrors_slab) hipHostFree(t.staging);
@@ -1178,6 +1219,16 @@ int vkj_seq_replay(vkj_handle sh, int iters, float* ms_total) {
     if (!s || iters < 1) return fail(VKJ_EINVAL, "vkj_seq_replay: bad argument");
     Ctx* c = s->ctx;
     if (int r = use(c)) return r;
+    if (s->mailbox) {
+        if (int r = c->stamp(&s->mailbox->begin, nullptr, 0, c->stream)) return r;
+        for (int it = 0; it < iters; it++)
+            if (int r = issue_all(c, s)) return r;
+        const uint64_t number = ++s->evaluations;
+        if (int r = c->stamp(&s->mailbox->end, &s->mailbox->done, number, c->stream)) return r;
+        if (int r = wait_for(c, s, number)) return r;
+        if (ms_total) *ms_total = (float)((double)(s->mailbox->end - s->mailbox->begin) / c->clock_khz);
+        return 0;
+    }
     HIP_TRY(hipEventRecord(c->ev_begin, c->stream));
     for (int it = 0; it < iters; it++)
         if (int r = issue_all(c, s)) return r;

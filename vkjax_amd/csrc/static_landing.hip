@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void move_landed(unsigned char* __restrict__ d
 
 // Every range of the table; block (x, y) copies its share of range y. Host memory is read and written at system scope, past the caches: what
 // an earlier launch found there is not what the host has put there since.
-__global__ __launch_bounds__(256) void carry_ranges(Carry what, int to_host) {
+__global__ __launch_bounds__(256) void carry_ranges(Carry what, int to_host, Notice notice) {
     const auto r = what.range[blockIdx.y];
     const uint32_t stride = gridDim.x * 256u, first = blockIdx.x * 256u + threadIdx.x;
     const bool vectors = (((uintptr_t)r.dst | (uintptr_t)r.src) & 15u) == 0;
@@ -62,9 +62,30 @@ __global__ __launch_bounds__(256) void carry_ranges(Carry what, int to_host) {
         if (to_host) __builtin_amdgcn_raw_buffer_store_b32(__builtin_amdgcn_raw_buffer_load_b32(from, w * 4u, 0, 0), to, w * 4u, 0, SYSTEM);
         else         __builtin_amdgcn_raw_buffer_store_b32(__builtin_amdgcn_raw_buffer_load_b32(from, w * 4u, 0, SYSTEM), to, w * 4u, 0, 0);
     }
+    if (notice.done == nullptr) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                    // this block's share is in the host's memory
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const uint32_t blocks = gridDim.x * gridDim.y;
+    if (blocks > 1u) {
+        if (__hip_atomic_fetch_add(notice.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u != blocks) return;
+        __hip_atomic_store(notice.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __hip_atomic_store(notice.done, notice.number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-int carry_on(const Carry& what, bool to_host, hipStream_t stream) {
+__global__ void write_stamp(uint64_t* clock, uint64_t* done, uint64_t number) {
+    __hip_atomic_store(clock, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (done) __hip_atomic_store(done, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+int stamp_on(uint64_t* clock, uint64_t* done, uint64_t number, hipStream_t stream) {
+    void* args[] = {&clock, &done, &number};
+    HIP_TRY(hipLaunchKernel((const void*)write_stamp, dim3(1), dim3(1), args, 0, stream));
+    return 0;
+}
+
+int carry_ranges_on(const Carry& what, bool to_host, const Notice& notice, hipStream_t stream) {
     if (!what.count) return 0;
     uint64_t most = 0;
     for (int k = 0; k < what.count; k++) most = std::max<uint64_t>(most, what.range[k].nbytes);
@@ -72,10 +93,14 @@ int carry_on(const Carry& what, bool to_host, hipStream_t stream) {
     const uint64_t blocks = std::min<uint64_t>(32u, (most + 4095u) / 4096u);
     Carry table = what;
     int out = to_host;
-    void* args[] = {&table, &out};
+    Notice last = notice;
+    void* args[] = {&table, &out, &last};
     HIP_TRY(hipLaunchKernel((const void*)carry_ranges, dim3((unsigned)blocks, (unsigned)what.count), dim3(256), args, 0, stream));
     return 0;
 }
+
+int carry_on(const Carry& what, bool to_host, hipStream_t stream) { return carry_ranges_on(what, to_host, Notice{}, stream); }
+int carry_out_on(const Carry& what, const Notice& notice, hipStream_t stream) { return carry_ranges_on(what, true, notice, stream); }
 
 int move_on(void* dst, const void* src, size_t nbytes, hipStream_t stream) {
     if (!nbytes) return 0;
@@ -102,7 +127,17 @@ int vkj::static_landing_init(Ctx* c) {
     HIP_TRY(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
     if (!p) return fail(VKJ_ENODEV, "vkj_ctx_create: the static landing array has no address on device %d", c->device);
     c->static_landing = p;
+    int khz = 0;
+    HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device));
+    HIP_TRY(hipMalloc((void**)&c->carry_count, 256));
+    HIP_TRY(hipMemset(c->carry_count, 0, 256));
+    HIP_TRY(hipDeviceSynchronize());
     c->carry = carry_on;
+    if (khz > 0) {
+        c->clock_khz = khz;
+        c->carry_out = carry_out_on;
+        c->stamp = stamp_on;
+    }
     return 0;
 }
 
