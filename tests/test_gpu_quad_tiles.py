@@ -1,0 +1,66 @@
+'''The kernels whose four waves share a 32 x 32 tile: contractions around whole k steps and whole vectors,
+windows whose taps change within and between k steps. Whole numbers, so every result is exact.'''
+import numpy as np
+import pytest
+
+from vkjax_amd import kernels as K, minijax as mj
+from tests.common import check_against_oracle
+
+lax, nn, jnp = mj.lax, mj.nn, mj.numpy
+rng = np.random.RandomState(11)
+
+
+def ints(lo, hi, *s):
+    return rng.randint(lo, hi, size=s).astype(np.float32)
+
+
+def layer(x, w, mean, scale, beta, rest):
+    return nn.relu((jnp.dot(x, w) - mean) * scale + beta + rest)
+
+
+def kernels_of(fn):
+    return [l.kernel for l in list(fn._jaxpr_interpreters.values())[0].launches]
+
+
+#one k step of 128 to six, each with the step before and behind full, and remainders within a vector and within a wave's slice of 32
+LENGTHS = (1, 3, 4, 31, 32, 33, 96, 97, 127, 128, 129, 160, 255, 256, 257, 384, 386, 512, 515, 640, 641, 768)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('m,n', ((2, 20), (33, 68), (65, 290), (200, 33)))
+def test_contractions(m, n):
+    for k in LENGTHS:
+        print('four waves per tile:', m, k, n, flush=True)
+        args = [ints(-4, 5, m, k), ints(-3, 4, k, n), ints(-5, 5, n), ints(1, 4, n), ints(-9, 9, n), ints(-50, 50, m, n)]
+        with K.overrides(conv_ksplit=True, conv_k_splits=1, conv_dense_rows=False):
+            _, _, fn = check_against_oracle(layer, args, exact=True)
+        assert kernels_of(fn) == ['conv_gemm_32x32x128_ks4'], kernels_of(fn)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('shares', (2, 5))
+def test_shared_tiles(shares):
+    for m, k, n in ((33, 700, 100), (70, 1300, 260)):
+        args = [ints(-4, 5, m, k), ints(-3, 4, k, n), ints(-5, 5, n), ints(1, 4, n), ints(-9, 9, n), ints(-50, 50, m, n)]
+        with K.overrides(conv_ksplit=True, conv_shares=shares, conv_k_splits=1):
+            _, _, fn = check_against_oracle(layer, args, exact=True)
+        assert kernels_of(fn) == ['conv_gemm_32x32x128_ks4_shared'], kernels_of(fn)
+
+
+#(input, kernel, strides, padding, dilation of the kernel): taps outside on each side, on none, windows wider than the image
+WINDOWS = [((1, 7, 5, 128), (3, 3, 128, 40), (1, 1), 'SAME', (1, 1)), ((2, 9, 8, 128), (3, 2, 128, 33), (2, 1), 'SAME', (1, 1)), ((1, 9, 9, 256), (3, 3, 256, 36), (1, 2), 'VALID', (2, 3)),
+           ((2, 6, 7, 64), (5, 5, 64, 32), (1, 1), 'SAME', (1, 1)), ((1, 4, 3, 192), (3, 5, 192, 20), (1, 1), ((3, 2), (0, 4)), (1, 1)), ((3, 5, 5, 128), (1, 1, 128, 64), (2, 2), 'VALID', (1, 1)),
+           ((1, 6, 6, 128), (2, 3, 128, 32), (1, 1), ((1, 0), (2, 1)), (3, 1))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('general', (False, True))
+@pytest.mark.parametrize('x,w,strides,padding,dilation', WINDOWS)
+def test_windows(x, w, strides, padding, dilation, general):
+    print('four waves per tile:', x, w, strides, padding, dilation, general, flush=True)
+    def f(x, w, shift):
+        return nn.relu(lax.conv_general_dilated(x, w, strides, padding, rhs_dilation=dilation, dimension_numbers=('NHWC', 'HWIO', 'NHWC')) + shift)
+    with K.overrides(conv_ksplit=True, conv_k_splits=1, conv_shares=1, conv_b_general=general, conv_split=False):
+        _, _, fn = check_against_oracle(f, [ints(-4, 5, *x), ints(-3, 4, *w), ints(-9, 9, w[-1])], exact=True)
+    if not (general and x[-1] % 128):
+        assert '_ks4' in kernels_of(fn)[-1], kernels_of(fn)

@@ -84,7 +84,7 @@ def build_call(force=True):
 
 def build_kernel(name, force=True):
     src  = os.path.join(CSRC, 'kernels', f'{name}.hip')
-    deps = [src] + [os.path.join(CSRC, 'kernels', h) for h in ('common.h', 'ew_opcodes.h', 'ew_apply.h', 'conv_split.h', 'split_bf16.h', 'wgrad_split.h')]
+    deps = [src] + [os.path.join(CSRC, 'kernels', h) for h in ('common.h', 'ew_opcodes.h', 'ew_apply.h', 'conv_quad.h', 'conv_split.h', 'split_bf16.h', 'wgrad_split.h')]
     out  = hsaco_path(name)
     if not force and _newer(out, deps):
         return out

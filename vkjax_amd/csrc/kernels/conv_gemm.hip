@@ -36,6 +36,7 @@
 
 #define CONV_MAX_EPI 6
 #define CONV_MAX_SHARES 8        // blocks that share a tile of the four-waves-per-tile kernels and add their sums themselves
+#define CONV_XCD_COLUMNWISE 5    // the XCDs take contiguous ranges of tiles column by column
 #define CONV_OOB 0x80000000u     // byte offset beyond any descriptor: loads give 0, stores are dropped
 
 enum EwOpConv : uint32_t {
@@ -66,16 +67,17 @@ struct ConvParams {
                                     // (acc - vector, * vector, + vector, + full tensor, max(acc, scalar)):
                                     // bit 20+k set = template step k is present;
                                     // bits 25-28: M tiles per block (at least 1);
-                                    // bits 29-31: four-waves-per-tile kernels: 0, or 1 + log2 of the number of XCD columns
+                                    // bits 29-31: four-waves-per-tile kernels: 0, 1 + log2 of the number of XCD columns, or CONV_XCD_COLUMNWISE
     uint32_t epi_desc[2];           // 10 bits per step, steps 0-2 in [0], 3-5 in [1]: bits 0-7 opcode * 2 +
                                     // (operand is the left argument), bits 8-9 kind: 1 scalar,
                                     // 2 per-feature vector [N], 3 full tensor laid out like out
     uint32_t x_bytes, w_bytes, out_bytes;   // sizes for the buffer descriptors (each below 2^31)
     uint32_t howo_magic, howo_shift;        // n / (Ho*Wo) = mulhi(n, magic) >> shift for 0 <= n < 2^31
     uint32_t wo_magic, wo_shift;            // same for Wo; magic 0 stands for a divisor of 1
-    int32_t LH, LW, xs_c;           // lhs dilation and feature stride
+    int32_t LH, LW, xs_c;           // lhs dilation and feature stride (four-waves-per-tile kernels: LH, LW are the constants of n / Cin, like howo_*)
     int32_t ws_r, ws_s, ws_c, ws_n; // rhs strides
-    int32_t os_b, os_h, os_w, os_n; // out strides
+    int32_t os_b, os_h, os_w, os_n; // out strides (four-waves-per-tile kernels: the constants of n / tiles_n, or tiles_m where tiles go to the
+                                    // XCDs column by column, and of n / (tiles_m * tiles_n); mixed kernels: those of their small tiles)
     int32_t split_tiles_m;          // mixed kernels only: the first split_tiles_m M tiles (of 64 rows) are computed as 64 x 64
                                     // tiles, the rows behind them as 32 x 32 tiles by the blocks that follow in the grid
     int32_t k_split_steps;          // four-waves-per-tile kernels only: 0, or the k steps one block sums. The grid then holds
@@ -86,7 +88,7 @@ struct ConvParams {
                                     // tiles allow: every block takes m_each = tiles_m / m_blocks consecutive tiles, the first
                                     // m_extra = tiles_m % m_blocks blocks one more; the M tiles per block in the flags are then
                                     // ignored. For grids sized to what the GPU holds at once.
-    int32_t m_each, m_extra;
+    int32_t m_each, m_extra;        // (four-waves-per-tile kernels: m_each is the number of slices)
     // The kernels on the bf16 matrix cores (conv_split.h) read some of these words in a way of their own:
     //   flags bit 25 (CONV_SPLIT_MASKED): the epilogue is the backward pass of a ReLU, (+ full tensor), mask, (second result), (* vector), its
     //     operands at fixed places of the pointer table: full tensor, activation, vector, limit, constant; bits 12-15 are then 0 or 1 (there is
@@ -218,16 +220,11 @@ __device__ __forceinline__ void conv_straight_steps(float (&y)[NV], const float 
 // registers, and with them resident waves, even when not taken): both operands on the 16-byte
 // path, k tiles that never straddle kernel taps, a row-major result, an epilogue that fits the
 // straight-line template.
-template <int WGM, int WGN, int TM, int TN, int BK, bool A_FAST, bool B_FAST, bool LEAN, int KSW = 1, bool SHARED = false>
+template <int WGM, int WGN, int TM, int TN, int BK, bool A_FAST, bool B_FAST, bool LEAN>
 __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const ConvRegion region, float* __restrict__ out, const float* __restrict__ x,
                                                const float* __restrict__ w, const ConvEpiPtrs& epi,
-                                               const ConvDerivedPtrs& Dp, const ConvParams& Pk, const ConvDerived& Dk,
-                                               float* __restrict__ partial = nullptr, uint32_t* __restrict__ arrivals = nullptr) {
-    // KSW > 1: KSW groups of WGM x WGN waves share one block tile, each taking a 1/KSW slice of every k
-    // step; their accumulators are added through LDS before the epilogue. For products whose handful of
-    // tiles would otherwise leave most of a CU's four MFMA units idle (a wave can drive only one).
-    static_assert(KSW == 1 || (LEAN && TM == 1 && TN == 1), "k-split blocks exist for the lean single-tile form only");
-    constexpr int BM = 32 * WGM * TM, BN = 32 * WGN * TN, NT = 64 * WGM * WGN * KSW;
+                                               const ConvDerivedPtrs& Dp, const ConvParams& Pk, const ConvDerived& Dk) {
+    constexpr int BM = 32 * WGM * TM, BN = 32 * WGN * TN, NT = 64 * WGM * WGN;
     constexpr int LDA = BK + 4, LDB = BN + 4;
     static_assert((BM * LDA) % 4 == 0 && (BK * LDB) % 4 == 0, "16-byte alignment of the LDS tiles");
     float* const As = pool;                         // [BM][LDA]
@@ -257,22 +254,10 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
     const bool c_contig = LEAN || (P.flags & 1u), flat_rows = P.flags & 2u, masked = P.flags & 4u;
     const int nepi = (P.flags >> 8) & 15u, epi_first_full = (int)((P.flags >> 16) & 15u) - 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int kw = wave / (WGM * WGN), wm = (wave % (WGM * WGN)) / WGN, wn = wave % WGN;
+    const int wm = wave / WGN, wn = wave % WGN;
     const int l32 = lane & 31, half = lane >> 5;
-    // A single 32 x 32 tile whose k steps are shared by KSW waves: every wave loads, parks in LDS and consumes its
-    // own slice of a k step, so the k loop needs no barrier between the waves; they drift apart and one wave's
-    // MFMAs cover the others' load latencies (a block of these kernels is usually alone on its CU).
-    constexpr bool WAVE_PRIVATE = KSW > 1 && WGM == 1 && WGN == 1 && A_FAST;
-    constexpr int  BKW_ = BK / KSW;
     // thread -> (row within a pass, 16-byte vector within the row) of the A tile, (k row, vector) of the B tile
-    const int a_r0 = WAVE_PRIVATE ? lane / (BKW_ / 4) : tid / (BK / 4);
-    const int a_kv = WAVE_PRIVATE ? kw * (BKW_ / 4) + lane % (BKW_ / 4) : tid % (BK / 4);
-    const int b_r0 = WAVE_PRIVATE ? kw * BKW_ + lane / (BN / 4) : tid / (BN / 4);
-    const int b_nv = WAVE_PRIVATE ? lane % (BN / 4) : tid % (BN / 4);
-    auto tile_barrier = [&]() {
-        if constexpr (WAVE_PRIVATE) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // LDS accesses of a wave execute in order
-        else __syncthreads();
-    };
+    const int a_r0 = tid / (BK / 4), a_kv = tid % (BK / 4), b_r0 = tid / (BN / 4), b_nv = tid % (BN / 4);
 
     // A block works through up to `chunk` consecutive M tiles of one N tile, one after the other,
     // as one flat sequence of k steps: while a step is computed the loads of the next one are in
@@ -281,50 +266,16 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
     // Consecutive block ids go to different XCDs (8 of them, each with its own L2). Hand every
     // XCD a contiguous range of work so that the N-tiles of one M-tile share an L2.
     const int chunk = LEAN ? (P.flags >> 25) & 15u : 1;         // the general variants take one tile per block
-    const int m_blocks = LEAN && KSW == 1 ? P.m_blocks : 0;
+    const int m_blocks = LEAN ? P.m_blocks : 0;
     // (every wave runs this once per block on the CU's one scalar unit: divisors that are powers of two, the usual
     // case for the M tiles per block and the number of N tiles, cost a shift instead of the long division sequence)
     auto div_small = [](int n, int d) { return (d & (d - 1)) == 0 ? n >> __builtin_ctz((unsigned)d) : n / d; };
     const int chunks_m = m_blocks > 0 ? m_blocks : div_small(region.tiles_m + chunk - 1, chunk);
     int work = (int)blockIdx.x - region.first_block;
-    // K_SPLIT kernels can share a tile's contraction among several blocks (for products with so few tiles that most
-    // CUs would stay idle while a few fetch all the weights): slice s sums k steps [kbase, kbase + ktiles)
-    constexpr bool K_SPLIT = KSW > 1 && BK == 128;
-    static_assert(!SHARED || K_SPLIT, "shared are tiles whose k steps four waves take");
-    int kbase = 0, ktiles = max(1, (P.K + BK - 1) / BK);       // K = 0 runs as one k step whose loads are all out of range
-    int slice = 0, slices = 1;
-    if constexpr (K_SPLIT) {
-        const int per = Pk.k_split_steps;
-        if (per > 0) {
-            const int tiles = chunks_m * region.tiles_n;
-            slice = work / tiles;
-            work -= slice * tiles;
-            kbase = slice * per;
-            slices = (ktiles + per - 1) / per;
-            ktiles = min(per, ktiles - kbase);
-            if constexpr (!SHARED) out += (size_t)slice * (size_t)P.M * (size_t)P.N;
-        }
-    }
-    // Four-waves-per-tile kernels (products with few tiles, often with the kernel operand as the large one): the host may
-    // ask for the XCDs to be laid over the tile grid as 8 / xn rows of xn columns (flags bits 29-31 hold 1 + log2 xn),
-    // each XCD owning a rectangle of tiles_m / (8 / xn) x tiles_n / xn tiles (both divisible; the host checks). An XCD's
-    // L2 then fetches 1 / (8 / xn) of the rows of A and 1 / xn of the columns of B, instead of a few rows of A and
-    // all of B.
-    const int xcd_code = KSW > 1 ? (int)(P.flags >> 29) : 0;
-    int chunk_m, tile_n;
-    if (xcd_code > 0) {
-        const int xn = 1 << (xcd_code - 1), sub_n = div_small(region.tiles_n, xn);
-        const int x = work & 7, l = work >> 3, xi = x >> (xcd_code - 1), xj = x & (xn - 1);
-        const int sub_m = region.tiles_m >> (4 - xcd_code);                     // tiles_m / (8 / xn)
-        const int lm = div_small(l, sub_n);
-        chunk_m = xi * sub_m + lm;
-        tile_n  = xj * sub_n + (l - lm * sub_n);
-    } else {
-        const int total = chunks_m * region.tiles_n, per = total / 8;
-        if (per > 0 && work < per * 8) work = (work & 7) * per + (work >> 3);
-        chunk_m = div_small(work, region.tiles_n);
-        tile_n  = work - chunk_m * region.tiles_n;
-    }
+    const int total = chunks_m * region.tiles_n, per = total / 8;
+    if (per > 0 && work < per * 8) work = (work & 7) * per + (work >> 3);
+    const int ktiles = max(1, (P.K + BK - 1) / BK);             // K = 0 runs as one k step whose loads are all out of range
+    const int chunk_m = div_small(work, region.tiles_n), tile_n = work - chunk_m * region.tiles_n;
     int tile_m0 = chunk_m * chunk, nsub = LEAN ? min(chunk, region.tiles_m - tile_m0) : 1;
     if (m_blocks > 0) {
         tile_m0 = chunk_m * P.m_each + min(chunk_m, P.m_extra);
@@ -344,9 +295,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
     // never waits on global memory for them. Thread t fetches column t of every step. Every step issues one load,
     // whatever its kind, so that none waits for the one before: an absent operand, one that is derived below, or a
     // full tensor (read in the epilogue) has a descriptor of size 0, which reads nothing and returns 0.
-    // Where a block is alone on its CU (the four-waves-per-tile kernels) they are requested right behind the first
-    // k tile's loads: one round trip to memory for both. Elsewhere they go first, and the other blocks' work covers them.
-    constexpr bool EPI_BEHIND_TILES = KSW > 1;
+    // They go first: the other blocks' work covers them.
     float e_reg[CONV_MAX_EPI], d_in[CONV_MAX_DERIVED + 1];
     uint32_t e_bytes[CONV_MAX_EPI], e_scale[CONV_MAX_EPI];       // (the same in every lane: worked out before the lanes part)
 #pragma unroll
@@ -356,24 +305,21 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
         e_bytes[e] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(kind == 1 ? 4u * present : kind == 2 ? (uint32_t)P.N * 4u * present : 0u));
         e_scale[e] = kind == 2 ? 4u : 0u;
     }
-    auto request_epilogue_operands = [&]() {
-        if (tid < BN) {
+    if (tid < BN) {
 #pragma unroll
-            for (int e = 0; e < CONV_MAX_EPI; ++e)
-                e_reg[e] = buffer_load_x1(make_rsrc(epi.p[e], e_bytes[e]), (uint32_t)(n0 + tid) * e_scale[e]);
-            if (Dk.nsteps) {
-                // the arrays of the derived operand: combined once the first k tile's loads are on their way (combining
-                // them at once would hold the wave, and with it the block's first barrier, for a round trip to memory)
+        for (int e = 0; e < CONV_MAX_EPI; ++e)
+            e_reg[e] = buffer_load_x1(make_rsrc(epi.p[e], e_bytes[e]), (uint32_t)(n0 + tid) * e_scale[e]);
+        if (Dk.nsteps) {
+            // the arrays of the derived operand: combined once the first k tile's loads are on their way (combining
+            // them at once would hold the wave, and with it the block's first barrier, for a round trip to memory)
 #pragma unroll
-                for (int k = 0; k <= CONV_MAX_DERIVED; ++k) {
-                    const bool vec = (Dk.vector_mask >> k) & 1u;
-                    d_in[k] = buffer_load_x1(make_rsrc(Dp.p[k], Dp.p[k] == nullptr ? 0u : vec ? (uint32_t)P.N * 4u : 4u),
-                                             vec ? (uint32_t)(n0 + tid) * 4u : 0u);
-                }
+            for (int k = 0; k <= CONV_MAX_DERIVED; ++k) {
+                const bool vec = (Dk.vector_mask >> k) & 1u;
+                d_in[k] = buffer_load_x1(make_rsrc(Dp.p[k], Dp.p[k] == nullptr ? 0u : vec ? (uint32_t)P.N * 4u : 4u),
+                                         vec ? (uint32_t)(n0 + tid) * 4u : 0u);
             }
         }
-    };
-    if constexpr (!EPI_BEHIND_TILES) request_epilogue_operands();
+    }
     // the first full-size operand (a residual input) is fetched for a whole tile at once, while
     // the tile's last k step is computed (for the largest tile that would not fit the register
     // file: it loads sub-tile by sub-tile in the epilogue)
@@ -387,7 +333,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
     // ---------------- per-thread load assignment ----------------
     // A fast: 16-byte vectors along k. A generic: one row, a run of consecutive k.
     constexpr int A_VPR   = BK / 4;                 // vectors per row
-    constexpr int A_RSTEP = WAVE_PRIVATE ? 64 / (BKW_ / 4) : NT / A_VPR;   // rows between a thread's vectors
+    constexpr int A_RSTEP = NT / A_VPR;             // rows between a thread's vectors
     constexpr int A_NV    = BM / A_RSTEP;           // vectors per thread
     constexpr int A_KG    = NT / BM;                // generic: k groups
     constexpr int A_KPT   = BK / A_KG;              // generic: k per thread
@@ -441,37 +387,27 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
             }
         }
         t_r = 0; t_s = 0; t_c = 0;
-        if constexpr (K_SPLIT) {
-            if (kbase > 0) {                          // a later slice of the contraction starts at its own tap and feature
-                const int k0 = kbase * BK, rs = k0 / P.Cin;
-                t_c = k0 - rs * P.Cin; t_r = rs / P.KW; t_s = rs - t_r * P.KW;
-            }
-        }
         ak = A_FAST ? a_kv * 4 : (tid / BM) * A_KPT;
         const int rs = ak / P.Cin;
         ac = ak - rs * P.Cin; ar = rs / P.KW; as_ = rs - ar * P.KW;
     };
 
     constexpr int B_VPR   = BN / 4;
-    constexpr int B_RSTEP = WAVE_PRIVATE ? 64 / B_VPR : NT / B_VPR;
-    constexpr int B_NV    = (WAVE_PRIVATE ? BKW_ : BK) / B_RSTEP;
+    constexpr int B_RSTEP = NT / B_VPR;
+    constexpr int B_NV    = BK / B_RSTEP;
     constexpr int B_KG    = NT / BN;                // generic: k groups
     constexpr int B_KPT   = BK / B_KG;
     // B fast: byte offset of this thread's first vector in tile 0, or out of range for columns >= N
     const int      b_n    = n0 + b_nv * 4;
     const uint32_t b_voff = b_n < P.N ? (uint32_t)(b_r0 * P.N + b_n) * 4u : CONV_OOB;
 
-    // what a thread has requested of the coming k step(s): one step ahead, two for the wave-private tiles, whose
-    // single block per CU has nothing else to cover a load's latency with
-    // (not for the small tiles of the mixed kernels, k step 64: their registers decide how many blocks share a CU;
-    // nor with element-wise loads of B, whose 16 values per step and stage would spill)
-    constexpr int STAGES = WAVE_PRIVATE && BK >= 128 && B_FAST ? 2 : 1;
-    f32x4 a_reg[STAGES][A_FAST ? A_NV : 1];
+    // what a thread has requested of the coming k step
+    f32x4 a_reg[A_FAST ? A_NV : 1];
     float a_sreg[A_FAST ? 1 : A_KPT];
-    f32x4 b_reg[STAGES][B_FAST ? B_NV : 1];
-    float b_sreg[STAGES][B_FAST ? 1 : B_KPT];
+    f32x4 b_reg[B_FAST ? B_NV : 1];
+    float b_sreg[B_FAST ? 1 : B_KPT];
 
-    auto load_tiles = [&](int k0, int st = 0) {
+    auto load_tiles = [&](int k0) {
         // ---- A ----
         if constexpr (A_FAST) {
             if (uniform_taps) {
@@ -481,14 +417,14 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
                 if (!masked && !tail) {
                     // the common case issues the loads with no vector arithmetic at all
 #pragma unroll
-                    for (int p = 0; p < A_NV; ++p) a_reg[st][p] = buffer_load_x4(x_rsrc, a_voff[p], soff);
+                    for (int p = 0; p < A_NV; ++p) a_reg[p] = buffer_load_x4(x_rsrc, a_voff[p], soff);
                 } else {
                     const uint32_t sh   = 31u - (uint32_t)(t_r * P.KW + t_s);
                     const bool     kbad = tail && k0 + a_kv * 4 >= P.K;
 #pragma unroll
                     for (int p = 0; p < A_NV; ++p) {
                         const uint32_t v = a_voff[p] | ((a_inv[p] << sh) & CONV_OOB);
-                        a_reg[st][p] = buffer_load_x4(x_rsrc, kbad ? CONV_OOB : v, soff);
+                        a_reg[p] = buffer_load_x4(x_rsrc, kbad ? CONV_OOB : v, soff);
                     }
                 }
             } else {
@@ -499,7 +435,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
                 for (int p = 0; p < A_NV; ++p) {
                     uint32_t v = (a_voff[p] + koff) | (a_voff[p] & CONV_OOB);
                     if (masked) v |= (a_inv[p] << sh) & CONV_OOB;
-                    a_reg[st][p] = buffer_load_x4(x_rsrc, kok ? v : CONV_OOB);
+                    a_reg[p] = buffer_load_x4(x_rsrc, kok ? v : CONV_OOB);
                 }
             }
         } else {
@@ -521,7 +457,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
             // rows k >= K fall beyond the descriptor and read as zeros
 #pragma unroll
             for (int p = 0; p < B_NV; ++p)
-                b_reg[st][p] = buffer_load_x4(w_rsrc, b_voff, (uint32_t)(k0 + p * B_RSTEP) * (uint32_t)P.N * 4u);
+                b_reg[p] = buffer_load_x4(w_rsrc, b_voff, (uint32_t)(k0 + p * B_RSTEP) * (uint32_t)P.N * 4u);
         } else {
             const int n = n0 + tid % BN;
             int k = k0 + (tid / BN) * B_KPT;
@@ -529,7 +465,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
             int c = k - rs * P.Cin, r = rs / P.KW, s = rs - r * P.KW;
 #pragma unroll
             for (int j = 0; j < B_KPT; ++j) {
-                b_sreg[st][j] = (k < P.K && n < P.N) ? w[r * Pk.ws_r + s * Pk.ws_s + c * Pk.ws_c + n * Pk.ws_n] : 0.f;
+                b_sreg[j] = (k < P.K && n < P.N) ? w[r * Pk.ws_r + s * Pk.ws_s + c * Pk.ws_c + n * Pk.ws_n] : 0.f;
                 ++k; ++c;
                 if (c == P.Cin) { c = 0; ++s; if (s == P.KW) { s = 0; ++r; } }
             }
@@ -544,7 +480,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
         }
     };
 
-    auto store_tiles = [&](int k0, int st = 0) {
+    auto store_tiles = [&](int k0) {
         if constexpr (A_FAST) {
             // A contraction that ends within a vector (only with a single tap): what lies behind it is the next row's. The kernel operand's rows
             // there read as zeros, which a value that is not finite would not leave alone.
@@ -552,12 +488,12 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
 #pragma unroll
                 for (int p = 0; p < A_NV; ++p)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) a_reg[st][p][q] = k0 + a_kv * 4 + q < P.K ? a_reg[st][p][q] : 0.f;
+                    for (int q = 0; q < 4; ++q) a_reg[p][q] = k0 + a_kv * 4 + q < P.K ? a_reg[p][q] : 0.f;
             }
 #pragma unroll
             for (int p = 0; p < A_NV; ++p) {
                 const int row = a_r0 + p * A_RSTEP, kv = a_kv;
-                *reinterpret_cast<f32x4*>(&As[row * LDA + kv * 4]) = a_reg[st][p];
+                *reinterpret_cast<f32x4*>(&As[row * LDA + kv * 4]) = a_reg[p];
             }
         } else {
             const int row = tid % BM, kb = (tid / BM) * A_KPT;
@@ -568,12 +504,12 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
 #pragma unroll
             for (int p = 0; p < B_NV; ++p) {
                 const int kr = b_r0 + p * B_RSTEP, nv = b_nv;
-                *reinterpret_cast<f32x4*>(&Bs[kr * LDB + nv * 4]) = b_reg[st][p];
+                *reinterpret_cast<f32x4*>(&Bs[kr * LDB + nv * 4]) = b_reg[p];
             }
         } else {
             const int n = tid % BN, kb = (tid / BN) * B_KPT;
 #pragma unroll
-            for (int j = 0; j < B_KPT; ++j) Bs[(kb + j) * LDB + n] = b_sreg[st][j];
+            for (int j = 0; j < B_KPT; ++j) Bs[(kb + j) * LDB + n] = b_sreg[j];
         }
     };
 
@@ -606,22 +542,9 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
         }
     };
 
-    // the same for a wave's quarter of the one tile of a block whose four waves share it (the result is a row-major matrix there)
-    auto quarter_tile = [&](auto&& fn) {
-        const int n = n0 + l32, first = 8 * __builtin_amdgcn_readfirstlane(kw);
-        const uint32_t base = n < P.N ? (uint32_t)((region.m_base + tile_m0 * BM + 4 * half) * P.N + n) * 4u : CONV_OOB, rowb = (uint32_t)P.N * 4u;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) fn(v, base, (uint32_t)(first + v) * rowb);
-    };
-
     float full[PREFETCH_FULL ? TM : 1][PREFETCH_FULL ? TN : 1][16];
-    float quarter[4] = {0.f, 0.f, 0.f, 0.f};                     // ... and of its residual, requested before the product is computed
     setup_rows(region.m_base + tile_m0 * BM);
-    load_tiles(kbase * BK);
-    if constexpr (EPI_BEHIND_TILES) request_epilogue_operands();
-    if constexpr (KSW > 1) {
-        if (P.flags & (8u << 20)) quarter_tile([&](int v, uint32_t vo, uint32_t so) { quarter[v] = buffer_load_x1_nt(f_rsrc, vo, so); });
-    }
+    load_tiles(0);
     if (tid < BN) {
         if (Dk.nsteps) {
             const float v = conv_derived_value(d_in, Dk);
@@ -639,11 +562,11 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
     // lanes 32-63 the second half. Fragments are double-buffered in registers: the LDS reads of
     // group g+1 are in flight while the MFMAs of group g execute.
     auto compute = [&]() {
-        constexpr int BKW = BK / KSW, G = BKW / 8;               // this wave's slice of the k step
+        constexpr int G = BK / 8;
         f32x4 af[2][TM];
         float bf[2][TN][4];
         auto load_frags = [&](int g, int buf) {
-            const int kk = kw * BKW + half * (BKW / 2) + g * 4;
+            const int kk = half * (BK / 2) + g * 4;
 #pragma unroll
             for (int i = 0; i < TM; ++i)
                 af[buf][i] = *reinterpret_cast<const f32x4*>(&As[((wm * TM + i) * 32 + l32) * LDA + kk]);
@@ -672,55 +595,33 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
-        if constexpr (STAGES == 2) {
-            // Two k steps of loads in flight per wave, the stages alternating (written out twice: the stage is a
-            // compile-time index into the registers). The waves meet once, behind the first store, which also
-            // publishes the epilogue operands parked in LDS, and again before the reduction reuses the tiles.
-            if (ktiles > 1) load_tiles((kbase + 1) * BK, 1);
-            for (int kt = 0; kt < ktiles; kt += 2) {
-                store_tiles((kbase + kt) * BK, 0);
-                if (kt == 0) __syncthreads(); else tile_barrier();
-                if (kt + 2 < ktiles) load_tiles((kbase + kt + 2) * BK, 0);
-                compute();
-                tile_barrier();
-                if (kt + 1 < ktiles) {
-                    store_tiles((kbase + kt + 1) * BK, 1);
-                    tile_barrier();
-                    if (kt + 3 < ktiles) load_tiles((kbase + kt + 3) * BK, 1);
-                    compute();
-                    tile_barrier();
-                }
-            }
+        // all k steps but the last: the next step's loads are in flight during the MFMAs
+        for (int kt = 1; kt < ktiles; ++kt) {
+            store_tiles((kt - 1) * BK);
             __syncthreads();
-        } else {
-            // all k steps but the last: the next step's loads are in flight during the MFMAs
-            for (int kt = 1; kt < ktiles; ++kt) {
-                store_tiles((kbase + kt - 1) * BK);
-                tile_barrier();
-                load_tiles((kbase + kt) * BK);
-                compute();
-                tile_barrier();
-            }
-            // last k step: the loads in flight are those of the next M tile's first step and of
-            // the residual operand
-            store_tiles((kbase + ktiles - 1) * BK);
-            __syncthreads();                 // (also where wave-private tiles publish the epilogue operands parked in LDS)
-            if (sub + 1 < nsub) {
-                setup_rows(m0 + BM);
-                load_tiles(kbase * BK);
-            }
-            if (first_full >= 0) {
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        sub_tile(m0, i, j, [&](int v, uint32_t vo, uint32_t so) {
-                            full[PREFETCH_FULL ? i : 0][PREFETCH_FULL ? j : 0][v] = buffer_load_x1(f_rsrc, vo, so);
-                        });
-            }
+            load_tiles(kt * BK);
             compute();
             __syncthreads();
         }
+        // last k step: the loads in flight are those of the next M tile's first step and of
+        // the residual operand
+        store_tiles((ktiles - 1) * BK);
+        __syncthreads();
+        if (sub + 1 < nsub) {
+            setup_rows(m0 + BM);
+            load_tiles(0);
+        }
+        if (first_full >= 0) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    sub_tile(m0, i, j, [&](int v, uint32_t vo, uint32_t so) {
+                        full[PREFETCH_FULL ? i : 0][PREFETCH_FULL ? j : 0][v] = buffer_load_x1(f_rsrc, vo, so);
+                    });
+        }
+        compute();
+        __syncthreads();
 
         // ---------------- epilogue + store of the finished M tile ----------------
         // Outputs that are not a row-major [M, N] matrix need (batch, y, x) of every row: decoded
@@ -732,49 +633,6 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
                 Rs[r] = m < P.M ? b * Pk.os_b + ho * Pk.os_h + wo * Pk.os_w : -1;
             }
             __syncthreads();
-        }
-        if constexpr (KSW > 1) {
-            // The k slices meet in LDS (the A and B tiles are done with), and every wave finishes a quarter of the tile: rows 8 kw + 4 half ..
-            // + 3 of its column. (The first wave finishing all of it, with the residual requested
-            // only then: the launches of ResNet-50 on one image 516 us, so 502.)
-            static_assert(KSW == 4 && WGM * WGN * TM * TN == 1 && KSW * 16 * 64 <= BM * LDA + BK * LDB, "sixteen values per lane of each of four waves, in the A and B tiles (B follows A)");
-            f32x4* const red = reinterpret_cast<f32x4*>(As);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) red[(kw * 4 + q) * 64 + lane] = f32x4{acc[0][0][4 * q], acc[0][0][4 * q + 1], acc[0][0][4 * q + 2], acc[0][0][4 * q + 3]};
-            __syncthreads();
-            f32x4 sum = red[kw * 64 + lane];
-#pragma unroll
-            for (int s = 1; s < KSW; ++s) sum += red[(s * 4 + kw) * 64 + lane];
-            if constexpr (SHARED) {
-                // A slice leaves its sums in memory; the block that arrives last at the tile's counter, which it sets back, adds all of them in
-                // their order. No block waits for another.
-                constexpr uint32_t TILE = BM * BN * 4u;
-                const int tile = chunk_m * region.tiles_n + tile_n;
-                const __amdgpu_buffer_rsrc_t p_rsrc = make_rsrc(reinterpret_cast<const char*>(partial) + (size_t)tile * (size_t)slices * TILE, (uint32_t)slices * TILE);
-                buffer_store_x4_agent(sum, p_rsrc, (uint32_t)tid * 16u, (uint32_t)slice * TILE);
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the sums have reached memory
-                __syncthreads();
-                if (tid == 0) {
-                    const uint32_t n = __hip_atomic_fetch_add(arrivals + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if (n + 1u == (uint32_t)slices) __hip_atomic_store(arrivals + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    Rs[0] = (int)n;
-                }
-                __syncthreads();
-                if (Rs[0] + 1 != slices) return;
-                f32x4 q[CONV_MAX_SHARES];                              // requested together; beyond the last slice the loads read zeros, which are not added
-#pragma unroll
-                for (int s = 0; s < CONV_MAX_SHARES; ++s) q[s] = buffer_load_x4_agent(p_rsrc, (uint32_t)tid * 16u, (uint32_t)s * TILE);
-                sum = q[0];
-#pragma unroll
-                for (int s = 1; s < CONV_MAX_SHARES; ++s)
-                    if (s < slices) sum += q[s];
-            }
-            float y[4] = {sum[0], sum[1], sum[2], sum[3]};
-            conv_straight_steps<4>(y, quarter, (P.flags >> 20) & 31u, (int)((P.flags >> 12) & 15u) - 1, Es, BN, l32, [&]() {
-                quarter_tile([&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], make_rsrc(epi.p[CONV_MAX_EPI - 1], P.out_bytes), vo, so); });
-            });
-            quarter_tile([&](int v, uint32_t vo, uint32_t so) { buffer_store_x1(y[v], o_rsrc, vo, so); });
-            return;                                               // one M tile per block, a row-major result
         }
         // From here on the accumulators are handled as separate scalars: element-wise updates of a
         // 16-register MFMA tuple make the compiler copy the whole tuple at every step.
@@ -851,13 +709,13 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
     }
 }
 
-#define CONV_KERNEL(name, WGM, WGN, TM, TN, BK, AF, BF, LEAN, ...)                                          \
-    extern "C" __global__ __launch_bounds__(64 * WGM * WGN * (1, ##__VA_ARGS__)) __attribute__((amdgpu_waves_per_eu(2))) void name( \
+#define CONV_KERNEL(name, WGM, WGN, TM, TN, BK, AF, BF, LEAN)                                               \
+    extern "C" __global__ __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(2))) void name( \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
         ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
         __shared__ __attribute__((aligned(16))) float pool[conv_pool_floats<WGM, WGN, TM, TN, BK>()];        \
         const ConvRegion all{0, P.tiles_m, P.tiles_n, 0};                                                    \
-        conv_gemm_body<WGM, WGN, TM, TN, BK, AF, BF, LEAN, ##__VA_ARGS__>(pool, all, out, x, w, epi, dp, P, D); \
+        conv_gemm_body<WGM, WGN, TM, TN, BK, AF, BF, LEAN>(pool, all, out, x, w, epi, dp, P, D);               \
     }
 
 // name = conv_gemm_<BM>x<BN>x<BK>_<a><b>  with a/b = f (16-byte loads) or g (generic strided loads),
@@ -873,24 +731,33 @@ CONV_TILE(64x64x32, 2, 2, 1, 1, 32)
 CONV_TILE(64x64x64, 2, 2, 1, 1, 64)
 CONV_TILE(32x32x32, 1, 1, 1, 1, 32)
 CONV_TILE(32x32x64, 1, 1, 1, 1, 64)
-// one 32 x 32 tile per block, the k step of 128 split over four waves (chunk 1; see KSW above)
-CONV_KERNEL(conv_gemm_32x32x128_ks4, 1, 1, 1, 1, 128, true, true, true, 4)
+#include "conv_quad.h"
+
+// one 32 x 32 tile per block, the k step of 128 split over four waves (chunk 1)
+#define CONV_QUAD_KERNEL(name, BK, BF)                                                                       \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BF ? 3 : 2))) void name(          \
+        float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
+        ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
+        __shared__ __attribute__((aligned(16))) float pool[conv_quad_floats<BK>()];                          \
+        const ConvRegion all{0, P.tiles_m, P.tiles_n, 0};                                                    \
+        conv_quad_body<BK, BF, false>(pool, all, out, x, w, epi, dp, P, D);                                  \
+    }
+CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4, 128, true)
 // the same with element-wise loads of the kernel operand (an output width that is no multiple of 4)
-CONV_KERNEL(conv_gemm_32x32x128_ks4g, 1, 1, 1, 1, 128, true, false, true, 4)
+CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4g, 128, false)
 // the same with a 64-long k step, for windows over 64 (or 192, ...) input features, whose taps a 128-long step would straddle
-CONV_KERNEL(conv_gemm_32x32x64_ks4, 1, 1, 1, 1, 64, true, true, true, 4)
-// The first two with several blocks per tile, each summing a slice of the contraction (k_split_steps): one block alone on its CU waits for its loads and
-// LDS reads between its matrix instructions (0.8 us per k step, 0.43 at the rate of the matrix cores; two together 1.36), and few tiles leave
-// CUs idle. A slice's sums make a round trip to memory and the counter another, 2 us for 32 x 32 numbers; a launch that adds them takes 3.2 and a start.
-// 196 x 2304 x 256 11.8 -> 10.8 us, 784 x 1152 x 128 11.6 -> 10.4, 196 x 1024 x 256 9.5 -> 7.5 (before: that launch), 588 x 4608 x 512 48.6 -> 34.8.
+CONV_QUAD_KERNEL(conv_gemm_32x32x64_ks4, 64, true)
+// The first two with several blocks per tile, each summing a slice of the contraction (k_split_steps): few tiles leave CUs idle. A slice's sums make a
+// round trip to memory and the counter another, 2 to 2.5 us for 32 x 32 numbers; a launch that adds them takes 3.2 and a start.
+// 196 x 2304 x 256: 13.2 us by one block per tile, 8.5 by four; 150 x 4608 x 512 22.4, 12.2 by three; 588 x 4608 x 512 38.6, 29.6 by four.
 #define CONV_SHARED_KERNEL(name, BF)                                                                         \
-    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void name(          \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BF ? 3 : 2))) void name(          \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
         float* __restrict__ partial, uint32_t* __restrict__ arrivals,                                        \
         ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
-        __shared__ __attribute__((aligned(16))) float pool[conv_pool_floats<1, 1, 1, 1, 128>()];             \
+        __shared__ __attribute__((aligned(16))) float pool[conv_quad_floats<128>()];                         \
         const ConvRegion all{0, P.tiles_m, P.tiles_n, 0};                                                    \
-        conv_gemm_body<1, 1, 1, 1, 128, true, BF, true, 4, true>(pool, all, out, x, w, epi, dp, P, D, partial, arrivals); \
+        conv_quad_body<128, BF, true>(pool, all, out, x, w, epi, dp, P, D, partial, arrivals);               \
     }
 CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4_shared, true)
 CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4g_shared, false)
@@ -898,14 +765,14 @@ CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4g_shared, false)
 // with four tiles sets the time, the average is 3.06). The first P.split_tiles_m M tiles are computed as 64 x 64
 // tiles, as many as fill every CU equally; the rows behind them as 32 x 32 tiles of a quarter of the work each
 // (four waves sharing every 64-long k step), which spread over the CUs in finer units. Both kinds of block have 256
-// threads and share one LDS pool; with the 64-long step the kernel needs 127 registers, so four blocks fit a CU
-// (the 128-long step of conv_gemm_32x32x128_ks4 takes 149: three blocks, and the small tiles would wait for
+// threads and share one LDS pool; with the 64-long step the kernel needs 120 registers, so four blocks fit a CU
+// (the 128-long step of conv_gemm_32x32x128_ks4 takes 164: three blocks, and the small tiles would wait for
 // the large ones). One M tile per block (chunk 1).
 #define CONV_MIX_KERNEL(name, BK)                                                                              \
     extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void name(            \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
         ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
-        constexpr int big = conv_pool_floats<2, 2, 1, 1, BK>(), small = conv_pool_floats<1, 1, 1, 1, 64>(); \
+        constexpr int big = conv_pool_floats<2, 2, 1, 1, BK>(), small = conv_quad_floats<64>();              \
         __shared__ __attribute__((aligned(16))) float pool[big > small ? big : small];                       \
         const int n_big = P.split_tiles_m * P.tiles_n;                                                       \
         if ((int)blockIdx.x < n_big) {                                                                       \
@@ -914,7 +781,7 @@ CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4g_shared, false)
         } else {                                                                                             \
             const int m_base = P.split_tiles_m * 64;                                                         \
             const ConvRegion r{n_big, (P.M - m_base + 31) / 32, (P.N + 31) / 32, m_base};                    \
-            conv_gemm_body<1, 1, 1, 1, 64, true, true, true, 4>(pool, r, out, x, w, epi, dp, P, D);         \
+            conv_quad_body<64, true, false>(pool, r, out, x, w, epi, dp, P, D);                              \
         }                                                                                                    \
     }
 CONV_MIX_KERNEL(conv_gemm_64x64x32_mix, 32)

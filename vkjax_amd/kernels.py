@@ -999,6 +999,7 @@ def _four_waves_pay(g: ConvGeometry, b_fast: bool, compute_units: int) -> bool:
 #themselves (conv_share_count). (Shared by eight blocks, 32 tiles x 36 k steps would take 11.2 us instead of 14.4, 32 x 16 7.9 instead of 9.5; but these
 #products are promised two launches: test_long_contractions_of_few_tiles_are_sliced, test_sliced_contractions.)
 CONV_SLICED_MAX_TILES = 32
+CONV_XCD_COLUMNWISE   = 5           #tiles go to the XCDs column by column
 
 
 def conv_k_splits(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int = 256) -> int:
@@ -1169,12 +1170,19 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
     for i, e in enumerate(epilogue):
         assert e.op < 128 and 1 <= e.kind <= 3
         descs[i // 3] |= ((e.op * 2 + int(e.operand_left)) | e.kind << 8) << (10 * (i % 3))
+    slices = g.shares.count if k_split_steps and g.k_splits == 1 else g.k_splits
+    #the kernels whose four waves share a tile divide by multiplying; they need no strides of the result and no dilation of the input
+    dilation, out_strides, per_block = _i32(g.LH, g.LW), _i32(*g.os), _i32(tiles_m // m_blocks if m_blocks else 0)
+    if ksplit or split_tiles_m:
+        rows, columns = (tiles_m, tiles_n) if ksplit else (_cdiv(M - split_tiles_m * 64, 32), _cdiv(N, 32))
+        dilation, per_block = _u32(*_magic_division(g.Cin)), _i32(slices)
+        out_strides = _u32(*_magic_division(rows if flags >> 29 == CONV_XCD_COLUMNWISE else columns), *_magic_division(rows * columns))
     params = (_i32(M, N, K, g.Ho, g.Wo, g.H, g.W, g.Cin, g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.DH, g.DW,
                    *g.xs[:3], tiles_m, tiles_n)
               #(rows beyond M are dropped by the descriptor's size: with slices, that of one slice's matrix)
               + _u32(flags, *descs, x_bytes, w_bytes, M * N * 4 if k_split_steps else (out.size - out_offset) * 4,
                      *_magic_division(g.Ho * g.Wo), *_magic_division(g.Wo))
-              + _i32(g.LH, g.LW, g.xs[3], *g.ws, *g.os, split_tiles_m, k_split_steps, m_blocks, tiles_m // m_blocks if m_blocks else 0, tiles_m % m_blocks if m_blocks else 0))
+              + dilation + _i32(g.xs[3], *g.ws) + out_strides + _i32(split_tiles_m, k_split_steps, m_blocks) + per_block + _i32(tiles_m % m_blocks if m_blocks else 0))
     derived_ptrs, derived_desc = _conv_derived(epilogue, N)
     params += derived_desc
     buffers = [(out, out_offset * 4), (lhs, lhs_offset * 4), (rhs, rhs_offset * 4)]
@@ -1189,7 +1197,7 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
     kernel  = f'conv_gemm_{tag}x{bk}_' + (('ks4' if b_fast else 'ks4g') + ('_shared' if shared else '') if ksplit else 'lean' if lean else ('f' if a_fast else 'g') + ('f' if b_fast else 'g'))
     nbytes  = 4 * (lhs.size + rhs.size + out.size) + sum(4 * e.operand.size for e in epilogue if e.operand is not None)
     nbytes += 4 * tap_buffer.size if taps else 0
-    blocks = (m_blocks or _cdiv(tiles_m, chunk)) * tiles_n * (g.shares.count if shared else g.k_splits)
+    blocks = (m_blocks or _cdiv(tiles_m, chunk)) * tiles_n * slices
     if split_tiles_m:
         kernel = f'conv_gemm_{tag}x{bk}_mix'
         blocks = split_tiles_m * tiles_n + _cdiv(M - split_tiles_m * 64, 32) * _cdiv(N, 32)
