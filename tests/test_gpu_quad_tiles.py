@@ -1,5 +1,5 @@
-'''The kernels whose four waves share a 32 x 32 tile: contractions around whole k steps and whole vectors,
-windows whose taps change within and between k steps. Whole numbers, so every result is exact.'''
+'''The kernels whose four waves share a 32 x 32 tile: contractions around whole k steps and whole vectors, tiles handed to the XCDs row by row and column by
+column, windows whose taps change within and between k steps. Whole numbers, so every result is exact.'''
 import numpy as np
 import pytest
 
@@ -27,22 +27,24 @@ LENGTHS = (1, 3, 4, 31, 32, 33, 96, 97, 127, 128, 129, 160, 255, 256, 257, 384, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('xcd', ('columns', 0, 'ranges'))
 @pytest.mark.parametrize('m,n', ((2, 20), (33, 68), (65, 290), (200, 33)))
-def test_contractions(m, n):
+def test_contractions(m, n, xcd):
     for k in LENGTHS:
-        print('four waves per tile:', m, k, n, flush=True)
+        print('four waves per tile:', m, k, n, xcd, flush=True)
         args = [ints(-4, 5, m, k), ints(-3, 4, k, n), ints(-5, 5, n), ints(1, 4, n), ints(-9, 9, n), ints(-50, 50, m, n)]
-        with K.overrides(conv_ksplit=True, conv_k_splits=1, conv_dense_rows=False):
+        with K.overrides(conv_ksplit=True, conv_k_splits=1, conv_xcd_columns=xcd, conv_dense_rows=False):
             _, _, fn = check_against_oracle(layer, args, exact=True)
         assert kernels_of(fn) == ['conv_gemm_32x32x128_ks4'], kernels_of(fn)
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('xcd', ('columns', 0))
 @pytest.mark.parametrize('shares', (2, 5))
-def test_shared_tiles(shares):
+def test_shared_tiles(shares, xcd):
     for m, k, n in ((33, 700, 100), (70, 1300, 260)):
         args = [ints(-4, 5, m, k), ints(-3, 4, k, n), ints(-5, 5, n), ints(1, 4, n), ints(-9, 9, n), ints(-50, 50, m, n)]
-        with K.overrides(conv_ksplit=True, conv_shares=shares, conv_k_splits=1):
+        with K.overrides(conv_ksplit=True, conv_shares=shares, conv_k_splits=1, conv_xcd_columns=xcd):
             _, _, fn = check_against_oracle(layer, args, exact=True)
         assert kernels_of(fn) == ['conv_gemm_32x32x128_ks4_shared'], kernels_of(fn)
 
@@ -64,3 +66,10 @@ def test_windows(x, w, strides, padding, dilation, general):
         _, _, fn = check_against_oracle(f, [ints(-4, 5, *x), ints(-3, 4, *w), ints(-9, 9, w[-1])], exact=True)
     if not (general and x[-1] % 128):
         assert '_ks4' in kernels_of(fn)[-1], kernels_of(fn)
+
+
+def test_ranges_of_tiles():
+    '''Column by column where that fetches less.'''
+    choose = K.choose_conv_xcd_columns
+    assert choose(256, 2048, 2048, 8, 64) == choose(196, 1024, 256, 7, 32) == choose(784, 128, 1152, 25, 4, 784 * 128) == K.CONV_XCD_COLUMNWISE
+    assert choose(1000, 300, 784, 32, 10) == choose(600, 256, 1024, 19, 8) == 0

@@ -57,7 +57,7 @@ class _Choices:
         wgrad_slices=None,               #slices of a kernel gradient's contraction (None: by the estimate)
         conv_k_splits=None,              #slices a contraction is cut into where that applies (None: by the heuristic, 1: never)
         conv_shares=None,                #blocks that share a tile of the four-waves-per-tile kernels and add its slices themselves (None: by the estimate; a pinned conv_k_splits or conv_split: never, 1: never)
-        conv_xcd_columns=0,              #four-waves-per-tile kernels: XCD columns over the tile grid (0: row-major ranges, None: least traffic)
+        conv_xcd_columns='ranges',       #four-waves-per-tile kernels: how tiles go to the XCDs ('ranges': row by row or column by column, by the operands' sizes; 0: row by row, 'columns': column by column, a number or None: rectangles of tiles)
         scatter_sort_threshold=1 << 18,  #update elements from which a row scatter-add sorts its updates instead of using atomics
         scatter_short_rows=None,         #several table rows per wave in the sorted scatter-add: None = where it pays, True = wherever rows are short enough, False = never
         reuse_equal_equations=True,      #an equation that repeats an earlier one is bound to that one's buffer
@@ -726,15 +726,22 @@ def choose_conv_chunk(tiles_m: int, tiles_n: int, compute_units: int = 256) -> i
     return chunk
 
 
-def choose_conv_xcd_columns(M: int, N: int, K: int, tiles_m: int, tiles_n: int) -> int:
-    '''How the 8 XCDs (each with an L2 of its own; workgroup b runs on XCD b % 8) are laid over the tile grid of a
-    four-waves-per-tile product: 0 = consecutive ranges of tiles in row-major order, else 1 + log2(xn) for 8 / xn rows of
-    xn columns of XCDs. With xm x xn XCDs every L2 fetches M / xm rows of A and N / xn columns of B: xn * |A| + xm * |B|
-    bytes over the chip. Row-major ranges are the default although they fetch the most: for the MLP's two wide products
-    (256 x 784 x 512 and 256 x 512 x 512) the layout with the least traffic, 2 x 4, halves what the L2s fetch (FETCH_SIZE
-    11.2 -> 5.4 MB per launch against 2.4 MB of operands) and the step takes 21.0 us instead of 20.4: these launches wait
-    for round trips, not for bytes. `conv_xcd_columns=None` asks for the least traffic among the layouts that divide
-    the tile grid.'''
+def choose_conv_xcd_columns(M: int, N: int, K: int, tiles_m: int, tiles_n: int, lhs_size: tp.Optional[int] = None) -> int:
+    '''How the tiles of a four-waves-per-tile product go to the 8 XCDs (each with an L2 of its own; workgroup b runs on XCD b % 8): 0 = consecutive
+    ranges of tiles, row by row, CONV_XCD_COLUMNWISE = column by column, else 1 + log2(xn) for 8 / xn rows of xn columns of XCDs.
+    Row by row an XCD with at least a row of tiles fetches the whole kernel operand, column by column the whole input: whichever fetches less.
+    256 x 2048 x 2048 27.0 -> 21.3 us, 784 x 1024 x 1024 21.8 -> 20.2, 400 x 2048 x 512 11.7 -> 11.4, 196 x 2304 x 256 in four slices 8.8 -> 8.5; ResNet-50
+    on six images of 160 x 160 633 -> 624 us, its training step on four of 128 x 128 2.42 -> 2.40 ms. (Column by column also where that fetches up to twice as
+    much: an MLP whose wide product does, 1000 x 1000 x 700, 37.1 -> 38.7 us.) `conv_xcd_columns=None` asks for the least traffic among the rectangles
+    that divide the tile grid.'''
+    if CHOICES.conv_xcd_columns == 'columns':
+        return CONV_XCD_COLUMNWISE
+    if CHOICES.conv_xcd_columns == 'ranges':
+        row, column = _cdiv(M * K if lhs_size is None else min(lhs_size, M * K), max(tiles_m, 1)), 32 * K
+        each = tiles_m * tiles_n // 8
+        by_rows    = row * min(tiles_m, _cdiv(each, max(tiles_n, 1))) + column * min(tiles_n, each)
+        by_columns = row * min(tiles_m, each) + column * min(tiles_n, _cdiv(each, max(tiles_m, 1)))
+        return CONV_XCD_COLUMNWISE if by_columns < by_rows else 0
     if (tiles_m * tiles_n) % 8:
         return 0
     if CHOICES.conv_xcd_columns is not None:
@@ -1044,22 +1051,21 @@ def conv_shared_tiles(g: ConvGeometry) -> int:
 
 
 def choose_conv_shares(tiles: int, ksteps: int, compute_units: int = 256) -> int:
-    '''The number of blocks per tile with the smallest estimated time. A CU holds four blocks; a k step of 128 takes 0.8 us alone on one, 1.36 us
-    beside one other, 1.85 beside two and 2.3 beside three. A block starts in about a step; leaving, counting and
-    adding slices takes 2.2 us and 2.5 ns per block. Measured (tiles x k steps: one block per tile, and with the chosen number): 56 x 18 17.7, 10.8 us;
-    56 x 8 9.1, 7.5; 100 x 9 11.4, 10.4; 104 x 18 18.0, 13.7; 112 x 36 30.6, 19.1; 160 x 36 31.9, 23.4; 296 x 18 27.9, 22.2; 304 x 36 48.6, 34.8;
-    400 x 36 50.9, 44.9; where it stays at one, more take as long or longer: 100 x 4 6.5, 7.1; 56 x 4 6.2, 6.8; 200 x 18 18.8, 19.1; 400 x 16 25.4, 26.3. (The
-    partial sums in a launch of their own: 56 x 18 11.8 with four slices, 56 x 8 9.5, 100 x 9 11.6, 112 x 36 22.3.)'''
-    together = (0.8, 1.36, 1.85, 2.3)
+    '''The number of blocks per tile with the smallest estimated time. A k step of 128 takes 0.56 us alone on a CU (0.5 without masks), 1 us
+    beside one other block, 1.47 beside two and 1.95 beside three. A block starts in about a step; leaving, counting and
+    adding slices takes 1.6 us and 2 ns per block. Measured (tiles x k steps: one block per tile, and with the chosen number; the kernel operands from
+    behind the L2s): 56 x 18 13.2, 8.5 us; 56 x 8 7.2, 6.9; 100 x 9 8.7, 8.3; 80 x 36 22.4, 12.2; 152 x 18 13.2, 12.0; 304 x 36 38.6, 29.6; where it stays at
+    one, more take longer: 100 x 4 5.2, 6.7; 128 x 7 6.8, 7.3; 152 x 8 7.2, 8.7; 208 x 16 11.4, 13.6; 512 x 16 21.5, 26.0.'''
+    together = (0.56, 1.0, 1.47, 1.95)
     def time(count):
         per    = _cdiv(ksteps, count)
         blocks = tiles * _cdiv(ksteps, per)
         on_cu  = _cdiv(blocks, compute_units)
-        each   = together[on_cu - 1] if on_cu <= 4 else 2.3 + 0.57 * (on_cu - 4)
-        return 2.5 + each * (per + 0.8) + (2.2 + 0.0025 * blocks if count > 1 else 0.0)
+        each   = together[on_cu - 1] if on_cu <= 4 else 1.95 + 0.49 * (on_cu - 4)
+        return 2.9 + each * (per + 1) + (1.6 + 0.002 * blocks if count > 1 else 0.0)
     alone = time(1)
     count = min(range(1, min(ksteps, CONV_MAX_SHARES) + 1), key=time)
-    return count if time(count) < 0.95 * alone else 1
+    return count if time(count) < 0.98 * alone else 1
 
 
 def conv_share_count(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int = 256) -> int:
@@ -1165,7 +1171,7 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
     flags = (int(c_contig) | int(flat_rows) << 1 | int(needs_masks) << 2 | len(epilogue) << 8 | first_full << 16
              | slots << 20 | chunk << 25 | ((tap_position + 1) << 12 if taps else 0))
     if ksplit:
-        flags |= choose_conv_xcd_columns(M, N, K, tiles_m, tiles_n) << 29
+        flags |= choose_conv_xcd_columns(M, N, K, tiles_m, tiles_n, lhs.size - lhs_offset) << 29
     descs = [0, 0]
     for i, e in enumerate(epilogue):
         assert e.op < 128 and 1 <= e.kind <= 3
