@@ -73,3 +73,22 @@ def test_ranges_of_tiles():
     choose = K.choose_conv_xcd_columns
     assert choose(256, 2048, 2048, 8, 64) == choose(196, 1024, 256, 7, 32) == choose(784, 128, 1152, 25, 4, 784 * 128) == K.CONV_XCD_COLUMNWISE
     assert choose(1000, 300, 784, 32, 10) == choose(600, 256, 1024, 19, 8) == 0
+
+
+def clipped(x, w):
+    return jnp.minimum(lax.dot_general(x, w, (((1,), (1,)), ((), ()))), np.float32(6)) / np.float32(2)
+
+
+@pytest.mark.parametrize('k,launches', ((1000, 2), (512, 2), (200, 1)))
+def test_long_products_stay_with_four_waves(k, launches):
+    '''A chain that these kernels have no epilogue for stays a launch of its own behind a long product.'''
+    import vkjax_amd
+    interp, _ = vkjax_amd.wrap(clipped, frontend='minijax', plan_only=True)._get_or_create_jaxpr_interpreter([ints(-4, 5, 64, k), ints(-3, 4, 2048, k)])
+    names = [l.kernel for l in interp.launches]
+    assert len(names) == launches and ('_ks4g' in names[0]) == (launches == 2), names
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('k', (200, 1000))
+def test_long_products_with_another_chain(k):
+    check_against_oracle(clipped, [ints(-4, 5, 64, k), ints(-3, 4, 2048, k)], exact=True)

@@ -314,6 +314,8 @@ def fuse_ops(all_ops, bufferpool, outvars):
                         continue
                     if geom.shares is not None and not K.conv_straight_epilogue(list(epilogue) + extra):
                         continue                                  #(the kernels whose blocks share tiles have no other)
+                    if not K.conv_epilogue_is_worth_leaving_four_waves(lhs, rhs, geom, list(epilogue) + extra):
+                        continue
                     if K.conv_is_dense_rows(lhs, geom) and not K.dense_rows_epilogue_supported(list(epilogue) + extra):
                         continue                                  #the chain stays a launch of its own
                     tap_at = [k for k, e in enumerate(epilogue) if e.op == K.CONV_TAP]

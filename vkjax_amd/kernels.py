@@ -1002,6 +1002,19 @@ def _four_waves_pay(g: ConvGeometry, b_fast: bool, compute_units: int) -> bool:
             or (rounds == 4 and g.K >= 1024))
 
 
+def conv_epilogue_is_worth_leaving_four_waves(lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: tp.Sequence[ConvEpilogueStep], compute_units: int = 256) -> bool:
+    '''False where an epilogue would take a long product from the four-waves-per-tile kernels, which have the usual chains only: the kernel that walks
+    any chain takes 0.65 us per 32 of the contraction (1.6 without 16-byte loads of the kernel operand), those 0.5 per 128, and the chain as a launch
+    of its own some 4 us. (64 x 1000 x 2048, transposed kernel operand: 51.7 us, against 9.2 and 4.5.)'''
+    if g.split is not None or g.k_splits > 1 or not epilogue or conv_straight_epilogue(epilogue) or g.K < 512 or _dense_rows_shape(lhs, g):
+        return True
+    g = _flatten_pointwise(g)
+    if g.K * g.N * 4 >= 2**31 or lhs.size * 4 >= 2**31 or g.M * g.N == 0:
+        return True
+    _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g)
+    return not (_four_waves_per_tile(g, a_fast, c_contig, compute_units, b_fast) and (b_fast or g.Cin % 128 == 0 or g.KH * g.KW == 1))
+
+
 #Up to here slices are added by a launch of their own, which also takes over chains longer than an epilogue; more tiles are shared by blocks that add them
 #themselves (conv_share_count). (Shared by eight blocks, 32 tiles x 36 k steps would take 11.2 us instead of 14.4, 32 x 16 7.9 instead of 9.5; but these
 #products are promised two launches: test_long_contractions_of_few_tiles_are_sliced, test_sliced_contractions.)
