@@ -3,6 +3,7 @@ column, windows whose taps change within and between k steps. Whole numbers, so 
 import numpy as np
 import pytest
 
+import vkjax_amd
 from vkjax_amd import kernels as K, minijax as mj
 from tests.common import check_against_oracle
 
@@ -75,6 +76,37 @@ def test_ranges_of_tiles():
     assert choose(1000, 300, 784, 32, 10) == choose(600, 256, 1024, 19, 8) == 0
 
 
+def transposed(x, w, mean, scale, beta, rest):
+    return nn.relu((lax.dot_general(x, w, (((1,), (1,)), ((), ()))) - mean) * scale + beta + rest)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('shares', (1, 3))
+@pytest.mark.parametrize('m,n', ((2, 20), (65, 291), (300, 36)))
+def test_transposed_kernel_operand(m, n, shares):
+    for k in LENGTHS:
+        print('four waves per tile, transposed:', m, k, n, shares, flush=True)
+        args = [ints(-4, 5, m, k), ints(-3, 4, n, k), ints(-5, 5, n), ints(1, 4, n), ints(-9, 9, n), ints(-50, 50, m, n)]
+        with K.overrides(conv_ksplit=True, conv_k_splits=1, conv_shares=shares, conv_dense_rows=False, conv_split=False):
+            _, _, fn = check_against_oracle(transposed, args, exact=True)
+        names = kernels_of(fn)
+        assert names == ['conv_gemm_32x32x128_ks4t' + ('_shared' if shares > 1 and k > 128 else '')] or (k == 1 and len(names) == 1), names
+
+
+@pytest.mark.gpu
+def test_what_lies_behind_a_row_is_not_added():
+    '''A contraction that ends within a vector: the next row's first value, infinite here, stays out of both operands.'''
+    x, w = ints(-4, 5, 40, 131), ints(-3, 4, 36, 131)
+    x[1:, 0] = w[1::2, 0] = np.inf
+    x[0, 0], w[0, 0] = 1, 1
+    def f(x, w): return lax.dot_general(x, w, (((1,), (1,)), ((), ())))
+    with K.overrides(conv_ksplit=True, conv_k_splits=1, conv_dense_rows=False, conv_split=False):
+        fn  = vkjax_amd.wrap(f, frontend='minijax')
+        got = fn(x, w)
+    assert kernels_of(fn) == ['conv_gemm_32x32x128_ks4t_shared'] or kernels_of(fn) == ['conv_gemm_32x32x128_ks4t'], kernels_of(fn)
+    assert np.array_equal(got[0, 0::2], w[0::2] @ x[0])
+
+
 def clipped(x, w):
     return jnp.minimum(lax.dot_general(x, w, (((1,), (1,)), ((), ()))), np.float32(6)) / np.float32(2)
 
@@ -82,10 +114,9 @@ def clipped(x, w):
 @pytest.mark.parametrize('k,launches', ((1000, 2), (512, 2), (200, 1)))
 def test_long_products_stay_with_four_waves(k, launches):
     '''A chain that these kernels have no epilogue for stays a launch of its own behind a long product.'''
-    import vkjax_amd
     interp, _ = vkjax_amd.wrap(clipped, frontend='minijax', plan_only=True)._get_or_create_jaxpr_interpreter([ints(-4, 5, 64, k), ints(-3, 4, 2048, k)])
     names = [l.kernel for l in interp.launches]
-    assert len(names) == launches and ('_ks4g' in names[0]) == (launches == 2), names
+    assert len(names) == launches and ('_ks4t' in names[0]) == (launches == 2), names
 
 
 @pytest.mark.gpu

@@ -734,33 +734,35 @@ CONV_TILE(32x32x64, 1, 1, 1, 1, 64)
 #include "conv_quad.h"
 
 // one 32 x 32 tile per block, the k step of 128 split over four waves (chunk 1)
-#define CONV_QUAD_KERNEL(name, BK, BF)                                                                       \
-    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BF ? 3 : 2))) void name(          \
+#define CONV_QUAD_KERNEL(name, BK, B_LOADS)                                                                       \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B_LOADS != QUAD_B_WORDS ? 3 : 2))) void name(          \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
         ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
         __shared__ __attribute__((aligned(16))) float pool[conv_quad_floats<BK>()];                          \
         const ConvRegion all{0, P.tiles_m, P.tiles_n, 0};                                                    \
-        conv_quad_body<BK, BF, false>(pool, all, out, x, w, epi, dp, P, D);                                  \
+        conv_quad_body<BK, B_LOADS, false>(pool, all, out, x, w, epi, dp, P, D);                                  \
     }
-CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4, 128, true)
-// the same with element-wise loads of the kernel operand (an output width that is no multiple of 4)
-CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4g, 128, false)
+CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4, 128, QUAD_B_COLUMNS)
+// the same for a transposed kernel operand, and with element-wise loads of it (any strides)
+CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4t, 128, QUAD_B_ROWS)
+CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4g, 128, QUAD_B_WORDS)
 // the same with a 64-long k step, for windows over 64 (or 192, ...) input features, whose taps a 128-long step would straddle
-CONV_QUAD_KERNEL(conv_gemm_32x32x64_ks4, 64, true)
-// The first two with several blocks per tile, each summing a slice of the contraction (k_split_steps): few tiles leave CUs idle. A slice's sums make a
+CONV_QUAD_KERNEL(conv_gemm_32x32x64_ks4, 64, QUAD_B_COLUMNS)
+// Those with a k step of 128 with several blocks per tile, each summing a slice of the contraction (k_split_steps): few tiles leave CUs idle. A slice's sums make a
 // round trip to memory and the counter another, 2 to 2.5 us for 32 x 32 numbers; a launch that adds them takes 3.2 and a start.
 // 196 x 2304 x 256: 13.2 us by one block per tile, 8.5 by four; 150 x 4608 x 512 22.4, 12.2 by three; 588 x 4608 x 512 38.6, 29.6 by four.
-#define CONV_SHARED_KERNEL(name, BF)                                                                         \
-    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BF ? 3 : 2))) void name(          \
+#define CONV_SHARED_KERNEL(name, B_LOADS)                                                                         \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B_LOADS != QUAD_B_WORDS ? 3 : 2))) void name(          \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
         float* __restrict__ partial, uint32_t* __restrict__ arrivals,                                        \
         ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
         __shared__ __attribute__((aligned(16))) float pool[conv_quad_floats<128>()];                         \
         const ConvRegion all{0, P.tiles_m, P.tiles_n, 0};                                                    \
-        conv_quad_body<128, BF, true>(pool, all, out, x, w, epi, dp, P, D, partial, arrivals);               \
+        conv_quad_body<128, B_LOADS, true>(pool, all, out, x, w, epi, dp, P, D, partial, arrivals);               \
     }
-CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4_shared, true)
-CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4g_shared, false)
+CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4_shared, QUAD_B_COLUMNS)
+CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4t_shared, QUAD_B_ROWS)
+CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4g_shared, QUAD_B_WORDS)
 // Mixed tiling for layers whose 64 x 64 tiles do not divide evenly among the CUs (784 tiles on 256 CUs: a CU
 // with four tiles sets the time, the average is 3.06). The first P.split_tiles_m M tiles are computed as 64 x 64
 // tiles, as many as fill every CU equally; the rows behind them as 32 x 32 tiles of a quarter of the work each
@@ -781,7 +783,7 @@ CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4g_shared, false)
         } else {                                                                                             \
             const int m_base = P.split_tiles_m * 64;                                                         \
             const ConvRegion r{n_big, (P.M - m_base + 31) / 32, (P.N + 31) / 32, m_base};                    \
-            conv_quad_body<64, true, false>(pool, r, out, x, w, epi, dp, P, D);                              \
+            conv_quad_body<64, QUAD_B_COLUMNS, false>(pool, r, out, x, w, epi, dp, P, D);                              \
         }                                                                                                    \
     }
 CONV_MIX_KERNEL(conv_gemm_64x64x32_mix, 32)

@@ -15,22 +15,27 @@
 // 483 -> 437 us, on six images of 160 x 160 690 -> 637, its training step on four of 128 x 128 2.54 -> 2.42 ms, a conv block 2 x 28 x 28 x 256 30.4 -> 25.4 us.
 #pragma once
 
-// LDS of one wave: its slices of the A tile ([32][BKW + 4]) and the B tile ([BKW][36])
+// How the kernel operand is loaded: element by element; 16-byte vectors along the columns; 16-byte vectors along the contraction, contiguous there (a
+// transposed matrix: one tap only), which is then handled like the A operand. 40 x 1000 x 2048 21.3 us element by element, 7.2 in vectors; 300 x 2000 x 500 38.1, 11.0.
+enum { QUAD_B_WORDS = 0, QUAD_B_COLUMNS = 1, QUAD_B_ROWS = 2 };
+
+// LDS of one wave: its slices of the A tile ([32][BKW + 4]) and the B tile ([BKW][36], or like A's)
 template <int BK> constexpr int conv_quad_wave_floats() { return 32 * (BK / 4 + 4) + BK / 4 * 36; }
 // ... of a block: those, the per-column epilogue operands, and a word (floats)
 template <int BK> constexpr int conv_quad_floats() { return 4 * conv_quad_wave_floats<BK>() + CONV_MAX_EPI * 32 + 4; }
 
-// BK: k step of the block. B_FAST: 16-byte loads of the kernel operand, else element by element. SHARED: several blocks share a tile, each summing a slice
+// BK: k step of the block. SHARED: several blocks share a tile, each summing a slice
 // of the contraction; a slice leaves its sums in `partial`, and the block that arrives last at the tile's counter adds them.
 // Requirements (the host checks them): 16-byte loads of A, K = KH * KW * Cin with one tap or Cin a multiple of BK / 4, a row-major result and an
 // epilogue that conv_straight_steps takes. ConvParams' os_* and LH, LW hold divisors here (see there).
-template <int BK, bool B_FAST, bool SHARED>
+template <int BK, int B_LOADS, bool SHARED>
 __device__ __forceinline__ void conv_quad_body(float* __restrict__ pool, const ConvRegion region, float* __restrict__ out, const float* __restrict__ x,
                                                const float* __restrict__ w, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp, const ConvParams& Pk,
                                                const ConvDerived& Dk, float* __restrict__ partial = nullptr, uint32_t* __restrict__ arrivals = nullptr) {
     constexpr int BKW = BK / 4, LDA = BKW + 4, LDB = 36;               // a wave's slice of a k step; row pitches in LDS (no bank conflicts)
     constexpr int G = BKW / 8, SLOTS = 4 * G;                          // groups of four matrix instructions: a lane holds four k, its half's, of each
-    constexpr int A_VPR = BKW / 4, A_RSTEP = 64 / A_VPR, A_NV = 32 / A_RSTEP, B_NV = BKW / 8, NV = A_NV + B_NV, B_N = B_FAST ? B_NV : BKW / 8;
+    constexpr int A_VPR = BKW / 4, A_RSTEP = 64 / A_VPR, A_NV = 32 / A_RSTEP, B_NV = BKW / 8, NV = A_NV + B_NV;
+    static_assert(B_LOADS != QUAD_B_ROWS || A_NV == B_NV, "the B tile has the A tile's layout");
     constexpr uint32_t TILE = 32 * 32 * 4;
 
     // every argument that the way to the loads needs, in one batch
@@ -47,7 +52,7 @@ __device__ __forceinline__ void conv_quad_body(float* __restrict__ pool, const C
     QUAD_PIN(inner_magic, os_b) QUAD_PIN(inner_shift, os_h) QUAD_PIN(all_magic, os_w) QUAD_PIN(all_shift, os_n) QUAD_PIN(cin_magic, LH) QUAD_PIN(cin_shift, LW)
     QUAD_PIN(per, k_split_steps) QUAD_PIN(slices, m_each)
 #undef QUAD_PIN
-    const bool flat_rows = P.flags & 2u, masked = P.flags & 4u, taps = P.KH * P.KW != 1;
+    const bool flat_rows = P.flags & 2u, masked = P.flags & 4u, taps = B_LOADS != QUAD_B_ROWS && P.KH * P.KW != 1;
     const int tid = threadIdx.x, lane = tid & 63, kw = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
     float* const As = pool + kw * conv_quad_wave_floats<BK>();          // [32][LDA], this wave's
     float* const Bs = As + 32 * LDA;                                    // [BKW][LDB]
@@ -127,30 +132,42 @@ __device__ __forceinline__ void conv_quad_body(float* __restrict__ pool, const C
     };
     at_tap();
     // what a step's loads have in common: worked out once, then the loads are issued one by one
-    uint32_t a_soff = 0u, b_soff = 0u;
+    uint32_t a_soff = 0u, b_soff = 0u, b_at[B_NV];                      // (b_at: of vectors along the contraction)
+    if constexpr (B_LOADS == QUAD_B_ROWS) {
+#pragma unroll
+        for (int p = 0; p < B_NV; ++p) {
+            const int n = n0 + a_row + p * A_RSTEP;
+            b_at[p] = n < P.N ? (uint32_t)(n * Pk.ws_n + a_k) * 4u : CONV_OOB;
+        }
+    }
     int b_first = 0;
     const int k_end = min(P.K, (kbase + ktiles) * BK);
     auto begin_loads = [&]() {
         if (k + BKW > k_end) {                                          // the contraction (the slice) ends here: later loads of this wave read nothing
 #pragma unroll
-            for (int p = 0; p < A_NV; ++p) a_at[p] = k + a_k >= k_end ? CONV_OOB : a_at[p];
+            for (int p = 0; p < A_NV; ++p) {
+                a_at[p] = k + a_k >= k_end ? CONV_OOB : a_at[p];
+                if constexpr (B_LOADS == QUAD_B_ROWS) b_at[p] = k + a_k >= k_end ? CONV_OOB : b_at[p];
+            }
         }
         a_soff = (uint32_t)(t_r * P.DH * P.xs_h + t_s * P.DW * P.xs_w + t_c) * 4u;
-        if constexpr (B_FAST) b_soff = k < k_end ? (uint32_t)k * (uint32_t)P.N * 4u : CONV_OOB - 4u;
+        if constexpr (B_LOADS == QUAD_B_COLUMNS) b_soff = k < k_end ? (uint32_t)k * (uint32_t)P.N * 4u : CONV_OOB - 4u;
+        else if constexpr (B_LOADS == QUAD_B_ROWS) b_soff = (uint32_t)k * 4u;
         else b_first = t_r * Pk.ws_r + t_s * Pk.ws_s + t_c * Pk.ws_c;
     };
-    const uint32_t b_voff = b_n < P.N ? (uint32_t)(b_k * P.N + b_n) * 4u : CONV_OOB;       // B fast; rows k >= K lie beyond the descriptor
-    const float* const b_at = w + (B_FAST ? 0 : (n0 + l32) * Pk.ws_n + half * (BKW / 2) * Pk.ws_c);
-    struct Stage { f32x4 a[A_NV]; f32x4 b[B_N]; };                      // what is on its way for one k step (B element by element: BKW / 2 numbers of a column)
+    const uint32_t b_voff = b_n < P.N ? (uint32_t)(b_k * P.N + b_n) * 4u : CONV_OOB;       // vectors along the columns; rows k >= K lie beyond the descriptor
+    const float* const b_words = w + (B_LOADS != QUAD_B_WORDS ? 0 : (n0 + l32) * Pk.ws_n + half * (BKW / 2) * Pk.ws_c);
+    struct Stage { f32x4 a[A_NV]; f32x4 b[B_NV]; };                      // what is on its way for one k step (B element by element: BKW / 2 numbers of a column)
     auto load_one = [&](Stage& st, int v) {
         if (v < A_NV) { st.a[v < A_NV ? v : 0] = buffer_load_x4(x_rsrc, a_at[v < A_NV ? v : 0], a_soff); return; }
         const int p = v - A_NV;
-        if constexpr (B_FAST) st.b[p] = buffer_load_x4(w_rsrc, b_voff, b_soff + (uint32_t)(p * 8) * (uint32_t)P.N * 4u);
+        if constexpr (B_LOADS == QUAD_B_COLUMNS) st.b[p] = buffer_load_x4(w_rsrc, b_voff, b_soff + (uint32_t)(p * 8) * (uint32_t)P.N * 4u);
+        else if constexpr (B_LOADS == QUAD_B_ROWS) st.b[p] = buffer_load_x4(w_rsrc, b_at[p], b_soff);
         else {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int j = 4 * p + q;
-                st.b[p][q] = n0 + l32 < P.N && k + half * (BKW / 2) + j < k_end ? b_at[b_first + j * Pk.ws_c] : 0.f;
+                st.b[p][q] = n0 + l32 < P.N && k + half * (BKW / 2) + j < k_end ? b_words[b_first + j * Pk.ws_c] : 0.f;
             }
         }
     };
@@ -168,34 +185,40 @@ __device__ __forceinline__ void conv_quad_body(float* __restrict__ pool, const C
         for (int v = 0; v < NV; ++v) load_one(st, v);
         end_loads();
     };
-    // A contraction that ends within a vector (only with a single tap): what lies behind it is the next row's. The kernel operand's rows there read as
-    // zeros, which a value that is not finite would not leave alone.
+    // A contraction that ends within a vector (only with a single tap): what lies behind it is the next row's, and zeros on the other side would not leave
+    // a value alone that is not finite.
     auto clear_tail = [&](Stage& st, int step) {
         const int first = step * BK + kw * BKW;
         if ((P.K & 3) != 0 && first + BKW > P.K) {
 #pragma unroll
             for (int p = 0; p < A_NV; ++p)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) st.a[p][q] = first + a_k + q < P.K ? st.a[p][q] : 0.f;
+                for (int q = 0; q < 4; ++q) {
+                    st.a[p][q] = first + a_k + q < P.K ? st.a[p][q] : 0.f;
+                    if constexpr (B_LOADS == QUAD_B_ROWS) st.b[p][q] = first + a_k + q < P.K ? st.b[p][q] : 0.f;
+                }
         }
     };
     auto store_one = [&](const Stage& st, int v) {
         if (v < A_NV) { *reinterpret_cast<f32x4*>(&As[(a_row + (v < A_NV ? v : 0) * A_RSTEP) * LDA + a_k]) = st.a[v < A_NV ? v : 0]; return; }
         const int p = v - A_NV;
-        if constexpr (B_FAST) *reinterpret_cast<f32x4*>(&Bs[(b_k + p * 8) * LDB + 4 * (lane % 8)]) = st.b[p];
+        if constexpr (B_LOADS == QUAD_B_ROWS) *reinterpret_cast<f32x4*>(&Bs[(a_row + p * A_RSTEP) * LDA + a_k]) = st.b[p];
+        else if constexpr (B_LOADS == QUAD_B_COLUMNS) *reinterpret_cast<f32x4*>(&Bs[(b_k + p * 8) * LDB + 4 * (lane % 8)]) = st.b[p];
         else {
 #pragma unroll
             for (int q = 0; q < 4; ++q) Bs[(half * (BKW / 2) + 4 * p + q) * LDB + l32] = st.b[p][q];
         }
     };
-    f32x4 fa[G];                                                        // fragments of the k step that is computed
-    float fb[G][4];
-    uint32_t a_frag = (uint32_t)(l32 * LDA + half * (BKW / 2)), b_frag = (uint32_t)(32 * LDA + half * (BKW / 2) * LDB + l32);
+    f32x4 fa[G], fb[G];                                                 // fragments of the k step that is computed
+    uint32_t a_frag = (uint32_t)(l32 * LDA + half * (BKW / 2)), b_frag = (uint32_t)(32 * LDA + (B_LOADS == QUAD_B_ROWS ? l32 * LDA + half * (BKW / 2) : half * (BKW / 2) * LDB + l32));
     asm volatile("" : "+v"(a_frag), "+v"(b_frag));                      // (one register each, not one per group)
     auto read_group = [&](int g) {                                      // lanes 0-31 take the first half of the wave's slice, lanes 32-63 the second
         fa[g] = *reinterpret_cast<const f32x4*>(&As[a_frag + g * 4]);
+        if constexpr (B_LOADS == QUAD_B_ROWS) fb[g] = *reinterpret_cast<const f32x4*>(&As[b_frag + g * 4]);
+        else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) fb[g][q] = As[b_frag + (g * 4 + q) * LDB];
+            for (int q = 0; q < 4; ++q) fb[g][q] = As[b_frag + (g * 4 + q) * LDB];
+        }
     };
     // LDS accesses of a wave execute in order; the compiler has to keep them in order, too
     auto in_order = [&]() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };

@@ -976,6 +976,33 @@ def _conv_fast_paths(lhs: Buffer, rhs: Buffer, g: ConvGeometry, lhs_offset: int 
     return needs_masks, x_bias, a_fast, b_fast, c_contig
 
 
+def dense_copy_applies(lhs: Buffer, g: ConvGeometry, out_size: tp.Optional[int] = None) -> bool:
+    '''A kernel operand of any layout may be copied into the dense one first: it is no bigger than the activations.'''
+    return g.N % 4 == 0 and g.M >= 256 and g.K * g.N <= lhs.size + (g.M * g.N if out_size is None else out_size) and min(g.ws) >= 0
+
+
+def _kernel_operand_in_rows(g: ConvGeometry, rhs_offset: int = 0) -> bool:
+    '''A transposed matrix: the four-waves-per-tile kernels read it with 16-byte loads along the contraction.'''
+    return g.KH * g.KW == 1 and g.ws[2] == 1 and g.ws[3] >= 0 and rhs_offset % 4 == 0 and not CHOICES.conv_b_general
+
+
+def _kernel_operand_in_vectors(lhs: Buffer, g: ConvGeometry, b_fast: bool, rhs_offset: int = 0) -> bool:
+    '''For the rule of the four-waves-per-tile kernels, transposed matrices count as dense ones where they would be copied into such a one.'''
+    return b_fast or (_kernel_operand_in_rows(g, rhs_offset) and dense_copy_applies(lhs, g))
+
+
+def conv_reads_transposed(lhs: Buffer, rhs: Buffer, g: ConvGeometry, rhs_offset: int = 0, compute_units: int = 256) -> bool:
+    '''A transposed matrix need not be copied into the dense layout: the product goes to the four-waves-per-tile kernels, as it would with the copy
+    (us with the copy, without: 1000 x 100 x 300 5.9, 4.4; 1000 x 1000 x 700 21.8, 18.0; 512 x 1024 x 1024 16.6, 11.6).'''
+    if not (_kernel_operand_in_rows(g, rhs_offset) and dense_copy_applies(lhs, g)):
+        return False
+    dense = _flatten_pointwise(g._replace(ws=(g.Cin * g.N, g.Cin * g.N, g.N, 1)))
+    if _dense_rows_shape(lhs, g._replace(ws=dense.ws)) or g.K * g.N * 4 >= 2**31 or lhs.size * 4 >= 2**31:
+        return False
+    _, _, a_fast, _, c_contig = _conv_fast_paths(lhs, rhs, dense)
+    return _four_waves_per_tile(dense, a_fast, c_contig, compute_units, True)
+
+
 def _four_waves_per_tile(g: ConvGeometry, a_fast: bool, c_contig: bool, compute_units: int, b_fast: bool = True) -> bool:
     '''A product with so few 32 x 32 tiles that one wave per tile leaves most MFMA units idle: four waves per tile,
     each taking a quarter of every (128-long) k step.'''
@@ -1006,13 +1033,17 @@ def conv_epilogue_is_worth_leaving_four_waves(lhs: Buffer, rhs: Buffer, g: ConvG
     '''False where an epilogue would take a long product from the four-waves-per-tile kernels, which have the usual chains only: the kernel that walks
     any chain takes 0.65 us per 32 of the contraction (1.6 without 16-byte loads of the kernel operand), those 0.5 per 128, and the chain as a launch
     of its own some 4 us. (64 x 1000 x 2048, transposed kernel operand: 51.7 us, against 9.2 and 4.5.)'''
-    if g.split is not None or g.k_splits > 1 or not epilogue or conv_straight_epilogue(epilogue) or g.K < 512 or _dense_rows_shape(lhs, g):
+    if g.split is not None or g.k_splits > 1 or not epilogue or conv_straight_epilogue(epilogue) or _dense_rows_shape(lhs, g):
+        return True
+    if conv_reads_transposed(lhs, rhs, g):
+        return False
+    if g.K < 512:
         return True
     g = _flatten_pointwise(g)
     if g.K * g.N * 4 >= 2**31 or lhs.size * 4 >= 2**31 or g.M * g.N == 0:
         return True
     _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g)
-    return not (_four_waves_per_tile(g, a_fast, c_contig, compute_units, b_fast) and (b_fast or g.Cin % 128 == 0 or g.KH * g.KW == 1))
+    return not (_four_waves_per_tile(g, a_fast, c_contig, compute_units, _kernel_operand_in_vectors(lhs, g, b_fast)) and (b_fast or g.Cin % 128 == 0 or g.KH * g.KW == 1))
 
 
 #Up to here slices are added by a launch of their own, which also takes over chains longer than an epilogue; more tiles are shared by blocks that add them
@@ -1034,7 +1065,7 @@ def conv_k_splits(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int 
     if g.K * g.N * 4 >= 2**31 or lhs.size * 4 >= 2**31 or g.M * g.N == 0:
         return 1
     _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g)
-    if not _four_waves_per_tile(g, a_fast, c_contig, compute_units, b_fast) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
+    if not _four_waves_per_tile(g, a_fast, c_contig, compute_units, _kernel_operand_in_vectors(lhs, g, b_fast)) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
         return 1
     tiles, ksteps = conv_shared_tiles(g), _cdiv(g.K, 128)
     if CHOICES.conv_k_splits is not None:
@@ -1092,7 +1123,7 @@ def conv_share_count(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: i
         return 1
     _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g)
     #(not the 64-long step: 196 x 9 of those 7.8 us, by two blocks each 9.3)
-    if not _four_waves_per_tile(g, a_fast, c_contig, compute_units, b_fast) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
+    if not _four_waves_per_tile(g, a_fast, c_contig, compute_units, _kernel_operand_in_vectors(lhs, g, b_fast)) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
         return 1
     tiles, ksteps = conv_shared_tiles(g), _cdiv(g.K, 128)
     if tiles > CONV_MAX_SHARED_TILES or (CHOICES.conv_shares is None and tiles <= CONV_SLICED_MAX_TILES):
@@ -1144,7 +1175,7 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
     flat_rows = g.batch == 1 and g.Wo == 1 and g.SH == 1 and g.PH == 0 and g.PW == 0 and not needs_masks
     #a product with so few 32 x 32 tiles that one wave per tile leaves most MFMA units idle: four waves per
     #tile, each taking a quarter of every (128-long) k step
-    ksplit = _four_waves_per_tile(g, a_fast, c_contig, compute_units, b_fast) and (not epilogue or slots != 0)
+    ksplit = _four_waves_per_tile(g, a_fast, c_contig, compute_units, _kernel_operand_in_vectors(lhs, g, b_fast, rhs_offset)) and (not epilogue or slots != 0)
     #(windows over 64 input features take a 64-long k step, with 16-byte loads of the kernel operand only)
     short_step = ksplit and g.Cin % 128 != 0 and g.KH * g.KW != 1
     if short_step and not b_fast:
@@ -1213,7 +1244,7 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
         assert operand_slots[-1] == (None, 0)
         operand_slots[-1] = (tap_buffer, 0)
     buffers += operand_slots + derived_ptrs
-    kernel  = f'conv_gemm_{tag}x{bk}_' + (('ks4' if b_fast else 'ks4g') + ('_shared' if shared else '') if ksplit else 'lean' if lean else ('f' if a_fast else 'g') + ('f' if b_fast else 'g'))
+    kernel  = f'conv_gemm_{tag}x{bk}_' + (('ks4' if b_fast else 'ks4t' if _kernel_operand_in_rows(g, rhs_offset) else 'ks4g') + ('_shared' if shared else '') if ksplit else 'lean' if lean else ('f' if a_fast else 'g') + ('f' if b_fast else 'g'))
     nbytes  = 4 * (lhs.size + rhs.size + out.size) + sum(4 * e.operand.size for e in epilogue if e.operand is not None)
     nbytes += 4 * tap_buffer.size if taps else 0
     blocks = (m_blocks or _cdiv(tiles_m, chunk)) * tiles_n * slices

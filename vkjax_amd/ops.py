@@ -721,8 +721,8 @@ def _with_dense_kernel(bufferpool, equation, rhs: Buffer, geom: 'K.ConvGeometry'
     layout first when it is no bigger than the activations: the GEMM kernel then reads it with 16-byte loads.
     Returns (ops, rhs, geometry, rhs offset).'''
     N, dense = geom.N, (geom.KW * geom.Cin * geom.N, geom.Cin * geom.N, geom.N, 1)
-    if ((geom.ws == dense and rhs_offset % 4 == 0) or N % 4 != 0 or geom.M < 256 or geom.K * N > lhs.size + outbuf.size
-            or builtins_min(geom.ws) < 0):
+    if ((geom.ws == dense and rhs_offset % 4 == 0) or not K.dense_copy_applies(lhs, geom, outbuf.size)
+            or K.conv_reads_transposed(lhs, rhs, geom, rhs_offset)):
         return [], rhs, geom, rhs_offset
     position = bufferpool.op_counter
     bufferpool.op_counter -= 1                  #the copy lives at the equation's own position
