@@ -735,7 +735,7 @@ CONV_TILE(32x32x64, 1, 1, 1, 1, 64)
 
 // one 32 x 32 tile per block, the k step of 128 split over four waves (chunk 1)
 #define CONV_QUAD_KERNEL(name, BK, B_LOADS)                                                                       \
-    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B_LOADS != QUAD_B_WORDS ? 3 : 2))) void name(          \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B_LOADS != QUAD_B_WORDS ? 4 : 3))) void name(          \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
         ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
         __shared__ __attribute__((aligned(16))) float pool[conv_quad_floats<BK>()];                          \
@@ -752,7 +752,7 @@ CONV_QUAD_KERNEL(conv_gemm_32x32x64_ks4, 64, QUAD_B_COLUMNS)
 // round trip to memory and the counter another, 2 to 2.5 us for 32 x 32 numbers; a launch that adds them takes 3.2 and a start.
 // 196 x 2304 x 256: 13.2 us by one block per tile, 8.5 by four; 150 x 4608 x 512 22.4, 12.2 by three; 588 x 4608 x 512 38.6, 29.6 by four.
 #define CONV_SHARED_KERNEL(name, B_LOADS)                                                                         \
-    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B_LOADS != QUAD_B_WORDS ? 3 : 2))) void name(          \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B_LOADS != QUAD_B_WORDS ? 4 : 3))) void name(          \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
         float* __restrict__ partial, uint32_t* __restrict__ arrivals,                                        \
         ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
@@ -767,9 +767,7 @@ CONV_SHARED_KERNEL(conv_gemm_32x32x128_ks4g_shared, QUAD_B_WORDS)
 // with four tiles sets the time, the average is 3.06). The first P.split_tiles_m M tiles are computed as 64 x 64
 // tiles, as many as fill every CU equally; the rows behind them as 32 x 32 tiles of a quarter of the work each
 // (four waves sharing every 64-long k step), which spread over the CUs in finer units. Both kinds of block have 256
-// threads and share one LDS pool; with the 64-long step the kernel needs 120 registers, so four blocks fit a CU
-// (the 128-long step of conv_gemm_32x32x128_ks4 takes 164: three blocks, and the small tiles would wait for
-// the large ones). One M tile per block (chunk 1).
+// threads and share one LDS pool; the kernel with the 64-long step needs 120 registers, so four blocks fit a CU. One M tile per block (chunk 1).
 #define CONV_MIX_KERNEL(name, BK)                                                                              \
     extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void name(            \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \

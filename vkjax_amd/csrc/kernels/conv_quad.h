@@ -6,13 +6,15 @@
 // every k step the way through LDS. So
 //   - divisions by what is known when the launch is recorded are multiplications by constants from the host, and whether a tap lies inside the input is
 //     worked out for the tap a load is for instead of for all of them beforehand;
-//   - the loads of two k steps are on their way before anything is waited for, the operands of the epilogue behind them, and they are used behind the loop;
+//   - the operands of the epilogue are requested behind the first tiles, and used behind the loop;
 //   - a wave reads the fragments of the coming k step, stores that step's tiles before it and requests a later step's between the matrix instructions of
 //     the one it computes: each slot below is one matrix instruction (64 cycles) and what fits beside it.
 // A k step of 128 takes 0.5 us where a block is alone on its CU (0.43 at the rate of the matrix cores) and everything else 3.5 us. Before, one k step after the
 // other, epilogue operands in front of the loop and long divisions at the start: 0.8 and 4.4 us. In ResNet-50 on one image, where the kernel operands come
 // from behind the L2s: 49 x 4608 x 512 in four slices 12.4 -> 9.3 us, 49 x 512 x 2048 7.1 -> 5.5, 3136 x 576 x 64 (steps of 64) 10.2 -> 8.2; the whole replay
-// 483 -> 437 us, on six images of 160 x 160 690 -> 637, its training step on four of 128 x 128 2.54 -> 2.42 ms, a conv block 2 x 28 x 28 x 256 30.4 -> 25.4 us.
+// 483 -> 429 us, on six images of 160 x 160 690 -> 609, its training step on four of 128 x 128 2.54 -> 2.35 ms, a conv block 2 x 28 x 28 x 256 30.4 -> 25.6 us.
+// With the loads of two more k steps on their way instead of one only three blocks fit a CU (164 registers, 126): 1960 x 2048 x 512 (992 tiles) 44.0
+// instead of 37.5 us, 900 x 256 x 512 6.4 instead of 5.9; 1960 x 2048 x 128 11.4 instead of 11.5.
 #pragma once
 
 // How the kernel operand is loaded: element by element; 16-byte vectors along the columns; 16-byte vectors along the contraction, contiguous there (a
@@ -231,9 +233,8 @@ __device__ __forceinline__ void conv_quad_body(float* __restrict__ pool, const C
         for (int v = 0; v < 4; ++v) fn(v, base, (uint32_t)(8 * kw + v) * rowb);
     };
 
-    Stage s0, s1;
-    load_all(s0);
-    load_all(s1);
+    Stage next;
+    load_all(next);
     // Epilogue operands: thread t fetches column t of every step. Every step issues one load, whatever its kind, so that none waits for the one before: an
     // absent operand, one that is derived behind the loop, or a full tensor has a descriptor of size 0, which reads nothing and returns 0.
     float e_reg[CONV_MAX_EPI], d_in[CONV_MAX_DERIVED + 1], quarter[4] = {0.f, 0.f, 0.f, 0.f};
@@ -268,18 +269,19 @@ __device__ __forceinline__ void conv_quad_body(float* __restrict__ pool, const C
     }
 
     f32x16 acc = f32x16{};
-    clear_tail(s0, kbase);
+    clear_tail(next, kbase);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) store_one(s0, v);
+    for (int v = 0; v < NV; ++v) store_one(next, v);
     in_order();
-    load_all(s0);
+    load_all(next);
 #pragma unroll
     for (int g = 0; g < G; ++g) read_group(g);
-    // One k step: the matrix instructions of the fragments at hand; between them the tiles of the next step (`next`) go to LDS, the loads of the step two
-    // later are issued into the registers that frees (behind the end they read nothing), and the next step's fragments are read, each group behind the last
+    // One k step: the matrix instructions of the fragments at hand; between them the tiles of the next step go to LDS, the loads of the one behind it are
+    // issued into the registers that frees (beyond the end they read nothing), and the next step's fragments are read, each group behind the last
     // instruction that uses the one before.
-    auto step = [&](Stage& next, int at) {
-        clear_tail(next, kbase + at + 1);
+#pragma nounroll
+    for (int at = 1; at < ktiles; ++at) {
+        clear_tail(next, kbase + at);
         in_order();
         begin_loads();
 #pragma unroll
@@ -296,11 +298,7 @@ __device__ __forceinline__ void conv_quad_body(float* __restrict__ pool, const C
             __builtin_amdgcn_sched_barrier(0);
         }
         end_loads();
-    };
-    int at = 0;
-#pragma nounroll
-    for (; at + 2 < ktiles; at += 2) { step(s1, at); step(s0, at + 1); }
-    if (at + 1 < ktiles) step(s1, at);
+    }
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[s / 4][s % 4], fb[s / 4][s % 4], acc, 0, 0, 0);
 
