@@ -87,5 +87,5 @@ def test_values_by_the_estimate(batch, size, cin, cout, window):
 
 def test_share_counts():
     '''One block per tile where that fills the CUs or the contraction is short; never more blocks than steps.'''
-    assert [K.choose_conv_shares(*a) for a in ((100, 4), (128, 4), (200, 18), (200, 8), (400, 16), (2048, 36))] == [1] * 6
-    assert all(1 < K.choose_conv_shares(*a) <= min(a[1], K.CONV_MAX_SHARES) for a in ((56, 18), (56, 8), (100, 9), (104, 18), (112, 36), (160, 36), (304, 36), (400, 36)))
+    assert [K.choose_conv_shares(*a) for a in ((100, 4), (128, 4), (200, 18), (200, 8), (400, 16), (2048, 36), (400, 36))] == [1] * 7
+    assert all(1 < K.choose_conv_shares(*a) <= min(a[1], K.CONV_MAX_SHARES) for a in ((56, 18), (56, 8), (100, 9), (104, 18), (112, 36), (160, 36), (304, 36)))

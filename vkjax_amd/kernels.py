@@ -1096,16 +1096,17 @@ def conv_shared_tiles(g: ConvGeometry) -> int:
 
 def choose_conv_shares(tiles: int, ksteps: int, compute_units: int = 256) -> int:
     '''The number of blocks per tile with the smallest estimated time. A k step of 128 takes 0.56 us alone on a CU (0.5 without masks), 1 us
-    beside one other block, 1.47 beside two and 1.95 beside three. A block starts in about a step; leaving, counting and
-    adding slices takes 1.6 us and 2 ns per block. Measured (tiles x k steps: one block per tile, and with the chosen number; the kernel operands from
-    behind the L2s): 56 x 18 13.2, 8.5 us; 56 x 8 7.2, 6.9; 100 x 9 8.7, 8.3; 80 x 36 22.4, 12.2; 152 x 18 13.2, 12.0; 304 x 36 38.6, 29.6; where it stays at
-    one, more take longer: 100 x 4 5.2, 6.7; 128 x 7 6.8, 7.3; 152 x 8 7.2, 8.7; 208 x 16 11.4, 13.6; 512 x 16 21.5, 26.0.'''
-    together = (0.56, 1.0, 1.47, 1.95)
+    beside one other block, 1.47 beside two and 1.95 beside three, which fill a CU; those that follow start as others end. A block starts in about a
+    step; leaving, counting and adding slices takes 1.6 us and 2 ns per block. Measured (tiles x k steps: one block per tile, and with the chosen number;
+    the kernel operands from behind the L2s): 56 x 18 13.3, 8.5 us; 56 x 8 7.0, 6.8; 100 x 9 8.6, 8.4; 80 x 36 22.7, 12.4; 152 x 18 13.3, 11.9; 304 x 36 39.2,
+    30.3 (by four blocks 34.6: a fifth on most CUs); where it stays at one, more take as long or longer: 100 x 4 5.0, 6.4; 128 x 7 6.7, 7.5; 152 x 8 7.4, 8.6;
+    208 x 16 11.4, 13.5; 400 x 36 39.4, 39.1.'''
+    together = (0.56, 1.0, 1.47, 1.95, 2.7, 2.95, 3.25, 3.5)
     def time(count):
         per    = _cdiv(ksteps, count)
         blocks = tiles * _cdiv(ksteps, per)
         on_cu  = _cdiv(blocks, compute_units)
-        each   = together[on_cu - 1] if on_cu <= 4 else 1.95 + 0.49 * (on_cu - 4)
+        each   = together[on_cu - 1] if on_cu <= 8 else 3.5 + 0.49 * (on_cu - 8)
         return 2.9 + each * (per + 1) + (1.6 + 0.002 * blocks if count > 1 else 0.0)
     alone = time(1)
     count = min(range(1, min(ksteps, CONV_MAX_SHARES) + 1), key=time)
