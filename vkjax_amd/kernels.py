@@ -1788,11 +1788,13 @@ def row_program(outs: tp.Sequence[Buffer], inputs: tp.Sequence[RowsInput], steps
     lanes = min(64, _pow2_at_least(R // vec)) if vectors == 1 else 64
     flags = [place['in', k] | (i.single << 16)
              | ((vec == 4 and i.column_stride == 1 and i.row_stride % 4 == 0 and i.base % 4 == 0) << 17) for k, i in enumerate(inputs)]
-    code = []
+    code, one_value = [], False                 #one_value: the accumulator is the same in all columns of a row
     for s in steps:
         slot = 0 if s.slot is None else s.slot[1] if s.slot[0] == 'out' else place[s.slot]
-        code += [ROWS_OPS[s.what] | s.op << 4 | bool(s.left) << 16 | bool(s.single) << 17 | (s.slot is not None) << 18 | slot << 20, s.imm]
-    params = (_u32(outer, R, lanes.bit_length() - 1, len(inputs), len(steps), *_pad([i.buffer.size * 4 for i in inputs], ROWS_MAX_IN),
+        once = s.what == 'apply' and one_value and (s.slot is None or s.single)
+        code += [ROWS_OPS[s.what] | s.op << 4 | bool(s.left) << 16 | bool(s.single) << 17 | (s.slot is not None) << 18 | once << 19 | slot << 20, s.imm]
+        one_value = {'apply': once, 'load': bool(s.single), 'put': one_value, 'out': one_value}.get(s.what, True)
+    params = (_u32(outer, R, lanes.bit_length() - 1 | 64 * waves << 8, len(inputs), len(steps), *_pad([i.buffer.size * 4 for i in inputs], ROWS_MAX_IN),
                    *_pad([i.base for i in inputs], ROWS_MAX_IN))
               + _i32(*_pad([i.row_stride for i in inputs], ROWS_MAX_IN), *_pad([i.column_stride for i in inputs], ROWS_MAX_IN))
               + _u32(*_pad(flags, ROWS_MAX_IN), *_pad(code, 2 * ROWS_MAX_CODE)))
