@@ -92,6 +92,19 @@ __device__ __forceinline__ int magic_div(int n, uint32_t magic, uint32_t shift) 
     return magic ? (int)(__umulhi((uint32_t)n, magic) >> shift) : n;
 }
 
+// Requests every 64 bytes of a kernel's first BYTES of arguments at once. Left to itself the compiler fetches an argument where it is first used, and each
+// line of 64 bytes that no fetch has touched before is a round trip to memory of its own, some 0.7 us one after the other in front of a launch's first load.
+// (For kernels that do not read their arguments in one go by themselves. Replays with and without: a convolutional network's training step 227.2, 225.8 us,
+// ResNet-50 on six images of 160 x 160 607, 603, on 64 images 3.90, 3.86 ms.)
+template <size_t BYTES>
+__device__ __forceinline__ void request_arguments() {
+    const uint32_t* const words = reinterpret_cast<const uint32_t*>(__builtin_amdgcn_kernarg_segment_ptr());
+    uint32_t all = words[(BYTES - 4) / 4];
+#pragma unroll
+    for (size_t at = 0; at + 4 < BYTES; at += 64) all |= words[at / 4];
+    asm volatile("" :: "s"(all));
+}
+
 // Consecutive workgroup ids are handed to the 8 XCDs in turn, and every XCD has an L2 of its own.
 // This renumbers the workgroups of a 1-D grid so that each XCD works through a contiguous range:
 // kernels whose neighbouring workgroups read overlapping data (windows, halos) then find the

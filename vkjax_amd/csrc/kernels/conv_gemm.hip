@@ -714,6 +714,7 @@ __device__ __forceinline__ void conv_gemm_body(float* __restrict__ pool, const C
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
         ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
         __shared__ __attribute__((aligned(16))) float pool[conv_pool_floats<WGM, WGN, TM, TN, BK>()];        \
+        request_arguments<3 * sizeof(void*) + sizeof(ConvEpiPtrs) + sizeof(ConvDerivedPtrs) + sizeof(ConvParams) + sizeof(ConvDerived)>(); \
         const ConvRegion all{0, P.tiles_m, P.tiles_n, 0};                                                    \
         conv_gemm_body<WGM, WGN, TM, TN, BK, AF, BF, LEAN>(pool, all, out, x, w, epi, dp, P, D);               \
     }

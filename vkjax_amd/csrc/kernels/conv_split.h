@@ -855,6 +855,7 @@ __device__ __forceinline__ void conv_split_body(u32x4* __restrict__ pool, float*
         __shared__ __attribute__((aligned(16))) u32x4 pool[PATCH ? 12 * CONV_PATCH_ROWS : 24 * 32 * WGM * TM];               \
         __shared__ float Es[CONV_MAX_EPI * 32 * WGN * TN];                                                                   \
         __shared__ int Rs[32 * WGM * TM];                                                                                    \
+        request_arguments<5 * sizeof(void*) + sizeof(ConvEpiPtrs) + sizeof(ConvDerivedPtrs) + sizeof(ConvParams) + sizeof(ConvDerived)>(); \
         conv_split_body<WGM, WGN, TM, TN, STEPS, PATCH, FINE, ##__VA_ARGS__>(pool, Es, Rs, out, x, w, partial, arrivals, epi, dp, P, D);    \
     }
 // _steps: 50176 x 128 x 512 with a ReLU6 68 us, with a scalar 62, with `relu(y) + r` 82 (each as launches of its own behind the product: 83, 82, 94;
@@ -1054,6 +1055,7 @@ __device__ __forceinline__ void conv_short_body(u32x4* __restrict__ Bs, float* _
         float* __restrict__ partial, uint32_t* __restrict__ arrivals, ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) { \
         __shared__ __attribute__((aligned(16))) u32x4 Bs[CONV_SHORT_COLS / 32 * 4 * 192];                                    \
         __shared__ float Es[CONV_MAX_EPI * CONV_SHORT_COLS];                                                                 \
+        request_arguments<5 * sizeof(void*) + sizeof(ConvEpiPtrs) + sizeof(ConvDerivedPtrs) + sizeof(ConvParams) + sizeof(ConvDerived)>(); \
         conv_short_body<STEPS>(Bs, Es, out, x, w, epi, dp, P, D);                                                            \
     }
 CONV_SHORT_KERNEL(conv_gemm_split_short, false)

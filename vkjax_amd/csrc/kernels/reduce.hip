@@ -558,6 +558,7 @@ __device__ __forceinline__ void scale_relu_backward_body(float* __restrict__ dx,
     extern "C" __global__ __launch_bounds__(256) void name(float* dx, float* sum_m, float* sum_mx, const float* ans,   \
                                                            const float* thr, const float* g, const float* alt,        \
                                                            const float* x, const float* kvec, ReduceParams P) {       \
+        request_arguments<9 * sizeof(void*) + sizeof(ReduceParams)>();                                                     \
         scale_relu_backward_body<VEC, SELECT, true>(dx, sum_m, sum_mx, ans, thr, g, alt, x, kvec, P);                        \
     }
 // _v4 needs inner % 4 == 0 and 16-byte aligned arrays
@@ -572,6 +573,7 @@ SCALE_RELU_BACKWARD_KERNEL(scale_backward_v4, 4, false)
 #define RELU_BACKWARD_KERNEL(name, VEC)                                                                                     \
     extern "C" __global__ __launch_bounds__(256) void name(float* m, float* sum_m, const float* ans, const float* thr,     \
                                                            const float* g, const float* alt, ReduceParams P) {             \
+        request_arguments<6 * sizeof(void*) + sizeof(ReduceParams)>();                                                     \
         scale_relu_backward_body<VEC, true, false>(m, sum_m, nullptr, ans, thr, g, alt, nullptr, nullptr, P);                \
     }
 RELU_BACKWARD_KERNEL(relu_backward_v1, 1)
@@ -881,9 +883,11 @@ __device__ __forceinline__ void pool2d_dispatch(uint32_t* __restrict__ out, cons
     else pool2d_body<KH, KW, 2>(out, in, P);
 }
 extern "C" __global__ __launch_bounds__(256) void pool2d_3x3_v4(uint32_t* __restrict__ out, const uint32_t* __restrict__ in, PoolParams P) {
+    request_arguments<2 * sizeof(void*) + sizeof(PoolParams)>();
     pool2d_dispatch<3, 3>(out, in, P);
 }
 extern "C" __global__ __launch_bounds__(256) void pool2d_2x2_v4(uint32_t* __restrict__ out, const uint32_t* __restrict__ in, PoolParams P) {
+    request_arguments<2 * sizeof(void*) + sizeof(PoolParams)>();
     pool2d_dispatch<2, 2>(out, in, P);
 }
 
@@ -971,6 +975,7 @@ __device__ __forceinline__ void pool2d_sum_body(float* __restrict__ out, const f
 #define POOL_SUM_KERNEL(name, KH, KW, SPREAD)                                                                               \
     extern "C" __global__ __launch_bounds__(256) void name(float* out, const float* in, const float* before, const float* after, \
                                                            const float* ans, const float* otherwise, PoolSumParams P) {    \
+        request_arguments<6 * sizeof(void*) + sizeof(PoolSumParams)>();                                                    \
         pool2d_sum_body<KH, KW, SPREAD>(out, in, before, after, ans, otherwise, P);                                          \
     }
 POOL_SUM_KERNEL(pool2d_sum_3x3_v4, 3, 3, false)
@@ -1273,17 +1278,20 @@ __device__ __forceinline__ void scatter_selected2d_3x3_s2_body(uint32_t* __restr
 }
 extern "C" __global__ __launch_bounds__(256) void scatter_selected2d_3x3_s2_v4(uint32_t* __restrict__ out, const uint32_t* __restrict__ source,
                                                                               const uint32_t* __restrict__ selected, PoolParams P) {
+    request_arguments<3 * sizeof(void*) + sizeof(PoolParams)>();
     scatter_selected2d_3x3_s2_body(out, source, selected, P);
 }
 
 #define SELECT_WINDOW_2D(KH, KW)                                                                                                    \
     extern "C" __global__ __launch_bounds__(256) void select_window2d_##KH##x##KW##_v4(uint32_t* __restrict__ sel,                   \
                                                                                       const uint32_t* __restrict__ operand, PoolParams P) { \
+        request_arguments<2 * sizeof(void*) + sizeof(PoolParams)>();                                                       \
         select_window2d_body<KH, KW>(sel, operand, P);                                                                              \
     }
 #define SCATTER_SELECTED_2D(KH, KW, NY, NX)                                                                                         \
     extern "C" __global__ __launch_bounds__(256) void scatter_selected2d_##KH##x##KW##_n##NY##x##NX##_v4(uint32_t* __restrict__ out, \
             const uint32_t* __restrict__ source, const uint32_t* __restrict__ selected, PoolParams P) {                             \
+        request_arguments<3 * sizeof(void*) + sizeof(PoolParams)>();                                                       \
         scatter_selected2d_body<KH, KW, NY, NX>(out, source, selected, P);                                                          \
     }
 SELECT_WINDOW_2D(3, 3)

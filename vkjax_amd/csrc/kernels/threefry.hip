@@ -186,17 +186,16 @@ __device__ __forceinline__ uint32_t threefry_split_word(uint32_t k0, uint32_t k1
 template <int VEC, int MODE, bool UNIFORM = false>
 __device__ __forceinline__ void threefry_stream_body(uint32_t* __restrict__ out, const uint32_t* __restrict__ key0,
                                                      const uint32_t* __restrict__ key1, const ThreefryStreamParams& P) {
-    uint32_t k0 = key0[0], k1 = key1[0];
-    if (P.key_split) {
-        const uint32_t s0 = threefry_split_word(k0, k1, P, P.key_word[0]), s1 = threefry_split_word(k0, k1, P, P.key_word[1]);
-        k0 = s0; k1 = s1;
-    }
-    uint32_t o[6] = {};
-    if constexpr (UNIFORM) {
+    uint32_t k0 = key0[0], k1 = key1[0], o[6] = {};
+    if constexpr (UNIFORM) {                         // requested with the key: behind the split they would be another round trip to memory
         const char* const args = reinterpret_cast<const char*>(__builtin_amdgcn_kernarg_segment_ptr());
         const uint32_t* const* const op_ptr = reinterpret_cast<const uint32_t* const*>(args + 24);
 #pragma unroll
         for (int k = 0; k < 6; ++k) o[k] = op_ptr[k][0];
+    }
+    if (P.key_split) {
+        const uint32_t s0 = threefry_split_word(k0, k1, P, P.key_word[0]), s1 = threefry_split_word(k0, k1, P, P.key_word[1]);
+        k0 = s0; k1 = s1;
     }
 #pragma nounroll
     for (uint64_t at = (blockIdx.x * 256ull + threadIdx.x) * VEC; at < P.h; at += gridDim.x * 256ull * VEC) {
@@ -253,6 +252,7 @@ __device__ __forceinline__ void threefry_stream_body(uint32_t* __restrict__ out,
 #define TF_STREAM_KERNEL(name, VEC, MODE, ...)                                                                         \
     extern "C" __global__ __launch_bounds__(256) void name(uint32_t* out, const uint32_t* key0, const uint32_t* key1,  \
                                                            ThreefryStreamPtrs operands, ThreefryStreamParams P) {      \
+        request_arguments<3 * sizeof(void*) + sizeof(ThreefryStreamPtrs) + sizeof(ThreefryStreamParams)>();             \
         threefry_stream_body<VEC, MODE, ##__VA_ARGS__>(out, key0, key1, P);                                            \
     }
 TF_STREAM_KERNEL(threefry2x32_stream_v1, 1, TF_HALVES)

@@ -132,6 +132,7 @@ __device__ __forceinline__ void wgrad_body(float* __restrict__ out, const float*
 #define WGRAD_KERNEL(name, VA, VB)                                                                          \
     extern "C" __global__ __launch_bounds__(256) void name(float* __restrict__ out, const float* __restrict__ x, \
                                                            const float* __restrict__ g, WgradParams P) {    \
+        request_arguments<3 * sizeof(void*) + sizeof(WgradParams)>();                                       \
         wgrad_body<VA, VB>(out, x, g, P);                                                                   \
     }
 // suffix: a = 16-byte loads of X (C % 4 == 0), b = 16-byte loads of G (N % 4 == 0), s = single words

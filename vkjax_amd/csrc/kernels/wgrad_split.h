@@ -346,6 +346,7 @@ __device__ __forceinline__ void wgrad_split_body(u32x4* __restrict__ lds, u32x2*
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ g, WgradParams P, WgradSplitParams Q) { \
         __shared__ __attribute__((aligned(16))) u32x4 lds[(PAIR ? 2 : 1) * 12 * 64 * (TM + TN)];                                               \
         __shared__ __attribute__((aligned(16))) u32x2 table[(PAIR ? 2 : 1) * 4 * 32];                                                          \
+        request_arguments<3 * sizeof(void*) + sizeof(WgradParams) + sizeof(WgradSplitParams)>();                                    \
         wgrad_split_body<TM, TN, VA, VB, PAIR>(lds, table, out, x, g, P, Q);                                                        \
     }
 WGRAD_SPLIT_KERNEL(wgrad_split_128x128_aa, 2, 2, true, true, 2, true)
