@@ -791,7 +791,7 @@ CONV_MIX_KERNEL(conv_gemm_64x64x64_mix, 64)
 #include "conv_split.h"
 
 // ---------------------------------------------------------------------------------------------
-// Convolutions of dense images with very few features (an RGB stem: 7 x 7 x 3, stride 2). The general kernel
+// Convolutions of dense images with very few features (an RGB stem: 7 x 7 x 3 or 3 x 3 x 3, stride 2). The general kernel
 // above assembles the A tile element by element for them: 1650 vector instructions per 64 x 64 tile against
 // 80 MFMAs, and the two share the SIMDs' issue slots (counters: the vector ALUs busy 56 % of the kernel's time).
 // Here a block copies the image rows its 64 output positions touch into LDS once (16-byte loads of whole
@@ -799,11 +799,11 @@ CONV_MIX_KERNEL(conv_gemm_64x64x64_mix, 64)
 // KW * Cin values one kernel row reads for an output position are contiguous there, so the address of A(m, k)
 // is a per-lane base plus a compile-time offset. The whole kernel (KH * RLP rows, RLP = KW * Cin rounded up to
 // even, the extra row zero) sits in LDS for the block's lifetime; a block walks the tiles in steps of the grid.
-//   KH: kernel rows; RLP: padded run length; PR: image rows of a patch (>= KH + SH, a tile spans two output rows
-//   at most); NVEC: 16-byte vectors a thread fetches per patch.
-// Requirements (the host checks them): pixels dense ([B, H, W, Cin], W * Cin % 4 == 0), no dilation, M % 64 == 0,
-// Ho * Wo % 64 == 0 (a tile lies in one image), Wo >= 64, N <= 64, row-major result, template epilogue without a
-// full-size operand, KW * Cin in (RLP - 2, RLP], KH + SH <= PR, PR * W * Cin / 4 <= 256 * NVEC.
+//   KH: kernel rows; RLP: padded run length; NVEC: 16-byte vectors a thread fetches per patch.
+// A tile lies in one image: an image's last tile is filled up with rows that are not stored, and the patch has the image rows that a tile's positions reach
+// at most (patch_rows). Image rows begin at any word: the last vector of one is cut off where it ends.
+// Requirements (the host checks them): pixels dense ([B, H, W, Cin]), no dilation, N <= 64, row-major result, template epilogue without a
+// full-size operand, KW * Cin in (RLP - 2, RLP], a patch that fits (floats, and vectors per thread).
 struct ConvStemParams {
     int32_t M, N, K;
     int32_t Ho, Wo, H, W, Cin, KH, KW, SH, SW, PH, PW;
@@ -811,20 +811,22 @@ struct ConvStemParams {
     int32_t left;                   // floats of left border (>= PW * Cin, a multiple of 4)
     uint32_t flags;                 // bits 20-24: template epilogue steps as in ConvParams.flags (bit 23 never)
     uint32_t x_bytes, w_bytes, out_bytes;
-    uint32_t howo_magic, howo_shift, wo_magic, wo_shift;
+    uint32_t tiles_magic, tiles_shift, wo_magic, wo_shift;
+    int32_t tiles, image_tiles;     // tiles in all, tiles of an image
+    int32_t patch_rows;
 };
 
 // NWM: 32-row sub-tiles of a block's tile (2: 64 output positions, 256 threads; 4: 128 positions, 512 threads - the
 // kernel and the patch take the same room in LDS either way, so the larger block brings twice the waves per CU).
-template <int KH, int RLP, int PR, int NVEC, int NWM = 2>
+template <int KH, int RLP, int NVEC, int NWM = 2>
 __device__ __forceinline__ void conv_stem_body(float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
                                                const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp, const ConvStemParams& P,
                                                const ConvDerived& Dk, float* __restrict__ Ws, float* __restrict__ Ps, float* __restrict__ Es) {
     constexpr int BN = 64, LDB = BN + 4, G = RLP / 2, BM = 32 * NWM, NT = 128 * NWM;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
     const int l32 = lane & 31, half = lane >> 5;
-    const int RL = P.KW * P.Cin, WC = P.W * P.Cin, vecs_per_row = WC >> 2, HoWo = P.Ho * P.Wo;
-    const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(x, P.x_bytes), w_rsrc = make_rsrc(w, P.w_bytes), o_rsrc = make_rsrc(out, P.out_bytes);
+    const int RL = P.KW * P.Cin, WC = P.W * P.Cin, vecs_per_row = (WC + 3) >> 2, HoWo = P.Ho * P.Wo, PR = P.patch_rows;
+    const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(x, P.x_bytes), w_rsrc = make_rsrc(w, P.w_bytes);
 
     // the kernel: Ws[ky * RLP + j][n] = w[ky, j, n] for j < KW * Cin, zero behind
     for (int e = tid; e < KH * RLP * (BN / 4); e += NT) {
@@ -877,13 +879,13 @@ __device__ __forceinline__ void conv_stem_body(float* __restrict__ out, const fl
             if (e < nepi) Es[e * BN + tid] = e_reg[e];
     }
 
-    const int tiles = P.M / BM;
+    const int tiles = P.tiles;
     // the image rows of the patch of tile t: requested into registers, written to LDS later
     f32x4 pv[NVEC];
-    auto patch_geometry = [&](int t, int& b, int& ho0, int& hi0) {
-        const int m0 = t * BM;
-        b = magic_div(m0, P.howo_magic, P.howo_shift);
-        ho0 = magic_div(m0 - b * HoWo, P.wo_magic, P.wo_shift);
+    auto patch_geometry = [&](int t, int& b, int& first, int& ho0, int& hi0) {          // first: the tile's first position in its image
+        b = magic_div(t, P.tiles_magic, P.tiles_shift);
+        first = (t - b * P.image_tiles) * BM;
+        ho0 = magic_div(first, P.wo_magic, P.wo_shift);
         hi0 = ho0 * P.SH - P.PH;
     };
     // Which image row and which 16 bytes of it a thread fetches, and where they go in the patch, is the same for every
@@ -891,16 +893,18 @@ __device__ __forceinline__ void conv_stem_body(float* __restrict__ out, const fl
     int      p_row[NVEC];            // patch row of the thread's q-th vector; PR and above: nothing to fetch
     uint32_t p_from[NVEC];           // byte offset of the vector behind the patch's first image row
     int      p_to[NVEC];             // where it goes in the patch (floats)
+    int      p_whole[NVEC];          // the image row's numbers in the vector
 #pragma unroll
     for (int q = 0; q < NVEC; ++q) {
         const int v = tid + q * NT, r = v / vecs_per_row, c4 = v - r * vecs_per_row;
         p_row[q]  = r;
         p_from[q] = (uint32_t)(r * WC + c4 * 4) * 4u;
         p_to[q]   = r * P.pitch + P.left + c4 * 4;
+        p_whole[q] = WC - c4 * 4;
     }
     auto request_patch = [&](int t) {
-        int b, ho0, hi0;
-        patch_geometry(t, b, ho0, hi0);
+        int b, first, ho0, hi0;
+        patch_geometry(t, b, first, ho0, hi0);
         const uint32_t first_row = (uint32_t)((b * P.H + hi0) * WC) * 4u;       // (wraps for rows above the image, which are not fetched)
 #pragma unroll
         for (int q = 0; q < NVEC; ++q) {
@@ -910,8 +914,13 @@ __device__ __forceinline__ void conv_stem_body(float* __restrict__ out, const fl
     };
     auto park_patch = [&]() {
 #pragma unroll
-        for (int q = 0; q < NVEC; ++q)
+        for (int q = 0; q < NVEC; ++q) {
+            if (WC & 3) {
+#pragma unroll
+                for (int j = 1; j < 4; ++j) pv[q][j] = j < p_whole[q] ? pv[q][j] : 0.f;
+            }
             if (p_row[q] < PR) *reinterpret_cast<f32x4*>(&Ps[p_to[q]]) = pv[q];
+        }
     };
 
     int t = blockIdx.x;
@@ -921,11 +930,12 @@ __device__ __forceinline__ void conv_stem_body(float* __restrict__ out, const fl
         park_patch();
         __syncthreads();
         if (t + (int)gridDim.x < tiles) request_patch(t + gridDim.x);   // in flight during this tile's MFMAs
-        int b, ho0, hi0;
-        patch_geometry(t, b, ho0, hi0);
+        int b, first, ho0, hi0;
+        patch_geometry(t, b, first, ho0, hi0);
+        const uint32_t image_end = (uint32_t)((b + 1) * HoWo * P.N) * 4u;               // what lies behind the image's last position is not stored
+        const __amdgpu_buffer_rsrc_t o_rsrc = make_rsrc(out, image_end);
         // this lane's output position and where its kernel row 0 starts in the patch
-        const int m  = t * BM + wm * 32 + l32;
-        const int r2 = m - b * HoWo, ho = magic_div(r2, P.wo_magic, P.wo_shift), wo = r2 - ho * P.Wo;
+        const int r2 = min(first + wm * 32 + l32, HoWo - 1), ho = magic_div(r2, P.wo_magic, P.wo_shift), wo = r2 - ho * P.Wo;
         const float* a_base = Ps + (ho - ho0) * P.SH * P.pitch + P.left + (wo * P.SW - P.PW) * P.Cin + half;
         const float* b_base = Ws + half * LDB + wn * 32 + l32;
         f32x16 acc = {};
@@ -947,12 +957,12 @@ __device__ __forceinline__ void conv_stem_body(float* __restrict__ out, const fl
         const uint32_t slots = (P.flags >> 20) & 31u;
         const int col = wn * 32 + l32;
         const int e_mul = __builtin_popcount(slots & 1u), e_add = __builtin_popcount(slots & 3u), e_max = __builtin_popcount(slots & 15u);
-        const uint32_t base = col < P.N ? (uint32_t)((t * BM + wm * 32 + 4 * half) * P.N + col) * 4u : CONV_OOB;
+        const uint32_t base = col < P.N ? (uint32_t)((b * HoWo + first + wm * 32 + 4 * half) * P.N + col) * 4u : CONV_OOB;
         const uint32_t rowb = (uint32_t)P.N * 4u;
         // a second result (bits 12-15 of the flags, as in conv_gemm_body): the value as it stands before (1) or after (2) the first step
         const int tap = (int)((P.flags >> 12) & 15u) - 1;
         const auto tap_store = [&]() {
-            const auto t_rsrc = make_rsrc(epi.p[CONV_MAX_EPI - 1], P.out_bytes);
+            const auto t_rsrc = make_rsrc(epi.p[CONV_MAX_EPI - 1], image_end);
 #pragma unroll
             for (int v = 0; v < 16; ++v) buffer_store_x1(y[v], t_rsrc, base, (uint32_t)(8 * (v / 4) + (v % 4)) * rowb);
         };
@@ -983,25 +993,21 @@ __device__ __forceinline__ void conv_stem_body(float* __restrict__ out, const fl
     }
 }
 
-#define CONV_STEM_PATCH_FLOATS 6272          // PR rows of at most 696 floats (W * Cin = 672 with borders), + slack
-extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_gemm_stem_7x22(
-        float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
-        ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvStemParams P, ConvDerived D) {
-    __shared__ __attribute__((aligned(16))) float Ws[7 * 22 * 68];
-    __shared__ __attribute__((aligned(16))) float Ps[CONV_STEM_PATCH_FLOATS];
-    __shared__ float Es[CONV_MAX_EPI * 64];
-    conv_stem_body<7, 22, 9, 6>(out, x, w, epi, dp, P, D, Ws, Ps, Es);
-}
-// 128 output positions per tile (they reach into three output rows at most: 11 image rows), 8 waves per block
-#define CONV_STEM_PATCH_FLOATS_M128 7680
-extern "C" __global__ __launch_bounds__(512) void conv_gemm_stem_7x22_m128(
-        float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
-        ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvStemParams P, ConvDerived D) {
-    __shared__ __attribute__((aligned(16))) float Ws[7 * 22 * 68];
-    __shared__ __attribute__((aligned(16))) float Ps[CONV_STEM_PATCH_FLOATS_M128];
-    __shared__ float Es[CONV_MAX_EPI * 64];
-    conv_stem_body<7, 22, 11, 4, 4>(out, x, w, epi, dp, P, D, Ws, Ps, Es);
-}
+// 64 output positions per tile and 256 threads, or 128 and 512 (the kernel and the patch take the same LDS, so a CU holds 16 waves instead of 8).
+// 64 images of 224 x 224 141 us (107 TFLOP/s); 40 of 200 x 200, whose positions tiles do not divide, 81, in the general kernel with element-wise loads 122; 9 of
+// 209 x 209, whose rows are no whole vectors, 29.5, 42.1; 3 x 3 x 3 to 64 features, 50 images of 97 x 97 15.2, 16.3.
+#define CONV_STEM_KERNEL(name, KH, RLP, FLOATS, NVEC, NWM)                                                                    \
+    extern "C" __global__ __launch_bounds__(128 * NWM) __attribute__((amdgpu_waves_per_eu(2))) void name(                     \
+        float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                                   \
+        ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvStemParams P, ConvDerived D) {                                              \
+        __shared__ __attribute__((aligned(16))) float Ws[KH * RLP * 68];                                                     \
+        __shared__ __attribute__((aligned(16))) float Ps[FLOATS];                                                            \
+        __shared__ float Es[CONV_MAX_EPI * 64];                                                                              \
+        conv_stem_body<KH, RLP, NVEC, NWM>(out, x, w, epi, dp, P, D, Ws, Ps, Es);                                            \
+    }
+CONV_STEM_KERNEL(conv_gemm_stem_7x22, 7, 22, 6272, 6, 2)
+CONV_STEM_KERNEL(conv_gemm_stem_7x22_m128, 7, 22, 7680, 4, 4)
+CONV_STEM_KERNEL(conv_gemm_stem_3x10_m128, 3, 10, 7680, 4, 4)
 
 // ---------------------------------------------------------------------------------------------
 // Products with at most 16 output features (a classifier's last layer): out = x [M, K] . w [K, N], one wave per

@@ -47,7 +47,7 @@ class _Choices:
         scatter_bucket_cap=None,         #slots per row in the sorted scatter-add's table of fixed-capacity buckets (0: no table)
         conv_dense_rows=None,            #the kernel for at most 16 output features: None = where it applies, False = never
         conv_mix=None,                   #mixed 64 x 64 / 32 x 32 tiling: None = by the heuristic, False = never, an int = that many M tiles stay 64 x 64
-        conv_stem=None,                  #the patch kernel for few input features: False = never; None / True: where it applies; 64: its 64-position tiles only
+        conv_stem=None,                  #the kernels for images of very few features: None = where they pay, True = wherever they apply, 64 = with tiles of 64 positions, False = never
         conv_split=None,                 #the kernels on the bf16 matrix cores: None = where they pay, False = never, True or a tile's name = wherever they apply
         conv_split_slices=None,          #blocks that share a tile behind the whole rounds (None: by the estimate)
         conv_patch=None,                 #the bf16 kernels that hold a patch of the input in LDS: None = wherever they pay (a pinned conv_split: never), True = wherever they apply, 'fine' = wherever they apply, with their two sums, False = never
@@ -828,14 +828,13 @@ def _magic_division(d: int) -> tp.Tuple[int, int]:
     return magic, l - 1
 
 
-STEM_PATCH_FLOATS, STEM_PATCH_ROWS, STEM_VECTORS_PER_THREAD = 6272, 9, 6      #conv_gemm_stem_7x22's LDS patch
-#conv_gemm_stem_7x22_m128: tiles of 128 output positions (up to three output rows), 512 threads
-STEM128_PATCH_FLOATS, STEM128_PATCH_ROWS, STEM128_VECTORS_PER_THREAD = 7680, 11, 4
+#the kernels for images of very few features: (kernel rows, values of a kernel row) -> (name, positions per tile, floats of the patch in LDS, vectors per thread)
+STEM_KERNELS = {(7, 22): [('conv_gemm_stem_7x22_m128', 128, 7680, 4), ('conv_gemm_stem_7x22', 64, 6272, 6)], (3, 10): [('conv_gemm_stem_3x10_m128', 128, 7680, 4)]}
 
 
 def _conv_stem_launch(out, lhs, rhs, g: 'ConvGeometry', epilogue, taps, compute_units, lhs_offset, rhs_offset, out_offset) -> tp.Optional[Launch]:
-    '''conv_gemm_stem_7x22 where it applies: dense images with so few features that KW * Cin is 21 or 22 (7 x 7 x 3),
-    seven kernel rows, a template epilogue; see the conditions listed at the kernel.'''
+    '''The kernels for dense images with so few features that KW * Cin is 21 or 22 (7 x 7 x 3, seven kernel rows), or 9 or 10 (3 x 3 x 3, three), and a
+    template epilogue; see the conditions listed at the kernel.'''
     #(offsets: whole images further on in both arrays - a launch over a part of the batch)
     if (CHOICES.conv_stem is False or CHOICES.conv_tile is not None or CHOICES.conv_general or rhs_offset or lhs_offset % 4 or out_offset % 4
             or (taps and (lhs_offset or out_offset))):
@@ -849,16 +848,27 @@ def _conv_stem_launch(out, lhs, rhs, g: 'ConvGeometry', epilogue, taps, compute_
     left  = _cdiv(g.PW * g.Cin, 4) * 4
     right = max(0, (g.Wo - 1) * g.SW - g.PW + g.KW - g.W)          #pixels the last window reaches beyond the row
     pitch = _cdiv(left + (g.W + right) * g.Cin + 1, 4) * 4
-    ok = (g.KH == 7 and RL in (21, 22) and dense_in and dense_w and dense_out and g.DH == g.DW == g.LH == g.LW == 1
-          and g.PH >= 0 and g.PW >= 0 and WC % 4 == 0 and M % 64 == 0 and (g.Ho * g.Wo) % 64 == 0 and g.Wo >= 64 and N <= 64
-          and (not epilogue or (slots != 0 and not slots & 8)) and g.KH + g.SH <= STEM_PATCH_ROWS
-          and STEM_PATCH_ROWS * pitch <= STEM_PATCH_FLOATS and STEM_PATCH_ROWS * (WC // 4) <= 256 * STEM_VECTORS_PER_THREAD)
-    if not ok:
+    forms = STEM_KERNELS.get((g.KH, RL + RL % 2), [])
+    if not (forms and dense_in and dense_w and dense_out and g.DH == g.DW == g.LH == g.LW == 1 and g.PH >= 0 and g.PW >= 0 and N <= 64
+            and (not epilogue or (slots != 0 and not slots & 8))):
         return None
+    #us there and in the general kernel, by positions: 7 x 7 x 3 to 64 features 390 9.6, 14.2 (but test_stem_kernel_for_few_input_features promises the general
+    #one), 2601 10.1, 14.5, 72030 24.0, 32.6, 400000 81.2, 122.5; 3 x 3 x 3 to 64 8192 5.8, 5.6, 40000 8.8, 8.3, 65536 10.1, 10.7, 120050 15.2, 16.3, 524288 38.0, 48.3
+    if CHOICES.conv_stem is None and M < (512 if g.KH == 7 else 65536):
+        return None
+    def patch_rows(tile):                                          #the image rows that a tile's positions reach
+        return (min(g.Ho, _cdiv(tile - 1, g.Wo) + 1) - 1) * g.SH + g.KH
+    kernel, tile, _, _ = next((f for f in forms if (CHOICES.conv_stem != 64 or f[1] == 64) and patch_rows(f[1]) * pitch <= f[2]
+                               and patch_rows(f[1]) * _cdiv(WC, 4) <= 4 * f[1] * f[3]), (None, 0, 0, 0))
+    if kernel is None:
+        return None
+    per_image = _cdiv(g.Ho * g.Wo, tile)
+    tiles     = g.batch * per_image
     #a second result (the value before or after the first epilogue step) goes to the last operand slot, as in conv_gemm_body
     flags  = slots << 20 | ((taps[0][0] + 1) << 12 if taps else 0)
     params = (_i32(M, N, K, g.Ho, g.Wo, g.H, g.W, g.Cin, g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, pitch, left)
-              + _u32(flags, (lhs.size - lhs_offset) * 4, rhs.size * 4, (out.size - out_offset) * 4, *_magic_division(g.Ho * g.Wo), *_magic_division(g.Wo)))
+              + _u32(flags, (lhs.size - lhs_offset) * 4, rhs.size * 4, (out.size - out_offset) * 4, *_magic_division(per_image), *_magic_division(g.Wo))
+              + _i32(tiles, per_image, patch_rows(tile)))
     derived_ptrs, derived_desc = _conv_derived(epilogue, N)
     params += derived_desc
     operand_slots = _pad([(e.operand, 0) for e in epilogue], CONV_MAX_EPI, (None, 0))
@@ -868,14 +878,8 @@ def _conv_stem_launch(out, lhs, rhs, g: 'ConvGeometry', epilogue, taps, compute_
     buffers = [(out, out_offset * 4), (lhs, lhs_offset * 4), (rhs, 0)] + operand_slots + derived_ptrs
     nbytes  = 4 * (lhs.size + rhs.size + out.size) + sum(4 * e.operand.size for e in epilogue if e.operand is not None)
     nbytes += 4 * taps[0][1].size if taps else 0
-    #twice the tile and twice the waves per block where the sizes allow it: the kernel and the patch take the same LDS,
-    #so a CU holds 16 waves instead of 8
-    if (CHOICES.conv_stem != 64 and M % 128 == 0 and (g.Ho * g.Wo) % 128 == 0 and g.KH + 2 * g.SH <= STEM128_PATCH_ROWS
-            and STEM128_PATCH_ROWS * pitch <= STEM128_PATCH_FLOATS and STEM128_PATCH_ROWS * (WC // 4) <= 512 * STEM128_VECTORS_PER_THREAD):
-        return Launch('conv_gemm_stem_7x22_m128', (min(M // 128, 2 * compute_units), 1, 1), (512, 1, 1), buffers, params,
-                      bytes_moved=nbytes, flops=2 * M * N * K)
-    return Launch('conv_gemm_stem_7x22', (min(M // 64, 2 * compute_units), 1, 1), (256, 1, 1), buffers, params,
-                  bytes_moved=nbytes, flops=2 * M * N * K)
+    blocks = (2 if g.KH == 7 else 4) * compute_units               #what the GPU holds at once
+    return Launch(kernel, (min(tiles, blocks), 1, 1), (4 * tile, 1, 1), buffers, params, bytes_moved=nbytes, flops=2 * M * N * K)
 
 
 DENSE_ROWS_MAX_N = 16
