@@ -123,3 +123,20 @@ def test_long_products_stay_with_four_waves(k, launches):
 @pytest.mark.parametrize('k', (200, 1000))
 def test_long_products_with_another_chain(k):
     check_against_oracle(clipped, [ints(-4, 5, 64, k), ints(-3, 4, 2048, k)], exact=True)
+
+
+def swapped(x, w):
+    return lax.conv_general_dilated(x, w, (1, 1), 'SAME', dimension_numbers=('NHWC', 'HWOI', 'NHWC'))
+
+
+@pytest.mark.parametrize('features,copied', ((32, False), (64, True), (256, True)))
+def test_long_products_of_few_rows_read_a_copy(features, copied):
+    '''A kernel operand with its last two dimensions swapped is copied into the dense layout where the contraction is long, however few the rows are.'''
+    interp, _ = vkjax_amd.wrap(swapped, frontend='minijax', plan_only=True)._get_or_create_jaxpr_interpreter([ints(-4, 5, 1, 5, 6, features), ints(-3, 4, 3, 3, 64, features)])
+    assert any('transpose' in l.kernel or l.kernel.startswith('ew_') for l in interp.launches[:1]) == copied, [l.kernel for l in interp.launches]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('features', (32, 64, 256))
+def test_swapped_kernel_operands(features):
+    check_against_oracle(swapped, [ints(-4, 5, 1, 5, 6, features), ints(-3, 4, 3, 3, 64, features)], exact=True)

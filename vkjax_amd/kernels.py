@@ -980,9 +980,17 @@ def _conv_fast_paths(lhs: Buffer, rhs: Buffer, g: ConvGeometry, lhs_offset: int 
     return needs_masks, x_bias, a_fast, b_fast, c_contig
 
 
+DENSE_COPY_MIN_K = 512
+
+
 def dense_copy_applies(lhs: Buffer, g: ConvGeometry, out_size: tp.Optional[int] = None) -> bool:
-    '''A kernel operand of any layout may be copied into the dense one first: it is no bigger than the activations.'''
-    return g.N % 4 == 0 and g.M >= 256 and g.K * g.N <= lhs.size + (g.M * g.N if out_size is None else out_size) and min(g.ws) >= 0
+    '''A kernel operand of any layout may be copied into the dense one first: it is no bigger than the activations, or the contraction is long. A
+    step of it with element-wise loads takes 1.6 us per 32 in the general kernels and 2 per 128 where four waves share a tile, with 16-byte loads 0.65
+    and 0.5; the copies of a network's kernels are one launch, at about 3 TB/s. Training steps of ResNet-50
+    without and with the second clause: 8 images of 160 x 160 3.30, 2.96 ms, 4 of 96 x 96 2.28, 2.03, 5 of 224 x 224 3.39, 3.06; from 1024 on only 2.98, 2.06, 3.07,
+    from 128 on 2.96, 2.03, 3.06.'''
+    small = g.M >= 256 and g.K * g.N <= lhs.size + (g.M * g.N if out_size is None else out_size)
+    return g.N % 4 == 0 and min(g.ws) >= 0 and (small or (g.K >= DENSE_COPY_MIN_K and g.N > DENSE_ROWS_MAX_N))
 
 
 def _kernel_operand_in_rows(g: ConvGeometry, rhs_offset: int = 0) -> bool:
