@@ -140,3 +140,18 @@ def test_long_products_of_few_rows_read_a_copy(features, copied):
 @pytest.mark.parametrize('features', (32, 64, 256))
 def test_swapped_kernel_operands(features):
     check_against_oracle(swapped, [ints(-4, 5, 1, 5, 6, features), ints(-3, 4, 3, 3, 64, features)], exact=True)
+
+
+#classes of an input dilated by 2 (or 3): every second (third) row and column of the result, each from its own taps
+CLASSES = [((2, 5, 6, 256), (3, 3, 256, 36), ((1, 2), (2, 1)), 2), ((1, 4, 9, 512), (2, 3, 512, 64), ((2, 1), (1, 1)), 2), ((3, 3, 3, 1024), (1, 1, 1024, 68), ((0, 1), (0, 1)), 2),
+           ((1, 3, 4, 128), (5, 5, 128, 32), ((4, 3), (2, 4)), 3), ((8, 5, 5, 512), (3, 3, 512, 512), ((1, 2), (1, 2)), 2)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('x,w,padding,dilation', CLASSES)
+def test_classes_of_a_dilated_input(x, w, padding, dilation):
+    print('dilated input:', x, w, padding, dilation, flush=True)
+    def f(x, w):
+        return lax.conv_general_dilated(x, w, (1, 1), padding, lhs_dilation=(dilation, dilation), dimension_numbers=('NHWC', 'HWIO', 'NHWC'))
+    _, _, fn = check_against_oracle(f, [ints(-4, 5, *x), ints(-3, 4, *w)], exact=True)
+    assert 'conv_gemm_32x32x128_ks4_strided' in kernels_of(fn), kernels_of(fn)

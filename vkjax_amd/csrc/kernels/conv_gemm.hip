@@ -735,13 +735,13 @@ CONV_TILE(32x32x64, 1, 1, 1, 1, 64)
 #include "conv_quad.h"
 
 // one 32 x 32 tile per block, the k step of 128 split over four waves (chunk 1)
-#define CONV_QUAD_KERNEL(name, BK, B_LOADS)                                                                       \
+#define CONV_QUAD_KERNEL(name, BK, B_LOADS, ...)                                                                       \
     extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B_LOADS != QUAD_B_WORDS ? 4 : 3))) void name(          \
         float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,                   \
         ConvEpiPtrs epi, ConvDerivedPtrs dp, ConvParams P, ConvDerived D) {                                  \
         __shared__ __attribute__((aligned(16))) float pool[conv_quad_floats<BK>()];                          \
         const ConvRegion all{0, P.tiles_m, P.tiles_n, 0};                                                    \
-        conv_quad_body<BK, B_LOADS, false>(pool, all, out, x, w, epi, dp, P, D);                                  \
+        conv_quad_body<BK, B_LOADS, false, ##__VA_ARGS__>(pool, all, out, x, w, epi, dp, P, D);                                  \
     }
 CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4, 128, QUAD_B_COLUMNS)
 // the same for a transposed kernel operand, and with element-wise loads of it (any strides)
@@ -749,6 +749,9 @@ CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4t, 128, QUAD_B_ROWS)
 CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4g, 128, QUAD_B_WORDS)
 // the same with a 64-long k step, for windows over 64 (or 192, ...) input features, whose taps a 128-long step would straddle
 CONV_QUAD_KERNEL(conv_gemm_32x32x64_ks4, 64, QUAD_B_COLUMNS)
+// the first for results whose rows lie apart: the input gradients of strided convolutions, one launch per class of positions. 8 images, 5 x 5 x 512 to
+// 10 x 10 x 512, 3 x 3 windows: its largest class 50.6 us in the general kernel, 14.8 here, the others 29.9 and 9.1, 28.6 and 9.2, 15.0 and 6.4.
+CONV_QUAD_KERNEL(conv_gemm_32x32x128_ks4_strided, 128, QUAD_B_COLUMNS, true)
 // Those with a k step of 128 with several blocks per tile, each summing a slice of the contraction (k_split_steps): few tiles leave CUs idle. A slice's sums make a
 // round trip to memory and the counter another, 2 to 2.5 us for 32 x 32 numbers; a launch that adds them takes 3.2 and a start.
 // 196 x 2304 x 256: 13.2 us by one block per tile, 8.5 by four; 150 x 4608 x 512 22.4, 12.2 by three; 588 x 4608 x 512 38.6, 29.6 by four.

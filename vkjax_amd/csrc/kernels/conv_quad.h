@@ -28,9 +28,10 @@ template <int BK> constexpr int conv_quad_floats() { return 4 * conv_quad_wave_f
 
 // BK: k step of the block. SHARED: several blocks share a tile, each summing a slice
 // of the contraction; a slice leaves its sums in `partial`, and the block that arrives last at the tile's counter adds them.
-// Requirements (the host checks them): 16-byte loads of A, K = KH * KW * Cin with one tap or Cin a multiple of BK / 4, a row-major result and an
+// STRIDED: the result's rows lie apart (a class of the outputs of a convolution over a dilated input): ConvParams' ws_* are its strides, and there is no epilogue.
+// Requirements (the host checks them): 16-byte loads of A, K = KH * KW * Cin with one tap or Cin a multiple of BK / 4, a row-major result (or STRIDED) and an
 // epilogue that conv_straight_steps takes. ConvParams' os_* and LH, LW hold divisors here (see there).
-template <int BK, int B_LOADS, bool SHARED>
+template <int BK, int B_LOADS, bool SHARED, bool STRIDED = false>
 __device__ __forceinline__ void conv_quad_body(float* __restrict__ pool, const ConvRegion region, float* __restrict__ out, const float* __restrict__ x,
                                                const float* __restrict__ w, const ConvEpiPtrs& epi, const ConvDerivedPtrs& Dp, const ConvParams& Pk,
                                                const ConvDerived& Dk, float* __restrict__ partial = nullptr, uint32_t* __restrict__ arrivals = nullptr) {
@@ -346,6 +347,18 @@ __device__ __forceinline__ void conv_quad_body(float* __restrict__ pool, const C
 #pragma unroll
         for (int s = 1; s < CONV_MAX_SHARES; ++s)
             if (s < P.slices) sum += q[s];
+    }
+    if constexpr (STRIDED) {
+        static_assert(B_LOADS == QUAD_B_COLUMNS, "the strides' places are free there");
+        const int n = n0 + l32;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int m = m0 + 8 * kw + 4 * half + v, b = magic_div(m, P.howo_magic, P.howo_shift), r2 = m - b * (P.Ho * P.Wo);
+            const int ho = magic_div(r2, P.wo_magic, P.wo_shift), wo = r2 - ho * P.Wo;
+            const uint32_t at = (uint32_t)(b * Pk.ws_r + ho * Pk.ws_s + wo * Pk.ws_c + n * Pk.ws_n) * 4u;
+            buffer_store_x1(sum[v], o_rsrc, m < P.M && n < P.N ? at : CONV_OOB);
+        }
+        return;
     }
     float y[4] = {sum[0], sum[1], sum[2], sum[3]};
     conv_straight_steps<4>(y, quarter, (P.flags >> 20) & 31u, (int)((P.flags >> 12) & 15u) - 1, Es, 32, l32, [&]() {

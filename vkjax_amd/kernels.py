@@ -1193,6 +1193,12 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
     short_step = ksplit and g.Cin % 128 != 0 and g.KH * g.KW != 1
     if short_step and not b_fast:
         ksplit = False
+    #results whose rows lie apart, without an epilogue and with dense kernel operands: the same by strides
+    strided = (not ksplit and not c_contig and b_fast and not epilogue and not taps and g.k_splits == 1 and min(g.os) >= 0
+               and (g.Cin % 32 == 0 or g.KH * g.KW == 1) and _four_waves_per_tile(g, a_fast, True, compute_units, True))
+    ksplit = ksplit or strided
+    if strided:
+        short_step = False
     if ksplit:
         tag, bm, bn, nt, bk, lean = '32x32', 32, 32, 256, 64 if short_step else 128, True
     tiles_m, tiles_n = _cdiv(M, bm), _cdiv(N, bn)
@@ -1202,7 +1208,7 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
         if (not ksplit or short_step or epilogue or taps or out_offset or out.size != g.k_splits * M * N
                 or _cdiv(_cdiv(K, 128), k_split_steps) != g.k_splits):
             raise ValueError('a sliced contraction needs the four-waves-per-tile kernel, no epilogue and one [M, N] matrix per non-empty slice')
-    elif g.shares is not None and ksplit and not short_step:
+    elif g.shares is not None and ksplit and not short_step and not strided:
         k_split_steps = _cdiv(_cdiv(K, bk), g.shares.count)
         assert _cdiv(_cdiv(K, bk), k_split_steps) == g.shares.count and tiles_m * tiles_n <= g.shares.arrivals.size and not out_offset
     chunk = (CHOICES.conv_chunk or choose_conv_chunk(tiles_m, tiles_n, compute_units)) if lean and not ksplit else 1
@@ -1245,7 +1251,7 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
               #(rows beyond M are dropped by the descriptor's size: with slices, that of one slice's matrix)
               + _u32(flags, *descs, x_bytes, w_bytes, M * N * 4 if k_split_steps else (out.size - out_offset) * 4,
                      *_magic_division(g.Ho * g.Wo), *_magic_division(g.Wo))
-              + dilation + _i32(g.xs[3], *g.ws) + out_strides + _i32(split_tiles_m, k_split_steps, m_blocks) + per_block + _i32(tiles_m % m_blocks if m_blocks else 0))
+              + dilation + _i32(g.xs[3], *(g.os if strided else g.ws)) + out_strides + _i32(split_tiles_m, k_split_steps, m_blocks) + per_block + _i32(tiles_m % m_blocks if m_blocks else 0))
     derived_ptrs, derived_desc = _conv_derived(epilogue, N)
     params += derived_desc
     buffers = [(out, out_offset * 4), (lhs, lhs_offset * 4), (rhs, rhs_offset * 4)]
@@ -1257,7 +1263,7 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
         assert operand_slots[-1] == (None, 0)
         operand_slots[-1] = (tap_buffer, 0)
     buffers += operand_slots + derived_ptrs
-    kernel  = f'conv_gemm_{tag}x{bk}_' + (('ks4' if b_fast else 'ks4t' if _kernel_operand_in_rows(g, rhs_offset) else 'ks4g') + ('_shared' if shared else '') if ksplit else 'lean' if lean else ('f' if a_fast else 'g') + ('f' if b_fast else 'g'))
+    kernel  = f'conv_gemm_{tag}x{bk}_' + (('ks4_strided' if strided else 'ks4' if b_fast else 'ks4t' if _kernel_operand_in_rows(g, rhs_offset) else 'ks4g') + ('_shared' if shared else '') if ksplit else 'lean' if lean else ('f' if a_fast else 'g') + ('f' if b_fast else 'g'))
     nbytes  = 4 * (lhs.size + rhs.size + out.size) + sum(4 * e.operand.size for e in epilogue if e.operand is not None)
     nbytes += 4 * tap_buffer.size if taps else 0
     blocks = (m_blocks or _cdiv(tiles_m, chunk)) * tiles_n * slices
