@@ -990,7 +990,8 @@ def dense_copy_applies(lhs: Buffer, g: ConvGeometry, out_size: tp.Optional[int] 
     without and with the second clause: 8 images of 160 x 160 3.30, 2.96 ms, 4 of 96 x 96 2.28, 2.03, 5 of 224 x 224 3.39, 3.06; from 1024 on only 2.98, 2.06, 3.07,
     from 128 on 2.96, 2.03, 3.06.'''
     small = g.M >= 256 and g.K * g.N <= lhs.size + (g.M * g.N if out_size is None else out_size)
-    return g.N % 4 == 0 and min(g.ws) >= 0 and (small or (g.K >= DENSE_COPY_MIN_K and g.N > DENSE_ROWS_MAX_N))
+    #(operands that the kernels refuse for their size are not copied first)
+    return g.N % 4 == 0 and min(g.ws) >= 0 and (small or (g.K >= DENSE_COPY_MIN_K and g.N > DENSE_ROWS_MAX_N and g.K * g.N * 4 < 2**31))
 
 
 def _kernel_operand_in_rows(g: ConvGeometry, rhs_offset: int = 0) -> bool:
