@@ -111,3 +111,34 @@ def test_where_they_apply():
     assert not short(200704, 64, 256, conv_split='128x64') and not short(200704, 64, 256, conv_short=False) and not short(200704, 64, 256, conv_split=False)
     image = lambda stride: lambda x, w: mj.lax.conv_general_dilated(x, w.reshape((1, 1) + w.shape), (stride, stride), 'VALID', dimension_numbers=('NHWC', 'HWIO', 'NHWC'))
     assert short(0, 64, 256, f=image(1), x=(64, 56, 56, 64)) and not short(0, 64, 256, f=image(2), x=(64, 112, 112, 64))
+
+
+def contract(of_lhs, of_rhs):
+    return lambda x, w: mj.lax.dot_general(x, w, (((of_lhs,), (of_rhs,)), ((), ())))
+
+
+def planned(f, *shapes, **choice):
+    with K.overrides(**choice):
+        launches = JaxprInterpreter(mj.make_jaxpr(f)(*[np.broadcast_to(np.float32(0), s) for s in shapes]), plan_only=True).launches
+    return [l.kernel for l in launches if l.kernel.startswith('conv_gemm')]
+
+
+@pytest.mark.parametrize('rows', (33, 40, 64))
+def test_operands_contracted_over_their_rows_are_not_for_them(rows):
+    '''Plan only: the kernel reads a row's features one behind the other. A dense layer's kernel gradient on so few samples, among others.'''
+    gradient = mj.grad(lambda w, x: (lambda y: jnp.sum(y * y))(jnp.dot(x, w)))
+    for choice in (dict(), dict(conv_short=True)):
+        assert not any('short' in k for k in planned(contract(0, 0), (rows, 4096), (rows, 4096), **choice))
+        assert not any('short' in k for k in planned(contract(0, 1), (rows, 4096), (4096, rows), **choice))
+        assert not any('short' in k for k in planned(gradient, (4096, 4096), (rows, 4096), **choice))
+    assert planned(contract(1, 1), (65536, 64), (256, 64)) == ['conv_gemm_split_short']           #(a transposed kernel operand is packed like any other)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('rows,m,n', ((64, 4096, 4096), (36, 70, 96), (64, 33, 257)))
+@pytest.mark.parametrize('of_rhs', (0, 1))
+def test_values_of_operands_contracted_over_their_rows(rows, m, n, of_rhs):
+    x, w = ints((rows, m)), ints((rows, n), -3, 4)
+    with K.overrides(**(dict() if m == 4096 else dict(conv_short=True))):
+        y = np.asarray(vkjax_amd.wrap(contract(0, of_rhs), frontend='minijax')(x, w.T.copy() if of_rhs else w))
+    assert np.array_equal(y, x.T @ w)                          #(exact in any order)
