@@ -142,3 +142,23 @@ def test_values_of_operands_contracted_over_their_rows(rows, m, n, of_rhs):
     with K.overrides(**(dict() if m == 4096 else dict(conv_short=True))):
         y = np.asarray(vkjax_amd.wrap(contract(0, of_rhs), frontend='minijax')(x, w.T.copy() if of_rhs else w))
     assert np.array_equal(y, x.T @ w)                          #(exact in any order)
+
+
+@pytest.mark.parametrize('k', (37, 38, 39, 61, 63))
+def test_contractions_that_are_no_whole_vectors_are_not_for_them(k):
+    '''Plan only.'''
+    for choice in (dict(), dict(conv_short=True)):
+        assert not any('short' in name for name in planned(jnp.dot, (200000, k), (k, 96), **choice))
+    assert planned(jnp.dot, (200000, 40), (40, 96)) == ['conv_gemm_split_short']
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('k', (33, 37, 62, 63))
+def test_rows_do_not_take_from_the_next(k):
+    '''Every other row is not finite, pinned to these kernels where they apply.'''
+    x, w = ints((131, k)), ints((k, 96), -3, 4)
+    x[1::4], x[3::4] = np.inf, np.nan
+    with K.overrides(conv_short=True):
+        y = np.asarray(vkjax_amd.wrap(jnp.dot, frontend='minijax')(x, w))
+    assert np.array_equal(y[::2], x[::2] @ w)                  #(exact in any order)
+    assert not np.isfinite(y[1::2]).any()

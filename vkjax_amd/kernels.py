@@ -1347,8 +1347,9 @@ def conv_patch_applies(g: ConvGeometry) -> bool:
 
 def conv_short_applies(g: ConvGeometry, c_contig: bool) -> bool:
     '''Dense rows of at most 64 features (a flattened geometry), the result's rows dense too.'''
-    #(the kernel has no stride along the contraction: an operand that is contracted over its rows is not for it)
-    return (c_contig and 0 < g.K <= 64 and g.xs[3] == 1 and g.xs[1] >= g.K and (g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.LH, g.LW) == (1,) * 4 + (0,) * 2 + (1,) * 2
+    #(the kernel has no stride along the contraction: an operand that is contracted over its rows is not for it; nor does it clear what the last vector
+    #of a row that is no whole number of them holds of the next row, which zeros on the other side would not keep out where it is not finite)
+    return (c_contig and 0 < g.K <= 64 and g.xs[3] == 1 and g.xs[1] >= g.K and _features_in_vectors(g) and (g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, g.LH, g.LW) == (1,) * 4 + (0,) * 2 + (1,) * 2
             and g.batch == 1 and g.Wo == 1 and g.Ho == g.H)
 
 
