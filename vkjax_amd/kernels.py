@@ -981,10 +981,11 @@ def _conv_fast_paths(lhs: Buffer, rhs: Buffer, g: ConvGeometry, lhs_offset: int 
 
 
 DENSE_COPY_MIN_K = 512
+DENSE_COPY_SMALL = 14 << 20         #values
 
 
 def dense_copy_applies(lhs: Buffer, g: ConvGeometry, out_size: tp.Optional[int] = None) -> bool:
-    '''A kernel operand of any layout may be copied into the dense one first: it is no bigger than the activations, or the contraction is long. A
+    '''A kernel operand of any layout counts as a dense one, into which it may be copied first: it is no bigger than the activations, or the contraction is long. A
     step of it with element-wise loads takes 1.6 us per 32 in the general kernels and 2 per 128 where four waves share a tile, with 16-byte loads 0.65
     and 0.5; the copies of a network's kernels are one launch, at about 3 TB/s. Training steps of ResNet-50
     without and with the second clause: 8 images of 160 x 160 3.30, 2.96 ms, 4 of 96 x 96 2.28, 2.03, 5 of 224 x 224 3.39, 3.06; from 1024 on only 2.98, 2.06, 3.07,
@@ -994,13 +995,23 @@ def dense_copy_applies(lhs: Buffer, g: ConvGeometry, out_size: tp.Optional[int] 
     return g.N % 4 == 0 and min(g.ws) >= 0 and (small or (g.K >= DENSE_COPY_MIN_K and g.N > DENSE_ROWS_MAX_N and g.K * g.N * 4 < 2**31))
 
 
+def dense_copy_pays(lhs: Buffer, g: ConvGeometry, out_size: tp.Optional[int] = None) -> bool:
+    '''... and it is copied where more than one tile of rows reads it, or where it is small: the copy reads and writes it once, and takes its room in HBM. us with
+    the copy, without. Transposed matrices that four waves per tile do not read as they are: 1 x 2048 x 50000 280, 223; 32 x 2048 x 50000 281, 249; 8 x 1024 x 128000
+    336, 310; 64 x 768 x 30524, one row of 64 x 64 tiles, 71, 62; 64 x 512 x 30000 (61 MB) 47, 42; 64 x 2048 x 50000 318, 338; but 64 x 512 x 20000, two rows of 32 x 32,
+    39, 50; 65 x 768 x 30524 92, 159; 128 x 4096 x 16384 264, 333; 256 x 2048 x 50000 612, 953. A tile of rows of a dilated input's class 25 x 512 x 8192 21, 28, x 4096 x
+    1024 31, 155. Windows: 16 rows x 9216 x 1024 (38 MB) 34, 44, x 1536 (57 MB) 36, 37, x 2048 44, 43; 4 rows x 18432 x 2048 82, 79; 49 rows x 4608 x 4096 52, 76.'''
+    one_tile = 32 if g.KH * g.KW != 1 else min(choose_conv_tile(g.M, g.N)[1], 64)
+    return dense_copy_applies(lhs, g, out_size) and (g.M > one_tile or g.K * g.N <= DENSE_COPY_SMALL)
+
+
 def _kernel_operand_in_rows(g: ConvGeometry, rhs_offset: int = 0) -> bool:
     '''A transposed matrix: the four-waves-per-tile kernels read it with 16-byte loads along the contraction.'''
     return g.KH * g.KW == 1 and g.ws[2] == 1 and g.ws[3] >= 0 and rhs_offset % 4 == 0 and not CHOICES.conv_b_general
 
 
 def _kernel_operand_in_vectors(lhs: Buffer, g: ConvGeometry, b_fast: bool, rhs_offset: int = 0) -> bool:
-    '''For the rule of the four-waves-per-tile kernels, transposed matrices count as dense ones where they would be copied into such a one.'''
+    '''For the rule of the four-waves-per-tile kernels, which read transposed matrices in vectors too: those count as dense ones where dense_copy_applies.'''
     return b_fast or (_kernel_operand_in_rows(g, rhs_offset) and dense_copy_applies(lhs, g))
 
 

@@ -718,10 +718,10 @@ def conv_general_dilated(bufferpool, equation):
 def _with_dense_kernel(bufferpool, equation, rhs: Buffer, geom: 'K.ConvGeometry', lhs: Buffer, outbuf: Buffer, rhs_offset: int = 0):
     '''A kernel operand that is not laid out [ky, kx, in, out] with `out` contiguous (the swapped and reversed
     kernel of an input gradient, a transposed weight matrix, every other tap of a kernel) is copied into that
-    layout first when it is no bigger than the activations: the GEMM kernel then reads it with 16-byte loads.
+    layout first where that pays (K.dense_copy_pays): the GEMM kernel then reads it with 16-byte loads.
     Returns (ops, rhs, geometry, rhs offset).'''
     N, dense = geom.N, (geom.KW * geom.Cin * geom.N, geom.Cin * geom.N, geom.N, 1)
-    if ((geom.ws == dense and rhs_offset % 4 == 0) or not K.dense_copy_applies(lhs, geom, outbuf.size)
+    if ((geom.ws == dense and rhs_offset % 4 == 0) or not K.dense_copy_pays(lhs, geom, outbuf.size)
             or K.conv_reads_transposed(lhs, rhs, geom, rhs_offset)):
         return [], rhs, geom, rhs_offset
     position = bufferpool.op_counter
