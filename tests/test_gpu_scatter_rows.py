@@ -71,3 +71,21 @@ def test_slots_by_the_rule():
     caps = [K.choose_scatter_bucket_cap(n, rows, cols) for n, rows, cols in ((262144, 65536, 256), (32000, 100000, 24), (262144, 1000, 256), (90000, 5000, 200), (1000, 3000000, 16), (5, 2**27, 4))]
     assert caps == [16, 8, 1024, 128, 4, 0]
     assert all(cap * rows <= max(8 * n, 1 << 24) for cap, (n, rows) in zip(caps, ((262144, 65536), (32000, 100000), (262144, 1000), (90000, 5000), (1000, 3000000), (5, 2**27))))
+
+
+def test_crowded_neighbours_do_not_share_a_wave():
+    '''Sixteen rows with a thousand updates each take about as long next to each other as far apart (in one wave, one after the other: some ten times as long).'''
+    rows, cols, each = 20000, 16, 1000
+    def time(crowded):
+        idx = np.repeat(np.asarray(crowded, np.int32), each)
+        program = JaxprInterpreter(mj.make_jaxpr(scatter)(*(args := [np.zeros((rows, cols), np.float32), idx, np.ones((idx.size, cols), np.float32)])))
+        assert program.launches[-1].kernel == 'scatter_rows_sum_short_f_v4'
+        program.upload_inputs(*args)
+        best = min(program.replay(2) for _ in range(6))
+        y, = program.read_outputs()
+        assert (y[crowded] == each).all() and y.sum() == idx.size * cols
+        return best
+    with K.overrides(scatter_sort_threshold=0):
+        apart, neighbours = time([997 * k + 5 for k in range(16)]), time(list(range(4096, 4096 + 16)))
+    print('crowded rows apart, neighbours:', apart, neighbours, flush=True)
+    assert neighbours < 3 * apart

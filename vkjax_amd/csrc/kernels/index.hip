@@ -338,7 +338,11 @@ __device__ __forceinline__ void scatter_rows_sum_body(uint32_t* __restrict__ out
 // Several rows per wave, 2^shift lanes for each (that many vectors hold a row): short rows leave a wave of their own mostly idle, and it is a chain of
 // counter, bucket, updates and store whatever their length. Buckets of up to SHORT entries within their slots are sorted in LDS, by counting for
 // each entry the smaller ones; a row with more is left to the whole wave afterwards. The sums of 262144 updates of 64 bytes into 100000 rows
-// 41.6 -> 16 us (24.6 MB).
+// 41.6 -> 17.5 us (24.6 MB).
+// Crowded rows are often neighbours (a vocabulary sorted by frequency), so a wave's rows are not: they lie as far apart as the grid has waves. Gather and
+// scatter-add of such indices (by Zipf's law) with neighbouring rows in a wave, and with these: 100000 x 16, 262144 updates 35.2, 14.4 ms (one row per wave 14.5);
+// 20000 x 24, 100000 12.5, 5.9 (5.8). Of evenly spread ones 38.3, 39.9 us (64.5), 500000 x 16, 500000 updates 71, 77 (185): the rows of 64 bytes are written one by
+// one. (Stretches of 1024 rows dealt out to 16 blocks: the same for both, but rows crowded over a whole stretch share a wave again.)
 template <int VEC, bool IS_FLOAT>
 __device__ __forceinline__ void scatter_short_rows_body(uint32_t* __restrict__ out, const uint32_t* __restrict__ operand,
                                                         const uint32_t* __restrict__ updates, uint32_t* count, const uint32_t* fixed,
@@ -348,7 +352,7 @@ __device__ __forceinline__ void scatter_short_rows_body(uint32_t* __restrict__ o
     typedef uint32_t vec_t __attribute__((ext_vector_type(VEC)));
     __shared__ uint32_t entries[4][2][64 / LEAST][SHORT];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u, lanes = 1u << shift, group = lane >> shift, mine = lane & (lanes - 1u), first = group << shift;
-    const uint32_t row = ((blockIdx.x * 4u + wave) << (6u - shift)) + group;
+    const uint32_t row = group * gridDim.x * 4u + blockIdx.x * 4u + wave;
     uint32_t n = 0;
     if (mine == 0u && row < P.n_rows) {
         n = count[row];

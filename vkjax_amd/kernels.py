@@ -2090,7 +2090,7 @@ def scatter_add_rows_sorted(out: Buffer, operand: Buffer, idx: Buffer, updates: 
     table_passes = 1 if operand_is_scalar else 2
     lanes = max(4, _pow2_at_least(row_len // vec))
     #Several rows per wave where there are more rows than waves the chip holds and few updates for each (us of gather and scatter-add, one row per
-    #wave and several; rows x row length, updates: 100000 x 16, 262144 63.6, 37.9; 100000 x 24, 32000 30.0, 15.9; 20000 x 24, 100000 25.5, 21.2; 40000 x 31, 131072 39.7, 35.8;
+    #wave and several; rows x row length, updates: 100000 x 16, 262144 64.5, 39.9; 100000 x 24, 32000 30.7, 17.5; 20000 x 24, 100000 25.8, 20.8; 40000 x 31, 131072 40.4, 36.6;
     #but 5000 x 24, 32000 12.8, 15.2; 12000 x 40, 96000 25.4, 28.8; 20000 x 16, 262144 42.3, 65.9; 30000 x 128, 60000 32.6, 33.4)
     short = (cap >= 8 and lanes <= 32 and
              (CHOICES.scatter_short_rows if CHOICES.scatter_short_rows is not None else row_len <= 64 and n_rows >= 8192 and n_idx <= 6 * n_rows))
