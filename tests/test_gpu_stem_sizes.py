@@ -44,3 +44,19 @@ def test_patches_that_do_not_fit():
     for width, stem in ((200, True), (1000, False)):
         interp, _ = vkjax_amd.wrap(f, frontend='minijax', plan_only=True)._get_or_create_jaxpr_interpreter([ints(-1, 2, 1, 20, width, 3), ints(-1, 2, 7, 7, 3, 16)])
         assert interp.launches[-1].kernel.startswith('conv_gemm_stem') == stem, interp.launches[-1].kernel
+
+
+@pytest.mark.parametrize('window,stride,images,size,features,stem', [
+    (7, 2, 1, 64, 8, True), (7, 2, 64, 224, 64, True), (7, 2, 9, 209, 4, True), (7, 2, 200, 24, 64, True), (7, 2, 100, 9, 64, True),
+    (7, 2, 300, 9, 64, False), (7, 2, 2000, 9, 64, False), (7, 2, 1000, 16, 8, False),
+    (3, 2, 50, 97, 64, True), (3, 2, 50, 97, 33, True), (3, 2, 50, 97, 32, False), (3, 2, 64, 224, 8, False), (3, 1, 90, 32, 64, True), (3, 1, 120, 32, 40, True),
+    (3, 2, 20, 141, 64, False), (3, 1, 2000, 9, 64, False), (3, 1, 1100, 8, 64, False), (3, 1, 300, 17, 64, False), (3, 2, 200, 41, 64, False)])
+def test_where_they_pay(window, stride, images, size, features, stem):
+    '''Plan only: few features, or images that fill their tiles badly, are left to the general kernel.'''
+    from vkjax_amd.jaxpr_interpreter import JaxprInterpreter
+    p = window // 2
+    def f(x, w):
+        return lax.conv_general_dilated(x, w, (stride, stride), ((p, p), (p, p)), dimension_numbers=('NHWC', 'HWIO', 'NHWC'))
+    zeros  = lambda *s: np.broadcast_to(np.float32(0), s)
+    launch = JaxprInterpreter(mj.make_jaxpr(f)(zeros(images, size, size, 3), zeros(window, window, 3, features)), plan_only=True).launches[-1]
+    assert launch.kernel.startswith('conv_gemm_stem') == stem, launch.kernel

@@ -832,6 +832,20 @@ def _magic_division(d: int) -> tp.Tuple[int, int]:
 STEM_KERNELS = {(7, 22): [('conv_gemm_stem_7x22_m128', 128, 7680, 4), ('conv_gemm_stem_7x22', 64, 6272, 6)], (3, 10): [('conv_gemm_stem_3x10_m128', 128, 7680, 4)]}
 
 
+def _conv_stem_pays(g: 'ConvGeometry', tile: int, tiles: int, compute_units: int) -> bool:
+    '''us there and in the general kernel, which takes its tiles across images and computes 32 columns where there are no more.'''
+    filled = g.M / (tile * tiles)
+    #7 x 7 x 3 to 64 features, by positions: 390 9.6, 14.2 (but test_stem_kernel_for_few_input_features promises the general one), 2601 10.1, 14.5, 72030 24.0, 32.6,
+    #400000 77, 119; to 8 99225 28, 33, 400000 74, 97. Images of fewer positions than a tile: 100 of 25 9.8, 14.5, 300 of 25 15.5, 14.6, 2000 of 25 48, 26; 1000 of 64 27.8,
+    #26.9, to 8 26.4, 23.2; 200 of 144 17.3, 18.3; 500 of 100 17.8, 26.9
+    if g.KH == 7:
+        return g.M >= 512 and (tiles <= compute_units or filled >= 0.55)
+    #3 x 3 x 3. Features: 120050 positions to 8 13.9, 10.7, to 32 15.2, 12.2, to 33 15.4, 15.9, to 64 16.0, 16.6. Positions, to 64: 40000 8.8, 8.3, 69629 12.2, 12.2, 92160 12.5,
+    #13.6, 175616 19.9, 21.0, 802816 55.9, 68.2; three tiles fit a CU, a few more are a second round: 94221 (754 tiles) 12.9, 13.8, 100820 (800) 15.9, 15.5, 112908 (888)
+    #16.3, 15.8, 120050 (950) 16.0, 16.6. Tiles: 2000 images of 81 22.0, 19.1, 1100 of 64 16.7, 12.0, 300 of 289 14.8, 13.5, 200 of 441 15.5, 13.4, 4000 of 36 34.4, 17.5
+    return g.N > 32 and g.M >= 73728 and filled >= 0.95 and not 3 < tiles / compute_units < 3.6
+
+
 def _conv_stem_launch(out, lhs, rhs, g: 'ConvGeometry', epilogue, taps, compute_units, lhs_offset, rhs_offset, out_offset) -> tp.Optional[Launch]:
     '''The kernels for dense images with so few features that KW * Cin is 21 or 22 (7 x 7 x 3, seven kernel rows), or 9 or 10 (3 x 3 x 3, three), and a
     template epilogue; see the conditions listed at the kernel.'''
@@ -852,10 +866,6 @@ def _conv_stem_launch(out, lhs, rhs, g: 'ConvGeometry', epilogue, taps, compute_
     if not (forms and dense_in and dense_w and dense_out and g.DH == g.DW == g.LH == g.LW == 1 and g.PH >= 0 and g.PW >= 0 and N <= 64
             and (not epilogue or (slots != 0 and not slots & 8))):
         return None
-    #us there and in the general kernel, by positions: 7 x 7 x 3 to 64 features 390 9.6, 14.2 (but test_stem_kernel_for_few_input_features promises the general
-    #one), 2601 10.1, 14.5, 72030 24.0, 32.6, 400000 81.2, 122.5; 3 x 3 x 3 to 64 8192 5.8, 5.6, 40000 8.8, 8.3, 65536 10.1, 10.7, 120050 15.2, 16.3, 524288 38.0, 48.3
-    if CHOICES.conv_stem is None and M < (512 if g.KH == 7 else 65536):
-        return None
     def patch_rows(tile):                                          #the image rows that a tile's positions reach
         return (min(g.Ho, _cdiv(tile - 1, g.Wo) + 1) - 1) * g.SH + g.KH
     kernel, tile, _, _ = next((f for f in forms if (CHOICES.conv_stem != 64 or f[1] == 64) and patch_rows(f[1]) * pitch <= f[2]
@@ -864,6 +874,8 @@ def _conv_stem_launch(out, lhs, rhs, g: 'ConvGeometry', epilogue, taps, compute_
         return None
     per_image = _cdiv(g.Ho * g.Wo, tile)
     tiles     = g.batch * per_image
+    if CHOICES.conv_stem is None and not _conv_stem_pays(g, tile, tiles, compute_units):
+        return None
     #a second result (the value before or after the first epilogue step) goes to the last operand slot, as in conv_gemm_body
     flags  = slots << 20 | ((taps[0][0] + 1) << 12 if taps else 0)
     params = (_i32(M, N, K, g.Ho, g.Wo, g.H, g.W, g.Cin, g.KH, g.KW, g.SH, g.SW, g.PH, g.PW, pitch, left)
