@@ -694,8 +694,8 @@ __device__ __forceinline__ void softmax_rows_body(float* __restrict__ out, const
     if (l == 0 && first + sub < outer) arg_out[first + sub] = total == total ? best : 0u;
 }
 
-#define SOFTMAX_ROWS(name, VEC, NV)                                                                                         \
-    extern "C" __global__ __launch_bounds__(256) void name(                                                                 \
+#define SOFTMAX_ROWS(name, VEC, NV, ...)                                                                                    \
+    extern "C" __global__ __launch_bounds__(256) __VA_ARGS__ void name(                                                     \
         float* __restrict__ out, const float* __restrict__ in, uint32_t* __restrict__ arg_out, SoftmaxParams P) {           \
         softmax_rows_body<VEC, NV>(out, in, arg_out, P);                                                                    \
     }
@@ -719,7 +719,8 @@ SOFTMAX_ROWS(softmax_rows_v1_n16, 1, 16)
 SOFTMAX_ROWS(softmax_rows_v1_n24, 1, 24)
 SOFTMAX_ROWS(softmax_rows_v1_n32, 1, 32)
 SOFTMAX_ROWS(softmax_rows_v1_n48, 1, 48)
-SOFTMAX_ROWS(softmax_rows_v1_n64, 1, 64)
+// (left alone the compiler takes 261 registers, and a SIMD has a single wave to wait with: 16384 rows of 3233 130 us, with labels 141, so 85 and 88)
+SOFTMAX_ROWS(softmax_rows_v1_n64, 1, 64, __attribute__((amdgpu_waves_per_eu(2))))
 
 struct ReduceGeneralParams {
     uint32_t n_out, n_red, op, type;
