@@ -109,3 +109,17 @@ def test_where_it_is_taken(xs, columns, taken):
     zeros  = lambda *s: np.broadcast_to(np.float32(0), s)
     interp = JaxprInterpreter(mj.make_jaxpr(conv)(zeros(*xs), zeros(3, 3, xs[3], columns)), plan_only=True)
     assert (RAGGED in [l.kernel for l in interp.launches]) == bool(taken)
+
+
+@pytest.mark.parametrize('images,size,features,columns,layout,there', [
+    (11, 31, 397, 397, 'HWIO', True), (1, 8, 104, 104, 'HWIO', True), (64, 7, 200, 200, 'HWIO', True), (60, 40, 60, 60, 'HWIO', True), (47, 23, 44, 216, 'HWIO', True), (60, 40, 22, 22, 'HWIO', True),
+    (15, 38, 52, 78, 'HWOI', True), (113, 22, 8, 288, 'HWIO', False), (17, 54, 36, 88, 'HWIO', False), (78, 11, 40, 224, 'HWIO', False), (36, 15, 68, 360, 'HWIO', False),
+    (38, 35, 100, 32, 'HWIO', False), (27, 26, 104, 24, 'HWIO', False), (10, 18, 104, 264, 'HWIO', False), (38, 56, 8, 218, 'HWIO', False), (93, 58, 72, 4, 'HWIO', False), (107, 43, 52, 24, 'HWIO', False), (24, 14, 33, 152, 'HWIO', False), (125, 32, 4, 286, 'HWOI', False)])
+def test_where_they_pay(images, size, features, columns, layout, there):
+    '''Plan only: not where so many features are padding, or columns, that the fp32 kernels are ahead.'''
+    def f(x, w):
+        return lax.conv_general_dilated(x, w, (1, 1), ((1, 1), (1, 1)), dimension_numbers=('NHWC', layout, 'NHWC'))
+    zeros   = lambda *s: np.broadcast_to(np.float32(0), s)
+    kernel  = zeros(3, 3, columns, features) if layout == 'HWOI' else zeros(3, 3, features, columns)
+    program = JaxprInterpreter(mj.make_jaxpr(f)(zeros(images, size, size, features), kernel), plan_only=True)
+    assert (RAGGED in [l.kernel for l in program.launches]) == there, [l.kernel for l in program.launches]
