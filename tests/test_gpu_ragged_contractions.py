@@ -69,3 +69,12 @@ def test_strided_pixels_of_an_odd_number_of_features():
 def test_many_rows_of_few_features_go_to_tiles():
     shapes = [(2048, 257, 10), (2049, 257, 10), (1280, 510, 16), (1281, 510, 16), (100000, 256, 10)]
     assert ['dense' in kernel(layer, [np.zeros(s, np.float32) for s in ((m, k), (k, n), (n,))]) for m, k, n in shapes] == [True, False, True, False, True]
+
+
+def test_short_contractions_keep_their_epilogue():
+    '''Plan only: a residual behind a product of few odd features is part of its launch.'''
+    f    = lambda x, w, b, r: nn.relu(jnp.dot(x, w) + b + r)
+    plan = lambda m, k, n: [l.kernel for l in JaxprInterpreter(mj.make_jaxpr(f)(*[np.zeros(s, np.float32) for s in ((m, k), (k, n), (n,), (m, n))]), plan_only=True).launches]
+    for m, k, n in ((551, 25, 16), (3910, 13, 4), (61, 9, 16), (359, 17, 13), (50, 31, 8)):
+        assert len(plan(m, k, n)) == 1 and 'dense' not in plan(m, k, n)[0], (m, k, n)
+    assert plan(50, 33, 8)[0] == 'dense_rows_n16' and plan(50, 28, 8)[0] == 'dense_rows_n16'

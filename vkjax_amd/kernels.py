@@ -898,6 +898,9 @@ DENSE_ROWS_MAX_N = 16
 #Rows x features up to which a wave per row serves contractions that are no multiple of four: a tile for 32 rows is faster beyond (us there and by tiles: 1024 x 511 x 8 4.6, 6.3;
 #5017 x 249 x 14 12.9, 5.0; 16384 x 511 x 8 36, 10; 131072 x 511 x 8 270, 57), and is as fast with multiples of four, whose sums are 2 to 3 times as far from 64 bits there
 #(4096 x 256 x 10 1.5e-7, here 7.7e-8; the others came from tiles with 64-wide steps, 3.9e-7 for 64 x 511 x 8, where they are 8.8e-8)
+#Of contractions that are no multiple of four: up to 32 long only this few results, because a tile takes one step for them and its epilogue any operand, which is a launch more here
+#(us here and by four waves per tile; 600 x 25 x 16 4.1, 3.4, with a residual 7.2, 4.0; 4000 x 13 x 4 4.0, 3.5, 7.3, 4.1; 50 x 7 x 8 2.8, 3.1, 5.6, 3.8)
+DENSE_ROWS_SHORT_RESULTS = 64
 DENSE_ROWS_MAX_RESULTS = 20480
 
 
@@ -910,7 +913,7 @@ def _dense_rows_shape(lhs: Buffer, g: 'ConvGeometry') -> bool:
     M, N, K = g.M, g.N, g.K
     flat = (g.batch == 1 and g.Wo == 1 and g.KH == g.KW == 1 and g.SH == 1 and g.PH == g.PW == 0 and g.LH == 1 and g.H == g.Ho
             and g.xs[3] == 1 and g.xs[1] >= K)
-    return (flat and 1 <= N <= DENSE_ROWS_MAX_N and (K % 4 == 0 or M * N <= DENSE_ROWS_MAX_RESULTS) and K > 0 and tuple(g.ws[2:]) == (N, 1) and tuple(g.os[1:]) == (N, N, 1)
+    return (flat and 1 <= N <= DENSE_ROWS_MAX_N and (K % 4 == 0 or M * N <= (DENSE_ROWS_MAX_RESULTS if K > 32 else DENSE_ROWS_SHORT_RESULTS)) and K > 0 and tuple(g.ws[2:]) == (N, 1) and tuple(g.os[1:]) == (N, N, 1)
             and lhs.size * 4 < 2**31 and M * N * 4 < 2**31)
 
 
