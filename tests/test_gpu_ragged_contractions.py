@@ -78,3 +78,18 @@ def test_short_contractions_keep_their_epilogue():
     for m, k, n in ((551, 25, 16), (3910, 13, 4), (61, 9, 16), (359, 17, 13), (50, 31, 8)):
         assert len(plan(m, k, n)) == 1 and 'dense' not in plan(m, k, n)[0], (m, k, n)
     assert plan(50, 33, 8)[0] == 'dense_rows_n16' and plan(50, 28, 8)[0] == 'dense_rows_n16'
+
+
+def test_large_full_tensors_behind_one_step():
+    f    = lambda x, w, b, r: nn.relu(jnp.dot(x, w) + b + r)
+    zero = lambda *s: np.broadcast_to(np.float32(0), s)
+    plan = lambda m, k, n: JaxprInterpreter(mj.make_jaxpr(f)(zero(m, k), zero(k, n), zero(n), zero(m, n)), plan_only=True).launches[0].kernel
+    for m, k, n, kernel in ((255921, 13, 104, 'gf'), (24088, 5, 256, 'gf'), (255921, 12, 104, 'lean'), (179393, 33, 64, 'lean'), (40426, 6, 104, 'lean')):
+        assert plan(m, k, n).endswith('_' + kernel), (m, k, n, plan(m, k, n))
+
+
+@pytest.mark.gpu
+def test_values_of_large_full_tensors_behind_one_step():
+    rng = np.random.default_rng(8)
+    x, w, b, r = (rng.integers(-4, 5, size=s).astype(np.float32) for s in ((60001, 7), (7, 90), (90,), (60001, 90)))
+    assert np.array_equal(vkjax_amd.wrap(lambda x, w, b, r: nn.relu(jnp.dot(x, w) + b + r), frontend='minijax')(x, w, b, r), np.maximum(x @ w + b + r, 0))

@@ -1211,6 +1211,11 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
     bk = choose_conv_bk(tag, g)
     needs_masks, x_bias, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g, lhs_offset, rhs_offset)
     slots = _epilogue_template_slots(epilogue)
+    #One step of a contraction that is no multiple of four, and a large full tensor behind it: all of it is time in memory, and the kernels that load word by word overlap
+    #that better than those that fetch the tensor a tile ahead (us by vectors and words: 255921 x 13 x 104 60.7, 49.4; 230625 x 6 x 104 52.9, 44.0; 221664 x 13 x 24 22.0, 17.3;
+    #24088 x 5 x 256 14.3, 13.4; but 40426 x 6 x 104 11.4, 11.9; 73931 x 5 x 48 10.8, 11.8; 179393 x 33 x 64 28.7, 31.2)
+    if K % 4 != 0 and K <= 32 and slots & 8 and M * N >= 5 << 20:
+        a_fast = False
     #the lean kernel variant covers the common case only (see the kernel source)
     lean = (a_fast and b_fast and c_contig and (g.Cin % bk == 0 or g.KH * g.KW == 1)
             and (not epilogue or slots != 0) and not CHOICES.conv_general)
