@@ -89,3 +89,17 @@ def test_share_counts():
     '''One block per tile where that fills the CUs or the contraction is short; never more blocks than steps.'''
     assert [K.choose_conv_shares(*a) for a in ((100, 4), (128, 4), (200, 18), (200, 8), (400, 16), (2048, 36), (400, 36))] == [1] * 7
     assert all(1 < K.choose_conv_shares(*a) <= min(a[1], K.CONV_MAX_SHARES) for a in ((56, 18), (56, 8), (100, 9), (104, 18), (112, 36), (160, 36), (304, 36)))
+
+
+def test_what_shared_tiles_need_is_refused_otherwise():
+    '''With the error that callers who try a part of a product expect, who then launch the whole of it.'''
+    buffer = lambda *shape: K.Buffer(None, np.dtype(np.float32), shape)
+    out, lhs, rhs = buffer(70, 40), buffer(70, 1026), buffer(1026, 40)
+    geom = K.ConvGeometry(batch=1, Ho=70, Wo=1, N=40, H=70, W=1, Cin=1026, KH=1, KW=1, xs=(0, 1026, 0, 1), ws=(1026 * 40, 1026 * 40, 40, 1), os=(70 * 40, 40, 40, 1))
+    with K.overrides(conv_ksplit=True):
+        def launch(count=3, partial=3 * 6 * 1024, arrivals=K.CONV_MAX_SHARED_TILES, **offsets):
+            return K.conv_gemm(out, lhs, rhs, geom._replace(shares=K.ConvShares(count, buffer(partial), buffer(arrivals))), **offsets)
+        assert launch().kernel == 'conv_gemm_32x32x128_ks4_shared'
+        for wrong in (dict(out_offset=4), dict(count=7, partial=7 * 6 * 1024), dict(arrivals=5), dict(partial=3 * 6 * 1024 - 1)):
+            with pytest.raises(ValueError):
+                launch(**wrong)

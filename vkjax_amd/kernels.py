@@ -1246,7 +1246,9 @@ def conv_gemm(out: Buffer, lhs: Buffer, rhs: Buffer, g: ConvGeometry, epilogue: 
             raise ValueError('a sliced contraction needs the four-waves-per-tile kernel, no epilogue and one [M, N] matrix per non-empty slice')
     elif g.shares is not None and ksplit and not short_step and not strided:
         k_split_steps = _cdiv(_cdiv(K, bk), g.shares.count)
-        assert _cdiv(_cdiv(K, bk), k_split_steps) == g.shares.count and tiles_m * tiles_n <= g.shares.arrivals.size and not out_offset
+        if (out_offset or _cdiv(_cdiv(K, bk), k_split_steps) != g.shares.count or tiles_m * tiles_n > g.shares.arrivals.size
+                or g.shares.partial.size < tiles_m * tiles_n * g.shares.count * 1024):
+            raise ValueError('shared tiles need a whole result, a non-empty slice for every block, and scratch for all of them')
     chunk = (CHOICES.conv_chunk or choose_conv_chunk(tiles_m, tiles_n, compute_units)) if lean and not ksplit else 1
     m_blocks = 0
     if lean and not ksplit and CHOICES.conv_chunk is None:
