@@ -97,3 +97,23 @@ def test_threads_with_programs_of_their_own():
     for t in threads: t.start()
     for t in threads: t.join()
     assert not failures, failures[:5]
+
+
+def test_more_programs_than_a_page_of_mailboxes():
+    '''Sequences that live together have places of their own, those that come later take the places of those that went.'''
+    x, w = numbers(1, 5, 24), numbers(2, 24, 40)
+    y    = x @ w
+    jaxpr, live = mj.make_jaxpr(steps)(x, w), []
+    for k in range(140):
+        program = JaxprInterpreter(jaxpr)
+        program.upload_inputs(x, w)
+        live.append(program)
+        if k % 3 == 2:
+            del live[k % len(live)]
+        for p in (live[0], live[-1]):
+            assert p.replay(1) > 0
+    assert len(live) > 64
+    for p in live:
+        p.replay(1)
+        for got, want in zip(p.read_outputs(), (y + 1, y.sum(axis=1), y * 2)):
+            assert np.array_equal(got, want)

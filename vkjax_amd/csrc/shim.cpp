@@ -178,6 +178,9 @@ int use(Ctx* c) {
 void destroy_ctx_objects(Ctx* c) {
     if (c->carry_count) hipFree(c->carry_count);
     c->carry_count = nullptr;
+    for (Mailbox* page : c->mailbox_pages) hipHostFree(page);
+    c->mailbox_pages.clear();
+    c->mailboxes.clear();
     if (c->ev_begin)    hipEventDestroy(c->ev_begin);
     if (c->ev_end)      hipEventDestroy(c->ev_end);
     if (c->ev_landed)   hipEventDestroy(c->ev_landed);
@@ -189,6 +192,34 @@ void destroy_ctx_objects(Ctx* c) {
     if (c->side_stream) hipStreamDestroy(c->side_stream);
     c->ev_begin = c->ev_end = c->ev_landed = c->ev_uploaded = c->ev_copied = nullptr;
     c->stream = c->copy_stream = c->side_stream = nullptr;
+}
+
+// A mailbox for a sequence: one that another has left, or one of another page
+int take_mailbox(Ctx* c, Mailbox** out) {
+    std::lock_guard<std::mutex> lock(c->mailbox_mutex);
+    if (c->mailboxes.empty()) {
+        constexpr size_t count = MAILBOX_PAGE / sizeof(Mailbox);
+        try {                                                                    // room for all of them: leaving one allocates nothing
+            c->mailbox_pages.reserve(c->mailbox_pages.size() + 1);
+            c->mailboxes.reserve(count * (c->mailbox_pages.size() + 1));
+        } catch (...) {
+            return fail(VKJ_ENOMEM, "vkj_seq_create: out of host memory");
+        }
+        void* page = nullptr;
+        HIP_TRY(hipSetDevice(c->device));
+        HIP_TRY(hipHostMalloc(&page, MAILBOX_PAGE, hipHostMallocDefault));
+        c->mailbox_pages.push_back((Mailbox*)page);
+        for (size_t k = count; k > 0; k--) c->mailboxes.push_back((Mailbox*)page + k - 1);
+    }
+    *out = c->mailboxes.back();
+    c->mailboxes.pop_back();
+    **out = Mailbox{};
+    return 0;
+}
+
+void leave_mailbox(Ctx* c, Mailbox* box) {
+    std::lock_guard<std::mutex> lock(c->mailbox_mutex);
+    c->mailboxes.push_back(box);
 }
 
 // A sequence lets go of a buffer it recorded; the memory of a buffer that vkj_buf_free has
@@ -981,13 +1012,10 @@ int vkj_seq_create(vkj_handle h, int profiling, vkj_handle* out) {
     s->ctx = c;
     s->profiling = profiling != 0;
     if (c->stamp) {
-        hipError_t e = hipSetDevice(c->device);
-        if (e == hipSuccess) e = hipHostMalloc((void**)&s->mailbox, sizeof(Mailbox), hipHostMallocDefault);
-        if (e != hipSuccess) {
+        if (int r = take_mailbox(c, &s->mailbox)) {
             delete s;
-            return hip_fail(e, "hipHostMalloc (mailbox)");
+            return r;
         }
-        *s->mailbox = Mailbox{0, 0, 0};
     }
     *out = to_handle(s);
     return 0;
@@ -999,7 +1027,7 @@ int vkj_seq_destroy(vkj_handle sh) {
     if (int r = use(s->ctx)) return r;
     hipStreamSynchronize(s->ctx->stream);
     hipStreamSynchronize(s->ctx->copy_stream);
-    if (s->mailbox) hipHostFree(s->mailbox);
+    if (s->mailbox) leave_mailbox(s->ctx, s->mailbox);          // (nothing on the stream writes to it any more)
     for (auto& m : s->slab_mirrors) hipHostFree(m.second);
     for (auto& t : s->uploads) {
         if (t.staging && !t.staging_mirrors_slab) hipHostFree(t.staging);

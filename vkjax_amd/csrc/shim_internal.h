@@ -53,9 +53,10 @@ constexpr size_t CARRY_OUT_MAX = 256u << 10;       // larger results leave with 
 // the wait for it take 15.4 us between two events, 11.4 with a synchronisation and 9.0 with a number. (Calls: affine layer on 8 samples 21.0 -> 17.0 us,
 // ResNet-50 on one image 553 -> 535; replays: 16 M random numbers 35.8 -> 33.7, a conv block 69.3 -> 67.0, softmax of 65536 rows 92 -> 90. Arguments of 784 KB
 // in pieces of 192 KB, copied to pinned memory while the piece before is on its way, took as long as in one: a launch for each costs what the overlap gives.)
-struct Mailbox { uint64_t done, begin, end; };       // begin, end: the clock of the GPU in front of and behind the launches of a replay
+struct Mailbox { uint64_t done, begin, end, unused[5]; };       // begin, end: the clock of the GPU in front of and behind the launches of a replay
 // What a launch writes behind its own results: `count` (device memory, zero between launches) tells its last block.
 struct Notice { uint32_t* count = nullptr; uint64_t* done = nullptr; uint64_t number = 0; };
+constexpr size_t MAILBOX_PAGE = 4096;
 constexpr double POLL_SECONDS = 1e-3;                 // from then on the stream is synchronised, which also reports errors
 constexpr int    POLLS_IN_A_ROW = 64;                 // evaluations after which it is in any case: the runtime lets go of finished launches then
 
@@ -85,6 +86,10 @@ struct Ctx {
     int       (*carry_out)(const Carry& what, const Notice& notice, hipStream_t stream) = nullptr;      // to the host, with a notice behind it
     int       (*stamp)(uint64_t* clock, uint64_t* done, uint64_t number, hipStream_t stream) = nullptr;
     uint32_t*   carry_count = nullptr;
+    // Mailboxes of the context's sequences, in pages of pinned memory that stay until the context goes; those that no sequence has. (A pinned allocation for each
+    // sequence took 26 us; building the smallest program 216 -> 190 us.)
+    std::mutex             mailbox_mutex;
+    std::vector<Mailbox*>  mailbox_pages, mailboxes;
     double      clock_khz = 0;
     int         polls = 0;
 };
