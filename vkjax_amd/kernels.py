@@ -1096,21 +1096,29 @@ CONV_SLICED_MAX_TILES = 32
 CONV_XCD_COLUMNWISE   = 5           #tiles go to the XCDs column by column
 
 
-def conv_k_splits(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int = 256) -> int:
+def conv_slicing(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int = 256) -> tp.Tuple[int, int]:
+    '''(slices, shares) of a product that the four-waves-per-tile kernels compute, at most one of them above 1: into how many slices its contraction is cut that
+    a launch of its own adds (conv_k_splits), and how many blocks share a tile and add theirs themselves (conv_share_count).'''
+    if _dense_rows_shape(lhs, g):
+        return 1, 1
+    f = _flatten_pointwise(g)
+    if f.K * f.N * 4 >= 2**31 or lhs.size * 4 >= 2**31 or f.M * f.N == 0:
+        return 1, 1
+    _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, f)
+    #(not the 64-long step: 196 x 9 of those 7.8 us, by two blocks each 9.3)
+    if not _four_waves_per_tile(f, a_fast, c_contig, compute_units, _kernel_operand_in_vectors(lhs, f, b_fast)) or (f.Cin % 128 != 0 and f.KH * f.KW != 1):
+        return 1, 1
+    tiles, ksteps = conv_shared_tiles(f), _cdiv(f.K, 128)
+    slices = conv_k_splits(tiles, ksteps, compute_units)
+    return slices, 1 if slices > 1 or g.k_splits > 1 or g.split is not None else conv_share_count(tiles, ksteps, compute_units)
+
+
+def conv_k_splits(tiles: int, ksteps: int, compute_units: int = 256) -> int:
     '''Into how many slices the contraction of a product with very few tiles is cut (1: not at all). With 32 blocks on
     256 CUs, a layer whose kernel operand is megabytes long (the 3 x 3 layers of a network's last stages at batch 1)
     is bound by the rate at which those few CUs fetch it; slices spread the fetch over the chip. Every slice keeps at
     least four k steps, at most four slices (the launch that adds them is an element-wise chain with room for a
     following scale, shift and ReLU), and never more blocks than CUs.'''
-    if _dense_rows_shape(lhs, g):
-        return 1
-    g = _flatten_pointwise(g)
-    if g.K * g.N * 4 >= 2**31 or lhs.size * 4 >= 2**31 or g.M * g.N == 0:
-        return 1
-    _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g)
-    if not _four_waves_per_tile(g, a_fast, c_contig, compute_units, _kernel_operand_in_vectors(lhs, g, b_fast)) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
-        return 1
-    tiles, ksteps = conv_shared_tiles(g), _cdiv(g.K, 128)
     if CHOICES.conv_k_splits is not None:
         want = CHOICES.conv_k_splits
     else:
@@ -1156,21 +1164,11 @@ def choose_conv_shares(tiles: int, ksteps: int, compute_units: int = 256) -> int
     return count if time(count) < 0.98 * alone else 1
 
 
-def conv_share_count(lhs: Buffer, rhs: Buffer, g: ConvGeometry, compute_units: int = 256) -> int:
-    '''How many blocks share a tile where the four-waves-per-tile kernels compute the product (1: no sharing).'''
+def conv_share_count(tiles: int, ksteps: int, compute_units: int = 256) -> int:
+    '''How many blocks share a tile (1: no sharing).'''
     pinned = CHOICES.conv_k_splits is not None or CHOICES.conv_split is not None          #(to the kernels themselves: one block per tile)
-    if (CHOICES.conv_shares == 1 or (CHOICES.conv_shares is None and pinned) or g.k_splits > 1 or g.split is not None
-            or _dense_rows_shape(lhs, g)):
-        return 1
-    g = _flatten_pointwise(g)
-    if g.K * g.N * 4 >= 2**31 or lhs.size * 4 >= 2**31 or g.M * g.N == 0:
-        return 1
-    _, _, a_fast, b_fast, c_contig = _conv_fast_paths(lhs, rhs, g)
-    #(not the 64-long step: 196 x 9 of those 7.8 us, by two blocks each 9.3)
-    if not _four_waves_per_tile(g, a_fast, c_contig, compute_units, _kernel_operand_in_vectors(lhs, g, b_fast)) or (g.Cin % 128 != 0 and g.KH * g.KW != 1):
-        return 1
-    tiles, ksteps = conv_shared_tiles(g), _cdiv(g.K, 128)
-    if tiles > CONV_MAX_SHARED_TILES or (CHOICES.conv_shares is None and tiles <= CONV_SLICED_MAX_TILES):
+    if (CHOICES.conv_shares == 1 or tiles > CONV_MAX_SHARED_TILES
+            or (CHOICES.conv_shares is None and (pinned or tiles <= CONV_SLICED_MAX_TILES))):
         return 1
     want = min(CHOICES.conv_shares, ksteps, CONV_MAX_SHARES) if CHOICES.conv_shares is not None else choose_conv_shares(tiles, ksteps, compute_units)
     return _cdiv(ksteps, _cdiv(ksteps, want))

@@ -617,8 +617,7 @@ def _product_ops(bufferpool, equation, outbuf, lhs, rhs, geom: 'K.ConvGeometry')
     '''The implicit-GEMM launch of a convolution or matrix product, with scratch for blocks that share its tiles; for a product with
     very few output tiles and a long contraction, a launch that sums slices of the contraction into a temporary and an element-wise
     launch that adds the slices in order (which later takes over the element-wise equations that follow).'''
-    splits = K.conv_k_splits(lhs, rhs, geom)
-    shares = K.conv_share_count(lhs, rhs, geom) if splits <= 1 else 1
+    splits, shares = K.conv_slicing(lhs, rhs, geom)
     if shares > 1:
         tiles = K.conv_shared_tiles(geom)
         geom  = geom._replace(shares=K.ConvShares(shares, bufferpool.shared_scratch(tiles * shares * 1024, 'slices of shared tiles'),
