@@ -114,7 +114,7 @@ def test_where_it_is_taken(xs, columns, taken):
 @pytest.mark.parametrize('images,size,features,columns,layout,there', [
     (11, 31, 397, 397, 'HWIO', True), (1, 8, 104, 104, 'HWIO', True), (64, 7, 200, 200, 'HWIO', True), (60, 40, 60, 60, 'HWIO', True), (47, 23, 44, 216, 'HWIO', True), (60, 40, 22, 22, 'HWIO', True),
     (15, 38, 52, 78, 'HWOI', True), (113, 22, 8, 288, 'HWIO', False), (17, 54, 36, 88, 'HWIO', False), (78, 11, 40, 224, 'HWIO', False), (36, 15, 68, 360, 'HWIO', False),
-    (38, 35, 100, 32, 'HWIO', False), (27, 26, 104, 24, 'HWIO', False), (10, 18, 104, 264, 'HWIO', False), (38, 56, 8, 218, 'HWIO', False), (93, 58, 72, 4, 'HWIO', False), (107, 43, 52, 24, 'HWIO', False), (24, 14, 33, 152, 'HWIO', False), (125, 32, 4, 286, 'HWOI', False)])
+    (38, 35, 100, 32, 'HWIO', False), (27, 26, 104, 24, 'HWIO', False), (38, 56, 8, 218, 'HWIO', False), (93, 58, 72, 4, 'HWIO', False), (107, 43, 52, 24, 'HWIO', False), (24, 14, 33, 152, 'HWIO', False), (79, 18, 68, 68, 'HWIO', True), (98, 26, 36, 36, 'HWIO', False), (15, 38, 40, 144, 'HWOI', True), (125, 43, 80, 8, 'HWOI', False), (7, 31, 120, 120, 'HWIO', True), (10, 18, 104, 264, 'HWIO', False), (125, 32, 4, 286, 'HWOI', False)])
 def test_where_they_pay(images, size, features, columns, layout, there):
     '''Plan only: not where so many features are padding, or columns, that the fp32 kernels are ahead.'''
     def f(x, w):

@@ -1397,36 +1397,38 @@ def _conv_short_pays(g: ConvGeometry) -> bool:
     return g.N % 32 == 0 and g.N >= 96 and g.K > 32 and g.M * g.N >= 1 << 24
 
 
-def _conv_ragged_pays(g: ConvGeometry, kernel_in_vectors: bool) -> bool:
+def _conv_ragged_pays(g: ConvGeometry, dense: bool, copied: bool) -> bool:
     '''3 x 3 windows over a number of features that is no multiple of 32, for which the fp32 kernels look every vector's tap up (or, without whole
     vectors, every word's): where the kernel that holds a patch, whose errors are no larger, is faster, its packing launch included (us there and here).
-    `kernel_in_vectors`: those kernels would load the kernel operand in vectors.'''
+    `dense`: the kernel operand is laid out as those load it in vectors; `copied`: it would be copied into that layout for them.'''
+    one_round = 200 <= _cdiv(g.M, 64) * _cdiv(g.N, 64) <= 256           #their 64 x 64 tiles keep every CU busy once
+    flops     = 2 * g.M * g.N * g.K
     #loads of words, images x size, features: 1 x 8, 22 15.8, 13.1; 60 x 40, 22 37.7, 27.8; 30 x 14, 41 25.3, 18.2; 11 x 31, 397 589, 209; 3 x 22, 417 219, 55; but 4 x 14, 17
-    #12.5, 13.5; 60 x 40, 9 18.5, 26.7
-    one_round = 200 <= _cdiv(g.M, 64) * _cdiv(g.N, 64) <= 256           #their 64 x 64 tiles keep every CU busy once (4704 x 33 to 152 22.4, 23.5)
+    #12.5, 13.5; 60 x 40, 9 18.5, 26.7; in one round 4704 x 33 to 152 22.4, 23.5
     if g.Cin % 4 != 0:
-        return g.Cin >= 20 and not (one_round and 33 <= g.Cin <= 36)
-    flops = 2 * g.M * g.N * g.K
-    #of vectors, where the kernel operand's loads are of words: 336 x 76 to 288 34, 19; 29602 x 52 to 78 69, 34; 11520 x 80 to 306 101, 51; 6272 x 152 to 30 65, 27; but
-    #125 x 32 x 32 x 4 to 286 153, 158
-    if not kernel_in_vectors:
-        return (g.Cin >= 100 and (g.N >= 24 or g.M <= 8192)) or (g.Cin >= 60 and g.M <= 1024) or (g.Cin >= 12 and flops >= 1.5e9)
-    #otherwise, padded to 32: by so much that the fp32 kernels are ahead until there are many operations (54692 x 8 to 288 48, 76; 49572 x 36 to 88 45, 51; 9438 x 40 to 224
-    #30, 32; 8100 x 68 to 360 43, 49; but 24986 x 44 to 216 (4.3 GFLOP) 58, 54, 68400 x 68 to 112 126, 99), ...
-    padded = _cdiv(g.Cin, 32) * 32 >= 1.35 * g.Cin
+        return g.Cin >= 20 and not (dense and one_round and 33 <= g.Cin <= 36)
+    #Of vectors, another layout of the kernel operand (that of an input gradient, often with the backward pass of a ReLU behind it, which is part of the launch here): by words 336 x
+    #76 to 288 34, 19; 29602 x 52 to 78 69, 34; 11520 x 80 to 306 101, 51; but 128000 x 4 to 286 153, 158; copied 21660 x 40 to 144 48, 37; but 231125 x 80 to 8 121, 137
+    if not dense:
+        return ((g.Cin >= 100 and (g.N >= 24 or g.M <= 8192)) or (g.Cin >= 60 and g.M <= 1024)
+                or (g.Cin >= 12 and flops >= 1.5e9 and not (copied and g.N <= 32 and g.Cin < 144)))
+    #the dense one; a long contraction (1 x 8, 104 27.7, 18.3; 64 x 7, 200 50, 39; 16 x 14, 136 35, 29), but not where those compute no column too many (60 x 28, 100 to 17 43.5,
+    #47.6; 46550 x 100 to 32 43.5, 48; 18252 x 104 to 24 30, 33; 15984 x 152 to 24 39, 34), nor in one round where a sixth of the features is padding (3240 x 104 to 264 33, 36; 2704
+    #x 132 to 296 35, 38; 6727 x 120 to 120 31.6, 29.3), ...
+    times = _cdiv(g.Cin, 32) * 32 / g.Cin
     if g.Cin >= 100:
-        #... a long contraction (1 x 8, 104 27.7, 18.3; 64 x 7, 200 50, 39; 16 x 14, 136 35, 29), but not where those compute no column too many (60 x 28, 100 to 17 43.5, 47.6;
-        #46550 x 100 to 32 43.5, 48; 18252 x 104 to 24 30, 33; 15984 x 152 to 24 39, 34), nor in one round (3240 x 104 to 264 33, 36; 2704 x
-        #132 to 296 35, 38; 3312 x 152 to 240 38.5, 35), ...
-        if g.Cin < 144 and (one_round or (g.N <= 32 and g.M > 8192)):
+        if g.Cin < 144 and ((one_round and times >= 1.2) or (g.N <= 32 and g.M > 8192)):
             return False
-        return g.N >= 24 or g.M <= 8192
+        if g.N >= 24 or g.M <= 8192:
+            return True
     #... few positions (4 x 14, 60 18.1, 16.9; 4 x 14, 80 22.6, 18.3; but 560 x 68 to 272 20.8, 21.8, 30 x 14, 72 21.7, 25.3), or many operations (60 x 40, 60
-    #71.9, 53.2; 2888 x 92 to 344 33, 29; but 10 x 40, 60 20.0, 25.0), fewer of them ...
-    #... for up to 64 columns, which those kernels pad (96000 x 36 to 36 47.8, 43.5; 57154 x 40 to 40 35, 33.5)
-    #(up to 32 those do not: 312852 x 72 to 4 137, 172; 197843 x 52 to 24 77, 96; 75625 x 80 to 32 49, 55)
-    return ((g.Cin >= 60 and not padded and g.M <= 1024) or (g.Cin >= 44 and g.N > 32 and flops >= (4e9 if padded else 1.5e9))
-            or (g.Cin >= 36 and 32 < g.N <= 64 and flops >= 1.5e9))
+    #71.9, 53.2; 2888 x 92 to 344 33, 29; 112896 x 240 to 8 171, 165; but 10 x 40, 60 20.0, 25.0), more of them where much is padding (54692 x 8 to 288 48, 76; 49572 x 36 to 88 45,
+    #51; 9438 x 40 to 224 30, 32; 8100 x 68 to 360 43, 49; 20800 x 68 to 68 34, 38; but 24986 x 44 to 216 58, 54, 25596 x 68 to 68 44.7, 41.7, 68400 x 68 to 112 126, 99), and not for
+    #up to 32 columns, which those do not pad (312852 x 72 to 4 137, 172; 197843 x 52 to 24 77, 96; 75625 x 80 to 32 49, 55); to 64, which they do, from fewer features on (96000 x 36 to 36
+    #47.8, 43.5; 57154 x 40 to 40 35, 33.5; but 66248 x 36 to 36 37, 40), or from more operations on (62424 x 40 to 328 176, 161)
+    return ((g.Cin >= 60 and times < 1.35 and g.M <= 1024) or (g.Cin >= 144 and flops >= 1.5e9)
+            or (g.Cin >= 44 and g.N > 32 and flops >= (4e9 if times >= 1.35 and g.M < 24576 else 1.5e9))
+            or (g.Cin >= 36 and g.N > 32 and flops >= (1.6e9 if g.N <= 64 else 8e9)))
 
 
 def _conv_patch_pays(g: ConvGeometry, c_contig: bool) -> bool:
@@ -1484,7 +1486,7 @@ def conv_split_plan(lhs: Buffer, g: ConvGeometry) -> tp.Optional[ConvSplit]:
     if wanted and conv_short_applies(g, c_contig) and (CHOICES.conv_short or _conv_short_pays(g)):
         return ConvSplit('128x64', _cdiv(M, 128) * _cdiv(N, 64), 1, short=True)
     ragged = (conv_ragged_applies(g) and not patch and CHOICES.conv_split is None and CHOICES.conv_split_slices is None
-              and (CHOICES.conv_ragged if CHOICES.conv_ragged is not None else _conv_ragged_pays(g, _dense_kernel(g) or dense_copy_pays(lhs, g))))
+              and (CHOICES.conv_ragged if CHOICES.conv_ragged is not None else _conv_ragged_pays(g, _dense_kernel(g), dense_copy_pays(lhs, g))))
     if not tiled and not ragged:
         return None
     if ragged:
