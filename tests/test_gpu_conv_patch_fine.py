@@ -109,3 +109,23 @@ def test_pinned_to_the_patch_kernels():
                 interp = JaxprInterpreter(mj.make_jaxpr(f)(zeros(2, 14, 14, 64), zeros(window, window, 64, 64)), plan_only=True)
                 name,  = [l.kernel for l in interp.launches if l.kernel.startswith('conv_gemm')]
                 assert name.endswith(expected) if expected else '_split' not in name, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('share', (0.004, 1 / 16, 1.0))
+@pytest.mark.parametrize('xs,columns', [([4, 7, 7, 1024], 256), ([12, 7, 7, 768], 512)], ids=lambda v: 'x'.join(map(str, v)) if isinstance(v, list) else str(v))
+def test_error_beside_shared_tiles(xs, columns, share):
+    '''Nor larger than that of the kernels whose blocks share a tile, which add shorter sums than one block does, and which would compute these products.'''
+    x, k = rng.standard_normal(xs).astype(np.float32), rng.standard_normal((3, 3, xs[3], columns)).astype(np.float32)
+    x   *= rng.random_sample(x.shape) < share
+    xp   = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1), (0, 0)))
+    exact = sum(xp[:, r:r + xs[1], s:s + xs[2]] @ k[r, s].astype(np.float64) for r in range(3) for s in range(3))
+    def error(kernel, **choice):
+        with K.overrides(**choice):
+            fn = vkjax_amd.wrap(conv, frontend='minijax')
+            y  = fn(x, k)
+        assert kernels_of(fn) == [kernel]
+        return np.linalg.norm(y - exact) / np.linalg.norm(exact)
+    here, there = error(FINE, conv_patch='fine'), error('conv_gemm_32x32x128_ks4_shared', conv_patch=False, conv_ragged=False)
+    print(f'{xs} {columns}, {share}: {here:.4g}, {there:.4g}', flush=True)
+    assert here <= 1.01 * there
